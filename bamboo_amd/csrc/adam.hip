@@ -192,11 +192,11 @@ extern "C" int bb_grad_clip_coef(int n_tensors, void* const* g, const int64_t* s
         }
         t.first_block[t.count] = (int)blocks;
         if (blocks > 0) {
-            hipLaunchKernelGGL(sumsq_partial_kernel, dim3((unsigned)blocks), dim3(256), 0, st, t, slots);
+            bb_launch(sumsq_partial_kernel, dim3((unsigned)blocks), dim3(256), 0, st, t, slots);
             BB_LAUNCH_CHECK();
         }
         // also with no blocks at all: out = {0, 1}
-        hipLaunchKernelGGL(clip_coef_kernel, dim3(1), dim3(256), 0, st, slots, blocks, first, max_norm, out, carry);
+        bb_launch(clip_coef_kernel, dim3(1), dim3(256), 0, st, slots, blocks, first, max_norm, out, carry);
         BB_LAUNCH_CHECK();
         first = 0;
     } while (i < n_tensors);
@@ -270,7 +270,7 @@ static int adam_multi_run(int n_tensors, void* const* g, void* const* p, void* c
         }
         if (t.count == 0) continue;
         t.first_block[t.count] = (int)blocks;
-        hipLaunchKernelGGL(adam_multi_kernel, dim3((unsigned)blocks), dim3(256), 0, st, t, h);
+        bb_launch(adam_multi_kernel, dim3((unsigned)blocks), dim3(256), 0, st, t, h);
         BB_LAUNCH_CHECK();
     }
     return BB_OK;

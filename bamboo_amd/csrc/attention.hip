@@ -40,6 +40,7 @@ struct AttnArgs {
     float scale;                                   // 1 / sqrt(d)
     DropKey drop;                                  // dropout on the probabilities (thresh 0: none)
 };
+template <> struct BbDropAt<AttnArgs> { static constexpr int32_t value = offsetof(AttnArgs, drop); };
 // index of probability (b, head, q, kv) in the [batch, heads, seq, seq] tensor that is never stored
 __device__ __forceinline__ uint64_t prob_index(const AttnArgs& a, int b, int head, int q) {
     return ((uint64_t)(b * a.heads + head) * a.seq + q) * a.seq;
@@ -753,14 +754,14 @@ extern "C" int bb_attention_fwd(int dtype, int mask, int batch, int heads, int s
     const dim3 grid(attn_grid(seq, batch * (heads / hp)));
     hipStream_t st = (hipStream_t)stream;
     if (head_dim == 128) {
-        if (a.drop.thresh) hipLaunchKernelGGL((attn_fwd_kernel<true, 1, 2>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((attn_fwd_kernel<false, 1, 2>), grid, dim3(256), 0, st, a);
+        if (a.drop.thresh) bb_launch((attn_fwd_kernel<true, 1, 2>), grid, dim3(256), 0, st, a);
+        else bb_launch((attn_fwd_kernel<false, 1, 2>), grid, dim3(256), 0, st, a);
     } else if (hp == 1) {
-        if (a.drop.thresh) hipLaunchKernelGGL((attn_fwd_kernel<true, 1>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((attn_fwd_kernel<false, 1>), grid, dim3(256), 0, st, a);
+        if (a.drop.thresh) bb_launch((attn_fwd_kernel<true, 1>), grid, dim3(256), 0, st, a);
+        else bb_launch((attn_fwd_kernel<false, 1>), grid, dim3(256), 0, st, a);
     } else {
-        if (a.drop.thresh) hipLaunchKernelGGL((attn_fwd_kernel<true, 2>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((attn_fwd_kernel<false, 2>), grid, dim3(256), 0, st, a);
+        if (a.drop.thresh) bb_launch((attn_fwd_kernel<true, 2>), grid, dim3(256), 0, st, a);
+        else bb_launch((attn_fwd_kernel<false, 2>), grid, dim3(256), 0, st, a);
     }
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -797,28 +798,28 @@ extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int s
         const dim3 grid2(attn_grid(seq, batch * heads * 2));
         if (a.drop.thresh) {
             BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)attn_bwd_dkv_kernel<true, 1, 2>, smem));
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<true, 1, 2>), grid, dim3(256), 0, st, a);
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<true, 1, 2>), grid2, dim3(256), smem, st, a);
+            bb_launch((attn_bwd_dq_kernel<true, 1, 2>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dkv_kernel<true, 1, 2>), grid2, dim3(256), smem, st, a);
         } else {
             BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)attn_bwd_dkv_kernel<false, 1, 2>, smem));
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<false, 1, 2>), grid, dim3(256), 0, st, a);
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<false, 1, 2>), grid2, dim3(256), smem, st, a);
+            bb_launch((attn_bwd_dq_kernel<false, 1, 2>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dkv_kernel<false, 1, 2>), grid2, dim3(256), smem, st, a);
         }
     } else if (hp == 1) {
         if (a.drop.thresh) {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<true, 1>), grid, dim3(256), 0, st, a);
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<true, 1>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dq_kernel<true, 1>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dkv_kernel<true, 1>), grid, dim3(256), 0, st, a);
         } else {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<false, 1>), grid, dim3(256), 0, st, a);
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<false, 1>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dq_kernel<false, 1>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dkv_kernel<false, 1>), grid, dim3(256), 0, st, a);
         }
     } else {
         if (a.drop.thresh) {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<true, 2>), grid, dim3(256), 0, st, a);
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<true, 2>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dq_kernel<true, 2>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dkv_kernel<true, 2>), grid, dim3(256), 0, st, a);
         } else {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<false, 2>), grid, dim3(256), 0, st, a);
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<false, 2>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dq_kernel<false, 2>), grid, dim3(256), 0, st, a);
+            bb_launch((attn_bwd_dkv_kernel<false, 2>), grid, dim3(256), 0, st, a);
         }
     }
     BB_LAUNCH_CHECK();

@@ -6,7 +6,9 @@
 #include <string.h>
 
 #include <mutex>
+#include <tuple>
 #include <unordered_map>
+#include <utility>
 
 #include "../../include/bamboo_hip.h"
 
@@ -214,6 +216,36 @@ static inline DropKey bb_drop_key(float p, uint32_t k0, uint32_t k1, uint64_t nu
         d.scale = 1.0f / (1.0f - p);
     }
     return d;
+}
+
+// ---- kernel launches -----------------------------------------------------------------------
+// Every launch of the library goes through bb_launch.  While the calling thread records a launch plan (plan.hip), the
+// launch is also copied into it -- kernel, grid, argument bytes --, so that a fixed sequence can be issued again later
+// without its callers.  BbDropAt<T>: where an argument type carries a dropout key (-1: nowhere), the one thing in such a
+// sequence that changes from replay to replay.
+struct BbPlan;
+extern thread_local BbPlan* bb_recording;
+void bb_record_launch(const void* fn, dim3 grid, dim3 block, size_t lds, int nargs, void* const* args, const uint32_t* sizes,
+                      const int32_t* drop_at);
+template <typename T> struct BbDropAt { static constexpr int32_t value = -1; };
+template <> struct BbDropAt<DropKey> { static constexpr int32_t value = 0; };
+
+template <typename... P, size_t... I>
+static inline void bb_launch_tuple(void (*kern)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, std::tuple<P...>& a,
+                                   std::index_sequence<I...>) {
+    void* args[] = {(void*)&std::get<I>(a)...};
+    (void)hipLaunchKernel((const void*)kern, grid, block, args, lds, st);   // BB_LAUNCH_CHECK reads the error
+    if (bb_recording) {
+        const uint32_t sizes[] = {(uint32_t)sizeof(P)...};
+        const int32_t drop_at[] = {BbDropAt<P>::value...};
+        bb_record_launch((const void*)kern, grid, block, lds, (int)sizeof...(P), args, sizes, drop_at);
+    }
+}
+template <typename... P, typename... A>
+static inline void bb_launch(void (*kern)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, A&&... args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one argument per kernel parameter");
+    std::tuple<P...> a{static_cast<P>(args)...};
+    bb_launch_tuple(kern, grid, block, lds, st, a, std::index_sequence_for<P...>{});
 }
 
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -333,7 +333,7 @@ __global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_acc2_kernel(co
 template <typename T, int IT>
 static int ln_fwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift,
                          void* y, float* mean, float* rinv, hipStream_t st) {
-    hipLaunchKernelGGL((layernorm_fwd_kernel<T, IT>), dim3((rows + 3) / 4), dim3(256), 0, st, kind, rows, cols, eps,
+    bb_launch((layernorm_fwd_kernel<T, IT>), dim3((rows + 3) / 4), dim3(256), 0, st, kind, rows, cols, eps,
                        (const T*)x, (const T*)gain, (const T*)shift, (T*)y, mean, rinv);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -347,7 +347,7 @@ static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x,
     const size_t smem = one_pass ? all : (size_t)3 * 2 * cols * sizeof(float);
     auto kern = layernorm_bwd_kernel<T, IT>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));   // raised on the first (never captured) call that needs it
-    hipLaunchKernelGGL(kern, dim3(LN_BWD_BLOCKS), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
+    bb_launch(kern, dim3(LN_BWD_BLOCKS), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
                        (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -400,7 +400,7 @@ static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, 
     if (rows == 0) return BB_OK;
     auto finish = [&]() -> int {
         const int nb = (cols + 63) / 64;
-        hipLaunchKernelGGL(reduce_partials_acc2_kernel, dim3(nb, 2), dim3(RED_WAVES * 64), 0, st, workspace, LN_BWD_BLOCKS,
+        bb_launch(reduce_partials_acc2_kernel, dim3(nb, 2), dim3(RED_WAVES * 64), 0, st, workspace, LN_BWD_BLOCKS,
                            (int64_t)2 * cols, cols, dgain, dshift);
         BB_LAUNCH_CHECK();
         return BB_OK;
@@ -531,10 +531,10 @@ extern "C" int bb_colsum_acc(int dtype, int rows, int cols, const void* x, int64
     hipStream_t st = (hipStream_t)stream;
     dim3 grid((cols + 64 * vec - 1) / (64 * vec), COLSUM_SPLITS);
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(colsum_partial_kernel<bf16>, grid, dim3(256), 0, st, rows, cols, (const bf16*)x, ldx, workspace);
+        bb_launch(colsum_partial_kernel<bf16>, grid, dim3(256), 0, st, rows, cols, (const bf16*)x, ldx, workspace);
     else
-        hipLaunchKernelGGL(colsum_partial_kernel<float>, grid, dim3(256), 0, st, rows, cols, (const float*)x, ldx, workspace);
-    hipLaunchKernelGGL(reduce_partials_acc_kernel, dim3((cols + 63) / 64), dim3(RED_WAVES * 64), 0, st, workspace, COLSUM_SPLITS,
+        bb_launch(colsum_partial_kernel<float>, grid, dim3(256), 0, st, rows, cols, (const float*)x, ldx, workspace);
+    bb_launch(reduce_partials_acc_kernel, dim3((cols + 63) / 64), dim3(RED_WAVES * 64), 0, st, workspace, COLSUM_SPLITS,
                        (int64_t)cols, cols, out);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -634,14 +634,14 @@ __global__ __launch_bounds__(256) void softmax_bwd_kernel(int sk, int64_t rows, 
 
 template <typename T, int IT>
 static int softmax_fwd_launch(int mask, int heads, int sq, int sk, int64_t rows, void* s, const int32_t* kl, hipStream_t st) {
-    hipLaunchKernelGGL((softmax_fwd_kernel<T, IT>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, mask, heads, sq, sk,
+    bb_launch((softmax_fwd_kernel<T, IT>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, mask, heads, sq, sk,
                        rows, (T*)s, kl);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
 template <typename T, int IT>
 static int softmax_bwd_launch(int sk, int64_t rows, const void* p, void* dp, hipStream_t st) {
-    hipLaunchKernelGGL((softmax_bwd_kernel<T, IT>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, sk, rows,
+    bb_launch((softmax_bwd_kernel<T, IT>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, sk, rows,
                        (const T*)p, (T*)dp);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -713,9 +713,9 @@ extern "C" int bb_residual_add(int dtype, int64_t n, const void* a, const void* 
     hipStream_t st = (hipStream_t)stream;
     const int64_t nvec = n / vec;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(add_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)a, (const bf16*)b, (bf16*)out);
+        bb_launch(add_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)a, (const bf16*)b, (bf16*)out);
     else
-        hipLaunchKernelGGL(add_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)a, (const float*)b, (float*)out);
+        bb_launch(add_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)a, (const float*)b, (float*)out);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -759,9 +759,9 @@ extern "C" int bb_sqrt_one_minus_fwd(int dtype, int64_t n, const void* x, void* 
     hipStream_t st = (hipStream_t)stream;
     const int64_t nvec = n / vec;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(sqrt1m_fwd_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)x, (bf16*)m);
+        bb_launch(sqrt1m_fwd_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)x, (bf16*)m);
     else
-        hipLaunchKernelGGL(sqrt1m_fwd_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)x, (float*)m);
+        bb_launch(sqrt1m_fwd_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)x, (float*)m);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -774,10 +774,10 @@ extern "C" int bb_sqrt_one_minus_bwd(int dtype, int64_t n, const void* dm, const
     hipStream_t st = (hipStream_t)stream;
     const int64_t nvec = n / vec;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(sqrt1m_bwd_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)dm, (const bf16*)m,
+        bb_launch(sqrt1m_bwd_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)dm, (const bf16*)m,
                            (bf16*)dx, accumulate);
     else
-        hipLaunchKernelGGL(sqrt1m_bwd_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)dm, (const float*)m,
+        bb_launch(sqrt1m_bwd_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)dm, (const float*)m,
                            (float*)dx, accumulate);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -813,9 +813,9 @@ extern "C" int bb_dropout_apply(int dtype, int64_t n, const void* src, void* dst
     const int64_t nvec = n / vec;
     hipStream_t st = (hipStream_t)stream;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(dropout_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)src, (bf16*)dst, key);
+        bb_launch(dropout_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const bf16*)src, (bf16*)dst, key);
     else
-        hipLaunchKernelGGL(dropout_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)src, (float*)dst, key);
+        bb_launch(dropout_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, (const float*)src, (float*)dst, key);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -865,9 +865,9 @@ extern "C" int bb_rowsum_fwd(int dtype, int rows, int cols, const void* x, void*
     if (rows == 0) return BB_OK;
     hipStream_t st = (hipStream_t)stream;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(rowsum_fwd_kernel<bf16>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const bf16*)x, (bf16*)y);
+        bb_launch(rowsum_fwd_kernel<bf16>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const bf16*)x, (bf16*)y);
     else
-        hipLaunchKernelGGL(rowsum_fwd_kernel<float>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const float*)x, (float*)y);
+        bb_launch(rowsum_fwd_kernel<float>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const float*)x, (float*)y);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -878,9 +878,9 @@ extern "C" int bb_rowsum_bwd(int dtype, int rows, int cols, const void* dy, void
     if (rows == 0) return BB_OK;
     hipStream_t st = (hipStream_t)stream;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(rowsum_bwd_kernel<bf16>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const bf16*)dy, (bf16*)dx);
+        bb_launch(rowsum_bwd_kernel<bf16>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const bf16*)dy, (bf16*)dx);
     else
-        hipLaunchKernelGGL(rowsum_bwd_kernel<float>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const float*)dy, (float*)dx);
+        bb_launch(rowsum_bwd_kernel<float>, dim3((rows + 3) / 4), dim3(256), 0, st, rows, cols, (const float*)dy, (float*)dx);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -915,11 +915,11 @@ extern "C" int bb_act_fwd(int dtype, int act, int64_t n, const void* x, void* ou
     const int64_t nvec = n / vec;
     dim3 grid(grid_for(nvec)), block(256);
     if (dtype == BB_BF16) {
-        if (dact) hipLaunchKernelGGL((act_kernel<bf16, true>), grid, block, 0, st, nvec, act, (const bf16*)x, (bf16*)out, (bf16*)dact);
-        else hipLaunchKernelGGL((act_kernel<bf16, false>), grid, block, 0, st, nvec, act, (const bf16*)x, (bf16*)out, (bf16*)nullptr);
+        if (dact) bb_launch((act_kernel<bf16, true>), grid, block, 0, st, nvec, act, (const bf16*)x, (bf16*)out, (bf16*)dact);
+        else bb_launch((act_kernel<bf16, false>), grid, block, 0, st, nvec, act, (const bf16*)x, (bf16*)out, (bf16*)nullptr);
     } else {
-        if (dact) hipLaunchKernelGGL((act_kernel<float, true>), grid, block, 0, st, nvec, act, (const float*)x, (float*)out, (float*)dact);
-        else hipLaunchKernelGGL((act_kernel<float, false>), grid, block, 0, st, nvec, act, (const float*)x, (float*)out, (float*)nullptr);
+        if (dact) bb_launch((act_kernel<float, true>), grid, block, 0, st, nvec, act, (const float*)x, (float*)out, (float*)dact);
+        else bb_launch((act_kernel<float, false>), grid, block, 0, st, nvec, act, (const float*)x, (float*)out, (float*)nullptr);
     }
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -948,15 +948,15 @@ extern "C" int bb_cast(int src_dtype, int dst_dtype, int64_t n, const void* src,
     hipStream_t st = (hipStream_t)stream;
     dim3 grid(grid_for(n)), block(256);
     if (src_dtype == BB_F32 && dst_dtype == BB_BF16)
-        hipLaunchKernelGGL((cast_kernel<float, bf16>), grid, block, 0, st, n, (const float*)src, (bf16*)dst);
+        bb_launch((cast_kernel<float, bf16>), grid, block, 0, st, n, (const float*)src, (bf16*)dst);
     else if (src_dtype == BB_BF16 && dst_dtype == BB_F32)
-        hipLaunchKernelGGL((cast_kernel<bf16, float>), grid, block, 0, st, n, (const bf16*)src, (float*)dst);
+        bb_launch((cast_kernel<bf16, float>), grid, block, 0, st, n, (const bf16*)src, (float*)dst);
     else if (src_dtype == BB_F32)
-        hipLaunchKernelGGL((cast_kernel<float, float>), grid, block, 0, st, n, (const float*)src, (float*)dst);
+        bb_launch((cast_kernel<float, float>), grid, block, 0, st, n, (const float*)src, (float*)dst);
     else if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0)
-        hipLaunchKernelGGL((copy_kernel<bf16>), dim3(grid_for(n / 8 + 1)), block, 0, st, n, (const bf16*)src, (bf16*)dst);
+        bb_launch((copy_kernel<bf16>), dim3(grid_for(n / 8 + 1)), block, 0, st, n, (const bf16*)src, (bf16*)dst);
     else
-        hipLaunchKernelGGL((cast_kernel<bf16, bf16>), grid, block, 0, st, n, (const bf16*)src, (bf16*)dst);
+        bb_launch((cast_kernel<bf16, bf16>), grid, block, 0, st, n, (const bf16*)src, (bf16*)dst);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -967,7 +967,7 @@ __global__ __launch_bounds__(256) void fill_kernel(float* dst, int64_t n, float 
 extern "C" int bb_fill_f32(float* dst, int64_t n, float value, void* stream) {
     BB_REQUIRE(n >= 0 && (dst || n == 0), "bb_fill_f32: bad arguments");
     if (n == 0) return BB_OK;
-    hipLaunchKernelGGL(fill_kernel, dim3(grid_for(n)), dim3(256), 0, (hipStream_t)stream, dst, n, value);
+    bb_launch(fill_kernel, dim3(grid_for(n)), dim3(256), 0, (hipStream_t)stream, dst, n, value);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -1014,10 +1014,10 @@ extern "C" int bb_mse_fwd_bwd(int dtype, int64_t n, const void* y, const void* t
     hipStream_t st = (hipStream_t)stream;
     const float gs = grad_scale * 2.0f / (float)n;
     if (dtype == BB_BF16)
-        hipLaunchKernelGGL(mse_partial_kernel<bf16>, dim3(MSE_BLOCKS), dim3(256), 0, st, n, (const bf16*)y, (const bf16*)target, (bf16*)dy, gs, workspace);
+        bb_launch(mse_partial_kernel<bf16>, dim3(MSE_BLOCKS), dim3(256), 0, st, n, (const bf16*)y, (const bf16*)target, (bf16*)dy, gs, workspace);
     else
-        hipLaunchKernelGGL(mse_partial_kernel<float>, dim3(MSE_BLOCKS), dim3(256), 0, st, n, (const float*)y, (const float*)target, (float*)dy, gs, workspace);
-    hipLaunchKernelGGL(mse_final_kernel, dim3(1), dim3(64), 0, st, workspace, 1.0f / (float)n, accumulate_loss, loss_out);
+        bb_launch(mse_partial_kernel<float>, dim3(MSE_BLOCKS), dim3(256), 0, st, n, (const float*)y, (const float*)target, (float*)dy, gs, workspace);
+    bb_launch(mse_final_kernel, dim3(1), dim3(64), 0, st, workspace, 1.0f / (float)n, accumulate_loss, loss_out);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -1549,13 +1549,13 @@ extern "C" int bb_batchnorm_fwd(int dtype, int rows, int cols, float eps, float 
     const int64_t nvec = (int64_t)rows * cols / vec;
     const dim3 block(BN_WAVES * 64);
     if (dtype == BB_BF16) {
-        hipLaunchKernelGGL((bn_colred_kernel<bf16, 0>), grid, block, 0, st, rows, cols, (const bf16*)x, nullptr, nullptr, nullptr, nullptr, workspace);
-        hipLaunchKernelGGL(bn_finish_kernel<bf16>, fgrid, dim3(256), 0, st, 1, rows, cols, eps, momentum, workspace, (const bf16*)x, mean, rstd, running_mean, running_var, nullptr, nullptr, nullptr);
-        hipLaunchKernelGGL(bn_apply_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, cols, relu, (const bf16*)x, mean, rstd, (const bf16*)gamma, (const bf16*)beta, (const bf16*)resid, (bf16*)y);
+        bb_launch((bn_colred_kernel<bf16, 0>), grid, block, 0, st, rows, cols, (const bf16*)x, nullptr, nullptr, nullptr, nullptr, workspace);
+        bb_launch(bn_finish_kernel<bf16>, fgrid, dim3(256), 0, st, 1, rows, cols, eps, momentum, workspace, (const bf16*)x, mean, rstd, running_mean, running_var, nullptr, nullptr, nullptr);
+        bb_launch(bn_apply_kernel<bf16>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, cols, relu, (const bf16*)x, mean, rstd, (const bf16*)gamma, (const bf16*)beta, (const bf16*)resid, (bf16*)y);
     } else {
-        hipLaunchKernelGGL((bn_colred_kernel<float, 0>), grid, block, 0, st, rows, cols, (const float*)x, nullptr, nullptr, nullptr, nullptr, workspace);
-        hipLaunchKernelGGL(bn_finish_kernel<float>, fgrid, dim3(256), 0, st, 1, rows, cols, eps, momentum, workspace, (const float*)x, mean, rstd, running_mean, running_var, nullptr, nullptr, nullptr);
-        hipLaunchKernelGGL(bn_apply_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, cols, relu, (const float*)x, mean, rstd, (const float*)gamma, (const float*)beta, (const float*)resid, (float*)y);
+        bb_launch((bn_colred_kernel<float, 0>), grid, block, 0, st, rows, cols, (const float*)x, nullptr, nullptr, nullptr, nullptr, workspace);
+        bb_launch(bn_finish_kernel<float>, fgrid, dim3(256), 0, st, 1, rows, cols, eps, momentum, workspace, (const float*)x, mean, rstd, running_mean, running_var, nullptr, nullptr, nullptr);
+        bb_launch(bn_apply_kernel<float>, dim3(grid_for(nvec)), dim3(256), 0, st, nvec, cols, relu, (const float*)x, mean, rstd, (const float*)gamma, (const float*)beta, (const float*)resid, (float*)y);
     }
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -1575,7 +1575,7 @@ extern "C" int bb_batchnorm_fwd_strips(int dtype, int rows, int cols, float eps,
     // about one block per CU; wide tensors get fewer row ranges (each repeats the strip reduction of its channels)
     const int slabs = (cols + 63) / 64;
     const int ranges = max(4, min(BN_FWD_ROW_RANGES, 256 / slabs));
-    hipLaunchKernelGGL(bn_fwd_strips_kernel, dim3(slabs, ranges), dim3(BN_STRIP_WAVES * 64), 0, st, rows, cols, eps, momentum, relu,
+    bb_launch(bn_fwd_strips_kernel, dim3(slabs, ranges), dim3(BN_STRIP_WAVES * 64), 0, st, rows, cols, eps, momentum, relu,
                        strip_stats, (const bf16*)x, (const bf16*)gamma, (const bf16*)beta, (const bf16*)resid, (bf16*)y, mean, rstd,
                        running_mean, running_var);
     BB_LAUNCH_CHECK();
@@ -1595,11 +1595,11 @@ extern "C" int bb_batchnorm_bwd(int dtype, int rows, int cols, const void* x, co
     dim3 agrid(slabs, max(4, min(64, 256 / slabs)));   // about one block per CU
     const dim3 block(BN_WAVES * 64);
     if (dtype == BB_BF16) {
-        hipLaunchKernelGGL((bn_colred_kernel<bf16, 2>), grid, block, 0, st, rows, cols, (const bf16*)x, mean, rstd, (const bf16*)dy, (const bf16*)relu_out, workspace);
-        hipLaunchKernelGGL(bn_bwd_finish_apply_kernel<bf16>, agrid, dim3(1024), 0, st, rows, cols, workspace, (const bf16*)x, mean, rstd, (const bf16*)gamma, (const bf16*)dy, (const bf16*)relu_out, (bf16*)dx, (bf16*)g_out, dgamma, dbeta);
+        bb_launch((bn_colred_kernel<bf16, 2>), grid, block, 0, st, rows, cols, (const bf16*)x, mean, rstd, (const bf16*)dy, (const bf16*)relu_out, workspace);
+        bb_launch(bn_bwd_finish_apply_kernel<bf16>, agrid, dim3(1024), 0, st, rows, cols, workspace, (const bf16*)x, mean, rstd, (const bf16*)gamma, (const bf16*)dy, (const bf16*)relu_out, (bf16*)dx, (bf16*)g_out, dgamma, dbeta);
     } else {
-        hipLaunchKernelGGL((bn_colred_kernel<float, 2>), grid, block, 0, st, rows, cols, (const float*)x, mean, rstd, (const float*)dy, (const float*)relu_out, workspace);
-        hipLaunchKernelGGL(bn_bwd_finish_apply_kernel<float>, agrid, dim3(1024), 0, st, rows, cols, workspace, (const float*)x, mean, rstd, (const float*)gamma, (const float*)dy, (const float*)relu_out, (float*)dx, (float*)g_out, dgamma, dbeta);
+        bb_launch((bn_colred_kernel<float, 2>), grid, block, 0, st, rows, cols, (const float*)x, mean, rstd, (const float*)dy, (const float*)relu_out, workspace);
+        bb_launch(bn_bwd_finish_apply_kernel<float>, agrid, dim3(1024), 0, st, rows, cols, workspace, (const float*)x, mean, rstd, (const float*)gamma, (const float*)dy, (const float*)relu_out, (float*)dx, (float*)g_out, dgamma, dbeta);
     }
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -1687,7 +1687,7 @@ extern "C" int bb_batchnorm_bwd_strip_sums(int dtype, int rows, int cols, const 
     BB_REQUIRE(x && mean && rstd && dy && strips, "bb_batchnorm_bwd_strip_sums: null pointer");
     BB_REQUIRE(!relu_out || g_out, "bb_batchnorm_bwd_strip_sums: with relu_out the masked gradient needs a place (g_out, may be dy)");
     const int nstrips = (rows + 31) / 32;
-    hipLaunchKernelGGL(bn_bwd_strip_sums_kernel, dim3((cols + 63) / 64, (nstrips + 3) / 4), dim3(256), 0, (hipStream_t)stream, rows, cols,
+    bb_launch(bn_bwd_strip_sums_kernel, dim3((cols + 63) / 64, (nstrips + 3) / 4), dim3(256), 0, (hipStream_t)stream, rows, cols,
                        (const bf16*)x, mean, rstd, (const bf16*)dy, (const bf16*)relu_out, (bf16*)g_out, strips);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -1702,7 +1702,7 @@ extern "C" int bb_batchnorm_bwd_strips(int dtype, int rows, int cols, const void
     BB_REQUIRE(x && gamma && mean && rstd && g && strips && dx && dgamma && dbeta, "bb_batchnorm_bwd_strips: null pointer");
     const int slabs = (cols + 63) / 64;
     dim3 agrid(slabs, max(4, min(64, 256 / slabs)));   // about one block per CU
-    hipLaunchKernelGGL(bn_bwd_strips_apply_kernel<bf16>, agrid, dim3(1024), 0, (hipStream_t)stream, rows, cols, strips, (const bf16*)x,
+    bb_launch(bn_bwd_strips_apply_kernel<bf16>, agrid, dim3(1024), 0, (hipStream_t)stream, rows, cols, strips, (const bf16*)x,
                        mean, rstd, (const bf16*)gamma, (const bf16*)g, (bf16*)dx, dgamma, dbeta);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -1766,11 +1766,11 @@ extern "C" int bb_patch3x3_strided(int dtype, int adjoint, int n, int h, int w, 
     const int64_t items = adjoint ? (int64_t)n * h * w * (c / vec) : (int64_t)n * ho * wo * 9 * (c / vec);
     dim3 grid(grid_for(items));
     if (dtype == BB_BF16) {
-        if (adjoint) hipLaunchKernelGGL((patch3x3_kernel<bf16, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
-        else hipLaunchKernelGGL((patch3x3_kernel<bf16, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
+        if (adjoint) bb_launch((patch3x3_kernel<bf16, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
+        else bb_launch((patch3x3_kernel<bf16, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
     } else {
-        if (adjoint) hipLaunchKernelGGL((patch3x3_kernel<float, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
-        else hipLaunchKernelGGL((patch3x3_kernel<float, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
+        if (adjoint) bb_launch((patch3x3_kernel<float, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
+        else bb_launch((patch3x3_kernel<float, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
     }
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -1820,11 +1820,11 @@ extern "C" int bb_subsample(int dtype, int adjoint, int n, int h, int w, int c, 
     const int ho = (h - 1) / stride + 1, wo = (w - 1) / stride + 1;
     dim3 grid(grid_for((int64_t)n * ho * wo * (c / vec)));
     if (dtype == BB_BF16) {
-        if (adjoint) hipLaunchKernelGGL((subsample_kernel<bf16, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
-        else hipLaunchKernelGGL((subsample_kernel<bf16, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
+        if (adjoint) bb_launch((subsample_kernel<bf16, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
+        else bb_launch((subsample_kernel<bf16, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const bf16*)src, (bf16*)dst);
     } else {
-        if (adjoint) hipLaunchKernelGGL((subsample_kernel<float, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
-        else hipLaunchKernelGGL((subsample_kernel<float, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
+        if (adjoint) bb_launch((subsample_kernel<float, true>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
+        else bb_launch((subsample_kernel<float, false>), grid, dim3(256), 0, st, n, h, w, c, stride, (const float*)src, (float*)dst);
     }
     BB_LAUNCH_CHECK();
     return BB_OK;

@@ -23,7 +23,7 @@ static int launch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     dim3 grid(g.tiles_m * g.tiles_n, 1, batches);
-    hipLaunchKernelGGL(kern, grid, dim3(WM * WN * 64), smem, st, g);
+    bb_launch(kern, grid, dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -52,7 +52,7 @@ static int launch_bf16_dma(GemmArgs& g, int batches, hipStream_t st) {
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     dim3 grid(g.tiles_m * g.tiles_n, 1, batches);
-    hipLaunchKernelGGL(kern, grid, dim3(WM * WN * 64), smem, st, g);
+    bb_launch(kern, grid, dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -69,7 +69,7 @@ template <int BM, int BN, int WM, int WN, bool TB> static int launch_bf16_dma_pe
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     const int total = g.tiles_m * g.tiles_n;
-    hipLaunchKernelGGL(kern, dim3(total < kPersistBlocks ? (total + 7) / 8 * 8 : kPersistBlocks), dim3(WM * WN * 64), smem, st, g);
+    bb_launch(kern, dim3(total < kPersistBlocks ? (total + 7) / 8 * 8 : kPersistBlocks), dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -81,7 +81,7 @@ static int launch_bf16_dma_stats(GemmArgs& g, hipStream_t st) {
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g);
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -93,7 +93,7 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g, bn);
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g, bn);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -240,10 +240,10 @@ template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hi
     if (pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) {
         g.tiles_n = (g.N + kF32SplitBN - 1) / kF32SplitBN;
         grid.x = g.tiles_m * g.tiles_n;
-        hipLaunchKernelGGL((gemm_f32_ksplit_kernel<TA, TB, kF32SplitGroups, kF32SplitBN>), grid, dim3(4 * kF32SplitBN * kF32SplitGroups), 0, st, g);
+        bb_launch((gemm_f32_ksplit_kernel<TA, TB, kF32SplitGroups, kF32SplitBN>), grid, dim3(4 * kF32SplitBN * kF32SplitGroups), 0, st, g);
     }
-    else if (tile == 64) hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, 64>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, 128>), grid, dim3(256), 0, st, g);
+    else if (tile == 64) bb_launch((gemm_f32_kernel<TA, TB, 64>), grid, dim3(256), 0, st, g);
+    else bb_launch((gemm_f32_kernel<TA, TB, 128>), grid, dim3(256), 0, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -424,7 +424,7 @@ static int launch_conv3x3(GemmArgs& g, const ConvArgs& cv, hipStream_t st) {
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g, cv);
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g, cv);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -518,7 +518,7 @@ extern "C" int bb_conv3x3_dgrad_bn(int dtype, int n, int h, int w, int cin, int 
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     const BnBwdArgs b = {bn->x, bn->mean, bn->rstd, bn->strips};
-    hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n), dim3(2 * 4 * 64), smem, (hipStream_t)stream, g, cv, b);
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n), dim3(2 * 4 * 64), smem, (hipStream_t)stream, g, cv, b);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -537,7 +537,7 @@ template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(Groupe
         blocks += g.tiles_m * g.tiles_n;
     }
     G.first_block[G.count] = blocks;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), smem, st, G);
+    bb_launch(kern, dim3(blocks), dim3(256), smem, st, G);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -581,9 +581,9 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
         }
         G.first_block[count] = blocks;
         const int layout = descs[0].layout;
-        if (layout == BB_NT) hipLaunchKernelGGL((gemm_f32_grouped_kernel<false, false, 64>), dim3(blocks), dim3(256), 0, st, G);
-        else if (layout == BB_NN) hipLaunchKernelGGL((gemm_f32_grouped_kernel<false, true, 64>), dim3(blocks), dim3(256), 0, st, G);
-        else hipLaunchKernelGGL((gemm_f32_grouped_kernel<true, true, 64>), dim3(blocks), dim3(256), 0, st, G);
+        if (layout == BB_NT) bb_launch((gemm_f32_grouped_kernel<false, false, 64>), dim3(blocks), dim3(256), 0, st, G);
+        else if (layout == BB_NN) bb_launch((gemm_f32_grouped_kernel<false, true, 64>), dim3(blocks), dim3(256), 0, st, G);
+        else bb_launch((gemm_f32_grouped_kernel<true, true, 64>), dim3(blocks), dim3(256), 0, st, G);
         BB_LAUNCH_CHECK();
         return BB_OK;
     }
@@ -732,7 +732,7 @@ extern "C" int bb_gemm_grouped_splitk(const bb_gemm_desc* descs, int count, void
         ws += (int64_t)splits * part;
     }
     const unsigned bx = (unsigned)((most + 255) / 256 > 1024 ? 1024 : (most + 255) / 256);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(bx, (unsigned)count), dim3(256), 0, (hipStream_t)stream, ra);
+    bb_launch(splitk_reduce_kernel, dim3(bx, (unsigned)count), dim3(256), 0, (hipStream_t)stream, ra);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }

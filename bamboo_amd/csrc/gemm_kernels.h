@@ -19,6 +19,7 @@ struct GemmArgs {
     float* strip_stats;  // [ceil(M / 32)][3][N]: per 32-row strip and output column (pivot, sum (c - pivot), sum (c - pivot)^2)
     DropKey drop;        // dropout on the product after bias and activation, before the residual (thresh 0: none)
 };
+template <> struct BbDropAt<GemmArgs> { static constexpr int32_t value = offsetof(GemmArgs, drop); };
 // Backward statistics of the batch normalisation whose (ReLU'd) output the product is the gradient of: the kernels
 // built with STATS = 2 leave, per 32-row strip and column, sum g and sum g * xhat of the stored (masked, bf16-rounded)
 // gradient g, with xhat = (x - mean) * rstd of the normalisation's input x ([M, N], rows ldc apart like C).

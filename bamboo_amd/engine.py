@@ -103,6 +103,9 @@ class PipelineEngine:
             raise PipelineError("use_graphs needs the engine built and run under a created stream "
                                 "(torch.cuda.stream(...)): the default stream cannot be captured")
         self._graphs = {}
+        # What every pass of (stage, micro-batch) launches is recorded when the pass is issued for the first time and
+        # replayed by one native call from then on (hip.Plan; see _issue): {(kind, stage, micro-batch): {operands: (plan, out)}}
+        self._plans = {}
         self.rc_stream = torch.cuda.Stream(self.device) if (rc_stream and self.r_stage_ids and eager_recovery) else None
         # When a redundant forward is issued (results never depend on it, only timing):
         #   "reference": where EagerRecoverySchedule puts it, in front of the own step that waits for a gradient
@@ -256,10 +259,17 @@ class PipelineEngine:
             # the stage in front of this one was lost and is now run by ITS predecessor
             # (reference engine.py:1266-1303): re-send what the lost stage had been given, then carry on
             fs, cs = self._prev_failover
-            self._generate_sched = lambda: schedule.PrevStageFailoverSchedule(
+            make = lambda: schedule.PrevStageFailoverSchedule(
                 self._train_sched(self.prev_stage), base(), failed_step=fs, curr_step=cs)
         else:
-            self._generate_sched = base
+            make = base
+        made = {}     # the instruction stream is the same in every batch until another generator is installed
+
+        def generate():
+            if self.micro_batches not in made:
+                made[self.micro_batches] = schedule.RecordedSchedule(make())
+            return made[self.micro_batches]
+        self._generate_sched = generate
 
     # ------------------------------------------------------------------ properties
     def is_first_stage(self):
@@ -414,6 +424,7 @@ class PipelineEngine:
     def _promote(self, absorbed, failed_step, curr_step):
         """Turn the shadow layers of ``absorbed`` into active layers of this process
         (reference engine.py:1190-1264)."""
+        self._plans.clear()    # contexts, and with them scratch buffers, may be replaced here
         if not self.eager_recovery:
             # lazy mode keeps CPU mirrors only: materialise the layers from them now
             self.module.build_layers(absorbed, self.param_buffers[absorbed])
@@ -452,13 +463,42 @@ class PipelineEngine:
         self._failover = (failed_step, curr_step)
         self._install_sched_generator()
 
-    # ------------------------------------------------------------------ graph replay
-    def _graphed(self, key, stream, issue):
-        """Run ``issue()`` (which only launches kernels of this library on ``stream`` and returns a
-        value that does not change between batches): eagerly the first time ``key`` occurs, captured
-        and launched the second time, replayed from then on."""
-        if not self.use_graphs or self.ctx.gemm_hook is not None:
+    # ------------------------------------------------------------------ replay
+    PLAN_VARIANTS = 4     # operand sets remembered per (kind, stage, micro-batch): a queue that hands out other buffers
+    #                       in every batch costs a recording each time, not memory
+
+    def _issue(self, slot, operands, ctx, issue):
+        """Run ``issue()``, which only launches kernels of this library on ``ctx.stream`` and returns a value that does not
+        change between batches, or replay what it launched.  ``slot`` = (kind, stage, micro-batch), ``operands``: what
+        identifies the buffers behind the recorded pointers.  A pass has 8 to 20 launches per layer, at about 10 us of host
+        time each through the layer code and 2 us from the recorded plan: stages of small layers are bound by that
+        (one layer of 128 columns, 4 micro-batches: 1.09 ms a batch issued from here, see _work of a pass in plan.hip)."""
+        if ctx.gemm_hook is not None:
             return issue()
+        if self.use_graphs:
+            return self._graphed((slot, operands), ctx.stream, issue)
+        plans = self._plans.get(slot)
+        if plans is None:
+            plans = self._plans[slot] = {}
+        known = plans.get(operands)
+        if known is not None:
+            known[0].launch(self.global_steps, ctx.stream)
+            return known[1]
+        ctx.dropout_keys = {}
+        try:
+            with hip.Plan.record() as plan:
+                out = issue()
+            plan.dropout(ctx.dropout_keys)
+        finally:
+            ctx.dropout_keys = None
+        while len(plans) >= self.PLAN_VARIANTS:
+            del plans[next(iter(plans))]
+        plans[operands] = (plan, out)
+        return out
+
+    def _graphed(self, key, stream, issue):
+        """:meth:`_issue` with HIP graphs: eagerly the first time ``key`` occurs, captured and launched the second time,
+        replayed from then on."""
         state = self._graphs.get(key)
         if state is None:
             self._graphs[key] = "seen"
@@ -555,15 +595,18 @@ class PipelineEngine:
         if redundant and self.rc_stream is not None:
             self.rc_stream.wait_event(self._fwd_done[buffer_id])
         kl = ctx.key_len
-        key = ("F", stage_id, buffer_id, id(ctx), inputs.data_ptr(), None if kl is None else kl.data_ptr())
+        operands = (id(ctx), inputs.data_ptr(), None if kl is None else kl.data_ptr(), redundant)
         # a redundant forward's stash is read by a backward pass only after a failover: it leaves out
         # what that backward pass can produce itself
         self._deferred[(stage_id, buffer_id)] = redundant
         note_rc = getattr(self.queue, "note_rc", None) if redundant else None
         if note_rc is not None:      # a queue that keeps a timeline of the redundant work (measurement only)
             note_rc(buffer_id, 0, "begin", ctx.stream)
-        out = self._graphed(key, ctx.stream, lambda: self.module.forward(inputs, stage_id, slot=buffer_id, ctx=ctx,
-                                                                         defer=redundant))
+        before = self.module.micro_offset
+        out = self._issue(("F", stage_id, buffer_id), operands, ctx,
+                          lambda: self.module.forward(inputs, stage_id, slot=buffer_id, ctx=ctx, defer=redundant))
+        if self.module.micro_offset == before:
+            self.module.note_replay(stage_id, buffer_id, inputs)
         if note_rc is not None:
             note_rc(buffer_id, len(self.module.func_buckets[stage_id]), "end", ctx.stream)
         self.pipe_buffers[out_key][buffer_id] = out
@@ -634,7 +677,11 @@ class PipelineEngine:
             note_rc = getattr(self.queue, "note_rc", None)
             if note_rc is not None:
                 note_rc(k, i, "begin", self.rc_stream)
-            out = self.module.forward(x, nxt, slot=k, ctx=ctx, defer=True, layers=(i, i + 1))
+            kl, before = ctx.key_len, self.module.micro_offset
+            out = self._issue((f"F{i}", nxt, k), (id(ctx), x.data_ptr(), None if kl is None else kl.data_ptr(), True), ctx,
+                              lambda: self.module.forward(x, nxt, slot=k, ctx=ctx, defer=True, layers=(i, i + 1)))
+            if i == 0 and self.module.micro_offset == before:
+                self.module.note_replay(nxt, k, x)
             if note_rc is not None:
                 note_rc(k, i + 1, "end", self.rc_stream)
             if i + 1 == n_layers:
@@ -700,10 +747,10 @@ class PipelineEngine:
         dst = self._input_grad_store[stage_id][buffer_id]
         kl = self.ctx.key_len
         deferred = self._deferred.get((stage_id, buffer_id), False)
-        key = ("B", stage_id, buffer_id, id(self.ctx), grad.data_ptr(), dst.data_ptr(),
-               None if kl is None else kl.data_ptr(), deferred)
-        self._graphed(key, self.ctx.stream, lambda: self.module.backward(grad, dst, stage_id, slot=buffer_id, ctx=self.ctx,
-                                                                         deferred=deferred))
+        operands = (id(self.ctx), grad.data_ptr(), dst.data_ptr(), None if kl is None else kl.data_ptr(), deferred,
+                    self.module.input_ptr(stage_id, buffer_id))
+        self._issue(("B", stage_id, buffer_id), operands, self.ctx,
+                    lambda: self.module.backward(grad, dst, stage_id, slot=buffer_id, ctx=self.ctx, deferred=deferred))
         key = f"input_grad_{stage_id}"
         if key in self.pipe_buffers:
             self.pipe_buffers[key][buffer_id] = dst

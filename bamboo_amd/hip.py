@@ -26,6 +26,7 @@ EXPORTS = (
     "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
     "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
     "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
+    "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_launches", "bb_plan_launch", "bb_plan_destroy",
     "bb_adam_multi", "bb_adam_multi_scaled", "bb_grad_clip_workspace", "bb_grad_clip_coef", "bb_cast", "bb_fill_f32",
 )
 
@@ -111,6 +112,11 @@ def lib():
     L.bb_graph_end.argtypes = [c_void_p, POINTER(c_void_p)]
     L.bb_graph_launch.argtypes = [c_void_p, c_void_p]
     L.bb_graph_destroy.argtypes = [c_void_p]
+    L.bb_plan_end.argtypes = [POINTER(c_void_p)]
+    L.bb_plan_dropout.argtypes = [c_void_p, c_int, POINTER(c_uint32), POINTER(c_uint32)] + [POINTER(c_int64)] * 4
+    L.bb_plan_launches.argtypes = [c_void_p]
+    L.bb_plan_launch.argtypes = [c_void_p, c_int64, c_void_p]
+    L.bb_plan_destroy.argtypes = [c_void_p]
     L.bb_act_fwd.argtypes = [c_int, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]
     L.bb_bn_workspace.argtypes = [c_int]
     L.bb_bn_workspace.restype = c_int64
@@ -574,6 +580,55 @@ class Graph:
         try:
             if self.exec:
                 lib().bb_graph_destroy(self.exec)
+        except Exception:
+            pass
+
+
+class Plan:
+    """The launches one call makes, recorded while it makes them and issued again by one call (``with Plan.record() as
+    plan: ...``, then ``plan.launch(step, stream)``).  ``plan.dropout(keys)`` names the dropout keys among the recorded
+    arguments: ``{(k0, k1): (base_seed, micro_batch, layer, site)}``; a launch derives them anew for its ``step``."""
+
+    def __init__(self):
+        self._plan = None
+
+    class _Recording:
+        def __init__(self, plan):
+            self.plan = plan
+
+        def __enter__(self):
+            check(lib().bb_plan_begin(), "bb_plan_begin")
+            return self.plan
+
+        def __exit__(self, exc_type, exc, tb):
+            if exc_type is not None:
+                lib().bb_plan_abort()
+                return False
+            out = c_void_p()
+            check(lib().bb_plan_end(byref(out)), "bb_plan_end")
+            self.plan._plan = out
+            return False
+
+    @classmethod
+    def record(cls):
+        return cls._Recording(cls())
+
+    def dropout(self, keys):
+        n = len(keys)
+        ids = [(c_int64 * n)(*column) for column in zip(*keys.values())] if n else [None] * 4
+        k0, k1 = (c_uint32 * n)(*[k[0] for k in keys]), (c_uint32 * n)(*[k[1] for k in keys])
+        check(lib().bb_plan_dropout(self._plan, n, k0, k1, *ids), "bb_plan_dropout")
+
+    def launch(self, step, stream):
+        check(lib().bb_plan_launch(self._plan, step, stream_ptr(stream)), "bb_plan_launch")
+
+    def __len__(self):
+        return int(lib().bb_plan_launches(self._plan))
+
+    def __del__(self):
+        try:
+            if self._plan:
+                lib().bb_plan_destroy(self._plan)
         except Exception:
             pass
 

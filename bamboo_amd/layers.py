@@ -36,6 +36,8 @@ class StageContext:
         # (base seed, batch counter, micro-batch): with a layer's index and the site inside it this names a dropout
         # mask; set per forward / backward call by whoever drives the stage
         self.dropout_base = None
+        # set while the launches of a call are recorded: {key: what it was made of}, see hip.Plan
+        self.dropout_keys = None
         self.redundant = False   # set per forward call: a redundant forward must not touch running statistics
         # set per forward call: leave out what only a backward pass reads (a redundant forward's stash is used
         # by a backward pass only after a failover); ``deferred`` tells that backward pass to produce it first
@@ -232,7 +234,11 @@ class TransformerLayer:
         if ctx.dropout_base is None or self.layer_idx is None:
             raise hip.HipKernelError("a layer with dropout needs ctx.dropout_base = (base seed, batch counter, micro-batch) "
                                      "and its layer index")
-        return self.dropout, hip.dropout_key(*ctx.dropout_base, self.layer_idx, site)
+        key = hip.dropout_key(*ctx.dropout_base, self.layer_idx, site)
+        if ctx.dropout_keys is not None:
+            base_seed, _, micro_batch = ctx.dropout_base
+            ctx.dropout_keys[key] = (base_seed, micro_batch, self.layer_idx, site)
+        return self.dropout, key
 
     def workspace_elems(self):
         n = max(self.hidden * 3, self.ffn)

@@ -556,6 +556,17 @@ class PipelineModule:
         hip.cast(x, kept[-1], stream=ctx.stream)
         return kept[-1]
 
+    def note_replay(self, stage_id, slot, forward_input):
+        """What :meth:`forward` keeps beside its launches, for a forward whose launches were replayed."""
+        self.micro_offset += 1
+        if self.activation_checkpoint_interval == 0:     # else the first group's kept input is a buffer of its own
+            self._stash[stage_id][slot][0]["x0"] = forward_input
+
+    def input_ptr(self, stage_id, slot):
+        """Address of the input the backward pass of ``slot`` will read (0: a buffer of the stash itself)."""
+        x = self._stash[stage_id][slot][0].get("x0") if self.activation_checkpoint_interval == 0 else None
+        return 0 if x is None else x.data_ptr()
+
     def backward(self, grad_output, grad_input, stage_id, slot=0, ctx=None, deferred=False):
         """Back-propagate through the layers of ``stage_id`` from the stash of ``slot``; parameter
         gradients accumulate in the stage's fp32 gradient arena, the input gradient is written to

@@ -177,6 +177,22 @@ class PipeSchedule(ABC):
         return next(self.it)
 
 
+class RecordedSchedule:
+    """The steps of a schedule, generated once and iterated in every batch."""
+
+    def __init__(self, pipe_schedule):
+        self._steps = [list(cmds) for cmds in pipe_schedule]
+        self._num_pipe_buffers = pipe_schedule.num_pipe_buffers()
+
+    def steps(self):
+        return iter(self._steps)
+
+    __iter__ = steps
+
+    def num_pipe_buffers(self):
+        return self._num_pipe_buffers
+
+
 class TrainSchedule(PipeSchedule):
     """1F1B training schedule of a stage; buffer id equals micro-batch id (M buffers)."""
 

@@ -401,6 +401,24 @@ int bb_graph_end(void* stream, void** exec_out);
 int bb_graph_launch(void* exec, void* stream);
 int bb_graph_destroy(void* exec);
 
+/* Launch plans: a fixed sequence of this library's launches issued again without its callers.
+ *   bb_plan_begin    the calling thread's launches run as always and are also recorded, until
+ *   bb_plan_end      returns the plan in *plan_out; bb_plan_abort drops what was recorded.
+ *   bb_plan_dropout  names the dropout keys inside the plan: launches recorded with the key (k0[i], k1[i]) get, on
+ *                    every replay, the key of (base_seed[i], step, micro_batch[i], layer[i], site[i]); fails if the plan
+ *                    holds a key that is not listed.
+ *   bb_plan_launch   issues the recorded launches in order on `stream`; `step` enters the dropout keys.
+ * The recorded arguments are device pointers and sizes: the buffers must still be there and unchanged in layout.
+ * A plan may be launched by one thread at a time. */
+int bb_plan_begin(void);
+int bb_plan_end(void** plan_out);
+int bb_plan_abort(void);
+int bb_plan_dropout(void* plan, int count, const uint32_t* k0, const uint32_t* k1, const int64_t* base_seed,
+                    const int64_t* micro_batch, const int64_t* layer, const int64_t* site);
+int bb_plan_launches(void* plan);
+int bb_plan_launch(void* plan, int64_t step, void* stream);
+int bb_plan_destroy(void* plan);
+
 #ifdef __cplusplus
 }
 #endif
