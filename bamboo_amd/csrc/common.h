@@ -91,11 +91,12 @@ template <> struct Elem<bf16> {
 
 // 16-byte vector load/store of VEC elements <-> float registers
 // One element's share of the backward sums of a batch normalisation (sum g, sum g * xhat with xhat = (x - mean) * rstd),
-// in explicitly rounded steps: whichever kernel adds the sums up -- the epilogue of the GEMM that writes g, or the
-// stand-alone pass -- the compiler contracts nothing, and with the same order of additions the bits are the same.
+// with every rounding written out (one multiply-add for the second sum, nothing left for the compiler to contract):
+// whichever kernel adds the sums up -- the epilogue of the GEMM that writes g, or the stand-alone pass -- with the same
+// order of additions the bits are the same.
 __device__ __forceinline__ void bn_bwd_sums_add(float g, float x, float mu, float rs, float& sg, float& sgx) {
-    sg = __fadd_rn(sg, g);
-    sgx = __fadd_rn(sgx, __fmul_rn(__fmul_rn(g, __fsub_rn(x, mu)), rs));
+    sg = sg + g;
+    sgx = __builtin_fmaf(g * (x - mu), rs, sgx);
 }
 __device__ __forceinline__ void load_vec(const float* p, float (&v)[4]) {
     f32x4 t = *(const f32x4*)p;

@@ -4,21 +4,18 @@
 // Stands in for F.linear / torch.matmul and their autograd backward in the reference layer
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:121,127,136-146,158).
 //
-// bf16 data path.  Both operand tiles are kept in LDS "k-contiguous": tile row r (an m- or
-// n-index) owns 64 consecutive k values = 8 chunks of 16 bytes, chunk c stored at chunk slot
-// c ^ swz(r) so that the 16-byte fragment reads of 16 consecutive rows hit distinct banks.
-// An operand whose memory layout is k-major (the transposed operand of NN / TN) is loaded as
-// 16-byte vectors along its contiguous dimension and transposed in registers before the LDS
-// store, so the MFMA side never changes.
+// bf16 data paths: tiles by DMA (gemm_bf16_dma_*), 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for
+// problems of few tiles, and a register-staged kernel for rows of C that are no whole vectors.
 #include "gemm_kernels.h"
+#include "gemm_wave.h"
 
 // =========================================================================================
 // host dispatch
 // =========================================================================================
-template <int BM, int BN, int WM, int WN, bool TA, bool TB>
+template <int BM, int BN, int WM, int WN>
 static int launch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     constexpr int smem = 2 * (BM + BN) * 64 * 2;
-    auto kern = gemm_bf16_kernel<BM, BN, WM, WN, TA, TB>;
+    auto kern = gemm_bf16_kernel<BM, BN, WM, WN>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -26,19 +23,6 @@ static int launch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     bb_launch(kern, grid, dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
-}
-
-// Tile choice: the largest tile that still gives every CU work; small problems (attention
-// heads: 64-wide operands) take the 128x64 / 64x128 tiles.
-enum Bf16Tile { T128x64 = 0, T64x128, T256x256, T256x128, T128x128 };
-static const char* const kBf16TileNames[] = {"128x64", "64x128", "256x256", "256x128", "128x128"};
-
-static Bf16Tile pick_bf16_tile(int M, int N, int64_t batches) {
-    const int64_t t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches;
-    if (N <= 64) return T128x64;
-    if (M <= 64) return T64x128;
-    if (M >= 256 && N >= 128 && t2128 >= 200) return T256x128;
-    return T128x128;
 }
 
 template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES = 4, int BK = 32>
@@ -74,10 +58,10 @@ template <int BM, int BN, int WM, int WN, bool TB> static int launch_bf16_dma_pe
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, int STAGES = 3>
 static int launch_bf16_dma_stats(GemmArgs& g, hipStream_t st) {
-    constexpr int smem = 3 * (BM + BN) * 64 * 2;
-    auto kern = gemm_bf16_dma_stats_kernel<BM, BN, WM, WN>;
+    constexpr int smem = STAGES * (BM + BN) * 64 * 2;
+    auto kern = gemm_bf16_dma_stats_kernel<BM, BN, WM, WN, STAGES>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -86,10 +70,10 @@ static int launch_bf16_dma_stats(GemmArgs& g, hipStream_t st) {
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, int STAGES = 3>
 static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t st) {
-    constexpr int smem = 3 * (BM + BN) * 64 * 2;
-    auto kern = gemm_bf16_dma_bnbwd_kernel<BM, BN, WM, WN>;
+    constexpr int smem = STAGES * (BM + BN) * 64 * 2;
+    auto kern = gemm_bf16_dma_bnbwd_kernel<BM, BN, WM, WN, STAGES>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -100,15 +84,22 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
 
 // DMA kernels need K % 32 == 0 and at least one full vector of rows; tile by problem size
 enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, D256x128k64s3, D128x128k64, D128x64k64s3, D128x64s3,
-               D64x128k64s3, D64x128s3, D256x192k64, D256x256p };
+               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4 };
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
-                                            "dma256x192k64", "dma256x256p"};
+                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4"};
 // The tile of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
 // what ran before), and every kernel adds up a contraction in the same order: a redundant forward and a normal forward
 // of the same layer give the same bits.
 static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
-    if (K % 32 != 0 || K < 64 || M < 128 || N < 128 || N % 8 != 0) return D_NONE;
+    //  - Problems of at most one 64x64 tile per CU take those, four stages deep: what such a launch waits for is the chain of
+    //    its k-tiles and its epilogue, and the more CUs share the loads the shorter both are.  128x64 / 64x64 tiles (us, back
+    //    to back): NT 256x512x512 6.8 / 6.3, 1050x512x2048 15.8 / 12.7, 3136x256x1024 10.5 / 9.0; NN 1050x512x1536 12.0 / 9.7;
+    //    eight stages 5 % slower (a second block finds no room), 408 tiles equal, more tiles slower.  The shapes the larger
+    //    tiles do not take (fewer than 128 rows or columns) run on it too.
+    const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches;
+    if (layout != BB_TN && K % 64 == 0 && K > 0 && N % 8 == 0 && (t64 <= 256 || M < 128 || N < 128)) return D64x64k64s4;
+    if ((K % 32 != 0 && layout != BB_TN) || K < 64 || M < 128 || N < 128 || N % 8 != 0) return D_NONE;
     // Rules read off sweeps of M 2048..16384 x N 768..6400 x K 1024/4096 (NT and NN) on MI355X (256 CUs,
     // one block of the 256-row tiles per CU).
     //  - Operands whose rows are k-contiguous (both of NT, A of NN) load faster as 64-wide k-tiles: one
@@ -187,8 +178,40 @@ static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layou
     return t;
 }
 
+// The wave-sliced kernels (gemm_wave.h) take the weight gradients whose 64x64 tiles are at most one per CU, and whatever the
+// DMA kernels do not take (contractions of odd lengths).  W_8: eight waves, 32-wide slices, two stages each (130 KB of LDS);
+// W_4: four waves, 64-wide slices, one stage (65 KB, two blocks a CU).  Measured back to back, 128x128 DMA tiles / W_8 (us):
+// TN 512x512x4096 55.7 / 18.8, 256x256x6272 80.8 / 21.9; register-staged kernel / W_8: NT 200x264x72 31.4 / 5.2.
+enum WaveMode { W_NONE = 0, W_8, W_4 };
+static WaveMode pick_wave(int M, int N, int K, int64_t batches, int layout, DmaTile dma) {
+    if (N % 8 != 0) return W_NONE;
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches;
+    if (dma != D_NONE && (tiles > 256 || layout != BB_TN)) return W_NONE;
+    return tiles <= 256 ? W_8 : W_4;
+}
+template <bool TA, bool TB, int KW, int BK, int NST> static int launch_bf16_wave(GemmArgs& g, int batches, hipStream_t st) {
+    auto kern = gemm_bf16_wave_kernel<TA, TB, KW, BK, NST, false>;
+    if constexpr (!TA && !TB) {
+        if (g.drop.thresh) kern = gemm_bf16_wave_kernel<TA, TB, KW, BK, NST, true>;
+    }
+    constexpr int smem = wave_gemm_lds(KW, BK, NST);
+    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
+    g.tiles_m = (g.M + 63) / 64;
+    g.tiles_n = (g.N + 63) / 64;
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(KW * 64), smem, st, g);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
+
 template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, hipStream_t st) {
-    switch (pick_dma_tile_for(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT, g.epilogue)) {
+    const int layout = TA ? BB_TN : TB ? BB_NN : BB_NT;
+    const DmaTile dma = pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.epilogue);
+    switch (pick_wave(g.M, g.N, g.K, batches, layout, dma)) {
+        case W_8: return launch_bf16_wave<TA, TB, 8, 32, 2>(g, batches, st);
+        case W_4: return launch_bf16_wave<TA, TB, 4, 64, 1>(g, batches, st);
+        default: break;
+    }
+    switch (dma) {
         case D256x256w8db: return launch_bf16_dma<256, 256, 2, 4, TA, TB, true>(g, batches, st);
         case D256x128w8db: return launch_bf16_dma<256, 128, 4, 2, TA, TB, true>(g, batches, st);
         case D128x128s3: return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
@@ -199,6 +222,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D128x64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3>(g, batches, st);
         case D64x128k64s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
         case D64x128s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
+        case D64x64k64s4:
+            if constexpr (!TA) return launch_bf16_dma<64, 64, 2, 2, TA, TB, true, 4, 64>(g, batches, st);
+            else break;
         case D256x256p:
             if constexpr (!TA) return launch_bf16_dma_persist<256, 256, 2, 4, TB>(g, st);
             else break;
@@ -208,12 +234,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
             else break;
         default: break;
     }
-    switch (pick_bf16_tile(g.M, g.N, batches)) {
-        case T128x64: return launch_bf16<128, 64, 4, 1, TA, TB>(g, batches, st);
-        case T64x128: return launch_bf16<64, 128, 1, 4, TA, TB>(g, batches, st);
-        case T256x128: return launch_bf16<256, 128, 4, 2, TA, TB>(g, batches, st);
-        default: return launch_bf16<128, 128, 2, 2, TA, TB>(g, batches, st);
-    }
+    if constexpr (!TA && !TB) return launch_bf16<128, 128, 2, 2>(g, batches, st);
+    bb_set_error("bb_gemm: no kernel for this problem");   // N % 8 == 0 is checked for the other layouts
+    return BB_EINVAL;
 }
 
 static int pick_f32_tile(int M, int N, int64_t batches) {
@@ -255,8 +278,10 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
     const int64_t batches = (int64_t)(d->nb1 > 0 ? d->nb1 : 1) * (d->nb2 > 0 ? d->nb2 : 1);
     if (d->dtype == BB_BF16) {
         const DmaTile dt = pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->epilogue);
-        snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
-                 dt != D_NONE ? kDmaTileNames[dt] : kBf16TileNames[pick_bf16_tile(d->M, d->N, batches)]);
+        const WaveMode wm = pick_wave(d->M, d->N, d->K, batches, d->layout, dt);
+        if (wm != W_NONE) snprintf(out, out_len, "bf16_%s_wave64x64k%d", layouts[d->layout], wm == W_8 ? 8 : 4);
+        else snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
+                 dt != D_NONE ? kDmaTileNames[dt] : "128x128");
     }
     else
     {
@@ -293,12 +318,11 @@ static int fill_args(const bb_gemm_desc* d, GemmArgs& g, int64_t& batches, bool&
     if (conv) {
         // B = patch matrix of an NHWC tensor, gathered by the grouped DMA kernel's loader
         BB_REQUIRE(d->layout == BB_TN && d->dtype == BB_BF16 && batches == 1, "bb_gemm: a patch-matrix B needs BB_TN, bf16, no batching");
-        BB_REQUIRE(d->conv_c > 0 && d->conv_c % 128 == 0 && d->conv_h > 0 && d->conv_w > 0 && d->conv_row0 >= 0,
-                   "bb_gemm: patch-matrix B: conv_c (%d) must be a positive multiple of 128, conv_h/conv_w positive", d->conv_c);
+        BB_REQUIRE(d->conv_c > 0 && d->conv_c % 64 == 0 && d->conv_h > 0 && d->conv_w > 0 && d->conv_row0 >= 0,
+                   "bb_gemm: patch-matrix B: conv_c (%d) must be a positive multiple of 64 (128x128 tiles take a multiple of 128), conv_h/conv_w positive", d->conv_c);
         BB_REQUIRE(d->N == 9 * d->conv_c, "bb_gemm: patch-matrix B: N (%d) must be 9 * conv_c (%d)", d->N, d->conv_c);
-        BB_REQUIRE(d->K % 32 == 0 && d->K >= 64 && d->M >= 128 && 32 / d->conv_w + 1 <= d->conv_h,
-                   "bb_gemm: patch-matrix B: K (%d) must be a multiple of 32 and >= 64, M (%d) >= 128, and 32 pixels must "
-                   "not span more than one image boundary (%d x %d)", d->K, d->M, d->conv_h, d->conv_w);
+        BB_REQUIRE(32 / d->conv_w + 1 <= d->conv_h,
+                   "bb_gemm: patch-matrix B: 32 pixels must not span more than one image boundary (%d x %d)", d->conv_h, d->conv_w);
         BB_REQUIRE(!d->bias && d->epilogue == BB_EPI_NONE, "bb_gemm: patch-matrix B takes no bias / epilogue");
     }
     // the contiguous dimension of every operand is read in 16-byte vectors
@@ -330,10 +354,12 @@ static int fill_args(const bb_gemm_desc* d, GemmArgs& g, int64_t& batches, bool&
     return BB_OK;
 }
 
-// The bias-gradient column sums ride inside the DMA kernel when it runs the problem; otherwise
+// The bias-gradient column sums ride inside the DMA and the wave-sliced kernels when they run the problem; otherwise
 // the stand-alone reduction computes them.
 static bool colsum_fusable(const bb_gemm_desc* d, int64_t batches) {
-    return d->colsum_out && d->dtype == BB_BF16 && batches == 1 && pick_dma_tile(d->M, d->N, d->K, 1, d->layout) != D_NONE;
+    if (!d->colsum_out || d->dtype != BB_BF16 || batches != 1) return false;
+    const DmaTile dma = pick_dma_tile(d->M, d->N, d->K, 1, d->layout);
+    return dma != D_NONE || pick_wave(d->M, d->N, d->K, 1, d->layout, dma) != W_NONE;
 }
 static int colsum_standalone(const bb_gemm_desc* d, void* stream) {
     BB_REQUIRE(d->colsum_ws, "bb_gemm: colsum_out on this problem needs colsum_ws");
@@ -375,8 +401,10 @@ extern "C" int bb_gemm_bn_bwd(const bb_gemm_desc* d, const bb_bn_bwd_stats* bn, 
     rc = fill_args(d, g, batches, ta, tb);
     if (rc) return rc;
     const BnBwdArgs b = {bn->x, bn->mean, bn->rstd, bn->strips};
-    // the tile the plain product of this shape would take, where it is one of the two built with the sums
-    if (pick_dma_tile(d->M, d->N, d->K, 1, BB_NN) == D256x128k64s3) return launch_bf16_dma_bnbwd<256, 128, 4, 2>(g, b, (hipStream_t)stream);
+    // the tile the plain product of this shape would take, where it is one of those built with the sums
+    const DmaTile dma = pick_dma_tile(d->M, d->N, d->K, 1, BB_NN);
+    if (dma == D64x64k64s4) return launch_bf16_dma_bnbwd<64, 64, 2, 2, 4>(g, b, (hipStream_t)stream);
+    if (dma == D256x128k64s3) return launch_bf16_dma_bnbwd<256, 128, 4, 2>(g, b, (hipStream_t)stream);
     return launch_bf16_dma_bnbwd<64, 128, 2, 2>(g, b, (hipStream_t)stream);
 }
 
@@ -392,8 +420,10 @@ extern "C" int bb_gemm(const bb_gemm_desc* d, void* stream) {
         int rc = fill_args(d, g, batches, ta, tb);
         if (rc) return rc;
         g.strip_stats = d->strip_stats;
-        // the two tiles that carry the statistics: 256x128 where the ordinary choice would be that tile, else 128x64
-        if (pick_dma_tile(d->M, d->N, d->K, 1, BB_NT) == D256x128k64s3) return launch_bf16_dma_stats<256, 128, 4, 2>(g, (hipStream_t)stream);
+        // the tiles that carry the statistics: 64x64 and 256x128 where the ordinary choice would be that tile, else 128x64
+        const DmaTile dma = pick_dma_tile(d->M, d->N, d->K, 1, BB_NT);
+        if (dma == D64x64k64s4) return launch_bf16_dma_stats<64, 64, 2, 2, 4>(g, (hipStream_t)stream);
+        if (dma == D256x128k64s3) return launch_bf16_dma_stats<256, 128, 4, 2>(g, (hipStream_t)stream);
         return launch_bf16_dma_stats<128, 64, 4, 1>(g, (hipStream_t)stream);
     }
     GemmArgs g;
@@ -429,6 +459,20 @@ static int launch_conv3x3(GemmArgs& g, const ConvArgs& cv, hipStream_t st) {
     return BB_OK;
 }
 
+template <int BM, int BN, int WM, int WN, int STAGES>
+static int launch_conv3x3_bnbwd(GemmArgs& g, const ConvArgs& cv, const BnBwdArgs& bn, hipStream_t st) {
+    constexpr int smem = STAGES * (BM + BN) * 64 * 2;
+    auto kern = conv3x3_bf16_igemm_bnbwd_kernel<BM, BN, WM, WN, STAGES>;
+    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
+    g.tiles_m = (g.M + BM - 1) / BM;
+    g.tiles_n = (g.N + BN - 1) / BN;
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n), dim3(WM * WN * 64), smem, st, g, cv, bn);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
+// one 64x64 tile per CU at most: as pick_dma_tile
+static bool conv_small_tiles(int M, int N) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 256; }
+
 extern "C" int bb_conv3x3_supported(int dtype, int mode, int n, int h, int w, int cin, int cout) {
     const int64_t rows = (int64_t)n * h * w;
     const int gathered = mode == BB_CONV_DGRAD ? cout : cin, produced = mode == BB_CONV_DGRAD ? cin : cout;
@@ -463,14 +507,17 @@ extern "C" int bb_conv3x3(int dtype, int mode, int n, int h, int w, int cin, int
     g.epilogue = BB_EPI_NONE;
     cv.h = h; cv.w = w; cv.c = dgrad ? cout : cin;
     hipStream_t st = (hipStream_t)stream;
+    const bool small = conv_small_tiles(g.M, g.N);
     if (!dgrad) {
         // B = the weight as it lies: [cout, 9 * cin], k-contiguous
         g.B = weight;
         g.ldb = 9 * (int64_t)cin;
         if (strip_stats) {
             g.strip_stats = strip_stats;
+            if (small) return launch_conv3x3<64, 64, 2, 2, false, 4, true>(g, cv, st);
             return launch_conv3x3<128, 64, 4, 2, false, 3, true>(g, cv, st);
         }
+        if (small) return launch_conv3x3<64, 64, 2, 2, false, 4>(g, cv, st);
         // eight waves on a 128x64 tile (32x32 per wave): with one block per CU, two waves per SIMD hide each other's
         // LDS and barrier waits (four waves: 21.6 us, eight: 19.4 us at 6272 pixels, 256 channels)
         return launch_conv3x3<128, 64, 4, 2, false, 3>(g, cv, st);
@@ -481,6 +528,7 @@ extern "C" int bb_conv3x3(int dtype, int mode, int n, int h, int w, int cin, int
     g.ldb = 9 * (int64_t)cin;
     cv.b_every = cout / 64;
     cv.b_wrap = -(int64_t)cout * g.ldb - cin;
+    if (small) return launch_conv3x3<64, 64, 2, 2, true, 4>(g, cv, st);
     return launch_conv3x3<64, 128, 2, 4, true, 3>(g, cv, st);
 }
 
@@ -512,15 +560,9 @@ extern "C" int bb_conv3x3_dgrad_bn(int dtype, int n, int h, int w, int cin, int 
     g.ldb = 9 * (int64_t)cin;
     cv.b_every = cout / 64;
     cv.b_wrap = -(int64_t)cout * g.ldb - cin;
-    constexpr int BM = 64, BN = 128, STAGES = 3, smem = STAGES * (BM + BN) * 64 * 2;
-    auto kern = conv3x3_bf16_igemm_bnbwd_kernel<BM, BN, 2, 4, STAGES>;
-    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
-    g.tiles_m = (g.M + BM - 1) / BM;
-    g.tiles_n = (g.N + BN - 1) / BN;
     const BnBwdArgs b = {bn->x, bn->mean, bn->rstd, bn->strips};
-    bb_launch(kern, dim3(g.tiles_m * g.tiles_n), dim3(2 * 4 * 64), smem, (hipStream_t)stream, g, cv, b);
-    BB_LAUNCH_CHECK();
-    return BB_OK;
+    if (conv_small_tiles(g.M, g.N)) return launch_conv3x3_bnbwd<64, 64, 2, 2, 4>(g, cv, b, (hipStream_t)stream);
+    return launch_conv3x3_bnbwd<64, 128, 2, 4, 3>(g, cv, b, (hipStream_t)stream);
 }
 
 template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(GroupedArgs& G, hipStream_t st) {
@@ -542,6 +584,29 @@ template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(Groupe
     return BB_OK;
 }
 
+// A layer's weight gradients with up to four 64x64 tiles per CU, i.e. at most one 128x128 tile: that one is a chain of
+// k-tiles nobody overlaps.  Eight waves a tile while there is one tile per CU, four (two blocks a CU) above.  128x128 tiles /
+// 64x64 tiles (us), rows x hidden (x 4 in the feed-forward): 300x256 12.1 / 7.3, 3378x192 61.6 / 16.9, 8000x192 132 / 31,
+// 1050x512 27.4 / 22.3, 3001x320 57.6 / 26.6; 2048x768 (1728 tiles) 48 / 56.
+constexpr int64_t kGroupedWaveTiles = 1024;
+template <int KW, int BK, int NST> static int launch_grouped_wave(GroupedArgs& G, bool conv, hipStream_t st) {
+    auto kern = conv ? gemm_bf16_wave_grouped_kernel<true, true, KW, BK, NST, true> : gemm_bf16_wave_grouped_kernel<true, true, KW, BK, NST>;
+    constexpr int smem = wave_gemm_lds(KW, BK, NST);
+    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
+    int blocks = 0;
+    for (int i = 0; i < G.count; ++i) {
+        GemmArgs& g = G.p[i];
+        g.tiles_m = (g.M + 63) / 64;
+        g.tiles_n = (g.N + 63) / 64;
+        G.first_block[i] = blocks;
+        blocks += g.tiles_m * g.tiles_n;
+    }
+    G.first_block[G.count] = blocks;
+    bb_launch(kern, dim3(blocks), dim3(KW * 64), smem, st, G);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
+
 extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream) {
     BB_REQUIRE(count >= 0 && (descs || count == 0), "bb_gemm_grouped: bad arguments");
     hipStream_t st = (hipStream_t)stream;
@@ -549,13 +614,19 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
     // kernel accepts; otherwise the problems run one after the other (same results)
     bool has_conv = false;
     for (int i = 0; i < count; ++i) has_conv = has_conv || descs[i].conv_c != 0;
-    bool fuse = count >= (has_conv ? 1 : 2) && count <= GROUP_MAX;
+    bool fuse = count >= (has_conv ? 1 : 2) && count <= GROUP_MAX, dma = true, wave = count > 0 && descs[0].layout == BB_TN;
+    int64_t tiles = 0;
     for (int i = 0; i < count && fuse; ++i) {
         const bb_gemm_desc& d = descs[i];
-        // the grouped kernel is built without dropout decisions in its epilogue: such a problem runs by itself
+        // the grouped kernels are built without dropout decisions in their epilogue: such a problem runs by itself
+        dma = dma && pick_dma_tile(d.M, d.N, d.K, 1, d.layout) != D_NONE && d.conv_c % 128 == 0;
+        wave = wave && pick_wave(d.M, d.N, d.K, 1, d.layout, D_NONE) != W_NONE;
         fuse = d.dtype == BB_BF16 && d.layout == descs[0].layout && d.nb1 <= 1 && d.nb2 <= 1 && d.M > 0 && d.N > 0 &&
-               d.dropout_p == 0.f && pick_dma_tile(d.M, d.N, d.K, 1, d.layout) != D_NONE;
+               d.dropout_p == 0.f && (dma || wave);
+        tiles += (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64);
     }
+    // weight gradients of few tiles: 64x64 tiles, the contraction dealt to the waves (see kGroupedWaveTiles)
+    wave = wave && (!dma || tiles <= (count > 1 ? kGroupedWaveTiles : 256));   // alone: as bb_gemm takes it
     // fp32: unbatched problems of one layout that all take the small tile (each alone would leave CUs idle) share a launch
     bool fuse32 = !fuse && !has_conv && count >= 2 && count <= GROUP_MAX;
     for (int i = 0; i < count && fuse32; ++i) {
@@ -587,9 +658,8 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
         BB_LAUNCH_CHECK();
         return BB_OK;
     }
-    // a patch-matrix B exists only inside the grouped kernel: no one-by-one route for it
-    BB_REQUIRE(fuse || !has_conv, "bb_gemm_grouped: a problem with a patch-matrix B must share a launch of bf16 BB_TN "
-                                  "problems the DMA kernel takes (M, N >= 128, K %% 32 == 0)");
+    // a patch-matrix B exists only inside the grouped kernels: no one-by-one route for it
+    BB_REQUIRE(fuse || !has_conv, "bb_gemm_grouped: a problem with a patch-matrix B must share a launch of unbatched bf16 BB_TN problems");
     if (!fuse) {
         for (int i = 0; i < count; ++i) {
             int rc = bb_gemm(&descs[i], stream);
@@ -604,9 +674,11 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
         bool ta, tb;
         int rc = fill_args(&descs[i], G.p[i], batches, ta, tb);
         if (rc) return rc;
-        if (descs[i].colsum_out) G.p[i].colsum = descs[i].colsum_out;  // every grouped problem runs the DMA kernel
+        if (descs[i].colsum_out) G.p[i].colsum = descs[i].colsum_out;  // both grouped kernels leave the sums
     }
     const int layout = descs[0].layout;
+    if (wave && tiles <= 256) return launch_grouped_wave<8, 32, 2>(G, has_conv, st);
+    if (wave) return launch_grouped_wave<4, 32, 2>(G, has_conv, st);
     if (layout == BB_NT) return launch_grouped<false, false>(G, st);
     if (layout == BB_NN) return launch_grouped<false, true>(G, st);
     if (has_conv) return launch_grouped<true, true, true>(G, st);
@@ -655,23 +727,34 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitkReduceAr
 // chunks of the contraction: 0 or 1 = run the group whole
 static int pick_splits(const bb_gemm_desc* descs, int count) {
     if (count < 1 || count > GROUP_MAX) return 0;
-    int64_t tiles = 0;
+    int64_t tiles = 0, tiles128 = 0;
     int kmin = 1 << 30;
     for (int i = 0; i < count; ++i) {
         const bb_gemm_desc& d = descs[i];
         if (d.dtype != BB_BF16 || d.c_dtype != BB_F32 || d.layout != descs[0].layout || d.nb1 > 1 || d.nb2 > 1 || d.M <= 0 ||
             d.N <= 0 || d.colsum_out || d.bias || d.epilogue != BB_EPI_NONE || d.alpha != 1.0f || d.N % 4 != 0 || d.dropout_p != 0.f ||
-            pick_dma_tile(d.M, d.N, d.K, 1, d.layout) == D_NONE)
+            (pick_dma_tile(d.M, d.N, d.K, 1, d.layout) == D_NONE && d.layout != BB_TN))
             return 0;
-        tiles += (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128);
+        tiles += (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64);
+        tiles128 += (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128);
         kmin = d.K < kmin ? d.K : kmin;
     }
-    // Two blocks per CU on average: with one, a CU's four waves have nobody to hide their load and barrier waits
-    // behind (the weight gradients of a ResNet block: 61.7 us at three chunks, 50.8 us at five).
-    int splits = (int)(256 * 2 / tiles);
+    // Few tiles: 64x64 ones with eight waves, and chunks while those leave half the CUs idle (at least 1024 rows a chunk, four
+    // slices a wave).  More tiles: whole on 64x64 tiles while the contraction is short, else chunks of 128x128 tiles for two
+    // blocks per CU -- with one, a CU's four waves have nobody to hide their load and barrier waits behind.  Weight gradients
+    // of a ResNet block, 128x128 tiles in their best split / this rule (us with the reduction), rows, middle channels: 12544,
+    // 128 52 / 23; 12544, 64 (patch matrix) / 17; 900, 128 14.6 / 8.7; 3136, 256 28.8 / 25.9; 648, 256 19.8 / 11.0;
+    // 6272, 256 40 on five chunks of 128x128 tiles, 44 whole.
+    int splits, least = 1024;
+    if (tiles <= 256) splits = tiles > 128 ? 1 : (int)(384 / tiles);
+    else if (tiles <= kGroupedWaveTiles && kmin <= 4096) return 1;
+    else {
+        splits = (int)(256 * 2 / tiles128);
+        least = 512;
+    }
     if (splits > SPLITK_MAX) splits = SPLITK_MAX;
     if (splits > GROUP_MAX / count) splits = GROUP_MAX / count;
-    while (splits > 1 && kmin / splits < 512) --splits;  // keep the pipelines of the chunks long
+    while (splits > 1 && kmin / splits < least) --splits;
     return splits;
 }
 

@@ -115,10 +115,12 @@ __device__ __forceinline__ void unpack_bf16x8(const u32x4& t, float (&v)[8]) {
 }
 // PRE: `pre` holds the 16 bytes of epilogue_operand(g) at xi (fetched earlier); PRE2: `pre2` those of g.resid at xi where
 // BB_EPI_MUL_POS has one
-template <bool DROP, bool PRE = false, bool PRE2 = false>
+// PREC: `c_lo`, `c_hi` hold the fp32 C at ci (accumulating problems)
+template <bool DROP, bool PRE = false, bool PRE2 = false, bool PREC = false>
 __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, int64_t xi, int m, int n, float (&v)[8],
                                                  const float (&b)[8], const u32x4& pre = u32x4{0u, 0u, 0u, 0u},
-                                                 const u32x4& pre2 = u32x4{0u, 0u, 0u, 0u}) {
+                                                 const u32x4& pre2 = u32x4{0u, 0u, 0u, 0u}, const f32x4& c_lo = f32x4{0.f, 0.f, 0.f, 0.f},
+                                                 const f32x4& c_hi = f32x4{0.f, 0.f, 0.f, 0.f}) {
     if (g.bias) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += b[e];
@@ -221,8 +223,8 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
         float* c = (float*)g.C + ci;
         f32x4 lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
         if (g.accumulate) {
-            lo += *(const f32x4*)c;
-            hi += *(const f32x4*)(c + 4);
+            lo += PREC ? c_lo : *(const f32x4*)c;
+            hi += PREC ? c_hi : *(const f32x4*)(c + 4);
         }
         *(f32x4*)c = lo;
         *(f32x4*)(c + 4) = hi;
@@ -248,11 +250,8 @@ __device__ __forceinline__ int swz(int row) {
     return ((row >> 1) & 7) ^ ((row & 1) << 2) ^ ((row >> 4) & 7);
 }
 
-// Loader of one operand tile: R tile rows (m or n index) x 64 k.  TR = operand memory is
-// k-major ([K, rows], rows contiguous).
-template <int R, int NT, bool TR> struct TileLoader;
-
-template <int R, int NT> struct TileLoader<R, NT, false> {
+// Loader of one operand tile: R tile rows (m or n index) x 64 k.
+template <int R, int NT> struct TileLoader {
     static constexpr int NCH = R * 8 / NT;  // 16-byte chunks per thread
     static_assert(NCH >= 1, "tile too small for the block");
     u32x4 regs[NCH];
@@ -278,52 +277,8 @@ template <int R, int NT> struct TileLoader<R, NT, false> {
     }
 };
 
-template <int R, int NT> struct TileLoader<R, NT, true> {
-    // each thread owns an 8-row x KB-k block: KB 16-byte loads, each 8 rows at one k
-    static constexpr int KB = 8 * R / NT;
-    static_assert(KB == 2 || KB == 4 || KB == 8, "unsupported tile/block combination");
-    static constexpr int NRB = R / 8;
-    u32x4 regs[KB];
-    __device__ __forceinline__ void gload(const bf16* base, int64_t ld, int row0, int rows, int k0,
-                                          int K, int tid) {
-        const int rb = tid % NRB, kb = tid / NRB;
-        const int gr = row0 + rb * 8;
-#pragma unroll
-        for (int j = 0; j < KB; ++j) {
-            const int gk = k0 + kb * KB + j;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (gr < rows && gk < K) v = *(const u32x4*)(base + (int64_t)gk * ld + gr);
-            regs[j] = v;
-        }
-    }
-    __device__ __forceinline__ void sstore(bf16* lds, int tid) const {
-        const int rb = tid % NRB, kb = tid / NRB;
-        const int ko = kb * KB;  // k offset inside the 64-wide tile
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            // row i of the block: element i of every loaded vector
-            uint32_t w[KB / 2];
-#pragma unroll
-            for (int j = 0; j < KB / 2; ++j) {
-                const uint32_t lo = regs[2 * j][i >> 1], hi = regs[2 * j + 1][i >> 1];
-                w[j] = (i & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-            }
-            const int r = rb * 8 + i;
-            bf16* dst = lds + r * 64 + ((((ko >> 3) ^ swz(r))) << 3) + (ko & 7);
-            if constexpr (KB == 8) {
-                u32x4 t = {w[0], w[1], w[2], w[3]};
-                *(u32x4*)dst = t;
-            } else if constexpr (KB == 4) {
-                u32x2 t = {w[0], w[1]};
-                *(u32x2*)dst = t;
-            } else {
-                *(uint32_t*)dst = w[0];
-            }
-        }
-    }
-};
-
-template <int BM, int BN, int WM, int WN, bool TA, bool TB>
+// NT products whose N is no multiple of 8 (rows of C that are no whole 16-byte vectors): register-staged tiles, scalar epilogue
+template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const GemmArgs g) {
     constexpr int NT = WM * WN * 64, BK = 64;
     constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
@@ -342,8 +297,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const GemmArgs g
     const bf16* B = (const bf16*)g.B + b1 * g.sB1 + b2 * g.sB2;
     const int64_t coff = b1 * g.sC1 + b2 * g.sC2;
 
-    TileLoader<BM, NT, TA> la;
-    TileLoader<BN, NT, TB> lb;
+    TileLoader<BM, NT> la;
+    TileLoader<BN, NT> lb;
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -478,6 +433,9 @@ __device__ __attribute__((aligned(128))) unsigned char bb_zero_line[128];
 // pixel's channel vector, or of a line of zeros where the tap falls outside the image.
 // CONV 2 (k-major operand): the weight [out, 9, in] read as B[k = (8 - tap) * out + o, n = i] (the flipped
 // filter of the input gradient): rows o advance by the k-tile, and every out / 64 k-tiles the tap changes.
+// chunk swizzle of a k-major tile: the four k-rows of a transposing read land on different banks (rows of 256 bytes and
+// more all start on bank 0, rows of 128 bytes on banks 0 and 32)
+template <int BR> __host__ __device__ constexpr int km_swizzle(int k) { return BR >= 128 ? 4 * (k & 3) : 4 * ((k >> 1) & 1); }
 template <int BR, bool KM, int NW, int BK = 32, bool VIS = false, int CONV = 0> struct DmaOperand {
     static constexpr int BYTES = BR * BK * 2;
     static constexpr int ROUNDS = BYTES / (1024 * NW);  // instructions per thread per k-tile
@@ -516,7 +474,7 @@ template <int BR, bool KM, int NW, int BK = 32, bool VIS = false, int CONV = 0> 
             } else {
                 constexpr int CPR = BR / 8, RPI = 64 / CPR;
                 const int k = q * RPI + lane / CPR;
-                const int c = (lane % CPR) ^ (4 * (k & 3));
+                const int c = (lane % CPR) ^ km_swizzle<BR>(k);
                 const int gc = min(row0 + c * 8, rows - 8);
                 src[i] = base + (int64_t)k * ld + gc;
             }
@@ -579,6 +537,18 @@ template <int BR, bool KM, int NW, int BK = 32, bool VIS = false, int CONV = 0> 
         if constexpr (CONV == 1) kstep = 0;
         if constexpr (CONV == 2) wrap = 0;
         if constexpr (CONV == 3) dpy = dpx = 0;
+    }
+    // k-major operand, last k-tile of a contraction that is no multiple of it: rows past its `left` read zeros
+    __device__ __forceinline__ void mask_tail(int left, int tid) {
+        static_assert(KM, "only a k-major operand has a ragged last k-tile");
+        constexpr int RPI = 64 / (BR / 8);
+        const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            if ((i * NW + wave) * RPI + lane / (BR / 8) < left) continue;
+            if constexpr (CONV == 3) py[i] = -(1 << 30);   // outside of every image
+            else src[i] = (const bf16*)(bb_zero_line + (lane & 7) * 16);
+        }
     }
     __device__ __forceinline__ const bf16* source(int i) const {
         if constexpr (CONV == 1) return ((inside[i] >> tap) & 1u) ? src[i] + (tapoff + c0) : zero;
@@ -649,7 +619,7 @@ template <int BR, int T, bool KM, int BK = 32> struct FragReader {
             sw = 0;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                const int c4 = ((wbase >> 5) + t) ^ j4;  // chunk-of-four index after the swizzle
+                const int c4 = ((wbase >> 5) + t) ^ (km_swizzle<BR>(j4) >> 2);  // chunk-of-four index after the swizzle
                 off[t] = (hi * 8 + j4) * (BR * 2) + ((c4 * 4 + lo) << 4) + within * 2;
             }
         }
@@ -731,7 +701,9 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         bf16x8 a[2][TM], b[2][TN];
     };
     Frags f0, f1;
-    const int KT = g.K / BK;
+    // a weight gradient's contraction (both operands k-major) may end inside a k-tile: the batch times an odd sequence length
+    constexpr bool RAGGED = AKM && BKM;
+    const int KT = RAGGED ? (g.K + BK - 1) / BK : g.K / BK;
 
     // ring positions: tile t lives in stage t % STAGES
     int issue_stage = 0, read_stage = 0;
@@ -830,6 +802,12 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     };
     auto stop_at_end = [&](int next_tile) {
         if (next_tile >= KT) {
+            if constexpr (RAGGED) {
+                if (next_tile == KT && g.K % BK != 0) {   // the last k-tile is the next to be issued
+                    opa.mask_tail(g.K % BK, tid);
+                    opb.mask_tail(g.K % BK, tid);
+                }
+            }
             opa.stop();
             opb.stop();
         }
@@ -840,14 +818,14 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     constexpr int PLD = 68;
     constexpr int NP = (TN + 1) / 2;   // pairs per row of accumulator tiles, the last one possibly a single
     const int prow = lane >> 3, pcol = (lane & 7) * 8;
-    // Only on the large tiles (one block per CU, two waves per SIMD whatever the kernel's register count): on the
-    // small ones the 32 registers would cost a resident block.
+    // Only on the large tiles (one block per CU, two waves per SIMD whatever the kernel's register count) and on the
+    // 64x64 one (a single patch, few accumulators): on the others the 32 registers would cost a resident block.
     // Some of the other kernels fetch a patch's operand(s) in one go at the top of that patch: the pointers of GemmArgs
     // may alias as far as the compiler knows, so left inside the row loop every load waits behind the previous row's
     // store (four round trips in a row per patch instead of one).
     // (HOIST: where that does not cost a resident block -- the kernels with the BatchNorm backward sums, whose three
     // operand reads per row are most of their epilogue)
-    constexpr bool PREF = BM * BN >= 256 * 128 && !VIS && CONV == 0 && STATS == 0;
+    constexpr bool PREF = (BM * BN >= 256 * 128 || BM * BN == 64 * 64) && !VIS && CONV == 0 && STATS == 0;
     constexpr bool HOIST = STATS == 2;
     const bf16* opnd = PREF || HOIST ? epilogue_operand(g) : nullptr;
     u32x4 opc[PREF || HOIST ? 4 : 1], opn[PREF ? 4 : 1];
@@ -1104,8 +1082,8 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
                 float t0 = 0.f, t1 = 0.f;
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
-                    t0 = __fadd_rn(t0, patch[r * PLD + lane]);
-                    t1 = __fadd_rn(t1, patch[(8 + r) * PLD + lane]);
+                    t0 = t0 + patch[r * PLD + lane];
+                    t1 = t1 + patch[(8 + r) * PLD + lane];
                 }
                 const int strip_row = m0 + wm * WTM + i * 32;
                 const int nc = n0 + wn * WTN + jp * 64 + lane;
@@ -1153,16 +1131,15 @@ template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGE
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
     gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, 0, 0, DROP>(g, blockIdx.x, blockIdx.z);
 }
-// the same with the strip statistics of the output (NT, 64-wide k-tiles, three stages)
-template <int BM, int BN, int WM, int WN>
+// the same with the strip statistics of the output (NT, 64-wide k-tiles)
+template <int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_stats_kernel(const GemmArgs g) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, false, false, true, 3, 64, false, 0, 1>(g, blockIdx.x, blockIdx.z);
+    gemm_bf16_dma_body<BM, BN, WM, WN, false, false, true, STAGES, 64, false, 0, 1>(g, blockIdx.x, blockIdx.z);
 }
-// input gradient of a 1x1 convolution (NN, 64-wide k-tiles, three stages) with the backward sums of the batch
-// normalisation in front of it
-template <int BM, int BN, int WM, int WN>
+// input gradient of a 1x1 convolution (NN, 64-wide k-tiles) with the backward sums of the batch normalisation in front of it
+template <int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_bnbwd_kernel(const GemmArgs g, const BnBwdArgs bn) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, false, true, true, 3, 64, false, 0, 2>(g, blockIdx.x, 0, false, ConvArgs{}, bn);
+    gemm_bf16_dma_body<BM, BN, WM, WN, false, true, true, STAGES, 64, false, 0, 2>(g, blockIdx.x, 0, false, ConvArgs{}, bn);
 }
 
 // Persistent variant for problems of more than one round of 256x256 tiles (NT and NN, 32-wide k-tiles, three stages,

@@ -712,7 +712,7 @@ class BottleNeck:
     ``hip.subsample``); the 3x3 convolution with stride 1, its input gradient (``hip.conv3x3``) and its weight
     gradient (``gemm_desc(..., conv=)``) are implicit GEMMs: the operand loader gathers the 3x3 neighbourhoods, no
     patch matrix is written.  Where the implicit kernels do not take the problem (a stride, fp32, channel counts that
-    are not multiples of 64, resp. 128 for the weight gradient) the same products run as GEMMs over the gathered patch
+    are not multiples of 64) the same products run as GEMMs over the gathered patch
     matrix ``[rows, 9*C]``.  Parameter names are the reference's; the 3x3 weight is kept as ``[out, 3, 3, in]``
     (tap-major, channel-minor) so that it is the ``[out, 9*in]`` GEMM operand as it lies in memory (the reference
     holds ``[out, in, 3, 3]``)."""
@@ -1021,7 +1021,7 @@ class BottleNeck:
             bn(4, "y2", "mean2", "rstd2", d_m0, st["a2"], d_m1, None, "bn_strips")         # d_y2
         # weight gradient of the 3x3 convolution: patch matrix gathered inside the GEMM, else built again here
         # (cheaper than stashing it)
-        wgrad_implicit = (self._implicit(ctx, hip.CONV_DGRAD) and cm % 128 == 0 and R % 32 == 0 and 32 // self.w + 1 <= self.h)
+        wgrad_implicit = self._implicit(ctx, hip.CONV_DGRAD) and cm % 64 == 0 and 32 // self.w + 1 <= self.h
         if not wgrad_implicit:
             hip.patch3x3(st["a1"], col, ctx.batch, self.h, self.w, cm, stride=self.stride, stream=sm)
         d_a1, d_m2 = ctx.buf("d_m0", (R, cm)), ctx.buf("d_m2", (R, cm))
