@@ -250,3 +250,15 @@ static inline void bb_launch(void (*kern)(P...), dim3 grid, dim3 block, size_t l
 }
 
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// out[p][c] += sum over rows of x[p][., c] for several fp32 matrices (elementwise.hip); partial[p]: bb_colsum_workspace(cols[p])
+// floats each, not shared
+constexpr int BB_COLSUM_GROUP = 16;
+struct BbColsumGroup {
+    const float* x[BB_COLSUM_GROUP];
+    float* partial[BB_COLSUM_GROUP];
+    float* out[BB_COLSUM_GROUP];
+    int64_t ldx[BB_COLSUM_GROUP];
+    int rows[BB_COLSUM_GROUP], cols[BB_COLSUM_GROUP], first_block[BB_COLSUM_GROUP + 1], count;
+};
+int bb_colsum_acc_grouped(BbColsumGroup& G, hipStream_t st);

@@ -295,8 +295,8 @@ constexpr int RED_WAVES = 16;
 // out[i] += sum_p partial[p * stride + i].  One block owns 64 columns; its sixteen waves sum
 // interleaved shares of the partial rows (p = w, w+16, ...) and the sixteen results are combined
 // in wave order, so the summation order is fixed by nparts alone.
-__global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_acc_kernel(const float* __restrict__ partial, int nparts,
-                                                                             int64_t stride, int n, float* __restrict__ out) {
+__device__ __forceinline__ void reduce_partials_acc_body(const float* __restrict__ partial, int nparts, int64_t stride, int n,
+                                                         float* __restrict__ out) {
     __shared__ float red[RED_WAVES][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + lane;
@@ -308,6 +308,10 @@ __global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_acc_kernel(con
         for (int w = 1; w < RED_WAVES; ++w) s += red[w][lane];
         out[i] += s;
     }
+}
+__global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_acc_kernel(const float* __restrict__ partial, int nparts,
+                                                                             int64_t stride, int n, float* __restrict__ out) {
+    reduce_partials_acc_body(partial, nparts, stride, n, out);
 }
 
 // two vectors at once (LayerNorm gain and shift gradients): blockIdx.y picks the half of every
@@ -486,12 +490,12 @@ extern "C" int bb_layernorm_bwd_static(int dtype, int kind, int rows, int cols, 
 constexpr int COLSUM_SPLITS = 64;
 
 template <typename T>
-__global__ __launch_bounds__(256) void colsum_partial_kernel(int rows, int cols, const T* __restrict__ x, int64_t ldx,
-                                                             float* __restrict__ partial) {
+__device__ __forceinline__ void colsum_partial_body(int block, int rows, int cols, const T* __restrict__ x, int64_t ldx,
+                                                    float* __restrict__ partial) {
     constexpr int VEC = Elem<T>::VEC;
     __shared__ float red[3][64 * VEC];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c0 = (blockIdx.x * 64 + lane) * VEC;
+    const int c0 = (block * 64 + lane) * VEC;
     float acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
@@ -517,9 +521,38 @@ __global__ __launch_bounds__(256) void colsum_partial_kernel(int rows, int cols,
         }
     }
 }
+template <typename T>
+__global__ __launch_bounds__(256) void colsum_partial_kernel(int rows, int cols, const T* __restrict__ x, int64_t ldx,
+                                                             float* __restrict__ partial) {
+    colsum_partial_body(blockIdx.x, rows, cols, x, ldx, partial);
+}
+// the column sums of several fp32 matrices in one pair of launches (the bias gradients of an fp32 layer), each with the
+// additions and the order of a call of its own
+__global__ __launch_bounds__(256) void colsum_partial_grouped_kernel(const BbColsumGroup G) {
+    int p = 0;
+    while (p + 1 < G.count && (int)blockIdx.x >= G.first_block[p + 1]) ++p;
+    colsum_partial_body(blockIdx.x - G.first_block[p], G.rows[p], G.cols[p], G.x[p], G.ldx[p], G.partial[p]);
+}
+__global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_grouped_kernel(const BbColsumGroup G) {
+    const int p = blockIdx.y;
+    if ((int)blockIdx.x * 64 < G.cols[p]) reduce_partials_acc_body(G.partial[p], COLSUM_SPLITS, G.cols[p], G.cols[p], G.out[p]);
+}
 
 extern "C" int64_t bb_colsum_workspace(int cols) { return (int64_t)COLSUM_SPLITS * cols; }
 
+int bb_colsum_acc_grouped(BbColsumGroup& G, hipStream_t st) {
+    int blocks = 0, most = 0;
+    for (int i = 0; i < G.count; ++i) {
+        G.first_block[i] = blocks;
+        blocks += (G.cols[i] + 255) / 256;
+        most = G.cols[i] > most ? G.cols[i] : most;
+    }
+    G.first_block[G.count] = blocks;
+    bb_launch(colsum_partial_grouped_kernel, dim3(blocks, COLSUM_SPLITS), dim3(256), 0, st, G);
+    bb_launch(reduce_partials_grouped_kernel, dim3((most + 63) / 64, G.count), dim3(RED_WAVES * 64), 0, st, G);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
 extern "C" int bb_colsum_acc(int dtype, int rows, int cols, const void* x, int64_t ldx, float* out, float* workspace,
                              void* stream) {
     BB_REQUIRE(dtype == BB_F32 || dtype == BB_BF16, "bb_colsum_acc: bad dtype %d", dtype);

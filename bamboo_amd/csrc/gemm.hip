@@ -5,8 +5,9 @@
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:121,127,136-146,158).
 //
 // bf16 data paths: tiles by DMA (gemm_bf16_dma_*), 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for
-// problems of few tiles, and a register-staged kernel for rows of C that are no whole vectors.
+// problems of few tiles, and a register-staged kernel for rows of C that are no whole vectors.  fp32: gemm_f32.h.
 #include "gemm_kernels.h"
+#include "gemm_f32.h"
 #include "gemm_wave.h"
 
 // =========================================================================================
@@ -239,36 +240,26 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
     return BB_EINVAL;
 }
 
-static int pick_f32_tile(int M, int N, int64_t batches) {
-    const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
-    return t128 < 2 * 256 ? 64 : 128;
-}
-// Problems with fewer than two 64x64 tiles per CU (one or two waves per SIMD, and some CUs with twice the tiles of
-// others) and at least 32 k-tiles wait for operands most of the time: they take 64x32 tiles whose contraction two
-// groups of two waves share (kF32SplitGroups; twice the tiles, each wave's chain of k-tiles halved).  NT and NN only:
-// the weight gradients (TN) of a layer share a grouped launch.
+// fp32 problems with fewer than two 64x64 tiles per CU and at least 16 k-tiles take 64x32 tiles whose contraction two groups of
+// two waves share: twice the tiles to deal to the CUs, each wave's chain of matrix instructions as long as before.  NT and NN
+// only: the weight gradients (TN) of a layer share a grouped launch.
 static constexpr int kF32SplitGroups = 2, kF32SplitBN = 32;
 static bool pick_f32_split(int M, int N, int K, int64_t batches, int layout) {
-    if (layout == BB_TN || pick_f32_tile(M, N, batches) != 64) return false;
-    const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches;
-    return t64 < 2 * 256 && K >= 512;
+    return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches < 2 * 256 && K >= 512;
 }
-template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hipStream_t st) {
-    // 64x64 tiles while 128x128 ones would leave most CUs with a single block (one wave per SIMD): shape only, and the
-    // same order of additions on both, so which one runs changes no bit
-    const int tile = pick_f32_tile(g.M, g.N, batches);
-    g.tiles_m = (g.M + tile - 1) / tile;
-    g.tiles_n = (g.N + tile - 1) / tile;
-    dim3 grid(g.tiles_m * g.tiles_n, 1, batches);
-    if (pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) {
-        g.tiles_n = (g.N + kF32SplitBN - 1) / kF32SplitBN;
-        grid.x = g.tiles_m * g.tiles_n;
-        bb_launch((gemm_f32_ksplit_kernel<TA, TB, kF32SplitGroups, kF32SplitBN>), grid, dim3(4 * kF32SplitBN * kF32SplitGroups), 0, st, g);
-    }
-    else if (tile == 64) bb_launch((gemm_f32_kernel<TA, TB, 64>), grid, dim3(256), 0, st, g);
-    else bb_launch((gemm_f32_kernel<TA, TB, 128>), grid, dim3(256), 0, st, g);
+template <bool TA, bool TB, int BN> static int launch_f32(GemmArgs& g, int batches, hipStream_t st) {
+    auto kern = gemm_f32_kernel<TA, TB, BN>;
+    g.tiles_m = (g.M + 63) / 64;
+    g.tiles_n = (g.N + BN - 1) / BN;
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(256), f32_gemm_lds(BN), st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
+}
+template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hipStream_t st) {
+    if (pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) {
+        if constexpr (!TA) return launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
+    }
+    return launch_f32<TA, TB, 64>(g, batches, st);
 }
 
 extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
@@ -283,13 +274,9 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
         else snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
                  dt != D_NONE ? kDmaTileNames[dt] : "128x128");
     }
-    else
-    {
-        const int tile = pick_f32_tile(d->M, d->N, batches);
-        if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
-            snprintf(out, out_len, "f32_%s_64x%dk%d", layouts[d->layout], kF32SplitBN, kF32SplitGroups);
-        else snprintf(out, out_len, "f32_%s_%dx%d", layouts[d->layout], tile, tile);
-    }
+    else if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
+        snprintf(out, out_len, "f32_%s_64x%dk%d", layouts[d->layout], kF32SplitBN, kF32SplitGroups);
+    else snprintf(out, out_len, "f32_%s_64x64", layouts[d->layout]);
     return BB_OK;
 }
 
@@ -334,6 +321,7 @@ static int fill_args(const bb_gemm_desc* d, GemmArgs& g, int64_t& batches, bool&
     BB_REQUIRE(d->sA1 % vec == 0 && d->sA2 % vec == 0 && d->sB1 % vec == 0 && d->sB2 % vec == 0,
                "bb_gemm: batch strides of A/B must be multiples of %d", vec);
     BB_REQUIRE(d->lda >= a_contig && ldb >= b_contig && d->ldc >= d->N, "bb_gemm: leading dimension too small");
+    BB_REQUIRE(d->dtype != BB_F32 || (d->lda < (1 << 22) && d->ldb < (1 << 22)), "bb_gemm: fp32 leading dimension too large");
     g.A = d->A; g.B = d->B; g.C = d->C;
     g.bias = d->bias; g.aux_in = d->aux_in; g.aux_out = d->aux_out; g.resid = d->resid;
     g.colsum = nullptr;
@@ -607,6 +595,31 @@ template <int KW, int BK, int NST> static int launch_grouped_wave(GroupedArgs& G
     return BB_OK;
 }
 
+// The bias gradients that ride on fp32 weight gradients: one pair of launches for all of them where their workspaces do not
+// overlap, else a pair each.
+static int colsum_f32(const bb_gemm_desc* descs, int count, void* stream) {
+    BbColsumGroup C;
+    C.count = 0;
+    bool apart = true;
+    for (int i = 0; i < count; ++i) {
+        const bb_gemm_desc& d = descs[i];
+        if (!d.colsum_out) continue;
+        BB_REQUIRE(d.colsum_ws, "bb_gemm_grouped: colsum_out on this problem needs colsum_ws");
+        const float *lo = d.colsum_ws, *hi = lo + bb_colsum_workspace(d.M);
+        for (int j = 0; j < C.count; ++j) apart = apart && (hi <= C.partial[j] || C.partial[j] + bb_colsum_workspace(C.cols[j]) <= lo);
+        C.x[C.count] = (const float*)d.A; C.partial[C.count] = d.colsum_ws; C.out[C.count] = d.colsum_out;
+        C.ldx[C.count] = d.lda; C.rows[C.count] = d.K; C.cols[C.count] = d.M;
+        ++C.count;
+    }
+    if (C.count == 0) return BB_OK;
+    if (apart) return bb_colsum_acc_grouped(C, (hipStream_t)stream);
+    for (int i = 0; i < count; ++i) {
+        int rc = descs[i].colsum_out ? colsum_standalone(&descs[i], stream) : BB_OK;
+        if (rc) return rc;
+    }
+    return BB_OK;
+}
+
 extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream) {
     BB_REQUIRE(count >= 0 && (descs || count == 0), "bb_gemm_grouped: bad arguments");
     hipStream_t st = (hipStream_t)stream;
@@ -627,12 +640,12 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
     }
     // weight gradients of few tiles: 64x64 tiles, the contraction dealt to the waves (see kGroupedWaveTiles)
     wave = wave && (!dma || tiles <= (count > 1 ? kGroupedWaveTiles : 256));   // alone: as bb_gemm takes it
-    // fp32: unbatched problems of one layout that all take the small tile (each alone would leave CUs idle) share a launch
+    // fp32: unbatched problems of one layout share a launch
     bool fuse32 = !fuse && !has_conv && count >= 2 && count <= GROUP_MAX;
     for (int i = 0; i < count && fuse32; ++i) {
         const bb_gemm_desc& d = descs[i];
-        fuse32 = d.dtype == BB_F32 && d.layout == descs[0].layout && d.nb1 <= 1 && d.nb2 <= 1 && d.M > 0 && d.N > 0 &&
-                 d.dropout_p == 0.f && pick_f32_tile(d.M, d.N, 1) == 64;
+        fuse32 = d.dtype == BB_F32 && d.layout == descs[0].layout && d.nb1 <= 1 && d.nb2 <= 1 && d.M > 0 && d.N > 0 && d.dropout_p == 0.f &&
+                 !pick_f32_split(d.M, d.N, d.K, 1, d.layout);
     }
     if (fuse32) {
         GroupedArgs G;
@@ -643,18 +656,18 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
             bool ta, tb;
             int rc = fill_args(&descs[i], G.p[i], batches, ta, tb);
             if (rc) return rc;
-            // the bias gradient that rides on a weight gradient: its own kernel, as on the one-by-one route
-            if (descs[i].colsum_out && (rc = colsum_standalone(&descs[i], stream)) != BB_OK) return rc;
             G.p[i].tiles_m = (G.p[i].M + 63) / 64;
             G.p[i].tiles_n = (G.p[i].N + 63) / 64;
             G.first_block[i] = blocks;
             blocks += G.p[i].tiles_m * G.p[i].tiles_n;
         }
         G.first_block[count] = blocks;
+        int rc = colsum_f32(descs, count, stream);
+        if (rc) return rc;
         const int layout = descs[0].layout;
-        if (layout == BB_NT) bb_launch((gemm_f32_grouped_kernel<false, false, 64>), dim3(blocks), dim3(256), 0, st, G);
-        else if (layout == BB_NN) bb_launch((gemm_f32_grouped_kernel<false, true, 64>), dim3(blocks), dim3(256), 0, st, G);
-        else bb_launch((gemm_f32_grouped_kernel<true, true, 64>), dim3(blocks), dim3(256), 0, st, G);
+        if (layout == BB_NT) bb_launch((gemm_f32_grouped_kernel<false, false>), dim3(blocks), dim3(256), f32_gemm_lds(64), st, G);
+        else if (layout == BB_NN) bb_launch((gemm_f32_grouped_kernel<false, true>), dim3(blocks), dim3(256), f32_gemm_lds(64), st, G);
+        else bb_launch((gemm_f32_grouped_kernel<true, true>), dim3(blocks), dim3(256), f32_gemm_lds(64), st, G);
         BB_LAUNCH_CHECK();
         return BB_OK;
     }

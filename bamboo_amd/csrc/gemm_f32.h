@@ -1,0 +1,294 @@
+// fp32 GEMM: v_mfma_f32_32x32x2_f32 on 64x64 tiles (four waves of 32x32), or on 64x32 tiles whose contraction two groups of
+// two waves share.
+#pragma once
+#include "gemm_kernels.h"
+
+// What bounds it: fp32 matrix instructions run on the vector ALU's multipliers (a dependent chain of them reaches 134-145 of
+// 157 TFLOP/s with one to three waves per SIMD, and every vector instruction beside them is matrix time lost: four selects per
+// 128 matrix cycles cost a tenth of the kernel).  So the main loop has none: operand tiles go global -> LDS by DMA with the
+// base in scalar registers, LDS addresses are computed once and the stage is in the instructions' offsets (the loop is unrolled
+// over the stages of 32-wide k-tiles), and a k-tile of 1024 matrix cycles has one barrier.  The values of a part of a
+// k-tile are fetched under the matrix instructions of the part before it.  What the epilogue reads is fetched before the main
+// loop (16 values per lane: one round trip instead of sixteen behind the stores).
+// LDS formats, per operand and stage:
+//   K-contiguous memory: [rows][32 k], 128 B a row = 8 chunks of 16 B, chunk c of row r at c ^ ((r >> 1) & 7).
+//   k-major memory: [32 k][rows]; 64-row tiles keep rows 0..31 of odd k at the place of rows 32..63 and vice versa, so that
+//     the two halves of a wave (k and k + 1) read different banks.
+// Every element adds up its contraction in pairs (k, k + 1), k ascending (groups: the even, resp. odd 16-wide k-tiles, group
+// 0's sum plus group 1's), whatever the tile: which kernel runs a problem changes no bit.
+// (volatile: pairs of reads merged into one instruction have no room for the stage's offset, i.e. cost an addition each)
+typedef const volatile __attribute__((address_space(3))) float lds_f32;
+template <int ROWS, bool KM> struct F32Operand {
+    static constexpr int BYTES = ROWS * 32 * 4, ROUNDS = BYTES / (1024 * 4);   // four waves load a stage
+    const float* base;          // wave-uniform: the tile's first row (K-contiguous) / column (k-major), the next k-tile
+    unsigned off[ROUNDS];       // the lane's 16 bytes from there
+    int k_lane[ROUNDS];         // ... and their k inside a k-tile
+    int64_t step;
+    __device__ __forceinline__ void init(const float* p, int64_t ld, int row0, int rows, int lane, int wave) {
+        base = p + (KM ? row0 : (int64_t)row0 * ld);
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int q = i * 4 + wave;
+            if constexpr (!KM) {
+                const int r = q * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+                k_lane[i] = c * 4;
+                off[i] = (unsigned)((int64_t)min(r, rows - 1 - row0) * ld + c * 4) * 4u;
+            } else {
+                constexpr int CPR = ROWS / 4, RPI = 64 / CPR;   // 16-byte chunks per k-row, k-rows per instruction
+                const int k = q * RPI + lane / CPR, c = (lane % CPR) ^ (ROWS == 64 ? 8 * (k & 1) : 0);
+                k_lane[i] = k;
+                off[i] = (unsigned)((int64_t)k * ld + min(c * 4, rows - 4 - row0)) * 4u;
+            }
+        }
+        step = KM ? 32 * ld : 32;
+    }
+    // `left`: contraction elements from the k-tile's start (< 32: the last, ragged one); lds: LDS address of the stage
+    __device__ __forceinline__ void issue(unsigned lds, int wave, int left, int lane) {
+        if (left >= 32) {
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + (i * 4 + wave) * 1024), "v"(off[i]), "s"(base) : "m0");
+        } else {
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i)
+                dma16_at(k_lane[i] < left ? (const unsigned char*)base + off[i] : bb_zero_line + (lane & 7) * 16, lds + (i * 4 + wave) * 1024);
+        }
+        base += step;
+    }
+};
+// The operand values of a wave: lane = row (lane & 31), its half's k of the pairs (4 c, 4 c + 1) and (4 c + 2, 4 c + 3) of
+// chunk c.  NC: chunks of a k-tile the wave takes, from chunk c0 on.
+template <int ROWS, bool KM, int NC> struct F32Reader {
+    unsigned at[KM ? 1 : NC];   // LDS addresses inside stage 0
+    __device__ __forceinline__ void init(unsigned lds, int row0, int c0, int lane) {
+        const int r = row0 + (lane & 31), h = lane >> 5;
+        if constexpr (KM) at[0] = lds + ((4 * c0 + h) * ROWS + (ROWS == 64 ? r ^ (32 * h) : r)) * 4;
+        else {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) at[c] = lds + r * 128 + (((c0 + c) ^ ((r >> 1) & 7)) << 4) + 4 * h;
+        }
+    }
+    // chunks FIRST .. FIRST + N - 1 of the stage STAGE_OFF bytes behind stage 0
+    template <int STAGE_OFF, int FIRST, int N> __device__ __forceinline__ void load(float (&v)[N][2]) const {
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            lds_f32* p = KM ? (lds_f32*)at[0] + STAGE_OFF / 4 + (FIRST + c) * 4 * ROWS : (lds_f32*)at[FIRST + c] + STAGE_OFF / 4;
+            v[c][0] = p[0];
+            v[c][1] = p[KM ? 2 * ROWS : 2];
+        }
+    }
+};
+
+// two stages of a 64x64 tile (32 KB), three of a 64x32 tile (36 KB): four blocks per CU either way, as the registers allow
+constexpr int f32_stages(int bn) { return bn == 64 ? 2 : 3; }
+constexpr int f32_gemm_lds(int bn) { return f32_stages(bn) * (64 + bn) * 128; }
+
+// The epilogue of a lane's sixteen elements (one column; register r: row m + 8 (r / 4) + r % 4).  `pre`: what it reads beside
+// the product -- the operand of the epilogue kind, else the C it accumulates into -- fetched before the main loop; `rest`: a
+// problem that reads both, or a masked residual, fetches the second here.  One branch over the kind around the sixteen, not
+// inside: the code stays small.
+__device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, int m0, int n, float bias, const float (&pre)[16], f32x16& v) {
+    const auto row = [&](int r) { return m0 + 8 * (r >> 2) + (r & 3); };
+    const bool has_opnd = epilogue_operand(g) != nullptr;
+    float rest[16], keep[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        rest[r] = pre[r];
+        keep[r] = 1.0f;
+    }
+    if (has_opnd && g.accumulate) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) rest[r] = ((const float*)g.C)[coff + (int64_t)min(row(r), g.M - 1) * g.ldc + n];
+    } else if (g.epilogue == BB_EPI_MUL_POS && g.resid) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) rest[r] = ((const float*)g.resid)[coff + (int64_t)min(row(r), g.M - 1) * g.ldaux + n];
+    }
+    if (g.drop.thresh) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) keep[r] = drop_factor(g, row(r), n);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = v[r] * g.alpha + bias;
+    float* aux = (float*)g.aux_out + coff + n;
+    if (g.epilogue == BB_EPI_ACT) {
+        if (g.aux_out) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (row(r) < g.M) aux[(int64_t)row(r) * g.ldaux] = v[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = act_f(v[r], g.act) * keep[r];
+    } else if (g.epilogue == BB_EPI_ACT_DACT) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float a, d;
+            act_dact_f(v[r], g.act, a, d);
+            if (row(r) < g.M) aux[(int64_t)row(r) * g.ldaux] = d * keep[r];
+            v[r] = a * keep[r];
+        }
+    } else if (g.epilogue == BB_EPI_DACT) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] *= dact_f(pre[r], g.act);
+    } else if (g.epilogue == BB_EPI_RESIDUAL) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = v[r] * keep[r] + pre[r];
+    } else if (g.epilogue == BB_EPI_MUL) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] *= pre[r];
+    } else if (g.epilogue == BB_EPI_MUL_POS) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = pre[r] > 0.f ? (g.resid ? v[r] + rest[r] : v[r]) : 0.f;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] *= keep[r];
+    }
+    float* c = (float*)g.C + coff + n;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        if (row(r) < g.M) c[(int64_t)row(r) * g.ldc] = g.accumulate ? rest[r] + v[r] : v[r];
+}
+
+// (block_id: the block's index among the problem's tiles; logical_id: it is not a hardware block id, so the tile order takes it
+// as it is instead of undoing the round-robin over the XCDs)
+template <bool TA, bool TB, int BN>
+__device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block_id, const int batch_id, const bool logical_id) {
+    static_assert(BN == 64 || BN == 32, "tiles: 64x64, 64x32 with the contraction shared by two groups");
+    constexpr int KG = 64 / BN;
+    using OpA = F32Operand<64, TA>;
+    using OpB = F32Operand<BN, TB>;
+    constexpr int STAGES = f32_stages(BN), STAGE = OpA::BYTES + OpB::BYTES, LOADS = OpA::ROUNDS + OpB::ROUNDS;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave & 1, wn = KG == 1 ? wave >> 1 : 0, grp = KG == 1 ? 0 : wave >> 1;
+    int tile_m, tile_n;
+    if (logical_id) panel_coords(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    else tile_coords(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    const int m0 = tile_m * 64, n0 = tile_n * BN;
+    const int b1 = batch_id / g.nb2, b2 = batch_id % g.nb2;
+    const int64_t coff = b1 * g.sC1 + b2 * g.sC2;
+    OpA opa;
+    OpB opb;
+    opa.init((const float*)g.A + b1 * g.sA1 + b2 * g.sA2, g.lda, m0, g.M, lane, wave);
+    opb.init((const float*)g.B + b1 * g.sB1 + b2 * g.sB2, g.ldb, n0, g.N, lane, wave);
+
+    constexpr int NC = 8 / KG;   // chunks of four k of a k-tile that this wave multiplies
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t*)smem;
+    F32Reader<64, TA, NC> ra;
+    F32Reader<BN, TB, NC> rb;
+    ra.init(lds0, wm * 32, grp * NC, lane);
+    rb.init(lds0 + OpA::BYTES, wn * 32, grp * NC, lane);
+
+    // what the epilogue reads: lane = column, register r = row acc_m + 8 (r / 4) + r % 4
+    const int n = n0 + wn * 32 + (lane & 31), acc_m = m0 + wm * 32 + 4 * (lane >> 5);
+    const float* opnd = (const float*)epilogue_operand(g);
+    const int64_t ld_pre = opnd ? g.ldaux : g.ldc;
+    if (!opnd && g.accumulate) opnd = (const float*)g.C;
+    float bias = 0.f, pre[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) pre[r] = 0.f;
+    const int nc = min(n, g.N - 1);    // clamped: what is read for a row or column past the end is not used
+    if (grp == 0) {
+        if (g.bias) bias = ((const float*)g.bias)[nc];
+        if (opnd) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) pre[r] = opnd[coff + (int64_t)min(acc_m + 8 * (r >> 2) + (r & 3), g.M - 1) * ld_pre + nc];
+        }
+    }
+
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+
+    const int KT = (g.K + 31) / 32;
+    int issued = 0, into = 0;
+    auto issue = [&]() {
+        const int left = g.K - issued * 32;
+        opa.issue(lds0 + into, wave, left, lane);
+        opb.issue(lds0 + into + OpA::BYTES, wave, left, lane);
+        into = into == (STAGES - 1) * STAGE ? 0 : into + STAGE;
+        ++issued;
+    };
+    // a k-tile is multiplied in two parts; the values of the next part -- behind the barrier that makes the next k-tile visible,
+    // where it begins one -- are fetched under the matrix instructions of this one, into the other register set
+    float fa[2][NC / 2][2], fb[2][NC / 2][2];
+    auto multiply = [&](const float (&x)[NC / 2][2], const float (&y)[NC / 2][2]) {
+#pragma unroll
+        for (int c = 0; c < NC / 2; ++c)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[c][i], y[c][i], acc, 0, 0, 0);
+    };
+    // the k-tile after kt - 1 has landed (in-order completion; with three stages one more may be in flight) and every wave has
+    // read that one: its stage takes the next
+    auto next_tile = [&](int kt) {
+        asm volatile("" ::: "memory");
+        if (STAGES == 3 && kt + 1 < KT) wait_vmcnt_lgkm0<LOADS>();
+        else wait_vmcnt_lgkm0<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (issued < KT) issue();
+    };
+    auto k_tile = [&](int kt, auto stage_c) {
+        constexpr int S = decltype(stage_c)::value, NX = (S + 1) % STAGES;
+        ra.template load<S * STAGE, NC / 2>(fa[1]);
+        rb.template load<S * STAGE, NC / 2>(fb[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fa[0], fb[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + 1 < KT) next_tile(kt + 1);
+        // (behind the last k-tile: of a stage that is there, for nobody; no branch around the reads)
+        ra.template load<NX * STAGE, 0>(fa[0]);
+        rb.template load<NX * STAGE, 0>(fb[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fa[1], fb[1]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (KT > 0) {
+        issue();
+        if (KT > 1) issue();
+        if (STAGES == 3 && KT > 2) issue();
+        // in-order completion: the first k-tile has landed
+        asm volatile("" ::: "memory");
+        if (KT > 2 && STAGES == 3) wait_vmcnt_lgkm0<2 * LOADS>();
+        else if (KT > 1) wait_vmcnt_lgkm0<LOADS>();
+        else wait_vmcnt_lgkm0<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        ra.template load<0, 0>(fa[0]);
+        rb.template load<0, 0>(fb[0]);
+        int kt = 0;
+        for (; kt + STAGES <= KT; kt += STAGES) {
+            k_tile(kt, std::integral_constant<int, 0>{});
+            k_tile(kt + 1, std::integral_constant<int, 1>{});
+            if constexpr (STAGES == 3) k_tile(kt + 2, std::integral_constant<int, 2>{});
+        }
+        if (kt < KT) k_tile(kt, std::integral_constant<int, 0>{});
+        if (STAGES == 3 && kt + 1 < KT) k_tile(kt + 1, std::integral_constant<int, 1>{});
+    }
+    if constexpr (KG > 1) {
+        // group 1's partial tile through the (drained) stages
+        float* part = (float*)smem + wm * (16 * 64);
+        __syncthreads();
+        if (grp == 1) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[r * 64 + lane] = acc[r];
+        }
+        __syncthreads();
+        if (grp == 1) return;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] += part[r * 64 + lane];
+    }
+    if (n < g.N) epilogue_f32(g, coff, acc_m, n, bias, pre, acc);
+}
+
+template <bool TA, bool TB, int BN>
+__global__ __launch_bounds__(256, 4) void gemm_f32_kernel(const GemmArgs g) {
+    gemm_f32_body<TA, TB, BN>(g, blockIdx.x, blockIdx.z, false);
+}
+// several unbatched problems in one launch (the weight gradients of an fp32 layer)
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 4) void gemm_f32_grouped_kernel(const GroupedArgs G) {
+    const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
+    int pi = 0;
+    while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
+    gemm_f32_body<TA, TB, 64>(G.p[pi], lid - G.first_block[pi], 0, true);
+}

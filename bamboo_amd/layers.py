@@ -84,6 +84,12 @@ class StageContext:
         if self.workspace is None or self.workspace.numel() < n:
             self.workspace = torch.empty(n, dtype=torch.float32, device=self.device)
 
+    def colsum_ws(self, wgrads, cols):
+        """Workspace of the bias gradient that joins the collected weight gradients: regions of their own, so that all
+        of them may share a launch (``TransformerLayer.workspace_elems`` has room for a layer's)."""
+        off = sum(hip.colsum_workspace(d.M) for d in wgrads)
+        return self.workspace[off: off + hip.colsum_workspace(cols)]
+
     def buf(self, name, shape):
         return self.scratch[name][: math.prod(shape)].view(shape)
 
@@ -241,7 +247,7 @@ class TransformerLayer:
         return self.dropout, key
 
     def workspace_elems(self):
-        n = max(self.hidden * 3, self.ffn)
+        n = 5 * self.hidden + self.ffn    # the four weight gradients of a grouped launch
         return max(hip.layernorm_bwd_workspace(self.hidden), hip.colsum_workspace(n))
 
     def flops_fwd(self, batch, seq):
@@ -369,7 +375,7 @@ class TransformerLayer:
         wgrads = []
         # ... and each carries its bias gradient (column sums of dy) in the same kernel
         wgrad = lambda dy, x, name: wgrads.append(hip.gemm_desc(
-            hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[name[:-len("weight")] + "bias"], colsum_ws=ws))
+            hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[name[:-len("weight")] + "bias"], colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
         if ctx.deferred and self.activation != "relu":
             self._ffn1(st, ctx)   # the forward of this stash left act' out: same kernel, same bits as a normal forward
         # the gradient behind a sublayer's dropout feeds the sublayer; the residual branch takes the one in front of it
@@ -541,7 +547,7 @@ class DecoderLayer(TransformerLayer):
         d_qkv, d_mem = ctx.buf("d_qkv", (R, 3 * h)), ctx.buf("d_mem", (R, h))
         wgrads = []
         wgrad = lambda dy, x, name, bias=None: wgrads.append(hip.gemm_desc(
-            hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[bias or (name[:-len("weight")] + "bias")], colsum_ws=ws))
+            hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[bias or (name[:-len("weight")] + "bias")], colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
 
         def flush():
             # the weight gradients collected so far, before a scratch buffer they read is written again
@@ -576,7 +582,7 @@ class DecoderLayer(TransformerLayer):
         self._attention_bwd(d_h0, d_qkv, self._src_views(st), ctx, site=self.SITE_SRC_ATTENTION, mask="none")
         wgrad(d_qkv[:, :h], st["n_src"], "src_attn.linears.0.weight")
         wgrads.append(hip.gemm_desc(hip.TN, d_qkv[:, h:], st["mem"], g["kv.weight"], accumulate=True,
-                                    colsum_out=g["kv.bias"], colsum_ws=ws))
+                                    colsum_out=g["kv.bias"], colsum_ws=ctx.colsum_ws(wgrads, 2 * h)))
         ctx.gemm(hip.NN, d_qkv[:, :h], w["src_attn.linears.0.weight"], d_h0, stream=sm)        # d_n_src
         ctx.gemm(hip.NN, d_qkv[:, h:], w["kv.weight"], d_mem, stream=sm)                       # gradient of the memory
         # d_x1 = d_x2 + LN_src'(d_n_src)  -> d_h1
