@@ -240,22 +240,42 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
     return BB_EINVAL;
 }
 
-// fp32 problems with fewer than two 64x64 tiles per CU and at least 16 k-tiles take 64x32 tiles whose contraction two groups of
+// fp32 problems of few tiles and a contraction of at most one slice a wave (the products of attention heads, the input gradients
+// of a narrow model, weight gradients over few rows) take 32x32 tiles, up to four per CU.  64x64 tiles / this (us, back to
+// back): NN 128x128x128 6.6 / 3.9, 512x1024x64 5.4 / 4.6, 2048x384x128 (768 tiles) 7.2 / 6.1, 2048x512x128 (1024) 7.3 / 7.0,
+// 2048x1024x128 (2048) 9.9 / 11.6.  Weight gradients share a launch with the others of their layer, so there the limit is
+// each problem's own (a problem gives the same bits alone and in a group): 128 rows x 128 (x 2 in the feed-forward) 7.8 / 4.8,
+// x 256 (x 4) 8.4 / 6.8, x 384 (576 tiles the largest) 11.0 / 12.2.  The layers' own forward products (NT, unbatched), whose last
+// bits decide ReLUs, keep the order of additions of the larger tiles, as in bf16.
+static bool pick_f32_wave(int M, int N, int K, int64_t batches, int layout) {
+    const int64_t tiles = (int64_t)((M + 31) / 32) * ((N + 31) / 32) * batches;
+    if (layout == BB_NT && batches == 1) return false;
+    return K <= kF32WaveK && tiles <= (layout == BB_TN && batches == 1 ? 256 : 1024);
+}
+// Longer fp32 contractions: problems with fewer than two 64x64 tiles per CU and at least 16 k-tiles take 64x32 tiles whose contraction two groups of
 // two waves share: twice the tiles to deal to the CUs, each wave's chain of matrix instructions as long as before.  NT and NN
 // only: the weight gradients (TN) of a layer share a grouped launch.
 static constexpr int kF32SplitGroups = 2, kF32SplitBN = 32;
 static bool pick_f32_split(int M, int N, int K, int64_t batches, int layout) {
     return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches < 2 * 256 && K >= 512;
 }
+template <bool TA, bool TB> static int launch_f32_wave(GemmArgs& g, int batches, hipStream_t st) {
+    auto kern = gemm_f32_wave_kernel<TA, TB>;
+    g.tiles_m = (g.M + 31) / 32;
+    g.tiles_n = (g.N + 31) / 32;
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(kF32Waves * 64), kF32WaveLds, st, g);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
 template <bool TA, bool TB, int BN> static int launch_f32(GemmArgs& g, int batches, hipStream_t st) {
-    auto kern = gemm_f32_kernel<TA, TB, BN>;
     g.tiles_m = (g.M + 63) / 64;
     g.tiles_n = (g.N + BN - 1) / BN;
-    bb_launch(kern, dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(256), f32_gemm_lds(BN), st, g);
+    bb_launch((gemm_f32_kernel<TA, TB, BN>), dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(256), f32_gemm_lds(BN), st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
 template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hipStream_t st) {
+    if (pick_f32_wave(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) return launch_f32_wave<TA, TB>(g, batches, st);
     if (pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) {
         if constexpr (!TA) return launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
     }
@@ -274,6 +294,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
         else snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
                  dt != D_NONE ? kDmaTileNames[dt] : "128x128");
     }
+    else if (pick_f32_wave(d->M, d->N, d->K, batches, d->layout)) snprintf(out, out_len, "f32_%s_wave32x32k%d", layouts[d->layout], kF32Waves);
     else if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
         snprintf(out, out_len, "f32_%s_64x%dk%d", layouts[d->layout], kF32SplitBN, kF32SplitGroups);
     else snprintf(out, out_len, "f32_%s_64x64", layouts[d->layout]);
@@ -640,24 +661,31 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
     }
     // weight gradients of few tiles: 64x64 tiles, the contraction dealt to the waves (see kGroupedWaveTiles)
     wave = wave && (!dma || tiles <= (count > 1 ? kGroupedWaveTiles : 256));   // alone: as bb_gemm takes it
-    // fp32: unbatched problems of one layout share a launch
+    // fp32: unbatched problems of one layout share a launch where one kernel takes them all (weight gradients of both kinds:
+    // the 64x64 tiles)
     bool fuse32 = !fuse && !has_conv && count >= 2 && count <= GROUP_MAX;
+    int few = 0;
     for (int i = 0; i < count && fuse32; ++i) {
         const bb_gemm_desc& d = descs[i];
+        const bool w = pick_f32_wave(d.M, d.N, d.K, 1, d.layout);
+        few += w;
         fuse32 = d.dtype == BB_F32 && d.layout == descs[0].layout && d.nb1 <= 1 && d.nb2 <= 1 && d.M > 0 && d.N > 0 && d.dropout_p == 0.f &&
-                 !pick_f32_split(d.M, d.N, d.K, 1, d.layout);
+                 (w || !pick_f32_split(d.M, d.N, d.K, 1, d.layout));
     }
+    const bool waves = few == count;
+    fuse32 = fuse32 && (waves || few == 0 || descs[0].layout == BB_TN);
     if (fuse32) {
         GroupedArgs G;
         G.count = count;
+        const int tile = waves ? 32 : 64;
         int blocks = 0;
         for (int i = 0; i < count; ++i) {
             int64_t batches;
             bool ta, tb;
             int rc = fill_args(&descs[i], G.p[i], batches, ta, tb);
             if (rc) return rc;
-            G.p[i].tiles_m = (G.p[i].M + 63) / 64;
-            G.p[i].tiles_n = (G.p[i].N + 63) / 64;
+            G.p[i].tiles_m = (G.p[i].M + tile - 1) / tile;
+            G.p[i].tiles_n = (G.p[i].N + tile - 1) / tile;
             G.first_block[i] = blocks;
             blocks += G.p[i].tiles_m * G.p[i].tiles_n;
         }
@@ -665,9 +693,10 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
         int rc = colsum_f32(descs, count, stream);
         if (rc) return rc;
         const int layout = descs[0].layout;
-        if (layout == BB_NT) bb_launch((gemm_f32_grouped_kernel<false, false>), dim3(blocks), dim3(256), f32_gemm_lds(64), st, G);
-        else if (layout == BB_NN) bb_launch((gemm_f32_grouped_kernel<false, true>), dim3(blocks), dim3(256), f32_gemm_lds(64), st, G);
-        else bb_launch((gemm_f32_grouped_kernel<true, true>), dim3(blocks), dim3(256), f32_gemm_lds(64), st, G);
+        const auto kern = layout == BB_NT   ? gemm_f32_grouped_kernel<false, false>
+                          : layout == BB_NN ? waves ? gemm_f32_wave_grouped_kernel<false, true> : gemm_f32_grouped_kernel<false, true>
+                                            : waves ? gemm_f32_wave_grouped_kernel<true, true> : gemm_f32_grouped_kernel<true, true>;
+        bb_launch(kern, dim3(blocks), dim3(256), waves ? kF32WaveLds : f32_gemm_lds(64), st, G);
         BB_LAUNCH_CHECK();
         return BB_OK;
     }

@@ -1,5 +1,5 @@
-// fp32 GEMM: v_mfma_f32_32x32x2_f32 on 64x64 tiles (four waves of 32x32), or on 64x32 tiles whose contraction two groups of
-// two waves share.
+// fp32 GEMM: v_mfma_f32_32x32x2_f32 on 64x64 tiles (four waves of 32x32), on 64x32 tiles whose contraction two groups of
+// two waves share, or on 32x32 tiles whose contraction four waves share.
 #pragma once
 #include "gemm_kernels.h"
 
@@ -14,12 +14,13 @@
 //   K-contiguous memory: [rows][32 k], 128 B a row = 8 chunks of 16 B, chunk c of row r at c ^ ((r >> 1) & 7).
 //   k-major memory: [32 k][rows]; 64-row tiles keep rows 0..31 of odd k at the place of rows 32..63 and vice versa, so that
 //     the two halves of a wave (k and k + 1) read different banks.
-// Every element adds up its contraction in pairs (k, k + 1), k ascending (groups: the even, resp. odd 16-wide k-tiles, group
-// 0's sum plus group 1's), whatever the tile: which kernel runs a problem changes no bit.
+// Every element adds up its contraction in pairs (k, k + 1), k ascending; groups and waves each add up their share of it (the
+// even, resp. odd 16-wide k-tiles; one 32-wide slice) and the shares' sums are added in order.  Which kernel runs a
+// problem is a matter of its shape and layout alone.
 // (volatile: pairs of reads merged into one instruction have no room for the stage's offset, i.e. cost an addition each)
 typedef const volatile __attribute__((address_space(3))) float lds_f32;
-template <int ROWS, bool KM> struct F32Operand {
-    static constexpr int BYTES = ROWS * 32 * 4, ROUNDS = BYTES / (1024 * 4);   // four waves load a stage
+template <int ROWS, bool KM, int NW = 4> struct F32Operand {
+    static constexpr int BYTES = ROWS * 32 * 4, ROUNDS = BYTES / (1024 * NW);   // NW waves load a stage
     const float* base;          // wave-uniform: the tile's first row (K-contiguous) / column (k-major), the next k-tile
     unsigned off[ROUNDS];       // the lane's 16 bytes from there
     int k_lane[ROUNDS];         // ... and their k inside a k-tile
@@ -28,7 +29,7 @@ template <int ROWS, bool KM> struct F32Operand {
         base = p + (KM ? row0 : (int64_t)row0 * ld);
 #pragma unroll
         for (int i = 0; i < ROUNDS; ++i) {
-            const int q = i * 4 + wave;
+            const int q = i * NW + wave;
             if constexpr (!KM) {
                 const int r = q * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
                 k_lane[i] = c * 4;
@@ -47,11 +48,11 @@ template <int ROWS, bool KM> struct F32Operand {
         if (left >= 32) {
 #pragma unroll
             for (int i = 0; i < ROUNDS; ++i)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + (i * 4 + wave) * 1024), "v"(off[i]), "s"(base) : "m0");
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + (i * NW + wave) * 1024), "v"(off[i]), "s"(base) : "m0");
         } else {
 #pragma unroll
             for (int i = 0; i < ROUNDS; ++i)
-                dma16_at(k_lane[i] < left ? (const unsigned char*)base + off[i] : bb_zero_line + (lane & 7) * 16, lds + (i * 4 + wave) * 1024);
+                dma16_at(k_lane[i] < left ? (const unsigned char*)base + off[i] : bb_zero_line + (lane & 7) * 16, lds + (i * NW + wave) * 1024);
         }
         base += step;
     }
@@ -83,44 +84,45 @@ template <int ROWS, bool KM, int NC> struct F32Reader {
 constexpr int f32_stages(int bn) { return bn == 64 ? 2 : 3; }
 constexpr int f32_gemm_lds(int bn) { return f32_stages(bn) * (64 + bn) * 128; }
 
-// The epilogue of a lane's sixteen elements (one column; register r: row m + 8 (r / 4) + r % 4).  `pre`: what it reads beside
+// The epilogue of a lane's NR elements -- sixteen, or four of a tile that several waves finish -- (one column; register r: row m + 8 (r / 4) + r % 4).  `pre`: what it reads beside
 // the product -- the operand of the epilogue kind, else the C it accumulates into -- fetched before the main loop; `rest`: a
-// problem that reads both, or a masked residual, fetches the second here.  One branch over the kind around the sixteen, not
+// problem that reads both, or a masked residual, fetches the second here.  One branch over the kind around them, not
 // inside: the code stays small.
-__device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, int m0, int n, float bias, const float (&pre)[16], f32x16& v) {
+template <int NR, typename V>
+__device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, int m0, int n, float bias, const float (&pre)[NR], V& v) {
     const auto row = [&](int r) { return m0 + 8 * (r >> 2) + (r & 3); };
     const bool has_opnd = epilogue_operand(g) != nullptr;
-    float rest[16], keep[16];
+    float rest[NR], keep[NR];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
+    for (int r = 0; r < NR; ++r) {
         rest[r] = pre[r];
         keep[r] = 1.0f;
     }
     if (has_opnd && g.accumulate) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) rest[r] = ((const float*)g.C)[coff + (int64_t)min(row(r), g.M - 1) * g.ldc + n];
+        for (int r = 0; r < NR; ++r) rest[r] = ((const float*)g.C)[coff + (int64_t)min(row(r), g.M - 1) * g.ldc + n];
     } else if (g.epilogue == BB_EPI_MUL_POS && g.resid) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) rest[r] = ((const float*)g.resid)[coff + (int64_t)min(row(r), g.M - 1) * g.ldaux + n];
+        for (int r = 0; r < NR; ++r) rest[r] = ((const float*)g.resid)[coff + (int64_t)min(row(r), g.M - 1) * g.ldaux + n];
     }
     if (g.drop.thresh) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) keep[r] = drop_factor(g, row(r), n);
+        for (int r = 0; r < NR; ++r) keep[r] = drop_factor(g, row(r), n);
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = v[r] * g.alpha + bias;
+    for (int r = 0; r < NR; ++r) v[r] = v[r] * g.alpha + bias;
     float* aux = (float*)g.aux_out + coff + n;
     if (g.epilogue == BB_EPI_ACT) {
         if (g.aux_out) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
+            for (int r = 0; r < NR; ++r)
                 if (row(r) < g.M) aux[(int64_t)row(r) * g.ldaux] = v[r];
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = act_f(v[r], g.act) * keep[r];
+        for (int r = 0; r < NR; ++r) v[r] = act_f(v[r], g.act) * keep[r];
     } else if (g.epilogue == BB_EPI_ACT_DACT) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+        for (int r = 0; r < NR; ++r) {
             float a, d;
             act_dact_f(v[r], g.act, a, d);
             if (row(r) < g.M) aux[(int64_t)row(r) * g.ldaux] = d * keep[r];
@@ -128,23 +130,23 @@ __device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, in
         }
     } else if (g.epilogue == BB_EPI_DACT) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] *= dact_f(pre[r], g.act);
+        for (int r = 0; r < NR; ++r) v[r] *= dact_f(pre[r], g.act);
     } else if (g.epilogue == BB_EPI_RESIDUAL) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = v[r] * keep[r] + pre[r];
+        for (int r = 0; r < NR; ++r) v[r] = v[r] * keep[r] + pre[r];
     } else if (g.epilogue == BB_EPI_MUL) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] *= pre[r];
+        for (int r = 0; r < NR; ++r) v[r] *= pre[r];
     } else if (g.epilogue == BB_EPI_MUL_POS) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = pre[r] > 0.f ? (g.resid ? v[r] + rest[r] : v[r]) : 0.f;
+        for (int r = 0; r < NR; ++r) v[r] = pre[r] > 0.f ? (g.resid ? v[r] + rest[r] : v[r]) : 0.f;
     } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] *= keep[r];
+        for (int r = 0; r < NR; ++r) v[r] *= keep[r];
     }
     float* c = (float*)g.C + coff + n;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
+    for (int r = 0; r < NR; ++r)
         if (row(r) < g.M) c[(int64_t)row(r) * g.ldc] = g.accumulate ? rest[r] + v[r] : v[r];
 }
 
@@ -277,7 +279,7 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[r] += part[r * 64 + lane];
     }
-    if (n < g.N) epilogue_f32(g, coff, acc_m, n, bias, pre, acc);
+    if (n < g.N) epilogue_f32<16>(g, coff, acc_m, n, bias, pre, acc);
 }
 
 template <bool TA, bool TB, int BN>
@@ -291,4 +293,96 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_grouped_kernel(const GroupedA
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
     gemm_f32_body<TA, TB, 64>(G.p[pi], lid - G.first_block[pi], 0, true);
+}
+
+// Problems of few tiles and a contraction of at most 128: 32x32 tiles, each of the four waves of a block one 32-wide slice.
+// What bounds such a problem is a chain -- per k-tile a wait for the loads, a barrier and 1024 cycles of dependent matrix
+// instructions, on a handful of CUs.  Here everything is in flight at once, nobody waits for anybody, and the chain is one
+// slice long on four times the CUs; the four partial tiles meet in LDS, are added in wave order, and each wave finishes eight
+// rows.  (us against the 64x64 tiles: see pick_f32_wave; the error against 64 bits at K = 128: 2.0e-7 -> 1.1e-7.)
+constexpr int kF32Waves = 4, kF32WaveK = kF32Waves * 32;
+constexpr int kF32WaveLds = kF32Waves * 2 * 32 * 128;
+template <bool TA, bool TB>
+__device__ __forceinline__ void gemm_f32_wave_body(const GemmArgs& g, const int block_id, const int batch_id, const bool logical_id) {
+    using OpA = F32Operand<32, TA, 1>;
+    using OpB = F32Operand<32, TB, 1>;
+    constexpr int KW = kF32Waves, SLICE = OpA::BYTES + OpB::BYTES;
+    static_assert(KW * SLICE == kF32WaveLds && SLICE >= 32 * 32 * 4, "a wave's partial tile takes the place of its slice");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int tile_m, tile_n;
+    if (logical_id) panel_coords(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    else tile_coords(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    const int m0 = tile_m * 32, n0 = tile_n * 32;
+    const int b1 = batch_id / g.nb2, b2 = batch_id % g.nb2;
+    const int64_t coff = b1 * g.sC1 + b2 * g.sC2;
+    OpA opa;
+    OpB opb;
+    opa.init((const float*)g.A + b1 * g.sA1 + b2 * g.sA2, g.lda, m0, g.M, lane, 0);
+    opb.init((const float*)g.B + b1 * g.sB1 + b2 * g.sB2, g.ldb, n0, g.N, lane, 0);
+    opa.base += wave * opa.step;
+    opb.base += wave * opb.step;
+    const unsigned lds = (unsigned)(uintptr_t)(lds_ptr_t*)smem + wave * SLICE;
+    F32Reader<32, TA, 8> ra;
+    F32Reader<32, TB, 8> rb;
+    ra.init(lds, 0, 0, lane);
+    rb.init(lds + OpA::BYTES, 0, 0, lane);
+    const int left = g.K - wave * 32;
+    if (left > 0) {
+        opa.issue(lds, 0, left, lane);
+        opb.issue(lds + OpA::BYTES, 0, left, lane);
+    }
+
+    // what the epilogue reads, for the rows this wave will finish: register e = row acc_m + e
+    const int n = n0 + (lane & 31), acc_m = m0 + 8 * wave + 4 * (lane >> 5), nc = min(n, g.N - 1);
+    const float* opnd = (const float*)epilogue_operand(g);
+    const int64_t ld_pre = opnd ? g.ldaux : g.ldc;
+    if (!opnd && g.accumulate) opnd = (const float*)g.C;
+    const float bias = g.bias ? ((const float*)g.bias)[nc] : 0.f;
+    float pre[4] = {0.f, 0.f, 0.f, 0.f};
+    if (opnd) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pre[e] = opnd[coff + (int64_t)min(acc_m + e, g.M - 1) * ld_pre + nc];
+    }
+
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if (left > 0) {
+        asm volatile("" ::: "memory");
+        wait_vmcnt_lgkm0<0>();
+        asm volatile("" ::: "memory");
+        float x[8][2], y[8][2];
+        ra.template load<0, 0>(x);
+        rb.template load<0, 0>(y);
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[c][i], y[c][i], acc, 0, 0, 0);
+    }
+
+    float* part = (float*)smem;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave * (SLICE / 4) + r * 64 + lane] = acc[r];
+    __syncthreads();
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = part[(4 * wave + e) * 64 + lane];
+#pragma unroll
+        for (int p = 1; p < KW; ++p) v[e] += part[p * (SLICE / 4) + (4 * wave + e) * 64 + lane];
+    }
+    if (n < g.N) epilogue_f32<4>(g, coff, acc_m, n, bias, pre, v);
+}
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 4) void gemm_f32_wave_kernel(const GemmArgs g) {
+    gemm_f32_wave_body<TA, TB>(g, blockIdx.x, blockIdx.z, false);
+}
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 4) void gemm_f32_wave_grouped_kernel(const GroupedArgs G) {
+    const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
+    int pi = 0;
+    while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
+    gemm_f32_wave_body<TA, TB>(G.p[pi], lid - G.first_block[pi], 0, true);
 }

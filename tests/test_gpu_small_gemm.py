@@ -1,4 +1,4 @@
-"""bf16 GEMMs of few tiles (contraction dealt to the waves of a block) and weight gradients over row counts that are no
+"""GEMMs of few tiles (contraction dealt to the waves of a block) and weight gradients over row counts that are no
 multiple of a k-tile, against fp64."""
 import pytest
 import torch
@@ -88,3 +88,54 @@ def test_conv_weight_gradient_over_ragged_pixels(hiplib, n, h, w, c, co):
         g = torch.zeros(co, 9 * c, device=DEV)
         hiplib.gemm_grouped([hiplib.gemm_desc(hiplib.TN, dy, x, g, accumulate=True, conv=(h, w))], splitk_ws=ws)
         assert rel(g, want) < 1e-5
+
+
+# One slice and a part of one, a ragged last slice, all four slices whole; fewer rows or columns than a tile, remainders, the
+# largest the rule takes (1024 tiles).  Sums of K products in fp32, K roundings at most: |error| <= K eps sum |a b| (eps = 2^-24).
+@pytest.mark.parametrize("M,N,K", [(4, 4, 4), (36, 28, 32), (32, 32, 36), (100, 72, 100), (128, 384, 128), (64, 128, 64), (8, 1024, 124),
+                                   (1024, 1024, 96)])
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+def test_fp32_products_of_few_tiles(hiplib, layout, M, N, K):
+    lay = {"nt": hiplib.NT, "nn": hiplib.NN, "tn": hiplib.TN}[layout]
+    mk = lambda *shape, seed: torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
+    A, B = mk(*((K, M) if layout == "tn" else (M, K)), seed=1), mk(*((N, K) if layout == "nt" else (K, N)), seed=2)
+    bias, X, G = mk(N, seed=3), mk(M, N, seed=4), mk(M, N, seed=5)
+    a, b = A.double().cpu(), B.double().cpu()
+    a, b = a.t() if layout == "tn" else a, b.t() if layout == "nt" else b
+    prod, bound = a @ b, (K + 4) * 2.0 ** -24 * (a.abs() @ b.abs() + bias.double().cpu().abs() + X.double().cpu().abs() + G.double().cpu().abs())
+    C = torch.full((M, N), float("nan"), device=DEV)
+    few = layout == "nn" or layout == "tn" and M * N < 1024 * 1024     # (a forward product keeps the larger tiles' order)
+    assert hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C)).endswith("wave32x32k4" if few else "64x64")
+    hiplib.gemm(lay, A, B, C, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X)
+    assert bool(((C.double().cpu() - (prod + bias.double().cpu() + X.double().cpu())).abs() <= bound).all())
+    acc = G.clone()
+    hiplib.gemm(lay, A, B, acc, accumulate=True)
+    assert bool(((acc.double().cpu() - (prod + G.double().cpu())).abs() <= bound).all())
+    if layout == "nt":
+        hiplib.gemm(lay, A, B, C, bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_RELU, aux_out=X)
+        u = prod + bias.double().cpu()
+        assert bool(((C.double().cpu() - u.clamp_min(0)).abs() <= bound).all()) and bool(((X.double().cpu() == (u > 0)) | (u.abs() <= bound)).all())
+    # a layer's problems in one launch give the bits they give alone, also beside one of many tiles
+    if layout == "tn":
+        for other in (64, 1024):
+            A2, one, two = mk(K, other, seed=6), G.clone(), torch.zeros(other, N, device=DEV)
+            big = torch.zeros(other, N, device=DEV)
+            hiplib.gemm(lay, A2, B, big, accumulate=True)
+            hiplib.gemm_grouped([hiplib.gemm_desc(lay, A, B, one, accumulate=True), hiplib.gemm_desc(lay, A2, B, two, accumulate=True)])
+            assert bool(((one.double().cpu() - (prod + G.double().cpu())).abs() <= bound).all())
+            if other == 64 and M * N < 1024 * 1024:
+                assert torch.equal(one, acc) and torch.equal(two, big)
+
+
+# the products of attention heads inside a [rows, 3 h] buffer, as one batched launch of few tiles
+@pytest.mark.parametrize("b,heads,seq", [(1, 1, 36), (2, 3, 64), (4, 2, 100), (1, 2, 512)])
+def test_fp32_batched_heads_of_few_tiles(hiplib, b, heads, seq):
+    d = 64
+    h = heads * d
+    qkv = torch.randn(b * seq, 3 * h, generator=torch.Generator().manual_seed(9)).to(DEV)
+    P = torch.empty(b, heads, seq, seq, device=DEV)
+    hiplib.gemm_batched(hiplib.NT, hiplib.dtype_code(torch.float32), seq, seq, d, qkv.data_ptr(), 3 * h, (seq * 3 * h, d), qkv.data_ptr() + 4 * h,
+                        3 * h, (seq * 3 * h, d), P.data_ptr(), seq, (heads * seq * seq, seq * seq), b, heads, alpha=0.125)
+    q, k = (qkv[:, i * h:(i + 1) * h].double().cpu().view(b, seq, heads, d).transpose(1, 2) for i in (0, 1))
+    bound = (d + 2) * 2.0 ** -24 * 0.125 * (q.abs() @ k.abs().transpose(-1, -2))
+    assert bool(((P.double().cpu() - 0.125 * q @ k.transpose(-1, -2)).abs() <= bound).all())
