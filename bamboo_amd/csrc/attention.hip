@@ -128,18 +128,36 @@ __device__ __forceinline__ bf16x8 pack_acc(const f32x16& a, int half) {
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 // Dropout over the sixteen accumulator registers of a lane whose rows acc_row(r, lane) are consecutive probability
 // indices from `base` on: registers 4g .. 4g + 3 hold four neighbouring indices, i.e. two hash pairs when the first is
-// even (every case with an even sequence length).  Kept values are scaled, dropped ones zeroed.
+// even (in every lane, where the sequence length is), else parts of three (12 heads x 2043^2 forward: 58 us; 85 where the lanes
+// of odd queries went another way).  Kept values are scaled, dropped ones zeroed.
 __device__ __forceinline__ void drop_acc_rows(const DropKey& k, uint64_t base, int lane, f32x16& v) {
-    const bool even = (base & 1) == 0;   // 8 g + 4 (lane >> 5) is even
-    if (k.small && even) {               // the rule: fewer than 2^32 probabilities, even sequence length
-        const uint32_t p0 = ((uint32_t)base >> 1) + 2 * (lane >> 5);
+    if (k.small) {                       // the rule: fewer than 2^32 probabilities
+        const uint32_t p0 = ((uint32_t)base >> 1) + 2 * (lane >> 5);   // 8 g + 4 (lane >> 5) is even
+        const bool odd = (base & 1) != 0;
+        if (__builtin_amdgcn_ballot_w64(odd) == 0) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint32_t x0 = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g), x1 = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g + 1);
+                v[4 * g] = bb_keep_even(x0, k.thresh) ? v[4 * g] * k.scale : 0.f;
+                v[4 * g + 1] = bb_keep_odd(x0, k.thresh) ? v[4 * g + 1] * k.scale : 0.f;
+                v[4 * g + 2] = bb_keep_even(x1, k.thresh) ? v[4 * g + 2] * k.scale : 0.f;
+                v[4 * g + 3] = bb_keep_odd(x1, k.thresh) ? v[4 * g + 3] * k.scale : 0.f;
+            }
+            return;
+        }
+        // an odd sequence length: every other query's row starts inside a pair
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const uint32_t x0 = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g), x1 = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g + 1);
-            v[4 * g] = bb_keep_even(x0, k.thresh) ? v[4 * g] * k.scale : 0.f;
-            v[4 * g + 1] = bb_keep_odd(x0, k.thresh) ? v[4 * g + 1] * k.scale : 0.f;
-            v[4 * g + 2] = bb_keep_even(x1, k.thresh) ? v[4 * g + 2] * k.scale : 0.f;
-            v[4 * g + 3] = bb_keep_odd(x1, k.thresh) ? v[4 * g + 3] * k.scale : 0.f;
+            uint32_t x[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) x[j] = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g + j);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                // the 16 bits of element e: half e % 2 of pair e / 2, or of the one further on where the first index is odd
+                const uint32_t even_bits = e & 1 ? x[e >> 1] >> 16 : x[e >> 1] & 0xffffu;
+                const uint32_t odd_bits = e & 1 ? x[(e + 1) >> 1] & 0xffffu : x[e >> 1] >> 16;
+                v[4 * g + e] = (odd ? odd_bits : even_bits) >= k.thresh ? v[4 * g + e] * k.scale : 0.f;
+            }
         }
         return;
     }
@@ -487,32 +505,50 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
             }
             // dropout: dP = dP~ o mask / (1 - p) before it meets P; P itself is masked (into what multiplied V in
             // the forward) only after dS has been formed from the unmasked probabilities
-            unsigned kept = 0xffffu;
+            unsigned kept = 0u;   // bit r (sixteen booleans cost the registers that K, V and the sums leave)
             if (DROP && a.drop.thresh) {
                 asm volatile("" ::: "memory");
                 const int qlane = t * 64 + u * 32 + 4 * (lane >> 5);
-                kept = 0u;
                 if (a.drop.small) {
-                    // 32-bit indices; a query past the end is masked out above, what is decided for it does not matter
-                    const uint32_t i0 = ((uint32_t)(b * a.heads + head) * (uint32_t)a.seq + (uint32_t)qlane) * (uint32_t)a.seq +
-                                        (uint32_t)min(mykv, last);
+                    // 32-bit indices; what is decided for a query past the end (masked out above) or a key past it (a whole
+                    // lane, never stored) does not matter
+                    const uint32_t i0 = ((uint32_t)(b * a.heads + head) * (uint32_t)a.seq + (uint32_t)qlane) * (uint32_t)a.seq + (uint32_t)mykv;
+                    if (a.seq % 2 == 0) {
+                        // Rows start even: lanes 2j and 2j + 1 (keys 2j, 2j + 1) need the two halves of one hash in every row.
+                        // Of two rows the even lane hashes the first and the odd lane the second, and they exchange the
+                        // other's halves: a hash (two quarter-rate multiplies) per two decisions, as where the indices of a
+                        // lane are neighbours.  (Backward of 8 x 16 heads x 1024^2 probabilities: 238 us with a hash per decision,
+                        // 223 with this; 128-wide heads, 2 x 8 x 512^2 causal: 89 and 67.)
+                        const uint32_t own = (lane & 1) * 16, other = 16 - own;
+                        const uint32_t j0 = i0 + (lane & 1) * (uint32_t)a.seq;
+                        uint32_t km = 0u, kt = 0u;   // bit r: this lane's decision of its row, the neighbour's row
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const uint32_t idx = i0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq;
-                        const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, idx >> 1);
-                        const bool keep = (idx & 1) ? bb_keep_odd(x, a.drop.thresh) : bb_keep_even(x, a.drop.thresh);
-                        kept |= keep ? 1u << r : 0u;
-                        dp[r] = keep ? dp[r] * a.drop.scale : 0.f;
+                        for (int r = 0; r < 16; r += 2) {
+                            const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, (j0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq) >> 1);
+                            const bool mine = ((x >> own) & 0xffffu) >= a.drop.thresh;
+                            const uint32_t sent = (uint32_t)__builtin_amdgcn_mov_dpp((int)((x >> other) & 0xffffu), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true);
+                            const bool theirs = sent >= a.drop.thresh;
+                            km |= mine ? 1u << r : 0u;
+                            kt |= theirs ? 1u << r : 0u;
+                        }
+                        kept = (lane & 1) ? km << 1 | kt : km | kt << 1;
+                    } else {
+#pragma unroll 2                        // (unrolled whole, this and the next loop cost the first one's registers)
+                        for (int r = 0; r < 16; ++r) {
+                            const uint32_t idx = i0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq;
+                            const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, idx >> 1);
+                            kept |= (((x >> ((idx & 1) * 16)) & 0xffffu) >= a.drop.thresh ? 1u : 0u) << r;
+                        }
                     }
                 } else {
-#pragma unroll
+#pragma unroll 1
                     for (int r = 0; r < 16; ++r) {
                         const int q = min(qlane + 8 * (r >> 2) + (r & 3), last);
-                        const bool keep = bb_dropout_keep(a.drop.k0, a.drop.k1, a.drop.thresh, prob_index(a, b, head, q) + min(mykv, last));
-                        kept |= keep ? 1u << r : 0u;
-                        dp[r] = keep ? dp[r] * a.drop.scale : 0.f;
+                        kept |= (bb_dropout_keep(a.drop.k0, a.drop.k1, a.drop.thresh, prob_index(a, b, head, q) + min(mykv, last)) ? 1u : 0u) << r;
                     }
                 }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dp[r] = (kept >> r) & 1u ? dp[r] * a.drop.scale : 0.f;
             }
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
