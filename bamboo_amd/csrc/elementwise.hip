@@ -1242,7 +1242,9 @@ __global__ __launch_bounds__(256) void bn_finish_kernel(int what, int rows, int 
 // block: all row ranges of a channel normalise with the same bits).  The block of the first row range also writes
 // mean, rstd and the running statistics.  Then y = gamma (x - mean) rstd + beta (+ resid) (ReLU) over the block's
 // rows, eight lanes per row of the 64 channels (128-byte segments).  The tensor is read once; repeating the small
-// strip reduction per row range is cheaper than a launch of its own.
+// strip reduction per row range is cheaper than a launch of its own.  (For few rows that reduction is what the launch waits for:
+// loads for all 256 strips / for the sixteens there are, us: 900 rows x 512 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 / 6.5;
+// the rows of a thread fetched ahead, all of them or the next one, gained nothing.)
 constexpr int BN_STRIP_WAVES = 16, BN_STRIP_MAX = 16;   // 16 * 16 strips = up to 8192 rows
 constexpr int BN_FWD_ROW_RANGES = 64;
 __global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int rows, int cols, float eps, float momentum, int relu,
@@ -1269,11 +1271,14 @@ __global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int 
     float p[BN_STRIP_MAX], a[BN_STRIP_MAX], b[BN_STRIP_MAX];
 #pragma unroll
     for (int j = 0; j < BN_STRIP_MAX; ++j) {
-        const int s = min(j * BN_STRIP_WAVES + wave, nstrips - 1);   // clamped: every load is issued, unused ones get n = 0
-        const float* t = strips + ((int64_t)s * 3) * cols + c;
-        p[j] = t[0];
-        a[j] = t[cols];
-        b[j] = t[2 * (int64_t)cols];
+        p[j] = a[j] = b[j] = 0.f;
+        if (j * BN_STRIP_WAVES < nstrips) {   // (the same in all waves: a scalar branch, and the loads inside still go out together)
+            const int s = min(j * BN_STRIP_WAVES + wave, nstrips - 1);   // clamped: unused ones get n = 0
+            const float* t = strips + ((int64_t)s * 3) * cols + c;
+            p[j] = t[0];
+            a[j] = t[cols];
+            b[j] = t[2 * (int64_t)cols];
+        }
     }
     float sm = 0.f;
 #pragma unroll
