@@ -287,7 +287,13 @@ __device__ __forceinline__ float sum_partials(const float* __restrict__ src, int
 #pragma unroll
         for (int j = 0; j < 8; ++j) s += v[j];
     }
-    for (; p < nparts; p += step) s += src[(int64_t)p * stride];
+    if (p < nparts) {   // the last few go out together as well
+        float v[7];
+#pragma unroll
+        for (int j = 0; j < 7; ++j) v[j] = p + j * step < nparts ? src[(int64_t)(p + j * step) * stride] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 7; ++j) s += v[j];
+    }
     return s;
 }
 constexpr int RED_WAVES = 16;
@@ -344,14 +350,18 @@ static int ln_fwd_launch(int kind, int rows, int cols, float eps, const void* x,
 }
 template <typename T, int IT>
 static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const float* mean,
-                         const float* rinv, const void* dy, const void* dres, void* dx, float* ws, hipStream_t st) {
+                         const float* rinv, const void* dy, const void* dres, void* dx, float* ws, int& blocks, hipStream_t st) {
     constexpr int LN_BWD_WAVES = ln_bwd_waves<T, IT>();
+    // a row per wave: blocks past the last row would only write zeros for the reduction to read (us, backward with its
+    // reduction, 256 blocks / as many as have rows: bf16 128 x 128 6.4 / 5.8, 300 x 768 8.5 / 7.5, 1024 x 512 7.2 / 6.7, 333 x 5120
+    // 61 / 49; from 4096 rows on all have)
+    blocks = min(LN_BWD_BLOCKS, (rows + LN_BWD_WAVES - 1) / LN_BWD_WAVES);
     const size_t all = (size_t)LN_BWD_WAVES * 2 * cols * sizeof(float);
     const int one_pass = all <= 128 * 1024;
     const size_t smem = one_pass ? all : (size_t)3 * 2 * cols * sizeof(float);
     auto kern = layernorm_bwd_kernel<T, IT>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));   // raised on the first (never captured) call that needs it
-    bb_launch(kern, dim3(LN_BWD_BLOCKS), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
+    bb_launch(kern, dim3(blocks), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
                        (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -402,9 +412,10 @@ static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, 
     BB_REQUIRE(x && gain && mean && rinv && dy && dx && dgain && dshift && workspace, "%s: null pointer", who);
     BB_REQUIRE((size_t)3 * 2 * cols * sizeof(float) <= 160 * 1024, "%s: cols (%d) too large (max 6826)", who, cols);
     if (rows == 0) return BB_OK;
+    int blocks = 0;
     auto finish = [&]() -> int {
         const int nb = (cols + 63) / 64;
-        bb_launch(reduce_partials_acc2_kernel, dim3(nb, 2), dim3(RED_WAVES * 64), 0, st, workspace, LN_BWD_BLOCKS,
+        bb_launch(reduce_partials_acc2_kernel, dim3(nb, 2), dim3(RED_WAVES * 64), 0, st, workspace, blocks,
                            (int64_t)2 * cols, cols, dgain, dshift);
         BB_LAUNCH_CHECK();
         return BB_OK;
@@ -414,9 +425,9 @@ static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, 
         return r ? r : finish();
     };
     if (dtype == BB_BF16)
-        BB_DISPATCH_IT(bf16, cols / 8, run(ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, st)));
+        BB_DISPATCH_IT(bf16, cols / 8, run(ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
     else
-        BB_DISPATCH_IT(float, cols / 4, run(ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, st)));
+        BB_DISPATCH_IT(float, cols / 4, run(ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
     return BB_EINVAL;
 }
 
