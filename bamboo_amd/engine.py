@@ -472,7 +472,7 @@ class PipelineEngine:
         change between batches, or replay what it launched.  ``slot`` = (kind, stage, micro-batch), ``operands``: what
         identifies the buffers behind the recorded pointers.  A pass has 8 to 20 launches per layer, at about 10 us of host
         time each through the layer code and 2 us from the recorded plan: stages of small layers are bound by that
-        (one layer of 128 columns, 4 micro-batches: 1.09 ms a batch issued from here, see _work of a pass in plan.hip)."""
+        (one layer of 128 columns, 4 micro-batches: 1.09 ms a batch issued from here, 0.45 ms replayed)."""
         if ctx.gemm_hook is not None:
             return issue()
         if self.use_graphs:
