@@ -27,12 +27,15 @@ struct AdamTable {
     int first_block[ADAM_MAX_TENSORS + 1];
     int count;
 };
+template <> struct BbPointersAt<AdamTable> : BbPointerRun<5 * ADAM_MAX_TENSORS> {};   // g, p, m, v, lowp
+static_assert(offsetof(AdamTable, size) == 5 * ADAM_MAX_TENSORS * sizeof(void*), "BbPointersAt<AdamTable>");
 
 struct AdamHyper {
     float lr, beta1, beta2, eps, bc1, bc2, wd;
     int mode, zero_grad;
     const float* gscale;  // device scalar every gradient is multiplied by first (gradient clipping), or null
 };
+template <> struct BbPointersAt<AdamHyper> { uint16_t at[1] = {offsetof(AdamHyper, gscale)}; };
 
 // The update is written with contraction disabled so that every operation rounds exactly as in
 // the scalar statement of the formula (multiply and add are not fused into an FMA).

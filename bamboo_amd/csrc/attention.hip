@@ -41,6 +41,8 @@ struct AttnArgs {
     DropKey drop;                                  // dropout on the probabilities (thresh 0: none)
 };
 template <> struct BbDropAt<AttnArgs> { static constexpr int32_t value = offsetof(AttnArgs, drop); };
+template <> struct BbPointersAt<AttnArgs> : BbPointerRun<12> {};   // q .. key_len
+static_assert(offsetof(AttnArgs, ld_qkv) == 12 * sizeof(void*), "BbPointersAt<AttnArgs>");
 // index of probability (b, head, q, kv) in the [batch, heads, seq, seq] tensor that is never stored
 __device__ __forceinline__ uint64_t prob_index(const AttnArgs& a, int b, int head, int q) {
     return ((uint64_t)(b * a.heads + head) * a.seq + q) * a.seq;

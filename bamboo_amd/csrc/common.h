@@ -1,12 +1,14 @@
 // Shared device/host helpers for the gfx950 kernels of libbamboo_hip.so.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string.h>
 
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <unordered_map>
 #include <utility>
 
@@ -222,14 +224,46 @@ static inline DropKey bb_drop_key(float p, uint32_t k0, uint32_t k1, uint64_t nu
 // ---- kernel launches -----------------------------------------------------------------------
 // Every launch of the library goes through bb_launch.  While the calling thread records a launch plan (plan.hip), the
 // launch is also copied into it -- kernel, grid, argument bytes --, so that a fixed sequence can be issued again later
-// without its callers.  BbDropAt<T>: where an argument type carries a dropout key (-1: nowhere), the one thing in such a
-// sequence that changes from replay to replay.
+// without its callers.  What may change from replay to replay is found by the arguments' types: BbDropAt<T> says where a
+// type carries a dropout key (-1: nowhere), BbPointersAt<T>::at where it carries device pointers.  Never by looking at the
+// bytes: two neighbouring 32-bit sizes can look like an address.
 struct BbPlan;
 extern thread_local BbPlan* bb_recording;
-void bb_record_launch(const void* fn, dim3 grid, dim3 block, size_t lds, int nargs, void* const* args, const uint32_t* sizes,
-                      const int32_t* drop_at);
+struct BbArgType {
+    uint32_t size;
+    int32_t drop_at;
+    uint32_t pointers;
+    const uint16_t* pointer_at;
+};
+void bb_record_launch(const void* fn, dim3 grid, dim3 block, size_t lds, int nargs, void* const* args, const BbArgType* types);
 template <typename T> struct BbDropAt { static constexpr int32_t value = -1; };
 template <> struct BbDropAt<DropKey> { static constexpr int32_t value = 0; };
+struct BbNoPointers {};
+// a struct that is a kernel argument says what it holds: a specialisation with `at`, or one derived from BbNoPointers
+template <typename T> struct BbPointersAt { static_assert(std::is_scalar<T>::value, "kernel argument: specialise BbPointersAt"); };
+template <> struct BbPointersAt<DropKey> : BbNoPointers {};
+// COUNT pointers one after the other, from the struct's start on
+template <int COUNT> struct BbPointerRun {
+    uint16_t at[COUNT];
+    constexpr BbPointerRun() : at{} {
+        for (int i = 0; i < COUNT; ++i) at[i] = (uint16_t)(i * sizeof(void*));
+    }
+};
+template <typename T> static BbArgType bb_arg_type() {
+    BbArgType t = {(uint32_t)sizeof(T), BbDropAt<T>::value, 0u, nullptr};
+    if constexpr (std::is_pointer<T>::value) {
+        static constexpr uint16_t first[] = {0};
+        t.pointers = 1;
+        t.pointer_at = first;
+    } else if constexpr (std::is_class<T>::value && !std::is_base_of<BbNoPointers, BbPointersAt<T>>::value) {
+        static constexpr BbPointersAt<T> where;
+        t.pointers = (uint32_t)(sizeof(where.at) / sizeof(uint16_t));
+        t.pointer_at = where.at;
+    } else {
+        (void)sizeof(BbPointersAt<T>);
+    }
+    return t;
+}
 
 template <typename... P, size_t... I>
 static inline void bb_launch_tuple(void (*kern)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, std::tuple<P...>& a,
@@ -237,9 +271,8 @@ static inline void bb_launch_tuple(void (*kern)(P...), dim3 grid, dim3 block, si
     void* args[] = {(void*)&std::get<I>(a)...};
     (void)hipLaunchKernel((const void*)kern, grid, block, args, lds, st);   // BB_LAUNCH_CHECK reads the error
     if (bb_recording) {
-        const uint32_t sizes[] = {(uint32_t)sizeof(P)...};
-        const int32_t drop_at[] = {BbDropAt<P>::value...};
-        bb_record_launch((const void*)kern, grid, block, lds, (int)sizeof...(P), args, sizes, drop_at);
+        const BbArgType types[] = {bb_arg_type<P>()...};
+        bb_record_launch((const void*)kern, grid, block, lds, (int)sizeof...(P), args, types);
     }
 }
 template <typename... P, typename... A>
@@ -261,4 +294,6 @@ struct BbColsumGroup {
     int64_t ldx[BB_COLSUM_GROUP];
     int rows[BB_COLSUM_GROUP], cols[BB_COLSUM_GROUP], first_block[BB_COLSUM_GROUP + 1], count;
 };
+template <> struct BbPointersAt<BbColsumGroup> : BbPointerRun<3 * BB_COLSUM_GROUP> {};   // x, partial, out
+static_assert(offsetof(BbColsumGroup, ldx) == 3 * BB_COLSUM_GROUP * sizeof(void*), "BbPointersAt<BbColsumGroup>");
 int bb_colsum_acc_grouped(BbColsumGroup& G, hipStream_t st);

@@ -743,6 +743,8 @@ struct SplitkReduceArgs {
     int M[GROUP_MAX], N[GROUP_MAX], accumulate[GROUP_MAX];
     int splits;
 };
+template <> struct BbPointersAt<SplitkReduceArgs> : BbPointerRun<2 * GROUP_MAX> {};   // ws, C
+static_assert(offsetof(SplitkReduceArgs, ldc) == 2 * GROUP_MAX * sizeof(void*), "BbPointersAt<SplitkReduceArgs>");
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitkReduceArgs a) {
     const int pi = blockIdx.y;
     const int M = a.M[pi], N = a.N[pi], splits = a.splits, accumulate = a.accumulate[pi];

@@ -20,6 +20,11 @@ struct GemmArgs {
     DropKey drop;        // dropout on the product after bias and activation, before the residual (thresh 0: none)
 };
 template <> struct BbDropAt<GemmArgs> { static constexpr int32_t value = offsetof(GemmArgs, drop); };
+template <> struct BbPointersAt<GemmArgs> {
+    uint16_t at[9] = {offsetof(GemmArgs, A), offsetof(GemmArgs, B), offsetof(GemmArgs, C), offsetof(GemmArgs, bias), offsetof(GemmArgs, aux_in),
+                      offsetof(GemmArgs, aux_out), offsetof(GemmArgs, resid), offsetof(GemmArgs, colsum), offsetof(GemmArgs, strip_stats)};
+};
+static_assert(sizeof(GemmArgs) == 240, "a new member of GemmArgs: a pointer belongs in BbPointersAt<GemmArgs>");
 // Backward statistics of the batch normalisation whose (ReLU'd) output the product is the gradient of: the kernels
 // built with STATS = 2 leave, per 32-row strip and column, sum g and sum g * xhat of the stored (masked, bf16-rounded)
 // gradient g, with xhat = (x - mean) * rstd of the normalisation's input x ([M, N], rows ldc apart like C).
@@ -29,6 +34,8 @@ struct BnBwdArgs {
     const float* rstd;
     float* strips;   // [ceil(M / 32)][2][N]
 };
+template <> struct BbPointersAt<BnBwdArgs> : BbPointerRun<4> {};
+static_assert(sizeof(BnBwdArgs) == 4 * sizeof(void*), "BbPointersAt<BnBwdArgs>");
 // keep-and-scale factor of element (m, n) of the [M, N] product
 __device__ __forceinline__ float drop_factor(const GemmArgs& g, int m, int n) {
     return bb_dropout_keep(g.drop.k0, g.drop.k1, g.drop.thresh, (uint64_t)m * (uint64_t)g.N + (uint64_t)n) ? g.drop.scale : 0.f;
@@ -428,6 +435,7 @@ struct ConvArgs {
     int b_every;      // input-gradient mode: k-tiles per tap of the B operand ...
     int64_t b_wrap;   // ... and what its pointers move by (on top of the k-tile step) when the tap changes
 };
+template <> struct BbPointersAt<ConvArgs> : BbNoPointers {};
 // what the taps outside the image read
 __device__ __attribute__((aligned(128))) unsigned char bb_zero_line[128];
 
@@ -1385,6 +1393,14 @@ struct GroupedArgs {
     GemmArgs p[GROUP_MAX];
     int first_block[GROUP_MAX + 1];
     int count;
+};
+template <> struct BbPointersAt<GroupedArgs> {
+    static constexpr int EACH = sizeof(BbPointersAt<GemmArgs>::at) / sizeof(uint16_t);
+    uint16_t at[GROUP_MAX * EACH];
+    constexpr BbPointersAt() : at{} {
+        const BbPointersAt<GemmArgs> one;
+        for (int i = 0; i < GROUP_MAX * EACH; ++i) at[i] = (uint16_t)(offsetof(GroupedArgs, p) + i / EACH * sizeof(GemmArgs) + one.at[i % EACH]);
+    }
 };
 // CONVB: some problems of the group read their B operand as the patch matrix of a 3x3 convolution
 template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, bool CONVB = false>

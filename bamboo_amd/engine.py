@@ -31,6 +31,7 @@ from .config import BambooConfig
 from .module import MirrorBuffer, PipelineError, PipelineModule, flat_mirror
 from .optim import FusedAdam
 from .p2p import AllReduceException, NextStageException, PrevStageException, SeededActivationQueue  # noqa: F401
+from .replay import Replay, form
 from .utils import get_redundant_stage_ids, get_redundant_user_stage_ids
 
 class PipelineEngine:
@@ -103,9 +104,10 @@ class PipelineEngine:
             raise PipelineError("use_graphs needs the engine built and run under a created stream "
                                 "(torch.cuda.stream(...)): the default stream cannot be captured")
         self._graphs = {}
-        # What every pass of (stage, micro-batch) launches is recorded when the pass is issued for the first time and
-        # replayed by one native call from then on (hip.Plan; see _issue): {(kind, stage, micro-batch): {operands: (plan, out)}}
-        self._plans = {}
+        # what every pass of (stage, micro-batch) launches is recorded when the pass is issued for the first time and
+        # replayed by one native call from then on (see _issue)
+        self._replay = Replay(model)
+        self._plans = self._replay.plans
         self.rc_stream = torch.cuda.Stream(self.device) if (rc_stream and self.r_stage_ids and eager_recovery) else None
         # When a redundant forward is issued (results never depend on it, only timing):
         #   "reference": where EagerRecoverySchedule puts it, in front of the own step that waits for a gradient
@@ -464,37 +466,23 @@ class PipelineEngine:
         self._install_sched_generator()
 
     # ------------------------------------------------------------------ replay
-    PLAN_VARIANTS = 4     # operand sets remembered per (kind, stage, micro-batch): a queue that hands out other buffers
-    #                       in every batch costs a recording each time, not memory
+    PLAN_VARIANTS = Replay.VARIANTS
 
-    def _issue(self, slot, operands, ctx, issue):
-        """Run ``issue()``, which only launches kernels of this library on ``ctx.stream`` and returns a value that does not
-        change between batches, or replay what it launched.  ``slot`` = (kind, stage, micro-batch), ``operands``: what
-        identifies the buffers behind the recorded pointers.  A pass has 8 to 20 launches per layer, at about 10 us of host
-        time each through the layer code and 2 us from the recorded plan: stages of small layers are bound by that
-        (one layer of 128 columns, 4 micro-batches: 1.09 ms a batch issued from here, 0.45 ms replayed)."""
+    def _issue(self, slot, ctx, operands, variant, issue, layers=None):
+        """Run ``issue()``, which only launches kernels of this library on ``ctx.stream``, or replay what it launched.
+        ``slot`` = (kind, stage, micro-batch); ``operands``, ``variant``, ``layers`` (default: all of the stage's): see
+        :meth:`Replay.run`.  A pass has 8 to 20 launches per layer, at about 10 us of host time each through the layer code
+        and 2 us from the recorded plan: stages of small layers are bound by that (one layer of 128 columns, 4 micro-batches:
+        1.09 ms a batch issued from here, 0.45 ms replayed)."""
         if ctx.gemm_hook is not None:
             return issue()
         if self.use_graphs:
-            return self._graphed((slot, operands), ctx.stream, issue)
-        plans = self._plans.get(slot)
-        if plans is None:
-            plans = self._plans[slot] = {}
-        known = plans.get(operands)
-        if known is not None:
-            known[0].launch(self.global_steps, ctx.stream)
-            return known[1]
-        ctx.dropout_keys = {}
-        try:
-            with hip.Plan.record() as plan:
-                out = issue()
-            plan.dropout(ctx.dropout_keys)
-        finally:
-            ctx.dropout_keys = None
-        while len(plans) >= self.PLAN_VARIANTS:
-            del plans[next(iter(plans))]
-        plans[operands] = (plan, out)
-        return out
+            # a captured graph holds the addresses
+            key = (slot, ctx, variant) + tuple((form(t), None if t is None else t.data_ptr()) for t in operands)
+            return self._graphed(key, ctx.stream, issue)
+        if layers is None:
+            layers = (0, len(self.module.func_buckets[slot[1]]))
+        return self._replay.run(slot, ctx, operands, variant, layers, self.global_steps, issue)
 
     def _graphed(self, key, stream, issue):
         """:meth:`_issue` with HIP graphs: eagerly the first time ``key`` occurs, captured and launched the second time,
@@ -594,8 +582,6 @@ class PipelineEngine:
         ctx.dropout_base = (self.module.base_seed, self.global_steps, buffer_id)
         if redundant and self.rc_stream is not None:
             self.rc_stream.wait_event(self._fwd_done[buffer_id])
-        kl = ctx.key_len
-        operands = (id(ctx), inputs.data_ptr(), None if kl is None else kl.data_ptr(), redundant)
         # a redundant forward's stash is read by a backward pass only after a failover: it leaves out
         # what that backward pass can produce itself
         self._deferred[(stage_id, buffer_id)] = redundant
@@ -603,7 +589,7 @@ class PipelineEngine:
         if note_rc is not None:      # a queue that keeps a timeline of the redundant work (measurement only)
             note_rc(buffer_id, 0, "begin", ctx.stream)
         before = self.module.micro_offset
-        out = self._issue(("F", stage_id, buffer_id), operands, ctx,
+        out = self._issue(("F", stage_id, buffer_id), ctx, (inputs, ctx.key_len), redundant,
                           lambda: self.module.forward(inputs, stage_id, slot=buffer_id, ctx=ctx, defer=redundant))
         if self.module.micro_offset == before:
             self.module.note_replay(stage_id, buffer_id, inputs)
@@ -677,9 +663,9 @@ class PipelineEngine:
             note_rc = getattr(self.queue, "note_rc", None)
             if note_rc is not None:
                 note_rc(k, i, "begin", self.rc_stream)
-            kl, before = ctx.key_len, self.module.micro_offset
-            out = self._issue((f"F{i}", nxt, k), (id(ctx), x.data_ptr(), None if kl is None else kl.data_ptr(), True), ctx,
-                              lambda: self.module.forward(x, nxt, slot=k, ctx=ctx, defer=True, layers=(i, i + 1)))
+            before = self.module.micro_offset
+            out = self._issue((f"F{i}", nxt, k), ctx, (x, ctx.key_len), True,
+                              lambda: self.module.forward(x, nxt, slot=k, ctx=ctx, defer=True, layers=(i, i + 1)), layers=(i, i + 1))
             if i == 0 and self.module.micro_offset == before:
                 self.module.note_replay(nxt, k, x)
             if note_rc is not None:
@@ -745,11 +731,9 @@ class PipelineEngine:
         self.ctx.key_len = self.queue.key_len(buffer_id)
         self.ctx.dropout_base = (self.module.base_seed, self.global_steps, buffer_id)
         dst = self._input_grad_store[stage_id][buffer_id]
-        kl = self.ctx.key_len
         deferred = self._deferred.get((stage_id, buffer_id), False)
-        operands = (id(self.ctx), grad.data_ptr(), dst.data_ptr(), None if kl is None else kl.data_ptr(), deferred,
-                    self.module.input_ptr(stage_id, buffer_id))
-        self._issue(("B", stage_id, buffer_id), operands, self.ctx,
+        x = self.module.kept_input(stage_id, buffer_id)
+        self._issue(("B", stage_id, buffer_id), self.ctx, (grad, dst, self.ctx.key_len, x), deferred,
                     lambda: self.module.backward(grad, dst, stage_id, slot=buffer_id, ctx=self.ctx, deferred=deferred))
         key = f"input_grad_{stage_id}"
         if key in self.pipe_buffers:

@@ -26,7 +26,7 @@ EXPORTS = (
     "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
     "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
     "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
-    "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_launches", "bb_plan_launch", "bb_plan_destroy",
+    "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_operands", "bb_plan_launches", "bb_plan_launch", "bb_plan_launch_on", "bb_plan_destroy",
     "bb_adam_multi", "bb_adam_multi_scaled", "bb_grad_clip_workspace", "bb_grad_clip_coef", "bb_cast", "bb_fill_f32",
 )
 
@@ -114,8 +114,10 @@ def lib():
     L.bb_graph_destroy.argtypes = [c_void_p]
     L.bb_plan_end.argtypes = [POINTER(c_void_p)]
     L.bb_plan_dropout.argtypes = [c_void_p, c_int, POINTER(c_uint32), POINTER(c_uint32)] + [POINTER(c_int64)] * 4
+    L.bb_plan_operands.argtypes = [c_void_p, c_int, POINTER(c_uint64), POINTER(c_int64)]
     L.bb_plan_launches.argtypes = [c_void_p]
     L.bb_plan_launch.argtypes = [c_void_p, c_int64, c_void_p]
+    L.bb_plan_launch_on.argtypes = [c_void_p, c_int, POINTER(c_uint64), c_int64, c_void_p]
     L.bb_plan_destroy.argtypes = [c_void_p]
     L.bb_act_fwd.argtypes = [c_int, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]
     L.bb_bn_workspace.argtypes = [c_int]
@@ -180,6 +182,13 @@ def stream_ptr(stream=None):
 
 def _ptr(t):
     return None if t is None else c_void_p(t.data_ptr())
+
+
+def extent_bytes(t):
+    """Bytes from a strided tensor's first element to the end of its last one."""
+    if t.numel() == 0:
+        return 0
+    return (sum((n - 1) * abs(s) for n, s in zip(t.shape, t.stride())) + 1) * t.element_size()
 
 
 def _row_major(t, name):
@@ -587,10 +596,13 @@ class Graph:
 class Plan:
     """The launches one call makes, recorded while it makes them and issued again by one call (``with Plan.record() as
     plan: ...``, then ``plan.launch(step, stream)``).  ``plan.dropout(keys)`` names the dropout keys among the recorded
-    arguments: ``{(k0, k1): (base_seed, micro_batch, layer, site)}``; a launch derives them anew for its ``step``."""
+    arguments: ``{(k0, k1): (base_seed, micro_batch, layer, site)}``; a launch derives them anew for its ``step``.
+    ``plan.operands(tensors)`` names what the call was given, as opposed to what it keeps: ``launch(..., tensors=)`` then
+    puts the addresses of other tensors in their place.  These must be as the recorded ones in all but the address; the caller
+    sees to that (``replay.Replay``), the plan holds no reference to them."""
 
     def __init__(self):
-        self._plan = None
+        self._plan, self._addresses = None, ()
 
     class _Recording:
         def __init__(self, plan):
@@ -619,8 +631,18 @@ class Plan:
         k0, k1 = (c_uint32 * n)(*[k[0] for k in keys]), (c_uint32 * n)(*[k[1] for k in keys])
         check(lib().bb_plan_dropout(self._plan, n, k0, k1, *ids), "bb_plan_dropout")
 
-    def launch(self, step, stream):
-        check(lib().bb_plan_launch(self._plan, step, stream_ptr(stream)), "bb_plan_launch")
+    def operands(self, tensors):
+        n = len(tensors)
+        self._addresses = (c_uint64 * n)(*[t.data_ptr() for t in tensors])
+        check(lib().bb_plan_operands(self._plan, n, self._addresses, (c_int64 * n)(*[extent_bytes(t) for t in tensors])), "bb_plan_operands")
+
+    def launch(self, step, stream, tensors=()):
+        n = len(self._addresses)
+        if len(tensors) != n:
+            raise HipKernelError(f"plan: {n} operands expected, got {len(tensors)}")
+        for i, t in enumerate(tensors):
+            self._addresses[i] = t.data_ptr()
+        check(lib().bb_plan_launch_on(self._plan, n, self._addresses if n else None, step, stream_ptr(stream)), "bb_plan_launch_on")
 
     def __len__(self):
         return int(lib().bb_plan_launches(self._plan))

@@ -90,6 +90,10 @@ class StageContext:
         off = sum(hip.colsum_workspace(d.M) for d in wgrads)
         return self.workspace[off: off + hip.colsum_workspace(cols)]
 
+    def buffers(self):
+        """The tensors of this lane: scratch and workspace."""
+        return list(self.scratch.values()) + ([] if self.workspace is None else [self.workspace])
+
     def buf(self, name, shape):
         return self.scratch[name][: math.prod(shape)].view(shape)
 

@@ -562,10 +562,16 @@ class PipelineModule:
         if self.activation_checkpoint_interval == 0:     # else the first group's kept input is a buffer of its own
             self._stash[stage_id][slot][0]["x0"] = forward_input
 
-    def input_ptr(self, stage_id, slot):
-        """Address of the input the backward pass of ``slot`` will read (0: a buffer of the stash itself)."""
-        x = self._stash[stage_id][slot][0].get("x0") if self.activation_checkpoint_interval == 0 else None
-        return 0 if x is None else x.data_ptr()
+    def kept_input(self, stage_id, slot):
+        """The tensor the forward pass of ``slot`` was given, which its backward pass reads (None: a buffer of the stash)."""
+        return self._stash[stage_id][slot][0].get("x0") if self.activation_checkpoint_interval == 0 else None
+
+    def pass_buffers(self, stage_id, slot, layers):
+        """The tensors of the stage that a pass of ``slot`` over the layers a..b-1 touches, beside what it is given."""
+        own = [t for st in self._stash[stage_id][slot][layers[0]: layers[1]] for name, t in st.items() if name != "x0"]
+        if self.activation_checkpoint_interval > 0:
+            own += self._kept[stage_id][slot]
+        return own + [self.stage_params[stage_id].compute, self.stage_params[stage_id].grad]
 
     def backward(self, grad_output, grad_input, stage_id, slot=0, ctx=None, deferred=False):
         """Back-propagate through the layers of ``stage_id`` from the stash of ``slot``; parameter

@@ -407,16 +407,22 @@ int bb_graph_destroy(void* exec);
  *   bb_plan_dropout  names the dropout keys inside the plan: launches recorded with the key (k0[i], k1[i]) get, on
  *                    every replay, the key of (base_seed[i], step, micro_batch[i], layer[i], site[i]); fails if the plan
  *                    holds a key that is not listed.
- *   bb_plan_launch   issues the recorded launches in order on `stream`; `step` enters the dropout keys.
- * The recorded arguments are device pointers and sizes: the buffers must still be there and unchanged in layout.
+ *   bb_plan_operands names what a replay is given anew: every recorded pointer into [address[i], address[i] + bytes[i])
+ *                    belongs to operand i (bytes[i] <= 0: to none).  Once per plan; the ranges must not overlap.
+ *   bb_plan_launch   issues the recorded launches in order on `stream`; `step` enters the dropout keys.  For a plan without
+ *                    operands; with them, bb_plan_launch_on takes the `count` addresses to use in their place.
+ * The recorded arguments are device pointers and sizes: buffers that are not operands must still be there, and operands must
+ * have the shape, type, strides and 16-byte alignment of the recorded ones (nothing here can check that).
  * A plan may be launched by one thread at a time. */
 int bb_plan_begin(void);
 int bb_plan_end(void** plan_out);
 int bb_plan_abort(void);
 int bb_plan_dropout(void* plan, int count, const uint32_t* k0, const uint32_t* k1, const int64_t* base_seed,
                     const int64_t* micro_batch, const int64_t* layer, const int64_t* site);
+int bb_plan_operands(void* plan, int count, const uint64_t* address, const int64_t* bytes);
 int bb_plan_launches(void* plan);
 int bb_plan_launch(void* plan, int64_t step, void* stream);
+int bb_plan_launch_on(void* plan, int count, const uint64_t* address, int64_t step, void* stream);
 int bb_plan_destroy(void* plan);
 
 #ifdef __cplusplus

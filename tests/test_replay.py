@@ -1,0 +1,182 @@
+"""Which passes are replayed from a recorded plan and which go through the layer code: host logic, no GPU needed."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from bamboo_amd import hip, replay
+from bamboo_amd.engine import PipelineEngine
+from bamboo_amd.layers import FinalLayerNorm, StageContext
+
+ROWS, COLS = 6, 8
+
+
+class FakePlan:
+    """Stands in for the native plan: counts replays and remembers what they were given."""
+
+    launches = []
+
+    class _Recording:
+        def __enter__(self):
+            return FakePlan()
+
+        def __exit__(self, *exc):
+            return False
+
+    @classmethod
+    def record(cls):
+        return cls._Recording()
+
+    def dropout(self, keys):
+        pass
+
+    def operands(self, tensors):
+        self.n = len(tensors)
+
+    def launch(self, step, stream, tensors=()):
+        FakePlan.launches.append([t.data_ptr() for t in tensors])
+
+
+class FakeGraph(FakePlan):
+    capture = classmethod(lambda cls, stream: cls._Recording())
+
+    def launch(self, stream):
+        FakePlan.launches.append(None)
+
+
+class Layer(FinalLayerNorm):
+    """A layer whose passes check their operands like the wrappers of the kernels do, and count."""
+
+    launches_only = True
+    feature_dim = out_features = COLS
+
+    def forward(self, x, st, ctx):
+        ctx.calls.append(("forward", self.eps))
+        hip._like("forward", x, out=st["out"])
+        st["x0"] = x
+        return st["out"]
+
+    def backward(self, d_out, d_x, st, ctx):
+        ctx.calls.append(("backward", self.eps))
+        hip._like("backward", d_out, out=st["out"], d_x=d_x, x0=st["x0"])
+        return d_x
+
+
+@pytest.fixture
+def stage(monkeypatch):
+    """An engine of one stage over CPU tensors: one layer, one micro-batch, passes called by hand."""
+    from bamboo_amd.module import PipelineModule
+    monkeypatch.setattr(hip, "Plan", FakePlan)
+    monkeypatch.setattr(hip, "Graph", FakeGraph)
+    FakePlan.launches = []
+    module = object.__new__(PipelineModule)
+    flat = torch.zeros(64)
+    layer = Layer(COLS)
+    module.__dict__.update(loss_fn=None, base_seed=3, micro_offset=0, activation_checkpoint_interval=0, dtype=torch.float32,
+                           func_buckets={1: [layer]}, _stash={1: [[{"out": torch.zeros(ROWS, COLS)}]]}, stage_seq={1: [ROWS, ROWS]},
+                           stage_params={1: SimpleNamespace(compute=flat, grad=flat)})
+    ctx = StageContext(1, ROWS, torch.float32, "cpu")
+    ctx.calls = []
+    engine = object.__new__(PipelineEngine)
+    lens = [None]
+    engine.__dict__.update(
+        module=module, ctx=ctx, rc_ctx=ctx, use_graphs=False, _graphs={}, _replay=replay.Replay(module), global_steps=0, num_stages=3, stage_id=1, stage_ids=[1],
+        r_stage_ids=[], rc_stream=None, rc_issue="reference", eager_recovery=False, _deferred={}, grad_layer={}, main_stream=None, device="cpu",
+        queue=SimpleNamespace(key_len=lambda k: lens[0]), pipe_buffers={"input_1": [None], "output_1": [None], "input_grad_1": [None]},
+        _input_grad_store={1: [torch.zeros(ROWS, COLS)]})
+
+    def forward(x, key_len=None):
+        lens[0] = key_len
+        engine.pipe_buffers["input_1"][0], engine.pipe_buffers["output_1"][0] = x, None
+        engine._exec_forward_pass(0, 1)
+        return engine.pipe_buffers["output_1"][0]
+
+    def backward(grad, key_len=None):
+        lens[0] = key_len
+        engine.grad_layer[1] = grad
+        engine._exec_backward_pass(0, 1)
+        return engine.pipe_buffers["input_grad_1"][0]
+    return SimpleNamespace(engine=engine, module=module, layer=layer, ctx=ctx, forward=forward, backward=backward,
+                           replayed=lambda: len(FakePlan.launches), issued=lambda: len(ctx.calls))
+
+
+def test_other_buffers_of_the_same_form_are_replayed(stage):
+    a, b = torch.randn(ROWS, COLS), torch.randn(ROWS, COLS)
+    out = stage.forward(a)
+    assert (stage.issued(), stage.replayed()) == (1, 0)
+    assert stage.forward(b) is out and (stage.issued(), stage.replayed()) == (1, 1)
+    assert FakePlan.launches[-1] == [b.data_ptr()]
+    assert stage.module.kept_input(1, 0) is b and stage.module.micro_offset == 2
+    d_x = stage.backward(a)
+    for g in (b, a):
+        assert stage.backward(g) is d_x
+        assert FakePlan.launches[-1] == [g.data_ptr(), d_x.data_ptr(), b.data_ptr()]
+    assert stage.issued() == 2 and all(len(v) == 1 for v in stage.engine._replay.plans.values())
+
+
+# operands in a place that a recorded pass knows, which the layer code refuses
+WRONG = {"rows": lambda t: t[: ROWS - 1], "columns": lambda t: t.view(-1)[: ROWS * (COLS - 4)].view(ROWS, COLS - 4),
+         "type": lambda t: t.view(torch.int32).view(torch.float16)[:, :COLS], "strides": lambda t: t.view(COLS, ROWS).t()}
+
+
+@pytest.mark.parametrize("graphs", [False, True], ids=["plans", "graphs"])
+@pytest.mark.parametrize("wrong", list(WRONG))
+def test_an_operand_of_another_form_in_a_known_place_is_refused(stage, wrong, graphs):
+    x, g = torch.randn(ROWS, COLS), torch.randn(ROWS, COLS)
+    stage.engine.use_graphs = graphs
+    for _ in range(3):
+        stage.forward(x)
+        stage.backward(g)
+    replays = stage.replayed()
+    assert replays == 4
+    bad_x, bad_g = WRONG[wrong](x), WRONG[wrong](g)
+    assert bad_x.data_ptr() == x.data_ptr() and bad_g.data_ptr() == g.data_ptr()
+    with pytest.raises(hip.HipKernelError):
+        stage.backward(bad_g)
+    with pytest.raises(hip.HipKernelError):
+        stage.forward(bad_x)
+    assert stage.replayed() == replays
+
+
+def test_key_lengths_of_another_form_are_another_pass(stage):
+    x, n = torch.randn(ROWS, COLS), torch.zeros(4, dtype=torch.int32)
+    for key_len in (n[:1], n[:2], n[:1].float(), None):
+        before = stage.issued()
+        stage.forward(x, key_len)
+        assert stage.issued() == before + 1      # through the layer code, which checks
+    stage.forward(x, torch.zeros(1, dtype=torch.int32))
+    assert stage.replayed() == 1
+
+
+def test_forms_remembered_are_bounded(stage):
+    base = torch.zeros(COLS * 64)
+    for i in range(12):
+        stage.forward(torch.as_strided(base, (ROWS, COLS), (COLS, 1)), torch.zeros(i + 1, dtype=torch.int32))
+    assert len(stage.engine._replay.plans[("F", 1, 0)]) == replay.Replay.VARIANTS
+
+
+def test_an_operand_inside_the_stages_own_buffers_is_not_recorded(stage):
+    """A pointer into both could not be told apart: such a pass always goes through the layer code."""
+    own = stage.module._stash[1][0][0]["out"]
+    for _ in range(2):
+        stage.forward(own)
+        x = torch.randn(ROWS, COLS)
+        stage.module._stash[1][0][0]["x0"] = x
+        stage.backward(x)
+    assert stage.replayed() == 0
+
+
+def test_plan_operands_on_the_host(monkeypatch):
+    """The native side: overlapping operands are refused, as are launches with another number of addresses."""
+    with hip.Plan.record() as plan:
+        pass
+    a = torch.zeros(16)
+    with pytest.raises(hip.HipKernelError, match="overlap"):
+        plan.operands([a, a[8:]])
+    plan.operands([a[:8], a[8:], a[:0]])
+    with pytest.raises(hip.HipKernelError, match="named"):
+        plan.operands([a])
+    with pytest.raises(hip.HipKernelError):
+        plan.launch(0, SimpleNamespace(cuda_stream=0), [a])
+    with pytest.raises(hip.HipKernelError):
+        hip.check(hip.lib().bb_plan_launch(plan._plan, 0, None), "bb_plan_launch")
