@@ -17,8 +17,10 @@ class FakePlan:
     launches = []
 
     class _Recording:
+        made = None
+
         def __enter__(self):
-            return FakePlan()
+            return FakePlan() if self.made is None else self.made
 
         def __exit__(self, *exc):
             return False
@@ -38,7 +40,11 @@ class FakePlan:
 
 
 class FakeGraph(FakePlan):
-    capture = classmethod(lambda cls, stream: cls._Recording())
+    @classmethod
+    def capture(cls, stream):
+        recording = cls._Recording()
+        recording.made = cls()
+        return recording
 
     def launch(self, stream):
         FakePlan.launches.append(None)
