@@ -22,7 +22,8 @@ def initialize(args=None, model=None, optimizer=None, model_parameters=None, tra
     """Same signature and return tuple as the reference's ``deepspeed.initialize``
     (deepspeed/__init__.py:61-168): ``(engine, optimizer, training_dataloader, lr_scheduler)``.
     ``engine_kwargs`` carries what the one-GPU build adds: ``activation_queue`` (stand-in for the
-    neighbouring stages) and ``rc_stream`` (issue redundant forwards on a second HIP stream)."""
+    neighbouring stages), ``rc_stream`` (issue redundant forwards on a second HIP stream) and ``replay``
+    (False: issue every pass launch by launch instead of replaying what it launched before)."""
     from .engine import PipelineEngine
     if not isinstance(model, PipelineModule):
         raise PipelineError("bamboo_amd.initialize accelerates the pipeline path only: model must be a PipelineModule")

@@ -39,7 +39,7 @@ class PipelineEngine:
                  lr_scheduler=None, mpu=None, dist_init_required=None, collate_fn=None, config=None,
                  config_params=None, redundancy_level=0, sync_save=False, eager_recovery=False, prev_state={},
                  activation_queue=None, rc_stream=False, install_signal_handler=True, use_graphs=False,
-                 rc_issue="reference", rc_backlog=None):
+                 rc_issue="reference", rc_backlog=None, replay=True):
         if not isinstance(model, PipelineModule):
             raise PipelineError("model must base PipelineModule")
         hip.init()
@@ -103,10 +103,11 @@ class PipelineEngine:
         if self.use_graphs and self.main_stream.cuda_stream == 0:
             raise PipelineError("use_graphs needs the engine built and run under a created stream "
                                 "(torch.cuda.stream(...)): the default stream cannot be captured")
-        self._graphs = {}
+        self._graphs = {}     # (kind, stage, micro-batch, ...) -> "seen" or (graph, what the pass returns)
         # what every pass of (stage, micro-batch) launches is recorded when the pass is issued for the first time and
-        # replayed by one native call from then on (see _issue)
-        self._replay = Replay(model)
+        # replayed by one native call from then on (see _issue); False: every pass is issued launch by launch
+        self.replay = bool(replay)
+        self._replay = Replay(model, self._graphs)
         self._plans = self._replay.plans
         self.rc_stream = torch.cuda.Stream(self.device) if (rc_stream and self.r_stage_ids and eager_recovery) else None
         # When a redundant forward is issued (results never depend on it, only timing):
@@ -474,29 +475,34 @@ class PipelineEngine:
         :meth:`Replay.run`.  A pass has 8 to 20 launches per layer, at about 10 us of host time each through the layer code
         and 2 us from the recorded plan: stages of small layers are bound by that (one layer of 128 columns, 4 micro-batches:
         1.09 ms a batch issued from here, 0.45 ms replayed)."""
-        if ctx.gemm_hook is not None:
+        if ctx.gemm_hook is not None or not (self.replay or self.use_graphs):
             return issue()
-        if self.use_graphs:
-            # a captured graph holds the addresses
-            key = (slot, ctx, variant) + tuple((form(t), None if t is None else t.data_ptr()) for t in operands)
-            return self._graphed(key, ctx.stream, issue)
         if layers is None:
             layers = (0, len(self.module.func_buckets[slot[1]]))
+        if self.use_graphs:
+            # a captured graph holds the addresses
+            key = slot + (ctx, variant) + tuple((form(t), None if t is None else t.data_ptr()) for t in operands)
+            return self._graphed(key, ctx, layers, issue)
         return self._replay.run(slot, ctx, operands, variant, layers, self.global_steps, issue)
 
-    def _graphed(self, key, stream, issue):
+    def _graphed(self, key, ctx, layers, issue):
         """:meth:`_issue` with HIP graphs: eagerly the first time ``key`` occurs, captured and launched the second time,
         replayed from then on."""
+        self._replay.settled(key[1], ctx, layers)
         state = self._graphs.get(key)
         if state is None:
+            out = issue()
+            self._replay.settled(key[1], ctx, layers)     # a layer may make attributes of its own in its first pass
             self._graphs[key] = "seen"
-            return issue()
+            return out
+        if state == "seen" and self._has_dropout([key[1]]):
+            return issue()     # a layer's dropout has been switched on since the constructor looked
         if state == "seen":
-            with hip.Graph.capture(stream) as graph:
+            with hip.Graph.capture(ctx.stream) as graph:
                 out = issue()
             self._graphs[key] = (graph, out)
         graph, out = self._graphs[key]
-        graph.launch(stream)
+        graph.launch(ctx.stream)
         return out
 
     # ------------------------------------------------------------------ instruction handlers

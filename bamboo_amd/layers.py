@@ -90,12 +90,20 @@ class StageContext:
         off = sum(hip.colsum_workspace(d.M) for d in wgrads)
         return self.workspace[off: off + hip.colsum_workspace(cols)]
 
+    def pass_state(self):
+        """What the launches of a pass on this lane depend on beside its operands and what is set per call."""
+        return [self, self.batch, self.dtype, self.stream, self.workspace, *self.scratch.values()]
+
     def buffers(self):
         """The tensors of this lane: scratch and workspace."""
         return list(self.scratch.values()) + ([] if self.workspace is None else [self.workspace])
 
     def buf(self, name, shape):
         return self.scratch[name][: math.prod(shape)].view(shape)
+
+
+class _Answers(dict):
+    """What a layer has found out about shapes: no setting of it."""
 
 
 class TransformerLayer:
@@ -112,6 +120,7 @@ class TransformerLayer:
     backward pass agree bit for bit.
     """
 
+    launches_only = True      # see replay.launches_only
     SITE_ATTENTION, SITE_SUBLAYER0, SITE_FFN, SITE_SUBLAYER1 = 0, 1, 2, 3
 
     # parameter registration order of the reference's ``EncoderLayer`` (self_attn, feed_forward, sublayer:
@@ -434,6 +443,7 @@ class DecoderLayer(TransformerLayer):
     feed-forward hidden, 3 last sublayer) plus 4 (memory-attention probabilities) and 5 (second sublayer).
     ``mask`` applies to the self-attention only (the script passes none)."""
 
+    launches_only = True
     SITE_SRC_ATTENTION, SITE_SUBLAYER_SRC = 4, 5
 
     REFERENCE_ORDER = tuple(
@@ -616,6 +626,7 @@ class FinalLayerNorm:
     transformer script (transformer.py:181,250).  Parameters ``a_2`` / ``b_2`` as in the reference's ``LayerNorm``
     module (transformer.py:77-88)."""
 
+    launches_only = True
     REFERENCE_ORDER = ("a_2", "b_2")
 
     def __init__(self, hidden, ln="annotated", ln_eps=None):
@@ -671,6 +682,7 @@ class SumLast:
     (transformer.py:250); ``[rows, hidden] -> [rows, 1]``, so that ``MSELoss`` compares with ``[batch, seq]`` labels
     (transformer.py:205-219,264)."""
 
+    launches_only = True
     REFERENCE_ORDER = ()
 
     def __init__(self, hidden):
@@ -727,6 +739,7 @@ class BottleNeck:
     (tap-major, channel-minor) so that it is the ``[out, 9*in]`` GEMM operand as it lies in memory (the reference
     holds ``[out, in, 3, 3]``)."""
 
+    launches_only = True
     EXPANSION = 4
 
     def __init__(self, in_channels, out_channels, stride=1, height=14, width=14, bn_eps=1e-5, bn_momentum=0.1):
@@ -738,7 +751,7 @@ class BottleNeck:
         self.eps, self.momentum = bn_eps, bn_momentum
         self.w_ = self.g_ = None
         self.running = None
-        self._stats_ok = {}    # (shapes, dtype) -> whether the GEMM of a 1x1 convolution leaves strip statistics
+        self._stats_ok = _Answers()    # (shapes, dtype) -> whether the GEMM of a 1x1 convolution leaves strip statistics
 
     @property
     def feature_dim(self):

@@ -566,6 +566,25 @@ class PipelineModule:
         """The tensor the forward pass of ``slot`` was given, which its backward pass reads (None: a buffer of the stash)."""
         return self._stash[stage_id][slot][0].get("x0") if self.activation_checkpoint_interval == 0 else None
 
+    def pass_state(self, stage_id, layers):
+        """What the launches of a pass over the layers a..b-1 depend on beside its operands: every object by itself, to be
+        compared by identity (a value inside a dict that a layer holds counts, one further down does not)."""
+        out = [self.base_seed, self.activation_checkpoint_interval, self._stash.get(stage_id), getattr(self, "_kept", {}).get(stage_id),
+               getattr(self, "stage_seq", {}).get(stage_id), vars(self).get("forward"), vars(self).get("backward")]
+        for layer in self.func_buckets[stage_id][layers[0]: layers[1]]:
+            own, cls = vars(layer), type(layer)
+            out += [layer, cls.forward, cls.backward]
+            out += own.values()
+            for v in own.values():
+                if type(v) is dict:
+                    out += v.values()
+        return out
+
+    def passes_launch_only(self):
+        """Whether :meth:`forward` and :meth:`backward` are those below: what they do beside launches is known (:meth:`note_replay`)."""
+        cls = type(self)
+        return cls.forward is PipelineModule.forward and cls.backward is PipelineModule.backward and not {"forward", "backward"} & set(vars(self))
+
     def pass_buffers(self, stage_id, slot, layers):
         """The tensors of the stage that a pass of ``slot`` over the layers a..b-1 touches, beside what it is given."""
         own = [t for st in self._stash[stage_id][slot][layers[0]: layers[1]] for name, t in st.items() if name != "x0"]

@@ -2,11 +2,35 @@
 
 A pass of one (stage, micro-batch) launches the same kernels on the same stage-owned buffers in every batch.  It is recorded
 while it is issued for the first time (:class:`hip.Plan`) and issued by one native call from then on.  The call skips the
-layer code, and with it every check of an operand, so a plan stands for operands of one *form* only: what the checks look at,
-all but the address.  Addresses are filled in at each launch; an operand of another form goes through the layer code again
-and is recorded, or refused there, like a first one.
+layer code, and with it every check of an operand and every look at a setting.  So
+
+* a plan stands for operands of one *form*: what the checks look at, all but the address.  Addresses are filled in at each
+  launch; an operand of another form goes through the layer code again and is recorded, or refused there, like a first one;
+* the plans of a stage stand for one *state* of its layers: the attributes of each layer, its weights and the buffers, compared
+  at every pass.  Another state drops them;
+* only layers that say so are replayed (``launches_only``): a pass of any other layer is issued as always.
 """
+from operator import is_
+
 from . import hip
+
+
+def launches_only(layer):
+    """Whether the passes of ``layer`` do nothing that a replay of their launches leaves out.  A class promises it for what it
+    defines by ``launches_only = True`` of its own; a subclass without it may define how its parameters start (below) and
+    no more, and nothing may be put over a method on the object or in place of one in the class."""
+    harmless = {"__init__", "__repr__", "__module__", "__qualname__", "__doc__", "__dict__", "__weakref__", "__annotations__",
+                "__parameters__", "__orig_bases__", "init_params", "num_params", "flops_fwd"}
+    promised = False
+    for cls in type(layer).__mro__[:-1]:
+        own = vars(cls)
+        if own.get("launches_only") is True:
+            promised = True
+            if any(getattr(own.get(m), "__module__", cls.__module__) != cls.__module__ for m in ("forward", "backward")):
+                return False
+        elif not set(own) <= harmless:
+            return False
+    return promised and not any(hasattr(type(layer), name) for name in vars(layer))
 
 
 def form(t):
@@ -27,18 +51,40 @@ def _apart(ranges, others=()):
 class Replay:
     VARIANTS = 4     # forms remembered per (kind, stage, micro-batch)
 
-    def __init__(self, module):
+    def __init__(self, module, *stores):
+        """``stores``: further dicts whose keys have the stage second, emptied with the plans when a stage's state changes."""
         self.module = module
         self.plans = {}      # (kind, stage, micro-batch) -> {form of the call: (plan, which operand or what it returns)}
+        self._stores = stores
+        self._states = {}    # (stage, layers) -> (state that what is stored was recorded under, whether it may be replayed)
+
+    def settled(self, stage_id, ctx, layers):
+        """Whether passes of these layers may be replayed; drops what was recorded under another state of theirs."""
+        new = self.module.pass_state(stage_id, layers) + ctx.pass_state()
+        old, fit = self._states.get((stage_id, layers), (None, False))
+        # identity: the list keeps every object alive, numbers and strings do not change, and dicts are in it with their values
+        if old is not None and len(old) == len(new) and all(map(is_, old, new)):
+            return fit
+        if old is not None:
+            for store in (self.plans,) + self._stores:
+                stale = [k for k in store if k[1] == stage_id]
+                if stale and store is not self.plans:
+                    ctx.stream.synchronize()     # captured graphs are destroyed here
+                for k in stale:
+                    del store[k]
+        fit = self.module.passes_launch_only() and all(map(launches_only, self.module.func_buckets[stage_id][slice(*layers)]))
+        self._states[(stage_id, layers)] = (new, fit)
+        return fit
 
     def run(self, slot, ctx, operands, variant, layers, step, issue):
         """``issue()``, or the replay of its launches.  ``operands``: the tensors (or None) the pass is given, which may be others
         in every call; everything else it touches belongs to the stage or to ``ctx``.  ``variant``: what else the pass depends
         on.  ``layers``: the pair (a, b) of the stage's layers it runs."""
-        plans = self.plans.setdefault(slot, {})
+        if not self.settled(slot[1], ctx, layers):
+            return issue()
         key = (ctx, variant) + tuple(map(form, operands))
         given = [t for t in operands if t is not None]
-        known = plans.get(key)
+        known = self.plans.get(slot, {}).get(key)
         if known is not None:
             plan, at, out = known
             plan.launch(step, ctx.stream, given)
@@ -58,6 +104,9 @@ class Replay:
             plan.operands(given)
         except hip.HipKernelError:      # the pass has run; it just cannot be replayed
             return out
+        if not self.settled(slot[1], ctx, layers):     # a layer may make attributes of its own in its first pass
+            return out
+        plans = self.plans.setdefault(slot, {})
         while len(plans) >= self.VARIANTS:
             del plans[next(iter(plans))]
         at = next((i for i, t in enumerate(operands) if t is out and t is not None), None)

@@ -210,3 +210,25 @@ def test_a_wrong_operand_on_a_later_batch_is_refused(hiplib, kind):
         refused(engine)
         q.key_lens[0] = n
     engine.train_batch()
+
+
+SETTINGS = [("encoder", "dropout", 0.0), ("encoder", "dropout", 0.25), ("encoder", "mask", "causal"), ("encoder", "eps", 1e-2), ("encoder", "base_seed", 77),
+            ("resnet", "momentum", 0.5), ("resnet", "eps", 1e-1), ("resnet", "running", None), ("tail", "dropout", 0.0)]
+
+
+@pytest.mark.parametrize("kind,name,value", SETTINGS)
+def test_settings_changed_between_batches_take_effect(hiplib, kind, name, value):
+    """As in an engine that replays nothing: the next batch runs with the new setting, in every layer."""
+    (a, _), (b, _) = make_engine(kind, replay=False), make_engine(kind)
+    for batch in range(5):
+        if batch == 2:
+            for engine in (a, b):
+                for sid in engine.module.func_buckets:
+                    for obj in [engine.module] if name == "base_seed" else engine.module.func_buckets[sid]:
+                        if hasattr(obj, name):
+                            setattr(obj, name, value)
+        a.train_batch()
+        b.train_batch()
+        torch.cuda.synchronize()
+        assert_same_state(a, b)
+    assert b._plans and not a._plans

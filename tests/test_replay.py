@@ -84,9 +84,9 @@ def stage(monkeypatch):
     ctx = StageContext(1, ROWS, torch.float32, "cpu")
     ctx.calls = []
     engine = object.__new__(PipelineEngine)
-    lens = [None]
+    lens, graphs = [None], {}
     engine.__dict__.update(
-        module=module, ctx=ctx, rc_ctx=ctx, use_graphs=False, _graphs={}, _replay=replay.Replay(module), global_steps=0, num_stages=3, stage_id=1, stage_ids=[1],
+        module=module, ctx=ctx, rc_ctx=ctx, use_graphs=False, replay=True, _graphs=graphs, _replay=replay.Replay(module, graphs), global_steps=0, num_stages=3, stage_id=1, stage_ids=[1],
         r_stage_ids=[], rc_stream=None, rc_issue="reference", eager_recovery=False, _deferred={}, grad_layer={}, main_stream=None, device="cpu",
         queue=SimpleNamespace(key_len=lambda k: lens[0]), pipe_buffers={"input_1": [None], "output_1": [None], "input_grad_1": [None]},
         _input_grad_store={1: [torch.zeros(ROWS, COLS)]})
@@ -186,3 +186,113 @@ def test_plan_operands_on_the_host(monkeypatch):
         plan.launch(0, SimpleNamespace(cuda_stream=0), [a])
     with pytest.raises(hip.HipKernelError):
         hip.check(hip.lib().bb_plan_launch(plan._plan, 0, None), "bb_plan_launch")
+
+
+# what a program may change between batches, and the next pass has to see
+CHANGES = {
+    "setting": lambda s: setattr(s.layer, "eps", 0.5),
+    "new-attribute": lambda s: setattr(s.layer, "extra", 1),
+    "base-seed": lambda s: setattr(s.module, "base_seed", 4),
+    "weight-in-place": lambda s: s.layer.w.update(a_2=torch.ones(COLS)),
+    "bind": lambda s: s.layer.bind({"a_2": torch.ones(COLS)}, {}),
+    "statistics": lambda s: s.layer.running.update({1: (torch.zeros(1), torch.ones(1))}),
+    "scratch": lambda s: s.ctx.scratch.update(d=torch.zeros(4)),
+    "workspace": lambda s: s.ctx.ensure_workspace(1000),
+    "layer": lambda s: s.module.func_buckets.update({1: [Layer(COLS)]}),
+    "stash": lambda s: s.module._stash.update({1: [[{"out": torch.zeros(ROWS, COLS)}]]}),
+}
+
+
+@pytest.mark.parametrize("graphs", [False, True], ids=["plans", "graphs"])
+@pytest.mark.parametrize("change", list(CHANGES))
+def test_a_change_between_batches_reaches_the_next_pass(stage, change, graphs):
+    stage.layer.w, stage.layer.running = {"a_2": torch.zeros(COLS)}, {1: (torch.zeros(1), torch.ones(1))}
+    stage.engine.use_graphs = graphs
+    stage.ctx.stream = SimpleNamespace(synchronize=lambda: None)
+    x, g = torch.randn(ROWS, COLS), torch.randn(ROWS, COLS)
+    for _ in range(3):
+        stage.forward(x)
+        stage.backward(g)
+    assert stage.replayed() == 4
+    CHANGES[change](stage)
+    issued = stage.issued()
+    for passes in (1, 2):
+        stage.forward(x)
+        stage.backward(g)
+        assert stage.issued() == issued + (2 * passes if graphs else 2)      # once each; a graph is captured on the second
+    stage.forward(x)
+    assert stage.issued() == issued + (4 if graphs else 2) and stage.ctx.calls[-1][1] == (0.5 if change == "setting" else stage.layer.eps)
+
+
+class Logging(Layer):
+    def forward(self, x, st, ctx):
+        return super().forward(x, st, ctx)
+
+
+class Helper(Layer):
+    def _scaled(self, x):
+        return x
+
+
+class Start(Layer):
+    """Defines only how its parameters start."""
+
+    def __init__(self, hidden):
+        super().__init__(hidden)
+
+    def init_params(self, master, seed):
+        pass
+
+
+class Promising(Logging):
+    launches_only = True
+
+
+def _shadowed():
+    layer = Layer(COLS)
+    layer.forward = lambda x, st, ctx: type(layer).forward(layer, x, st, ctx)
+    return layer
+
+
+@pytest.mark.parametrize("make,replayed", [(lambda: Logging(COLS), False), (lambda: Helper(COLS), False), (_shadowed, False), (lambda: Start(COLS), True),
+                                           (lambda: Promising(COLS), False), (lambda: Layer(COLS), True)])
+def test_layers_that_do_more_than_launch_are_not_replayed(stage, make, replayed):
+    """Python code of a subclass, or put over a method of the object, runs in every pass; a class that promises to launch
+    only has to do so for every method on the way to the promising base."""
+    layer = make()
+    stage.module.func_buckets[1] = [layer]
+    assert replay.launches_only(layer) == replayed
+    x = torch.randn(ROWS, COLS)
+    for _ in range(3):
+        stage.forward(x)
+    assert stage.issued() == (1 if replayed else 3)
+
+
+def test_a_class_whose_passes_were_replaced_is_not_replayed(stage, monkeypatch):
+    x = torch.randn(ROWS, COLS)
+    stage.forward(x)
+    inner = Layer.forward
+
+    def wrapped(self, x, st, ctx):
+        return inner(self, x, st, ctx)
+    wrapped.__module__ = "elsewhere"
+    monkeypatch.setattr(Layer, "forward", wrapped)
+    for _ in range(2):
+        stage.forward(x)
+    assert stage.replayed() == 0 and stage.issued() == 3
+
+
+def test_replaying_can_be_switched_off(stage):
+    x = torch.randn(ROWS, COLS)
+    stage.forward(x)
+    stage.engine.replay = False
+    stage.forward(x)
+    assert stage.replayed() == 0 and stage.issued() == 2
+
+
+def test_the_frameworks_layers_promise_to_launch_only():
+    from bamboo_amd import BottleNeck, DecoderLayer, FinalLayerNorm, SumLast, TransformerLayer
+    from perf import cases
+    for layer in (TransformerLayer(64, 1, 64), DecoderLayer(64, 1, 64), FinalLayerNorm(64), SumLast(64), BottleNeck(64, 16), BottleNeck(64, 16, stride=2),
+                  cases._Encoder(64, 1, 64), cases._Block(64, 16)):
+        assert replay.launches_only(layer)
