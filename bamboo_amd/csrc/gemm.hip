@@ -267,14 +267,17 @@ template <bool TA, bool TB> static int launch_f32_wave(GemmArgs& g, int batches,
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
-template <bool TA, bool TB, int BN> static int launch_f32(GemmArgs& g, int batches, hipStream_t st) {
+// rows too wide for the kernels' 32-bit offsets inside a tile (64 rows of 2^22 elements are 2^30 bytes): 64x64 tiles with 64-bit ones
+static bool f32_wide(int64_t lda, int64_t ldb) { return lda >= (1 << 22) || ldb >= (1 << 22); }
+template <bool TA, bool TB, int BN, bool WIDE = false> static int launch_f32(GemmArgs& g, int batches, hipStream_t st) {
     g.tiles_m = (g.M + 63) / 64;
     g.tiles_n = (g.N + BN - 1) / BN;
-    bb_launch((gemm_f32_kernel<TA, TB, BN>), dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(256), f32_gemm_lds(BN), st, g);
+    bb_launch((gemm_f32_kernel<TA, TB, BN, WIDE>), dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(256), f32_gemm_lds(BN), st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
 template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hipStream_t st) {
+    if (f32_wide(g.lda, g.ldb)) return launch_f32<TA, TB, 64, true>(g, batches, st);
     if (pick_f32_wave(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) return launch_f32_wave<TA, TB>(g, batches, st);
     if (pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) {
         if constexpr (!TA) return launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
@@ -294,6 +297,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
         else snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
                  dt != D_NONE ? kDmaTileNames[dt] : "128x128");
     }
+    else if (f32_wide(d->lda, d->ldb)) snprintf(out, out_len, "f32_%s_64x64wide", layouts[d->layout]);
     else if (pick_f32_wave(d->M, d->N, d->K, batches, d->layout)) snprintf(out, out_len, "f32_%s_wave32x32k%d", layouts[d->layout], kF32Waves);
     else if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
         snprintf(out, out_len, "f32_%s_64x%dk%d", layouts[d->layout], kF32SplitBN, kF32SplitGroups);
@@ -342,7 +346,6 @@ static int fill_args(const bb_gemm_desc* d, GemmArgs& g, int64_t& batches, bool&
     BB_REQUIRE(d->sA1 % vec == 0 && d->sA2 % vec == 0 && d->sB1 % vec == 0 && d->sB2 % vec == 0,
                "bb_gemm: batch strides of A/B must be multiples of %d", vec);
     BB_REQUIRE(d->lda >= a_contig && ldb >= b_contig && d->ldc >= d->N, "bb_gemm: leading dimension too small");
-    BB_REQUIRE(d->dtype != BB_F32 || (d->lda < (1 << 22) && d->ldb < (1 << 22)), "bb_gemm: fp32 leading dimension too large");
     g.A = d->A; g.B = d->B; g.C = d->C;
     g.bias = d->bias; g.aux_in = d->aux_in; g.aux_out = d->aux_out; g.resid = d->resid;
     g.colsum = nullptr;
@@ -670,6 +673,7 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
         const bool w = pick_f32_wave(d.M, d.N, d.K, 1, d.layout);
         few += w;
         fuse32 = d.dtype == BB_F32 && d.layout == descs[0].layout && d.nb1 <= 1 && d.nb2 <= 1 && d.M > 0 && d.N > 0 && d.dropout_p == 0.f &&
+                 !f32_wide(d.lda, d.ldb) &&
                  (w || !pick_f32_split(d.M, d.N, d.K, 1, d.layout));
     }
     const bool waves = few == count;

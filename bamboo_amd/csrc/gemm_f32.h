@@ -19,10 +19,12 @@
 // problem is a matter of its shape and layout alone.
 // (volatile: pairs of reads merged into one instruction have no room for the stage's offset, i.e. cost an addition each)
 typedef const volatile __attribute__((address_space(3))) float lds_f32;
-template <int ROWS, bool KM, int NW = 4> struct F32Operand {
+// WIDE: rows of 2^22 elements and more, whose tile does not fit the 32-bit offsets: 64-bit addresses, added up per load
+template <int ROWS, bool KM, int NW = 4, bool WIDE = false> struct F32Operand {
+    using Offset = std::conditional_t<WIDE, int64_t, unsigned>;
     static constexpr int BYTES = ROWS * 32 * 4, ROUNDS = BYTES / (1024 * NW);   // NW waves load a stage
     const float* base;          // wave-uniform: the tile's first row (K-contiguous) / column (k-major), the next k-tile
-    unsigned off[ROUNDS];       // the lane's 16 bytes from there
+    Offset off[ROUNDS];         // the lane's 16 bytes from there
     int k_lane[ROUNDS];         // ... and their k inside a k-tile
     int64_t step;
     __device__ __forceinline__ void init(const float* p, int64_t ld, int row0, int rows, int lane, int wave) {
@@ -33,22 +35,22 @@ template <int ROWS, bool KM, int NW = 4> struct F32Operand {
             if constexpr (!KM) {
                 const int r = q * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
                 k_lane[i] = c * 4;
-                off[i] = (unsigned)((int64_t)min(r, rows - 1 - row0) * ld + c * 4) * 4u;
+                off[i] = (Offset)((int64_t)min(r, rows - 1 - row0) * ld + c * 4) * (Offset)4;
             } else {
                 constexpr int CPR = ROWS / 4, RPI = 64 / CPR;   // 16-byte chunks per k-row, k-rows per instruction
                 const int k = q * RPI + lane / CPR, c = (lane % CPR) ^ (ROWS == 64 ? 8 * (k & 1) : 0);
                 k_lane[i] = k;
-                off[i] = (unsigned)((int64_t)k * ld + min(c * 4, rows - 4 - row0)) * 4u;
+                off[i] = (Offset)((int64_t)k * ld + min(c * 4, rows - 4 - row0)) * (Offset)4;
             }
         }
         step = KM ? 32 * ld : 32;
     }
     // `left`: contraction elements from the k-tile's start (< 32: the last, ragged one); lds: LDS address of the stage
     __device__ __forceinline__ void issue(unsigned lds, int wave, int left, int lane) {
-        if (left >= 32) {
+        if (!WIDE && left >= 32) {
 #pragma unroll
             for (int i = 0; i < ROUNDS; ++i)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + (i * NW + wave) * 1024), "v"(off[i]), "s"(base) : "m0");
+                if constexpr (!WIDE) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds + (i * NW + wave) * 1024), "v"(off[i]), "s"(base) : "m0");
         } else {
 #pragma unroll
             for (int i = 0; i < ROUNDS; ++i)
@@ -152,12 +154,12 @@ __device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, in
 
 // (block_id: the block's index among the problem's tiles; logical_id: it is not a hardware block id, so the tile order takes it
 // as it is instead of undoing the round-robin over the XCDs)
-template <bool TA, bool TB, int BN>
+template <bool TA, bool TB, int BN, bool WIDE = false>
 __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block_id, const int batch_id, const bool logical_id) {
     static_assert(BN == 64 || BN == 32, "tiles: 64x64, 64x32 with the contraction shared by two groups");
     constexpr int KG = 64 / BN;
-    using OpA = F32Operand<64, TA>;
-    using OpB = F32Operand<BN, TB>;
+    using OpA = F32Operand<64, TA, 4, WIDE>;
+    using OpB = F32Operand<BN, TB, 4, WIDE>;
     constexpr int STAGES = f32_stages(BN), STAGE = OpA::BYTES + OpB::BYTES, LOADS = OpA::ROUNDS + OpB::ROUNDS;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -282,9 +284,9 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block
     if (n < g.N) epilogue_f32<16>(g, coff, acc_m, n, bias, pre, acc);
 }
 
-template <bool TA, bool TB, int BN>
-__global__ __launch_bounds__(256, 4) void gemm_f32_kernel(const GemmArgs g) {
-    gemm_f32_body<TA, TB, BN>(g, blockIdx.x, blockIdx.z, false);
+template <bool TA, bool TB, int BN, bool WIDE = false>
+__global__ __launch_bounds__(256, WIDE ? 2 : 4) void gemm_f32_kernel(const GemmArgs g) {
+    gemm_f32_body<TA, TB, BN, WIDE>(g, blockIdx.x, blockIdx.z, false);
 }
 // several unbatched problems in one launch (the weight gradients of an fp32 layer)
 template <bool TA, bool TB>

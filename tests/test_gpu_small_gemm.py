@@ -139,3 +139,24 @@ def test_fp32_batched_heads_of_few_tiles(hiplib, b, heads, seq):
     q, k = (qkv[:, i * h:(i + 1) * h].double().cpu().view(b, seq, heads, d).transpose(1, 2) for i in (0, 1))
     bound = (d + 2) * 2.0 ** -24 * 0.125 * (q.abs() @ k.abs().transpose(-1, -2))
     assert bool(((P.double().cpu() - 0.125 * q @ k.transpose(-1, -2)).abs() <= bound).all())
+
+
+# the first row pitch that the 32-bit offsets inside a tile are not used for, and one where 64 rows pass 2^32 bytes; K with and
+# without a ragged last k-tile.  |error| <= K eps sum |a b|, as above.
+@pytest.mark.parametrize("ld", [1 << 22, (1 << 24) + (1 << 20) + 4])
+@pytest.mark.parametrize("layout,M,N,K", [("nt", 70, 36, 64), ("nt", 3, 64, 100), ("nn", 66, 68, 44), ("tn", 64, 72, 40)])
+def test_fp32_rows_of_any_pitch(hiplib, layout, M, N, K, ld):
+    lay = {"nt": hiplib.NT, "nn": hiplib.NN, "tn": hiplib.TN}[layout]
+    g = torch.Generator().manual_seed(3)
+    shapes = ((K, M) if layout == "tn" else (M, K), (N, K) if layout == "nt" else (K, N))
+    host = [torch.randn(s, generator=g) for s in shapes]
+    A, B = [torch.as_strided(torch.empty((t.shape[0] - 1) * ld + t.shape[1], device=DEV), t.shape, (ld, 1)).copy_(t) for t in host]
+    C, C2, C3 = (torch.full((M, N), float("nan"), device=DEV) for _ in range(3))
+    descs = [hiplib.gemm_desc(lay, A, B, c) for c in (C, C2, C3)]
+    assert hiplib.gemm_variant(descs[0]).endswith("64x64wide")
+    hiplib.gemm(lay, A, B, C)
+    hiplib.gemm_grouped(descs[1:])
+    a, b = host[0].double(), host[1].double()
+    a, b = (a.t() if layout == "tn" else a), (b.t() if layout == "nt" else b)
+    bound = K * 2.0 ** -24 * (a.abs() @ b.abs())
+    assert ((C.double().cpu() - a @ b).abs() <= bound).all() and torch.equal(C, C2) and torch.equal(C, C3)
