@@ -26,12 +26,12 @@ static int launch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES = 4, int BK = 32>
+template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES = 4, int BK = 32, bool RAGK = false>
 static int launch_bf16_dma(GemmArgs& g, int batches, hipStream_t st) {
     constexpr int smem = STAGES * (BM + BN) * BK * 2;
-    auto kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK>;
+    auto kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, RAGK>;
     if constexpr (!AKM && !BKM) {       // dropout goes with forward (NT) products only: fill_args refuses the others
-        if (g.drop.thresh) kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, true>;
+        if (g.drop.thresh) kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, true, RAGK>;
     }
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -83,12 +83,12 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
     return BB_OK;
 }
 
-// DMA kernels need K % 32 == 0 and at least one full vector of rows; tile by problem size
+// DMA kernels need at least one full vector of rows, and but for weight gradients and D128x128k64r K % 32 == 0; tile by problem size
 enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, D256x128k64s3, D128x128k64, D128x64k64s3, D128x64s3,
-               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4 };
+               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r };
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
-                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4"};
+                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r"};
 // The tile of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
 // what ran before), and every kernel adds up a contraction in the same order: a redundant forward and a normal forward
 // of the same layer give the same bits.
@@ -100,7 +100,15 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     //    tiles do not take (fewer than 128 rows or columns) run on it too.
     const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches;
     if (layout != BB_TN && K % 64 == 0 && K > 0 && N % 8 == 0 && (t64 <= 256 || M < 128 || N < 128)) return D64x64k64s4;
-    if ((K % 32 != 0 && layout != BB_TN) || K < 64 || M < 128 || N < 128 || N % 8 != 0) return D_NONE;
+    if ((K % 32 != 0 && layout != BB_TN) || K < 64 || M < 128 || N < 128 || N % 8 != 0) {
+        //  - What is left goes to the wave-sliced 64x64 tiles (pick_wave) while these are at most two per CU, i.e. one round of
+        //    them.  Beyond that they read more and hide less than 128x128 tiles with a masked last k-tile (us, 64x64 / 128x128):
+        //    NT 2048x1000x1000 (512 tiles) 13.2 / 14.4, 4096x1000x1000 21.9 / 17.7, 8192x4096x72 67 / 30, 8192x4096x4008 499 / 316;
+        //    NN 8192x1000x4008 132 / 78; 48 heads, NN 1032x80x1032 50 / 34, NT 1032x1032x80 111 / 55; TN 1032x80x1032 53 / 39.
+        if (N % 8 != 0 || t64 <= 512) return D_NONE;
+        if (layout != BB_TN) return D128x128k64r;
+        return K >= 64 ? D128x128s3 : D_NONE;
+    }
     // Rules read off sweeps of M 2048..16384 x N 768..6400 x K 1024/4096 (NT and NN) on MI355X (256 CUs,
     // one block of the 256-row tiles per CU).
     //  - Operands whose rows are k-contiguous (both of NT, A of NN) load faster as 64-wide k-tiles: one
@@ -179,8 +187,8 @@ static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layou
     return t;
 }
 
-// The wave-sliced kernels (gemm_wave.h) take the weight gradients whose 64x64 tiles are at most one per CU, and whatever the
-// DMA kernels do not take (contractions of odd lengths).  W_8: eight waves, 32-wide slices, two stages each (130 KB of LDS);
+// The wave-sliced kernels (gemm_wave.h) take the weight gradients whose 64x64 tiles are at most one per CU, and what the
+// DMA kernels do not take (contractions of odd lengths, few tiles).  W_8: eight waves, 32-wide slices, two stages each (130 KB of LDS);
 // W_4: four waves, 64-wide slices, one stage (65 KB, two blocks a CU).  Measured back to back, 128x128 DMA tiles / W_8 (us):
 // TN 512x512x4096 55.7 / 18.8, 256x256x6272 80.8 / 21.9; register-staged kernel / W_8: NT 200x264x72 31.4 / 5.2.
 enum WaveMode { W_NONE = 0, W_8, W_4 };
@@ -219,6 +227,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D256x256k64: return launch_bf16_dma<256, 256, 2, 4, TA, TB, true, 2, 64>(g, batches, st);
         case D256x128k64s3: return launch_bf16_dma<256, 128, 4, 2, TA, TB, true, 3, 64>(g, batches, st);
         case D128x128k64: return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64>(g, batches, st);
+        case D128x128k64r:
+            if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64, true>(g, batches, st);
+            else break;
         case D128x64k64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3, 64>(g, batches, st);
         case D128x64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3>(g, batches, st);
         case D64x128k64s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
@@ -644,6 +655,12 @@ static int colsum_f32(const bb_gemm_desc* descs, int count, void* stream) {
     return BB_OK;
 }
 
+// whether the grouped DMA kernel takes the problem: it masks the contraction's end for weight gradients only
+static bool shared_launch_dma(const bb_gemm_desc& d) {
+    const DmaTile t = pick_dma_tile(d.M, d.N, d.K, 1, d.layout);
+    return t != D_NONE && t != D128x128k64r;
+}
+
 extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream) {
     BB_REQUIRE(count >= 0 && (descs || count == 0), "bb_gemm_grouped: bad arguments");
     hipStream_t st = (hipStream_t)stream;
@@ -656,7 +673,7 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
     for (int i = 0; i < count && fuse; ++i) {
         const bb_gemm_desc& d = descs[i];
         // the grouped kernels are built without dropout decisions in their epilogue: such a problem runs by itself
-        dma = dma && pick_dma_tile(d.M, d.N, d.K, 1, d.layout) != D_NONE && d.conv_c % 128 == 0;
+        dma = dma && shared_launch_dma(d) && d.conv_c % 128 == 0;
         wave = wave && pick_wave(d.M, d.N, d.K, 1, d.layout, D_NONE) != W_NONE;
         fuse = d.dtype == BB_BF16 && d.layout == descs[0].layout && d.nb1 <= 1 && d.nb2 <= 1 && d.M > 0 && d.N > 0 &&
                d.dropout_p == 0.f && (dma || wave);
@@ -781,7 +798,7 @@ static int pick_splits(const bb_gemm_desc* descs, int count) {
         const bb_gemm_desc& d = descs[i];
         if (d.dtype != BB_BF16 || d.c_dtype != BB_F32 || d.layout != descs[0].layout || d.nb1 > 1 || d.nb2 > 1 || d.M <= 0 ||
             d.N <= 0 || d.colsum_out || d.bias || d.epilogue != BB_EPI_NONE || d.alpha != 1.0f || d.N % 4 != 0 || d.dropout_p != 0.f ||
-            (pick_dma_tile(d.M, d.N, d.K, 1, d.layout) == D_NONE && d.layout != BB_TN))
+            (!shared_launch_dma(d) && d.layout != BB_TN))
             return 0;
         tiles += (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64);
         tiles128 += (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128);

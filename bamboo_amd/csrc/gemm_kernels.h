@@ -551,14 +551,18 @@ template <int BR, bool KM, int NW, int BK = 32, bool VIS = false, int CONV = 0> 
         if constexpr (CONV == 2) wrap = 0;
         if constexpr (CONV == 3) dpy = dpx = 0;
     }
-    // k-major operand, last k-tile of a contraction that is no multiple of it: rows past its `left` read zeros
+    // last k-tile of a contraction that is no multiple of it: k past its `left` reads zeros (where rows are k-contiguous `left`
+    // is a multiple of 8: a lane's 16 bytes are inside or outside as a whole)
     __device__ __forceinline__ void mask_tail(int left, int tid) {
-        static_assert(KM, "only a k-major operand has a ragged last k-tile");
-        constexpr int RPI = 64 / (BR / 8);
         const int lane = tid & 63, wave = tid >> 6;
 #pragma unroll
         for (int i = 0; i < ROUNDS; ++i) {
-            if ((i * NW + wave) * RPI + lane / (BR / 8) < left) continue;
+            const int q = i * NW + wave;
+            int k;     // of the lane's bytes, as init() deals them
+            if constexpr (KM) k = q * (64 / (BR / 8)) + lane / (BR / 8);
+            else if constexpr (BK == 64) k = ((lane & 7) ^ (((q * 8 + (lane >> 3)) >> 1) & 7)) * 8;
+            else k = ((lane & 3) ^ (((q * 16 + (lane >> 2)) >> 2) & 3)) * 8;
+            if (k < left) continue;
             if constexpr (CONV == 3) py[i] = -(1 << 30);   // outside of every image
             else src[i] = (const bf16*)(bb_zero_line + (lane & 7) * 16);
         }
@@ -657,7 +661,7 @@ template <int BR, int T, bool KM, int BK = 32> struct FragReader {
 // the epilogue also leaves that normalisation's backward sums per strip (BnBwdArgs), so that its backward pass has no
 // reduction over the tensor left.
 template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, int BK = 32, bool VIS = false, int CONV = 0,
-          int STATS = 0, bool DROP = false>
+          int STATS = 0, bool DROP = false, bool RAGK = false>
 __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int block_id, const int batch_id,
                                                    const bool logical_id = false, const ConvArgs& cv = ConvArgs{},
                                                    const BnBwdArgs& bn = BnBwdArgs{}) {
@@ -714,8 +718,9 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         bf16x8 a[2][TM], b[2][TN];
     };
     Frags f0, f1;
-    // a weight gradient's contraction (both operands k-major) may end inside a k-tile: the batch times an odd sequence length
-    constexpr bool RAGGED = AKM && BKM;
+    // a weight gradient's contraction (both operands k-major) may end inside a k-tile: the batch times an odd sequence length;
+    // that of another product (RAGK) by any multiple of 8
+    constexpr bool RAGGED = (AKM && BKM) || RAGK;
     const int KT = RAGGED ? (g.K + BK - 1) / BK : g.K / BK;
 
     // ring positions: tile t lives in stage t % STAGES
@@ -1139,10 +1144,11 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
 }
 
 // DROP: the epilogue can apply dropout (g.drop).  A kernel of its own, so that the keep decisions' registers cost the
-// kernels without dropout nothing (they decide how many blocks of the small tiles a CU holds).
-template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, int BK, bool DROP = false>
+// kernels without dropout nothing (they decide how many blocks of the small tiles a CU holds).  RAGK: contractions of any
+// length, likewise.
+template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, int BK, bool DROP = false, bool RAGK = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, 0, 0, DROP>(g, blockIdx.x, blockIdx.z);
+    gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, 0, 0, DROP, RAGK>(g, blockIdx.x, blockIdx.z);
 }
 // the same with the strip statistics of the output (NT, 64-wide k-tiles)
 template <int BM, int BN, int WM, int WN, int STAGES>

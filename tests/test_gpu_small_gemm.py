@@ -53,6 +53,48 @@ def test_products_of_few_tiles(hiplib, layout, M, N, K):
     assert torch.equal(G, G2)
 
 
+# More 64x64 tiles than two a CU and a contraction that ends inside a k-tile: k-tiles of 8 to 56, one k-tile in all, rows and
+# columns off the tile.  bf16 results: half an ulp, at most 2^-8 of |C|, beside the fp32 sums' K eps sum |a b|.
+@pytest.mark.parametrize("M,N,K", [(3001, 1000, 8), (4100, 520, 40), (2100, 1096, 72), (33000, 72, 88), (2049, 1032, 1000), (96, 33000, 136)])
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+def test_large_products_of_ragged_contractions(hiplib, layout, M, N, K):
+    lay = hiplib.NT if layout == "nt" else hiplib.NN
+    A, B = rand(M, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    C = wide[:M, :N]
+    assert hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C)).endswith("dma128x128k64r")
+    hiplib.gemm(lay, A, B, C)
+    a, b = A.double(), (B.double().t() if layout == "nt" else B.double()).contiguous()
+    want, slack = a @ b, K * 2.0 ** -24 * (a.abs() @ b.abs())
+    assert ((C.double() - want).abs() <= 2.0 ** -8 * (want.abs() + slack) + slack).all()
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()       # nothing written past the rows and columns
+    if layout == "nt":      # as a member of a group it runs by itself; with dropout, the kernel that decides
+        C2, C3 = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        hiplib.gemm_grouped([hiplib.gemm_desc(lay, A, B, C2), hiplib.gemm_desc(lay, A, B, C3)])
+        assert torch.equal(C, C2) and torch.equal(C, C3)
+        key = hiplib.dropout_key(1, 2, 3, 4, 5)
+        hiplib.gemm(lay, A, B, C2, dropout=(0.25, key))
+        hiplib.dropout_apply(C3, C3, 0.25, key)
+        assert torch.equal(C2 == 0, C3 == 0) and rel(C2, C3) < 1e-2     # two roundings against one
+
+
+# heads of a width that the fused attention does not take: the products of a materialised attention, forward and backward
+@pytest.mark.parametrize("b,h,s,d", [(3, 12, 520, 72), (1, 24, 1032, 40), (2, 20, 456, 80)])
+def test_attention_products_of_ragged_lengths(hiplib, b, h, s, d):
+    P, X = rand(b, h, s, s, seed=1), rand(b * s, 3 * h * d, seed=2)
+    heads = X.view(b, s, 3, h, d).permute(2, 0, 3, 1, 4).double()      # [3, b, h, s, d]
+    sp, sx = (h * s * s, s * s), (s * 3 * h * d, d)
+    at = lambda t, i: t.data_ptr() + i * h * d * t.element_size()
+    for lay, want in ((hiplib.NN, P.double() @ heads[1].contiguous()), (hiplib.TN, P.double().transpose(2, 3).contiguous() @ heads[1].contiguous())):
+        out = torch.full_like(X, 7.0)
+        hiplib.gemm_batched(lay, hiplib.BF16, s, d, s, P.data_ptr(), s, sp, at(X, 1), 3 * h * d, sx, at(out, 2), 3 * h * d, sx, b, h)
+        got = out.view(b, s, 3, h, d).permute(2, 0, 3, 1, 4)
+        assert rel(got[2], want) < 1e-2 and (got[:2] == 7).all()
+    S = torch.empty(b, h, s, s, dtype=torch.bfloat16, device=DEV)
+    hiplib.gemm_batched(hiplib.NT, hiplib.BF16, s, s, d, at(X, 0), 3 * h * d, sx, at(X, 1), 3 * h * d, sx, S.data_ptr(), s, sp, b, h)
+    assert rel(S, heads[0].contiguous() @ heads[1].transpose(2, 3).contiguous()) < 1e-2
+
+
 # (rows, shapes of dy and x): few tiles (eight waves a tile), up to four tiles a CU (four waves), 128x128 tiles
 @pytest.mark.parametrize("rows,shapes", [(1, [(64, 64), (8, 72)]), (31, [(128, 128), (384, 128)]), (1050, [(192, 768), (576, 192)]),
                                          (333, [(512, 2048), (2048, 512), (512, 512)]), (2049, [(1024, 4096), (4096, 1024)]),
