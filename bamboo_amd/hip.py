@@ -184,11 +184,12 @@ def _ptr(t):
     return None if t is None else c_void_p(t.data_ptr())
 
 
-def extent_bytes(t):
-    """Bytes from a strided tensor's first element to the end of its last one."""
-    if t.numel() == 0:
-        return 0
-    return (sum((n - 1) * abs(s) for n, s in zip(t.shape, t.stride())) + 1) * t.element_size()
+def address_range(t):
+    """(address of a strided tensor's first element, address behind its last one)."""
+    lo, n = t.data_ptr(), t.numel()
+    if n and not t.is_contiguous():
+        n = sum((n - 1) * s for n, s in zip(t.shape, t.stride())) + 1
+    return lo, lo + n * t.element_size()
 
 
 def _row_major(t, name):
@@ -597,9 +598,9 @@ class Plan:
     """The launches one call makes, recorded while it makes them and issued again by one call (``with Plan.record() as
     plan: ...``, then ``plan.launch(step, stream)``).  ``plan.dropout(keys)`` names the dropout keys among the recorded
     arguments: ``{(k0, k1): (base_seed, micro_batch, layer, site)}``; a launch derives them anew for its ``step``.
-    ``plan.operands(tensors)`` names what the call was given, as opposed to what it keeps: ``launch(..., tensors=)`` then
-    puts the addresses of other tensors in their place.  These must be as the recorded ones in all but the address; the caller
-    sees to that (``replay.Replay``), the plan holds no reference to them."""
+    ``plan.operands(ranges)`` names what the call was given, as opposed to what it keeps, by (first, last + 1) address of each
+    tensor: ``launch(..., tensors=)`` then puts the addresses of other tensors in their place.  These must be as the recorded
+    ones in all but the address; the caller sees to that (``replay.Replay``), the plan holds no reference to them."""
 
     def __init__(self):
         self._plan, self._addresses = None, ()
@@ -631,10 +632,10 @@ class Plan:
         k0, k1 = (c_uint32 * n)(*[k[0] for k in keys]), (c_uint32 * n)(*[k[1] for k in keys])
         check(lib().bb_plan_dropout(self._plan, n, k0, k1, *ids), "bb_plan_dropout")
 
-    def operands(self, tensors):
-        n = len(tensors)
-        self._addresses = (c_uint64 * n)(*[t.data_ptr() for t in tensors])
-        check(lib().bb_plan_operands(self._plan, n, self._addresses, (c_int64 * n)(*[extent_bytes(t) for t in tensors])), "bb_plan_operands")
+    def operands(self, ranges):
+        n = len(ranges)
+        self._addresses = (c_uint64 * n)(*[lo for lo, _ in ranges])
+        check(lib().bb_plan_operands(self._plan, n, self._addresses, (c_int64 * n)(*[hi - lo for lo, hi in ranges])), "bb_plan_operands")
 
     def launch(self, step, stream, tensors=()):
         n = len(self._addresses)

@@ -585,6 +585,14 @@ class PipelineModule:
         cls = type(self)
         return cls.forward is PipelineModule.forward and cls.backward is PipelineModule.backward and not {"forward", "backward"} & set(vars(self))
 
+    def stage_memory(self, stage_id):
+        """The blocks of memory that the passes of a stage use, beside what they are given: stash, parameters, gradients, and
+        what its layers hold of their own (running statistics)."""
+        sp = self.stage_params[stage_id]
+        held = [t for layer in self.func_buckets[stage_id] for v in vars(layer).values() if type(v) is dict
+                for pair in v.values() if type(pair) is tuple for t in pair if isinstance(t, torch.Tensor)]
+        return [a for key, a in self._stash_arena.items() if key in (stage_id, (stage_id, "kept"))] + [sp.compute, sp.grad] + held
+
     def pass_buffers(self, stage_id, slot, layers):
         """The tensors of the stage that a pass of ``slot`` over the layers a..b-1 touches, beside what it is given."""
         own = [t for st in self._stash[stage_id][slot][layers[0]: layers[1]] for name, t in st.items() if name != "x0"]

@@ -15,22 +15,33 @@ from operator import is_
 from . import hip
 
 
-def launches_only(layer):
-    """Whether the passes of ``layer`` do nothing that a replay of their launches leaves out.  A class promises it for what it
-    defines by ``launches_only = True`` of its own; a subclass without it may define how its parameters start (below) and
-    no more, and nothing may be put over a method on the object or in place of one in the class."""
-    harmless = {"__init__", "__repr__", "__module__", "__qualname__", "__doc__", "__dict__", "__weakref__", "__annotations__",
-                "__parameters__", "__orig_bases__", "init_params", "num_params", "flops_fwd"}
+# what a class may define without saying anything about its passes
+_HARMLESS = {"__init__", "__repr__", "__module__", "__qualname__", "__doc__", "__dict__", "__weakref__", "__annotations__", "__parameters__",
+             "__orig_bases__", "init_params", "num_params", "flops_fwd"}
+
+
+def _promises(kind):
     promised = False
-    for cls in type(layer).__mro__[:-1]:
+    for cls in kind.__mro__[:-1]:
         own = vars(cls)
         if own.get("launches_only") is True:
             promised = True
             if any(getattr(own.get(m), "__module__", cls.__module__) != cls.__module__ for m in ("forward", "backward")):
                 return False
-        elif not set(own) <= harmless:
+        elif not own.keys() <= _HARMLESS:
             return False
-    return promised and not any(hasattr(type(layer), name) for name in vars(layer))
+    return promised
+
+
+def launches_only(layers):
+    """Whether the passes of ``layers`` do nothing that a replay of their launches leaves out.  A class promises it for what it
+    defines by ``launches_only = True`` of its own; a subclass without it may define how its parameters start
+    (``_HARMLESS``) and no more, and nothing may be put over a method on the object or in place of one in the class."""
+    kinds = set(map(type, layers))
+    if not all(map(_promises, kinds)):
+        return False
+    names = {kind: set(dir(kind)) - {"__dict__"} for kind in kinds}
+    return all(names[type(layer)].isdisjoint(vars(layer)) for layer in layers)
 
 
 def form(t):
@@ -38,14 +49,13 @@ def form(t):
     return None if t is None else (t.shape, t.dtype, t.stride(), t.device, t.data_ptr() & 15)
 
 
-def _ranges(tensors):
-    return [(t.data_ptr(), t.data_ptr() + hip.extent_bytes(t)) for t in tensors]
-
-
-def _apart(ranges, others=()):
-    """Whether none of ``ranges`` meets another one or one of ``others``."""
-    meets = lambda a, b: a[0] < b[1] and b[0] < a[1]
-    return not any(meets(a, b) for i, a in enumerate(ranges) for b in ranges[:i] + list(others))
+def _apart(ranges, others):
+    """Whether none of ``ranges`` meets one of ``others``."""
+    for lo2, hi2 in others:
+        for lo, hi in ranges:
+            if lo < hi2 and lo2 < hi:
+                return False
+    return True
 
 
 class Replay:
@@ -56,15 +66,17 @@ class Replay:
         self.module = module
         self.plans = {}      # (kind, stage, micro-batch) -> {form of the call: (plan, which operand or what it returns)}
         self._stores = stores
-        self._states = {}    # (stage, layers) -> (state that what is stored was recorded under, whether it may be replayed)
+        # (stage, layers) -> (state that what is stored was recorded under, the memory passes use under it; None: not to be replayed)
+        self._states = {}
+        self._kinds = set()  # (kind, stage, layers) of the passes seen
 
     def settled(self, stage_id, ctx, layers):
         """Whether passes of these layers may be replayed; drops what was recorded under another state of theirs."""
         new = self.module.pass_state(stage_id, layers) + ctx.pass_state()
-        old, fit = self._states.get((stage_id, layers), (None, False))
+        old, memory = self._states.get((stage_id, layers), (None, None))
         # identity: the list keeps every object alive, numbers and strings do not change, and dicts are in it with their values
         if old is not None and len(old) == len(new) and all(map(is_, old, new)):
-            return fit
+            return memory is not None
         if old is not None:
             for store in (self.plans,) + self._stores:
                 stale = [k for k in store if k[1] == stage_id]
@@ -72,9 +84,19 @@ class Replay:
                     ctx.stream.synchronize()     # captured graphs are destroyed here
                 for k in stale:
                     del store[k]
-        fit = self.module.passes_launch_only() and all(map(launches_only, self.module.func_buckets[stage_id][slice(*layers)]))
-        self._states[(stage_id, layers)] = (new, fit)
+        fit = self.module.passes_launch_only() and launches_only(self.module.func_buckets[stage_id][slice(*layers)])
+        memory = list(map(hip.address_range, self.module.stage_memory(stage_id) + ctx.buffers())) if fit else None
+        self._states[(stage_id, layers)] = (new, memory)
         return fit
+
+    def _told_apart(self, slot, ctx, ranges, layers):
+        """Whether a recorded pointer can belong to one operand only, and to nothing else that the pass uses."""
+        if not all(_apart([r], ranges[:i]) for i, r in enumerate(ranges)):
+            return False
+        # (first against the stage's blocks of memory, then against what the pass itself has of them: one layer's input lies
+        # in the same block as its output)
+        return _apart(ranges, self._states[(slot[1], layers)][1]) or \
+            _apart(ranges, map(hip.address_range, self.module.pass_buffers(slot[1], slot[2], layers) + ctx.buffers()))
 
     def run(self, slot, ctx, operands, variant, layers, step, issue):
         """``issue()``, or the replay of its launches.  ``operands``: the tensors (or None) the pass is given, which may be others
@@ -89,9 +111,9 @@ class Replay:
             plan, at, out = known
             plan.launch(step, ctx.stream, given)
             return out if at is None else operands[at]
-        own = self.module.pass_buffers(slot[1], slot[2], layers) + ctx.buffers()
-        if not _apart(_ranges(given), _ranges(own)):
-            return issue()     # a pointer into both would be taken for the operand's
+        ranges = list(map(hip.address_range, given))
+        if not self._told_apart(slot, ctx, ranges, layers):
+            return issue()
         ctx.dropout_keys = {}
         try:
             with hip.Plan.record() as plan:
@@ -101,11 +123,15 @@ class Replay:
             ctx.dropout_keys = None
         try:
             plan.dropout(keys)
-            plan.operands(given)
+            plan.operands(ranges)
         except hip.HipKernelError:      # the pass has run; it just cannot be replayed
             return out
-        if not self.settled(slot[1], ctx, layers):     # a layer may make attributes of its own in its first pass
-            return out
+        kind = (slot[0], slot[1], layers)
+        if kind not in self._kinds:
+            # a layer may make attributes of its own in its first pass: what was recorded in front of that is of no use
+            self._kinds.add(kind)
+            if not self.settled(slot[1], ctx, layers):
+                return out
         plans = self.plans.setdefault(slot, {})
         while len(plans) >= self.VARIANTS:
             del plans[next(iter(plans))]

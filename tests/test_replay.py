@@ -32,8 +32,8 @@ class FakePlan:
     def dropout(self, keys):
         pass
 
-    def operands(self, tensors):
-        self.n = len(tensors)
+    def operands(self, ranges):
+        self.n = len(ranges)
 
     def launch(self, step, stream, tensors=()):
         FakePlan.launches.append([t.data_ptr() for t in tensors])
@@ -76,10 +76,10 @@ def stage(monkeypatch):
     monkeypatch.setattr(hip, "Graph", FakeGraph)
     FakePlan.launches = []
     module = object.__new__(PipelineModule)
-    flat = torch.zeros(64)
+    flat, arena = torch.zeros(64), torch.zeros(ROWS * COLS)
     layer = Layer(COLS)
     module.__dict__.update(loss_fn=None, base_seed=3, micro_offset=0, activation_checkpoint_interval=0, dtype=torch.float32,
-                           func_buckets={1: [layer]}, _stash={1: [[{"out": torch.zeros(ROWS, COLS)}]]}, stage_seq={1: [ROWS, ROWS]},
+                           func_buckets={1: [layer]}, _stash={1: [[{"out": arena.view(ROWS, COLS)}]]}, _stash_arena={1: arena}, stage_seq={1: [ROWS, ROWS]},
                            stage_params={1: SimpleNamespace(compute=flat, grad=flat)})
     ctx = StageContext(1, ROWS, torch.float32, "cpu")
     ctx.calls = []
@@ -178,10 +178,10 @@ def test_plan_operands_on_the_host(monkeypatch):
         pass
     a = torch.zeros(16)
     with pytest.raises(hip.HipKernelError, match="overlap"):
-        plan.operands([a, a[8:]])
-    plan.operands([a[:8], a[8:], a[:0]])
+        plan.operands(list(map(hip.address_range, (a, a[8:]))))
+    plan.operands(list(map(hip.address_range, (a[:8], a[8:], a[:0]))))
     with pytest.raises(hip.HipKernelError, match="named"):
-        plan.operands([a])
+        plan.operands([hip.address_range(a)])
     with pytest.raises(hip.HipKernelError):
         plan.launch(0, SimpleNamespace(cuda_stream=0), [a])
     with pytest.raises(hip.HipKernelError):
@@ -261,7 +261,7 @@ def test_layers_that_do_more_than_launch_are_not_replayed(stage, make, replayed)
     only has to do so for every method on the way to the promising base."""
     layer = make()
     stage.module.func_buckets[1] = [layer]
-    assert replay.launches_only(layer) == replayed
+    assert replay.launches_only([layer]) == replayed
     x = torch.randn(ROWS, COLS)
     for _ in range(3):
         stage.forward(x)
@@ -293,6 +293,15 @@ def test_replaying_can_be_switched_off(stage):
 def test_the_frameworks_layers_promise_to_launch_only():
     from bamboo_amd import BottleNeck, DecoderLayer, FinalLayerNorm, SumLast, TransformerLayer
     from perf import cases
-    for layer in (TransformerLayer(64, 1, 64), DecoderLayer(64, 1, 64), FinalLayerNorm(64), SumLast(64), BottleNeck(64, 16), BottleNeck(64, 16, stride=2),
-                  cases._Encoder(64, 1, 64), cases._Block(64, 16)):
-        assert replay.launches_only(layer)
+    layers = (TransformerLayer(64, 1, 64), DecoderLayer(64, 1, 64), FinalLayerNorm(64), SumLast(64), BottleNeck(64, 16), BottleNeck(64, 16, stride=2),
+              cases._Encoder(64, 1, 64), cases._Block(64, 16))
+    assert replay.launches_only(layers) and not replay.launches_only(layers + (Helper(COLS),))
+
+
+def test_address_ranges():
+    t = torch.zeros(4, 6)
+    at, es = t.data_ptr(), t.element_size()
+    for view, last in ((t, 23), (t[1:3], 17), (t.t(), 23), (t[:, 2:4], 21), (t[::2, 1:2], 13), (t[:1].expand(3, 6), 5)):
+        assert hip.address_range(view) == (view.data_ptr(), at + (last + 1) * es)
+    lo, hi = hip.address_range(t[:0])
+    assert lo == hi
