@@ -1252,9 +1252,10 @@ __global__ __launch_bounds__(256) void bn_finish_kernel(int what, int rows, int 
 // w + 16, ..., the sixteen partial sums added in wave order by every thread (a fixed order, the same in every
 // block: all row ranges of a channel normalise with the same bits).  The block of the first row range also writes
 // mean, rstd and the running statistics.  Then y = gamma (x - mean) rstd + beta (+ resid) (ReLU) over the block's
-// rows, eight lanes per row of the 64 channels (128-byte segments).  The tensor is read once; repeating the small
-// strip reduction per row range is cheaper than a launch of its own.  (For few rows that reduction is what the launch waits for:
-// loads for all 256 strips / for the sixteens there are, us: 900 rows x 512 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 / 6.5;
+// rows, eight lanes per row of the 64 channels (128-byte segments).  The tensor is read once, but every block reads all
+// strips of its channels: at 6272 rows 150 KB a block, 38.5 MB a launch of 256 blocks, out of L2 -- 12 times the tensor at 256
+// columns, 3 times at 1024 (L1's read requests: 41.9 and 51.5 MB in all).  What it was taken against is a launch of its own for
+// the statistics (5.4 + 5.5 us against 7.9 at 6272 x 256).  (For few rows the reduction is what the launch waits for: loads for all 256 strips / for the sixteens there are, us: 900 rows x 512 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 / 6.5;
 // the rows of a thread fetched ahead, all of them or the next one, gained nothing.)
 constexpr int BN_STRIP_WAVES = 16, BN_STRIP_MAX = 16;   // 16 * 16 strips = up to 8192 rows
 constexpr int BN_FWD_ROW_RANGES = 64;
@@ -1495,7 +1496,8 @@ __global__ __launch_bounds__(1024) void bn_bwd_finish_apply_kernel(int rows, int
 // The same after a kernel that left the sums per 32-row strip (the GEMM or convolution that produced the gradient,
 // which has the ReLU mask applied already): a block adds up the strips of its 64 channels -- sixteen thread groups
 // take the strips q, q + 16, ... in that order, the sixteen sums are added in group order: the same bits in every
-// block -- and applies the folded dx = k g + a x + b to its rows.
+// block -- and applies the folded dx = k g + a x + b to its rows.  (Every block reads all strips of its channels, at 6272 rows
+// 25.7 MB a launch beside two tensors of 3.2 at 256 columns, 12.8 at 1024: L1's read requests 32.3 and 51.6 MB.)
 template <typename T>
 __global__ __launch_bounds__(1024) void bn_bwd_strips_apply_kernel(int rows, int cols, const float* __restrict__ strips,
                                                                    const T* __restrict__ x, const float* __restrict__ mean,

@@ -4,8 +4,9 @@
 // Stands in for F.linear / torch.matmul and their autograd backward in the reference layer
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:121,127,136-146,158).
 //
-// bf16 data paths: tiles by DMA (gemm_bf16_dma_*), 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for
-// problems of few tiles, and a register-staged kernel for rows of C that are no whole vectors.  fp32: gemm_f32.h.
+// bf16 data paths: tiles by DMA (gemm_bf16_dma_*); 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for weight
+// gradients of few tiles and few tiles of an odd contraction length; a register-staged kernel for rows of C that are no
+// whole vectors (N % 8 != 0, NT).  fp32: gemm_f32.h.
 #include "gemm_kernels.h"
 #include "gemm_f32.h"
 #include "gemm_wave.h"
@@ -89,9 +90,9 @@ enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, 
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
                                             "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r"};
-// The tile of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
-// what ran before), and every kernel adds up a contraction in the same order: a redundant forward and a normal forward
-// of the same layer give the same bits.
+// The kernel of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
+// what ran before): a redundant forward and a normal forward of the same layer give the same bits.  All tiles below add up
+// a contraction in the same order; the wave-sliced kernels (pick_wave) in another.
 static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     //  - Problems of at most one 64x64 tile per CU take those, four stages deep: what such a launch waits for is the chain of
     //    its k-tiles and its epilogue, and the more CUs share the loads the shorter both are.  128x64 / 64x64 tiles (us, back

@@ -385,8 +385,9 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const GemmArgs g
 //       c ^ (4 * (k & 3)); fragments by two ds_read_b64_tr_b16 (the hardware transposes a
 //       4k x 16row block across 16 lanes: lane j reads row k0 + j/4, cols 4*(j%4)..+3 and
 //       receives column j, k0..k0+3).
-// Rows beyond M / N are clamped to the last valid row (their results are never stored);
-// K must be a multiple of 32.
+// Rows beyond M / N are clamped to the last valid row (their results are never stored).
+// A contraction that is no multiple of the k-tile ends in a masked one (mask_tail) where both
+// operands are k-major and where the kernel is built for it (RAGK); the others need whole k-tiles.
 // =========================================================================================
 typedef __attribute__((address_space(3))) void lds_ptr_t;
 typedef const __attribute__((address_space(1))) void gbl_ptr_t;

@@ -1,5 +1,5 @@
-// bf16 weight gradients (and products of any contraction length) that do not fill the chip: 64x64 tiles whose contraction is
-// dealt to the KW waves of a block.
+// bf16 weight gradients, and products whose contraction is no multiple of 32, that do not fill the chip: 64x64 tiles whose
+// contraction is dealt to the KW waves of a block.
 #pragma once
 #include "gemm_kernels.h"
 
@@ -11,7 +11,8 @@
 // segment of eight columns (KW = 8: the whole epilogue is one pass, its operands fetched before the main loop).
 // No operand byte is loaded twice by a block (the slices are disjoint), so this costs no traffic against any other
 // 64x64 tiling; against larger tiles it costs loads, which is why it is for problems of few tiles.  A sum is added up in
-// another order than in the DMA kernels; forward products, whose last bits decide ReLUs, stay with those (64x64 tiles there).
+// another order than in the DMA kernels; forward products, whose last bits decide ReLUs, stay with those (64x64 tiles there)
+// where K % 32 == 0.
 // The contraction may have any length: slices past its end read a line of zeros.
 // 64 rows x BK k of one operand, loaded by one wave.  CONV (k-major): the rows are columns of the 3x3 patch matrix of an NHWC
 // tensor, k its pixels; a 64-wide tile lies inside one tap (the channel count is a multiple of 64), a lane reads the channels
