@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 def test_replayed_plans_equal_eager_launches(hiplib, dropout, ckpt, first_stage):
     """Four batches with optimizer steps: outputs, sent gradients and weights of an engine that replays its passes (from
     the second batch on, with this batch's dropout keys) and of one whose launch observer keeps it eager.  A first stage
-    gets its inputs in other buffers every batch: more variants than the engine remembers."""
+    gets its inputs in other buffers every batch."""
     hid, heads, ffn, S, mb, M, seq = 128, 2, 256, 4, 2, 3, 72
     sid = 0 if first_stage else 1
 
