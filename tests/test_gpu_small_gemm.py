@@ -68,6 +68,10 @@ def test_large_products_of_ragged_contractions(hiplib, layout, M, N, K):
     want, slack = a @ b, K * 2.0 ** -24 * (a.abs() @ b.abs())
     assert ((C.double() - want).abs() <= 2.0 ** -8 * (want.abs() + slack) + slack).all()
     assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()       # nothing written past the rows and columns
+    bias, X = rand(N, seed=3), rand(M, N, seed=4)
+    R = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    hiplib.gemm(lay, A, B, R, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X, alpha=0.5)
+    assert rel(R, 0.5 * want + bias.double() + X.double()) < 1e-2
     if layout == "nt":      # as a member of a group it runs by itself; with dropout, the kernel that decides
         C2, C3 = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
         hiplib.gemm_grouped([hiplib.gemm_desc(lay, A, B, C2), hiplib.gemm_desc(lay, A, B, C3)])
@@ -98,7 +102,7 @@ def test_attention_products_of_ragged_lengths(hiplib, b, h, s, d):
 # (rows, shapes of dy and x): few tiles (eight waves a tile), up to four tiles a CU (four waves), 128x128 tiles
 @pytest.mark.parametrize("rows,shapes", [(1, [(64, 64), (8, 72)]), (31, [(128, 128), (384, 128)]), (1050, [(192, 768), (576, 192)]),
                                          (333, [(512, 2048), (2048, 512), (512, 512)]), (2049, [(1024, 4096), (4096, 1024)]),
-                                         (95, [(1024, 4096), (4096, 1024)])])
+                                         (95, [(1024, 4096), (4096, 1024)]), (100, [(33000, 72), (72, 33000)])])
 def test_weight_gradients_over_ragged_rows(hiplib, rows, shapes):
     descs, want = [], []
     for i, (m, n) in enumerate(shapes):
