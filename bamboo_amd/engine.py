@@ -427,7 +427,7 @@ class PipelineEngine:
     def _promote(self, absorbed, failed_step, curr_step):
         """Turn the shadow layers of ``absorbed`` into active layers of this process
         (reference engine.py:1190-1264)."""
-        self._plans.clear()    # contexts, and with them scratch buffers, may be replaced here
+        self._replay.forget()  # contexts, and with them scratch buffers, may be replaced here
         if not self.eager_recovery:
             # lazy mode keeps CPU mirrors only: materialise the layers from them now
             self.module.build_layers(absorbed, self.param_buffers[absorbed])

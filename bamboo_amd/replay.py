@@ -70,6 +70,12 @@ class Replay:
         self._states = {}
         self._kinds = set()  # (kind, stage, layers) of the passes seen
 
+    def forget(self):
+        """Drop every plan, and with the states the references to what the passes used."""
+        self.plans.clear()
+        self._states.clear()
+        self._kinds.clear()
+
     def settled(self, stage_id, ctx, layers):
         """Whether passes of these layers may be replayed; drops what was recorded under another state of theirs."""
         new = self.module.pass_state(stage_id, layers) + ctx.pass_state()

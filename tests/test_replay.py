@@ -298,6 +298,21 @@ def test_the_frameworks_layers_promise_to_launch_only():
     assert replay.launches_only(layers) and not replay.launches_only(layers + (Helper(COLS),))
 
 
+def test_forgetting_gives_the_buffers_back(stage):
+    """A failover replaces lanes: neither plans nor the states they were compared with keep the old one's scratch."""
+    import weakref
+    stage.ctx.scratch["d"] = torch.zeros(4)
+    x = torch.randn(ROWS, COLS)
+    stage.forward(x)
+    old = weakref.ref(stage.ctx.scratch["d"])
+    del stage.ctx.scratch["d"]
+    assert old() is not None
+    stage.engine._replay.forget()
+    assert old() is None and not stage.engine._replay.plans
+    stage.forward(x)
+    assert stage.issued() == 2
+
+
 def test_address_ranges():
     t = torch.zeros(4, 6)
     at, es = t.data_ptr(), t.element_size()
