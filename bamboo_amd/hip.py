@@ -25,7 +25,7 @@ LN_CODES = {"standard": LN_STANDARD, "annotated": LN_ANNOTATED}
 EXPORTS = (
     "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
     "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
-    "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
+    "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_attention_probs_supported", "bb_attention_probs_fwd", "bb_attention_probs_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
     "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_operands", "bb_plan_launches", "bb_plan_launch", "bb_plan_launch_on", "bb_plan_destroy",
     "bb_adam_multi", "bb_adam_multi_scaled", "bb_grad_clip_workspace", "bb_grad_clip_coef", "bb_cast", "bb_fill_f32",
 )
@@ -103,6 +103,11 @@ def lib():
     L.bb_attention_bwd.argtypes = [c_int] * 6 + [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_float, c_uint32,
                                    c_uint32, c_void_p]
+    L.bb_attention_probs_supported.argtypes = [c_int] * 5
+    L.bb_attention_probs_fwd.argtypes = [c_int] * 6 + [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
+                                         c_void_p, c_float, c_uint32, c_uint32, c_void_p]
+    L.bb_attention_probs_bwd.argtypes = [c_int] * 6 + [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
+                                         c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_float, c_uint32, c_uint32, c_void_p]
     L.bb_dropout_apply.argtypes = [c_int, c_int64, c_void_p, c_void_p, c_float, c_uint32, c_uint32, c_void_p]
     L.bb_dropout_keep_host.argtypes = [c_float, c_uint32, c_uint32, c_uint64]
     L.bb_residual_add.argtypes = [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]
@@ -499,6 +504,44 @@ def attention_bwd(qkv, out, d_out, lse, delta, d_qkv, batch, heads, seq, mask, k
                                  _ptr(d_out), out.stride(0), _ptr(lse), _ptr(delta), c_void_p(dq),
                                  c_void_p(dq + h * es), c_void_p(dq + 2 * h * es), d_qkv.stride(0), _ptr(key_len),
                                  *_drop_args(dropout), stream_ptr(stream)), "bb_attention_bwd")
+
+
+def attention_probs_supported(dtype, batch, heads, seq, head_dim):
+    """Whether :func:`attention_probs_fwd` and its backward take this shape and are the faster way (decided on the host)."""
+    return dtype == torch.float32 and bool(lib().bb_attention_probs_supported(F32, batch, heads, seq, head_dim))
+
+
+def _check_attention_probs(what, qkv, prob, batch, heads, seq, key_len, out=None, d_out=None, d_qkv=None, d_score=None):
+    """As :func:`_check_attention`; prob / d_score: fp32 [batch, heads, seq, seq], contiguous."""
+    if qkv.dim() != 2 or qkv.dtype != torch.float32 or qkv.shape[1] % (3 * heads) != 0:
+        raise HipKernelError(f"{what}: qkv must be fp32 [rows, 3 * heads * d], got {qkv.dtype} {tuple(qkv.shape)} for {heads} heads")
+    rows, h = batch * seq, qkv.shape[1] // 3
+    for name, t, width in (("qkv", qkv, 3 * h), ("d_qkv", d_qkv, 3 * h), ("out", out, h), ("d_out", d_out, h)):
+        if t is not None and (t.dim() != 2 or tuple(t.shape) != (rows, width) or t.stride(1) != 1 or t.stride(0) < width or
+                              t.dtype != qkv.dtype):
+            raise HipKernelError(f"{what}: {name} must be [{rows}, {width}] of {qkv.dtype} with unit inner stride for batch={batch} "
+                                 f"heads={heads} seq={seq}, got {tuple(t.shape)} {t.dtype} strides {t.stride()}")
+    _vector(what, batch * heads * seq * seq, torch.float32, prob=prob, d_score=d_score)
+    _vector(what, batch, torch.int32, key_len=key_len)
+
+
+def attention_probs_fwd(qkv, out, prob, batch, heads, seq, mask, key_len=None, stream=None, dropout=None):
+    """:func:`attention_fwd` in fp32, keeping the probabilities (in front of dropout) in ``prob``: fp32 [batch, heads, seq, seq]."""
+    _check_attention_probs("attention_probs_fwd", qkv, prob, batch, heads, seq, key_len, out=out)
+    h, es, q = qkv.shape[1] // 3, qkv.element_size(), qkv.data_ptr()
+    check(lib().bb_attention_probs_fwd(dtype_code(qkv.dtype), mask, batch, heads, seq, h // heads, c_void_p(q), c_void_p(q + h * es),
+                                       c_void_p(q + 2 * h * es), qkv.stride(0), _ptr(out), out.stride(0), _ptr(prob), _ptr(key_len),
+                                       *_drop_args(dropout), stream_ptr(stream)), "bb_attention_probs_fwd")
+
+
+def attention_probs_bwd(qkv, d_out, prob, d_score, d_qkv, batch, heads, seq, mask, key_len=None, stream=None, dropout=None):
+    """Input gradients of :func:`attention_probs_fwd`; ``d_score``: scratch like ``prob``."""
+    _check_attention_probs("attention_probs_bwd", qkv, prob, batch, heads, seq, key_len, d_out=d_out, d_qkv=d_qkv, d_score=d_score)
+    h, es, q, dq = qkv.shape[1] // 3, qkv.element_size(), qkv.data_ptr(), d_qkv.data_ptr()
+    check(lib().bb_attention_probs_bwd(dtype_code(qkv.dtype), mask, batch, heads, seq, h // heads, c_void_p(q), c_void_p(q + h * es),
+                                       c_void_p(q + 2 * h * es), qkv.stride(0), _ptr(d_out), d_out.stride(0), _ptr(prob), _ptr(d_score),
+                                       c_void_p(dq), c_void_p(dq + h * es), c_void_p(dq + 2 * h * es), d_qkv.stride(0), _ptr(key_len),
+                                       *_drop_args(dropout), stream_ptr(stream)), "bb_attention_probs_bwd")
 
 
 def dropout_apply(src, dst, p, key, stream=None):

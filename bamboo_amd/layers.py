@@ -211,10 +211,15 @@ class TransformerLayer:
     def fused_attention(self, ctx):
         """bf16 with 64- or 128-wide heads, or with an even number of 32-wide heads (the reference's GPT-2 script
         defaults to 512 / 16 = 32, gpt2.py:212-214: the kernels then take the heads in pairs), runs the fused attention
-        kernels (no score matrix in HBM).  Everything else -- fp32, the correctness configuration, and bf16 with another
-        head width -- materialises the probabilities like the reference does: batched head products and the masked
-        softmax kernels."""
+        kernels (no score matrix in HBM).  Everything else keeps the probabilities like the reference does: fp32, the
+        correctness configuration, with kernels of its own where they take the shape (``kept_probs_kernels``), the rest,
+        bf16 with another head width among it, as batched head products and masked softmax kernels."""
         return ctx.dtype == torch.bfloat16 and (self.head_dim in (64, 128) or (self.head_dim == 32 and self.heads % 2 == 0))
+
+    def kept_probs_kernels(self, ctx):
+        """fp32 attention that keeps the probabilities in one launch forward and two backward; a matter of the shape alone, so
+        that a redundant forward and a normal forward of the same layer take the same kernels."""
+        return hip.attention_probs_supported(ctx.dtype, ctx.batch, self.heads, ctx.seq, self.head_dim)
 
     def stash_specs(self, ctx):
         R, h, f = ctx.rows, self.hidden, self.ffn
@@ -242,7 +247,7 @@ class TransformerLayer:
         return specs + self.forward_scratch_specs(ctx)
 
     def forward_scratch_specs(self, ctx):
-        if self.dropout > 0 and not self.fused_attention(ctx):
+        if self.dropout > 0 and not self.fused_attention(ctx) and not self.kept_probs_kernels(ctx):
             return [("prob_drop", (ctx.batch, self.heads, ctx.seq, ctx.seq), ctx.dtype)]   # dropped-out probabilities
         return []
 
@@ -282,6 +287,10 @@ class TransformerLayer:
             hip.attention_fwd(st["qkv"], st["ctx"], st["lse"], ctx.batch, self.heads, s, hip.MASK_CODES[mask],
                               ctx.key_len if mask == "key_padding" else None, stream=ctx.stream, dropout=drop)
             return
+        if self.kept_probs_kernels(ctx):
+            hip.attention_probs_fwd(st["qkv"], st["ctx"], st["prob"], ctx.batch, self.heads, s, hip.MASK_CODES[mask],
+                                    ctx.key_len if mask == "key_padding" else None, stream=ctx.stream, dropout=drop)
+            return
         es = st["qkv"].element_size()
         q = st["qkv"].data_ptr()
         k, v = q + h * es, q + 2 * h * es
@@ -309,6 +318,11 @@ class TransformerLayer:
             hip.attention_bwd(st["qkv"], st["ctx"], d_ctx, st["lse"], delta, d_qkv, ctx.batch, self.heads, s,
                               hip.MASK_CODES[mask], ctx.key_len if mask == "key_padding" else None, stream=ctx.stream,
                               dropout=drop)
+            return
+        if self.kept_probs_kernels(ctx):
+            hip.attention_probs_bwd(st["qkv"], d_ctx, st["prob"], ctx.buf("d_prob", tuple(st["prob"].shape)), d_qkv, ctx.batch,
+                                    self.heads, s, hip.MASK_CODES[mask], ctx.key_len if mask == "key_padding" else None,
+                                    stream=ctx.stream, dropout=drop)
             return
         es = st["qkv"].element_size()
         q = st["qkv"].data_ptr()
