@@ -271,6 +271,21 @@ static constexpr int kF32SplitGroups = 2, kF32SplitBN = 32;
 static bool pick_f32_split(int M, int N, int K, int64_t batches, int layout) {
     return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches < 2 * 256 && K >= 512;
 }
+// Of what is left for the tiles of 64x64 and 64x32, problems of at most 128 64x64 tiles take four blocks a tile instead, with the same
+// bits (gemm_f32_quarter_kernel): until then every CU has at most two of them.  Larger tiles / this (us, back to back): NT
+// 128x128x128 7.0 / 5.2, 512x512x256 (64 tiles) 10.7 / 5.8, 1000x448x448 (112) 16.3 / 10.2, 1024x512x512 (128) 11.2 / 11.4,
+// 1024x512x2048 32.3 / 29.9, 512x1536x256 (192) 11.4 / 11.2, 1000x1344x448 (336) 25.1 / 26.8, 2048x768x768 (384) 29.0 / 37.9; NN alike.
+static bool pick_f32_quarter(int M, int N, int64_t batches, int layout) {
+    return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches <= 128;
+}
+template <bool TA, bool TB, int KG> static int launch_f32_quarter(GemmArgs& g, int batches, hipStream_t st) {
+    auto kern = gemm_f32_quarter_kernel<TA, TB, KG>;
+    g.tiles_m = (g.M + 31) / 32;
+    g.tiles_n = (g.N + 31) / 32;
+    bb_launch(kern, dim3(g.tiles_m * g.tiles_n, 1, batches), dim3(256 * KG), kF32QuarterLds, st, g);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
 template <bool TA, bool TB> static int launch_f32_wave(GemmArgs& g, int batches, hipStream_t st) {
     auto kern = gemm_f32_wave_kernel<TA, TB>;
     g.tiles_m = (g.M + 31) / 32;
@@ -291,8 +306,11 @@ template <bool TA, bool TB, int BN, bool WIDE = false> static int launch_f32(Gem
 template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hipStream_t st) {
     if (f32_wide(g.lda, g.ldb)) return launch_f32<TA, TB, 64, true>(g, batches, st);
     if (pick_f32_wave(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) return launch_f32_wave<TA, TB>(g, batches, st);
-    if (pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) {
-        if constexpr (!TA) return launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
+    const bool split = pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT);
+    if constexpr (!TA) {
+        if (pick_f32_quarter(g.M, g.N, batches, TB ? BB_NN : BB_NT))
+            return split ? launch_f32_quarter<TA, TB, 2>(g, batches, st) : launch_f32_quarter<TA, TB, 1>(g, batches, st);
+        if (split) return launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
     }
     return launch_f32<TA, TB, 64>(g, batches, st);
 }
@@ -311,9 +329,12 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
     }
     else if (f32_wide(d->lda, d->ldb)) snprintf(out, out_len, "f32_%s_64x64wide", layouts[d->layout]);
     else if (pick_f32_wave(d->M, d->N, d->K, batches, d->layout)) snprintf(out, out_len, "f32_%s_wave32x32k%d", layouts[d->layout], kF32Waves);
-    else if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
-        snprintf(out, out_len, "f32_%s_64x%dk%d", layouts[d->layout], kF32SplitBN, kF32SplitGroups);
-    else snprintf(out, out_len, "f32_%s_64x64", layouts[d->layout]);
+    else {
+        const char* quarter = pick_f32_quarter(d->M, d->N, batches, d->layout) ? "quarter" : "";
+        if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
+            snprintf(out, out_len, "f32_%s_%s64x%dk%d", layouts[d->layout], quarter, kF32SplitBN, kF32SplitGroups);
+        else snprintf(out, out_len, "f32_%s_%s64x64", layouts[d->layout], quarter);
+    }
     return BB_OK;
 }
 

@@ -1,5 +1,5 @@
 // fp32 GEMM: v_mfma_f32_32x32x2_f32 on 64x64 tiles (four waves of 32x32), on 64x32 tiles whose contraction two groups of
-// two waves share, or on 32x32 tiles whose contraction four waves share.
+// two waves share, or on 32x32 tiles whose contraction four waves share; v_mfma_f32_16x16x4_f32 on quarters of a 64x64 tile.
 #pragma once
 #include "gemm_kernels.h"
 
@@ -20,7 +20,8 @@
 // (volatile: pairs of reads merged into one instruction have no room for the stage's offset, i.e. cost an addition each)
 typedef const volatile __attribute__((address_space(3))) float lds_f32;
 // WIDE: rows of 2^22 elements and more, whose tile does not fit the 32-bit offsets: 64-bit addresses, added up per load
-template <int ROWS, bool KM, int NW = 4, bool WIDE = false> struct F32Operand {
+// QUADS: read in groups of four k (16x16x4 instructions): 32-wide rows keep columns 0..15 of k % 4 >= 2 at the place of columns 16..31
+template <int ROWS, bool KM, int NW = 4, bool WIDE = false, bool QUADS = false> struct F32Operand {
     using Offset = std::conditional_t<WIDE, int64_t, unsigned>;
     static constexpr int BYTES = ROWS * 32 * 4, ROUNDS = BYTES / (1024 * NW);   // NW waves load a stage
     const float* base;          // wave-uniform: the tile's first row (K-contiguous) / column (k-major), the next k-tile
@@ -38,7 +39,7 @@ template <int ROWS, bool KM, int NW = 4, bool WIDE = false> struct F32Operand {
                 off[i] = (Offset)((int64_t)min(r, rows - 1 - row0) * ld + c * 4) * (Offset)4;
             } else {
                 constexpr int CPR = ROWS / 4, RPI = 64 / CPR;   // 16-byte chunks per k-row, k-rows per instruction
-                const int k = q * RPI + lane / CPR, c = (lane % CPR) ^ (ROWS == 64 ? 8 * (k & 1) : 0);
+                const int k = q * RPI + lane / CPR, c = (lane % CPR) ^ (ROWS == 64 ? 8 * (k & 1) : QUADS ? 4 * ((k >> 1) & 1) : 0);
                 k_lane[i] = k;
                 off[i] = (Offset)((int64_t)k * ld + min(c * 4, rows - 4 - row0)) * (Offset)4;
             }
@@ -387,4 +388,153 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_wave_grouped_kernel(const Gro
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
     gemm_f32_wave_body<TA, TB>(G.p[pi], lid - G.first_block[pi], 0, true);
+}
+
+// Problems of few 64x64 tiles: each tile as four blocks of 32x32, a wave 16x16 of it by v_mfma_f32_16x16x4_f32.  What bounds such a
+// problem is the chain of one tile: a 64x64 tile's wave spends 32 matrix cycles on every k, this one 8 on four times the CUs, and
+// four k-tiles of 64 are in flight from the start (us against the larger tiles: see pick_f32_quarter).  Both instructions add their k one by one, ascending (checked bit for bit against
+// a chain of multiply-adds), so the result has the bits of the larger tile: which kernel runs a product changes none of them.
+// KG: groups of four waves that share the contraction as those of the 64x32 tiles do (16-wide halves of every 32, added in order).
+constexpr int kF32QuarterStages = 4;
+constexpr int kF32QuarterLds = kF32QuarterStages * 2 * 2 * 32 * 128;
+template <bool TA, bool TB, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void gemm_f32_quarter_kernel(const GemmArgs g) {
+    constexpr int NW = 4 * KG, NST = kF32QuarterStages;
+    using OpA = F32Operand<32, TA, 4, false, true>;     // a k-tile of 32: four instructions
+    using OpB = F32Operand<32, TB, 4, false, true>;
+    constexpr int TILE = OpA::BYTES + OpB::BYTES, STAGE = 2 * TILE, LOADS = 16 / NW;   // instructions a wave and stage
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int quad = wave & 3, grp = wave >> 2, wm = quad & 1, wn = quad >> 1;
+    int tile_m, tile_n;
+    tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    const int m0 = tile_m * 32, n0 = tile_n * 32;
+    const int b1 = blockIdx.z / g.nb2, b2 = blockIdx.z % g.nb2;
+    const int64_t coff = b1 * g.sC1 + b2 * g.sC2;
+    // a stage is two 32-wide k-tiles of both operands; with one group every wave loads a quarter of each, with two a group loads one k-tile
+    OpA opa;
+    OpB opb;
+    opa.init((const float*)g.A + b1 * g.sA1 + b2 * g.sA2, g.lda, m0, g.M, lane, quad);
+    opb.init((const float*)g.B + b1 * g.sB1 + b2 * g.sB2, g.ldb, n0, g.N, lane, quad);
+    if (KG == 2 && grp == 1) {
+        opa.base += opa.step;
+        opb.base += opb.step;
+    }
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t*)smem;
+
+    // what the epilogue reads: lane = column, register r = row acc_m + r
+    const int n = n0 + wn * 16 + (lane & 15), acc_m = m0 + wm * 16 + 4 * (lane >> 4), nc = min(n, g.N - 1);
+    const float* opnd = (const float*)epilogue_operand(g);
+    const int64_t ld_pre = opnd ? g.ldaux : g.ldc;
+    if (!opnd && g.accumulate) opnd = (const float*)g.C;
+    float bias = 0.f, pre[4] = {0.f, 0.f, 0.f, 0.f};
+    if (grp == 0) {
+        if (g.bias) bias = ((const float*)g.bias)[nc];
+        if (opnd) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pre[e] = opnd[coff + (int64_t)min(acc_m + e, g.M - 1) * ld_pre + nc];
+        }
+    }
+
+    const int KS = (g.K + 63) / 64;   // stages of 64
+    int into = 0, issued = 0;
+    auto issue = [&]() {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (KG == 2 && h != grp) continue;
+            const int left = g.K - issued * 64 - h * 32;
+            const unsigned at = lds0 + into + h * TILE;
+            opa.issue(at, quad, left, lane);
+            opb.issue(at + OpA::BYTES, quad, left, lane);
+        }
+        if (KG == 2) {   // the other group's k-tile
+            opa.base += opa.step;
+            opb.base += opb.step;
+        }
+        into = into == (NST - 1) * STAGE ? 0 : into + STAGE;
+        ++issued;
+    };
+    // stage s has landed when at most (stages issued behind it) x LOADS are in flight: completion is in order
+    auto landed = [&](int behind) {
+        asm volatile("" ::: "memory");
+        if (behind >= 3) wait_vmcnt_lgkm0<3 * LOADS>();
+        else if (behind == 2) wait_vmcnt_lgkm0<2 * LOADS>();
+        else if (behind == 1) wait_vmcnt_lgkm0<LOADS>();
+        else wait_vmcnt_lgkm0<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    static_assert(NST == 4, "landed()");
+
+    constexpr int NC = 8 / KG;         // chunks of four k of a k-tile that this wave multiplies
+    const int fr = lane & 15, kq = lane >> 4;
+    unsigned at_a[TA ? 1 : NC], at_b[TB ? 1 : NC];
+    const int ra = wm * 16 + fr, rb = wn * 16 + fr;
+    if constexpr (TA) at_a[0] = lds0 + ((4 * grp * NC + kq) * 32 + (ra ^ (16 * (kq >> 1)))) * 4;
+    else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) at_a[c] = lds0 + ra * 128 + (((grp * NC + c) ^ ((ra >> 1) & 7)) << 4) + 4 * kq;
+    }
+    if constexpr (TB) at_b[0] = lds0 + OpA::BYTES + ((4 * grp * NC + kq) * 32 + (rb ^ (16 * (kq >> 1)))) * 4;
+    else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) at_b[c] = lds0 + OpA::BYTES + rb * 128 + (((grp * NC + c) ^ ((rb >> 1) & 7)) << 4) + 4 * kq;
+    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float fa[2][NC], fb[2][NC];
+    auto load = [&](auto off_c, float (&a)[NC], float (&b)[NC]) {
+        constexpr int OFF = decltype(off_c)::value;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            a[c] = TA ? *((lds_f32*)at_a[0] + OFF / 4 + c * 128) : *((lds_f32*)at_a[TA ? 0 : c] + OFF / 4);
+            b[c] = TB ? *((lds_f32*)at_b[0] + OFF / 4 + c * 128) : *((lds_f32*)at_b[TB ? 0 : c] + OFF / 4);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const float (&a)[NC], const float (&b)[NC]) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c], b[c], acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // a stage: its second k-tile is read under the first one's products, the next stage's first -- behind the barrier that makes it
+    // visible and frees the stage before this one -- under the second one's
+    auto stage = [&](int s, auto stage_c) {
+        constexpr int S = decltype(stage_c)::value, NX = (S + 1) % NST;
+        load(std::integral_constant<int, S * STAGE + TILE>{}, fa[1], fb[1]);
+        multiply(fa[0], fb[0]);
+        if (s + 1 < KS) {
+            landed(issued - s - 2);
+            if (issued < KS) issue();
+        }
+        load(std::integral_constant<int, NX * STAGE>{}, fa[0], fb[0]);   // (behind the last stage: of one that is there, for nobody)
+        multiply(fa[1], fb[1]);
+    };
+    if (KS > 0) {
+        for (int p = 0; p < NST && p < KS; ++p) issue();
+        landed(issued - 1);
+        load(std::integral_constant<int, 0>{}, fa[0], fb[0]);
+        int s = 0;
+        for (; s + NST <= KS; s += NST) {
+            stage(s, std::integral_constant<int, 0>{});
+            stage(s + 1, std::integral_constant<int, 1>{});
+            stage(s + 2, std::integral_constant<int, 2>{});
+            stage(s + 3, std::integral_constant<int, 3>{});
+        }
+        if (s < KS) stage(s, std::integral_constant<int, 0>{});
+        if (s + 1 < KS) stage(s + 1, std::integral_constant<int, 1>{});
+        if (s + 2 < KS) stage(s + 2, std::integral_constant<int, 2>{});
+    }
+    if constexpr (KG > 1) {
+        float* part = (float*)smem + quad * (4 * 64);
+        __syncthreads();
+        if (grp == 1) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[r * 64 + lane] = acc[r];
+        }
+        __syncthreads();
+        if (grp == 1) return;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] += part[r * 64 + lane];
+    }
+    if (n < g.N) epilogue_f32<4>(g, coff, acc_m, n, bias, pre, acc);
 }

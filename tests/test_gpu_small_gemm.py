@@ -206,3 +206,35 @@ def test_fp32_rows_of_any_pitch(hiplib, layout, M, N, K, ld):
     a, b = (a.t() if layout == "tn" else a), (b.t() if layout == "nt" else b)
     bound = K * 2.0 ** -24 * (a.abs() @ b.abs())
     assert ((C.double().cpu() - a @ b).abs() <= bound).all() and torch.equal(C, C2) and torch.equal(C, C3)
+
+
+# Products of few tiles against the same rows inside a product of many, which the larger tiles run: the same bits.  Contractions of
+# a part of a k-tile, around 64, around the four stages of the ring, and long ones that two groups share; rows and columns of
+# less than a tile, with remainders, and the most tiles the rule takes (128).
+@pytest.mark.parametrize("M,N,K", [(4, 4, 4), (32, 36, 60), (33, 64, 64), (70, 100, 68), (128, 128, 252), (100, 72, 256), (64, 260, 260), (512, 900, 320),
+                                   (36, 28, 512), (70, 132, 524), (130, 64, 580), (1024, 512, 1036)])
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+def test_fp32_quarter_tiles_have_the_bits_of_whole_ones(hiplib, layout, M, N, K):
+    if layout == "nn" and K <= 128:
+        pytest.skip("32x32 tiles with a slice a wave")
+    lay = hiplib.NT if layout == "nt" else hiplib.NN
+    mk = lambda *shape, seed: torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
+    rows = max(M, 64 * (130 * 64 // N + 1))     # more than 128 tiles, fewer than the 512 from which on no contraction is shared
+    A, B = mk(rows, K, seed=1), mk(*((N, K) if layout == "nt" else (K, N)), seed=2)
+    bias, X, G = mk(N, seed=3), mk(rows, N, seed=4), mk(rows, N, seed=5)
+    few, many = hiplib.gemm_variant(hiplib.gemm_desc(lay, A[:M], B, G[:M])), hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, G))
+    assert few == many.replace("64x", "quarter64x", 1) and "quarter" not in many
+    for kw in (dict(bias=bias, epilogue=hiplib.EPI_RESIDUAL), dict(epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_GELU_TANH), dict(accumulate=True, alpha=0.5),
+               dict(epilogue=hiplib.EPI_MUL_POS)):
+        out = []
+        for m in (M, rows):
+            C, aux = G[:m].clone(), X[:m].clone()
+            extra = {hiplib.EPI_RESIDUAL: dict(resid=aux), hiplib.EPI_ACT_DACT: dict(aux_out=aux), hiplib.EPI_MUL_POS: dict(aux_in=aux, resid=G[:m])}
+            hiplib.gemm(lay, A[:m], B, C, **kw, **extra.get(kw.get("epilogue"), {}))
+            out.append((C[:M], aux[:M]))
+        assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), kw
+    prod = A[:M].double().cpu() @ (B.double().cpu().t() if layout == "nt" else B.double().cpu())
+    C = torch.full((M, N), float("nan"), device=DEV)
+    hiplib.gemm(lay, A[:M], B, C)
+    bound = K * 2.0 ** -24 * (A[:M].double().cpu().abs() @ (B.double().cpu().t() if layout == "nt" else B.double().cpu()).abs())
+    assert bool(((C.double().cpu() - prod).abs() <= bound).all())
