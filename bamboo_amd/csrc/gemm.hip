@@ -96,9 +96,10 @@ static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8d
 static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     //  - Problems of at most one 64x64 tile per CU take those, four stages deep: what such a launch waits for is the chain of
     //    its k-tiles and its epilogue, and the more CUs share the loads the shorter both are.  128x64 / 64x64 tiles (us, back
-    //    to back): NT 256x512x512 6.8 / 6.3, 1050x512x2048 15.8 / 12.7, 3136x256x1024 10.5 / 9.0; NN 1050x512x1536 12.0 / 9.7;
-    //    eight stages 5 % slower (a second block finds no room), 408 tiles equal, more tiles slower.  The shapes the larger
-    //    tiles do not take (fewer than 128 rows or columns) run on it too.
+    //    to back): NT 640x1024x4096 (160 tiles of 64x64) 24.1 / 16.4, 2048x1024x4096 (512) 26.3 / 27.9, 1500x1344x448 (504) 6.5 /
+    //    7.5; NN 24.2 / 17.1, 25.5 / 29.8, 8.5 / 7.6.  One-wave tiles of 32x32 on four times the CUs: slower everywhere (100x1600x6400
+    //    21.4 / 24.0), a wave has too many transfers to issue.  The shapes the larger tiles do not take (fewer than 128
+    //    rows or columns) run on it too.
     const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches;
     if (layout != BB_TN && K % 64 == 0 && K > 0 && N % 8 == 0 && (t64 <= 256 || M < 128 || N < 128)) return D64x64k64s4;
     if ((K % 32 != 0 && layout != BB_TN) || K < 64 || M < 128 || N < 128 || N % 8 != 0) {
@@ -131,16 +132,20 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches;
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
-    //  - Problems with so few 128x128 tiles that half the CUs would idle (the 256-channel convolutions of a
-    //    ResNet stage: 98 tiles) take 128x64 tiles: twice the blocks.
-    //    (a k-major operand needs 128 rows for its swizzle, so NT narrows N and NN narrows M; TN keeps
-    //    128x128).
-    //  - A short forward contraction (K <= 512: the 1x1 convolution out of 256 channels) leaves a launch that is mostly
-    //    its epilogue: 128x64 tiles, so that every CU stores a share (6272x1024x256: 15 us on 100 tiles of 256x128,
-    //    13 us on 784 of 128x64; the input gradient of the same shape gains nothing from 64x128 tiles).
-    if (K <= 512 && nt) return k64 ? D128x64k64s3 : D128x64s3;
-    if (t128 <= 128 && nt) return k64 ? D128x64k64s3 : D128x64s3;
-    if (t128 <= 128 && nn) return k64 ? D64x128k64s3 : D64x128s3;
+    //  - Problems of at most 400 tiles of 128x64 (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle) take those: up
+    //    to two per CU, whose chains run under each other.  128x128 / this, plain and with a residual (us): NT 1200x1600x1600 (250
+    //    tiles) 20.3 23.5 / 12.6 13.5, 3000x832x832 (312) 12.7 16.1 / 11.4 12.3, 4096x768x768 (384) 12.4 14.3 / 13.6 11.7, x3072
+    //    34.7 37.5 / 32.6 31.7, 3136x1024x256 (400) 8.3 9.7 / 7.7 8.3, 8192x512x512 (512) 10.8 12.0 / 12.8 10.5; NN 21.0 24.0 / 12.4
+    //    13.1, 13.2 16.2 / 11.3 12.0, 11.9 14.2 / 13.8 11.8, 34.5 37.4 / 31.6 31.3, 8.0 9.6 / 7.7 8.4, 10.3 11.6 / 13.9 14.2.  More of
+    //    them: 256x128 tiles, also for short contractions (NT 6272x1024x256 12.8 14.0 on 128x64, 10.3 11.4 on 256x128).
+    //    32-wide k-tiles (K % 64 != 0) as before: 128x64 tiles up to 128 tiles of 128x128 and for short forward contractions.
+    if (k64) {
+        if (nt && (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches <= 400) return D128x64k64s3;
+        if (nn && (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches <= 400) return D64x128k64s3;
+    } else {
+        if ((K <= 512 || t128 <= 128) && nt) return D128x64s3;
+        if (t128 <= 128 && nn) return D64x128s3;
+    }
     //  - NT problems whose 256x256 tiles would fill under 70 % of their rounds may take 256x192 tiles (six
     //    accumulator tiles per wave, about 9 % below the 256x256 tile at equal fill) instead of falling back
     //    to 128x128: compared by the share of the occupied tile slots that is real output.  (Alone, the QKV

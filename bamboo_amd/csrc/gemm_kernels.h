@@ -429,6 +429,13 @@ __device__ __forceinline__ void dma16_at(const void* src, unsigned lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "m0");
 }
 
+// the same by no lane or by all of them (live: 0 or -1): a masked-off transfer moves nothing, but is counted like any other, so
+// that a loop may issue -- and wait for -- the same number of them whether there is something left to load or not.  The
+// callers' waves are full.
+__device__ __forceinline__ void dma16_masked(const void* src, unsigned lds, int live) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(live) : "m0");
+}
+
 // 3x3 convolution (stride 1, pad 1, NHWC) as an implicit GEMM: the patch matrix [pixels, 9 * channels] is never
 // built, the A loader gathers its rows from the activation tensor instead.
 struct ConvArgs {
@@ -619,6 +626,13 @@ template <int BR, bool KM, int NW, int BK = 32, bool VIS = false, int CONV = 0> 
         next_pixels(I);
         if constexpr (I == ROUNDS - 1) advance();
     }
+    // (past the end the sources run on: nothing is read there)
+    template <int I> __device__ __forceinline__ void issue_masked(unsigned tile, int wave, int live) {
+        dma16_masked(source(I), tile + (I * NW + wave) * 1024, live);
+        src[I] += step;
+        next_pixels(I);
+        if constexpr (I == ROUNDS - 1) advance();
+    }
 };
 
 // per-lane fragment offsets (bytes inside an operand tile) and the fragment fetch
@@ -746,6 +760,8 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // bias gradient riding along: the waves of the first block column (and first wave column)
     // add up the A fragments they hold anyway: lane (m, kg) sees 8 of the 16 k values per step
     const bool do_colsum = AKM && g.colsum != nullptr && tile_n == 0 && wn == 0;
+    // the main loop of the small tiles, see there
+    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && TM * TN <= 2 && !AKM && !RAGK && !VIS;
     float csum[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) csum[i] = 0.f;
@@ -838,13 +854,15 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     constexpr int NP = (TN + 1) / 2;   // pairs per row of accumulator tiles, the last one possibly a single
     const int prow = lane >> 3, pcol = (lane & 7) * 8;
     // Only on the large tiles (one block per CU, two waves per SIMD whatever the kernel's register count) and on the
-    // 64x64 one (a single patch, few accumulators): on the others the 32 registers would cost a resident block.
+    // small ones (a single patch, few accumulators): on the others the 32 registers would cost a resident block.
     // Some of the other kernels fetch a patch's operand(s) in one go at the top of that patch: the pointers of GemmArgs
     // may alias as far as the compiler knows, so left inside the row loop every load waits behind the previous row's
     // store (four round trips in a row per patch instead of one).
     // (HOIST: where that does not cost a resident block -- the kernels with the BatchNorm backward sums, whose three
     // operand reads per row are most of their epilogue)
-    constexpr bool PREF = (BM * BN >= 256 * 128 || BM * BN == 64 * 64) && !VIS && CONV == 0 && STATS == 0;
+    // EARLY: the kernels whose waves finish one patch each and have the registers fetch it -- and the bias -- before the main loop.
+    constexpr bool EARLY = AHEAD && TM * NP == 1;
+    constexpr bool PREF = (BM * BN >= 256 * 128 || EARLY) && !VIS && CONV == 0 && STATS == 0;
     constexpr bool HOIST = STATS == 2;
     const bf16* opnd = PREF || HOIST ? epilogue_operand(g) : nullptr;
     u32x4 opc[PREF || HOIST ? 4 : 1], opn[PREF ? 4 : 1];
@@ -871,7 +889,106 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         }
     };
 
-    if constexpr (BK == 64) {
+    // bias of the lane's eight columns, mean and 1 / deviation of the normalisation (STATS 2)
+    float b8[8], mu8[8], rs8[8];
+    auto column_values = [&](bool live, int n) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b8[e] = mu8[e] = rs8[e] = 0.f;
+        if (g.bias && live) load_vec((const bf16*)g.bias + n, b8);
+        if constexpr (STATS == 2) {
+            if (live) {
+                const f32x4 m_lo = *(const f32x4*)(bn.mean + n), m_hi = *(const f32x4*)(bn.mean + n + 4);
+                const f32x4 r_lo = *(const f32x4*)(bn.rstd + n), r_hi = *(const f32x4*)(bn.rstd + n + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    mu8[e] = m_lo[e];
+                    mu8[4 + e] = m_hi[e];
+                    rs8[e] = r_lo[e];
+                    rs8[4 + e] = r_hi[e];
+                }
+            }
+        }
+    };
+    if constexpr (EARLY) {
+        const int n = n0 + wn * WTN + pcol;
+        column_values((TN >= 2 || pcol < 32) && n < g.N, n);
+        fetch(std::integral_constant<int, 0>{}, opc);
+    }
+
+    if constexpr (AHEAD) {
+        // Small tiles, of which a CU holds one or two: what they wait for is the chain of one k-tile -- the wait for its loads, a
+        // barrier, LDS reads, a few matrix instructions.  So all fragments of a k-tile are read a whole k-tile ahead into a
+        // second register set, under the matrix instructions of the one before: one LDS round trip and one barrier a k-tile,
+        // nothing behind them.  All stages are in flight at first; k-tile kt + STAGES goes into the stage of k-tile kt, which the
+        // barrier in front of it has shown to be read.  The loop has no branch but its end: past the last k-tile the transfers
+        // are masked off (as branches around them the same loop was slower than the one below, 100x1600x6400 42 us: accumulators moved
+        // between register sets at every merge).  Before (halves of a k-tile read half a k-tile ahead) and now, us: 64x64 tiles, NT
+        // 1024x512x2048 11.7 / 9.5, 512x1024x4096 20.0 / 15.7, 100x1600x6400 29.1 / 21.3, 0.25 -> 0.17 us a k-tile, where LDS moves
+        // 32 KB of fragments and 16 KB of transfers; 128x64 and 64x128 gain by the epilogue's early operands: 2043x768x768 with a
+        // residual 8.6 / 7.8, x3072 21.2 / 20.2 (NT), 21.0 / 19.4 (NN).
+        struct Tile {
+            bf16x8 a[4][TM], b[4][TN];
+        } t0, t1;
+        constexpr int NM = 4 * TM * TN, NF = 4 * (TM + TN), RM = NM / 2;   // matrix instructions, fragments; reads go with the first RM
+        const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t*)smem;
+        const int uwave = __builtin_amdgcn_readfirstlane(wave);
+        int stage = 0;     // of the k-tile that is multiplied
+        auto feed = [&](auto k_c, unsigned at, int live) {
+            constexpr int k = decltype(k_c)::value;
+            if constexpr (k < OpA::ROUNDS) opa.template issue_masked<k>(at, uwave, live);
+            else opb.template issue_masked<k - OpA::ROUNDS>(at + OpA::BYTES, uwave, live);
+        };
+        auto step = [&](const Tile& cur, Tile& nxt, int kt) {
+            // k-tile kt + 1 has landed (in-order completion: the STAGES - 2 after it may be in flight), every wave has read k-tile kt
+            asm volatile("" ::: "memory");
+            wait_vmcnt_lgkm0<(STAGES - 2) * LOADS>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const unsigned into = lds0 + stage * STAGE_BYTES;
+            const int live = __builtin_amdgcn_readfirstlane((kt + STAGES - KT) >> 31);
+            stage = stage + 1 == STAGES ? 0 : stage + 1;
+            const unsigned char* src = smem + stage * STAGE_BYTES;
+            static_for(
+                [&](auto idx) {
+                    constexpr int m = decltype(idx)::value, ks = m / (TM * TN), i = m % (TM * TN) / TN, j = m % TN;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.a[ks][i], cur.b[ks][j], acc[i][j], 0, 0, 0);
+                    if constexpr (m < RM) {
+                        static_for(
+                            [&](auto r) {
+                                constexpr int q = (NF * m) / RM + decltype(r)::value, fk = q / (TM + TN), t = q % (TM + TN);
+                                if constexpr (t < TM) nxt.a[fk][t] = fa.load(src, t, fk);
+                                else nxt.b[fk][t - TM] = fb.load(src + OpA::BYTES, t - TM, fk);
+                            },
+                            std::make_integer_sequence<int, (NF * (m + 1)) / RM - (NF * m) / RM>{});
+                    } else {
+                        static_for([&](auto d) { feed(std::integral_constant<int, (LOADS * (m - RM)) / (NM - RM) + decltype(d)::value>{}, into, live); },
+                                   std::make_integer_sequence<int, (LOADS * (m - RM + 1)) / (NM - RM) - (LOADS * (m - RM)) / (NM - RM)>{});
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                },
+                std::make_integer_sequence<int, NM>{});
+        };
+#pragma unroll
+        for (int t = 0; t < STAGES; ++t)
+            static_for([&](auto k_c) { feed(k_c, lds0 + t * STAGE_BYTES, __builtin_amdgcn_readfirstlane((t - KT) >> 31)); }, std::make_integer_sequence<int, LOADS>{});
+        asm volatile("" ::: "memory");
+        wait_vmcnt_lgkm0<(STAGES - 1) * LOADS>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) t0.a[ks][i] = fa.load(smem, i, ks);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) t0.b[ks][j] = fb.load(smem + OpA::BYTES, j, ks);
+        }
+        int kt = 0;
+        for (; kt + 1 < KT; kt += 2) {
+            step(t0, t1, kt);
+            step(t1, t0, kt + 1);
+        }
+        if (kt < KT) step(t0, t1, kt);
+    } else if constexpr (BK == 64) {
         // Two stages of 64-wide k-tiles, each multiplied as two 32-wide halves from the two fragment
         // sets.  Per tile one barrier, in the middle of its second half: by then every wave has read
         // the tile's last fragments (so its stage can take tile kt+2) and tile kt+1, issued one whole
@@ -1025,7 +1142,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // 128-byte row segments (256 bytes for fp32 outputs).
     // An odd tile count per row ends with a single tile: its 32 columns use half of the patch and half of
     // the lanes of the row pass.
-    if constexpr (PREF && !(BK == 64 && STAGES >= 3)) fetch(std::integral_constant<int, 0>{}, opc);
+    if constexpr (PREF && !EARLY && !(BK == 64 && STAGES >= 3)) fetch(std::integral_constant<int, 0>{}, opc);
     wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before their stages become the patch
     __syncthreads();
     float* patch = (float*)smem + wave * (32 * PLD);
@@ -1039,33 +1156,19 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
                 for (int r = 0; r < 16; ++r)
                     patch[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * PLD + h * 32 + (lane & 31)] = acc[i][jp * 2 + h][r] * g.alpha;
             asm volatile("" ::: "memory");
-            if constexpr (HOIST) fetch(idx, opc);
-            else if constexpr (decltype(idx)::value + 1 < TM * NP) fetch(std::integral_constant<int, decltype(idx)::value + 1>{}, opn);
+            if constexpr (HOIST && !EARLY) fetch(idx, opc);
+            else if constexpr (PREF && decltype(idx)::value + 1 < TM * NP) fetch(std::integral_constant<int, decltype(idx)::value + 1>{}, opn);
             const int n = n0 + wn * WTN + jp * 64 + pcol;
             const bool live = (NH == 2 || pcol < 32) && n < g.N;
             // per patch: the bias of the lane's eight columns once, the offsets of its first row by multiplication
             // and of the other three by addition (a 64-bit multiply is several quarter-rate instructions)
-            float b8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (g.bias && live) load_vec((const bf16*)g.bias + n, b8);
+            if constexpr (!EARLY) column_values(live, n);
             const int m_first = m0 + wm * WTM + i * 32 + prow;
             int64_t ci = coff + (int64_t)m_first * g.ldc + n, xi = coff + (int64_t)m_first * g.ldaux + n;
             // STATS 2: the lane's sums over its four rows, for its eight columns
-            float mu8[8], rs8[8], sg[8], sgx[8];
-            if constexpr (STATS == 2) {
+            float sg[8], sgx[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) mu8[e] = rs8[e] = sg[e] = sgx[e] = 0.f;
-                if (live) {
-                    const f32x4 m_lo = *(const f32x4*)(bn.mean + n), m_hi = *(const f32x4*)(bn.mean + n + 4);
-                    const f32x4 r_lo = *(const f32x4*)(bn.rstd + n), r_hi = *(const f32x4*)(bn.rstd + n + 4);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        mu8[e] = m_lo[e];
-                        mu8[4 + e] = m_hi[e];
-                        rs8[e] = r_lo[e];
-                        rs8[4 + e] = r_hi[e];
-                    }
-                }
-            }
+            for (int e = 0; e < 8; ++e) sg[e] = sgx[e] = 0.f;
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
                 const int m = m_first + it * 8;
