@@ -72,23 +72,28 @@ __device__ __forceinline__ void dma_rows8(const bf16* gbase, int64_t ld, int row
     const int gr = min(row0 + r, last_row);
     dma16(gbase + (int64_t)gr * ld + c * 8, tile + idx * 1024);
 }
-// Whole 64-row tile: this wave's two instructions (row groups wave and wave + 4).  Full tiles
-// take a wave-uniform base plus the lane's fixed offset; only a tile that reaches past the last
-// row pays for per-lane clamping.
-struct LaneOff { uint32_t o0, o1; };
-__device__ __forceinline__ LaneOff lane_off(int64_t ld, int wave, int lane) {
-    const int r0 = wave * 8 + (lane >> 3), r1 = r0 + 32;
-    return {(uint32_t)(r0 * ld + (((lane & 7) ^ fsw(r0)) << 3)), (uint32_t)(r1 * ld + (((lane & 7) ^ fsw(r1)) << 3))};
+// Whole 64-row tile by W waves: row groups wave, wave + W, ...  Full tiles take a wave-uniform base plus the lane's fixed
+// offset; only a tile that reaches past the last row pays for per-lane clamping.
+template <int W> struct LaneOff { uint32_t o[8 / W]; };
+template <int W> __device__ __forceinline__ LaneOff<W> lane_off(int64_t ld, int wave, int lane) {
+    LaneOff<W> l;
+#pragma unroll
+    for (int i = 0; i < 8 / W; ++i) {
+        const int r = (wave + i * W) * 8 + (lane >> 3);
+        l.o[i] = (uint32_t)(r * ld + (((lane & 7) ^ fsw(r)) << 3));
+    }
+    return l;
 }
+template <int W>
 __device__ __forceinline__ void dma_tile64(const bf16* gbase, int64_t ld, int row0, int last_row, unsigned char* tile,
-                                           int wave, int lane, LaneOff lo) {
+                                           int wave, int lane, const LaneOff<W>& lo) {
     if (row0 + 63 <= last_row) {
         const bf16* g = gbase + (int64_t)row0 * ld;
-        dma16(g + lo.o0, tile + wave * 1024);
-        dma16(g + lo.o1, tile + (wave + 4) * 1024);
+#pragma unroll
+        for (int i = 0; i < 8 / W; ++i) dma16(g + lo.o[i], tile + (wave + i * W) * 1024);
     } else {
-        dma_rows8(gbase, ld, row0, last_row, tile, wave, lane);
-        dma_rows8(gbase, ld, row0, last_row, tile, wave + 4, lane);
+#pragma unroll
+        for (int i = 0; i < 8 / W; ++i) dma_rows8(gbase, ld, row0, last_row, tile, wave + i * W, lane);
     }
 }
 // 4-byte variant for the per-row fp32 statistics: 64 consecutive floats
@@ -199,36 +204,49 @@ __device__ __forceinline__ BlockMap map_block(int nbh) {
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
     return {j / per_xcd, (j % per_xcd) * 8 + xcd};
 }
-static unsigned attn_grid(int seq, int nbh) { return (unsigned)(8 * ((nbh + 7) / 8) * ((seq + 127) / 128)); }
+static unsigned attn_grid(int seq, int rows, int nbh) { return (unsigned)(8 * ((nbh + 7) / 8) * ((seq + rows - 1) / rows)); }
+
+// A block has W waves of 32 rows each, and G groups of such waves that share the walk over the tiles (group g: tiles g, g + G,
+// ...; a ring each); what the groups have summed up meets in LDS at the end, added in group order.  One group of four where the
+// grid gives every CU more than one block; below that what bounds a launch is a wave's walk over its tiles with nobody beside it on
+// its SIMD, so the walk is shared, and where half the CUs had no block the blocks are halved too (measured: see attn_shape).
+// this wave's column tiles of those the other groups have for the same rows: parts holds [group][wave][tiles][16][64] floats
+template <int W, int G, int T> __device__ __forceinline__ void attn_park(float* parts, int grp, int w, int lane, const f32x16 (&v)[T]) {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) parts[(((grp * W + w) * T + t) * 16 + r) * 64 + lane] = v[t][r];
+}
 
 // =========================================================================================
-// forward: block = 128 queries (4 waves x 32), loop over 64-key tiles
+// forward: block = 128 queries (4 waves x 32; W, G: see above), loop over 64-key tiles
 // =========================================================================================
 // HP: heads per block (1: one head, 2: a pair of 32-wide heads); NPAN: 64-wide column panels of a head (1; 2 for
 // 128-wide heads, HP = 1: a tile in LDS is then two [64][64] panels behind each other, each in the format above);
 // KS k-steps of a head's scores, DT 32-wide output tiles of a head
-template <bool DROP, int HP, int NPAN = 1>
-__global__ __launch_bounds__(256, (!DROP && NPAN == 1 && HP == 1) ? 4 : 2) void attn_fwd_kernel(const AttnArgs a) {
+template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 1) ? 4 : 2) void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
-    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * 2 * TILE];  // 2 stages x (K, V)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];  // G rings of 2 stages x (K, V)
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
+    unsigned char* smem = smem_all + grp * (4 * TILE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
-    const int qb = (a.seq + 127) / 128 - 1 - bm.rank;  // long (late) query blocks first
+    const int qb = (a.seq + ROWS - 1) / ROWS - 1 - bm.rank;  // long (late) query blocks first
     const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP;
     const int64_t row_base = (int64_t)b * a.seq;
     const bf16* Q = a.q + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* K = a.k + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* V = a.v + row_base * a.ld_qkv + hg * (64 * NPAN);
-    const int q0 = qb * 128 + wave * 32;
+    const int q0 = qb * ROWS + wave * 32;
     const int myq = q0 + (lane & 31);
     const int last = a.seq - 1;
 
     // block-wide key range
     int kv_end = a.seq;
-    if (a.mask == BB_MASK_CAUSAL) kv_end = min(a.seq, qb * 128 + 128);
+    if (a.mask == BB_MASK_CAUSAL) kv_end = min(a.seq, qb * ROWS + ROWS);
     else if (a.mask == BB_MASK_KEY_PADDING) kv_end = min(a.seq, a.key_len[b]);
     const int ntiles = (kv_end + 63) / 64;
     const int my_limit = kv_limit(a, b, myq);
@@ -252,32 +270,33 @@ __global__ __launch_bounds__(256, (!DROP && NPAN == 1 && HP == 1) ? 4 : 2) void 
         lsum[hh] = 0.f;
     }
 
-    const LaneOff lo = lane_off(a.ld_qkv, wave, lane);
-    auto issue = [&](int t) {
-        unsigned char* st = smem + (t & 1) * (2 * TILE);
+    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
+    auto issue = [&](int t, int slot) {
+        unsigned char* st = smem + slot * (2 * TILE);
         const int kv0 = t * 64;
 #pragma unroll
         for (int p = 0; p < NPAN; ++p) {
-            dma_tile64(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
-            dma_tile64(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
+            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
+            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
         }
     };
 
-    if (ntiles > 0) issue(0);
-    for (int t = 0; t < ntiles; ++t) {
+    if (grp < ntiles) issue(grp, 0);
+    for (int i = 0; i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
+        const int t = i * G + grp, slot = i & 1;
         asm volatile("" ::: "memory");
-        if (t + 1 < ntiles) {
-            issue(t + 1);
-            wait_vm<4 * NPAN>();
+        if (t + G < ntiles) {
+            issue(t + G, slot ^ 1);
+            wait_vm<16 / W * NPAN>();
         } else {
             wait_vm<0>();
         }
         block_sync();
-        const unsigned char* kt = smem + (t & 1) * (2 * TILE);
+        const unsigned char* kt = smem + slot * (2 * TILE);
         const unsigned char* vt = kt + TILE;
         const int kv0 = t * 64;
         // waves whose queries all precede this tile have nothing to add (causal)
-        const bool active = !(a.mask == BB_MASK_CAUSAL && kv0 > q0 + 31);
+        const bool active = (G == 1 || t < ntiles) && !(a.mask == BB_MASK_CAUSAL && kv0 > q0 + 31);
         if (active) {
 #pragma unroll
           for (int hh = 0; hh < HP; ++hh) {
@@ -349,6 +368,43 @@ __global__ __launch_bounds__(256, (!DROP && NPAN == 1 && HP == 1) ? 4 : 2) void 
         }
         block_sync();
     }
+    if constexpr (G > 1) {
+        // each group's context against the maximum of all of them; the first 2 NPAN groups finish a column tile each
+        float* stats = (float*)smem_all + W * G * (2 * NPAN) * 1024;   // [group][wave][HP][m, sum][64]
+        attn_park<W, G>((float*)smem_all, grp, wave, lane, o);
+#pragma unroll
+        for (int hh = 0; hh < HP; ++hh) {
+            stats[(((grp * W + wave) * HP + hh) * 2) * 64 + lane] = m[hh];
+            stats[(((grp * W + wave) * HP + hh) * 2 + 1) * 64 + lane] = lsum[hh];
+        }
+        __syncthreads();
+        float scale[G][HP];
+#pragma unroll
+        for (int hh = 0; hh < HP; ++hh) {
+            float all = -INFINITY, sum = 0.f;
+#pragma unroll
+            for (int g = 0; g < G; ++g) all = fmaxf(all, stats[(((g * W + wave) * HP + hh) * 2) * 64 + lane]);
+            const float safe = all == -INFINITY ? 0.f : all;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                scale[g][hh] = __builtin_amdgcn_exp2f(stats[(((g * W + wave) * HP + hh) * 2) * 64 + lane] - safe);
+                sum += stats[(((g * W + wave) * HP + hh) * 2 + 1) * 64 + lane] * scale[g][hh];
+            }
+            m[hh] = all;
+            lsum[hh] = sum;
+        }
+#pragma unroll
+        for (int dt = 0; dt < 2 * NPAN; ++dt) {
+            if (dt % G != grp) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float v = 0.f;
+#pragma unroll
+                for (int g = 0; g < G; ++g) v += ((float*)smem_all)[(((g * W + wave) * (2 * NPAN) + dt) * 16 + r) * 64 + lane] * scale[g][dt / DT];
+                o[dt][r] = v;
+            }
+        }
+    }
     float inv[HP];
 #pragma unroll
     for (int hh = 0; hh < HP; ++hh) {
@@ -358,7 +414,8 @@ __global__ __launch_bounds__(256, (!DROP && NPAN == 1 && HP == 1) ? 4 : 2) void 
     if (myq < a.seq) {
         bf16* op = a.out + (row_base + myq) * a.ld_o + hg * (64 * NPAN);
 #pragma unroll
-        for (int dt = 0; dt < 2 * NPAN; ++dt)
+        for (int dt = 0; dt < 2 * NPAN; ++dt) {
+            if (dt % G != grp) continue;
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int d = dt * 32 + 8 * g4 + 4 * (lane >> 5);
@@ -367,9 +424,10 @@ __global__ __launch_bounds__(256, (!DROP && NPAN == 1 && HP == 1) ? 4 : 2) void 
                            pack2bf(o[dt][g4 * 4 + 2] * iv, o[dt][g4 * 4 + 3] * iv)};
                 *(u32x2*)(op + d) = w;
             }
+        }
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh)
-            if (lane < 32) a.lse[((int64_t)b * a.heads + head0 + hh) * a.seq + myq] = m[hh] + log2f(lsum[hh]);
+            if (lane < 32 && grp == 0) a.lse[((int64_t)b * a.heads + head0 + hh) * a.seq + myq] = m[hh] + log2f(lsum[hh]);
     }
 }
 
@@ -379,17 +437,15 @@ __global__ __launch_bounds__(256, (!DROP && NPAN == 1 && HP == 1) ? 4 : 2) void 
 // NPAN = 2 (128-wide heads): a block accumulates dK and dV for ONE 64-wide half `fh` of the head's columns (the grid
 // has two blocks per head and key block); scores and dP take the full 128 columns in both, i.e. are made twice -- a wave
 // that held all four output tiles of dK and of dV next to K, V, S and dP would need more registers than it has.
-template <bool DROP, int HP, int NPAN = 1>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
+template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
-    constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192;
-    // 2 stages x (Q tile, dO tile: 8 KiB per panel, lse 256 B per head, delta 256 B per head); two panels: more than the
-    // 64 KiB a kernel may declare, so the launch brings it
+    constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192, ROWS = W * 32;
+    // per group 2 stages x (Q tile, dO tile: 8 KiB per panel, lse 256 B per head, delta 256 B per head)
     constexpr int STAGE = 2 * TILE + 512 * HP;
-    __shared__ __attribute__((aligned(16))) unsigned char smem_fixed[NPAN == 1 ? 2 * STAGE : 16];
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_launch[];
-    unsigned char* smem = NPAN == 1 ? smem_fixed : smem_launch;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
+    unsigned char* smem = smem_all + grp * (2 * STAGE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(a.batch * groups * NPAN);
     if (bm.bh >= a.batch * groups * NPAN) return;
@@ -404,15 +460,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
     // the statistics of the block's heads lie behind each other: [batch, heads, seq]
     const float* LSE = a.lse + ((int64_t)b * a.heads + head0) * a.seq;
     const float* DELTA = a.delta + ((int64_t)b * a.heads + head0) * a.seq;
-    const int kv0 = kb * 128 + wave * 32;
+    const int kv0 = kb * ROWS + wave * 32;
     const int mykv = kv0 + (lane & 31);
     const int last = a.seq - 1;
     const int pad_limit = a.mask == BB_MASK_KEY_PADDING ? min(a.seq, a.key_len[b]) : a.seq;
 
     // query range that can see keys of this block
-    const int q_begin = a.mask == BB_MASK_CAUSAL ? (kb * 128) / 64 : 0;  // first 64-query tile
-    // a block whose 128 keys are all padding has nothing to accumulate: it only stores its zeros
-    const int ntiles = kb * 128 >= pad_limit ? 0 : (a.seq + 63) / 64;
+    const int q_begin = a.mask == BB_MASK_CAUSAL ? (kb * ROWS) / 64 : 0;  // first 64-query tile
+    // a block whose keys are all padding has nothing to accumulate: it only stores its zeros
+    const int ntiles = kb * ROWS >= pad_limit ? 0 : (a.seq + 63) / 64;
 
     bf16x8 kf[4 * NPAN], vf[4 * NPAN];
     {
@@ -429,33 +485,30 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
 #pragma unroll
         for (int r = 0; r < 16; ++r) dk[t][r] = dv[t][r] = 0.f;
 
-    const LaneOff lo = lane_off(a.ld_qkv, wave, lane), lo_o = lane_off(a.ld_o, wave, lane);
+    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane), lo_o = lane_off<W>(a.ld_o, wave, lane);
     auto issue = [&](int t, int slot) {
         unsigned char* st = smem + slot * STAGE;
         const int qs = t * 64;
 #pragma unroll
         for (int p = 0; p < NPAN; ++p) {
-            dma_tile64(Q + p * 64, a.ld_qkv, qs, last, st + p * 8192, wave, lane, lo);
-            dma_tile64(DO + p * 64, a.ld_o, qs, last, st + TILE + p * 8192, wave, lane, lo_o);
+            dma_tile64<W>(Q + p * 64, a.ld_qkv, qs, last, st + p * 8192, wave, lane, lo);
+            dma_tile64<W>(DO + p * 64, a.ld_o, qs, last, st + TILE + p * 8192, wave, lane, lo_o);
         }
-        // one extra load for waves 0 and 1 (one head), for all four waves (a pair): lse of the heads, then delta
-        if constexpr (HP == 1) {
-            if (wave == 0) dma_f32x64(LSE, qs, last, st + 2 * TILE, lane);
-            if (wave == 1) dma_f32x64(DELTA, qs, last, st + 2 * TILE + 256, lane);
-        } else {
-            const float* src = (wave >> 1 ? DELTA : LSE) + (int64_t)(wave & 1) * a.seq;
-            dma_f32x64(src, qs, last, st + 2 * TILE + (wave >> 1) * 512 + (wave & 1) * 256, lane);
-        }
+        // extra loads, dealt to the waves: lse of the block's heads, then delta
+#pragma unroll
+        for (int j = 0; j < 2 * HP; ++j)
+            if (j % W == wave) dma_f32x64((j / HP ? DELTA : LSE) + (int64_t)(j % HP) * a.seq, qs, last, st + 2 * TILE + j * 256, lane);
     };
 
-    if (q_begin < ntiles) issue(q_begin, 0);
-    for (int t = q_begin; t < ntiles; ++t) {
-        const int slot = (t - q_begin) & 1;
+    if (q_begin + grp < ntiles) issue(q_begin + grp, 0);
+    for (int i = 0; q_begin + i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
+        const int t = q_begin + i * G + grp, slot = i & 1;
         asm volatile("" ::: "memory");
-        if (t + 1 < ntiles) {
-            issue(t + 1, slot ^ 1);
-            // the waves with an extra load wait for one more newer load than the others
-            if (HP == 2 || wave < 2) wait_vm<4 * NPAN + 1>(); else wait_vm<4 * NPAN>();
+        if (t + G < ntiles) {
+            issue(t + G, slot ^ 1);
+            // the waves with extra loads wait for as many newer loads more than the others
+            constexpr int LOADS = 16 / W * NPAN, EACH = 2 * HP / W, MORE = 2 * HP % W;
+            if (MORE == 0 || wave < MORE) wait_vm<LOADS + EACH + (MORE ? 1 : 0)>(); else wait_vm<LOADS + EACH>();
         } else {
             wait_vm<0>();
         }
@@ -468,7 +521,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
         for (int u = 0; u < 2; ++u) {
             const int qs = t * 64 + u * 32;
             if (a.mask == BB_MASK_CAUSAL && qs + 31 < kv0) continue;  // all queries precede this wave's keys
-            if (qs >= a.seq) continue;
+            if (qs >= a.seq) continue;   // (nor is there a tile past the last one)
 #pragma unroll
           for (int hh = 0; hh < HP; ++hh) {
             const float* lse_t = lse_all + 64 * hh;
@@ -578,6 +631,28 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
         }
         block_sync();
     }
+    if constexpr (G > 1) {
+        // the groups' sums, first dV, then dK (one after the other: together they would not find room)
+        float* parts = (float*)smem_all;
+        auto join = [&](f32x16 (&v)[2]) {
+            attn_park<W, G>(parts, grp, wave, lane, v);
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (t % G != grp) continue;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float x = parts[((wave * 2 + t) * 16 + r) * 64 + lane];
+#pragma unroll
+                    for (int g = 1; g < G; ++g) x += parts[(((g * W + wave) * 2 + t) * 16 + r) * 64 + lane];
+                    v[t][r] = x;
+                }
+            }
+            __syncthreads();
+        };
+        join(dv);
+        join(dk);
+    }
     if (mykv >= pad_limit) {  // a padded key takes no probability mass: its gradients are zero
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -591,6 +666,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
         for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
+                if (dt % G != grp) continue;
                 const int d = dt * 32 + 8 * g4 + 4 * (lane >> 5);
                 u32x2 wk = {pack2bf(dk[dt][g4 * 4] * a.scale, dk[dt][g4 * 4 + 1] * a.scale),
                             pack2bf(dk[dt][g4 * 4 + 2] * a.scale, dk[dt][g4 * 4 + 3] * a.scale)};
@@ -604,27 +680,28 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(const AttnArgs a) 
 // =========================================================================================
 // backward dQ: block = 128 queries (4 waves x 32), loop over 64-key tiles
 // =========================================================================================
-template <bool DROP, int HP, int NPAN = 1>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
+template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
-    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * 2 * TILE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
+    unsigned char* smem = smem_all + grp * (4 * TILE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
-    const int qb = (a.seq + 127) / 128 - 1 - bm.rank;
+    const int qb = (a.seq + ROWS - 1) / ROWS - 1 - bm.rank;
     const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP;
     const int64_t row_base = (int64_t)b * a.seq;
     const bf16* Q = a.q + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* K = a.k + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* V = a.v + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* DO = a.d_o + row_base * a.ld_o + hg * (64 * NPAN);
-    const int q0 = qb * 128 + wave * 32;
+    const int q0 = qb * ROWS + wave * 32;
     const int myq = q0 + (lane & 31);
     const int last = a.seq - 1;
     int kv_end = a.seq;
-    if (a.mask == BB_MASK_CAUSAL) kv_end = min(a.seq, qb * 128 + 128);
+    if (a.mask == BB_MASK_CAUSAL) kv_end = min(a.seq, qb * ROWS + ROWS);
     else if (a.mask == BB_MASK_KEY_PADDING) kv_end = min(a.seq, a.key_len[b]);
     const int ntiles = (kv_end + 63) / 64;
     // rows past the end compute on clamped inputs and are not stored
@@ -660,7 +737,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
                 for (int e = 0; e < 8; ++e) dl = fmaf((float)dof[ks][e], (float)of[e], dl);
             }
             dl += __shfl_xor(dl, 32, 64);
-            if (lane < 32 && myq < a.seq) a.delta[stat] = dl;
+            if (lane < 32 && myq < a.seq && grp == 0) a.delta[stat] = dl;
             my_delta[hh] = dl;
         }
     }
@@ -670,30 +747,31 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq[t][r] = 0.f;
 
-    const LaneOff lo = lane_off(a.ld_qkv, wave, lane);
-    auto issue = [&](int t) {
-        unsigned char* st = smem + (t & 1) * (2 * TILE);
+    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
+    auto issue = [&](int t, int slot) {
+        unsigned char* st = smem + slot * (2 * TILE);
         const int kv0 = t * 64;
 #pragma unroll
         for (int p = 0; p < NPAN; ++p) {
-            dma_tile64(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
-            dma_tile64(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
+            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
+            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
         }
     };
-    if (ntiles > 0) issue(0);
-    for (int t = 0; t < ntiles; ++t) {
+    if (grp < ntiles) issue(grp, 0);
+    for (int i = 0; i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
+        const int t = i * G + grp, slot = i & 1;
         asm volatile("" ::: "memory");
-        if (t + 1 < ntiles) {
-            issue(t + 1);
-            wait_vm<4 * NPAN>();
+        if (t + G < ntiles) {
+            issue(t + G, slot ^ 1);
+            wait_vm<16 / W * NPAN>();
         } else {
             wait_vm<0>();
         }
         block_sync();
-        const unsigned char* kt = smem + (t & 1) * (2 * TILE);
+        const unsigned char* kt = smem + slot * (2 * TILE);
         const unsigned char* vt = kt + TILE;
         const int kv0 = t * 64;
-        const bool active = !(a.mask == BB_MASK_CAUSAL && kv0 > q0 + 31);
+        const bool active = (G == 1 || t < ntiles) && !(a.mask == BB_MASK_CAUSAL && kv0 > q0 + 31);
         if (active) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -739,12 +817,29 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
         }
         block_sync();
     }
+    if constexpr (G > 1) {
+        float* parts = (float*)smem_all;
+        attn_park<W, G>(parts, grp, wave, lane, dq);
+        __syncthreads();
+#pragma unroll
+        for (int dt = 0; dt < 2 * NPAN; ++dt) {
+            if (dt % G != grp) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float x = parts[((wave * (2 * NPAN) + dt) * 16 + r) * 64 + lane];
+#pragma unroll
+                for (int g = 1; g < G; ++g) x += parts[(((g * W + wave) * (2 * NPAN) + dt) * 16 + r) * 64 + lane];
+                dq[dt][r] = x;
+            }
+        }
+    }
     if (myq < a.seq) {
         bf16* dqp = a.dq + (row_base + myq) * a.ld_dqkv + hg * (64 * NPAN);
 #pragma unroll
         for (int dt = 0; dt < 2 * NPAN; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
+                if (dt % G != grp) continue;
                 const int d = dt * 32 + 8 * g4 + 4 * (lane >> 5);
                 u32x2 w = {pack2bf(dq[dt][g4 * 4] * a.scale, dq[dt][g4 * 4 + 1] * a.scale),
                            pack2bf(dq[dt][g4 * 4 + 2] * a.scale, dq[dt][g4 * 4 + 3] * a.scale)};
@@ -770,6 +865,63 @@ static int check_attn(const char* name, int dtype, int mask, int batch, int head
     return BB_OK;
 }
 
+// LDS: the rings, or what the groups leave for each other
+template <int HP, int NPAN, int W, int G> constexpr size_t attn_lds(bool dkv) {
+    const size_t ring = G * (dkv ? 2 * (2 * NPAN * 8192 + 512 * HP) : 4 * NPAN * 8192);
+    const size_t parts = G == 1 ? 0 : (size_t)W * G * ((dkv ? 2 : 2 * NPAN) * 4096 + (dkv ? 0 : HP * 512));
+    return ring > parts ? ring : parts;
+}
+template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int threads, size_t lds, const AttnArgs& a, hipStream_t st) {
+    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));
+    bb_launch(kern, dim3(attn_grid(seq, rows, nbh)), dim3(threads), lds, st, a);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
+// dropout is a kernel of its own: its keep decisions cost registers that decide how many blocks a CU holds
+struct attn_fwd_launch {
+    template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
+        auto kern = a.drop.thresh ? attn_fwd_kernel<true, HP, NPAN, W, G> : attn_fwd_kernel<false, HP, NPAN, W, G>;
+        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(false), a, st);
+    }
+};
+struct attn_dq_launch {
+    template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
+        auto kern = a.drop.thresh ? attn_bwd_dq_kernel<true, HP, NPAN, W, G> : attn_bwd_dq_kernel<false, HP, NPAN, W, G>;
+        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(false), a, st);
+    }
+};
+struct attn_dkv_launch {
+    template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
+        auto kern = a.drop.thresh ? attn_bwd_dkv_kernel<true, HP, NPAN, W, G> : attn_bwd_dkv_kernel<false, HP, NPAN, W, G>;
+        return attn_go(kern, seq, W * 32, nbh * NPAN, W * G * 64, attn_lds<HP, NPAN, W, G>(true), a, st);   // 128-wide heads: a block per half
+    }
+};
+// The shape of a block, by the number of blocks of 128 rows and the length of the walk (a pair of heads walks twice).  Four
+// waves / four waves in two groups / two in four (us, forward, backward): 12 heads of 64, 2043 keys (192 blocks) 27 78 / 20 64 /
+// 24 78; 4 x 16 heads, 512 causal (256) 13.4 31.5 / 10.8 29.7 / 12.1 35.0; 2 x 25 heads, 300 (150) 7.4 20.7 / 7.7 23.3 / 9.6 24.2;
+// 16 heads, 1024 causal (128) 22.1 50.4 / 16.2 42.7 / 11.1 29.8; 2 x 4 heads, 512 causal (32) 12.7 29.4 / 10.3 27.6 / 7.6 20.8; 4
+// heads, 1024 causal with dropout (32) 28.3 80.5 / 24.3 65.6 / 15.2 40.7; 6 x 8 heads, 175 (96) 7.1 17.2 / 7.2 19.9 / 6.2 17.3; 8
+// x 8 pairs of 32, 128, dropout (64) 8.6 23.9 / 8.9 24.7 / 7.4 23.4; 2 x 16 heads, 100 (32) 5.8 14.0 / 5.9 16.4 / 5.6 15.7.  Heads of
+// 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.
+// Attention without a mask keeps the one walk.  Groups add the same terms in another order: as near the exact sums as before, but
+// not the same last bits, and the stage that ends the reference's script (no mask; a LayerNorm whose rows are summed up, which
+// cancels to 1e-4 of its terms) passes gradients on in which such bits show as 3 to 5 %.
+template <typename L, int HP, int NPAN> static int attn_shape(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
+    const int64_t blocks = (int64_t)nbh * ((seq + 127) / 128), walk = (int64_t)seq * HP;
+    if (a.mask != BB_MASK_NONE) {
+        if constexpr (NPAN == 1) {
+            if (blocks <= 128 && walk >= 160) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
+        }
+        if (blocks <= 256 && walk >= 448) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
+    }
+    return L::template go<HP, NPAN, 4, 1>(seq, nbh, a, st);
+}
+template <typename L> static int attn_launch(int head_dim, int seq, int batch, int heads, const AttnArgs& a, hipStream_t st) {
+    if (head_dim == 128) return attn_shape<L, 1, 2>(seq, batch * heads, a, st);
+    if (head_dim == 64) return attn_shape<L, 1, 1>(seq, batch * heads, a, st);
+    return attn_shape<L, 2, 1>(seq, batch * (heads / 2), a, st);    // pairs of heads
+}
+
 extern "C" int bb_attention_fwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
                                 const void* k, const void* v, int64_t ld_qkv, void* out, int64_t ld_out, float* lse,
                                 const int32_t* key_len, float dropout_p, uint32_t dropout_k0, uint32_t dropout_k1,
@@ -787,22 +939,7 @@ extern "C" int bb_attention_fwd(int dtype, int mask, int batch, int heads, int s
     a.batch = batch; a.heads = heads; a.seq = seq; a.mask = mask;
     a.scale = 1.0f / sqrtf((float)head_dim);
     a.scale_log2 = a.scale * 1.4426950408889634f;
-    // dropout is a kernel of its own: its keep decisions cost registers that decide how many blocks a CU holds
-    const int hp = head_dim == 32 ? 2 : 1;   // heads per block
-    const dim3 grid(attn_grid(seq, batch * (heads / hp)));
-    hipStream_t st = (hipStream_t)stream;
-    if (head_dim == 128) {
-        if (a.drop.thresh) bb_launch((attn_fwd_kernel<true, 1, 2>), grid, dim3(256), 0, st, a);
-        else bb_launch((attn_fwd_kernel<false, 1, 2>), grid, dim3(256), 0, st, a);
-    } else if (hp == 1) {
-        if (a.drop.thresh) bb_launch((attn_fwd_kernel<true, 1>), grid, dim3(256), 0, st, a);
-        else bb_launch((attn_fwd_kernel<false, 1>), grid, dim3(256), 0, st, a);
-    } else {
-        if (a.drop.thresh) bb_launch((attn_fwd_kernel<true, 2>), grid, dim3(256), 0, st, a);
-        else bb_launch((attn_fwd_kernel<false, 2>), grid, dim3(256), 0, st, a);
-    }
-    BB_LAUNCH_CHECK();
-    return BB_OK;
+    return attn_launch<attn_fwd_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
 }
 
 extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
@@ -826,40 +963,8 @@ extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int s
     a.batch = batch; a.heads = heads; a.seq = seq; a.mask = mask;
     a.scale = 1.0f / sqrtf((float)head_dim);
     a.scale_log2 = a.scale * 1.4426950408889634f;
-    hipStream_t st = (hipStream_t)stream;
     // the dQ kernel first: it also leaves delta = rowsum(dO o O) of its queries for the dK / dV kernel
-    const int hp = head_dim == 32 ? 2 : 1;   // heads per block
-    dim3 grid(attn_grid(seq, batch * (heads / hp)));
-    if (head_dim == 128) {
-        // two dK / dV blocks per head and key block (one per 64-wide half of the columns), their LDS from the launch
-        constexpr int smem = 2 * (2 * 2 * 8192 + 512);
-        const dim3 grid2(attn_grid(seq, batch * heads * 2));
-        if (a.drop.thresh) {
-            BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)attn_bwd_dkv_kernel<true, 1, 2>, smem));
-            bb_launch((attn_bwd_dq_kernel<true, 1, 2>), grid, dim3(256), 0, st, a);
-            bb_launch((attn_bwd_dkv_kernel<true, 1, 2>), grid2, dim3(256), smem, st, a);
-        } else {
-            BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)attn_bwd_dkv_kernel<false, 1, 2>, smem));
-            bb_launch((attn_bwd_dq_kernel<false, 1, 2>), grid, dim3(256), 0, st, a);
-            bb_launch((attn_bwd_dkv_kernel<false, 1, 2>), grid2, dim3(256), smem, st, a);
-        }
-    } else if (hp == 1) {
-        if (a.drop.thresh) {
-            bb_launch((attn_bwd_dq_kernel<true, 1>), grid, dim3(256), 0, st, a);
-            bb_launch((attn_bwd_dkv_kernel<true, 1>), grid, dim3(256), 0, st, a);
-        } else {
-            bb_launch((attn_bwd_dq_kernel<false, 1>), grid, dim3(256), 0, st, a);
-            bb_launch((attn_bwd_dkv_kernel<false, 1>), grid, dim3(256), 0, st, a);
-        }
-    } else {
-        if (a.drop.thresh) {
-            bb_launch((attn_bwd_dq_kernel<true, 2>), grid, dim3(256), 0, st, a);
-            bb_launch((attn_bwd_dkv_kernel<true, 2>), grid, dim3(256), 0, st, a);
-        } else {
-            bb_launch((attn_bwd_dq_kernel<false, 2>), grid, dim3(256), 0, st, a);
-            bb_launch((attn_bwd_dkv_kernel<false, 2>), grid, dim3(256), 0, st, a);
-        }
-    }
-    BB_LAUNCH_CHECK();
-    return BB_OK;
+    rc = attn_launch<attn_dq_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
+    if (rc) return rc;
+    return attn_launch<attn_dkv_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
 }
