@@ -86,10 +86,10 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
 
 // DMA kernels need at least one full vector of rows, and but for weight gradients and D128x128k64r K % 32 == 0; tile by problem size
 enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, D256x128k64s3, D128x128k64, D128x64k64s3, D128x64s3,
-               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r };
+               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3 };
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
-                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r"};
+                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3"};
 // The kernel of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
 // what ran before): a redundant forward and a normal forward of the same layer give the same bits.  All tiles below add up
 // a contraction in the same order; the wave-sliced kernels (pick_wave) in another.
@@ -132,16 +132,20 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches;
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
-    //  - Problems of at most 400 tiles of 128x64 (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle) take those: up
-    //    to two per CU, whose chains run under each other.  128x128 / this, plain and with a residual (us): NT 1200x1600x1600 (250
-    //    tiles) 20.3 23.5 / 12.6 13.5, 3000x832x832 (312) 12.7 16.1 / 11.4 12.3, 4096x768x768 (384) 12.4 14.3 / 13.6 11.7, x3072
-    //    34.7 37.5 / 32.6 31.7, 3136x1024x256 (400) 8.3 9.7 / 7.7 8.3, 8192x512x512 (512) 10.8 12.0 / 12.8 10.5; NN 21.0 24.0 / 12.4
-    //    13.1, 13.2 16.2 / 11.3 12.0, 11.9 14.2 / 13.8 11.8, 34.5 37.4 / 31.6 31.3, 8.0 9.6 / 7.7 8.4, 10.3 11.6 / 13.9 14.2.  More of
-    //    them: 256x128 tiles, also for short contractions (NT 6272x1024x256 12.8 14.0 on 128x64, 10.3 11.4 on 256x128).
+    //  - Problems of at most one tile of 128x64 per CU (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle) take those,
+    //    short contractions also up to 400, whose chains run under each other; then 128x128 tiles of three stages, one per CU, up to
+    //    a round of them.  128x64 / 128x128 (64x128 / 128x128), plain and with a residual (us): NT 1200x1600x1600 (250 tiles of
+    //    128x64) 12.3 12.9 / 15.1 16.8, 2300x1024x1024 (288) 12.2 12.8 / 11.7 12.9, 4096x768x768 (384) 10.8 11.3 / 10.4 11.4, x3072 30.2
+    //    30.8 / 25.1 26.5, 3136x1024x256 (400) 7.4 8.1 / 7.8 8.7, 6272x512x128 (392) 6.7 7.4 / 7.1 8.0; NN 12.1 12.7 / 15.1 16.5, 12.2 12.9 /
+    //    11.8 13.1, 10.9 11.5 / 10.7 11.5, 30.4 30.6 / 25.3 26.7, 7.4 8.2 / 7.9 8.8.  A round of 128x128 with two stages or 32-wide k-tiles
+    //    (two and three blocks per CU) / this: NT 8192x512x512 10.7 11.9 / 9.6 10.5, x2048 26.2 28.9 / 21.1 22.4, NN 10.2 11.5 / 9.8 10.6,
+    //    26.2 28.9 / 21.4 22.4; 256x128 / this where a few rows stand against many columns: 640x6400x1600 24.1 25.6 / 17.3 19.0.  More
+    //    of them: 256x128 tiles, also for short contractions (NT 6272x1024x256 12.8 14.0 on 128x64, 10.3 11.4 on 256x128).
     //    32-wide k-tiles (K % 64 != 0) as before: 128x64 tiles up to 128 tiles of 128x128 and for short forward contractions.
     if (k64) {
-        if (nt && (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches <= 400) return D128x64k64s3;
-        if (nn && (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches <= 400) return D64x128k64s3;
+        const int64_t halves = nt ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
+        if (halves <= (K >= 768 ? 256 : 400)) return nt ? D128x64k64s3 : D64x128k64s3;
+        if (t128 <= 256) return D128x128k64s3;
     } else {
         if ((K <= 512 || t128 <= 128) && nt) return D128x64s3;
         if (t128 <= 128 && nn) return D64x128s3;
@@ -171,7 +175,13 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
             if (t2128 * 10 >= slots2 * 9) return mid;
             return full70 ? D256x256k64 : small;
         }
-        if (k64) return full85 || (K >= 2048 && full70) ? D256x256w8db : small;
+        // NN: below 85 % the tiles whose rounds are better filled (256x256 one, 128x128 three a CU; full, they are equal), 128x128 /
+        // 256x256 (us): 4096x6400x1600 (78 % of two rounds, 69 % of three) 103 / 89, 6656x4096x1024 76 / 71, x512 48 / 47,
+        // 6144x4096x1024 (75 %, 100 % of two) 65 / 69
+        if (k64) {
+            const int64_t slots3 = (t128 + 767) / 768 * 768;
+            return full85 || (full70 && (K >= 2048 || t256 * slots3 > t128 * slots)) ? D256x256w8db : small;
+        }
         return full70 || K >= 1536 ? D256x256w8db : small;
     }
     if (big_ok && t2128 > 256) return k64 && nt ? D256x256k64 : D256x256w8db;
@@ -235,6 +245,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D128x128k64: return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64>(g, batches, st);
         case D128x128k64r:
             if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64, true>(g, batches, st);
+            else break;
+        case D128x128k64s3:
+            if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
             else break;
         case D128x64k64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3, 64>(g, batches, st);
         case D128x64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3>(g, batches, st);

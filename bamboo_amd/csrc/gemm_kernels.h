@@ -760,8 +760,8 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // bias gradient riding along: the waves of the first block column (and first wave column)
     // add up the A fragments they hold anyway: lane (m, kg) sees 8 of the 16 k values per step
     const bool do_colsum = AKM && g.colsum != nullptr && tile_n == 0 && wn == 0;
-    // the main loop of the small tiles, see there
-    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && TM * TN <= 2 && !AKM && !RAGK && !VIS;
+    // the main loop of the smaller tiles, see there
+    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS;
     float csum[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) csum[i] = 0.f;
@@ -854,7 +854,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     constexpr int NP = (TN + 1) / 2;   // pairs per row of accumulator tiles, the last one possibly a single
     const int prow = lane >> 3, pcol = (lane & 7) * 8;
     // Only on the large tiles (one block per CU, two waves per SIMD whatever the kernel's register count) and on the
-    // small ones (a single patch, few accumulators): on the others the 32 registers would cost a resident block.
+    // ones that read ahead: on the others the 32 registers would cost a resident block.
     // Some of the other kernels fetch a patch's operand(s) in one go at the top of that patch: the pointers of GemmArgs
     // may alias as far as the compiler knows, so left inside the row loop every load waits behind the previous row's
     // store (four round trips in a row per patch instead of one).
@@ -862,7 +862,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // operand reads per row are most of their epilogue)
     // EARLY: the kernels whose waves finish one patch each and have the registers fetch it -- and the bias -- before the main loop.
     constexpr bool EARLY = AHEAD && TM * NP == 1;
-    constexpr bool PREF = (BM * BN >= 256 * 128 || EARLY) && !VIS && CONV == 0 && STATS == 0;
+    constexpr bool PREF = (BM * BN >= 256 * 128 || AHEAD) && !VIS && CONV == 0 && STATS == 0;
     constexpr bool HOIST = STATS == 2;
     const bf16* opnd = PREF || HOIST ? epilogue_operand(g) : nullptr;
     u32x4 opc[PREF || HOIST ? 4 : 1], opn[PREF ? 4 : 1];
@@ -925,7 +925,9 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         // between register sets at every merge).  Before (halves of a k-tile read half a k-tile ahead) and now, us: 64x64 tiles, NT
         // 1024x512x2048 11.7 / 9.5, 512x1024x4096 20.0 / 15.7, 100x1600x6400 29.1 / 21.3, 0.25 -> 0.17 us a k-tile, where LDS moves
         // 32 KB of fragments and 16 KB of transfers; 128x64 and 64x128 gain by the epilogue's early operands: 2043x768x768 with a
-        // residual 8.6 / 7.8, x3072 21.2 / 20.2 (NT), 21.0 / 19.4 (NN).
+        // residual 8.6 / 7.8, x3072 21.2 / 20.2 (NT), 21.0 / 19.4 (NN).  128x128 tiles, one a CU with three stages: the loop below with
+        // two blocks a CU 26.2, this one 21.1 (NT 8192x512x2048).  256x128 tiles are 2 to 6 % faster on it alone and no faster in a
+        // stage, where the matrix cores' clock gives way: they keep the loop below.
         struct Tile {
             bf16x8 a[4][TM], b[4][TN];
         } t0, t1;
@@ -1142,7 +1144,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // 128-byte row segments (256 bytes for fp32 outputs).
     // An odd tile count per row ends with a single tile: its 32 columns use half of the patch and half of
     // the lanes of the row pass.
-    if constexpr (PREF && !EARLY && !(BK == 64 && STAGES >= 3)) fetch(std::integral_constant<int, 0>{}, opc);
+    if constexpr (PREF && !EARLY && (AHEAD || !(BK == 64 && STAGES >= 3))) fetch(std::integral_constant<int, 0>{}, opc);
     wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before their stages become the patch
     __syncthreads();
     float* patch = (float*)smem + wave * (32 * PLD);

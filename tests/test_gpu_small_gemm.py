@@ -240,6 +240,34 @@ def test_fp32_quarter_tiles_have_the_bits_of_whole_ones(hiplib, layout, M, N, K)
     assert bool(((C.double().cpu() - prod).abs() <= bound).all())
 
 
+# 128x128 tiles of three stages, whose loop reads fragments a k-tile ahead, against the same rows inside a product of tiles that do
+# not: the same bits, for fewer k-tiles than the ring has stages up to odd and even numbers of them beyond; ragged rows and columns.
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("K", [128, 192, 256, 320, 448, 832])
+def test_128_tiles_that_read_ahead_have_the_bits_of_others(hiplib, K, layout):
+    lay, M, N, rows = getattr(hiplib, layout.upper()), 5500, 616, 14000
+    A, B = rand(rows, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2, scale=0.2)
+    bias, X, R = rand(N, seed=3), rand(rows, N, seed=4), rand(rows, N, seed=5)
+    names = [hiplib.gemm_variant(hiplib.gemm_desc(lay, A[:m], B, X[:m])) for m in (M, rows)]
+    assert names[0].endswith("dma128x128k64s3") and names[1].endswith(("dma256x256k64", "dma256x192k64", "dma256x256w8db")), names
+    for kw in (dict(bias=bias), dict(bias=bias, epilogue=hiplib.EPI_RESIDUAL), dict(epilogue=hiplib.EPI_MUL), dict(epilogue=hiplib.EPI_MUL_POS),
+               dict(bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_GELU_TANH), dict(bias=bias, dropout=(0.1, (7, 9)))):
+        if "dropout" in kw and layout == "nn":
+            continue
+        out = []
+        for m in (M, rows):
+            C, aux = torch.full((m, N), float("nan"), dtype=torch.bfloat16, device=DEV), X[:m].clone()
+            extra = {hiplib.EPI_RESIDUAL: dict(resid=aux), hiplib.EPI_MUL: dict(aux_in=aux), hiplib.EPI_MUL_POS: dict(aux_in=aux, resid=R[:m]),
+                     hiplib.EPI_ACT_DACT: dict(aux_out=aux)}
+            hiplib.gemm(lay, A[:m], B, C, **kw, **extra.get(kw.get("epilogue"), {}))
+            out.append((C[:M], aux[:M]))
+        assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), kw
+    prod = A[:M].float() @ (B.float().t() if layout == "nt" else B.float())
+    C = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    hiplib.gemm(lay, A[:M], B, C)
+    assert rel(C, prod) < 2.0 ** -8      # half an ulp of bf16, and the sums' K eps
+
+
 # The small tiles' loop against the same rows inside a product that 256x128 tiles run: the same bits.  One k-tile, as many as the
 # ring has stages and one more, odd and even numbers of them beyond; rows off the tile; every epilogue that fetches an operand.
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 448, 576])
