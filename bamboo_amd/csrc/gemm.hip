@@ -631,17 +631,29 @@ extern "C" int bb_conv3x3_dgrad_bn(int dtype, int n, int h, int w, int cin, int 
 template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(GroupedArgs& G, hipStream_t st) {
     constexpr int BM = 128, BN = 128, STAGES = 3;
     constexpr int smem = STAGES * (BM + BN) * 32 * 2;
-    auto kern = gemm_bf16_dma_grouped_kernel<BM, BN, 2, 2, TA, TB, true, STAGES, CONVB>;
-    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
-    int blocks = 0;
+    int blocks = 0, kmin = G.p[0].K;
     for (int i = 0; i < G.count; ++i) {
         GemmArgs& g = G.p[i];
         g.tiles_m = (g.M + BM - 1) / BM;
         g.tiles_n = (g.N + BN - 1) / BN;
         G.first_block[i] = blocks;
         blocks += g.tiles_m * g.tiles_n;
+        kmin = g.K < kmin ? g.K : kmin;
     }
     G.first_block[G.count] = blocks;
+    auto kern = gemm_bf16_dma_grouped_kernel<BM, BN, 2, 2, TA, TB, true, STAGES, CONVB, !TA && !TB>;
+    // Weight gradients over many rows whose blocks, three a CU, fill their rounds: lock step keeps the three, which started
+    // together, on the same operand panels (459 instead of 720 MiB read per launch).  Where blocks of a CU start apart, or the
+    // contraction is too short for them to drift, it only adds waits.  In lock step / free (us), hidden size (x 4 in the feed-forward) and
+    // rows: 1024 8192 222 / 224 (a stage of it gains half a percent), 16384 435 / 449; 4096 119 / 115, 2048 67.2 / 65.8; 768 (56 % of a
+    // round) 2048 48.3 / 45.4, 12000 263 / 209; 960 (94 %) 8192 220 / 216; 1600 (85 % of three rounds) 4096 336 / 305.
+    // ResNet blocks, 6272 pixels: 256 middle channels 41.3 / 37.6, 512 120 / 102.  Forward products 406 / 411 (8192x1024, x 4), input
+    // gradients 384 / 362.
+    if constexpr (TA && !CONVB) {
+        const int slots = (blocks + 767) / 768 * 768;
+        if (kmin >= 8192 && (int64_t)blocks * 100 >= (int64_t)slots * 95) kern = gemm_bf16_dma_grouped_kernel<BM, BN, 2, 2, TA, TB, true, STAGES, false, true>;
+    }
+    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     bb_launch(kern, dim3(blocks), dim3(256), smem, st, G);
     BB_LAUNCH_CHECK();
     return BB_OK;

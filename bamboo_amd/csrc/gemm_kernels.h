@@ -1515,7 +1515,8 @@ template <> struct BbPointersAt<GroupedArgs> {
     }
 };
 // CONVB: some problems of the group read their B operand as the patch matrix of a 3x3 convolution
-template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, bool CONVB = false>
+// LOCK: the waves of a block in lock step (compiler-visible DMA, see DmaOperand): see launch_grouped for where that pays
+template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, bool CONVB = false, bool LOCK = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_grouped_kernel(const GroupedArgs G) {
     // The tiles of all problems form one list; an XCD takes a contiguous stretch of it, so its
     // resident blocks are a few wide rectangles of one or two problems (few distinct operand
@@ -1523,14 +1524,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_grouped_kernel(cons
     const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
-    // compiler-visible DMA here: the lock step it forces on the waves keeps the three resident blocks of a CU
-    // on the same operand panels (459 instead of 720 MiB read per launch at the same kernel speed; the stage
-    // gains half a percent with the second stream running)
     if constexpr (CONVB) {
         if (G.p[pi].conv_c > 0) {
-            gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, 32, true, 3>(G.p[pi], lid - G.first_block[pi], 0, true);
+            gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, 32, LOCK, 3>(G.p[pi], lid - G.first_block[pi], 0, true);
             return;
         }
     }
-    gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, 32, true>(G.p[pi], lid - G.first_block[pi], 0, true);
+    gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, 32, LOCK>(G.p[pi], lid - G.first_block[pi], 0, true);
 }

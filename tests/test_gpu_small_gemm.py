@@ -295,3 +295,19 @@ def test_small_tiles_have_the_bits_of_large_ones(hiplib, M, tile, K):
     C = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
     hiplib.gemm(lay, A[:M], B, C)
     assert rel(C, prod) < 2.0 ** -8      # half an ulp of bf16, and the sums' K eps
+
+
+# Weight gradients whose 128x128 tiles fill a round, three a CU: in lock step from 8192 rows on, free below, ragged and whole
+# contractions; against each problem by itself (the same k order, free): the same bits, bias gradients too.
+@pytest.mark.parametrize("rows", [8184, 8192, 8201])
+def test_weight_gradients_of_a_full_round(hiplib, rows):
+    shapes = [(3072, 1024), (2048, 1024), (3584, 1024), (1024, 3584)]
+    ops = [(rand(rows, m, seed=2 * i), rand(rows, n, seed=2 * i + 1)) for i, (m, n) in enumerate(shapes)]
+    runs = []
+    for grouped in (True, False):
+        C, bias = [torch.ones(m, n, device=DEV) for m, n in shapes], [torch.ones(m, device=DEV) for m, _ in shapes]
+        descs = [hiplib.gemm_desc(hiplib.TN, a, b, c, accumulate=True, colsum_out=s) for (a, b), c, s in zip(ops, C, bias)]
+        for group in [descs] if grouped else [[d] for d in descs]:
+            hiplib.gemm_grouped(group)
+        runs.append(C + bias)
+    assert all(torch.equal(x, y) for x, y in zip(*runs))
