@@ -4,7 +4,7 @@
 // contiguous memory, rows are kept in registers between the passes of a kernel, and all
 // reductions are butterfly shuffles or fixed-order partial sums (no atomics: results are
 // reproducible bit for bit).
-#include "common.h"
+#include "partials.h"
 
 #include <stdarg.h>
 
@@ -276,28 +276,6 @@ __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_ke
     }
 }
 
-// Sum of partial rows p = first, first + step, ... in that order, eight loads in flight at a time.
-__device__ __forceinline__ float sum_partials(const float* __restrict__ src, int first, int step, int nparts, int64_t stride) {
-    float s = 0.f;
-    int p = first;
-    for (; p + 7 * step < nparts; p += 8 * step) {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = src[(int64_t)(p + j * step) * stride];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s += v[j];
-    }
-    if (p < nparts) {   // the last few go out together as well
-        float v[7];
-#pragma unroll
-        for (int j = 0; j < 7; ++j) v[j] = p + j * step < nparts ? src[(int64_t)(p + j * step) * stride] : 0.f;
-#pragma unroll
-        for (int j = 0; j < 7; ++j) s += v[j];
-    }
-    return s;
-}
-constexpr int RED_WAVES = 16;
-
 // out[i] += sum_p partial[p * stride + i].  One block owns 64 columns; its sixteen waves sum
 // interleaved shares of the partial rows (p = w, w+16, ...) and the sixteen results are combined
 // in wave order, so the summation order is fixed by nparts alone.
@@ -320,24 +298,34 @@ __global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_acc_kernel(con
     reduce_partials_acc_body(partial, nparts, stride, n, out);
 }
 
-// two vectors at once (LayerNorm gain and shift gradients): blockIdx.y picks the half of every
-// partial row and the output
-__global__ __launch_bounds__(RED_WAVES * 64) void reduce_partials_acc2_kernel(const float* __restrict__ partial, int nparts,
-                                                                              int64_t stride, int n, float* __restrict__ out0,
-                                                                              float* __restrict__ out1) {
-    __shared__ float red[RED_WAVES][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    const float* src = partial + (int64_t)blockIdx.y * n;
-    float* out = blockIdx.y == 0 ? out0 : out1;
-    red[wave][lane] = i < n ? sum_partials(src + i, wave, RED_WAVES, nparts, stride) : 0.f;
-    __syncthreads();
-    if (wave == 0 && i < n) {
-        float s = red[0][lane];
-#pragma unroll
-        for (int w = 1; w < RED_WAVES; ++w) s += red[w][lane];
-        out[i] += s;
+// gain and shift gradients of LayerNorms
+__global__ __launch_bounds__(RED_WAVES * 64) void partial_sums_kernel(const PartialSums a) {
+    __shared__ float red[RED_WAVES * 64];
+    partial_sums_block<RED_WAVES>(a, blockIdx.x, red);
+}
+int bb_partial_sums_args(const char* who, const bb_partial_sums* sums, int count, PartialSums& a) {
+    BB_REQUIRE(count >= 0 && count <= PARTIAL_SUMS_MAX && (sums || count == 0), "%s: 0 to %d partial sums, got %d", who, PARTIAL_SUMS_MAX, count);
+    a = {};
+    for (int i = 0; i < count; ++i) {
+        const bb_partial_sums& s = sums[i];
+        BB_REQUIRE(s.partial && s.out0 && s.out1 && s.parts >= 0 && s.n > 0 && s.n <= (1 << 24), "%s: bad partial sums (n = %d, parts = %d)", who, s.n, s.parts);
+        a.partial[i] = s.partial; a.out0[i] = s.out0; a.out1[i] = s.out1;
+        a.nparts[i] = s.parts; a.n[i] = s.n;
+        a.first_block[i] = a.blocks;
+        a.blocks += s.parts > 0 ? 2 * ((s.n + 63) / 64) : 0;
     }
+    a.count = count;
+    a.first_block[count] = a.blocks;
+    a.blocks = (a.blocks + 7) / 8 * 8;
+    return BB_OK;
+}
+extern "C" int bb_partial_sums_acc(const bb_partial_sums* sums, int count, void* stream) {
+    PartialSums a;
+    int rc = bb_partial_sums_args("bb_partial_sums_acc", sums, count, a);
+    if (rc || a.blocks == 0) return rc;
+    bb_launch(partial_sums_kernel, dim3(a.first_block[count]), dim3(RED_WAVES * 64), 0, (hipStream_t)stream, a);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
 }
 
 template <typename T, int IT>
@@ -403,32 +391,30 @@ extern "C" int bb_layernorm_fwd(int dtype, int kind, int rows, int cols, float e
 
 extern "C" int64_t bb_layernorm_bwd_workspace(int cols) { return (int64_t)LN_BWD_BLOCKS * 2 * cols; }
 
-static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
-                      const float* mean, const float* rinv, const void* dy, const void* dres, void* dx, float* dgain,
-                      float* dshift, float* workspace, hipStream_t st) {
+// blocks leaves their number, and the first launch of the two goes out; the second adds up what they left
+static int ln_bwd_rows(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
+                       const float* mean, const float* rinv, const void* dy, const void* dres, void* dx, float* workspace, int& blocks,
+                       hipStream_t st) {
+    blocks = 0;
     int rc = check_rowop(who, dtype, rows, cols);
     if (rc) return rc;
     BB_REQUIRE(kind == BB_LN_STANDARD || kind == BB_LN_ANNOTATED, "%s: bad kind %d", who, kind);
-    BB_REQUIRE(x && gain && mean && rinv && dy && dx && dgain && dshift && workspace, "%s: null pointer", who);
+    BB_REQUIRE(x && gain && mean && rinv && dy && dx && workspace, "%s: null pointer", who);
     BB_REQUIRE((size_t)3 * 2 * cols * sizeof(float) <= 160 * 1024, "%s: cols (%d) too large (max 6826)", who, cols);
     if (rows == 0) return BB_OK;
-    int blocks = 0;
-    auto finish = [&]() -> int {
-        const int nb = (cols + 63) / 64;
-        bb_launch(reduce_partials_acc2_kernel, dim3(nb, 2), dim3(RED_WAVES * 64), 0, st, workspace, blocks,
-                           (int64_t)2 * cols, cols, dgain, dshift);
-        BB_LAUNCH_CHECK();
-        return BB_OK;
-    };
-    auto run = [&](auto launch) -> int {
-        int r = launch;
-        return r ? r : finish();
-    };
     if (dtype == BB_BF16)
-        BB_DISPATCH_IT(bf16, cols / 8, run(ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
+        BB_DISPATCH_IT(bf16, cols / 8, (ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
     else
-        BB_DISPATCH_IT(float, cols / 4, run(ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
+        BB_DISPATCH_IT(float, cols / 4, (ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
     return BB_EINVAL;
+}
+static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
+                      const float* mean, const float* rinv, const void* dy, const void* dres, void* dx, float* dgain,
+                      float* dshift, float* workspace, hipStream_t st) {
+    BB_REQUIRE(dgain && dshift, "%s: null pointer", who);
+    bb_partial_sums sums = {workspace, dgain, dshift, 0, cols};
+    int rc = ln_bwd_rows(who, dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, sums.parts, st);
+    return rc || sums.parts == 0 ? rc : bb_partial_sums_acc(&sums, 1, st);
 }
 
 extern "C" int bb_layernorm_bwd(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
@@ -436,6 +422,15 @@ extern "C" int bb_layernorm_bwd(int dtype, int kind, int rows, int cols, float e
                                 float* dgain, float* dshift, float* workspace, void* stream) {
     return ln_bwd_run("bb_layernorm_bwd", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, dgain, dshift, workspace,
                       (hipStream_t)stream);
+}
+
+extern "C" int bb_layernorm_bwd_rows(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain, const float* mean,
+                                     const float* rinv, const void* dy, const void* dres, void* dx, float* dgain, float* dshift,
+                                     float* partials, bb_partial_sums* sums, void* stream) {
+    BB_REQUIRE(dgain && dshift && sums, "bb_layernorm_bwd_rows: null pointer");
+    *sums = {partials, dgain, dshift, 0, cols};
+    return ln_bwd_rows("bb_layernorm_bwd_rows", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, partials, sums->parts,
+                       (hipStream_t)stream);
 }
 
 // ---- the same for callers that cannot allocate ---------------------------------------------------------------

@@ -654,7 +654,7 @@ template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(Groupe
         if (kmin >= 8192 && (int64_t)blocks * 100 >= (int64_t)slots * 95) kern = gemm_bf16_dma_grouped_kernel<BM, BN, 2, 2, TA, TB, true, STAGES, false, true>;
     }
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
-    bb_launch(kern, dim3(blocks), dim3(256), smem, st, G);
+    bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(256), smem, st, G);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -677,7 +677,7 @@ template <int KW, int BK, int NST> static int launch_grouped_wave(GroupedArgs& G
         blocks += g.tiles_m * g.tiles_n;
     }
     G.first_block[G.count] = blocks;
-    bb_launch(kern, dim3(blocks), dim3(KW * 64), smem, st, G);
+    bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(KW * 64), smem, st, G);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -713,9 +713,12 @@ static bool shared_launch_dma(const bb_gemm_desc& d) {
     return t != D_NONE && t != D128x128k64r;
 }
 
-extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream) {
+extern "C" int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const bb_partial_sums* sums, int nsums, void* stream) {
     BB_REQUIRE(count >= 0 && (descs || count == 0), "bb_gemm_grouped: bad arguments");
     hipStream_t st = (hipStream_t)stream;
+    PartialSums ride;
+    int ride_rc = bb_partial_sums_args("bb_gemm_grouped_sums", sums, nsums, ride);
+    if (ride_rc) return ride_rc;
     // one launch when every problem is an unbatched bf16 problem of one layout that the DMA
     // kernel accepts; otherwise the problems run one after the other (same results)
     bool has_conv = false;
@@ -750,6 +753,7 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
     if (fuse32) {
         GroupedArgs G;
         G.count = count;
+        G.ride = ride;
         const int tile = waves ? 32 : 64;
         int blocks = 0;
         for (int i = 0; i < count; ++i) {
@@ -769,21 +773,24 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
         const auto kern = layout == BB_NT   ? gemm_f32_grouped_kernel<false, false>
                           : layout == BB_NN ? waves ? gemm_f32_wave_grouped_kernel<false, true> : gemm_f32_grouped_kernel<false, true>
                                             : waves ? gemm_f32_wave_grouped_kernel<true, true> : gemm_f32_grouped_kernel<true, true>;
-        bb_launch(kern, dim3(blocks), dim3(256), waves ? kF32WaveLds : f32_gemm_lds(64), st, G);
+        bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(256), waves ? kF32WaveLds : f32_gemm_lds(64), st, G);
         BB_LAUNCH_CHECK();
         return BB_OK;
     }
     // a patch-matrix B exists only inside the grouped kernels: no one-by-one route for it
     BB_REQUIRE(fuse || !has_conv, "bb_gemm_grouped: a problem with a patch-matrix B must share a launch of unbatched bf16 BB_TN problems");
     if (!fuse) {
+        int rc = bb_partial_sums_acc(sums, nsums, stream);
+        if (rc) return rc;
         for (int i = 0; i < count; ++i) {
-            int rc = bb_gemm(&descs[i], stream);
+            rc = bb_gemm(&descs[i], stream);
             if (rc) return rc;
         }
         return BB_OK;
     }
     GroupedArgs G;
     G.count = count;
+    G.ride = ride;
     for (int i = 0; i < count; ++i) {
         int64_t batches;
         bool ta, tb;
@@ -798,6 +805,9 @@ extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* strea
     if (layout == BB_NN) return launch_grouped<false, true>(G, st);
     if (has_conv) return launch_grouped<true, true, true>(G, st);
     return launch_grouped<true, true>(G, st);
+}
+extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream) {
+    return bb_gemm_grouped_sums(descs, count, nullptr, 0, stream);
 }
 
 // =========================================================================================

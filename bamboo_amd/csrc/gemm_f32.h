@@ -292,7 +292,8 @@ __global__ __launch_bounds__(256, WIDE ? 2 : 4) void gemm_f32_kernel(const GemmA
 // several unbatched problems in one launch (the weight gradients of an fp32 layer)
 template <bool TA, bool TB>
 __global__ __launch_bounds__(256, 4) void gemm_f32_grouped_kernel(const GroupedArgs G) {
-    const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
+    const int lid = grouped_place<4>(G);
+    if (lid < 0) return;
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
     gemm_f32_body<TA, TB, 64>(G.p[pi], lid - G.first_block[pi], 0, true);
@@ -384,7 +385,8 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_wave_kernel(const GemmArgs g)
 }
 template <bool TA, bool TB>
 __global__ __launch_bounds__(256, 4) void gemm_f32_wave_grouped_kernel(const GroupedArgs G) {
-    const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
+    const int lid = grouped_place<4>(G);
+    if (lid < 0) return;
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
     gemm_f32_wave_body<TA, TB>(G.p[pi], lid - G.first_block[pi], 0, true);

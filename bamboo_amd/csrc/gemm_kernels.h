@@ -1,7 +1,7 @@
 // Device side of the GEMM family (kernels, operand loaders, fragment readers, epilogues) and the per-kernel launch
 // templates; the host-side tile choice and the C entry points are in gemm.hip.
 #pragma once
-#include "common.h"
+#include "partials.h"
 
 #include <utility>
 
@@ -1505,15 +1505,28 @@ struct GroupedArgs {
     GemmArgs p[GROUP_MAX];
     int first_block[GROUP_MAX + 1];
     int count;
+    PartialSums ride;   // sums of an earlier launch's partial rows, done by blocks in front of the tiles'
 };
+static_assert(sizeof(GroupedArgs) <= 4096, "kernel arguments");
 template <> struct BbPointersAt<GroupedArgs> {
     static constexpr int EACH = sizeof(BbPointersAt<GemmArgs>::at) / sizeof(uint16_t);
-    uint16_t at[GROUP_MAX * EACH];
+    uint16_t at[GROUP_MAX * EACH + 3 * PARTIAL_SUMS_MAX];
     constexpr BbPointersAt() : at{} {
         const BbPointersAt<GemmArgs> one;
+        for (int i = 0; i < 3 * PARTIAL_SUMS_MAX; ++i) at[GROUP_MAX * EACH + i] = (uint16_t)(offsetof(GroupedArgs, ride) + i * sizeof(void*));
         for (int i = 0; i < GROUP_MAX * EACH; ++i) at[i] = (uint16_t)(offsetof(GroupedArgs, p) + i / EACH * sizeof(GemmArgs) + one.at[i % EACH]);
     }
 };
+// The block's place among the tiles of a shared launch, or -1 for one of the blocks in front, whose sums are done then.  What such
+// sums take by themselves is a launch that waits for the memory a few times (3.2 us at 1050 rows of 512 columns, 4.6 at 8192 of 1024,
+// once a LayerNorm); here they are under the tiles.
+template <int WAVES> __device__ __forceinline__ int grouped_place(const GroupedArgs& G) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int b = (int)blockIdx.x - G.ride.blocks;
+    if (b >= 0) return xcd_contiguous(b, G.first_block[G.count]);
+    partial_sums_block<WAVES>(G.ride, blockIdx.x, (float*)smem);
+    return -1;
+}
 // CONVB: some problems of the group read their B operand as the patch matrix of a 3x3 convolution
 // LOCK: the waves of a block in lock step (compiler-visible DMA, see DmaOperand): see launch_grouped for where that pays
 template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, bool CONVB = false, bool LOCK = false>
@@ -1521,7 +1534,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_grouped_kernel(cons
     // The tiles of all problems form one list; an XCD takes a contiguous stretch of it, so its
     // resident blocks are a few wide rectangles of one or two problems (few distinct operand
     // panels in its L2) rather than a narrow slice of every problem.
-    const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
+    const int lid = grouped_place<WM * WN>(G);
+    if (lid < 0) return;
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
     if constexpr (CONVB) {

@@ -265,7 +265,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_bf16_wave_kernel(const GemmArgs 
 // CONVB: some of them read B as the patch matrix of a 3x3 convolution
 template <bool AKM, bool BKM, int KW, int BK, int NST, bool CONVB = false>
 __global__ __launch_bounds__(KW * 64) void gemm_bf16_wave_grouped_kernel(const GroupedArgs G) {
-    const int lid = xcd_contiguous(blockIdx.x, G.first_block[G.count]);
+    const int lid = grouped_place<KW>(G);
+    if (lid < 0) return;
     int pi = 0;
     while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
     int tile_m, tile_n;

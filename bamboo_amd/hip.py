@@ -23,8 +23,8 @@ MASK_CODES = {"none": MASK_NONE, "causal": MASK_CAUSAL, "key_padding": MASK_KEY_
 LN_CODES = {"standard": LN_STANDARD, "annotated": LN_ANNOTATED}
 
 EXPORTS = (
-    "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
-    "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
+    "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_grouped_sums", "bb_partial_sums_acc", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
+    "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_rows", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
     "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_attention_probs_supported", "bb_attention_probs_fwd", "bb_attention_probs_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
     "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_operands", "bb_plan_launches", "bb_plan_launch", "bb_plan_launch_on", "bb_plan_destroy",
     "bb_adam_multi", "bb_adam_multi_scaled", "bb_grad_clip_workspace", "bb_grad_clip_coef", "bb_cast", "bb_fill_f32",
@@ -52,6 +52,10 @@ class GemmDesc(Structure):
         ("strip_stats", c_void_p),
         ("dropout_p", c_float), ("dropout_k0", c_uint32), ("dropout_k1", c_uint32),
     ]
+
+
+class PartialSums(Structure):
+    _fields_ = [("partial", c_void_p), ("out0", c_void_p), ("out1", c_void_p), ("parts", c_int32), ("n", c_int32)]
 
 
 class BnBwdStats(Structure):
@@ -90,6 +94,9 @@ def lib():
     L.bb_layernorm_bwd_workspace.argtypes = [c_int]
     L.bb_layernorm_bwd_workspace.restype = c_int64
     L.bb_layernorm_bwd.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 11
+    L.bb_layernorm_bwd_rows.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 10 + [POINTER(PartialSums), c_void_p]
+    L.bb_partial_sums_acc.argtypes = [POINTER(PartialSums), c_int, c_void_p]
+    L.bb_gemm_grouped_sums.argtypes = [POINTER(GemmDesc), c_int, POINTER(PartialSums), c_int, c_void_p]
     L.bb_layernorm_bwd_static.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 10
     L.bb_rowsum_fwd.argtypes = [c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
     L.bb_rowsum_bwd.argtypes = [c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
@@ -300,13 +307,19 @@ def gemm_splitk_workspace(descs):
     return int(lib().bb_gemm_splitk_workspace(arr, len(descs)))
 
 
-def gemm_grouped(descs, stream=None, splitk_ws=None, hook=None):
+def gemm_grouped(descs, stream=None, splitk_ws=None, hook=None, sums=()):
     """Independent GEMMs of one layout in one launch (falls back to one launch each inside the
     library when they cannot share a kernel).  With ``splitk_ws`` (a tensor of at least
     ``gemm_splitk_workspace(descs)`` bytes) problems with few output tiles and a long contraction
-    are cut along the contraction and reduced in fixed order."""
+    are cut along the contraction and reduced in fixed order.  ``sums``: what :func:`layernorm_bwd_rows` left to add,
+    done in the same launch where there is one."""
     arr = (GemmDesc * len(descs))(*descs)
-    if splitk_ws is not None:
+    if sums:
+        if splitk_ws is not None:
+            raise HipKernelError("gemm_grouped: sums go with the launch that is not cut")
+        left = (PartialSums * len(sums))(*sums)
+        call = lambda: check(lib().bb_gemm_grouped_sums(arr, len(descs), left, len(sums), stream_ptr(stream)), "bb_gemm_grouped_sums")
+    elif splitk_ws is not None:
         nbytes = splitk_ws.numel() * splitk_ws.element_size()
         call = lambda: check(lib().bb_gemm_grouped_splitk(arr, len(descs), _ptr(splitk_ws), nbytes, stream_ptr(stream)),
                              "bb_gemm_grouped_splitk")
@@ -394,6 +407,25 @@ def layernorm_bwd(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, workspace, k
     check(lib().bb_layernorm_bwd(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(mean),
                                  _ptr(rinv), _ptr(dy), _ptr(dres), _ptr(dx), _ptr(dgain), _ptr(dshift),
                                  _ptr(workspace), stream_ptr(stream)), "bb_layernorm_bwd")
+
+
+def layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partials, kind, eps, stream=None):
+    """:func:`layernorm_bwd` without its second launch: the gain and shift gradients are left as sums per block in ``partials``,
+    which stays untouched until ``gemm_grouped(sums=)`` or :func:`partial_sums` has added up what this returns."""
+    rows, cols = x.shape
+    _check_ln_bwd("layernorm_bwd_rows", x, gain, mean, rinv, dy, dres, dx, dgain, dshift)
+    if partials.numel() < layernorm_bwd_workspace(cols) or partials.dtype != torch.float32:
+        raise HipKernelError("layernorm_bwd_rows: partials too small")
+    sums = PartialSums()
+    check(lib().bb_layernorm_bwd_rows(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(mean), _ptr(rinv), _ptr(dy),
+                                      _ptr(dres), _ptr(dx), _ptr(dgain), _ptr(dshift), _ptr(partials), byref(sums), stream_ptr(stream)),
+          "bb_layernorm_bwd_rows")
+    return sums
+
+
+def partial_sums(sums, stream=None):
+    """Adds up what calls of :func:`layernorm_bwd_rows` left."""
+    check(lib().bb_partial_sums_acc((PartialSums * len(sums))(*sums), len(sums), stream_ptr(stream)), "bb_partial_sums_acc")
 
 
 def layernorm_bwd_static(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, kind, eps, stream=None):

@@ -240,7 +240,8 @@ class TransformerLayer:
         dt = ctx.dtype
         attn = ("attn_delta", (ctx.batch, self.heads, ctx.seq), torch.float32) if self.fused_attention(ctx) else \
             ("d_prob", (ctx.batch, self.heads, ctx.seq, ctx.seq), dt)
-        specs = [("d_ffn", (R, f), dt), ("d_h0", (R, h), dt), ("d_h1", (R, h), dt), ("d_qkv", (R, 3 * h), dt), attn]
+        specs = [("d_ffn", (R, f), dt), ("d_h0", (R, h), dt), ("d_h1", (R, h), dt), ("d_qkv", (R, 3 * h), dt), attn,
+                 ("ln_partials", (2, hip.layernorm_bwd_workspace(h)), torch.float32)]
         if self.dropout > 0:
             # the gradients behind the two sublayer dropouts: the weight gradients read them at the end of the layer
             specs += [("d_drop0", (R, h), dt), ("d_drop1", (R, h), dt)]
@@ -266,11 +267,17 @@ class TransformerLayer:
 
     def workspace_elems(self):
         n = 5 * self.hidden + self.ffn    # the four weight gradients of a grouped launch
-        return max(hip.layernorm_bwd_workspace(self.hidden), hip.colsum_workspace(n))
+        return hip.colsum_workspace(n)
 
     def flops_fwd(self, batch, seq):
         h, f = self.hidden, self.ffn
         return batch * seq * (8 * h * h + 4 * h * f) + 4 * batch * seq * seq * h
+
+    def _layernorm_bwd(self, sums, ctx, x, norm, mean, rinv, dy, dres, dx):
+        """LayerNorm backward; its gain's and shift's gradients join ``sums``, at most two until the launch that adds them up."""
+        partials = ctx.buf("ln_partials", (2, hip.layernorm_bwd_workspace(self.hidden)))[len(sums)]
+        sums.append(hip.layernorm_bwd_rows(x, self.w[norm + ".a_2"], mean, rinv, dy, dres, dx, self.g[norm + ".a_2"], self.g[norm + ".b_2"],
+                                           partials, hip.LN_CODES[self.ln], self.eps, stream=ctx.stream))
 
     # ------------------------------------------------------------------ attention core
     def _heads_gemm(self, ctx, layout, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, alpha=1.0):
@@ -392,14 +399,13 @@ class TransformerLayer:
     def backward(self, d_out, d_x, st, ctx):
         """d_out: gradient of st['out']; writes the input gradient into d_x; parameter
         gradients are accumulated (fp32)."""
-        w, g, sm, ws = self.w, self.g, ctx.stream, ctx.workspace
+        w, g, sm = self.w, self.g, ctx.stream
         R, h, f = ctx.rows, self.hidden, self.ffn
-        kind, act = hip.LN_CODES[self.ln], hip.ACT_CODES[self.activation]
         d_ffn, d_h0, d_h1 = ctx.buf("d_ffn", (R, f)), ctx.buf("d_h0", (R, h)), ctx.buf("d_h1", (R, h))
         d_qkv = ctx.buf("d_qkv", (R, 3 * h))
         # weight gradients dW += dy^T x are collected and issued as one grouped launch at the end:
-        # each alone has too few output tiles to fill the GPU
-        wgrads = []
+        # each alone has too few output tiles to fill the GPU; the sums of the LayerNorms' parameter gradients go with them
+        wgrads, sums = [], []
         # ... and each carries its bias gradient (column sums of dy) in the same kernel
         wgrad = lambda dy, x, name: wgrads.append(hip.gemm_desc(
             hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[name[:-len("weight")] + "bias"], colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
@@ -421,8 +427,7 @@ class TransformerLayer:
         wgrad(d_ffn, st["n2"], "feed_forward.w_1.weight")
         ctx.gemm(hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
         # d_x1 = d_out + LN2'(d_n2)
-        hip.layernorm_bwd(st["x1"], w["sublayer.1.norm.a_2"], st["mean2"], st["rinv2"], d_h0, d_out, d_h1,
-                          g["sublayer.1.norm.a_2"], g["sublayer.1.norm.b_2"], ws, kind, self.eps, stream=sm)
+        self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h1)
         # attention output projection
         d_proj = d_h1
         if self.dropout > 0:
@@ -435,10 +440,9 @@ class TransformerLayer:
         wgrad(d_qkv, st["n1"], "qkv.weight")
         ctx.gemm(hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
         # d_x0 = d_x1 + LN1'(d_n1)
-        hip.layernorm_bwd(st["x0"], w["sublayer.0.norm.a_2"], st["mean1"], st["rinv1"], d_h0, d_h1, d_x,
-                          g["sublayer.0.norm.a_2"], g["sublayer.0.norm.b_2"], ws, kind, self.eps, stream=sm)
+        self._layernorm_bwd(sums, ctx, st["x0"], "sublayer.0.norm", st["mean1"], st["rinv1"], d_h0, d_h1, d_x)
         # d_out (d_drop1), d_ffn, d_h1 (d_drop0) and d_qkv still hold the four output gradients here
-        ctx.gemm_grouped(wgrads, stream=sm)
+        ctx.gemm_grouped(wgrads, stream=sm, sums=sums)
         return d_x
 
 
@@ -567,21 +571,21 @@ class DecoderLayer(TransformerLayer):
         return st["out"]
 
     def backward(self, d_out, d_x, st, ctx):
-        w, g, sm, ws = self.w, self.g, ctx.stream, ctx.workspace
+        w, g, sm = self.w, self.g, ctx.stream
         R, h, f = ctx.rows, self.hidden, self.ffn
-        kind = hip.LN_CODES[self.ln]
         d_ffn, d_h0, d_h1, d_h2 = (ctx.buf("d_ffn", (R, f)), ctx.buf("d_h0", (R, h)), ctx.buf("d_h1", (R, h)),
                                    ctx.buf("d_h2", (R, h)))
         d_qkv, d_mem = ctx.buf("d_qkv", (R, 3 * h)), ctx.buf("d_mem", (R, h))
-        wgrads = []
+        wgrads, sums = [], []
         wgrad = lambda dy, x, name, bias=None: wgrads.append(hip.gemm_desc(
             hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[bias or (name[:-len("weight")] + "bias")], colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
 
         def flush():
             # the weight gradients collected so far, before a scratch buffer they read is written again
             if wgrads:
-                ctx.gemm_grouped(list(wgrads), stream=sm)
+                ctx.gemm_grouped(list(wgrads), stream=sm, sums=list(sums))
                 wgrads.clear()
+                sums.clear()
         if ctx.deferred and self.activation != "relu":
             self._ffn1(st, ctx)
         # ---- sublayer 2: feed-forward (as in TransformerLayer.backward)
@@ -598,8 +602,7 @@ class DecoderLayer(TransformerLayer):
         wgrad(d_ffn, st["n2"], "feed_forward.w_1.weight")
         ctx.gemm(hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
         # d_x2 = d_out + LN2'(d_n2)  -> d_h2
-        hip.layernorm_bwd(st["x2"], w["sublayer.2.norm.a_2"], st["mean2"], st["rinv2"], d_h0, d_out, d_h2,
-                          g["sublayer.2.norm.a_2"], g["sublayer.2.norm.b_2"], ws, kind, self.eps, stream=sm)
+        self._layernorm_bwd(sums, ctx, st["x2"], "sublayer.2.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h2)
         # ---- sublayer 1: attention over the memory
         d_proj = d_h2
         if self.dropout > 0:
@@ -614,8 +617,7 @@ class DecoderLayer(TransformerLayer):
         ctx.gemm(hip.NN, d_qkv[:, :h], w["src_attn.linears.0.weight"], d_h0, stream=sm)        # d_n_src
         ctx.gemm(hip.NN, d_qkv[:, h:], w["kv.weight"], d_mem, stream=sm)                       # gradient of the memory
         # d_x1 = d_x2 + LN_src'(d_n_src)  -> d_h1
-        hip.layernorm_bwd(st["x1"], w["sublayer.1.norm.a_2"], st["mean_src"], st["rinv_src"], d_h0, d_h2, d_h1,
-                          g["sublayer.1.norm.a_2"], g["sublayer.1.norm.b_2"], ws, kind, self.eps, stream=sm)
+        self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean_src"], st["rinv_src"], d_h0, d_h2, d_h1)
         flush()      # d_qkv, d_ffn and the first sublayers' gradient buffers are free again
         # ---- sublayer 0: self-attention
         d_proj0 = d_h1
@@ -628,8 +630,7 @@ class DecoderLayer(TransformerLayer):
         wgrad(d_qkv, st["n1"], "qkv.weight")
         ctx.gemm(hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
         # d_x = d_x1 + LN0'(d_n1) + d_mem * dm/dx
-        hip.layernorm_bwd(st["x0"], w["sublayer.0.norm.a_2"], st["mean1"], st["rinv1"], d_h0, d_h1, d_x,
-                          g["sublayer.0.norm.a_2"], g["sublayer.0.norm.b_2"], ws, kind, self.eps, stream=sm)
+        self._layernorm_bwd(sums, ctx, st["x0"], "sublayer.0.norm", st["mean1"], st["rinv1"], d_h0, d_h1, d_x)
         hip.sqrt_one_minus_bwd(d_mem, st["mem"], d_x, accumulate=True, stream=sm)
         flush()
         return d_x

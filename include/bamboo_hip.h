@@ -148,6 +148,20 @@ int64_t bb_strip_stats_workspace(int rows, int cols);
  * is how the four weight-gradient products of a layer (autograd of transformer.py:136-146,158)
  * fill the GPU although each has few output tiles.                                         */
 int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream);
+/* Sums of partial rows an earlier launch left: out0[i] += sum over p < parts of partial[p * 2n + i],
+ * out1[i] likewise of partial[p * 2n + n + i], i < n, in a fixed order.                       */
+#define BB_PARTIAL_SUMS_MAX 4
+typedef struct bb_partial_sums {
+    const float* partial;
+    float* out0;
+    float* out1;
+    int parts, n;
+} bb_partial_sums;
+int bb_partial_sums_acc(const bb_partial_sums* sums, int count, void* stream);
+/* bb_gemm_grouped, with such sums (at most BB_PARTIAL_SUMS_MAX; their outputs are no operand of a
+ * problem) done in the same launch where there is one: the gain and shift gradients of a layer's
+ * LayerNorms (bb_layernorm_bwd_rows) beside its weight gradients.                             */
+int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const bb_partial_sums* sums, int nsums, void* stream);
 /* bb_gemm_grouped for problems with an fp32 C, few output tiles and a long contraction (weight
  * gradients dW += dy^T x of narrow layers, e.g. the three convolutions of resnet.py:49-75 over
  * K = N*H*W rows): the contraction is cut into chunks that run as problems of their own into fp32
@@ -175,6 +189,13 @@ int bb_layernorm_bwd(int dtype, int kind, int rows, int cols, float eps, const v
                      const void* gain, const float* mean, const float* rinv, const void* dy,
                      const void* dres, void* dx, float* dgain, float* dshift,
                      float* workspace, void* stream);
+/* The first half of it: dx, and per-block sums of dgain / dshift in `partials` (at least
+ * bb_layernorm_bwd_workspace(cols) elements, the caller's until they are added up).  *sums says what is
+ * left to add, for bb_partial_sums_acc or bb_gemm_grouped_sums; together the same bits.               */
+int bb_layernorm_bwd_rows(int dtype, int kind, int rows, int cols, float eps, const void* x,
+                          const void* gain, const float* mean, const float* rinv, const void* dy,
+                          const void* dres, void* dx, float* dgain, float* dshift, float* partials,
+                          bb_partial_sums* sums, void* stream);
 /* The same without a workspace, for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * per-block partial sums live in an array inside the library's device image (4 MiB per GPU, held until

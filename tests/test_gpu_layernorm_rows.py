@@ -25,3 +25,40 @@ def test_layernorm_bwd_row_counts(hiplib, dtype, rows, cols):
     assert bool(((dshift.double() + 0.5 - dy.double().sum(0)).abs() <= eps * (1 + dy.double().abs().sum(0))).all())
     # dx: two sums of `cols` terms; in bf16 the rounding of what is stored
     assert float((dx.double() - want).norm() / want.norm()) < (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5)
+
+
+# The parameter gradients left as sums per block and added up beside weight gradients: in every kernel that a group may take (eight
+# and four waves, 128x128 tiles free and in lock step; fp32 tiles and waves), one problem at a time where it may take none, and by
+# themselves.  Two LayerNorms, columns that are no multiple of a block's 64; the same bits as one call after the other, and the
+# weight gradients' too.
+@pytest.mark.parametrize("dtype,rows,cols,ffn", [(torch.bfloat16, 5, 72, 64), (torch.bfloat16, 128, 128, 512), (torch.bfloat16, 300, 512, 2048),
+                                                 (torch.bfloat16, 1050, 520, 2048), (torch.bfloat16, 700, 1600, 6400), (torch.bfloat16, 8192, 1024, 4096),
+                                                 (torch.bfloat16, 64, 1032, 40), (torch.float32, 128, 128, 512), (torch.float32, 300, 512, 2048),
+                                                 (torch.float32, 36, 68, 4)])
+def test_parameter_gradients_beside_weight_gradients(hiplib, dtype, rows, cols, ffn):
+    g = torch.Generator().manual_seed(rows + cols)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)
+    x, dy, res, gain = rand(rows, cols), rand(rows, cols), rand(rows, cols), rand(cols)
+    mean, rinv = x.float().mean(1), 1 / (x.float().var(1, unbiased=False) + 1e-5).sqrt()
+    act = rand(rows, ffn)
+    outs = []
+    for how in ("one by one", "beside", "by themselves"):
+        dx = [torch.empty_like(x) for _ in range(2)]
+        vec = [torch.full((cols,), 0.5, device=DEV) for _ in range(4)]
+        ws = [torch.full((hiplib.layernorm_bwd_workspace(cols),), float("nan"), device=DEV) for _ in range(2)]
+        W = [torch.ones(cols, cols, device=DEV), torch.ones(ffn, cols, device=DEV), torch.ones(cols, ffn, device=DEV)]
+        descs = [hiplib.gemm_desc(hiplib.TN, a, b, c, accumulate=True) for a, b, c in ((dy, x, W[0]), (act, x, W[1]), (dy, act, W[2]))]
+        sums = []
+        for i, d in enumerate((dy, res)):
+            args = (x, gain, mean, rinv, d, res if i == 0 else None, dx[i], vec[2 * i], vec[2 * i + 1], ws[i], hiplib.LN_STANDARD, 1e-5)
+            if how == "one by one":
+                hiplib.layernorm_bwd(*args)
+            else:
+                sums.append(hiplib.layernorm_bwd_rows(*args))
+        if how == "by themselves":
+            hiplib.partial_sums(sums)
+        hiplib.gemm_grouped(descs, sums=sums if how == "beside" else ())
+        outs.append(dx + vec + W)
+    assert all(torch.equal(a, b) for other in outs[1:] for a, b in zip(outs[0], other))
+    with pytest.raises(hiplib.HipKernelError):
+        hiplib.gemm_grouped(descs, sums=sums * 3)      # more than a launch takes
