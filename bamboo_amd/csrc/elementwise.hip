@@ -128,14 +128,28 @@ template <typename T, int IT> constexpr int ln_bwd_waves() {
     return IT * Elem<T>::VEC <= 16 ? 16 : IT * Elem<T>::VEC <= 32 ? 8 : 4;
 }
 
+// the elements first, first + 1, ... (VEC of them, first even) of a tensor behind its dropout
+template <int VEC> __device__ __forceinline__ void drop_vec(const DropKey& key, int64_t first, float (&v)[VEC]) {
+#pragma unroll
+    for (int e = 0; e < VEC; e += 2) {   // one hash per two neighbouring elements
+        const uint32_t x = key.small ? bb_dropout_pair_bits32(key.k0, key.k1, (uint32_t)(first + e) >> 1)
+                                     : bb_dropout_pair_bits(key.k0, key.k1, (uint64_t)(first + e) >> 1);
+        v[e] = bb_keep_even(x, key.thresh) ? v[e] * key.scale : 0.f;
+        v[e + 1] = bb_keep_odd(x, key.thresh) ? v[e + 1] * key.scale : 0.f;
+    }
+}
+
 // dx per row, dgain/dshift partial sums per block (fixed row->block assignment).
-template <typename T, int IT>
+// DROP: dropped = dropout(dx) as well, what dropout_kernel makes of the stored dx: its launch, and its pass over dx, are saved
+// (two launches / one, bf16, us: 8192x1024 21.0 / 16.7, 4096x1600 20.9 / 18.6, 2048x4096 34.3 / 32.4)
+template <typename T, int IT, bool DROP>
 __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_kernel(int kind, int rows, int cols, float eps,
                                                             const T* __restrict__ x, const T* __restrict__ gain,
                                                             const float* __restrict__ mean_in,
                                                             const float* __restrict__ rinv_in, const T* __restrict__ dy,
                                                             const T* __restrict__ dres, T* __restrict__ dx,
-                                                            float* __restrict__ partial, int one_pass) {
+                                                            float* __restrict__ partial, int one_pass, T* __restrict__ dropped,
+                                                            const DropKey key) {
     constexpr int VEC = Elem<T>::VEC, LN_BWD_WAVES = ln_bwd_waves<T, IT>();
     extern __shared__ float red[];  // [all waves][2][cols] (one pass) or [3 waves][2][cols] for the cross-wave sum
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -205,6 +219,19 @@ __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_ke
                     for (int e = 0; e < VEC; ++e) o[e] += rv[e];
                 }
                 store_vec(dxr + c * VEC, o);
+                if constexpr (DROP) {
+                    const int64_t first = (int64_t)row * cols + c * VEC;
+                    if constexpr (sizeof(T) == 2) {   // as stored
+#pragma unroll
+                        for (int e = 0; e < VEC; e += 2) {
+                            const uint32_t pair = pack2bf(o[e], o[e + 1]);
+                            o[e] = __uint_as_float(pair << 16);
+                            o[e + 1] = __uint_as_float(pair & 0xffff0000u);
+                        }
+                    }
+                    drop_vec<VEC>(key, first, o);
+                    store_vec(dropped + first, o);
+                }
             }
         }
     }
@@ -338,7 +365,8 @@ static int ln_fwd_launch(int kind, int rows, int cols, float eps, const void* x,
 }
 template <typename T, int IT>
 static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const float* mean,
-                         const float* rinv, const void* dy, const void* dres, void* dx, float* ws, int& blocks, hipStream_t st) {
+                         const float* rinv, const void* dy, const void* dres, void* dx, float* ws, int& blocks, hipStream_t st,
+                         void* dropped, const DropKey& key) {
     constexpr int LN_BWD_WAVES = ln_bwd_waves<T, IT>();
     // a row per wave: blocks past the last row would only write zeros for the reduction to read (us, backward with its
     // reduction, 256 blocks / as many as have rows: bf16 128 x 128 6.4 / 5.8, 300 x 768 8.5 / 7.5, 1024 x 512 7.2 / 6.7, 333 x 5120
@@ -347,10 +375,10 @@ static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x,
     const size_t all = (size_t)LN_BWD_WAVES * 2 * cols * sizeof(float);
     const int one_pass = all <= 128 * 1024;
     const size_t smem = one_pass ? all : (size_t)3 * 2 * cols * sizeof(float);
-    auto kern = layernorm_bwd_kernel<T, IT>;
+    auto kern = key.thresh ? layernorm_bwd_kernel<T, IT, true> : layernorm_bwd_kernel<T, IT, false>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));   // raised on the first (never captured) call that needs it
     bb_launch(kern, dim3(blocks), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
-                       (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass);
+                       (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass, (T*)dropped, key);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -394,7 +422,7 @@ extern "C" int64_t bb_layernorm_bwd_workspace(int cols) { return (int64_t)LN_BWD
 // blocks leaves their number, and the first launch of the two goes out; the second adds up what they left
 static int ln_bwd_rows(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
                        const float* mean, const float* rinv, const void* dy, const void* dres, void* dx, float* workspace, int& blocks,
-                       hipStream_t st) {
+                       hipStream_t st, void* dropped = nullptr, const DropKey& key = DropKey{}) {
     blocks = 0;
     int rc = check_rowop(who, dtype, rows, cols);
     if (rc) return rc;
@@ -403,9 +431,9 @@ static int ln_bwd_rows(const char* who, int dtype, int kind, int rows, int cols,
     BB_REQUIRE((size_t)3 * 2 * cols * sizeof(float) <= 160 * 1024, "%s: cols (%d) too large (max 6826)", who, cols);
     if (rows == 0) return BB_OK;
     if (dtype == BB_BF16)
-        BB_DISPATCH_IT(bf16, cols / 8, (ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
+        BB_DISPATCH_IT(bf16, cols / 8, (ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st, dropped, key)));
     else
-        BB_DISPATCH_IT(float, cols / 4, (ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st)));
+        BB_DISPATCH_IT(float, cols / 4, (ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st, dropped, key)));
     return BB_EINVAL;
 }
 static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
@@ -426,11 +454,22 @@ extern "C" int bb_layernorm_bwd(int dtype, int kind, int rows, int cols, float e
 
 extern "C" int bb_layernorm_bwd_rows(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain, const float* mean,
                                      const float* rinv, const void* dy, const void* dres, void* dx, float* dgain, float* dshift,
-                                     float* partials, bb_partial_sums* sums, void* stream) {
+                                     float* partials, bb_partial_sums* sums, void* dropped, float p, uint32_t k0, uint32_t k1, void* stream) {
     BB_REQUIRE(dgain && dshift && sums, "bb_layernorm_bwd_rows: null pointer");
+    BB_REQUIRE(!dropped || (p >= 0.f && p < 1.f), "bb_layernorm_bwd_rows: p must be in [0, 1)");
     *sums = {partials, dgain, dshift, 0, cols};
+    DropKey key = {};
+    if (dropped && rows > 0 && cols > 0) {
+        key = bb_drop_key(p, k0, k1, (uint64_t)rows * (uint64_t)cols);
+        // a probability too small to drop anything: a copy, as bb_dropout_apply makes it
+        if (!key.thresh) {
+            const int rc = bb_layernorm_bwd_rows(dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partials, sums,
+                                                 nullptr, 0.f, 0, 0, stream);
+            return rc ? rc : bb_dropout_apply(dtype, (int64_t)rows * cols, dx, dropped, p, k0, k1, stream);
+        }
+    }
     return ln_bwd_rows("bb_layernorm_bwd_rows", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, partials, sums->parts,
-                       (hipStream_t)stream);
+                       (hipStream_t)stream, dropped, key);
 }
 
 // ---- the same for callers that cannot allocate ---------------------------------------------------------------
@@ -447,7 +486,7 @@ static std::mutex g_ln_static_mu;
 
 template <typename T, int IT> static hipError_t ln_bwd_allow_one_pass() {
     // the largest dynamic LDS request the kernel makes for cols <= BB_LN_BWD_STATIC_MAX_COLS: the one-pass layout
-    return bb_allow_dynamic_lds((const void*)layernorm_bwd_kernel<T, IT>, 128 * 1024);
+    return bb_allow_dynamic_lds((const void*)layernorm_bwd_kernel<T, IT, false>, 128 * 1024);
 }
 // once per device, with that device current: the address of the device's copy, and every LDS-limit change the
 // entry point could otherwise need on its first call
@@ -831,13 +870,7 @@ __global__ __launch_bounds__(256) void dropout_kernel(int64_t nvec, const T* src
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nvec; i += (int64_t)gridDim.x * 256) {
         float v[VEC];
         load_vec(src + i * VEC, v);
-#pragma unroll
-        for (int e = 0; e < VEC; e += 2) {   // VEC is even: one hash per two neighbouring elements
-            const uint32_t x = key.small ? bb_dropout_pair_bits32(key.k0, key.k1, (uint32_t)(i * VEC + e) >> 1)
-                                         : bb_dropout_pair_bits(key.k0, key.k1, (uint64_t)(i * VEC + e) >> 1);
-            v[e] = bb_keep_even(x, key.thresh) ? v[e] * key.scale : 0.f;
-            v[e + 1] = bb_keep_odd(x, key.thresh) ? v[e + 1] * key.scale : 0.f;
-        }
+        drop_vec<VEC>(key, i * VEC, v);
         store_vec(dst + i * VEC, v);
     }
 }

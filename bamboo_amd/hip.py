@@ -94,7 +94,8 @@ def lib():
     L.bb_layernorm_bwd_workspace.argtypes = [c_int]
     L.bb_layernorm_bwd_workspace.restype = c_int64
     L.bb_layernorm_bwd.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 11
-    L.bb_layernorm_bwd_rows.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 10 + [POINTER(PartialSums), c_void_p]
+    L.bb_layernorm_bwd_rows.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 10 + [
+        POINTER(PartialSums), c_void_p, c_float, c_uint32, c_uint32, c_void_p]
     L.bb_partial_sums_acc.argtypes = [POINTER(PartialSums), c_int, c_void_p]
     L.bb_gemm_grouped_sums.argtypes = [POINTER(GemmDesc), c_int, POINTER(PartialSums), c_int, c_void_p]
     L.bb_layernorm_bwd_static.argtypes = [c_int, c_int, c_int, c_int, c_float] + [c_void_p] * 10
@@ -409,17 +410,20 @@ def layernorm_bwd(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, workspace, k
                                  _ptr(workspace), stream_ptr(stream)), "bb_layernorm_bwd")
 
 
-def layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partials, kind, eps, stream=None):
+def layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partials, kind, eps, stream=None, dropped=None, dropout=None):
     """:func:`layernorm_bwd` without its second launch: the gain and shift gradients are left as sums per block in ``partials``,
-    which stays untouched until ``gemm_grouped(sums=)`` or :func:`partial_sums` has added up what this returns."""
+    which stays untouched until ``gemm_grouped(sums=)`` or :func:`partial_sums` has added up what this returns.
+    ``dropped``: what ``dropout_apply(dx, dropped, *dropout)`` would make, in the same launch."""
     rows, cols = x.shape
+    _like("layernorm_bwd_rows", x, dropped=dropped)
+    p, key = dropout if dropped is not None else (0.0, (0, 0))
     _check_ln_bwd("layernorm_bwd_rows", x, gain, mean, rinv, dy, dres, dx, dgain, dshift)
     if partials.numel() < layernorm_bwd_workspace(cols) or partials.dtype != torch.float32:
         raise HipKernelError("layernorm_bwd_rows: partials too small")
     sums = PartialSums()
     check(lib().bb_layernorm_bwd_rows(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(mean), _ptr(rinv), _ptr(dy),
-                                      _ptr(dres), _ptr(dx), _ptr(dgain), _ptr(dshift), _ptr(partials), byref(sums), stream_ptr(stream)),
-          "bb_layernorm_bwd_rows")
+                                      _ptr(dres), _ptr(dx), _ptr(dgain), _ptr(dshift), _ptr(partials), byref(sums), _ptr(dropped), float(p),
+                                      int(key[0]), int(key[1]), stream_ptr(stream)), "bb_layernorm_bwd_rows")
     return sums
 
 

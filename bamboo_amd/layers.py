@@ -273,11 +273,13 @@ class TransformerLayer:
         h, f = self.hidden, self.ffn
         return batch * seq * (8 * h * h + 4 * h * f) + 4 * batch * seq * seq * h
 
-    def _layernorm_bwd(self, sums, ctx, x, norm, mean, rinv, dy, dres, dx):
-        """LayerNorm backward; its gain's and shift's gradients join ``sums``, at most two until the launch that adds them up."""
+    def _layernorm_bwd(self, sums, ctx, x, norm, mean, rinv, dy, dres, dx, dropped=None, site=None):
+        """LayerNorm backward; its gain's and shift's gradients join ``sums``, at most two until the launch that adds them up.
+        ``dropped``: the gradient behind the dropout ``site`` of the sublayer in front as well."""
         partials = ctx.buf("ln_partials", (2, hip.layernorm_bwd_workspace(self.hidden)))[len(sums)]
         sums.append(hip.layernorm_bwd_rows(x, self.w[norm + ".a_2"], mean, rinv, dy, dres, dx, self.g[norm + ".a_2"], self.g[norm + ".b_2"],
-                                           partials, hip.LN_CODES[self.ln], self.eps, stream=ctx.stream))
+                                           partials, hip.LN_CODES[self.ln], self.eps, stream=ctx.stream, dropped=dropped,
+                                           dropout=None if dropped is None else self._drop(ctx, site)))
 
     # ------------------------------------------------------------------ attention core
     def _heads_gemm(self, ctx, layout, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, alpha=1.0):
@@ -427,12 +429,10 @@ class TransformerLayer:
         wgrad(d_ffn, st["n2"], "feed_forward.w_1.weight")
         ctx.gemm(hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
         # d_x1 = d_out + LN2'(d_n2)
-        self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h1)
+        d_drop = ctx.buf("d_drop0", (R, h)) if self.dropout > 0 else None
+        self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h1, d_drop, self.SITE_SUBLAYER0)
         # attention output projection
-        d_proj = d_h1
-        if self.dropout > 0:
-            d_proj = ctx.buf("d_drop0", (R, h))
-            hip.dropout_apply(d_h1, d_proj, *self._drop(ctx, self.SITE_SUBLAYER0), stream=sm)
+        d_proj = d_h1 if d_drop is None else d_drop
         wgrad(d_proj, st["ctx"], "self_attn.linears.3.weight")
         ctx.gemm(hip.NN, d_proj, w["self_attn.linears.3.weight"], d_h0, stream=sm)
         self._attention_bwd(d_h0, d_qkv, st, ctx)
@@ -602,12 +602,10 @@ class DecoderLayer(TransformerLayer):
         wgrad(d_ffn, st["n2"], "feed_forward.w_1.weight")
         ctx.gemm(hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
         # d_x2 = d_out + LN2'(d_n2)  -> d_h2
-        self._layernorm_bwd(sums, ctx, st["x2"], "sublayer.2.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h2)
+        d_drop = ctx.buf("d_drop_src", (R, h)) if self.dropout > 0 else None
+        self._layernorm_bwd(sums, ctx, st["x2"], "sublayer.2.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h2, d_drop, self.SITE_SUBLAYER_SRC)
         # ---- sublayer 1: attention over the memory
-        d_proj = d_h2
-        if self.dropout > 0:
-            d_proj = ctx.buf("d_drop_src", (R, h))
-            hip.dropout_apply(d_h2, d_proj, *self._drop(ctx, self.SITE_SUBLAYER_SRC), stream=sm)
+        d_proj = d_h2 if d_drop is None else d_drop
         wgrad(d_proj, st["ctx_src"], "src_attn.linears.3.weight")
         ctx.gemm(hip.NN, d_proj, w["src_attn.linears.3.weight"], d_h0, stream=sm)
         self._attention_bwd(d_h0, d_qkv, self._src_views(st), ctx, site=self.SITE_SRC_ATTENTION, mask="none")
@@ -617,13 +615,11 @@ class DecoderLayer(TransformerLayer):
         ctx.gemm(hip.NN, d_qkv[:, :h], w["src_attn.linears.0.weight"], d_h0, stream=sm)        # d_n_src
         ctx.gemm(hip.NN, d_qkv[:, h:], w["kv.weight"], d_mem, stream=sm)                       # gradient of the memory
         # d_x1 = d_x2 + LN_src'(d_n_src)  -> d_h1
-        self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean_src"], st["rinv_src"], d_h0, d_h2, d_h1)
+        d_drop = ctx.buf("d_drop0", (R, h)) if self.dropout > 0 else None
+        self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean_src"], st["rinv_src"], d_h0, d_h2, d_h1, d_drop, self.SITE_SUBLAYER0)
         flush()      # d_qkv, d_ffn and the first sublayers' gradient buffers are free again
         # ---- sublayer 0: self-attention
-        d_proj0 = d_h1
-        if self.dropout > 0:
-            d_proj0 = ctx.buf("d_drop0", (R, h))
-            hip.dropout_apply(d_h1, d_proj0, *self._drop(ctx, self.SITE_SUBLAYER0), stream=sm)
+        d_proj0 = d_h1 if d_drop is None else d_drop
         wgrad(d_proj0, st["ctx"], "self_attn.linears.3.weight")
         ctx.gemm(hip.NN, d_proj0, w["self_attn.linears.3.weight"], d_h0, stream=sm)
         self._attention_bwd(d_h0, d_qkv, st, ctx, site=self.SITE_ATTENTION)

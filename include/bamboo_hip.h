@@ -191,11 +191,12 @@ int bb_layernorm_bwd(int dtype, int kind, int rows, int cols, float eps, const v
                      float* workspace, void* stream);
 /* The first half of it: dx, and per-block sums of dgain / dshift in `partials` (at least
  * bb_layernorm_bwd_workspace(cols) elements, the caller's until they are added up).  *sums says what is
- * left to add, for bb_partial_sums_acc or bb_gemm_grouped_sums; together the same bits.               */
+ * left to add, for bb_partial_sums_acc or bb_gemm_grouped_sums; together the same bits.  dropped
+ * (may be NULL): [rows, cols], what bb_dropout_apply(p, k0, k1) makes of dx.                          */
 int bb_layernorm_bwd_rows(int dtype, int kind, int rows, int cols, float eps, const void* x,
                           const void* gain, const float* mean, const float* rinv, const void* dy,
                           const void* dres, void* dx, float* dgain, float* dshift, float* partials,
-                          bb_partial_sums* sums, void* stream);
+                          bb_partial_sums* sums, void* dropped, float p, uint32_t k0, uint32_t k1, void* stream);
 /* The same without a workspace, for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * per-block partial sums live in an array inside the library's device image (4 MiB per GPU, held until

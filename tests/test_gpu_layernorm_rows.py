@@ -62,3 +62,27 @@ def test_parameter_gradients_beside_weight_gradients(hiplib, dtype, rows, cols, 
     assert all(torch.equal(a, b) for other in outs[1:] for a, b in zip(outs[0], other))
     with pytest.raises(hiplib.HipKernelError):
         hiplib.gemm_grouped(descs, sums=sums * 3)      # more than a launch takes
+
+
+# The gradient behind a dropout, written beside the one in front of it: the same bits as the dropout of what is stored, and dx and the
+# parameter gradients as without; every width of the kernel, with and without a residual; a probability too small to drop anything.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,cols,p", [(1, 64, 0.1), (37, 72, 0.5), (4097, 512, 0.1), (300, 1032, 0.1), (50, 2304, 0.3), (21, 4104, 0.1), (40, 128, 1e-7)])
+def test_gradient_behind_a_dropout(hiplib, dtype, rows, cols, p):
+    if dtype == torch.float32 and cols > 4096:
+        cols = 4096
+    g = torch.Generator().manual_seed(rows + cols)
+    x, dy, res, gain = (torch.randn(*s, generator=g).to(dtype).to(DEV) for s in ((rows, cols), (rows, cols), (rows, cols), (cols,)))
+    mean, rinv = x.float().mean(1), 1 / (x.float().var(1, unbiased=False) + 1e-5).sqrt()
+    for dres in (None, res):
+        outs = []
+        for together in (False, True):
+            dx, dropped = torch.empty_like(x), torch.full_like(x, float("nan"))
+            vec = [torch.zeros(cols, device=DEV) for _ in range(2)]
+            ws = torch.full((hiplib.layernorm_bwd_workspace(cols),), float("nan"), device=DEV)
+            kw = dict(dropped=dropped, dropout=(p, (11, 23))) if together else {}
+            hiplib.partial_sums([hiplib.layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, *vec, ws, hiplib.LN_STANDARD, 1e-5, **kw)])
+            if not together:
+                hiplib.dropout_apply(dx, dropped, p, (11, 23))
+            outs.append([dx, dropped, *vec])
+        assert all(torch.equal(a, b) for a, b in zip(*outs))
