@@ -364,6 +364,13 @@ class TransformerLayer:
     # ------------------------------------------------------------------ forward / backward
     def forward(self, x, st, ctx):
         """x: [rows, hidden] (kept by reference in the stash); returns st['out']."""
+        self.rebuild(x, st, ctx)
+        ctx.gemm(hip.NT, st["act"], self.w["feed_forward.w_2.weight"], st["out"], bias=self.w["feed_forward.w_2.bias"],
+                 epilogue=hip.EPI_RESIDUAL, resid=st["x1"], dropout=self._drop(ctx, self.SITE_SUBLAYER1), stream=ctx.stream)
+        return st["out"]
+
+    def rebuild(self, x, st, ctx):
+        """``forward`` as far as this layer's backward pass needs it: all but its last product."""
         w, sm = self.w, ctx.stream
         kind, act = hip.LN_CODES[self.ln], hip.ACT_CODES[self.activation]
         st["x0"] = x
@@ -386,9 +393,6 @@ class TransformerLayer:
                      epilogue=hip.EPI_ACT, act=act, dropout=self._drop(ctx, self.SITE_FFN), stream=sm)
         else:
             self._ffn1(st, ctx)
-        ctx.gemm(hip.NT, st["act"], w["feed_forward.w_2.weight"], st["out"], bias=w["feed_forward.w_2.bias"],
-                 epilogue=hip.EPI_RESIDUAL, resid=st["x1"], dropout=self._drop(ctx, self.SITE_SUBLAYER1), stream=sm)
-        return st["out"]
 
     def _ffn1(self, st, ctx):
         """act and act' of the feed-forward's hidden layer; under dropout both carry the keep factor, so the backward
@@ -537,6 +541,12 @@ class DecoderLayer(TransformerLayer):
         return {"qkv": st["qkv_src"], "ctx": st["ctx_src"], "lse": st.get("lse_src"), "prob": st.get("prob_src")}
 
     def forward(self, x, st, ctx):
+        self.rebuild(x, st, ctx)
+        ctx.gemm(hip.NT, st["act"], self.w["feed_forward.w_2.weight"], st["out"], bias=self.w["feed_forward.w_2.bias"],
+                 epilogue=hip.EPI_RESIDUAL, resid=st["x2"], dropout=self._drop(ctx, self.SITE_SUBLAYER1), stream=ctx.stream)
+        return st["out"]
+
+    def rebuild(self, x, st, ctx):
         w, sm = self.w, ctx.stream
         kind, act = hip.LN_CODES[self.ln], hip.ACT_CODES[self.activation]
         h = self.hidden
@@ -566,9 +576,6 @@ class DecoderLayer(TransformerLayer):
                      epilogue=hip.EPI_ACT, act=act, dropout=self._drop(ctx, self.SITE_FFN), stream=sm)
         else:
             self._ffn1(st, ctx)
-        ctx.gemm(hip.NT, st["act"], w["feed_forward.w_2.weight"], st["out"], bias=w["feed_forward.w_2.bias"],
-                 epilogue=hip.EPI_RESIDUAL, resid=st["x2"], dropout=self._drop(ctx, self.SITE_SUBLAYER1), stream=sm)
-        return st["out"]
 
     def backward(self, d_out, d_x, st, ctx):
         w, g, sm = self.w, self.g, ctx.stream

@@ -548,13 +548,36 @@ class PipelineModule:
             return x
         kept = self._kept[stage_id][slot]
         for g, (a, b) in enumerate(self._checkpoint_groups(stage_id)):
-            hip.cast(x, kept[g], stream=ctx.stream)   # same-type copy: the group's input outlives the work stash
+            if x is not kept[g]:
+                hip.cast(x, kept[g], stream=ctx.stream)   # same-type copy: the group's input outlives the work stash
             x = kept[g]
-            for i in range(a, b):
+            for i in range(a, b - 1):
                 ctx.seq = seqs[i]
                 x = layers[i].forward(x, stash[i], ctx)
-        hip.cast(x, kept[-1], stream=ctx.stream)
+            ctx.seq = seqs[b - 1]
+            x = self._forward_into(kept[g + 1], layers[b - 1], x, stash[b - 1], ctx)
+        if x is not kept[-1]:
+            hip.cast(x, kept[-1], stream=ctx.stream)
         return kept[-1]
+
+    @staticmethod
+    def _forward_into(dst, layer, x, st, ctx):
+        """A layer's forward pass, its output at ``dst`` where the layer writes it to the stash's ``out`` (else where it returns it)."""
+        out = st.get("out")
+        if out is None or out.shape != dst.shape or out.dtype != dst.dtype:
+            return layer.forward(x, st, ctx)
+        st["out"] = dst
+        try:
+            return layer.forward(x, st, ctx)
+        finally:
+            st["out"] = out
+
+    @staticmethod
+    def _rebuild(layer):
+        """What fills the stash of a group's last layer for its backward pass: its ``rebuild``, if whoever defines the layer's
+        ``forward`` defines that too, else ``forward``."""
+        owner = next(cls for cls in type(layer).__mro__ if "forward" in vars(cls))
+        return layer.rebuild if "rebuild" in vars(owner) and "forward" not in vars(layer) else layer.forward
 
     def note_replay(self, stage_id, slot, forward_input):
         """What :meth:`forward` keeps beside its launches, for a forward whose launches were replayed."""
@@ -618,9 +641,11 @@ class PipelineModule:
                 # update running statistics a second time
                 was, ctx.redundant = ctx.redundant, True
                 x = self._kept[stage_id][slot][g]
-                for i in range(a, b):
+                for i in range(a, b - 1):
                     ctx.seq = seqs[i]
                     x = layers[i].forward(x, stash[i], ctx)
+                ctx.seq = seqs[b - 1]
+                self._rebuild(layers[b - 1])(x, stash[b - 1], ctx)
                 ctx.redundant = was
             presummed = False
             for i in range(b - 1, a - 1, -1):
