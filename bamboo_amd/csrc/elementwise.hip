@@ -1272,36 +1272,56 @@ __global__ __launch_bounds__(256) void bn_finish_kernel(int what, int rows, int 
 }
 
 // Forward BatchNorm from the strip triples a convolution's GEMM epilogue leaves (per 32 rows and channel: pivot p,
-// S1 = sum (x - p), S2 = sum (x - p)^2), statistics and normalisation in ONE launch.  A block owns 64 channels and
-// one of gridDim.y row ranges.  Every block first turns the strips of its channels into mean and variance -- a
+// S1 = sum (x - p), S2 = sum (x - p)^2), statistics and normalisation in ONE launch.  A block owns a slab of channels and
+// one of the row ranges.  Every block first turns the strips of its channels into mean and variance -- a
 // strip's mean is p + S1/n and its sum of squared deviations M2 = S2 - S1^2/n (no cancellation: p is a sample of the
 // strip); two passes over the triples, which stay in registers (at most 8192 rows): mean = sum n_s mean_s / rows,
-// then sum (M2_s + n_s (mean_s - mean)^2) -- lane = channel (256-byte reads), its sixteen waves taking strips w,
-// w + 16, ..., the sixteen partial sums added in wave order by every thread (a fixed order, the same in every
+// then sum (M2_s + n_s (mean_s - mean)^2) -- lane = channel, sixteen groups of threads taking strips w,
+// w + 16, ..., the sixteen partial sums added in that order by every thread (a fixed order, the same in every
 // block: all row ranges of a channel normalise with the same bits).  The block of the first row range also writes
 // mean, rstd and the running statistics.  Then y = gamma (x - mean) rstd + beta (+ resid) (ReLU) over the block's
-// rows, eight lanes per row of the 64 channels (128-byte segments).  The tensor is read once, but every block reads all
-// strips of its channels: at 6272 rows 150 KB a block, 38.5 MB a launch of 256 blocks, out of L2 -- 12 times the tensor at 256
-// columns, 3 times at 1024 (L1's read requests: 41.9 and 51.5 MB in all).  What it was taken against is a launch of its own for
-// the statistics (5.4 + 5.5 us against 7.9 at 6272 x 256).  (For few rows the reduction is what the launch waits for: loads for all 256 strips / for the sixteens there are, us: 900 rows x 512 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 / 6.5;
-// the rows of a thread fetched ahead, all of them or the next one, gained nothing.)
-constexpr int BN_STRIP_WAVES = 16, BN_STRIP_MAX = 16;   // 16 * 16 strips = up to 8192 rows
-constexpr int BN_FWD_ROW_RANGES = 64;
-__global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int rows, int cols, float eps, float momentum, int relu,
+// rows, eight channels a lane.  The tensor is read once, but every block reads all
+// strips of its channels: at 6272 rows 150 KB a block of 64, 38.5 MB a launch of 256 blocks, out of L2 -- 12 times the tensor at 256
+// columns (half that with 32), 3 times at 1024 (L1's read requests with 64: 41.9 and 51.5 MB in all).  What it was taken against is a launch of its own for
+// the statistics (5.4 + 5.5 us against 7.9 at 6272 x 256).  (For few rows the reduction is what the launch waits for: loads for all 256 strips / for the sixteens there are, us, on 64 channels a block: 900 rows x 512
+// 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 / 6.5; the rows of a thread fetched ahead, all of them or the next one, gained nothing.)
+//
+// A slab is 32 channels, each of the sixteen shares a group of 32 threads: with 64 a launch of as many blocks reads twice as much of
+// the strips.  64 channels / 32 / and the strips' counts without a division each (us): 6272 x 256 6.6 / 5.6 / 5.15, 3136 x 1024 6.9 /
+// 6.4 / 5.9, 900 x 512 5.3 / 4.6 / 4.2, 200 x 64 5.0 / 4.4 / 3.9, 6272 x 1024 8.6 / 7.8 / 7.4, with a residual 9.9 / 9.5 / 9.3.  (All slabs of a row
+// range on one XCD, which then reads every strip: 9.7 and 11.9.  The backward twin, which reads two tensors and fewer strips,
+// gains nothing by it: 4.3 / 4.4 at 6272 x 256, 7.8 / 8.6 x 1024.)
+constexpr int BN_STRIP_GROUPS = 16, BN_STRIP_MAX = 16;   // 16 * 16 strips = up to 8192 rows
+constexpr int BN_SLAB = 32, BN_STRIP_THREADS = BN_STRIP_GROUPS * BN_SLAB;
+// about one block per CU; wide tensors get fewer row ranges (each repeats the strip reduction of its channels)
+static int bn_row_ranges(int cols) { return max(4, min(64, 128 / ((cols + 63) / 64))); }
+static int bn_strip_blocks(int cols) { return ((cols + 63) / 64 * bn_row_ranges(cols) + 7) / 8 * 16; }
+// The slab and the row range of a block (false: one that only fills the grid up): the two slabs of 64 channels, which share lines of the
+// tensor, on one XCD, and there for as many row ranges as come out: that XCD reads few channels' strips.
+__device__ __forceinline__ bool bn_place(int cols, int ranges, int& slab, int& range) {
+    const int lines = (cols + 63) / 64, at = blockIdx.x / 16 * 8 + blockIdx.x % 8;
+    slab = at % lines * 2 + blockIdx.x / 8 % 2;
+    range = at / lines;
+    return range < ranges;
+}
+__global__ __launch_bounds__(BN_STRIP_THREADS) void bn_fwd_strips_kernel(int rows, int cols, int ranges, float eps, float momentum, int relu,
                                                             const float* __restrict__ strips, const bf16* __restrict__ x,
                                                             const bf16* __restrict__ gamma, const bf16* __restrict__ beta,
                                                             const bf16* __restrict__ resid, bf16* __restrict__ y,
                                                             float* __restrict__ mean, float* __restrict__ rstd,
                                                             float* __restrict__ run_mean, float* __restrict__ run_var) {
-    __shared__ float red[2][BN_STRIP_WAVES][64];
-    __shared__ float fold[2][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = min(blockIdx.x * 64 + lane, cols - 1);   // lanes past the last channel repeat it and store nothing
+    constexpr int LPR = BN_SLAB / 8, RPP = BN_STRIP_THREADS / LPR;
+    __shared__ float red[2][BN_STRIP_GROUPS][BN_SLAB];
+    __shared__ float fold[2][BN_SLAB];
+    const int lane = threadIdx.x % BN_SLAB, grp = threadIdx.x / BN_SLAB;
+    int slab, range;
+    if (!bn_place(cols, ranges, slab, range)) return;
+    const int c = min(slab * BN_SLAB + lane, cols - 1);   // lanes past the last channel repeat it and store nothing
     const int nstrips = (rows + 31) / 32;
     // the rows this thread normalises first are fetched now, so that they travel while the statistics are reduced
-    const int v8 = (threadIdx.x & 7) * 8, c0 = blockIdx.x * 64 + v8;
-    const int per = (rows + gridDim.y - 1) / gridDim.y;
-    const int r0 = blockIdx.y * per + (threadIdx.x >> 3), r1 = min(rows, ((int)blockIdx.y + 1) * per);
+    const int v8 = (threadIdx.x % LPR) * 8, c0 = slab * BN_SLAB + v8;
+    const int per = (rows + ranges - 1) / ranges;
+    const int r0 = range * per + threadIdx.x / LPR, r1 = min(rows, (range + 1) * per);
     const bool first = c0 < cols && r0 < r1;
     float xv[8], rv[8];
     if (first) {
@@ -1312,8 +1332,8 @@ __global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int 
 #pragma unroll
     for (int j = 0; j < BN_STRIP_MAX; ++j) {
         p[j] = a[j] = b[j] = 0.f;
-        if (j * BN_STRIP_WAVES < nstrips) {   // (the same in all waves: a scalar branch, and the loads inside still go out together)
-            const int s = min(j * BN_STRIP_WAVES + wave, nstrips - 1);   // clamped: unused ones get n = 0
+        if (j * BN_STRIP_GROUPS < nstrips) {   // (the same in all waves: a scalar branch, and the loads inside still go out together)
+            const int s = min(j * BN_STRIP_GROUPS + grp, nstrips - 1);   // clamped: unused ones get n = 0
             const float* t = strips + ((int64_t)s * 3) * cols + c;
             p[j] = t[0];
             a[j] = t[cols];
@@ -1321,22 +1341,23 @@ __global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int 
         }
     }
     float sm = 0.f;
+    const float last_n = (float)(rows - (nstrips - 1) * 32), last_inv = 1.0f / last_n;   // 1 / 32 exactly where the strip is whole
 #pragma unroll
     for (int j = 0; j < BN_STRIP_MAX; ++j) {
-        const int s = j * BN_STRIP_WAVES + wave;
-        const int cnt = s < nstrips ? min(32, rows - s * 32) : 0;
-        const float n = (float)cnt, inv = cnt == 32 ? 0.03125f : cnt > 0 ? 1.0f / n : 0.f;
+        const int s = j * BN_STRIP_GROUPS + grp;
+        const bool whole = s < nstrips - 1, any = s < nstrips;
+        const float n = whole ? 32.f : any ? last_n : 0.f, inv = whole ? 0.03125f : any ? last_inv : 0.f;
         const float m = p[j] + a[j] * inv;           // the strip's mean
-        b[j] = cnt > 0 ? b[j] - a[j] * a[j] * inv : 0.f;   // its sum of squared deviations
+        b[j] = any ? b[j] - a[j] * a[j] * inv : 0.f;   // its sum of squared deviations
         p[j] = m;
         a[j] = n;
         sm += n * m;
     }
-    red[0][wave][lane] = sm;
+    red[0][grp][lane] = sm;
     __syncthreads();
     float tot = 0.f;
 #pragma unroll
-    for (int w = 0; w < BN_STRIP_WAVES; ++w) tot += red[0][w][lane];
+    for (int w = 0; w < BN_STRIP_GROUPS; ++w) tot += red[0][w][lane];
     const float mu = tot / (float)rows;
     float sq = 0.f;
 #pragma unroll
@@ -1344,18 +1365,18 @@ __global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int 
         const float d = p[j] - mu;
         sq += b[j] + a[j] * d * d;
     }
-    red[1][wave][lane] = sq;
+    red[1][grp][lane] = sq;
     __syncthreads();
-    if (wave == 0) {
+    if (grp == 0) {
         float q = 0.f;
 #pragma unroll
-        for (int w = 0; w < BN_STRIP_WAVES; ++w) q += red[1][w][lane];
+        for (int w = 0; w < BN_STRIP_GROUPS; ++w) q += red[1][w][lane];
         const float var = fmaxf(q / (float)rows, 0.f);
         const float rs = 1.0f / sqrtf(var + eps);
         const float sc = Elem<bf16>::load(gamma + c) * rs;
         fold[0][lane] = sc;
         fold[1][lane] = Elem<bf16>::load(beta + c) - mu * sc;
-        if (blockIdx.y == 0 && blockIdx.x * 64 + lane < cols) {
+        if (range == 0 && slab * BN_SLAB + lane < cols) {
             mean[c] = mu;
             rstd[c] = rs;
             if (run_mean) {  // nn.BatchNorm2d: running_var uses the unbiased estimate
@@ -1373,7 +1394,7 @@ __global__ __launch_bounds__(BN_STRIP_WAVES * 64) void bn_fwd_strips_kernel(int 
         sc[e] = fold[0][v8 + e];
         sh[e] = fold[1][v8 + e];
     }
-    for (int r = r0; r < r1; r += BN_STRIP_WAVES * 8) {
+    for (int r = r0; r < r1; r += RPP) {
         const int64_t off = (int64_t)r * cols + c0;
         if (r != r0) {
             load_vec(x + off, xv);
@@ -1648,13 +1669,12 @@ extern "C" int bb_batchnorm_fwd_strips(int dtype, int rows, int cols, float eps,
     if (rc) return rc;
     BB_REQUIRE(dtype == BB_BF16, "bb_batchnorm_fwd_strips: bf16 only (the kernels that leave strip statistics are)");
     BB_REQUIRE(x && gamma && beta && y && mean && rstd && strip_stats, "bb_batchnorm_fwd_strips: null pointer");
-    BB_REQUIRE(rows <= 32 * BN_STRIP_WAVES * BN_STRIP_MAX, "bb_batchnorm_fwd_strips: at most %d rows", 32 * BN_STRIP_WAVES * BN_STRIP_MAX);
+    BB_REQUIRE(rows <= 32 * BN_STRIP_GROUPS * BN_STRIP_MAX, "bb_batchnorm_fwd_strips: at most %d rows", 32 * BN_STRIP_GROUPS * BN_STRIP_MAX);
     BB_REQUIRE((running_mean == nullptr) == (running_var == nullptr), "bb_batchnorm_fwd_strips: give both running buffers or none");
     hipStream_t st = (hipStream_t)stream;
     // about one block per CU; wide tensors get fewer row ranges (each repeats the strip reduction of its channels)
-    const int slabs = (cols + 63) / 64;
-    const int ranges = max(4, min(BN_FWD_ROW_RANGES, 256 / slabs));
-    bb_launch(bn_fwd_strips_kernel, dim3(slabs, ranges), dim3(BN_STRIP_WAVES * 64), 0, st, rows, cols, eps, momentum, relu,
+    const int ranges = bn_row_ranges(cols);
+    bb_launch(bn_fwd_strips_kernel, dim3(bn_strip_blocks(cols)), dim3(BN_STRIP_THREADS), 0, st, rows, cols, ranges, eps, momentum, relu,
                        strip_stats, (const bf16*)x, (const bf16*)gamma, (const bf16*)beta, (const bf16*)resid, (bf16*)y, mean, rstd,
                        running_mean, running_var);
     BB_LAUNCH_CHECK();
