@@ -1,5 +1,5 @@
-// fp32 GEMM: v_mfma_f32_32x32x2_f32 on 64x64 tiles (four waves of 32x32), on 64x32 tiles whose contraction two groups of
-// two waves share, or on 32x32 tiles whose contraction four waves share; v_mfma_f32_16x16x4_f32 on quarters of a 64x64 tile.
+// fp32 GEMM: v_mfma_f32_16x16x4_f32 on 64x64 tiles (four waves of 32x32), on 64x32 tiles whose contraction two groups of
+// two waves share, or on quarters of a 64x64 tile; v_mfma_f32_32x32x2_f32 on 32x32 tiles whose contraction four waves share.
 #pragma once
 #include "gemm_kernels.h"
 
@@ -12,9 +12,13 @@
 // loop (16 values per lane: one round trip instead of sixteen behind the stores).
 // LDS formats, per operand and stage:
 //   K-contiguous memory: [rows][32 k], 128 B a row = 8 chunks of 16 B, chunk c of row r at c ^ ((r >> 1) & 7).
-//   k-major memory: [32 k][rows]; 64-row tiles keep rows 0..31 of odd k at the place of rows 32..63 and vice versa, so that
-//     the two halves of a wave (k and k + 1) read different banks.
-// Every element adds up its contraction in pairs (k, k + 1), k ascending; groups and waves each add up their share of it (the
+//   k-major memory: [32 k][rows]; the 16-row blocks of a k-row change places by k % 4 (64 rows) or k / 2 % 2 (32).
+// A 16x16x4 instruction's operand is sixteen rows and four k: one chunk of each row, all 64 banks once.  The same tiles on 32x32x2,
+// whose operand is two of the four words of 32 rows' chunks -- every bank in use twice, half the banks not at all --, and on
+// 16x16x4, four independent accumulators a wave (us): NT 2048x3072x768 92.1 / 82.8, 4096x4096x4096 1094 / 998, 2048x768x3072 (64x32
+// tiles) 92.2 / 87.2; NN, one operand k-major, 82.5 / 78.8, 1013 / 964, 85.4 / 84.0; TN 4096x4096x4096 1020 / 982, short ones equal.
+// (2048 tokens x 768, forward and backward of two layers: 19.05 / 18.4 ms.)
+// Every element adds up its contraction one by one, k ascending, whichever instruction does it; groups and waves each add up their share of it (the
 // even, resp. odd 16-wide k-tiles; one 32-wide slice) and the shares' sums are added in order.  Which kernel runs a
 // problem is a matter of its shape and layout alone.
 // (volatile: pairs of reads merged into one instruction have no room for the stage's offset, i.e. cost an addition each)
@@ -39,7 +43,7 @@ template <int ROWS, bool KM, int NW = 4, bool WIDE = false, bool QUADS = false> 
                 off[i] = (Offset)((int64_t)min(r, rows - 1 - row0) * ld + c * 4) * (Offset)4;
             } else {
                 constexpr int CPR = ROWS / 4, RPI = 64 / CPR;   // 16-byte chunks per k-row, k-rows per instruction
-                const int k = q * RPI + lane / CPR, c = (lane % CPR) ^ (ROWS == 64 ? 8 * (k & 1) : QUADS ? 4 * ((k >> 1) & 1) : 0);
+                const int k = q * RPI + lane / CPR, c = (lane % CPR) ^ (!QUADS ? 0 : ROWS == 64 ? 4 * (k & 3) : 4 * ((k >> 1) & 1));
                 k_lane[i] = k;
                 off[i] = (Offset)((int64_t)k * ld + min(c * 4, rows - 4 - row0)) * (Offset)4;
             }
@@ -60,25 +64,49 @@ template <int ROWS, bool KM, int NW = 4, bool WIDE = false, bool QUADS = false> 
         base += step;
     }
 };
-// The operand values of a wave: lane = row (lane & 31), its half's k of the pairs (4 c, 4 c + 1) and (4 c + 2, 4 c + 3) of
-// chunk c.  NC: chunks of a k-tile the wave takes, from chunk c0 on.
-template <int ROWS, bool KM, int NC> struct F32Reader {
-    unsigned at[KM ? 1 : NC];   // LDS addresses inside stage 0
+// The operand values of a wave's 32 rows: lane = row (lane & 15) of either half, k (lane >> 4) of each chunk of four.  NC: chunks of a
+// k-tile the wave takes, from chunk c0 on.
+template <int ROWS, bool KM, int NC> struct F32QuadReader {
+    unsigned at[KM ? 2 : NC];   // LDS addresses inside stage 0; k-major: of either half
     __device__ __forceinline__ void init(unsigned lds, int row0, int c0, int lane) {
-        const int r = row0 + (lane & 31), h = lane >> 5;
-        if constexpr (KM) at[0] = lds + ((4 * c0 + h) * ROWS + (ROWS == 64 ? r ^ (32 * h) : r)) * 4;
+        const int r = row0 + (lane & 15), kq = lane >> 4;
+        if constexpr (KM) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) at[i] = lds + ((4 * c0 + kq) * ROWS + ((r + 16 * i) ^ (ROWS == 64 ? 16 * kq : 16 * (kq >> 1)))) * 4;
+        } else {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) at[c] = lds + r * 128 + (((c0 + c) ^ ((r >> 1) & 7)) << 4) + 4 * kq;
+        }
+    }
+    // chunks FIRST .. FIRST + N - 1 of the stage STAGE_OFF bytes behind stage 0
+    template <int STAGE_OFF, int FIRST, int N> __device__ __forceinline__ void load(float (&v)[N][2]) const {
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                v[c][i] = KM ? *((lds_f32*)at[KM ? i : 0] + STAGE_OFF / 4 + (FIRST + c) * 4 * ROWS) : *((lds_f32*)at[KM ? 0 : FIRST + c] + STAGE_OFF / 4 + i * 16 * 32);
+    }
+};
+
+// The same for 32x32x2 instructions, of a tile of 32 rows: lane = row (lane & 31), its half's k of the pairs (4 c, 4 c + 1) and
+// (4 c + 2, 4 c + 3) of chunk c.
+template <bool KM, int NC> struct F32Reader {
+    unsigned at[KM ? 1 : NC];   // LDS addresses inside stage 0
+    __device__ __forceinline__ void init(unsigned lds, int lane) {
+        const int r = lane & 31, h = lane >> 5;
+        if constexpr (KM) at[0] = lds + (h * 32 + r) * 4;
         else {
 #pragma unroll
-            for (int c = 0; c < NC; ++c) at[c] = lds + r * 128 + (((c0 + c) ^ ((r >> 1) & 7)) << 4) + 4 * h;
+            for (int c = 0; c < NC; ++c) at[c] = lds + r * 128 + ((c ^ ((r >> 1) & 7)) << 4) + 4 * h;
         }
     }
     // chunks FIRST .. FIRST + N - 1 of the stage STAGE_OFF bytes behind stage 0
     template <int STAGE_OFF, int FIRST, int N> __device__ __forceinline__ void load(float (&v)[N][2]) const {
 #pragma unroll
         for (int c = 0; c < N; ++c) {
-            lds_f32* p = KM ? (lds_f32*)at[0] + STAGE_OFF / 4 + (FIRST + c) * 4 * ROWS : (lds_f32*)at[FIRST + c] + STAGE_OFF / 4;
+            lds_f32* p = KM ? (lds_f32*)at[0] + STAGE_OFF / 4 + (FIRST + c) * 128 : (lds_f32*)at[FIRST + c] + STAGE_OFF / 4;
             v[c][0] = p[0];
-            v[c][1] = p[KM ? 2 * ROWS : 2];
+            v[c][1] = p[KM ? 64 : 2];
         }
     }
 };
@@ -91,9 +119,9 @@ constexpr int f32_gemm_lds(int bn) { return f32_stages(bn) * (64 + bn) * 128; }
 // the product -- the operand of the epilogue kind, else the C it accumulates into -- fetched before the main loop; `rest`: a
 // problem that reads both, or a masked residual, fetches the second here.  One branch over the kind around them, not
 // inside: the code stays small.
-template <int NR, typename V>
+template <int NR, int STEP = 8, typename V>
 __device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, int m0, int n, float bias, const float (&pre)[NR], V& v) {
-    const auto row = [&](int r) { return m0 + 8 * (r >> 2) + (r & 3); };
+    const auto row = [&](int r) { return m0 + STEP * (r >> 2) + (r & 3); };
     const bool has_opnd = epilogue_operand(g) != nullptr;
     float rest[NR], keep[NR];
 #pragma unroll
@@ -159,8 +187,8 @@ template <bool TA, bool TB, int BN, bool WIDE = false>
 __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block_id, const int batch_id, const bool logical_id) {
     static_assert(BN == 64 || BN == 32, "tiles: 64x64, 64x32 with the contraction shared by two groups");
     constexpr int KG = 64 / BN;
-    using OpA = F32Operand<64, TA, 4, WIDE>;
-    using OpB = F32Operand<BN, TB, 4, WIDE>;
+    using OpA = F32Operand<64, TA, 4, WIDE, true>;
+    using OpB = F32Operand<BN, TB, 4, WIDE, true>;
     constexpr int STAGES = f32_stages(BN), STAGE = OpA::BYTES + OpB::BYTES, LOADS = OpA::ROUNDS + OpB::ROUNDS;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -178,31 +206,38 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block
 
     constexpr int NC = 8 / KG;   // chunks of four k of a k-tile that this wave multiplies
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t*)smem;
-    F32Reader<64, TA, NC> ra;
-    F32Reader<BN, TB, NC> rb;
+    F32QuadReader<64, TA, NC> ra;
+    F32QuadReader<BN, TB, NC> rb;
     ra.init(lds0, wm * 32, grp * NC, lane);
     rb.init(lds0 + OpA::BYTES, wn * 32, grp * NC, lane);
 
-    // what the epilogue reads: lane = column, register r = row acc_m + 8 (r / 4) + r % 4
-    const int n = n0 + wn * 32 + (lane & 31), acc_m = m0 + wm * 32 + 4 * (lane >> 5);
+    // what the epilogue reads: lane = column n + 16 j, register r = row acc_m + 16 (r / 4) + r % 4
+    const int n = n0 + wn * 32 + (lane & 15), acc_m = m0 + wm * 32 + 4 * (lane >> 4);
     const float* opnd = (const float*)epilogue_operand(g);
     const int64_t ld_pre = opnd ? g.ldaux : g.ldc;
     if (!opnd && g.accumulate) opnd = (const float*)g.C;
-    float bias = 0.f, pre[16];
+    float bias[2] = {0.f, 0.f}, pre[2][8];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) pre[r] = 0.f;
-    const int nc = min(n, g.N - 1);    // clamped: what is read for a row or column past the end is not used
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) pre[j][r] = 0.f;
     if (grp == 0) {
-        if (g.bias) bias = ((const float*)g.bias)[nc];
-        if (opnd) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) pre[r] = opnd[coff + (int64_t)min(acc_m + 8 * (r >> 2) + (r & 3), g.M - 1) * ld_pre + nc];
+        for (int j = 0; j < 2; ++j) {
+            const int nc = min(n + 16 * j, g.N - 1);    // clamped: what is read for a row or column past the end is not used
+            if (g.bias) bias[j] = ((const float*)g.bias)[nc];
+            if (opnd) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) pre[j][r] = opnd[coff + (int64_t)min(acc_m + 16 * (r >> 2) + (r & 3), g.M - 1) * ld_pre + nc];
+            }
         }
     }
 
-    f32x16 acc;
+    f32x4 acc[2][2];   // [row half][column half]
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int KT = (g.K + 31) / 32;
     int issued = 0, into = 0;
@@ -220,7 +255,7 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block
 #pragma unroll
         for (int c = 0; c < NC / 2; ++c)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[c][i], y[c][i], acc, 0, 0, 0);
+            for (int t = 0; t < 4; ++t) acc[t >> 1][t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c][t >> 1], y[c][t & 1], acc[t >> 1][t & 1], 0, 0, 0);
     };
     // the k-tile after kt - 1 has landed (in-order completion; with three stages one more may be in flight) and every wave has
     // read that one: its stage takes the next
@@ -271,18 +306,28 @@ __device__ __forceinline__ void gemm_f32_body(const GemmArgs& g, const int block
     }
     if constexpr (KG > 1) {
         // group 1's partial tile through the (drained) stages
-        float* part = (float*)smem + wm * (16 * 64);
+        f32x4* part = (f32x4*)smem + wm * (4 * 64);
         __syncthreads();
         if (grp == 1) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) part[r * 64 + lane] = acc[r];
+            for (int t = 0; t < 4; ++t) part[t * 64 + lane] = acc[t >> 1][t & 1];
         }
         __syncthreads();
         if (grp == 1) return;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] += part[r * 64 + lane];
+        for (int t = 0; t < 4; ++t) {
+            const f32x4 other = part[t * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[t >> 1][t & 1][e] += other[e];
+        }
     }
-    if (n < g.N) epilogue_f32<16>(g, coff, acc_m, n, bias, pre, acc);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        float v[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[r] = acc[r >> 2][j][r & 3];
+        if (n + 16 * j < g.N) epilogue_f32<8, 16>(g, coff, acc_m, n + 16 * j, bias[j], pre[j], v);
+    }
 }
 
 template <bool TA, bool TB, int BN, bool WIDE = false>
@@ -327,10 +372,10 @@ __device__ __forceinline__ void gemm_f32_wave_body(const GemmArgs& g, const int 
     opa.base += wave * opa.step;
     opb.base += wave * opb.step;
     const unsigned lds = (unsigned)(uintptr_t)(lds_ptr_t*)smem + wave * SLICE;
-    F32Reader<32, TA, 8> ra;
-    F32Reader<32, TB, 8> rb;
-    ra.init(lds, 0, 0, lane);
-    rb.init(lds + OpA::BYTES, 0, 0, lane);
+    F32Reader<TA, 8> ra;
+    F32Reader<TB, 8> rb;
+    ra.init(lds, lane);
+    rb.init(lds + OpA::BYTES, lane);
     const int left = g.K - wave * 32;
     if (left > 0) {
         opa.issue(lds, 0, left, lane);

@@ -311,3 +311,33 @@ def test_weight_gradients_of_a_full_round(hiplib, rows):
             hiplib.gemm_grouped(group)
         runs.append(C + bias)
     assert all(torch.equal(x, y) for x, y in zip(*runs))
+
+
+# fp32 tiles of 64x64 and 64x32 whose waves hold four 16x16 accumulators: columns and rows that end in either half of either, every
+# operand order and the epilogues that read and write beside the product.  A chain of K multiply-adds errs by at most K eps of the
+# terms' sum; what the epilogue adds, a few roundings more.
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("M,N,K", [(2052, 420, 36), (2084, 436, 132), (2112, 404, 64), (2076, 1028, 100)])
+def test_f32_tiles_at_their_edges(hiplib, M, N, K, layout):
+    lay = getattr(hiplib, layout.upper())
+    a, b = torch.randn(M, K, generator=torch.Generator().manual_seed(1)), torch.randn(N, K, generator=torch.Generator().manual_seed(2))
+    A, B = (a.t() if layout == "tn" else a).contiguous().to(DEV), (b if layout == "nt" else b.t()).contiguous().to(DEV)
+    x, bias = torch.randn(M, N, generator=torch.Generator().manual_seed(3)).to(DEV), torch.randn(N, generator=torch.Generator().manual_seed(4)).to(DEV)
+    prod = (a.double() @ b.double().t()).to(DEV)
+    bound = (K + 4) * 2.0 ** -24 * ((a.double().abs() @ b.double().abs().t()).to(DEV) + x.double().abs() + bias.double().abs())
+    C = torch.full((M, N), float("nan"), device=DEV)
+    hiplib.gemm(lay, A, B, C)
+    assert bool(((C.double() - prod).abs() <= bound).all())
+    C = x.clone()
+    hiplib.gemm(lay, A, B, C, accumulate=True)
+    assert bool(((C.double() - prod - x.double()).abs() <= bound).all())
+    if layout != "tn":
+        C = torch.full((M, N), float("nan"), device=DEV)
+        hiplib.gemm(lay, A, B, C, bias=bias if layout == "nt" else None, epilogue=hiplib.EPI_RESIDUAL, resid=x)
+        want = prod + x.double() + (bias.double() if layout == "nt" else 0)
+        assert bool(((C.double() - want).abs() <= bound).all())
+    if layout == "nt":
+        act, dact = torch.full((M, N), float("nan"), device=DEV), torch.full((M, N), float("nan"), device=DEV)
+        hiplib.gemm(lay, A, B, act, bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_RELU, aux_out=dact)
+        want = prod + bias.double()
+        assert bool(((act.double() - want.clamp(min=0)).abs() <= bound).all()) and bool(((dact == 1) == (act > 0)).all())
