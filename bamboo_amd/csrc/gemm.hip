@@ -292,10 +292,11 @@ static bool pick_f32_split(int M, int N, int K, int64_t batches, int layout) {
 // Of what is left for the tiles of 64x64 and 64x32, problems of at most 128 64x64 tiles take four blocks a tile instead, with the same
 // bits (gemm_f32_quarter_kernel): until then every CU has at most two of them.  Larger tiles / this (us, back to back): NT
 // 128x128x128 7.0 / 5.2, 512x512x256 (64 tiles) 10.7 / 5.8, 1000x448x448 (112) 16.3 / 10.2, 1024x512x512 (128) 11.2 / 11.4,
-// 1024x512x2048 32.3 / 29.9, 512x1536x256 (192) 11.4 / 11.2, 1000x1344x448 (336) 25.1 / 26.8, 2048x768x768 (384) 29.0 / 37.9; NN alike.
-static bool pick_f32_quarter(int M, int N, int64_t batches, int layout) {
-    return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches <= 128;
-}
+// 1024x512x2048 32.3 / 29.9, 512x1536x256 (192) 11.4 / 11.2, 1000x1344x448 (336) 25.1 / 26.8, 2048x768x768 (384) 29.0 / 37.9; NN alike.  TN: 64x64x4096 85 / 41, 512x512x2048 45 / 24, 512x1024x1000 (128)
+// 25.2 / 18.3; the weight gradients of a layer together, hidden size (x 4 in the feed-forward) and rows: 128 (48 tiles) 7680 159 / 80, 200 10.7 /
+// 7.5; 192 (108) 3000 67 / 46; 256 (192) 1072 29.4 / 31.2, 320 (300) 600 28.2 / 31.6; ResNet blocks of 64 channels (17) 6272 pixels 131 / 65.
+static constexpr int kF32QuarterTiles = 128;
+static bool pick_f32_quarter(int M, int N, int64_t batches) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches <= kF32QuarterTiles; }
 template <bool TA, bool TB, int KG> static int launch_f32_quarter(GemmArgs& g, int batches, hipStream_t st) {
     auto kern = gemm_f32_quarter_kernel<TA, TB, KG>;
     g.tiles_m = (g.M + 31) / 32;
@@ -325,10 +326,10 @@ template <bool TA, bool TB> static int dispatch_f32(GemmArgs& g, int batches, hi
     if (f32_wide(g.lda, g.ldb)) return launch_f32<TA, TB, 64, true>(g, batches, st);
     if (pick_f32_wave(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT)) return launch_f32_wave<TA, TB>(g, batches, st);
     const bool split = pick_f32_split(g.M, g.N, g.K, batches, TA ? BB_TN : TB ? BB_NN : BB_NT);
+    const bool quarter = pick_f32_quarter(g.M, g.N, batches);
+    if (quarter && !split) return launch_f32_quarter<TA, TB, 1>(g, batches, st);
     if constexpr (!TA) {
-        if (pick_f32_quarter(g.M, g.N, batches, TB ? BB_NN : BB_NT))
-            return split ? launch_f32_quarter<TA, TB, 2>(g, batches, st) : launch_f32_quarter<TA, TB, 1>(g, batches, st);
-        if (split) return launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
+        if (split) return quarter ? launch_f32_quarter<TA, TB, 2>(g, batches, st) : launch_f32<TA, TB, kF32SplitBN>(g, batches, st);
     }
     return launch_f32<TA, TB, 64>(g, batches, st);
 }
@@ -348,7 +349,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
     else if (f32_wide(d->lda, d->ldb)) snprintf(out, out_len, "f32_%s_64x64wide", layouts[d->layout]);
     else if (pick_f32_wave(d->M, d->N, d->K, batches, d->layout)) snprintf(out, out_len, "f32_%s_wave32x32k%d", layouts[d->layout], kF32Waves);
     else {
-        const char* quarter = pick_f32_quarter(d->M, d->N, batches, d->layout) ? "quarter" : "";
+        const char* quarter = pick_f32_quarter(d->M, d->N, batches) ? "quarter" : "";
         if (pick_f32_split(d->M, d->N, d->K, batches, d->layout))
             snprintf(out, out_len, "f32_%s_%s64x%dk%d", layouts[d->layout], quarter, kF32SplitBN, kF32SplitGroups);
         else snprintf(out, out_len, "f32_%s_%s64x64", layouts[d->layout], quarter);
@@ -754,7 +755,11 @@ extern "C" int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const 
         GroupedArgs G;
         G.count = count;
         G.ride = ride;
-        const int tile = waves ? 32 : 64;
+        int64_t tiles64 = 0;
+        for (int i = 0; i < count; ++i) tiles64 += (int64_t)((descs[i].M + 63) / 64) * ((descs[i].N + 63) / 64);
+        // weight gradients: on quarter tiles (the bits of 64x64 ones) by the tiles of all of them
+        const bool quarter = !waves && descs[0].layout == BB_TN && tiles64 <= kF32QuarterTiles;
+        const int tile = waves || quarter ? 32 : 64;
         int blocks = 0;
         for (int i = 0; i < count; ++i) {
             int64_t batches;
@@ -770,10 +775,11 @@ extern "C" int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const 
         int rc = colsum_f32(descs, count, stream);
         if (rc) return rc;
         const int layout = descs[0].layout;
-        const auto kern = layout == BB_NT   ? gemm_f32_grouped_kernel<false, false>
+        const auto kern = quarter            ? gemm_f32_quarter_grouped_kernel
+                          : layout == BB_NT ? gemm_f32_grouped_kernel<false, false>
                           : layout == BB_NN ? waves ? gemm_f32_wave_grouped_kernel<false, true> : gemm_f32_grouped_kernel<false, true>
                                             : waves ? gemm_f32_wave_grouped_kernel<true, true> : gemm_f32_grouped_kernel<true, true>;
-        bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(256), waves ? kF32WaveLds : f32_gemm_lds(64), st, G);
+        bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(256), waves ? kF32WaveLds : quarter ? kF32QuarterLds : f32_gemm_lds(64), st, G);
         BB_LAUNCH_CHECK();
         return BB_OK;
     }

@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_wave_grouped_kernel(const Gro
 constexpr int kF32QuarterStages = 4;
 constexpr int kF32QuarterLds = kF32QuarterStages * 2 * 2 * 32 * 128;
 template <bool TA, bool TB, int KG>
-__global__ __launch_bounds__(256 * KG, 2) void gemm_f32_quarter_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm_f32_quarter_body(const GemmArgs& g, const int block_id, const int batch_id, const bool logical_id) {
     constexpr int NW = 4 * KG, NST = kF32QuarterStages;
     using OpA = F32Operand<32, TA, 4, false, true>;     // a k-tile of 32: four instructions
     using OpB = F32Operand<32, TB, 4, false, true>;
@@ -454,9 +454,10 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_f32_quarter_kernel(const Gem
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int quad = wave & 3, grp = wave >> 2, wm = quad & 1, wn = quad >> 1;
     int tile_m, tile_n;
-    tile_coords(blockIdx.x, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    if (logical_id) panel_coords(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    else tile_coords(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
     const int m0 = tile_m * 32, n0 = tile_n * 32;
-    const int b1 = blockIdx.z / g.nb2, b2 = blockIdx.z % g.nb2;
+    const int b1 = batch_id / g.nb2, b2 = batch_id % g.nb2;
     const int64_t coff = b1 * g.sC1 + b2 * g.sC2;
     // a stage is two 32-wide k-tiles of both operands; with one group every wave loads a quarter of each, with two a group loads one k-tile
     OpA opa;
@@ -584,4 +585,16 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_f32_quarter_kernel(const Gem
         for (int r = 0; r < 4; ++r) acc[r] += part[r * 64 + lane];
     }
     if (n < g.N) epilogue_f32<4>(g, coff, acc_m, n, bias, pre, acc);
+}
+template <bool TA, bool TB, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void gemm_f32_quarter_kernel(const GemmArgs g) {
+    gemm_f32_quarter_body<TA, TB, KG>(g, blockIdx.x, blockIdx.z, false);
+}
+// weight gradients of few tiles over many rows
+__global__ __launch_bounds__(256, 2) void gemm_f32_quarter_grouped_kernel(const GroupedArgs G) {
+    const int lid = grouped_place<4>(G);
+    if (lid < 0) return;
+    int pi = 0;
+    while (pi + 1 < G.count && lid >= G.first_block[pi + 1]) ++pi;
+    gemm_f32_quarter_body<true, true, 1>(G.p[pi], lid - G.first_block[pi], 0, true);
 }

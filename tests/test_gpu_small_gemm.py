@@ -341,3 +341,22 @@ def test_f32_tiles_at_their_edges(hiplib, M, N, K, layout):
         hiplib.gemm(lay, A, B, act, bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_RELU, aux_out=dact)
         want = prod + bias.double()
         assert bool(((act.double() - want.clamp(min=0)).abs() <= bound).all()) and bool(((dact == 1) == (act > 0)).all())
+
+
+# fp32 weight gradients on quarter tiles against the same in a group of too many tiles for them, and each alone: the same bits.
+@pytest.mark.parametrize("rows", [132, 196, 260, 1000])
+@pytest.mark.parametrize("shapes", [[(384, 128), (128, 512)], [(68, 36), (100, 644), (4, 32)], [(512, 512), (256, 1024)]])
+def test_f32_weight_gradients_on_quarter_tiles(hiplib, rows, shapes):
+    f32 = lambda *s, seed: torch.randn(*s, generator=torch.Generator().manual_seed(seed)).to(DEV)
+    ops = [(f32(rows, m, seed=2 * i), f32(rows, n, seed=2 * i + 1)) for i, (m, n) in enumerate(shapes + [(1024, 768)])]
+    outs = []
+    for how in ("few", "many", "alone"):
+        C = [torch.ones(a.shape[1], b.shape[1], device=DEV) for a, b in ops]
+        descs = [hiplib.gemm_desc(hiplib.TN, a, b, c, accumulate=True) for (a, b), c in zip(ops, C)]
+        for group in {"few": [descs[:-1]], "many": [descs], "alone": [[d] for d in descs[:-1]]}[how]:
+            hiplib.gemm_grouped(group)
+        outs.append(C[:-1])
+    assert all(torch.equal(a, b) for other in outs[1:] for a, b in zip(outs[0], other))
+    for (a, b), c in zip(ops, outs[0]):
+        prod, terms = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+        assert bool(((c.double() - 1 - prod).abs() <= (rows + 4) * 2.0 ** -24 * (terms + 1)).all())
