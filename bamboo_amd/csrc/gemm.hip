@@ -133,10 +133,10 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
     //  - Problems of at most one tile of 128x64 per CU (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle) take those,
-    //    short contractions also up to 400, whose chains run under each other; then 128x128 tiles of three stages, one per CU, up to
+    //    short contractions also up to 400, very short ones up to 512, whose chains run under each other; then 128x128 tiles of three stages, one per CU, up to
     //    a round of them.  128x64 / 128x128 (64x128 / 128x128), plain and with a residual (us): NT 1200x1600x1600 (250 tiles of
     //    128x64) 12.3 12.9 / 15.1 16.8, 2300x1024x1024 (288) 12.2 12.8 / 11.7 12.9, 4096x768x768 (384) 10.8 11.3 / 10.4 11.4, x3072 30.2
-    //    30.8 / 25.1 26.5, 3136x1024x256 (400) 7.4 8.1 / 7.8 8.7, 6272x512x128 (392) 6.7 7.4 / 7.1 8.0; NN 12.1 12.7 / 15.1 16.5, 12.2 12.9 /
+    //    30.8 / 25.1 26.5, 3136x1024x256 (400) 7.4 8.1 / 7.8 8.7, 6272x512x128 (392) 6.7 7.4 / 7.1 8.0, 8112x512x128 (512) 6.8 / 7.8; NN 12.1 12.7 / 15.1 16.5, 12.2 12.9 /
     //    11.8 13.1, 10.9 11.5 / 10.7 11.5, 30.4 30.6 / 25.3 26.7, 7.4 8.2 / 7.9 8.8.  A round of 128x128 with two stages or 32-wide k-tiles
     //    (two and three blocks per CU) / this: NT 8192x512x512 10.7 11.9 / 9.6 10.5, x2048 26.2 28.9 / 21.1 22.4, NN 10.2 11.5 / 9.8 10.6,
     //    26.2 28.9 / 21.4 22.4; 256x128 / this where a few rows stand against many columns: 640x6400x1600 24.1 25.6 / 17.3 19.0.  More
@@ -144,7 +144,8 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     //    32-wide k-tiles (K % 64 != 0) as before: 128x64 tiles up to 128 tiles of 128x128 and for short forward contractions.
     if (k64) {
         const int64_t halves = nt ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
-        if (halves <= (K >= 768 ? 256 : 400)) return nt ? D128x64k64s3 : D64x128k64s3;
+        // (one or two k-tiles forward: whatever their size -- the launch is its epilogue, which many small tiles share out)
+        if ((nt && K < 256) || halves <= (K >= 768 ? 256 : K >= 512 ? 400 : 512)) return nt ? D128x64k64s3 : D64x128k64s3;
         if (t128 <= 256) return D128x128k64s3;
     } else {
         if ((K <= 512 || t128 <= 128) && nt) return D128x64s3;

@@ -217,9 +217,11 @@ class TransformerLayer:
         return ctx.dtype == torch.bfloat16 and (self.head_dim in (64, 128) or (self.head_dim == 32 and self.heads % 2 == 0))
 
     def kept_probs_kernels(self, ctx):
-        """fp32 attention that keeps the probabilities in one launch forward and two backward; a matter of the shape alone, so
-        that a redundant forward and a normal forward of the same layer take the same kernels."""
-        return hip.attention_probs_supported(ctx.dtype, ctx.batch, self.heads, ctx.seq, self.head_dim)
+        """fp32 attention that keeps the probabilities in one launch forward and two backward; a matter of the layer and the shape
+        alone, so that a redundant forward and a normal forward of the same layer take the same kernels.  Layers with a ReLU keep
+        the head products and the softmax kernel: another order of additions moves a ReLU's input by an fp32 rounding, and of
+        those that lie that close to zero, one in some millions, the gradient of the unit comes or goes."""
+        return self.activation != "relu" and hip.attention_probs_supported(ctx.dtype, ctx.batch, self.heads, ctx.seq, self.head_dim)
 
     def stash_specs(self, ctx):
         R, h, f = ctx.rows, self.hidden, self.ffn

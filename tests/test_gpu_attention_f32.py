@@ -53,7 +53,7 @@ def test_kept_probabilities(hiplib, mask, b, a, s, d, p):
     lens = torch.tensor([0, 1, s, s][:b] if b > 1 else [s - 1], dtype=torch.int32, device=DEV) if mask == "key_padding" else None
     got = []
     for kernels in (True, False):
-        layer = TransformerLayer(h, a, 4 * h, mask=mask, dropout=p)
+        layer = TransformerLayer(h, a, 4 * h, mask=mask, dropout=p, activation="gelu_tanh")
         layer.layer_idx = 3
         ctx = StageContext(b, s, torch.float32, torch.device(DEV))
         ctx.key_len, ctx.dropout_base = lens, (11, 2, 1)
