@@ -250,7 +250,8 @@ class TransformerLayer:
         return specs + self.forward_scratch_specs(ctx)
 
     def forward_scratch_specs(self, ctx):
-        if self.dropout > 0 and not self.fused_attention(ctx) and not self.kept_probs_kernels(ctx):
+        # (whichever kernels run now: the activation, which decides between them, may change between passes)
+        if self.dropout > 0 and not self.fused_attention(ctx):
             return [("prob_drop", (ctx.batch, self.heads, ctx.seq, ctx.seq), ctx.dtype)]   # dropped-out probabilities
         return []
 
