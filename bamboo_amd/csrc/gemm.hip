@@ -107,7 +107,8 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
         //    them.  Beyond that they read more and hide less than 128x128 tiles with a masked last k-tile (us, 64x64 / 128x128):
         //    NT 2048x1000x1000 (512 tiles) 13.2 / 14.4, 4096x1000x1000 21.9 / 17.7, 8192x4096x72 67 / 30, 8192x4096x4008 499 / 316;
         //    NN 8192x1000x4008 132 / 78; 48 heads, NN 1032x80x1032 50 / 34, NT 1032x1032x80 111 / 55; TN 1032x80x1032 53 / 39.
-        if (N % 8 != 0 || t64 <= 512) return D_NONE;
+        //    (An empty contraction has no k-tile to start with: the wave-sliced tiles go straight to their epilogue.)
+        if (N % 8 != 0 || t64 <= 512 || K == 0) return D_NONE;
         if (layout != BB_TN) return D128x128k64r;
         return K >= 64 ? D128x128s3 : D_NONE;
     }
