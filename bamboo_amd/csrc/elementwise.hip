@@ -346,10 +346,22 @@ int bb_partial_sums_args(const char* who, const bb_partial_sums* sums, int count
     a.blocks = (a.blocks + 7) / 8 * 8;
     return BB_OK;
 }
+bool bb_partial_sums_apart(const bb_partial_sums* sums, int count) {
+    const auto apart = [](const float* x, int nx, const float* y, int ny) { return x + nx <= y || y + ny <= x; };
+    for (int i = 0; i < count; ++i)
+        for (int j = 0; j < i; ++j)
+            for (const float* x : {sums[i].out0, sums[i].out1})
+                if (!apart(x, sums[i].n, sums[j].out0, sums[j].n) || !apart(x, sums[i].n, sums[j].out1, sums[j].n)) return false;
+    return true;
+}
 extern "C" int bb_partial_sums_acc(const bb_partial_sums* sums, int count, void* stream) {
     PartialSums a;
     int rc = bb_partial_sums_args("bb_partial_sums_acc", sums, count, a);
     if (rc || a.blocks == 0) return rc;
+    if (!bb_partial_sums_apart(sums, count)) {
+        for (int i = 0; i < count && rc == BB_OK; ++i) rc = bb_partial_sums_acc(sums + i, 1, stream);
+        return rc;
+    }
     bb_launch(partial_sums_kernel, dim3(a.first_block[count]), dim3(RED_WAVES * 64), 0, (hipStream_t)stream, a);
     BB_LAUNCH_CHECK();
     return BB_OK;

@@ -722,6 +722,10 @@ extern "C" int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const 
     PartialSums ride;
     int ride_rc = bb_partial_sums_args("bb_gemm_grouped_sums", sums, nsums, ride);
     if (ride_rc) return ride_rc;
+    if (!bb_partial_sums_apart(sums, nsums)) {     // into the same memory: one after the other, in launches of their own
+        ride_rc = bb_partial_sums_acc(sums, nsums, stream);
+        return ride_rc ? ride_rc : bb_gemm_grouped_sums(descs, count, nullptr, 0, stream);
+    }
     // one launch when every problem is an unbatched bf16 problem of one layout that the DMA
     // kernel accepts; otherwise the problems run one after the other (same results)
     bool has_conv = false;

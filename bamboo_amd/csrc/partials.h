@@ -64,3 +64,5 @@ template <int WAVES> __device__ __forceinline__ void partial_sums_block(const Pa
 
 // checked (elementwise.hip)
 int bb_partial_sums_args(const char* who, const bb_partial_sums* sums, int count, PartialSums& a);
+// whether no two of them add into the same memory: the blocks of a launch add without atomics
+bool bb_partial_sums_apart(const bb_partial_sums* sums, int count);

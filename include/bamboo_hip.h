@@ -149,7 +149,8 @@ int64_t bb_strip_stats_workspace(int rows, int cols);
  * fill the GPU although each has few output tiles.                                         */
 int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream);
 /* Sums of partial rows an earlier launch left: out0[i] += sum over p < parts of partial[p * 2n + i],
- * out1[i] likewise of partial[p * 2n + n + i], i < n, in a fixed order.                       */
+ * out1[i] likewise of partial[p * 2n + n + i], i < n, in a fixed order.  out0 and out1 of an entry do not
+ * overlap; entries that add into the same memory are done one after the other, in launches of their own. */
 #define BB_PARTIAL_SUMS_MAX 4
 typedef struct bb_partial_sums {
     const float* partial;
@@ -158,9 +159,10 @@ typedef struct bb_partial_sums {
     int parts, n;
 } bb_partial_sums;
 int bb_partial_sums_acc(const bb_partial_sums* sums, int count, void* stream);
-/* bb_gemm_grouped, with such sums (at most BB_PARTIAL_SUMS_MAX; their outputs are no operand of a
- * problem) done in the same launch where there is one: the gain and shift gradients of a layer's
- * LayerNorms (bb_layernorm_bwd_rows) beside its weight gradients.                             */
+/* bb_gemm_grouped, with such sums (at most BB_PARTIAL_SUMS_MAX) done in the same launch where there is
+ * one: the gain and shift gradients of a layer's LayerNorms (bb_layernorm_bwd_rows) beside its weight
+ * gradients.  The problems neither read nor write what the sums add into, and do not write their
+ * `partial`: the two run side by side.                                                         */
 int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const bb_partial_sums* sums, int nsums, void* stream);
 /* bb_gemm_grouped for problems with an fp32 C, few output tiles and a long contraction (weight
  * gradients dW += dy^T x of narrow layers, e.g. the three convolutions of resnet.py:49-75 over

@@ -86,3 +86,33 @@ def test_gradient_behind_a_dropout(hiplib, dtype, rows, cols, p):
                 hiplib.dropout_apply(dx, dropped, p, (11, 23))
             outs.append([dx, dropped, *vec])
         assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+# Two LayerNorms whose parameters are one (and a third beside them): sums that meet in the same memory, or in a part of it, are added
+# one after the other; the bits of calls one by one, in a launch of their own and beside weight gradients.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("shift", [0, 64])
+def test_sums_into_the_same_gradients(hiplib, dtype, shift):
+    rows, cols = 300, 136
+    g = torch.Generator().manual_seed(shift)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)
+    x, dys, gain = rand(rows, cols), [rand(rows, cols) for _ in range(3)], rand(cols)
+    mean, rinv = x.float().mean(1), 1 / (x.float().var(1, unbiased=False) + 1e-5).sqrt()
+    outs = []
+    for how in ("one by one", "by themselves", "beside"):
+        store, W = torch.full((4, 256), 0.5, device=DEV), [torch.ones(cols, cols, device=DEV) for _ in range(2)]
+        into = [(store[0, :cols], store[1, :cols]), (store[1, shift:shift + cols], store[0, shift:shift + cols]), (store[2, :cols], store[3, :cols])]
+        sums = []
+        for dy, (dgain, dshift) in zip(dys, into):
+            ws = torch.full((hiplib.layernorm_bwd_workspace(cols),), float("nan"), device=DEV)
+            args = (x, gain, mean, rinv, dy, None, torch.empty_like(x), dgain, dshift, ws, hiplib.LN_STANDARD, 1e-5)
+            if how == "one by one":
+                hiplib.layernorm_bwd(*args)
+            else:
+                sums.append((hiplib.layernorm_bwd_rows(*args), ws))
+        if how == "by themselves":
+            hiplib.partial_sums([s for s, _ in sums])
+        descs = [hiplib.gemm_desc(hiplib.TN, dy, x, w, accumulate=True) for dy, w in zip(dys, W)]
+        hiplib.gemm_grouped(descs, sums=[s for s, _ in sums] if how == "beside" else ())
+        outs.append([store] + W)
+    assert all(torch.equal(a, b) for other in outs[1:] for a, b in zip(outs[0], other))
