@@ -18,6 +18,7 @@ import torch
 
 from . import hip
 from .layers import StageContext
+from .replay import PASS_METHODS
 from .utils import partition_balanced, partition_uniform
 
 
@@ -592,11 +593,17 @@ class PipelineModule:
     def pass_state(self, stage_id, layers):
         """What the launches of a pass over the layers a..b-1 depend on beside its operands: every object by itself, to be
         compared by identity (a value inside a dict that a layer holds counts, one further down does not)."""
+        own, kind = vars(self), type(self)
         out = [self.base_seed, self.activation_checkpoint_interval, self._stash.get(stage_id), getattr(self, "_kept", {}).get(stage_id),
-               getattr(self, "stage_seq", {}).get(stage_id), vars(self).get("forward"), vars(self).get("backward")]
-        for layer in self.func_buckets[stage_id][layers[0]: layers[1]]:
-            own, cls = vars(layer), type(layer)
-            out += [layer, cls.forward, cls.backward]
+               getattr(self, "stage_seq", {}).get(stage_id)]
+        for m in _PASSES:
+            out += (own.get(m), getattr(kind, m))
+        layers = self.func_buckets[stage_id][layers[0]: layers[1]]
+        for cls in dict.fromkeys(map(type, layers)):
+            out += [getattr(cls, m, None) for m in PASS_METHODS]
+        for layer in layers:
+            own = vars(layer)
+            out.append(layer)
             out += own.values()
             for v in own.values():
                 if type(v) is dict:
@@ -604,9 +611,8 @@ class PipelineModule:
         return out
 
     def passes_launch_only(self):
-        """Whether :meth:`forward` and :meth:`backward` are those below: what they do beside launches is known (:meth:`note_replay`)."""
-        cls = type(self)
-        return cls.forward is PipelineModule.forward and cls.backward is PipelineModule.backward and not {"forward", "backward"} & set(vars(self))
+        """Whether a pass is made of the methods below: what they do beside launches is known (:meth:`note_replay`)."""
+        return all(getattr(type(self), m) is f for m, f in _PASSES.items()) and _PASSES.keys().isdisjoint(vars(self))
 
     def stage_memory(self, stage_id):
         """The blocks of memory that the passes of a stage use, beside what they are given: stash, parameters, gradients, and
@@ -688,3 +694,7 @@ class PipelineModule:
         ctx.ensure_workspace(ws)
         ctx.seq = seq
         return ctx
+
+
+# the methods a pass is made of, as they are here
+_PASSES = {m: getattr(PipelineModule, m) for m in ("forward", "backward", "_forward_into", "_rebuild")}

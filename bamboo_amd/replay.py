@@ -20,13 +20,17 @@ _HARMLESS = {"__init__", "__repr__", "__module__", "__qualname__", "__doc__", "_
              "__orig_bases__", "init_params", "num_params", "flops_fwd"}
 
 
+# what a pass of a stage calls on a layer
+PASS_METHODS = ("forward", "backward", "rebuild", "grad_sink")
+
+
 def _promises(kind):
     promised = False
     for cls in kind.__mro__[:-1]:
         own = vars(cls)
         if own.get("launches_only") is True:
             promised = True
-            if any(getattr(own.get(m), "__module__", cls.__module__) != cls.__module__ for m in ("forward", "backward")):
+            if any(getattr(own.get(m), "__module__", cls.__module__) != cls.__module__ for m in PASS_METHODS):
                 return False
         elif not own.keys() <= _HARMLESS:
             return False

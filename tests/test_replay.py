@@ -282,6 +282,61 @@ def test_a_class_whose_passes_were_replaced_is_not_replayed(stage, monkeypatch):
     assert stage.replayed() == 0 and stage.issued() == 3
 
 
+class Rebuilt(Layer):
+    launches_only = True
+
+    def forward(self, x, st, ctx):
+        return super().forward(x, st, ctx)
+
+    def rebuild(self, x, st, ctx):
+        pass
+
+    def grad_sink(self, st, ctx):
+        pass
+
+
+@pytest.mark.parametrize("method", replay.PASS_METHODS)
+def test_a_method_of_a_pass_replaced_in_its_class_is_seen(stage, monkeypatch, method):
+    """By one of the class's own module: recorded anew.  By another's: its Python code runs in every pass."""
+    stage.module.func_buckets[1] = [Rebuilt(COLS)]
+    x, inner = torch.randn(ROWS, COLS), getattr(Rebuilt, method)
+    stage.forward(x)
+    stage.forward(x)
+    assert (stage.issued(), stage.replayed()) == (1, 1)
+
+    def other(self, *a):
+        return inner(self, *a)
+    monkeypatch.setattr(Rebuilt, method, other)
+    for replayed in (1, 2):
+        stage.forward(x)
+        assert (stage.issued(), stage.replayed()) == (2, replayed)
+
+    def wrapped(self, *a):
+        return inner(self, *a)
+    wrapped.__module__ = "elsewhere"
+    monkeypatch.setattr(Rebuilt, method, wrapped)
+    for issued in (3, 4):
+        stage.forward(x)
+        assert (stage.issued(), stage.replayed()) == (issued, 2)
+
+
+@pytest.mark.parametrize("method", ["forward", "backward", "_forward_into", "_rebuild"])
+@pytest.mark.parametrize("where", ["class", "object"])
+def test_a_method_a_pass_is_made_of_replaced_in_the_module_is_seen(stage, monkeypatch, method, where):
+    x = torch.randn(ROWS, COLS)
+    stage.forward(x)
+    stage.forward(x)
+    assert (stage.issued(), stage.replayed()) == (1, 1)
+    target = stage.module if where == "object" else type(stage.module)
+    inner = getattr(target, method)
+    bound = where == "object" or method.startswith("_")
+    other = (lambda *a, **kw: inner(*a, **kw)) if bound else (lambda self, *a, **kw: inner(self, *a, **kw))
+    monkeypatch.setattr(target, method, staticmethod(other) if where == "class" and bound else other)
+    for issued in (2, 3):
+        stage.forward(x)
+        assert (stage.issued(), stage.replayed()) == (issued, 1)
+
+
 def test_replaying_can_be_switched_off(stage):
     x = torch.randn(ROWS, COLS)
     stage.forward(x)
