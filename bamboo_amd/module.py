@@ -13,6 +13,7 @@ import math
 import os
 import re
 from collections import OrderedDict
+from operator import attrgetter
 
 import torch
 
@@ -593,15 +594,13 @@ class PipelineModule:
     def pass_state(self, stage_id, layers):
         """What the launches of a pass over the layers a..b-1 depend on beside its operands: every object by itself, to be
         compared by identity (a value inside a dict that a layer holds counts, one further down does not)."""
-        own, kind = vars(self), type(self)
-        out = [self.base_seed, self.activation_checkpoint_interval, self._stash.get(stage_id), getattr(self, "_kept", {}).get(stage_id),
-               getattr(self, "stage_seq", {}).get(stage_id)]
-        for m in _PASSES:
-            out += (own.get(m), getattr(kind, m))
-        layers = self.func_buckets[stage_id][layers[0]: layers[1]]
-        for cls in dict.fromkeys(map(type, layers)):
-            out += [getattr(cls, m, None) for m in PASS_METHODS]
-        for layer in layers:
+        own, cls = vars(self), None
+        out = [self.base_seed, self.activation_checkpoint_interval, self._stash.get(stage_id), own.get("_kept", _EMPTY).get(stage_id),
+               own.get("stage_seq", _EMPTY).get(stage_id), *map(own.get, _PASSES), *_PASSES_OF(type(self))]
+        for layer in self.func_buckets[stage_id][layers[0]: layers[1]]:
+            if type(layer) is not cls:     # (once where neighbours are of one class)
+                cls = type(layer)
+                out += [getattr(cls, m, None) for m in PASS_METHODS]
             own = vars(layer)
             out.append(layer)
             out += own.values()
@@ -698,3 +697,5 @@ class PipelineModule:
 
 # the methods a pass is made of, as they are here
 _PASSES = {m: getattr(PipelineModule, m) for m in ("forward", "backward", "_forward_into", "_rebuild")}
+_PASSES_OF = attrgetter(*_PASSES)
+_EMPTY = {}
