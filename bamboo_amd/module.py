@@ -19,7 +19,6 @@ import torch
 
 from . import hip
 from .layers import StageContext
-from .replay import PASS_METHODS
 from .utils import partition_balanced, partition_uniform
 
 
@@ -594,17 +593,19 @@ class PipelineModule:
     def pass_state(self, stage_id, layers):
         """What the launches of a pass over the layers a..b-1 depend on beside its operands: every object by itself, to be
         compared by identity (a value inside a dict that a layer holds counts, one further down does not)."""
-        own, cls = vars(self), None
+        own, cls = self.__dict__, None
         out = [self.base_seed, self.activation_checkpoint_interval, self._stash.get(stage_id), own.get("_kept", _EMPTY).get(stage_id),
-               own.get("stage_seq", _EMPTY).get(stage_id), *map(own.get, _PASSES), *_PASSES_OF(type(self))]
-        for layer in self.func_buckets[stage_id][layers[0]: layers[1]]:
+               own.get("stage_seq", _EMPTY).get(stage_id), own.get("forward"), own.get("backward"), own.get("_forward_into"), own.get("_rebuild"),
+               *_PASSES_OF(type(self))]
+        a, b = layers
+        for layer in self.func_buckets[stage_id][a:b]:
             if type(layer) is not cls:     # (once where neighbours are of one class)
                 cls = type(layer)
-                out += [getattr(cls, m, None) for m in PASS_METHODS]
-            own = vars(layer)
+                out += (cls.forward, cls.backward, getattr(cls, "rebuild", None), getattr(cls, "grad_sink", None))   # PASS_METHODS
+            own = layer.__dict__.values()
             out.append(layer)
-            out += own.values()
-            for v in own.values():
+            out += own
+            for v in own:
                 if type(v) is dict:
                     out += v.values()
         return out

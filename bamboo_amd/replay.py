@@ -20,7 +20,7 @@ _HARMLESS = {"__init__", "__repr__", "__module__", "__qualname__", "__doc__", "_
              "__orig_bases__", "init_params", "num_params", "flops_fwd"}
 
 
-# what a pass of a stage calls on a layer
+# what a pass of a stage calls on a layer (the state of a stage lists them one by one: PipelineModule.pass_state)
 PASS_METHODS = ("forward", "backward", "rebuild", "grad_sink")
 
 
@@ -82,7 +82,8 @@ class Replay:
 
     def settled(self, stage_id, ctx, layers):
         """Whether passes of these layers may be replayed; drops what was recorded under another state of theirs."""
-        new = self.module.pass_state(stage_id, layers) + ctx.pass_state()
+        new = self.module.pass_state(stage_id, layers)
+        new += ctx.pass_state()
         old, memory = self._states.get((stage_id, layers), (None, None))
         # identity: the list keeps every object alive, numbers and strings do not change, and dicts are in it with their values
         if old is not None and len(old) == len(new) and all(map(is_, old, new)):
