@@ -392,9 +392,9 @@ def layernorm_bwd_workspace(cols):
     return int(lib().bb_layernorm_bwd_workspace(cols))
 
 
-def _check_ln_bwd(what, x, gain, mean, rinv, dy, dres, dx, dgain, dshift):
+def _check_ln_bwd(what, x, gain, mean, rinv, dy, dres, dx, dgain, dshift, dropped=None):
     rows, cols = x.shape
-    _like(what, x, dy=dy, dres=dres, dx=dx)
+    _like(what, x, dy=dy, dres=dres, dx=dx, dropped=dropped)
     _vector(what, cols, x.dtype, gain=gain)
     _vector(what, rows, torch.float32, mean=mean, rinv=rinv)
     _vector(what, cols, torch.float32, dgain=dgain, dshift=dshift)
@@ -415,9 +415,8 @@ def layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partial
     which stays untouched until ``gemm_grouped(sums=)`` or :func:`partial_sums` has added up what this returns.
     ``dropped``: what ``dropout_apply(dx, dropped, *dropout)`` would make, in the same launch."""
     rows, cols = x.shape
-    _like("layernorm_bwd_rows", x, dropped=dropped)
     p, key = dropout if dropped is not None else (0.0, (0, 0))
-    _check_ln_bwd("layernorm_bwd_rows", x, gain, mean, rinv, dy, dres, dx, dgain, dshift)
+    _check_ln_bwd("layernorm_bwd_rows", x, gain, mean, rinv, dy, dres, dx, dgain, dshift, dropped)
     if partials.numel() < layernorm_bwd_workspace(cols) or partials.dtype != torch.float32:
         raise HipKernelError("layernorm_bwd_rows: partials too small")
     sums = PartialSums()

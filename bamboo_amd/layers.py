@@ -122,6 +122,7 @@ class TransformerLayer:
 
     launches_only = True      # see replay.launches_only
     SITE_ATTENTION, SITE_SUBLAYER0, SITE_FFN, SITE_SUBLAYER1 = 0, 1, 2, 3
+    LN_PARTIALS = "ln_partials0", "ln_partials1"     # scratch of the LayerNorms whose parameter gradients wait for a launch together
 
     # parameter registration order of the reference's ``EncoderLayer`` (self_attn, feed_forward, sublayer:
     # transformer.py:161-168): the order of its ``state_dict()``, hence of the layer wire format
@@ -243,7 +244,7 @@ class TransformerLayer:
         attn = ("attn_delta", (ctx.batch, self.heads, ctx.seq), torch.float32) if self.fused_attention(ctx) else \
             ("d_prob", (ctx.batch, self.heads, ctx.seq, ctx.seq), dt)
         specs = [("d_ffn", (R, f), dt), ("d_h0", (R, h), dt), ("d_h1", (R, h), dt), ("d_qkv", (R, 3 * h), dt), attn,
-                 ("ln_partials", (2, hip.layernorm_bwd_workspace(h)), torch.float32)]
+                 *((name, (hip.layernorm_bwd_workspace(h),), torch.float32) for name in self.LN_PARTIALS)]
         if self.dropout > 0:
             # the gradients behind the two sublayer dropouts: the weight gradients read them at the end of the layer
             specs += [("d_drop0", (R, h), dt), ("d_drop1", (R, h), dt)]
@@ -279,7 +280,7 @@ class TransformerLayer:
     def _layernorm_bwd(self, sums, ctx, x, norm, mean, rinv, dy, dres, dx, dropped=None, site=None):
         """LayerNorm backward; its gain's and shift's gradients join ``sums``, at most two until the launch that adds them up.
         ``dropped``: the gradient behind the dropout ``site`` of the sublayer in front as well."""
-        partials = ctx.buf("ln_partials", (2, hip.layernorm_bwd_workspace(self.hidden)))[len(sums)]
+        partials = ctx.scratch[self.LN_PARTIALS[len(sums)]]
         sums.append(hip.layernorm_bwd_rows(x, self.w[norm + ".a_2"], mean, rinv, dy, dres, dx, self.g[norm + ".a_2"], self.g[norm + ".b_2"],
                                            partials, hip.LN_CODES[self.ln], self.eps, stream=ctx.stream, dropped=dropped,
                                            dropout=None if dropped is None else self._drop(ctx, site)))
