@@ -27,12 +27,12 @@ static int launch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES = 4, int BK = 32, bool RAGK = false, bool READ_AHEAD = true>
+template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES = 4, int BK = 32, bool RAGK = false>
 static int launch_bf16_dma(GemmArgs& g, int batches, hipStream_t st) {
     constexpr int smem = STAGES * (BM + BN) * BK * 2;
-    auto kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, RAGK, READ_AHEAD>;
+    auto kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, RAGK>;
     if constexpr (!AKM && !BKM) {       // dropout goes with forward (NT) products only: fill_args refuses the others
-        if (g.drop.thresh) kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, true, RAGK, READ_AHEAD>;
+        if (g.drop.thresh) kern = gemm_bf16_dma_kernel<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, true, RAGK>;
     }
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -60,10 +60,10 @@ template <int BM, int BN, int WM, int WN, bool TB> static int launch_bf16_dma_pe
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES = 3, bool READ_AHEAD = true>
+template <int BM, int BN, int WM, int WN, int STAGES = 3>
 static int launch_bf16_dma_stats(GemmArgs& g, hipStream_t st) {
     constexpr int smem = STAGES * (BM + BN) * 64 * 2;
-    auto kern = gemm_bf16_dma_stats_kernel<BM, BN, WM, WN, STAGES, READ_AHEAD>;
+    auto kern = gemm_bf16_dma_stats_kernel<BM, BN, WM, WN, STAGES>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -205,23 +205,6 @@ static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layou
     return t;
 }
 
-// Which main loop the 128x64 (NT) and 64x128 (NN) tiles of 64-wide k-tiles run; both give the same bits.  The one that reads a k-tile
-// ahead also fetches the epilogue's operand in front of the products, which inside a stage comes from memory: with an operand it
-// is the better one at any size.  Without, it shortens the chain of one tile, i.e. pays where a CU has one tile and that has more than
-// a few k-tiles; where blocks share a CU and cover for each other, its whole k-tile of fragments in front of the first product
-// only comes later.  The other loop / the one that reads ahead (us, back to back, outputs and operands from a ring of 600 MB):
-// NT 2043x768 (192 tiles) x 128 with a bias 5.2 / 5.4, with a residual 7.5 / 5.9, x 448 6.6 / 6.4 and 9.1 / 7.1, x 1024 9.5 / 8.8 and 12.0 /
-// 9.3; 12168x256 (384) x 128 6.4 / 7.0 and 9.1 / 8.7, x 512 9.2 / 9.6 and 12.3 / 11.0; 12168x512 (764) x 128 10.1 / 10.7 and 16.5 / 13.1; NN
-// 192 tiles x 128 4.8 / 5.1 and 7.3 / 5.8, x 448 6.4 / 6.4 and 9.0 / 7.2, 382 x 128 6.6 / 6.8 and 9.3 / 8.6, x 512 9.4 / 9.6 and 12.0 / 11.1.
-// (Inside a stage of 18 images, 26x26, 128 channels: 12168x512x128 11.3 / 12.0.)
-static bool read_ahead(const GemmArgs& g, int64_t tiles) { return epilogue_operand(g) || (tiles <= 256 && g.K >= 448); }
-// ... with strip statistics: 6272x256 (196 tiles) x 128 5.8 / 5.9, x 256 6.5 / 6.4, x 512 7.6 / 7.3; 3136x1024 (400) x 256 8.5 / 8.9, x 512
-// 10.6 / 10.8.  (The BatchNorm backward sums read operands in any case.)
-static bool read_ahead_stats(const GemmArgs& g, int64_t tiles) { return tiles <= 256 && g.K >= 256; }
-static int64_t tile_count(const GemmArgs& g, int bm, int bn, int64_t batches = 1) {
-    return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * batches;
-}
-
 // The wave-sliced kernels (gemm_wave.h) take the weight gradients whose 64x64 tiles are at most one per CU, and what the
 // DMA kernels do not take (contractions of odd lengths, few tiles).  W_8: eight waves, 32-wide slices, two stages each (130 KB of LDS);
 // W_4: four waves, 64-wide slices, one stage (65 KB, two blocks a CU).  Measured back to back, 128x128 DMA tiles / W_8 (us):
@@ -268,17 +251,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D128x128k64s3:
             if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
             else break;
-        case D128x64k64s3:
-            if constexpr (!TA && !TB) {
-                if (!read_ahead(g, tile_count(g, 128, 64, batches))) return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3, 64, false, false>(g, batches, st);
-                return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3, 64>(g, batches, st);
-            } else break;
+        case D128x64k64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3, 64>(g, batches, st);
         case D128x64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3>(g, batches, st);
-        case D64x128k64s3:
-            if constexpr (!TA && TB) {
-                if (!read_ahead(g, tile_count(g, 64, 128, batches))) return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64, false, false>(g, batches, st);
-                return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
-            } else break;
+        case D64x128k64s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
         case D64x128s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
         case D64x64k64s4:
             if constexpr (!TA) return launch_bf16_dma<64, 64, 2, 2, TA, TB, true, 4, 64>(g, batches, st);
@@ -515,7 +490,6 @@ extern "C" int bb_gemm(const bb_gemm_desc* d, void* stream) {
         const DmaTile dma = pick_dma_tile(d->M, d->N, d->K, 1, BB_NT);
         if (dma == D64x64k64s4) return launch_bf16_dma_stats<64, 64, 2, 2, 4>(g, (hipStream_t)stream);
         if (dma == D256x128k64s3) return launch_bf16_dma_stats<256, 128, 4, 2>(g, (hipStream_t)stream);
-        if (!read_ahead_stats(g, tile_count(g, 128, 64))) return launch_bf16_dma_stats<128, 64, 4, 1, 3, false>(g, (hipStream_t)stream);
         return launch_bf16_dma_stats<128, 64, 4, 1>(g, (hipStream_t)stream);
     }
     GemmArgs g;

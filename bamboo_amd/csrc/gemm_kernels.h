@@ -108,7 +108,7 @@ __device__ __forceinline__ void epilogue_elem(const GemmArgs& g, int64_t coff, i
 // The operand the epilogue kind reads beside the product (nullptr: none): the kernels fetch its 16 bytes per lane a
 // patch ahead of their use (epilogue_vec8_at<DROP, true>), so that the loads' latency passes under the previous
 // patch's work instead of in front of every patch's stores.
-__host__ __device__ __forceinline__ const bf16* epilogue_operand(const GemmArgs& g) {
+__device__ __forceinline__ const bf16* epilogue_operand(const GemmArgs& g) {
     if (g.epilogue == BB_EPI_DACT || g.epilogue == BB_EPI_MUL || g.epilogue == BB_EPI_MUL_POS) return (const bf16*)g.aux_in;
     if (g.epilogue == BB_EPI_RESIDUAL) return (const bf16*)g.resid;
     return nullptr;
@@ -676,7 +676,7 @@ template <int BR, int T, bool KM, int BK = 32> struct FragReader {
 // the epilogue also leaves that normalisation's backward sums per strip (BnBwdArgs), so that its backward pass has no
 // reduction over the tensor left.
 template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, int BK = 32, bool VIS = false, int CONV = 0,
-          int STATS = 0, bool DROP = false, bool RAGK = false, bool READ_AHEAD = true>
+          int STATS = 0, bool DROP = false, bool RAGK = false>
 __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int block_id, const int batch_id,
                                                    const bool logical_id = false, const ConvArgs& cv = ConvArgs{},
                                                    const BnBwdArgs& bn = BnBwdArgs{}) {
@@ -761,8 +761,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // add up the A fragments they hold anyway: lane (m, kg) sees 8 of the 16 k values per step
     const bool do_colsum = AKM && g.colsum != nullptr && tile_n == 0 && wn == 0;
     // the main loop of the smaller tiles, see there
-    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS &&
-                           READ_AHEAD;
+    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS;
     float csum[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) csum[i] = 0.f;
@@ -1252,15 +1251,15 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
 
 // DROP: the epilogue can apply dropout (g.drop).  A kernel of its own, so that the keep decisions' registers cost the
 // kernels without dropout nothing (they decide how many blocks of the small tiles a CU holds).  RAGK: contractions of any
-// length, likewise.  READ_AHEAD = false: the small tiles on the main loop of the larger ones (see read_ahead).
-template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, int BK, bool DROP = false, bool RAGK = false, bool READ_AHEAD = true>
+// length, likewise.
+template <int BM, int BN, int WM, int WN, bool AKM, bool BKM, bool DB, int STAGES, int BK, bool DROP = false, bool RAGK = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, 0, 0, DROP, RAGK, READ_AHEAD>(g, blockIdx.x, blockIdx.z);
+    gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, 0, 0, DROP, RAGK>(g, blockIdx.x, blockIdx.z);
 }
 // the same with the strip statistics of the output (NT, 64-wide k-tiles)
-template <int BM, int BN, int WM, int WN, int STAGES, bool READ_AHEAD>
+template <int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_stats_kernel(const GemmArgs g) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, false, false, true, STAGES, 64, false, 0, 1, false, false, READ_AHEAD>(g, blockIdx.x, blockIdx.z);
+    gemm_bf16_dma_body<BM, BN, WM, WN, false, false, true, STAGES, 64, false, 0, 1>(g, blockIdx.x, blockIdx.z);
 }
 // input gradient of a 1x1 convolution (NN, 64-wide k-tiles) with the backward sums of the batch normalisation in front of it
 template <int BM, int BN, int WM, int WN, int STAGES>

@@ -360,54 +360,3 @@ def test_f32_weight_gradients_on_quarter_tiles(hiplib, rows, shapes):
     for (a, b), c in zip(ops, outs[0]):
         prod, terms = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
         assert bool(((c.double() - 1 - prod).abs() <= (rows + 4) * 2.0 ** -24 * (terms + 1)).all())
-
-
-# 128x64 and 64x128 tiles have two main loops, chosen by the tiles, the contraction and what the epilogue reads: either side of each
-# limit (170 and 330 tiles of the 256; K of 384 / 448) against the other and against fp64, ragged rows and columns.
-@pytest.mark.parametrize("layout", ["nt", "nn"])
-@pytest.mark.parametrize("K", [128, 192, 384, 448, 576])
-def test_both_loops_of_half_tiles(hiplib, K, layout):
-    lay, N = getattr(hiplib, layout.upper()), 616
-    few, many = 2050, 4200
-    A, B = rand(many, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2, scale=0.2)
-    bias, X, R = rand(N, seed=3), rand(many, N, seed=4), rand(many, N, seed=5)
-    for m in (few, many):
-        assert hiplib.gemm_variant(hiplib.gemm_desc(lay, A[:m], B, X[:m])).endswith("dma128x64k64s3" if layout == "nt" else "dma64x128k64s3")
-    cases = [dict(bias=bias), dict(bias=bias, epilogue=hiplib.EPI_RESIDUAL), dict(epilogue=hiplib.EPI_MUL_POS),
-             dict(bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_GELU_TANH)]
-    if layout == "nt":
-        cases += [dict(bias=bias, dropout=(0.1, (7, 9))), dict(bias=bias, epilogue=hiplib.EPI_RESIDUAL, dropout=(0.1, (7, 9)))]
-    for kw in cases:
-        out = []
-        for m in (few, many):
-            C, aux = torch.full((m, N), float("nan"), dtype=torch.bfloat16, device=DEV), X[:m].clone()
-            extra = {hiplib.EPI_RESIDUAL: dict(resid=aux), hiplib.EPI_MUL_POS: dict(aux_in=aux, resid=R[:m]), hiplib.EPI_ACT_DACT: dict(aux_out=aux)}
-            hiplib.gemm(lay, A[:m], B, C, **kw, **extra.get(kw.get("epilogue"), {}))
-            out.append((C, aux))
-        assert torch.equal(out[0][0], out[1][0][:few]) and torch.equal(out[0][1], out[1][1][:few]), kw
-        if list(kw) == ["bias"]:
-            prod = A.double().cpu() @ (B.double().cpu().t() if layout == "nt" else B.double().cpu()) + bias.double().cpu()
-            assert rel(out[1][0], prod) < 2.0 ** -8      # half an ulp of bf16, and the sums' K eps
-
-
-# ... with the strip statistics, whose loops part at 256 columns of contraction; BatchNorm backward sums beside them
-@pytest.mark.parametrize("K", [128, 192, 256, 512, 640])
-def test_both_loops_leave_the_same_strips(hiplib, K):
-    N, few, many = 640, 2048, 4224
-    A, B, Bk = rand(many, K, seed=1), rand(N, K, seed=2, scale=0.2), rand(K, N, seed=3, scale=0.2)
-    X, Y, R = rand(many, N, seed=4), rand(many, N, seed=5), rand(many, N, seed=6)
-    mean, rstd = torch.randn(N, generator=torch.Generator().manual_seed(7)).to(DEV), torch.full((N,), 0.7, device=DEV)
-    runs = [[] for _ in range(4)]
-    for m in (few, many):
-        C, strips = torch.full((m, N), float("nan"), dtype=torch.bfloat16, device=DEV), torch.full((hiplib.strip_stats_workspace(m, N),), float("nan"), device=DEV)
-        hiplib.gemm(hiplib.NT, A[:m], B, C, strip_stats=strips)
-        runs[0].append((C[:few], strips[: hiplib.strip_stats_workspace(few, N)]))
-        for run, (relu_out, skip) in zip(runs[1:], ((None, None), (X, None), (X, R))):
-            C, strips = torch.full_like(C, float("nan")), torch.full((hiplib.bn_bwd_strips_workspace(m, N),), float("nan"), device=DEV)
-            hiplib.gemm_bn_bwd(A[:m], Bk, C, relu_out if relu_out is None else relu_out[:m], Y[:m], mean, rstd, strips, resid=skip if skip is None else skip[:m])
-            run.append((C[:few], strips[: hiplib.bn_bwd_strips_workspace(few, N)]))
-    for (c0, s0), (c1, s1) in runs:
-        assert torch.equal(c0, c1) and torch.equal(s0, s1) and bool(torch.isfinite(s0).all())
-    want = A.double().cpu() @ Bk.double().cpu()
-    assert rel(runs[1][1][0], want[:few]) < 2.0 ** -8
-    assert rel(runs[0][1][0], (A.double().cpu() @ B.double().cpu().t())[:few]) < 2.0 ** -8
