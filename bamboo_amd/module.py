@@ -13,7 +13,6 @@ import math
 import os
 import re
 from collections import OrderedDict
-from operator import attrgetter
 
 import torch
 
@@ -592,16 +591,22 @@ class PipelineModule:
 
     def pass_state(self, stage_id, layers):
         """What the launches of a pass over the layers a..b-1 depend on beside its operands: every object by itself, to be
-        compared by identity (a value inside a dict that a layer holds counts, one further down does not)."""
-        own, cls = self.__dict__, None
-        out = [self.base_seed, self.activation_checkpoint_interval, self._stash.get(stage_id), own.get("_kept", _EMPTY).get(stage_id),
-               own.get("stage_seq", _EMPTY).get(stage_id), own.get("forward"), own.get("backward"), own.get("_forward_into"), own.get("_rebuild"),
-               *_PASSES_OF(type(self))]
+        compared by identity (a value inside a dict that a layer holds counts, one further down does not).  Methods: those that
+        a pass of these layers calls; this is host work of every pass."""
+        own, kind, cls, ckpt = self.__dict__, type(self), None, self.activation_checkpoint_interval
+        out = [self.base_seed, ckpt, self._stash.get(stage_id), own.get("_kept", _EMPTY).get(stage_id),
+               own.get("stage_seq", _EMPTY).get(stage_id), own.get("forward"), own.get("backward"), kind.forward, kind.backward]
+        if ckpt:
+            out += (own.get("_forward_into"), own.get("_rebuild"), kind._forward_into, kind._rebuild)
         a, b = layers
         for layer in self.func_buckets[stage_id][a:b]:
             if type(layer) is not cls:     # (once where neighbours are of one class)
                 cls = type(layer)
-                out += (cls.forward, cls.backward, getattr(cls, "rebuild", None), getattr(cls, "grad_sink", None))   # PASS_METHODS
+                out += (cls.forward, cls.backward)
+                if ckpt:
+                    out.append(getattr(cls, "rebuild", None))
+                if b - a > 1:
+                    out.append(getattr(cls, "grad_sink", None))
             own = layer.__dict__.values()
             out.append(layer)
             out += own
@@ -698,5 +703,4 @@ class PipelineModule:
 
 # the methods a pass is made of, as they are here
 _PASSES = {m: getattr(PipelineModule, m) for m in ("forward", "backward", "_forward_into", "_rebuild")}
-_PASSES_OF = attrgetter(*_PASSES)
 _EMPTY = {}

@@ -20,7 +20,7 @@ _HARMLESS = {"__init__", "__repr__", "__module__", "__qualname__", "__doc__", "_
              "__orig_bases__", "init_params", "num_params", "flops_fwd"}
 
 
-# what a pass of a stage calls on a layer (the state of a stage lists them one by one: PipelineModule.pass_state)
+# what passes call on a layer (PipelineModule.pass_state has those of a given pass)
 PASS_METHODS = ("forward", "backward", "rebuild", "grad_sink")
 
 

@@ -295,35 +295,49 @@ class Rebuilt(Layer):
         pass
 
 
+def checkpointed(stage, monkeypatch):
+    """The stage's passes as one checkpoint group: with the methods that only such passes call."""
+    kept = torch.zeros(2, ROWS, COLS)
+    monkeypatch.setattr(hip, "cast", lambda src, dst, stream=None: dst.copy_(src))
+    stage.module.__dict__.update(activation_checkpoint_interval=len(stage.module.func_buckets[1]), _kept={1: [list(kept)]})
+    stage.module._stash_arena[(1, "kept")] = kept
+
+
 @pytest.mark.parametrize("method", replay.PASS_METHODS)
 def test_a_method_of_a_pass_replaced_in_its_class_is_seen(stage, monkeypatch, method):
     """By one of the class's own module: recorded anew.  By another's: its Python code runs in every pass."""
-    stage.module.func_buckets[1] = [Rebuilt(COLS)]
+    stage.module.func_buckets[1], n = [Rebuilt(COLS), Rebuilt(COLS)], 2
+    stage.module._stash[1][0].append({"out": torch.zeros(ROWS, COLS)})
+    stage.module.stage_seq[1].append(ROWS)
+    if method == "rebuild":
+        checkpointed(stage, monkeypatch)
     x, inner = torch.randn(ROWS, COLS), getattr(Rebuilt, method)
     stage.forward(x)
     stage.forward(x)
-    assert (stage.issued(), stage.replayed()) == (1, 1)
+    assert (stage.issued(), stage.replayed()) == (n, 1)
 
     def other(self, *a):
         return inner(self, *a)
     monkeypatch.setattr(Rebuilt, method, other)
     for replayed in (1, 2):
         stage.forward(x)
-        assert (stage.issued(), stage.replayed()) == (2, replayed)
+        assert (stage.issued(), stage.replayed()) == (2 * n, replayed)
 
     def wrapped(self, *a):
         return inner(self, *a)
     wrapped.__module__ = "elsewhere"
     monkeypatch.setattr(Rebuilt, method, wrapped)
-    for issued in (3, 4):
+    for passes in (3, 4):
         stage.forward(x)
-        assert (stage.issued(), stage.replayed()) == (issued, 2)
+        assert (stage.issued(), stage.replayed()) == (passes * n, 2)
 
 
 @pytest.mark.parametrize("method", ["forward", "backward", "_forward_into", "_rebuild"])
 @pytest.mark.parametrize("where", ["class", "object"])
 def test_a_method_a_pass_is_made_of_replaced_in_the_module_is_seen(stage, monkeypatch, method, where):
     x = torch.randn(ROWS, COLS)
+    if method.startswith("_"):
+        checkpointed(stage, monkeypatch)
     stage.forward(x)
     stage.forward(x)
     assert (stage.issued(), stage.replayed()) == (1, 1)
