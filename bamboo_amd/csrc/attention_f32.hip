@@ -67,7 +67,10 @@ __device__ __forceinline__ int f32_sample_len(const AttnF32Args& a, int b) {
 }
 // Rows of a matrix, read through a buffer descriptor: a lane's offset in a vector register, the row in a scalar one, so that a
 // load costs the matrix cores no vector instruction, and what lies past the last row reads as zero.  No load stands behind a
-// branch: at a merge the compiler would wait for all that are in flight.
+// branch: at a merge the compiler would wait for all that are in flight.  The kernels count on the zeros (a ragged sequence is read
+// up to 31 rows past its end), and with that on the range check of a raw buffer taking the scalar offset in, also where that
+// alone lies beyond the end.  So it does on gfx950: of a range of 1000 bytes inside a larger allocation, all 3509 words past it read
+// as zero, 3392 of them under a scalar offset beyond it (step 100 bytes, up to 6300).
 struct Rows {
     __amdgpu_buffer_rsrc_t desc;
     unsigned ld;   // bytes

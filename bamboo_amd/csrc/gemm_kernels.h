@@ -430,8 +430,10 @@ __device__ __forceinline__ void dma16_at(const void* src, unsigned lds) {
 }
 
 // the same by no lane or by all of them (live: 0 or -1): a masked-off transfer moves nothing, but is counted like any other, so
-// that a loop may issue -- and wait for -- the same number of them whether there is something left to load or not.  The
-// callers' waves are full.
+// that a loop may issue -- and wait for -- the same number of them whether there is something left to load or not.  (vmcnt counts
+// vector memory instructions as they issue, whatever EXEC holds; compiled code relies on that where a short branch is not worth a
+// jump.  Seen on an MI355X: behind one transfer of a cold line and eight masked ones, s_waitcnt vmcnt(8) found the line landed in all
+// of 262144 words, vmcnt(9), which does not wait for it, missed 13948.)  The callers' waves are full.
 __device__ __forceinline__ void dma16_masked(const void* src, unsigned lds, int live) {
     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(live) : "m0");
 }

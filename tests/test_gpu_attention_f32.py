@@ -95,3 +95,26 @@ def test_kept_probabilities(hiplib, mask, b, a, s, d, p):
         err = float((t - w).double().norm()) / max(float(w.double().norm()), floor if name[0] == "d" else 0.0)
         assert err < 2 * tol, (name, err, tol)
     assert torch.equal(got[0][0] == 0, got[1][0] == 0)      # the masked probabilities, exactly
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask", ["none", "causal", "key_padding"])
+@pytest.mark.parametrize("b,a,s,d", [(1, 1, 4, 32), (2, 2, 36, 64), (1, 3, 100, 128), (2, 1, 132, 64)])
+def test_nothing_past_the_end_is_taken_in(hiplib, mask, b, a, s, d):
+    """A ragged sequence is read in whole tiles: what lies behind the operands, of a sample or of all of them, reads as zero.  With
+    NaN there, and without: the same bits."""
+    h, n = a * d, b * s
+    g = torch.Generator(device=DEV).manual_seed(s)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    qkv, d_ctx = rand(n, 3 * h), rand(n, h)
+    lens = torch.tensor([s - 1, s][:b], dtype=torch.int32, device=DEV) if mask == "key_padding" else None
+    runs = []
+    for behind in (0.0, float("nan")):
+        pad = lambda t: torch.cat([t.reshape(-1), torch.full((64 * t.shape[-1],), behind, device=DEV)])[: t.numel()].view(t.shape)
+        new = lambda *shape: pad(torch.full(shape, float("nan"), device=DEV))
+        q, dc, out, prob, d_score, d_qkv = pad(qkv), pad(d_ctx), new(n, h), new(b, a, s, s), new(b, a, s, s), new(n, 3 * h)
+        hip.attention_probs_fwd(q, out, prob, b, a, s, hip.MASK_CODES[mask], lens)
+        hip.attention_probs_bwd(q, dc, prob, d_score, d_qkv, b, a, s, hip.MASK_CODES[mask], lens)
+        runs.append((out, prob, d_qkv))
+    for x, y in zip(*runs):
+        assert bool(torch.isfinite(x).all()) and torch.equal(x, y)
