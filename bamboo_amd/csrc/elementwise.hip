@@ -1283,26 +1283,26 @@ __global__ __launch_bounds__(256) void bn_finish_kernel(int what, int rows, int 
     }
 }
 
-// Forward BatchNorm from the strip triples a convolution's GEMM epilogue leaves (per 32 rows and channel: pivot p,
-// S1 = sum (x - p), S2 = sum (x - p)^2), statistics and normalisation in ONE launch.  A block owns a slab of channels and
-// one of the row ranges.  Every block first turns the strips of its channels into mean and variance -- a
-// strip's mean is p + S1/n and its sum of squared deviations M2 = S2 - S1^2/n (no cancellation: p is a sample of the
-// strip); two passes over the triples, which stay in registers (at most 8192 rows): mean = sum n_s mean_s / rows,
-// then sum (M2_s + n_s (mean_s - mean)^2) -- lane = channel, sixteen groups of threads taking strips w,
-// w + 16, ..., the sixteen partial sums added in that order by every thread (a fixed order, the same in every
-// block: all row ranges of a channel normalise with the same bits).  The block of the first row range also writes
-// mean, rstd and the running statistics.  Then y = gamma (x - mean) rstd + beta (+ resid) (ReLU) over the block's
-// rows, eight channels a lane.  The tensor is read once, but every block reads all
-// strips of its channels: at 6272 rows 150 KB a block of 64, 38.5 MB a launch of 256 blocks, out of L2 -- 12 times the tensor at 256
-// columns (half that with 32), 3 times at 1024 (L1's read requests with 64: 41.9 and 51.5 MB in all).  What it was taken against is a launch of its own for
-// the statistics (5.4 + 5.5 us against 7.9 at 6272 x 256).  (For few rows the reduction is what the launch waits for: loads for all 256 strips / for the sixteens there are, us, on 64 channels a block: 900 rows x 512
-// 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 / 6.5; the rows of a thread fetched ahead, all of them or the next one, gained nothing.)
+// Forward BatchNorm from the strip triples a convolution's GEMM epilogue leaves (per 32 rows and channel: pivot p, S1 = sum (x -
+// p), S2 = sum (x - p)^2), statistics and normalisation in ONE launch.  A block owns a slab of channels and one of the row
+// ranges.  Every block first turns the strips of its channels into mean and variance -- a strip's mean is p + S1/n and its sum of
+// squared deviations M2 = S2 - S1^2/n (no cancellation: p is a sample of the strip); two passes over the triples, which stay in
+// registers (at most 8192 rows): mean = sum n_s mean_s / rows, then sum (M2_s + n_s (mean_s - mean)^2) -- lane = channel, sixteen
+// groups of threads taking strips w, w + 16, ..., the sixteen partial sums added in that order by every thread (a fixed order,
+// the same in every block: all row ranges of a channel normalise with the same bits).  The block of the first row range also
+// writes mean, rstd and the running statistics.  Then y = gamma (x - mean) rstd + beta (+ resid) (ReLU) over the block's rows,
+// eight channels a lane.  The tensor is read once, but every block reads all strips of its channels: at 6272 rows 150 KB a block
+// of 64, 38.5 MB a launch of 256 blocks, out of L2 -- 12 times the tensor at 256 columns (half that with 32), 3 times at 1024
+// (L1's read requests with 64: 41.9 and 51.5 MB in all).  What it was taken against is a launch of its own for the statistics
+// (5.4 + 5.5 us against 7.9 at 6272 x 256).  (For few rows the reduction is what the launch waits for: loads for all 256 strips /
+// for the sixteens there are, us, on 64 channels a block: 900 rows x 512 6.6 / 5.35, 3136 x 1024 7.85 / 7.05, 6272 x 256 6.9 /
+// 6.5; the rows of a thread fetched ahead, all of them or the next one, gained nothing.)
 //
-// A slab is 32 channels, each of the sixteen shares a group of 32 threads: with 64 a launch of as many blocks reads twice as much of
-// the strips.  64 channels / 32 / and the strips' counts without a division each (us): 6272 x 256 6.6 / 5.6 / 5.15, 3136 x 1024 6.9 /
-// 6.4 / 5.9, 900 x 512 5.3 / 4.6 / 4.2, 200 x 64 5.0 / 4.4 / 3.9, 6272 x 1024 8.6 / 7.8 / 7.4, with a residual 9.9 / 9.5 / 9.3.  (All slabs of a row
-// range on one XCD, which then reads every strip: 9.7 and 11.9.  The backward twin, which reads two tensors and fewer strips,
-// gains nothing by it: 4.3 / 4.4 at 6272 x 256, 7.8 / 8.6 x 1024.)
+// A slab is 32 channels, each of the sixteen shares a group of 32 threads: with 64 a launch of as many blocks reads twice as much
+// of the strips.  64 channels / 32 / and the strips' counts without a division each (us): 6272 x 256 6.6 / 5.6 / 5.15, 3136 x
+// 1024 6.9 / 6.4 / 5.9, 900 x 512 5.3 / 4.6 / 4.2, 200 x 64 5.0 / 4.4 / 3.9, 6272 x 1024 8.6 / 7.8 / 7.4, with a residual 9.9 /
+// 9.5 / 9.3.  (All slabs of a row range on one XCD, which then reads every strip: 9.7 and 11.9.  The backward twin, which reads
+// two tensors and fewer strips, gains nothing by it: 4.3 / 4.4 at 6272 x 256, 7.8 / 8.6 x 1024.)
 constexpr int BN_STRIP_GROUPS = 16, BN_STRIP_MAX = 16;   // 16 * 16 strips = up to 8192 rows
 constexpr int BN_SLAB = 32, BN_STRIP_THREADS = BN_STRIP_GROUPS * BN_SLAB;
 // about one block per CU; wide tensors get fewer row ranges (each repeats the strip reduction of its channels)
@@ -1684,7 +1684,6 @@ extern "C" int bb_batchnorm_fwd_strips(int dtype, int rows, int cols, float eps,
     BB_REQUIRE(rows <= 32 * BN_STRIP_GROUPS * BN_STRIP_MAX, "bb_batchnorm_fwd_strips: at most %d rows", 32 * BN_STRIP_GROUPS * BN_STRIP_MAX);
     BB_REQUIRE((running_mean == nullptr) == (running_var == nullptr), "bb_batchnorm_fwd_strips: give both running buffers or none");
     hipStream_t st = (hipStream_t)stream;
-    // about one block per CU; wide tensors get fewer row ranges (each repeats the strip reduction of its channels)
     const int ranges = bn_row_ranges(cols);
     bb_launch(bn_fwd_strips_kernel, dim3(bn_strip_blocks(cols)), dim3(BN_STRIP_THREADS), 0, st, rows, cols, ranges, eps, momentum, relu,
                        strip_stats, (const bf16*)x, (const bf16*)gamma, (const bf16*)beta, (const bf16*)resid, (bf16*)y, mean, rstd,

@@ -133,15 +133,24 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches;
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
-    //  - Problems of at most one tile of 128x64 per CU (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle) take those,
-    //    short contractions also up to 400, very short ones up to 512, whose chains run under each other; then 128x128 tiles of three stages, one per CU, up to
-    //    a round of them.  128x64 / 128x128 (64x128 / 128x128), plain and with a residual (us): NT 1200x1600x1600 (250 tiles of
-    //    128x64) 12.3 12.9 / 15.1 16.8, 2300x1024x1024 (288) 12.2 12.8 / 11.7 12.9, 4096x768x768 (384) 10.8 11.3 / 10.4 11.4, x3072 30.2
-    //    30.8 / 25.1 26.5, 3136x1024x256 (400) 7.4 8.1 / 7.8 8.7, 6272x512x128 (392) 6.7 7.4 / 7.1 8.0, 8112x512x128 (512) 6.8 / 7.8; NN 12.1 12.7 / 15.1 16.5, 12.2 12.9 /
-    //    11.8 13.1, 10.9 11.5 / 10.7 11.5, 30.4 30.6 / 25.3 26.7, 7.4 8.2 / 7.9 8.8.  A round of 128x128 with two stages or 32-wide k-tiles
-    //    (two and three blocks per CU) / this: NT 8192x512x512 10.7 11.9 / 9.6 10.5, x2048 26.2 28.9 / 21.1 22.4, NN 10.2 11.5 / 9.8 10.6,
-    //    26.2 28.9 / 21.4 22.4; 256x128 / this where a few rows stand against many columns: 640x6400x1600 24.1 25.6 / 17.3 19.0.  More
-    //    of them: 256x128 tiles, also for short contractions (NT 6272x1024x256 12.8 14.0 on 128x64, 10.3 11.4 on 256x128).
+    //  - Problems of at most one tile of 128x64 per CU (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle)
+    //    take those, short contractions also up to 400, very short ones up to 512, whose chains run under each other; then
+    //    128x128 tiles of three stages, one per CU, up to a round of them.  128x64 / 128x128 (64x128 / 128x128), plain and
+    //    with a residual (us): NT 1200x1600x1600 (250 tiles of 128x64) 12.3 12.9 / 15.1 16.8, 2300x1024x1024 (288) 12.2 12.8
+    //    / 11.7 12.9, 4096x768x768 (384) 10.8 11.3 / 10.4 11.4, x3072 30.2 30.8 / 25.1 26.5, 3136x1024x256 (400) 7.4 8.1 /
+    //    7.8 8.7, 6272x512x128 (392) 6.7 7.4 / 7.1 8.0, 8112x512x128 (512) 6.8 / 7.8; NN 12.1 12.7 / 15.1 16.5, 12.2 12.9 /
+    //    11.8 13.1, 10.9 11.5 / 10.7 11.5, 30.4 30.6 / 25.3 26.7, 7.4 8.2 / 7.9 8.8.  A round of 128x128 with two stages or
+    //    32-wide k-tiles (two and three blocks per CU) / this: NT 8192x512x512 10.7 11.9 / 9.6 10.5, x2048 26.2 28.9 / 21.1
+    //    22.4, NN 10.2 11.5 / 9.8 10.6, 26.2 28.9 / 21.4 22.4; 256x128 / this where a few rows stand against many columns:
+    //    640x6400x1600 24.1 25.6 / 17.3 19.0.  More of them: 256x128 tiles, also for short contractions (NT 6272x1024x256
+    //    12.8 14.0 on 128x64, 10.3 11.4 on 256x128).
+    //    (Their loop reads a k-tile ahead, which alone is not the faster way for all of them: with no operand for the epilogue
+    //    to fetch and blocks that share a CU, or few k-tiles, the loop of the larger tiles / this is (us) NT 12168x512x128 9.7 /
+    //    10.3, 25088x512x128 17.2 / 18.5, 3136x1024x256 7.4 / 7.9, 12168x256x512 9.3 / 9.6, but 12168x128x512 6.8 / 6.7, and with a
+    //    residual from memory 12168x512x128 16.5 / 13.1.  Split by such a rule no stage gained: 18 images of 26x26, 128 channels
+    //    (us, this / split) 2841 / 2846, 32 of 28x28, 64 channels 3213 / 3220, 384-wide encoders over 3066 rows 3060 / 3081,
+    //    512-wide over 2048 2818 / 2795.  In the third the products that stayed on this loop went from 9.9 to 10.7 us, with the
+    //    same code, as if it had to be fetched again where two kernels alternate.)
     //    32-wide k-tiles (K % 64 != 0) as before: 128x64 tiles up to 128 tiles of 128x128 and for short forward contractions.
     if (k64) {
         const int64_t halves = nt ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
@@ -291,12 +300,13 @@ static constexpr int kF32SplitGroups = 2, kF32SplitBN = 32;
 static bool pick_f32_split(int M, int N, int K, int64_t batches, int layout) {
     return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches < 2 * 256 && K >= 512;
 }
-// Of what is left for the tiles of 64x64 and 64x32, problems of at most 128 64x64 tiles take four blocks a tile instead, with the same
-// bits (gemm_f32_quarter_kernel): until then every CU has at most two of them.  Larger tiles / this (us, back to back): NT
+// Of what is left for the tiles of 64x64 and 64x32, problems of at most 128 64x64 tiles take four blocks a tile instead, with the
+// same bits (gemm_f32_quarter_kernel): until then every CU has at most two of them.  Larger tiles / this (us, back to back): NT
 // 128x128x128 7.0 / 5.2, 512x512x256 (64 tiles) 10.7 / 5.8, 1000x448x448 (112) 16.3 / 10.2, 1024x512x512 (128) 11.2 / 11.4,
-// 1024x512x2048 32.3 / 29.9, 512x1536x256 (192) 11.4 / 11.2, 1000x1344x448 (336) 25.1 / 26.8, 2048x768x768 (384) 29.0 / 37.9; NN alike.  TN: 64x64x4096 85 / 41, 512x512x2048 45 / 24, 512x1024x1000 (128)
-// 25.2 / 18.3; the weight gradients of a layer together, hidden size (x 4 in the feed-forward) and rows: 128 (48 tiles) 7680 159 / 80, 200 10.7 /
-// 7.5; 192 (108) 3000 67 / 46; 256 (192) 1072 29.4 / 31.2, 320 (300) 600 28.2 / 31.6; ResNet blocks of 64 channels (17) 6272 pixels 131 / 65.
+// 1024x512x2048 32.3 / 29.9, 512x1536x256 (192) 11.4 / 11.2, 1000x1344x448 (336) 25.1 / 26.8, 2048x768x768 (384) 29.0 / 37.9; NN
+// alike.  TN: 64x64x4096 85 / 41, 512x512x2048 45 / 24, 512x1024x1000 (128) 25.2 / 18.3; the weight gradients of a layer
+// together, hidden size (x 4 in the feed-forward) and rows: 128 (48 tiles) 7680 159 / 80, 200 10.7 / 7.5; 192 (108) 3000 67 / 46;
+// 256 (192) 1072 29.4 / 31.2, 320 (300) 600 28.2 / 31.6; ResNet blocks of 64 channels (17) 6272 pixels 131 / 65.
 static constexpr int kF32QuarterTiles = 128;
 static bool pick_f32_quarter(int M, int N, int64_t batches) { return (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches <= kF32QuarterTiles; }
 template <bool TA, bool TB, int KG> static int launch_f32_quarter(GemmArgs& g, int batches, hipStream_t st) {

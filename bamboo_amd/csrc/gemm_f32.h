@@ -115,10 +115,10 @@ template <bool KM, int NC> struct F32Reader {
 constexpr int f32_stages(int bn) { return bn == 64 ? 2 : 3; }
 constexpr int f32_gemm_lds(int bn) { return f32_stages(bn) * (64 + bn) * 128; }
 
-// The epilogue of a lane's NR elements -- sixteen, or four of a tile that several waves finish -- (one column; register r: row m + 8 (r / 4) + r % 4).  `pre`: what it reads beside
-// the product -- the operand of the epilogue kind, else the C it accumulates into -- fetched before the main loop; `rest`: a
-// problem that reads both, or a masked residual, fetches the second here.  One branch over the kind around them, not
-// inside: the code stays small.
+// The epilogue of a lane's NR elements -- sixteen, or four of a tile that several waves finish -- (one column; register r: row m
+// + STEP (r / 4) + r % 4).  `pre`: what it reads beside the product -- the operand of the epilogue kind, else the C it accumulates
+// into -- fetched before the main loop; `rest`: a problem that reads both, or a masked residual, fetches the second here.  One
+// branch over the kind around them, not inside: the code stays small.
 template <int NR, int STEP = 8, typename V>
 __device__ __forceinline__ void epilogue_f32(const GemmArgs& g, int64_t coff, int m0, int n, float bias, const float (&pre)[NR], V& v) {
     const auto row = [&](int r) { return m0 + STEP * (r >> 2) + (r & 3); };
@@ -437,10 +437,11 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_wave_grouped_kernel(const Gro
     gemm_f32_wave_body<TA, TB>(G.p[pi], lid - G.first_block[pi], 0, true);
 }
 
-// Problems of few 64x64 tiles: each tile as four blocks of 32x32, a wave 16x16 of it by v_mfma_f32_16x16x4_f32.  What bounds such a
-// problem is the chain of one tile: a 64x64 tile's wave spends 32 matrix cycles on every k, this one 8 on four times the CUs, and
-// four k-tiles of 64 are in flight from the start (us against the larger tiles: see pick_f32_quarter).  Both instructions add their k one by one, ascending (checked bit for bit against
-// a chain of multiply-adds), so the result has the bits of the larger tile: which kernel runs a product changes none of them.
+// Problems of few 64x64 tiles: each tile as four blocks of 32x32, a wave 16x16 of it by v_mfma_f32_16x16x4_f32.  What bounds such
+// a problem is the chain of one tile: a 64x64 tile's wave spends 32 matrix cycles on every k, this one 8 on four times the CUs,
+// and four k-tiles of 64 are in flight from the start (us against the larger tiles: see pick_f32_quarter).  Both instructions add
+// their k one by one, ascending (checked bit for bit against a chain of multiply-adds), so the result has the bits of the larger
+// tile: which kernel runs a product changes none of them.
 // KG: groups of four waves that share the contraction as those of the 64x32 tiles do (16-wide halves of every 32, added in order).
 constexpr int kF32QuarterStages = 4;
 constexpr int kF32QuarterLds = kF32QuarterStages * 2 * 2 * 32 * 128;

@@ -267,9 +267,9 @@ int bb_attention_bwd(int dtype, int mask, int batch, int heads, int seq, int hea
                      int64_t ld_dqkv, const int32_t* key_len, float dropout_p, uint32_t dropout_k0, uint32_t dropout_k1, void* stream);
 
 /* The same attention with the probabilities kept (fp32; head_dim 32, 64 or 128, seq a multiple of 4 and at most 1024;
- * bb_attention_probs_supported: and this is the faster way).  prob: [batch, heads, seq, seq], written in full by the forward, in front of dropout; the
- * backward reads it and leaves the gradient of the scaled scores in d_score (same size; key tiles that the mask rules out for
- * all of a 32-query block are not written).  Masked scores are replaced by -1e9 before the softmax; what the rows of such
+ * bb_attention_probs_supported: and this is the faster way).  prob: [batch, heads, seq, seq], written in full by the forward,
+ * in front of dropout; the backward reads it and leaves the gradient of the scaled scores in d_score (same size; key tiles
+ * that the mask rules out for all of a 32-query block are not written).  Masked scores are replaced by -1e9 before the softmax; what the rows of such
  * keys hold beyond the last 32-wide tile some query of a block may see is not read.                             */
 int bb_attention_probs_supported(int dtype, int batch, int heads, int seq, int head_dim);
 int bb_attention_probs_fwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k,
