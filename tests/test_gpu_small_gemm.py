@@ -210,13 +210,15 @@ def test_fp32_rows_of_any_pitch(hiplib, layout, M, N, K, ld):
 
 # Products of few tiles against the same rows inside a product of many, which the larger tiles run: the same bits.  Contractions of
 # a part of a k-tile, around 64, around the four stages of the ring, and long ones that two groups share; rows and columns of
-# less than a tile, with remainders, and the most tiles the rule takes (128).
-@pytest.mark.parametrize("M,N,K", [(4, 4, 4), (32, 36, 60), (33, 64, 64), (70, 100, 68), (128, 128, 252), (100, 72, 256), (64, 260, 260), (512, 900, 320),
-                                   (36, 28, 512), (70, 132, 524), (130, 64, 580), (1024, 512, 1036)])
-@pytest.mark.parametrize("layout", ["nt", "nn"])
+# less than a tile, with remainders, and the most tiles the rule takes (128).  (NN with at most 128 columns of contraction is the
+# 32x32 wave tiles': test_fp32_products_of_few_tiles.  Its shortest here fill three of the ring's four stages.)
+QUARTER = [(4, 4, 4), (32, 36, 60), (33, 64, 64), (70, 100, 68), (128, 128, 252), (100, 72, 256), (64, 260, 260), (512, 900, 320),
+           (36, 28, 512), (70, 132, 524), (130, 64, 580), (1024, 512, 1036)]
+
+
+@pytest.mark.parametrize("layout,M,N,K", [("nt", *s) for s in QUARTER] + [("nn", *s) for s in QUARTER if s[2] > 128] +
+                         [("nn", 4, 4, 132), ("nn", 33, 64, 188), ("nn", 70, 100, 192), ("nn", 32, 36, 196)])
 def test_fp32_quarter_tiles_have_the_bits_of_whole_ones(hiplib, layout, M, N, K):
-    if layout == "nn" and K <= 128:
-        pytest.skip("32x32 tiles with a slice a wave")
     lay = hiplib.NT if layout == "nt" else hiplib.NN
     mk = lambda *shape, seed: torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
     rows = max(M, 64 * (130 * 64 // N + 1))     # more than 128 tiles, fewer than the 512 from which on no contraction is shared
