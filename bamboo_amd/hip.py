@@ -721,7 +721,10 @@ class Plan:
             raise HipKernelError(f"plan: {n} operands expected, got {len(tensors)}")
         for i, t in enumerate(tensors):
             self._addresses[i] = t.data_ptr()
-        check(lib().bb_plan_launch_on(self._plan, n, self._addresses if n else None, step, stream_ptr(stream)), "bb_plan_launch_on")
+        rc = lib().bb_plan_launch_on(self._plan, n, self._addresses if n else None, step,
+                                     (torch.cuda.current_stream() if stream is None else stream).cuda_stream)
+        if rc:
+            check(rc, "bb_plan_launch_on")
 
     def __len__(self):
         return int(lib().bb_plan_launches(self._plan))

@@ -62,6 +62,9 @@ def _apart(ranges, others):
     return True
 
 
+_NONE = {}
+
+
 class Replay:
     VARIANTS = 4     # forms remembered per (kind, stage, micro-batch)
 
@@ -117,7 +120,7 @@ class Replay:
             return issue()
         key = (ctx, variant) + tuple(map(form, operands))
         given = [t for t in operands if t is not None]
-        known = self.plans.get(slot, {}).get(key)
+        known = self.plans.get(slot, _NONE).get(key)
         if known is not None:
             plan, at, out = known
             plan.launch(step, ctx.stream, given)
