@@ -60,10 +60,10 @@ template <int BM, int BN, int WM, int WN, bool TB> static int launch_bf16_dma_pe
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES = 3>
+template <int BM, int BN, int WM, int WN, int STAGES = 3, bool WIDE = false>
 static int launch_bf16_dma_stats(GemmArgs& g, hipStream_t st) {
     constexpr int smem = STAGES * (BM + BN) * 64 * 2;
-    auto kern = gemm_bf16_dma_stats_kernel<BM, BN, WM, WN, STAGES>;
+    auto kern = gemm_bf16_dma_stats_kernel<BM, BN, WM, WN, STAGES, WIDE>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -72,10 +72,10 @@ static int launch_bf16_dma_stats(GemmArgs& g, hipStream_t st) {
     return BB_OK;
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES = 3>
+template <int BM, int BN, int WM, int WN, int STAGES = 3, bool WIDE = false>
 static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t st) {
     constexpr int smem = STAGES * (BM + BN) * 64 * 2;
-    auto kern = gemm_bf16_dma_bnbwd_kernel<BM, BN, WM, WN, STAGES>;
+    auto kern = gemm_bf16_dma_bnbwd_kernel<BM, BN, WM, WN, STAGES, WIDE>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -214,6 +214,12 @@ static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layou
     return t;
 }
 
+// NT and NN kernels reach a tile's rows by 32-bit offsets (DmaLanes); operands whose rows lie further apart take the kernel with
+// an address per lane.
+static DmaTile narrow_or_wide(DmaTile t, int layout, int64_t lda, int64_t ldb) {
+    return t != D_NONE && layout != BB_TN && (lda >= kDmaMaxLd || ldb >= kDmaMaxLd) ? D128x128k64r : t;
+}
+
 // The wave-sliced kernels (gemm_wave.h) take the weight gradients whose 64x64 tiles are at most one per CU, and what the
 // DMA kernels do not take (contractions of odd lengths, few tiles).  W_8: eight waves, 32-wide slices, two stages each (130 KB of LDS);
 // W_4: four waves, 64-wide slices, one stage (65 KB, two blocks a CU).  Measured back to back, 128x128 DMA tiles / W_8 (us):
@@ -241,7 +247,7 @@ template <bool TA, bool TB, int KW, int BK, int NST> static int launch_bf16_wave
 
 template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     const int layout = TA ? BB_TN : TB ? BB_NN : BB_NT;
-    const DmaTile dma = pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.epilogue);
+    const DmaTile dma = narrow_or_wide(pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.epilogue), layout, g.lda, g.ldb);
     switch (pick_wave(g.M, g.N, g.K, batches, layout, dma)) {
         case W_8: return launch_bf16_wave<TA, TB, 8, 32, 2>(g, batches, st);
         case W_4: return launch_bf16_wave<TA, TB, 4, 64, 1>(g, batches, st);
@@ -352,7 +358,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
     BB_REQUIRE(d->layout >= BB_NT && d->layout <= BB_TN, "bb_gemm_variant: bad layout %d", d->layout);
     const int64_t batches = (int64_t)(d->nb1 > 0 ? d->nb1 : 1) * (d->nb2 > 0 ? d->nb2 : 1);
     if (d->dtype == BB_BF16) {
-        const DmaTile dt = pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->epilogue);
+        const DmaTile dt = narrow_or_wide(pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->epilogue), d->layout, d->lda, d->ldb);
         const WaveMode wm = pick_wave(d->M, d->N, d->K, batches, d->layout, dt);
         if (wm != W_NONE) snprintf(out, out_len, "bf16_%s_wave64x64k%d", layouts[d->layout], wm == W_8 ? 8 : 4);
         else snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
@@ -478,7 +484,8 @@ extern "C" int bb_gemm_bn_bwd(const bb_gemm_desc* d, const bb_bn_bwd_stats* bn, 
     if (rc) return rc;
     const BnBwdArgs b = {bn->x, bn->mean, bn->rstd, bn->strips};
     // the tile the plain product of this shape would take, where it is one of those built with the sums
-    const DmaTile dma = pick_dma_tile(d->M, d->N, d->K, 1, BB_NN);
+    const DmaTile dma = narrow_or_wide(pick_dma_tile(d->M, d->N, d->K, 1, BB_NN), BB_NN, g.lda, g.ldb);
+    if (dma == D128x128k64r) return launch_bf16_dma_bnbwd<64, 128, 2, 2, 3, true>(g, b, (hipStream_t)stream);
     if (dma == D64x64k64s4) return launch_bf16_dma_bnbwd<64, 64, 2, 2, 4>(g, b, (hipStream_t)stream);
     if (dma == D256x128k64s3) return launch_bf16_dma_bnbwd<256, 128, 4, 2>(g, b, (hipStream_t)stream);
     return launch_bf16_dma_bnbwd<64, 128, 2, 2>(g, b, (hipStream_t)stream);
@@ -497,7 +504,8 @@ extern "C" int bb_gemm(const bb_gemm_desc* d, void* stream) {
         if (rc) return rc;
         g.strip_stats = d->strip_stats;
         // the tiles that carry the statistics: 64x64 and 256x128 where the ordinary choice would be that tile, else 128x64
-        const DmaTile dma = pick_dma_tile(d->M, d->N, d->K, 1, BB_NT);
+        const DmaTile dma = narrow_or_wide(pick_dma_tile(d->M, d->N, d->K, 1, BB_NT), BB_NT, g.lda, g.ldb);
+        if (dma == D128x128k64r) return launch_bf16_dma_stats<128, 64, 4, 1, 3, true>(g, (hipStream_t)stream);
         if (dma == D64x64k64s4) return launch_bf16_dma_stats<64, 64, 2, 2, 4>(g, (hipStream_t)stream);
         if (dma == D256x128k64s3) return launch_bf16_dma_stats<256, 128, 4, 2>(g, (hipStream_t)stream);
         return launch_bf16_dma_stats<128, 64, 4, 1>(g, (hipStream_t)stream);
@@ -722,7 +730,7 @@ static int colsum_f32(const bb_gemm_desc* descs, int count, void* stream) {
 
 // whether the grouped DMA kernel takes the problem: it masks the contraction's end for weight gradients only
 static bool shared_launch_dma(const bb_gemm_desc& d) {
-    const DmaTile t = pick_dma_tile(d.M, d.N, d.K, 1, d.layout);
+    const DmaTile t = narrow_or_wide(pick_dma_tile(d.M, d.N, d.K, 1, d.layout), d.layout, d.lda, d.ldb);
     return t != D_NONE && t != D128x128k64r;
 }
 

@@ -44,21 +44,30 @@ __device__ __forceinline__ float drop_factor(const GemmArgs& g, int m, int n) {
 // ---- tile order: consecutive logical tiles land on the same XCD (workgroups are dealt
 // round-robin over the 8 XCDs, each with a private L2), and walk the output in column
 // panels of GROUP_M row-tiles so that an XCD's resident tiles share A rows and B columns.
+// n / d of wave-uniform values, n >= 0, d > 0: by a reciprocal, once more for what that leaves, and a correction (the second quotient
+// is off by at most one).  Half the instructions of an integer division, and every kernel starts with two of them in a chain.
+__device__ __forceinline__ int uniform_div(int n, int d) {
+    const float inv = __builtin_amdgcn_rcpf((float)d);
+    int q = __builtin_amdgcn_readfirstlane((int)((float)n * inv));
+    q += __builtin_amdgcn_readfirstlane((int)((float)(n - q * d) * inv));
+    const int r = n - q * d;
+    return r < 0 ? q - 1 : r >= d ? q + 1 : q;
+}
 // logical tile -> (row tile, column tile): column panels of GROUP_M row-tiles
 template <int GROUP_M = 8>
 __device__ __forceinline__ void panel_coords(int lid, int tiles_m, int tiles_n, int& tm, int& tn) {
     const int width = GROUP_M * tiles_n;
-    const int group = lid / width;
+    const int group = uniform_div(lid, width);
     const int first_m = group * GROUP_M;
-    const int gsize = min(tiles_m - first_m, GROUP_M);
-    tm = first_m + (lid % width) % gsize;
-    tn = (lid % width) / gsize;
+    const int gsize = min(tiles_m - first_m, GROUP_M), in = lid - group * width;
+    tn = uniform_div(in, gsize);
+    tm = first_m + in - tn * gsize;
 }
 // block id -> logical tile such that XCD x (which receives the block ids = x mod 8) owns the
 // contiguous range [x * total / 8, (x + 1) * total / 8) of logical tiles
 __device__ __forceinline__ int xcd_contiguous(int bid, int total) {
-    const int per = total / 8;
-    return (per > 0 && bid < per * 8) ? (bid % 8) * per + bid / 8 : bid;
+    const unsigned per = (unsigned)total / 8, b = (unsigned)bid;
+    return b < per * 8 ? (int)((b % 8) * per + b / 8) : bid;
 }
 template <int GROUP_M = 8>
 __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
@@ -123,11 +132,23 @@ __device__ __forceinline__ void unpack_bf16x8(const u32x4& t, float (&v)[8]) {
 // PRE: `pre` holds the 16 bytes of epilogue_operand(g) at xi (fetched earlier); PRE2: `pre2` those of g.resid at xi where
 // BB_EPI_MUL_POS has one
 // PREC: `c_lo`, `c_hi` hold the fp32 C at ci (accumulating problems)
-template <bool DROP, bool PRE = false, bool PRE2 = false, bool PREC = false>
+// KIND: the epilogue kind where the caller has branched on it already (-1: g.epilogue)
+// HELD: nothing is stored, the bytes for C and for a second output are returned in `held` (bf16 C)
+struct HeldStore {
+    u32x4 c, aux;
+};
+__device__ __forceinline__ u32x4 pack_bf16x8(const float (&v)[8]) {
+    u32x4 t;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = pack2bf(v[2 * i], v[2 * i + 1]);
+    return t;
+}
+template <bool DROP, bool PRE = false, bool PRE2 = false, bool PREC = false, int KIND = -1, bool HELD = false>
 __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, int64_t xi, int m, int n, float (&v)[8],
                                                  const float (&b)[8], const u32x4& pre = u32x4{0u, 0u, 0u, 0u},
                                                  const u32x4& pre2 = u32x4{0u, 0u, 0u, 0u}, const f32x4& c_lo = f32x4{0.f, 0.f, 0.f, 0.f},
-                                                 const f32x4& c_hi = f32x4{0.f, 0.f, 0.f, 0.f}) {
+                                                 const f32x4& c_hi = f32x4{0.f, 0.f, 0.f, 0.f}, HeldStore* held = nullptr) {
+    const int kind = KIND >= 0 ? KIND : g.epilogue;
     if (g.bias) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += b[e];
@@ -147,8 +168,9 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
             keep[2 * e + 1] = bb_keep_odd(x, g.drop.thresh) ? g.drop.scale : 0.f;
         }
     }
-    if (g.epilogue == BB_EPI_ACT) {
-        if (g.aux_out) store_vec((bf16*)g.aux_out + xi, v);
+    if (kind == BB_EPI_ACT) {
+        if constexpr (HELD) held->aux = pack_bf16x8(v);
+        else if (g.aux_out) store_vec((bf16*)g.aux_out + xi, v);
         // one branch over the kind for the eight elements (inside the element loop the compiler turns it into
         // both evaluations and a select per element)
         if (g.act == BB_ACT_RELU) {
@@ -162,7 +184,7 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] *= keep[e];
         }
-    } else if (g.epilogue == BB_EPI_DACT) {
+    } else if (kind == BB_EPI_DACT) {
         float u[8];
         if constexpr (PRE) unpack_bf16x8(pre, u);
         else load_vec((const bf16*)g.aux_in + xi, u);
@@ -173,7 +195,7 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] *= dgelu_tanh_f(u[e]);
         }
-    } else if (g.epilogue == BB_EPI_RESIDUAL) {
+    } else if (kind == BB_EPI_RESIDUAL) {
         float r[8];
         if constexpr (PRE) unpack_bf16x8(pre, r);
         else load_vec((const bf16*)g.resid + xi, r);
@@ -183,13 +205,13 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += r[e];
-    } else if (g.epilogue == BB_EPI_MUL) {
+    } else if (kind == BB_EPI_MUL) {
         float d[8];
         if constexpr (PRE) unpack_bf16x8(pre, d);
         else load_vec((const bf16*)g.aux_in + xi, d);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= d[e];
-    } else if (g.epilogue == BB_EPI_MUL_POS) {
+    } else if (kind == BB_EPI_MUL_POS) {
         float d[8];
         if constexpr (PRE) unpack_bf16x8(pre, d);
         else load_vec((const bf16*)g.aux_in + xi, d);
@@ -202,7 +224,7 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = d[e] > 0.f ? v[e] : 0.f;
-    } else if (g.epilogue == BB_EPI_ACT_DACT) {
+    } else if (kind == BB_EPI_ACT_DACT) {
         float d[8];
         if (g.act == BB_ACT_RELU) {
 #pragma unroll
@@ -221,12 +243,15 @@ __device__ __forceinline__ void epilogue_vec8_at(const GemmArgs& g, int64_t ci, 
                 d[e] *= keep[e];
             }
         }
-        store_vec((bf16*)g.aux_out + xi, d);
+        if constexpr (HELD) held->aux = pack_bf16x8(d);
+        else store_vec((bf16*)g.aux_out + xi, d);
     } else if (drop) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= keep[e];
     }
-    if (g.c_f32) {
+    if constexpr (HELD) {
+        held->c = pack_bf16x8(v);
+    } else if (g.c_f32) {
         float* c = (float*)g.C + ci;
         f32x4 lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
         if (g.accumulate) {
@@ -438,6 +463,14 @@ __device__ __forceinline__ void dma16_masked(const void* src, unsigned lds, int 
     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(live) : "m0");
 }
 
+// both with a wave-uniform base and a byte offset per lane
+__device__ __forceinline__ void dma16_base(const void* base, unsigned off, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0");
+}
+__device__ __forceinline__ void dma16_base_masked(const void* base, unsigned off, unsigned lds, int live) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(live) : "m0");
+}
+
 // 3x3 convolution (stride 1, pad 1, NHWC) as an implicit GEMM: the patch matrix [pixels, 9 * channels] is never
 // built, the A loader gathers its rows from the activation tensor instead.
 struct ConvArgs {
@@ -637,6 +670,60 @@ template <int BR, bool KM, int NW, int BK = 32, bool VIS = false, int CONV = 0> 
     }
 };
 
+// DmaOperand for plain operands whose contraction is whole k-tiles: one base for the tile, which moves on in scalar registers, and a
+// 32-bit byte offset per lane and round that never changes.  (A 64-bit address per lane and round costs a vector addition per
+// transfer and two 64-bit multiplications per round before the first of them can go out.)  The offsets of a tile's 256 rows have
+// to fit: leading dimensions below kDmaMaxLd, what the host sends here.
+constexpr int64_t kDmaMaxLd = 1 << 22;
+template <int BR, bool KM, int NW, int BK = 32, bool VIS = false> struct DmaLanes {
+    static constexpr int BYTES = BR * BK * 2;
+    static constexpr int ROUNDS = BYTES / (1024 * NW);
+    static_assert(ROUNDS >= 1 && BR <= 256, "tile too small for the block, or too large for the offsets");
+    const char* base;
+    int64_t step;      // bytes per k-tile
+    unsigned off[ROUNDS];
+
+    __device__ __forceinline__ void init(const bf16* at, int64_t ld, int row0, int rows, int tid) {
+        const int ld2 = (int)ld * 2;
+        if constexpr (!KM) {
+            constexpr int CPR = BK / 8;               // 16-byte chunks per row: as DmaOperand deals them
+            const int r0 = tid / CPR, last = rows - 1 - row0;
+            static_assert(CPR == 8 ? NW * 4 % 8 == 0 : NW * 4 % 4 == 0, "a round later the chunks lie as in the round before");
+            const int c = CPR == 8 ? (tid & 7) ^ ((r0 >> 1) & 7) : (tid & 3) ^ ((r0 >> 2) & 3);
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i) off[i] = __umul24((unsigned)min(r0 + i * (NW * 64 / CPR), last), (unsigned)ld2) + c * 16;
+            base = (const char*)(at + (int64_t)row0 * ld);
+            step = BK * 2;
+        } else {
+            constexpr int CPR = BR / 8;
+            const int k0 = tid / CPR, rel = rows - 8 - row0;
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i) {
+                const int k = k0 + i * (NW * 64 / CPR);
+                const int c = (tid % CPR) ^ km_swizzle<BR>(k);
+                off[i] = __umul24((unsigned)k, (unsigned)ld2) + min(c * 8, rel) * 2;
+            }
+            base = (const char*)(at + row0);
+            step = BK * 2 * ld;
+        }
+    }
+    __device__ __forceinline__ void stop() { step = 0; }
+    __device__ __forceinline__ void mask_tail(int, int) {}   // (whole k-tiles only)
+    template <int I> __device__ __forceinline__ void issue_one(unsigned char* tile, int wave) {
+        if constexpr (VIS) __builtin_amdgcn_global_load_lds((gbl_ptr_t*)(base + off[I]), (lds_ptr_t*)(tile + (I * NW + wave) * 1024), 16, 0, 0);
+        else dma16_base(base, off[I], __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr_t*)(tile + (I * NW + wave) * 1024)));
+        if constexpr (I == ROUNDS - 1) base += step;
+    }
+    __device__ __forceinline__ void issue(unsigned char* tile, int wave) {
+        static_for([&](auto i) { issue_one<decltype(i)::value>(tile, wave); }, std::make_integer_sequence<int, ROUNDS>{});
+    }
+    // (past the end the base runs on: nothing is read there)
+    template <int I> __device__ __forceinline__ void issue_masked(unsigned tile, int wave, int live) {
+        dma16_base_masked(base, off[I], tile + (I * NW + wave) * 1024, live);
+        if constexpr (I == ROUNDS - 1) base += step;
+    }
+};
+
 // per-lane fragment offsets (bytes inside an operand tile) and the fragment fetch
 template <int BR, int T, bool KM, int BK = 32> struct FragReader {
     int off[KM ? T : 1];
@@ -691,12 +778,15 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // CONV 3: its weight gradient (B = the patch matrix, gathered)
     static_assert(CONV == 0 || (CONV == 3 ? AKM && BKM : !AKM && (CONV == 2) == BKM),
                   "implicit convolution: NT forward, NN input gradient, TN weight gradient");
-    using OpA = DmaOperand<BM, AKM, NW, BK, VIS, CONV == 1 || CONV == 2 ? 1 : 0>;
-    using OpB = DmaOperand<BN, BKM, NW, BK, VIS, CONV >= 2 ? CONV : 0>;
+    constexpr bool PLAIN = CONV == 0 && !AKM && !RAGK;   // NT and NN over whole k-tiles
+    using OpA = std::conditional_t<PLAIN, DmaLanes<BM, AKM, NW, BK, VIS>, DmaOperand<BM, AKM, NW, BK, VIS, CONV == 1 || CONV == 2 ? 1 : 0>>;
+    using OpB = std::conditional_t<PLAIN, DmaLanes<BN, BKM, NW, BK, VIS>, DmaOperand<BN, BKM, NW, BK, VIS, CONV >= 2 ? CONV : 0>>;
     constexpr int STAGE_BYTES = OpA::BYTES + OpB::BYTES;
     constexpr int LOADS = OpA::ROUNDS + OpB::ROUNDS;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
+    // what leads to the first transfer, fetched together: the compiler fetches arguments where they are used, one wait after the other
+    asm volatile("" ::"s"(g.A), "s"(g.B), "s"(g.lda), "s"(g.ldb), "s"(g.M), "s"(g.N), "s"(g.K), "s"(g.tiles_m), "s"(g.tiles_n));
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
     int tile_m, tile_n;
@@ -706,10 +796,15 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     if (logical_id) panel_coords<8>(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
     else tile_coords<GROUP_M>(block_id, g.tiles_m, g.tiles_n, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int b1 = batch_id / g.nb2, b2 = batch_id % g.nb2;
-    const bf16* A = (const bf16*)g.A + b1 * g.sA1 + b2 * g.sA2;
-    const bf16* B = (const bf16*)g.B + b1 * g.sB1 + b2 * g.sB2;
-    const int64_t coff = b1 * g.sC1 + b2 * g.sC2;
+    const bf16* A = (const bf16*)g.A;
+    const bf16* B = (const bf16*)g.B;
+    int64_t coff = 0;
+    if (batch_id != 0) {     // (the division and the strides are some fifty instructions in front of the first load)
+        const int b1 = batch_id / g.nb2, b2 = batch_id % g.nb2;
+        A += b1 * g.sA1 + b2 * g.sA2;
+        B += b1 * g.sB1 + b2 * g.sB2;
+        coff = b1 * g.sC1 + b2 * g.sC2;
+    }
 
     OpA opa;
     OpB opb;
@@ -723,6 +818,13 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     fa.init(wm * WTM, lane);
     fb.init(wn * WTN, lane);
 
+    // Transposed products (B times A) where the epilogue takes the accumulators as they are: a lane then has a row of C, four
+    // neighbouring columns in four registers.  The kernels with column statistics keep a column per lane.
+    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS;
+    constexpr bool DIRECT = STATS == 0 && (AHEAD || (BM == 256 && BN == 128 && PLAIN && BK == 64));
+    auto mfma = [](const bf16x8& a, const bf16x8& b, const f32x16& c) {
+        return DIRECT ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    };
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -762,8 +864,6 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // bias gradient riding along: the waves of the first block column (and first wave column)
     // add up the A fragments they hold anyway: lane (m, kg) sees 8 of the 16 k values per step
     const bool do_colsum = AKM && g.colsum != nullptr && tile_n == 0 && wn == 0;
-    // the main loop of the smaller tiles, see there
-    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS;
     float csum[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) csum[i] = 0.f;
@@ -772,7 +872,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[ks][i], f.b[ks][j], acc[i][j], 0, 0, 0);
+                acc[i][j] = mfma(f.a[ks][i], f.b[ks][j], acc[i][j]);
         if constexpr (AKM) {
             if (do_colsum) {
 #pragma unroll
@@ -799,7 +899,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         static_for(
             [&](auto idx) {
                 constexpr int m = decltype(idx)::value, i = m / TN, j = m % TN;
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[ks][i], f.b[ks][j], acc[i][j], 0, 0, 0);
+                acc[i][j] = mfma(f.a[ks][i], f.b[ks][j], acc[i][j]);
                 if constexpr (AKM && j == 0) {
                     if (do_colsum) {
                         float t = 0.f;
@@ -850,21 +950,50 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         }
     };
 
-    // the operand of the epilogue kinds that read one, fetched a patch ahead of its use: the four 16-byte pieces of
-    // patch q; patch 0's go out at the top of the last k-tile
+    // DIRECT: the lane's row and first column of the wave's tiles; of a 32x32 tile it finishes columns 16 h .. 16 h + 7 (h = 0, 1; the
+    // lane 32 further on the eight behind them).  What the epilogue reads beside the product -- the bias, the operand of the
+    // kinds that have one -- is fetched in one go, clamped to the matrix (what lies outside is not stored): behind the first
+    // transfers where the registers are there, else at the loop's end, the first tile's operand under the last k-tile.
+    constexpr int TILES = TM * TN;
+    constexpr bool BEFORE = DIRECT && AHEAD && TILES <= 2;
+    constexpr bool UNDER = DIRECT && BM == 256;
+    const int drow = m0 + wm * WTM + (lane & 31), dcol = n0 + wn * WTN + 8 * (lane >> 5);
+    u32x4 dop[DIRECT ? TILES : 1][2], dbias[DIRECT ? TN : 1][2];
+    auto fetch_bias = [&]() {
+        if constexpr (!DIRECT) return;
+        else {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (g.bias) dbias[j][h] = *(const u32x4*)((const bf16*)g.bias + min(dcol + j * 32 + h * 16, g.N - 8));
+        }
+    };
+    auto fetch_operand = [&](auto first_c, auto count_c) {
+        if constexpr (DIRECT) {
+            const bf16* dopnd = epilogue_operand(g);
+            if (!dopnd) return;
+            static_for(
+                [&](auto t_c) {
+                    constexpr int t = decltype(first_c)::value + decltype(t_c)::value, i = t / TN, j = t % TN;
+                    const bf16* p = dopnd + coff + (int64_t)min(drow + i * 32, g.M - 1) * g.ldaux;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) dop[t][h] = *(const u32x4*)(p + min(dcol + j * 32 + h * 16, g.N - 8));
+                },
+                std::make_integer_sequence<int, decltype(count_c)::value>{});
+        }
+    };
+
+    // the kernels with column statistics: the operands of a patch of two tiles side by side, in four 16-byte pieces
     constexpr int PLD = 68;
     constexpr int NP = (TN + 1) / 2;   // pairs per row of accumulator tiles, the last one possibly a single
     const int prow = lane >> 3, pcol = (lane & 7) * 8;
-    // Only on the large tiles (one block per CU, two waves per SIMD whatever the kernel's register count) and on the
-    // ones that read ahead: on the others the 32 registers would cost a resident block.
-    // Some of the other kernels fetch a patch's operand(s) in one go at the top of that patch: the pointers of GemmArgs
-    // may alias as far as the compiler knows, so left inside the row loop every load waits behind the previous row's
-    // store (four round trips in a row per patch instead of one).
-    // (HOIST: where that does not cost a resident block -- the kernels with the BatchNorm backward sums, whose three
-    // operand reads per row are most of their epilogue)
+    // HOIST: fetched in one go, at the top of the patch.  The pointers of GemmArgs may alias as far as the compiler knows, so
+    // left inside the row loop every load waits behind the previous row's store (four round trips in a row per patch instead
+    // of one; the three operand reads per row of the BatchNorm backward sums are most of their epilogue).
     // EARLY: the kernels whose waves finish one patch each and have the registers fetch it -- and the bias -- before the main loop.
-    constexpr bool EARLY = AHEAD && TM * NP == 1;
-    constexpr bool PREF = (BM * BN >= 256 * 128 || AHEAD) && !VIS && CONV == 0 && STATS == 0;
+    constexpr bool EARLY = AHEAD && TM * NP == 1 && !DIRECT;
+    constexpr bool PREF = BM * BN >= 256 * 128 && !VIS && CONV == 0 && STATS == 0 && !DIRECT;
     constexpr bool HOIST = STATS == 2;
     const bf16* opnd = PREF || HOIST ? epilogue_operand(g) : nullptr;
     u32x4 opc[PREF || HOIST ? 4 : 1], opn[PREF ? 4 : 1];
@@ -955,7 +1084,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
             static_for(
                 [&](auto idx) {
                     constexpr int m = decltype(idx)::value, ks = m / (TM * TN), i = m % (TM * TN) / TN, j = m % TN;
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.a[ks][i], cur.b[ks][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = mfma(cur.a[ks][i], cur.b[ks][j], acc[i][j]);
                     if constexpr (m < RM) {
                         static_for(
                             [&](auto r) {
@@ -975,6 +1104,13 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
 #pragma unroll
         for (int t = 0; t < STAGES; ++t)
             static_for([&](auto k_c) { feed(k_c, lds0 + t * STAGE_BYTES, __builtin_amdgcn_readfirstlane((t - KT) >> 31)); }, std::make_integer_sequence<int, LOADS>{});
+        // (behind the transfers: the waits below count those that are newer than the one waited for, more of them do no harm)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (BEFORE) {
+            fetch_bias();
+            fetch_operand(std::integral_constant<int, 0>{}, std::integral_constant<int, TILES>{});
+        }
         asm volatile("" ::: "memory");
         wait_vmcnt_lgkm0<(STAGES - 1) * LOADS>();
         __builtin_amdgcn_s_barrier();
@@ -1028,6 +1164,9 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
             if constexpr (STAGES >= 3) {
                 if constexpr (PREF) {
                     if (kt == KT - 1) fetch(std::integral_constant<int, 0>{}, opc);
+                }
+                if constexpr (UNDER) {
+                    if (kt == KT - 1) fetch_operand(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
                 }
                 // the DMA instructions of tile kt+STAGES-1 a third each between the MFMAs of the first three quarters
                 // (issued in one burst at the top they queue up in front of the texture path and the waves behind
@@ -1140,13 +1279,100 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         }
     }
 
+    if constexpr (DIRECT) {
+        // Epilogue from the registers.  Columns 0-3 | 8-11 of a 32x32 tile's row are in a lane's registers 0-3 | 4-7, columns 4-7 | 12-15
+        // in those of the lane 32 further on: registers 4-7 of the lower lanes change places with 0-3 of the upper ones, and each
+        // lane has eight neighbouring columns, 16 bytes of C; the two lanes of a row and the tiles next to each other fill its
+        // 128-byte lines in stores that follow each other.  No LDS, no barrier, and one branch over the epilogue's kind for all
+        // tiles.  (Before, every wave parked pairs of tiles in LDS and read them back by rows of eight lanes, with the branches in every
+        // one of four passes: about 2600 cycles for the single 32x32 tile a wave has in the 64x64 kernels, a third of what a
+        // product of two k-tiles takes there.)  Back to back with the shorter way to the first transfer, before / now (us): NT
+        // 128x128x128 4.1 / 3.2, 1050x512x512 5.4 / 4.4, 1050x512x2048 9.6 / 8.3; 128x64 tiles 1024x1536x512 7.4 / 6.4; 256x128
+        // tiles 2043x2304x768 15.6 / 13.6, 8192x3072x1024 63.5 / 60.5, NN 8192x1024x1024 23.3 / 21.6; with an operand to multiply by or
+        // two outputs 20.4 / 20.4 and 22.4 / 22.5 (2043x3072x768).  256x256 tiles keep LDS: stores of 32 bytes a row fill a line in
+        // four instructions, and with two outputs and GELU between them 8192x4096x1024 takes 99 us instead of 89 (130 when each
+        // piece is stored as it is made).
+        if constexpr (!BEFORE) {
+            fetch_bias();
+            fetch_operand(std::integral_constant<int, UNDER ? 1 : 0>{}, std::integral_constant<int, UNDER ? TILES - 1 : TILES>{});   // (tile 0's is on its way)
+        }
+        wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before the block's LDS is another's
+        // accumulators of columns 16 h .. 16 h + 15 of a tile -> the lane's eight
+        auto columns = [&](const f32x16& c, auto h_c, float (&v)[8]) {
+            constexpr int h = decltype(h_c)::value;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                typedef __attribute__((ext_vector_type(2))) unsigned u2;
+                const u2 w = __builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(__float_as_uint(c[h * 8 + e]), __float_as_uint(c[h * 8 + 4 + e]), false, false));
+                v[e] = __uint_as_float(w[0]);
+                v[4 + e] = __uint_as_float(w[1]);
+            }
+            if (g.alpha != 1.0f) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] *= g.alpha;
+            }
+        };
+        // HELD: the pieces of a row are made first and stored one behind the other, a whole line at a time
+        auto finish = [&](auto kind_c, auto held_c) {
+            constexpr int kind = decltype(kind_c)::value;
+            constexpr bool HELD = decltype(held_c)::value;
+            static_for(
+                [&](auto i_c) {
+                    constexpr int i = decltype(i_c)::value;
+                    const int m = drow + i * 32;
+                    const int64_t ci = coff + (int64_t)m * g.ldc + dcol, xi = coff + (int64_t)m * g.ldaux + dcol;
+                    HeldStore held[HELD ? TN : 1][2];
+                    static_for(
+                        [&](auto p_c) {
+                            constexpr int j = decltype(p_c)::value / 2, h = decltype(p_c)::value % 2, t = i * TN + j;
+                            float v[8], b8[8];
+                            columns(acc[i][j], std::integral_constant<int, h>{}, v);
+                            if (g.bias) unpack_bf16x8(dbias[j][h], b8);
+                            const int n = dcol + j * 32 + h * 16, o = j * 32 + h * 16;
+                            if (HELD || (m < g.M && n < g.N))
+                                epilogue_vec8_at<DROP, true, false, false, kind, HELD>(g, ci + o, xi + o, HELD ? min(m, g.M - 1) : m, HELD ? min(n, g.N - 8) : n, v, b8, dop[t][h],
+                                                                                       u32x4{0u, 0u, 0u, 0u}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, &held[HELD ? j : 0][h]);
+                        },
+                        std::make_integer_sequence<int, 2 * TN>{});
+                    if constexpr (HELD) {
+                        const bool two = kind == BB_EPI_ACT_DACT || (kind == BB_EPI_ACT && g.aux_out);
+                        if (m < g.M) {
+#pragma unroll
+                            for (int p = 0; p < 2 * TN; ++p)
+                                if (dcol + p * 16 < g.N) *(u32x4*)((bf16*)g.C + ci + p * 16) = held[p / 2][p % 2].c;
+                            if (two) {
+#pragma unroll
+                                for (int p = 0; p < 2 * TN; ++p)
+                                    if (dcol + p * 16 < g.N) *(u32x4*)((bf16*)g.aux_out + xi + p * 16) = held[p / 2][p % 2].aux;
+                            }
+                        }
+                    }
+                },
+                std::make_integer_sequence<int, TM>{});
+        };
+        if (g.c_f32) {
+            finish(std::integral_constant<int, -1>{}, std::false_type{});
+            return;
+        }
+        switch (g.epilogue) {
+            case BB_EPI_ACT: finish(std::integral_constant<int, BB_EPI_ACT>{}, std::true_type{}); break;
+            case BB_EPI_DACT: finish(std::integral_constant<int, BB_EPI_DACT>{}, std::true_type{}); break;
+            case BB_EPI_RESIDUAL: finish(std::integral_constant<int, BB_EPI_RESIDUAL>{}, std::true_type{}); break;
+            case BB_EPI_MUL: finish(std::integral_constant<int, BB_EPI_MUL>{}, std::true_type{}); break;
+            case BB_EPI_MUL_POS: finish(std::integral_constant<int, BB_EPI_MUL_POS>{}, std::true_type{}); break;
+            case BB_EPI_ACT_DACT: finish(std::integral_constant<int, BB_EPI_ACT_DACT>{}, std::true_type{}); break;
+            default: finish(std::integral_constant<int, BB_EPI_NONE>{}, std::true_type{}); break;
+        }
+        return;
+    }
+
     // Epilogue through LDS: every wave parks two horizontally adjacent 32x32 accumulator tiles in a
     // private [32][64 (+4 pad)] fp32 patch; then one wave instruction covers 8 rows x 64 columns, lane l
     // taking 8 consecutive columns of row l/8, so every global load / store of the epilogue moves whole
     // 128-byte row segments (256 bytes for fp32 outputs).
     // An odd tile count per row ends with a single tile: its 32 columns use half of the patch and half of
     // the lanes of the row pass.
-    if constexpr (PREF && !EARLY && (AHEAD || !(BK == 64 && STAGES >= 3))) fetch(std::integral_constant<int, 0>{}, opc);
+    if constexpr (PREF && !(BK == 64 && STAGES >= 3)) fetch(std::integral_constant<int, 0>{}, opc);
     wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before their stages become the patch
     __syncthreads();
     float* patch = (float*)smem + wave * (32 * PLD);
@@ -1259,14 +1485,15 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
     gemm_bf16_dma_body<BM, BN, WM, WN, AKM, BKM, DB, STAGES, BK, false, 0, 0, DROP, RAGK>(g, blockIdx.x, blockIdx.z);
 }
 // the same with the strip statistics of the output (NT, 64-wide k-tiles)
-template <int BM, int BN, int WM, int WN, int STAGES>
+// WIDE: rows further apart than DmaLanes reaches (by the loader of the kernels for any contraction)
+template <int BM, int BN, int WM, int WN, int STAGES, bool WIDE>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_stats_kernel(const GemmArgs g) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, false, false, true, STAGES, 64, false, 0, 1>(g, blockIdx.x, blockIdx.z);
+    gemm_bf16_dma_body<BM, BN, WM, WN, false, false, true, STAGES, 64, false, 0, 1, false, WIDE>(g, blockIdx.x, 0);
 }
 // input gradient of a 1x1 convolution (NN, 64-wide k-tiles) with the backward sums of the batch normalisation in front of it
-template <int BM, int BN, int WM, int WN, int STAGES>
+template <int BM, int BN, int WM, int WN, int STAGES, bool WIDE>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_bnbwd_kernel(const GemmArgs g, const BnBwdArgs bn) {
-    gemm_bf16_dma_body<BM, BN, WM, WN, false, true, true, STAGES, 64, false, 0, 2>(g, blockIdx.x, 0, false, ConvArgs{}, bn);
+    gemm_bf16_dma_body<BM, BN, WM, WN, false, true, true, STAGES, 64, false, 0, 2, false, WIDE>(g, blockIdx.x, 0, false, ConvArgs{}, bn);
 }
 
 // Persistent variant for problems of more than one round of 256x256 tiles (NT and NN, 32-wide k-tiles, three stages,
