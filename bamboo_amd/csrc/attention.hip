@@ -199,9 +199,9 @@ __device__ __forceinline__ int kv_limit(const AttnArgs& a, int b, int q) {
 // the pair's K and V stay in that XCD's L2 - and, under a causal mask, the same mix of long and
 // short blocks as every other XCD, longest first (rank 0 = most work).
 struct BlockMap { int rank, bh; };
-__device__ __forceinline__ BlockMap map_block(int nbh) {
+__device__ __forceinline__ BlockMap map_block(int block, int nbh) {
     const int per_xcd = (nbh + 7) >> 3;
-    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int xcd = block & 7, j = block >> 3;
     return {j / per_xcd, (j % per_xcd) * 8 + xcd};
 }
 static unsigned attn_grid(int seq, int rows, int nbh) { return (unsigned)(8 * ((nbh + 7) / 8) * ((seq + rows - 1) / rows)); }
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
     const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
     unsigned char* smem = smem_all + grp * (4 * TILE);
     const int groups = a.heads / HP;
-    const BlockMap bm = map_block(a.batch * groups);
+    const BlockMap bm = map_block(blockIdx.x, a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
     const int qb = (a.seq + ROWS - 1) / ROWS - 1 - bm.rank;  // long (late) query blocks first
     const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP;
@@ -437,17 +437,17 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
 // NPAN = 2 (128-wide heads): a block accumulates dK and dV for ONE 64-wide half `fh` of the head's columns (the grid
 // has two blocks per head and key block); scores and dP take the full 128 columns in both, i.e. are made twice -- a wave
 // that held all four output tiles of dK and of dV next to K, V, S and dP would need more registers than it has.
-template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
+// OWN: no dQ kernel has run before this one: the block makes delta of all its queries itself, in LDS from OWN_AT on
+template <bool DROP, int HP, int NPAN, int W, int G, bool OWN>
+__device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int block, unsigned char* smem_all, const int own_at) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192, ROWS = W * 32;
     // per group 2 stages x (Q tile, dO tile: 8 KiB per panel, lse 256 B per head, delta 256 B per head)
     constexpr int STAGE = 2 * TILE + 512 * HP;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
     unsigned char* smem = smem_all + grp * (2 * STAGE);
     const int groups = a.heads / HP;
-    const BlockMap bm = map_block(a.batch * groups * NPAN);
+    const BlockMap bm = map_block(block, a.batch * groups * NPAN);
     if (bm.bh >= a.batch * groups * NPAN) return;
     const int kb = bm.rank;  // early key blocks are seen by the most queries
     const int fh = bm.bh % NPAN, bg = bm.bh / NPAN;
@@ -496,18 +496,45 @@ __global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnA
         }
         // extra loads, dealt to the waves: lse of the block's heads, then delta
 #pragma unroll
-        for (int j = 0; j < 2 * HP; ++j)
+        for (int j = 0; j < (OWN ? 1 : 2) * HP; ++j)
             if (j % W == wave) dma_f32x64((j / HP ? DELTA : LSE) + (int64_t)(j % HP) * a.seq, qs, last, st + 2 * TILE + j * 256, lane);
     };
 
     if (q_begin + grp < ntiles) issue(q_begin + grp, 0);
+    const int own_rows = (a.seq + 63) / 64 * 64;     // of a head's deltas in LDS
+    if constexpr (OWN) {
+        // as the dQ kernel makes them, in its order of additions: a lane and its partner (lane ^ 32) have the halves of each
+        // 16-column step of a row
+        float* own = (float*)(smem_all + own_at);
+        const bf16* O = a.o + row_base * a.ld_o + hg * (64 * NPAN);
+        for (int q = q_begin * 64 + (tid >> 6) * 32 + (lane & 31); q < ntiles * 64; q += W * G * 32) {
+            const int64_t at = (int64_t)min(q, last) * a.ld_o + (lane >> 5) * 8;
+            bf16x8 df[4 * NPAN], of[4 * NPAN];
+#pragma unroll
+            for (int ks = 0; ks < 4 * NPAN; ++ks) {
+                df[ks] = *(const bf16x8*)(DO + at + ks * 16);
+                of[ks] = *(const bf16x8*)(O + at + ks * 16);
+            }
+#pragma unroll
+            for (int hh = 0; hh < HP; ++hh) {
+                float dl = 0.f;
+#pragma unroll
+                for (int k = 0; k < KS; ++k)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) dl = fmaf((float)df[hh * KS + k][e], (float)of[hh * KS + k][e], dl);
+                dl += __shfl_xor(dl, 32, 64);
+                if (lane < 32) own[hh * own_rows + q] = dl;
+            }
+        }
+        // (the first tile's wait and barrier make them visible)
+    }
     for (int i = 0; q_begin + i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
         const int t = q_begin + i * G + grp, slot = i & 1;
         asm volatile("" ::: "memory");
         if (t + G < ntiles) {
             issue(t + G, slot ^ 1);
             // the waves with extra loads wait for as many newer loads more than the others
-            constexpr int LOADS = 16 / W * NPAN, EACH = 2 * HP / W, MORE = 2 * HP % W;
+            constexpr int LOADS = 16 / W * NPAN, EXTRA = (OWN ? 1 : 2) * HP, EACH = EXTRA / W, MORE = EXTRA % W;
             if (MORE == 0 || wave < MORE) wait_vm<LOADS + EACH + (MORE ? 1 : 0)>(); else wait_vm<LOADS + EACH>();
         } else {
             wait_vm<0>();
@@ -525,7 +552,7 @@ __global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnA
 #pragma unroll
           for (int hh = 0; hh < HP; ++hh) {
             const float* lse_t = lse_all + 64 * hh;
-            const float* del_t = del_all + 64 * hh;
+            const float* del_t = OWN ? (const float*)(smem_all + own_at) + hh * own_rows + t * 64 : del_all + 64 * hh;
             const int head = head0 + hh;
             // S[q][kv] and dP[q][kv]
             f32x16 s, dp;
@@ -680,15 +707,14 @@ __global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnA
 // =========================================================================================
 // backward dQ: block = 128 queries (4 waves x 32), loop over 64-key tiles
 // =========================================================================================
-template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
+template <bool DROP, int HP, int NPAN, int W, int G>
+__device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int block, unsigned char* smem_all) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
     unsigned char* smem = smem_all + grp * (4 * TILE);
     const int groups = a.heads / HP;
-    const BlockMap bm = map_block(a.batch * groups);
+    const BlockMap bm = map_block(block, a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
     const int qb = (a.seq + ROWS - 1) / ROWS - 1 - bm.rank;
     const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP;
@@ -848,6 +874,25 @@ __global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dq_kernel(const AttnAr
     }
 }
 
+template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
+    attn_bwd_dkv_block<DROP, HP, NPAN, W, G, false>(a, blockIdx.x, smem_all, 0);
+}
+template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
+    attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x, smem_all);
+}
+// Both in one launch, where there is room for all their blocks (attn_bwd_launch): first the dK / dV blocks, whose walks are the
+// longer ones, then the dQ blocks.
+template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_kernel(const AttnArgs a, const int dkv_blocks, const int own_at) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
+    if ((int)blockIdx.x < dkv_blocks) attn_bwd_dkv_block<DROP, HP, NPAN, W, G, true>(a, blockIdx.x, smem_all, own_at);
+    else attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x - dkv_blocks, smem_all);
+}
+
 // =========================================================================================
 // host entry points
 // =========================================================================================
@@ -894,6 +939,33 @@ struct attn_dkv_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_bwd_dkv_kernel<true, HP, NPAN, W, G> : attn_bwd_dkv_kernel<false, HP, NPAN, W, G>;
         return attn_go(kern, seq, W * 32, nbh * NPAN, W * G * 64, attn_lds<HP, NPAN, W, G>(true), a, st);   // 128-wide heads: a block per half
+    }
+};
+// Both backward kernels: in one launch where all blocks of the two find room at once (two blocks of four waves a CU, one of eight),
+// else one after the other.  Each alone is bound by its longest walk while at most half of the chip has work; together they take
+// the longer of the two instead of the sum, and a launch less.  What it costs is delta a second time, by every dK / dV block for the
+// queries it will meet, and registers: beyond a round both weigh more than what overlaps.  One after the other / together (us): 2 x 2
+// heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (64 + 64 blocks) 23.8 / 16.1; 6 x 8, 175 (96 + 96) 17.7 / 12.0; 2 x
+// 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two heads of 128, 512, dropout 69.0 /
+// 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
+// 192) 68 / 73, 4 x 16, 256 causal (256 + 256 of eight) 18.0 / 18.5.  The bits are the same.
+static constexpr int kOwnDeltaSeq = 2048;    // longest sequence whose deltas a block keeps in LDS
+struct attn_bwd_launch {
+    template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
+        const int64_t rows = (seq + W * 32 - 1) / (W * 32), slots = 256 * 8 / (W * G);
+        if (seq > kOwnDeltaSeq || nbh * rows * (NPAN + 1) > slots) {
+            // the dQ kernel first: it also leaves delta = rowsum(dO o O) of its queries for the dK / dV kernel
+            const int rc = attn_dq_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
+            return rc ? rc : attn_dkv_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
+        }
+        const unsigned dkv = attn_grid(seq, W * 32, nbh * NPAN), dq = attn_grid(seq, W * 32, nbh);
+        constexpr size_t own_at = attn_lds<HP, NPAN, W, G>(true) > attn_lds<HP, NPAN, W, G>(false) ? attn_lds<HP, NPAN, W, G>(true) : attn_lds<HP, NPAN, W, G>(false);
+        const size_t lds = own_at + (size_t)HP * ((seq + 63) / 64 * 64) * sizeof(float);
+        auto kern = a.drop.thresh ? attn_bwd_kernel<true, HP, NPAN, W, G> : attn_bwd_kernel<false, HP, NPAN, W, G>;
+        BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));
+        bb_launch(kern, dim3(dkv + dq), dim3(W * G * 64), lds, st, a, (int)dkv, (int)own_at);
+        BB_LAUNCH_CHECK();
+        return BB_OK;
     }
 };
 // The shape of a block, by the number of blocks of 128 rows and the length of the walk (a pair of heads walks twice).  Four
@@ -963,8 +1035,5 @@ extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int s
     a.batch = batch; a.heads = heads; a.seq = seq; a.mask = mask;
     a.scale = 1.0f / sqrtf((float)head_dim);
     a.scale_log2 = a.scale * 1.4426950408889634f;
-    // the dQ kernel first: it also leaves delta = rowsum(dO o O) of its queries for the dK / dV kernel
-    rc = attn_launch<attn_dq_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
-    if (rc) return rc;
-    return attn_launch<attn_dkv_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
+    return attn_launch<attn_bwd_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
 }

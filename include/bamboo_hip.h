@@ -260,7 +260,8 @@ int bb_attention_fwd(int dtype, int mask, int batch, int heads, int seq, int hea
                      const int32_t* key_len, float dropout_p, uint32_t dropout_k0, uint32_t dropout_k1, void* stream);
 /* Backward of bb_attention_fwd: dq, dk, dv (same addressing as q, k, v with row stride ld_dqkv)
  * from d_out, the forward's out and lse.  delta: fp32 workspace [batch, heads, seq].
- * Deterministic (no atomics): dK/dV and dQ are produced by two passes over the score tiles. */
+ * Deterministic (no atomics): dK/dV and dQ are produced by two passes over the score tiles, in two launches or, where
+ * the chip has room for both, in one (delta is then left as it was). */
 int bb_attention_bwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
                      const void* k, const void* v, int64_t ld_qkv, const void* out, const void* d_out,
                      int64_t ld_out, const float* lse, float* delta, void* dq, void* dk, void* dv,
