@@ -21,6 +21,8 @@
 // double-buffered.  All reductions have a fixed order: results are reproducible bit for bit.
 #include "common.h"
 
+#include <type_traits>
+
 typedef __attribute__((address_space(3))) void lds_ptr_t;
 typedef const __attribute__((address_space(1))) void gbl_ptr_t;
 typedef __attribute__((ext_vector_type(4))) short s16x4;
@@ -52,9 +54,10 @@ __device__ __forceinline__ uint64_t prob_index(const AttnArgs& a, int b, int hea
 // inline assembly: while the compiler sees such a load in flight it turns every wait for an LDS
 // read into lgkmcnt(0).  Unseen, fragment waits keep their exact counts; the kernels wait for
 // these loads explicitly (wait_vm) before each barrier, as they always did.
-__device__ __forceinline__ void dma16(const void* src, const unsigned char* lds_dst) {
+// (wave-uniform base, a byte offset per lane)
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, const unsigned char* lds_dst) {
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr_t*)lds_dst);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0), "v"(src) : "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(off), "s"(base) : "m0");
 }
 __device__ __forceinline__ void dma4(const void* src, const unsigned char* lds_dst) {
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr_t*)lds_dst);
@@ -64,36 +67,32 @@ __device__ __forceinline__ void dma4(const void* src, const unsigned char* lds_d
 // ---- LDS tile format: [rows][64] bf16, 128 B per row, 16-byte chunk c of row r at slot c ^ fsw(r)
 __device__ __forceinline__ int fsw(int r) { return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1); }
 
-// one wave-instruction moves 8 rows; instruction `idx` of a tile covers rows idx*8 .. idx*8+7
-__device__ __forceinline__ void dma_rows8(const bf16* gbase, int64_t ld, int row0, int last_row, unsigned char* tile,
-                                          int idx, int lane) {
-    const int r = idx * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ fsw(r);
-    const int gr = min(row0 + r, last_row);
-    dma16(gbase + (int64_t)gr * ld + c * 8, tile + idx * 1024);
-}
-// Whole 64-row tile by W waves: row groups wave, wave + W, ...  Full tiles take a wave-uniform base plus the lane's fixed
-// offset; only a tile that reaches past the last row pays for per-lane clamping.
+// Whole 64-row tile by W waves, eight rows an instruction: row groups wave, wave + W, ...  A wave-uniform base plus the lane's
+// offset in bytes (leading dimensions below 2^24: 63 rows fit 32 bits), which only a tile that reaches past the last row clamps.
 template <int W> struct LaneOff { uint32_t o[8 / W]; };
+template <int W> __device__ __forceinline__ uint32_t lane_row(int i, int wave, int lane) { return (wave + i * W) * 8 + (lane >> 3); }
 template <int W> __device__ __forceinline__ LaneOff<W> lane_off(int64_t ld, int wave, int lane) {
     LaneOff<W> l;
 #pragma unroll
     for (int i = 0; i < 8 / W; ++i) {
-        const int r = (wave + i * W) * 8 + (lane >> 3);
-        l.o[i] = (uint32_t)(r * ld + (((lane & 7) ^ fsw(r)) << 3));
+        const uint32_t r = lane_row<W>(i, wave, lane);
+        l.o[i] = (r * (uint32_t)ld + (((lane & 7) ^ fsw(r)) << 3)) * 2;
     }
     return l;
 }
 template <int W>
 __device__ __forceinline__ void dma_tile64(const bf16* gbase, int64_t ld, int row0, int last_row, unsigned char* tile,
                                            int wave, int lane, const LaneOff<W>& lo) {
+    const bf16* g = gbase + (int64_t)row0 * ld;
     if (row0 + 63 <= last_row) {
-        const bf16* g = gbase + (int64_t)row0 * ld;
 #pragma unroll
-        for (int i = 0; i < 8 / W; ++i) dma16(g + lo.o[i], tile + (wave + i * W) * 1024);
+        for (int i = 0; i < 8 / W; ++i) dma16(g, lo.o[i], tile + (wave + i * W) * 1024);
     } else {
 #pragma unroll
-        for (int i = 0; i < 8 / W; ++i) dma_rows8(gbase, ld, row0, last_row, tile, wave + i * W, lane);
+        for (int i = 0; i < 8 / W; ++i) {
+            const uint32_t r = lane_row<W>(i, wave, lane), past = max((int)r - (last_row - row0), 0);
+            dma16(g, lo.o[i] - past * (uint32_t)ld * 2, tile + (wave + i * W) * 1024);
+        }
     }
 }
 // 4-byte variant for the per-row fp32 statistics: 64 consecutive floats
@@ -229,7 +228,7 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];  // G rings of 2 stages x (K, V)
-    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
+    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = uw % W, grp = G == 1 ? 0 : uw / W;
     unsigned char* smem = smem_all + grp * (4 * TILE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(blockIdx.x, a.batch * groups);
@@ -252,6 +251,18 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
     const int my_limit = kv_limit(a, b, myq);
     const int wave_min_limit = kv_limit(a, b, q0);  // limits grow with the query index
 
+    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
+    auto issue = [&](int t, int slot) {
+        unsigned char* st = smem + slot * (2 * TILE);
+        const int kv0 = t * 64;
+#pragma unroll
+        for (int p = 0; p < NPAN; ++p) {
+            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
+            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
+        }
+    };
+
+    if (grp < ntiles) issue(grp, 0);
     bf16x8 qf[4 * NPAN];
     {
         const bf16* qp = Q + (int64_t)min(myq, last) * a.ld_qkv + (lane >> 5) * 8;
@@ -270,18 +281,10 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
         lsum[hh] = 0.f;
     }
 
-    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
-    auto issue = [&](int t, int slot) {
-        unsigned char* st = smem + slot * (2 * TILE);
-        const int kv0 = t * 64;
-#pragma unroll
-        for (int p = 0; p < NPAN; ++p) {
-            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
-            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
-        }
-    };
-
-    if (grp < ntiles) issue(grp, 0);
+    // The first tile and the queries: waited for in full, or the compiler, which counts its own loads only, puts the waits for the
+    // queries into the loop, where they hold for the transfers of the next tile (8 x 16 heads of 64, 1024 causal 37.7 -> 34.6 us).
+    asm volatile("" ::: "memory");
+    wait_vm<0>();
     for (int i = 0; i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
         const int t = i * G + grp, slot = i & 1;
         asm volatile("" ::: "memory");
@@ -432,6 +435,84 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
 }
 
 // =========================================================================================
+// backward: the walk of a wave over its sub-tiles, shared by both kernels
+// =========================================================================================
+// A sub-tile's work is a chain: scores (matrix cores, operands from LDS), probabilities (vector ALU) with the gradients of the scores
+// beside them (matrix cores), dS (vector ALU), the products with P and dS (matrix cores).  PIPE: the scores of the sub-tile after it
+// go beside dS, so that a wave starts a sub-tile on the vector ALU at once, and operands are read from LDS a phase ahead.  What it gives
+// is latency, where a SIMD has one wave: 2 x 8 heads of 64, 1024 keys 38.2 us one after the other, 33.1 this way.  Beyond that the two are
+// equal (8 x 16 heads, 1024: 140 us, 865 TFLOP/s of matrix work; two, three or four waves a SIMD the same within 3 %; without the
+// exponentials 121, without LDS reads 118): what bounds it is power, a clock of 2.1 GHz.  A wave walks only sub-tiles of 32 that
+// hold a pair its mask keeps; with the waits outside of the loop (below) 8 x 16 heads, 1024 causal 100.8 -> 90.9, unmasked 157 -> 139.
+constexpr bool attn_bwd_pipe(int npan) { return npan == 1; }
+// stages of a ring: three where a tile's last products come behind the barrier that hands the next tile out, two where three do not fit
+constexpr int attn_bwd_stages(int npan, int g) { return npan == 1 && g <= 2 ? 3 : 2; }
+template <int HP, int G, int STAGES, int STAGE, bool PIPE, typename Live, typename FetchS, typename FetchG, typename Scores, typename Grads, typename Probs, typename Contract, typename Issue>
+__device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int iters, const Live& live, const FetchS& fetch_scores, const FetchG& fetch_grads, const Scores& scores, const Grads& score_grads,
+                                              const Probs& probs, const Contract& contract, const Issue& issue) {
+    constexpr int J = 2 * HP;      // sub-tiles of a tile, heads of a pair one after the other
+    using First = std::integral_constant<int, 0>;
+    int stage = 0;
+    auto begin = [&](const unsigned char* st, auto j_c) {      // a wave's first sub-tile, or the first behind a turn it could not look past
+        fetch_scores(st, j_c);
+        fetch_grads(st, j_c);
+        scores(j_c);
+    };
+    if constexpr (PIPE) {
+        if (live(t, 0)) begin(smem, First{});
+    }
+    for (int i = 0; i < iters; ++i, t += G) {   // the barriers are the block's: every group goes round as often
+        const unsigned char* st = smem + stage * STAGE;
+        const int after = stage + 1 == STAGES ? 0 : stage + 1, free = STAGES == 2 ? stage : after + 1 == STAGES ? 0 : after + 1;
+        const unsigned char* st_after = smem + after * STAGE;
+        // the next tile, on its way for a whole tile by now, has landed for all waves; all are done with the stage that the one
+        // after it is sent to
+        auto turn = [&]() {
+            if (i + 1 < iters) {
+                asm volatile("" ::: "memory");
+                wait_vm<0>();
+                block_sync();
+                issue(t + 2 * G, free);
+            }
+        };
+        auto step = [&](auto j_c) {
+            constexpr int j = decltype(j_c)::value;
+            constexpr bool LAST = j == J - 1;
+            constexpr bool BEHIND = LAST && STAGES == 2;      // the next tile comes in behind the last products of this one
+            using Next = std::integral_constant<int, LAST ? 0 : j + 1>;
+            const bool run = live(t, j / HP), next = LAST ? i + 1 < iters && live(t + G, 0) : live(t, (j + 1) / HP);
+            if constexpr (PIPE && LAST && STAGES == 3) turn();
+            const unsigned char* st_next = LAST ? st_after : st;
+            if (run) {
+                if constexpr (!PIPE) begin(st, j_c);
+                // (of no use behind the wave's last sub-tile: branches around them would keep them apart from what they go beside)
+                if constexpr (PIPE && !BEHIND) fetch_scores(st_next, Next{});
+                score_grads(j_c);
+                probs(st, t, j_c);
+                if constexpr (PIPE && !BEHIND) {
+                    fetch_grads(st_next, Next{});
+                    scores(Next{});
+                }
+                contract(st, t, j_c);
+            } else if constexpr (PIPE && !BEHIND) {
+                if (next) begin(st_next, Next{});
+            }
+            if constexpr (LAST && STAGES == 2) {
+                turn();
+                if (PIPE && next) begin(st_after, Next{});
+            }
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        if constexpr (HP == 2) {
+            step(std::integral_constant<int, 2>{});
+            step(std::integral_constant<int, 3>{});
+        }
+        stage = after;
+    }
+}
+
+// =========================================================================================
 // backward dK, dV: block = 128 keys (4 waves x 32), loop over 64-query tiles
 // =========================================================================================
 // NPAN = 2 (128-wide heads): a block accumulates dK and dV for ONE 64-wide half `fh` of the head's columns (the grid
@@ -442,10 +523,11 @@ template <bool DROP, int HP, int NPAN, int W, int G, bool OWN>
 __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int block, unsigned char* smem_all, const int own_at) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192, ROWS = W * 32;
-    // per group 2 stages x (Q tile, dO tile: 8 KiB per panel, lse 256 B per head, delta 256 B per head)
-    constexpr int STAGE = 2 * TILE + 512 * HP;
-    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
-    unsigned char* smem = smem_all + grp * (2 * STAGE);
+    // per group STAGES x (Q tile, dO tile: 8 KiB per panel, lse 256 B per head, delta 256 B per head)
+    constexpr bool PIPE = attn_bwd_pipe(NPAN);
+    constexpr int STAGE = 2 * TILE + 512 * HP, STAGES = attn_bwd_stages(NPAN, G), BUFS = PIPE ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = uw % W, grp = G == 1 ? 0 : uw / W;
+    unsigned char* smem = smem_all + grp * (STAGES * STAGE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(block, a.batch * groups * NPAN);
     if (bm.bh >= a.batch * groups * NPAN) return;
@@ -470,6 +552,23 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
     // a block whose keys are all padding has nothing to accumulate: it only stores its zeros
     const int ntiles = kb * ROWS >= pad_limit ? 0 : (a.seq + 63) / 64;
 
+    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane), lo_o = lane_off<W>(a.ld_o, wave, lane);
+    auto issue = [&](int t, int slot) {
+        unsigned char* st = smem + slot * STAGE;
+        const int qs = t * 64;
+#pragma unroll
+        for (int p = 0; p < NPAN; ++p) {
+            dma_tile64<W>(Q + p * 64, a.ld_qkv, qs, last, st + p * 8192, wave, lane, lo);
+            dma_tile64<W>(DO + p * 64, a.ld_o, qs, last, st + TILE + p * 8192, wave, lane, lo_o);
+        }
+        // extra loads, dealt to the waves: lse of the block's heads, then delta
+#pragma unroll
+        for (int j = 0; j < (OWN ? 1 : 2) * HP; ++j)
+            if (j % W == wave) dma_f32x64((j / HP ? DELTA : LSE) + (int64_t)(j % HP) * a.seq, qs, last, st + 2 * TILE + j * 256, lane);
+    };
+    const int t0 = q_begin + grp, iters = max(0, (ntiles - q_begin + G - 1) / G);
+    if (t0 < ntiles) issue(t0, 0);
+    if (t0 + G < ntiles) issue(t0 + G, 1);
     bf16x8 kf[4 * NPAN], vf[4 * NPAN];
     {
         const int64_t off = (int64_t)min(mykv, last) * a.ld_qkv + (lane >> 5) * 8;
@@ -485,22 +584,6 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
 #pragma unroll
         for (int r = 0; r < 16; ++r) dk[t][r] = dv[t][r] = 0.f;
 
-    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane), lo_o = lane_off<W>(a.ld_o, wave, lane);
-    auto issue = [&](int t, int slot) {
-        unsigned char* st = smem + slot * STAGE;
-        const int qs = t * 64;
-#pragma unroll
-        for (int p = 0; p < NPAN; ++p) {
-            dma_tile64<W>(Q + p * 64, a.ld_qkv, qs, last, st + p * 8192, wave, lane, lo);
-            dma_tile64<W>(DO + p * 64, a.ld_o, qs, last, st + TILE + p * 8192, wave, lane, lo_o);
-        }
-        // extra loads, dealt to the waves: lse of the block's heads, then delta
-#pragma unroll
-        for (int j = 0; j < (OWN ? 1 : 2) * HP; ++j)
-            if (j % W == wave) dma_f32x64((j / HP ? DELTA : LSE) + (int64_t)(j % HP) * a.seq, qs, last, st + 2 * TILE + j * 256, lane);
-    };
-
-    if (q_begin + grp < ntiles) issue(q_begin + grp, 0);
     const int own_rows = (a.seq + 63) / 64 * 64;     // of a head's deltas in LDS
     if constexpr (OWN) {
         // as the dQ kernel makes them, in its order of additions: a lane and its partner (lane ^ 32) have the halves of each
@@ -528,135 +611,141 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
         }
         // (the first tile's wait and barrier make them visible)
     }
-    for (int i = 0; q_begin + i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
-        const int t = q_begin + i * G + grp, slot = i & 1;
-        asm volatile("" ::: "memory");
-        if (t + G < ntiles) {
-            issue(t + G, slot ^ 1);
-            // the waves with extra loads wait for as many newer loads more than the others
-            constexpr int LOADS = 16 / W * NPAN, EXTRA = (OWN ? 1 : 2) * HP, EACH = EXTRA / W, MORE = EXTRA % W;
-            if (MORE == 0 || wave < MORE) wait_vm<LOADS + EACH + (MORE ? 1 : 0)>(); else wait_vm<LOADS + EACH>();
-        } else {
-            wait_vm<0>();
+    // the wave's sub-tiles of 32 queries: not those that all precede its keys, nor any for keys past the end or all padding
+    const int sub_begin = a.mask == BB_MASK_CAUSAL ? kv0 / 32 : 0, sub_end = kv0 >= pad_limit ? 0 : (a.seq + 31) / 32;
+    auto live = [&](int t, int u) { const int sub = t * 2 + u; return t < ntiles && sub >= sub_begin && sub < sub_end; };
+    f32x16 s[BUFS], dp;
+    // operands of the scores S and of their gradients dP, from LDS
+    bf16x8 fs[KS], fdp[KS];
+    auto fetch_scores = [&](const unsigned char* st, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) fs[k] = frag_kc(st + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+    };
+    auto fetch_grads = [&](const unsigned char* st, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) fdp[k] = frag_kc(st + TILE + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+    };
+    auto scores = [&](auto j_c) {
+        constexpr int hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[k], kf[hh * KS + k], s[n], 0, 0, 0);
+    };
+    auto score_grads = [&](auto j_c) {
+        constexpr int hh = decltype(j_c)::value % HP;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dp[r] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fdp[k], vf[hh * KS + k], dp, 0, 0, 0);
+    };
+    // P = exp2(S * c - lse[q]); rows q = acc_row(r), column kv = lane.  Only sub-tiles on the causal diagonal or past the last query
+    // mask per element; keys beyond the padding limit are whole lanes and are cleared once, after the loop.
+    auto probs = [&](const unsigned char* st, int t, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        const float* lse_t = (const float*)(st + 2 * TILE) + 64 * hh;
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+            const int ql = u * 32 + 8 * g4 + 4 * (lane >> 5);
+            const f32x4 l4 = *(const f32x4*)(lse_t + ql);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[n][g4 * 4 + e] = __builtin_amdgcn_exp2f(fmaf(s[n][g4 * 4 + e], a.scale_log2, -l4[e]));
         }
-        block_sync();
-        const unsigned char* qt = smem + slot * STAGE;
-        const unsigned char* dot = qt + TILE;
-        const float* lse_all = (const float*)(qt + 2 * TILE);
-        const float* del_all = lse_all + 64 * HP;
+        const int qs = t * 64 + u * 32;
+        if ((a.mask == BB_MASK_CAUSAL && qs < kv0 + 31) || qs + 32 > a.seq) {
+            asm volatile("" ::: "memory");  // a real branch: most sub-tiles skip it
+            const int qlane = qs + 4 * (lane >> 5);  // register r holds query qlane + 8*(r/4) + r%4
+            const int qmin = a.mask == BB_MASK_CAUSAL ? mykv : 0;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int qs = t * 64 + u * 32;
-            if (a.mask == BB_MASK_CAUSAL && qs + 31 < kv0) continue;  // all queries precede this wave's keys
-            if (qs >= a.seq) continue;   // (nor is there a tile past the last one)
-#pragma unroll
-          for (int hh = 0; hh < HP; ++hh) {
-            const float* lse_t = lse_all + 64 * hh;
-            const float* del_t = OWN ? (const float*)(smem_all + own_at) + hh * own_rows + t * 64 : del_all + 64 * hh;
-            const int head = head0 + hh;
-            // S[q][kv] and dP[q][kv]
-            f32x16 s, dp;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-#pragma unroll
-            for (int k = 0; k < KS; ++k) {
-                const int ks = hh * KS + k;
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_kc(qt + (ks >> 2) * 8192, u * 32, ks & 3, lane), kf[ks], s, 0, 0, 0);
-                dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_kc(dot + (ks >> 2) * 8192, u * 32, ks & 3, lane), vf[ks], dp, 0, 0, 0);
+            for (int r = 0; r < 16; ++r) {
+                const int q = qlane + 8 * (r >> 2) + (r & 3);
+                s[n][r] = q >= qmin && q < a.seq ? s[n][r] : 0.f;
             }
-            // P = exp2(S * c - lse[q]); dS = P * (dP - delta[q]); rows q = acc_row(r), column kv = lane.
-            // Only sub-tiles on the causal diagonal or past the last query mask per element; keys
-            // beyond the padding limit are whole lanes and are cleared once, after the loop.
-            const bool need_mask = (a.mask == BB_MASK_CAUSAL && qs < kv0 + 31) || qs + 32 > a.seq;
+        }
+    };
+    // dS = P * (dP - delta[q]), then dV^T += dO^T P~ ; dK^T += Q^T dS (contraction over the 32 queries of the sub-tile)
+    auto contract = [&](const unsigned char* st, int t, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        const float* del_t = OWN ? (const float*)(smem_all + own_at) + hh * own_rows + t * 64 : (const float*)(st + 2 * TILE) + 64 * HP + 64 * hh;
+        const int head = head0 + hh;
+        // dropout: dP = dP~ o mask / (1 - p) before it meets P; P itself is masked (into what multiplied V in
+        // the forward) only after dS has been formed from the unmasked probabilities
+        unsigned kept = 0u;   // bit r (sixteen booleans cost the registers that K, V and the sums leave)
+        if (DROP && a.drop.thresh) {
+            asm volatile("" ::: "memory");
+            const int qlane = t * 64 + u * 32 + 4 * (lane >> 5);
+            if (a.drop.small) {
+                // 32-bit indices; what is decided for a query past the end (masked out above) or a key past it (a whole
+                // lane, never stored) does not matter
+                const uint32_t i0 = ((uint32_t)(b * a.heads + head) * (uint32_t)a.seq + (uint32_t)qlane) * (uint32_t)a.seq + (uint32_t)mykv;
+                if (a.seq % 2 == 0) {
+                    // Rows start even: lanes 2j and 2j + 1 (keys 2j, 2j + 1) need the two halves of one hash in every row.
+                    // Of two rows the even lane hashes the first and the odd lane the second, and they exchange the
+                    // other's halves: a hash (two quarter-rate multiplies) per two decisions, as where the indices of a
+                    // lane are neighbours.  (Backward of 8 x 16 heads x 1024^2 probabilities: 238 us with a hash per decision,
+                    // 223 with this; 128-wide heads, 2 x 8 x 512^2 causal: 89 and 67.)
+                    const uint32_t own = (lane & 1) * 16, other = 16 - own;
+                    const uint32_t j0 = i0 + (lane & 1) * (uint32_t)a.seq;
+                    uint32_t km = 0u, kt = 0u;   // bit r: this lane's decision of its row, the neighbour's row
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int ql = u * 32 + 8 * g4 + 4 * (lane >> 5);
-                const f32x4 l4 = *(const f32x4*)(lse_t + ql);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s[g4 * 4 + e] = __builtin_amdgcn_exp2f(fmaf(s[g4 * 4 + e], a.scale_log2, -l4[e]));
-            }
-            if (need_mask) {
-                asm volatile("" ::: "memory");  // a real branch: most sub-tiles skip it
-                const int qlane = t * 64 + u * 32 + 4 * (lane >> 5);  // register r holds query qlane + 8*(r/4) + r%4
-                const int qmin = a.mask == BB_MASK_CAUSAL ? mykv : 0;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int q = qlane + 8 * (r >> 2) + (r & 3);
-                    s[r] = q >= qmin && q < a.seq ? s[r] : 0.f;
-                }
-            }
-            // dropout: dP = dP~ o mask / (1 - p) before it meets P; P itself is masked (into what multiplied V in
-            // the forward) only after dS has been formed from the unmasked probabilities
-            unsigned kept = 0u;   // bit r (sixteen booleans cost the registers that K, V and the sums leave)
-            if (DROP && a.drop.thresh) {
-                asm volatile("" ::: "memory");
-                const int qlane = t * 64 + u * 32 + 4 * (lane >> 5);
-                if (a.drop.small) {
-                    // 32-bit indices; what is decided for a query past the end (masked out above) or a key past it (a whole
-                    // lane, never stored) does not matter
-                    const uint32_t i0 = ((uint32_t)(b * a.heads + head) * (uint32_t)a.seq + (uint32_t)qlane) * (uint32_t)a.seq + (uint32_t)mykv;
-                    if (a.seq % 2 == 0) {
-                        // Rows start even: lanes 2j and 2j + 1 (keys 2j, 2j + 1) need the two halves of one hash in every row.
-                        // Of two rows the even lane hashes the first and the odd lane the second, and they exchange the
-                        // other's halves: a hash (two quarter-rate multiplies) per two decisions, as where the indices of a
-                        // lane are neighbours.  (Backward of 8 x 16 heads x 1024^2 probabilities: 238 us with a hash per decision,
-                        // 223 with this; 128-wide heads, 2 x 8 x 512^2 causal: 89 and 67.)
-                        const uint32_t own = (lane & 1) * 16, other = 16 - own;
-                        const uint32_t j0 = i0 + (lane & 1) * (uint32_t)a.seq;
-                        uint32_t km = 0u, kt = 0u;   // bit r: this lane's decision of its row, the neighbour's row
-#pragma unroll
-                        for (int r = 0; r < 16; r += 2) {
-                            const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, (j0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq) >> 1);
-                            const bool mine = ((x >> own) & 0xffffu) >= a.drop.thresh;
-                            const uint32_t sent = (uint32_t)__builtin_amdgcn_mov_dpp((int)((x >> other) & 0xffffu), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true);
-                            const bool theirs = sent >= a.drop.thresh;
-                            km |= mine ? 1u << r : 0u;
-                            kt |= theirs ? 1u << r : 0u;
-                        }
-                        kept = (lane & 1) ? km << 1 | kt : km | kt << 1;
-                    } else {
-#pragma unroll 2                        // (unrolled whole, this and the next loop cost the first one's registers)
-                        for (int r = 0; r < 16; ++r) {
-                            const uint32_t idx = i0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq;
-                            const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, idx >> 1);
-                            kept |= (((x >> ((idx & 1) * 16)) & 0xffffu) >= a.drop.thresh ? 1u : 0u) << r;
-                        }
+                    for (int r = 0; r < 16; r += 2) {
+                        const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, (j0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq) >> 1);
+                        const bool mine = ((x >> own) & 0xffffu) >= a.drop.thresh;
+                        const uint32_t sent = (uint32_t)__builtin_amdgcn_mov_dpp((int)((x >> other) & 0xffffu), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true);
+                        const bool theirs = sent >= a.drop.thresh;
+                        km |= mine ? 1u << r : 0u;
+                        kt |= theirs ? 1u << r : 0u;
                     }
+                    kept = (lane & 1) ? km << 1 | kt : km | kt << 1;
                 } else {
-#pragma unroll 1
+#pragma unroll 2                        // (unrolled whole, this and the next loop cost the first one's registers)
                     for (int r = 0; r < 16; ++r) {
-                        const int q = min(qlane + 8 * (r >> 2) + (r & 3), last);
-                        kept |= (bb_dropout_keep(a.drop.k0, a.drop.k1, a.drop.thresh, prob_index(a, b, head, q) + min(mykv, last)) ? 1u : 0u) << r;
+                        const uint32_t idx = i0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq;
+                        const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, idx >> 1);
+                        kept |= (((x >> ((idx & 1) * 16)) & 0xffffu) >= a.drop.thresh ? 1u : 0u) << r;
                     }
                 }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) dp[r] = (kept >> r) & 1u ? dp[r] * a.drop.scale : 0.f;
-            }
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int ql = u * 32 + 8 * g4 + 4 * (lane >> 5);
-                const f32x4 d4 = *(const f32x4*)(del_t + ql);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) dp[g4 * 4 + e] = s[g4 * 4 + e] * (dp[g4 * 4 + e] - d4[e]);
-            }
-            if (DROP && a.drop.thresh) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = (kept >> r) & 1u ? s[r] * a.drop.scale : 0.f;
-            }
-            // dV^T += dO^T P~ ; dK^T += Q^T dS   (contraction over the 32 queries of this sub-tile)
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const bf16x8 pf = pack_acc(s, kk), dsf = pack_acc(dp, kk);
-#pragma unroll
-                for (int d = 0; d < DT; ++d) {
-                    const int dt = hh * DT + d;
-                    dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(dot + fh * 8192, u * 32 + kk * 16, dt * 32, lane), pf, dv[dt], 0, 0, 0);
-                    dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(qt + fh * 8192, u * 32 + kk * 16, dt * 32, lane), dsf, dk[dt], 0, 0, 0);
+            } else {
+#pragma unroll 1
+                for (int r = 0; r < 16; ++r) {
+                    const int q = min(qlane + 8 * (r >> 2) + (r & 3), last);
+                    kept |= (bb_dropout_keep(a.drop.k0, a.drop.k1, a.drop.thresh, prob_index(a, b, head, q) + min(mykv, last)) ? 1u : 0u) << r;
                 }
             }
-          }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dp[r] = (kept >> r) & 1u ? dp[r] * a.drop.scale : 0.f;
         }
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+            const int ql = u * 32 + 8 * g4 + 4 * (lane >> 5);
+            const f32x4 d4 = *(const f32x4*)(del_t + ql);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dp[g4 * 4 + e] = s[n][g4 * 4 + e] * (dp[g4 * 4 + e] - d4[e]);
+        }
+        if (DROP && a.drop.thresh) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[n][r] = (kept >> r) & 1u ? s[n][r] * a.drop.scale : 0.f;
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            if (PIPE && kk) __builtin_amdgcn_sched_barrier(0);   // (the fragments of both halves at once find no registers)
+            const bf16x8 pf = pack_acc(s[n], kk), dsf = pack_acc(dp, kk);
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const int dt = hh * DT + d;
+                dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + TILE + fh * 8192, u * 32 + kk * 16, dt * 32, lane), pf, dv[dt], 0, 0, 0);
+                dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + fh * 8192, u * 32 + kk * 16, dt * 32, lane), dsf, dk[dt], 0, 0, 0);
+            }
+        }
+    };
+    if (iters > 0) {
+        asm volatile("" ::: "memory");
+        wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
+        attn_bwd_walk<HP, G, STAGES, STAGE, PIPE>(smem, t0, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
         // the groups' sums, first dV, then dK (one after the other: together they would not find room)
@@ -711,8 +800,10 @@ template <bool DROP, int HP, int NPAN, int W, int G>
 __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int block, unsigned char* smem_all) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
-    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % W, grp = G == 1 ? 0 : (tid >> 6) / W;
-    unsigned char* smem = smem_all + grp * (4 * TILE);
+    constexpr bool PIPE = attn_bwd_pipe(NPAN);
+    constexpr int STAGES = attn_bwd_stages(NPAN, G), BUFS = PIPE ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = uw % W, grp = G == 1 ? 0 : uw / W;
+    unsigned char* smem = smem_all + grp * (STAGES * 2 * TILE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(block, a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
@@ -734,6 +825,18 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
     const int my_limit = kv_limit(a, b, myq);
     const int wave_min_limit = kv_limit(a, b, q0);  // limits grow with the query index
 
+    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
+    auto issue = [&](int t, int slot) {
+        unsigned char* st = smem + slot * (2 * TILE);
+        const int kv0 = t * 64;
+#pragma unroll
+        for (int p = 0; p < NPAN; ++p) {
+            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
+            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
+        }
+    };
+    if (grp < ntiles) issue(grp, 0);
+    if (grp + G < ntiles) issue(grp + G, 1);
     bf16x8 qf[4 * NPAN], dof[4 * NPAN];
     {
         const int64_t r = min(myq, last);
@@ -773,75 +876,75 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq[t][r] = 0.f;
 
-    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
-    auto issue = [&](int t, int slot) {
-        unsigned char* st = smem + slot * (2 * TILE);
-        const int kv0 = t * 64;
+    // the wave's sub-tiles of 32 keys: up to the last one that some query of it may see, none for queries past the end
+    const int sub_end = q0 >= a.seq ? 0 : a.mask == BB_MASK_CAUSAL ? q0 / 32 + 1 : (kv_end + 31) / 32;
+    auto live = [&](int t, int u) { return t < ntiles && t * 2 + u < sub_end; };
+    f32x16 s[BUFS], dp;
+    // operands of the scores S and of their gradients dP, from LDS
+    bf16x8 fs[KS], fdp[KS];
+    auto fetch_scores = [&](const unsigned char* st, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
 #pragma unroll
-        for (int p = 0; p < NPAN; ++p) {
-            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
-            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
+        for (int k = 0; k < KS; ++k) fs[k] = frag_kc(st + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+    };
+    auto fetch_grads = [&](const unsigned char* st, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) fdp[k] = frag_kc(st + TILE + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+    };
+    auto scores = [&](auto j_c) {
+        constexpr int hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[k], qf[hh * KS + k], s[n], 0, 0, 0);
+    };
+    auto score_grads = [&](auto j_c) {
+        constexpr int hh = decltype(j_c)::value % HP;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dp[r] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fdp[k], dof[hh * KS + k], dp, 0, 0, 0);
+    };
+    auto probs = [&](const unsigned char*, int t, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        const int kv = t * 64 + u * 32;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] = __builtin_amdgcn_exp2f(fmaf(s[n][r], a.scale_log2, -my_lse[hh]));
+        if (kv + 32 > wave_min_limit) {
+            asm volatile("" ::: "memory");  // a real branch: only tiles on the mask boundary pay for it
+            const int lim = my_limit - kv - 4 * (lane >> 5);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[n][r] = 8 * (r >> 2) + (r & 3) < lim ? s[n][r] : 0.f;
         }
     };
-    if (grp < ntiles) issue(grp, 0);
-    for (int i = 0; i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
-        const int t = i * G + grp, slot = i & 1;
-        asm volatile("" ::: "memory");
-        if (t + G < ntiles) {
-            issue(t + G, slot ^ 1);
-            wait_vm<16 / W * NPAN>();
-        } else {
-            wait_vm<0>();
+    auto contract = [&](const unsigned char* st, int t, auto j_c) {
+        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        if (DROP && a.drop.thresh) {
+            asm volatile("" ::: "memory");
+            const uint64_t base = prob_index(a, b, head0 + hh, min(myq, last)) + t * 64 + u * 32;
+            drop_acc_rows(a.drop, base, lane, dp);
         }
-        block_sync();
-        const unsigned char* kt = smem + slot * (2 * TILE);
-        const unsigned char* vt = kt + TILE;
-        const int kv0 = t * 64;
-        const bool active = (G == 1 || t < ntiles) && !(a.mask == BB_MASK_CAUSAL && kv0 > q0 + 31);
-        if (active) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+        for (int r = 0; r < 16; ++r) dp[r] = s[n][r] * (dp[r] - my_delta[hh]);
+        // dQ^T += K^T dS^T (contraction over the 32 keys of this sub-tile)
 #pragma unroll
-              for (int hh = 0; hh < HP; ++hh) {
-                const int head = head0 + hh;
-                f32x16 s, dp;
+        for (int kk = 0; kk < 2; ++kk) {
+            const bf16x8 dsf = pack_acc(dp, kk);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-#pragma unroll
-                for (int k = 0; k < KS; ++k) {
-                    const int ks = hh * KS + k;
-                    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_kc(kt + (ks >> 2) * 8192, u * 32, ks & 3, lane), qf[ks], s, 0, 0, 0);
-                    dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_kc(vt + (ks >> 2) * 8192, u * 32, ks & 3, lane), dof[ks], dp, 0, 0, 0);
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], a.scale_log2, -my_lse[hh]));
-                if (kv0 + u * 32 + 32 > wave_min_limit) {
-                    asm volatile("" ::: "memory");  // a real branch: only tiles on the mask boundary pay for it
-                    const int lim = my_limit - kv0 - u * 32 - 4 * (lane >> 5);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) < lim ? s[r] : 0.f;
-                }
-                if (DROP && a.drop.thresh) {
-                    asm volatile("" ::: "memory");
-                    const uint64_t base = prob_index(a, b, head, min(myq, last)) + kv0 + u * 32;
-                    drop_acc_rows(a.drop, base, lane, dp);
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) dp[r] = s[r] * (dp[r] - my_delta[hh]);
-                // dQ^T += K^T dS^T (contraction over the 32 keys of this sub-tile)
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) {
-                    const bf16x8 dsf = pack_acc(dp, kk);
-#pragma unroll
-                    for (int d = 0; d < DT; ++d) {
-                        const int dt = hh * DT + d;
-                        dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(kt + (dt >> 1) * 8192, u * 32 + kk * 16, (dt & 1) * 32, lane), dsf, dq[dt], 0, 0, 0);
-                    }
-                }
-              }
+            for (int d = 0; d < DT; ++d) {
+                const int dt = hh * DT + d;
+                dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + (dt >> 1) * 8192, u * 32 + kk * 16, (dt & 1) * 32, lane), dsf, dq[dt], 0, 0, 0);
             }
         }
+    };
+    const int iters = (ntiles + G - 1) / G;
+    if (iters > 0) {
+        asm volatile("" ::: "memory");
+        wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
+        attn_bwd_walk<HP, G, STAGES, 2 * TILE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
         float* parts = (float*)smem_all;
@@ -911,8 +1014,8 @@ static int check_attn(const char* name, int dtype, int mask, int batch, int head
 }
 
 // LDS: the rings, or what the groups leave for each other
-template <int HP, int NPAN, int W, int G> constexpr size_t attn_lds(bool dkv) {
-    const size_t ring = G * (dkv ? 2 * (2 * NPAN * 8192 + 512 * HP) : 4 * NPAN * 8192);
+template <int HP, int NPAN, int W, int G> constexpr size_t attn_lds(bool bwd, bool dkv) {
+    const size_t ring = G * (size_t)(bwd ? attn_bwd_stages(NPAN, G) : 2) * (2 * NPAN * 8192 + (dkv ? 512 * HP : 0));
     const size_t parts = G == 1 ? 0 : (size_t)W * G * ((dkv ? 2 : 2 * NPAN) * 4096 + (dkv ? 0 : HP * 512));
     return ring > parts ? ring : parts;
 }
@@ -926,19 +1029,19 @@ template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int
 struct attn_fwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_fwd_kernel<true, HP, NPAN, W, G> : attn_fwd_kernel<false, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(false), a, st);
+        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(false, false), a, st);
     }
 };
 struct attn_dq_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_bwd_dq_kernel<true, HP, NPAN, W, G> : attn_bwd_dq_kernel<false, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(false), a, st);
+        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(true, false), a, st);
     }
 };
 struct attn_dkv_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_bwd_dkv_kernel<true, HP, NPAN, W, G> : attn_bwd_dkv_kernel<false, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh * NPAN, W * G * 64, attn_lds<HP, NPAN, W, G>(true), a, st);   // 128-wide heads: a block per half
+        return attn_go(kern, seq, W * 32, nbh * NPAN, W * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);   // 128-wide heads: a block per half
     }
 };
 // Both backward kernels: in one launch where all blocks of the two find room at once (two blocks of four waves a CU, one of eight),
@@ -959,7 +1062,7 @@ struct attn_bwd_launch {
             return rc ? rc : attn_dkv_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
         }
         const unsigned dkv = attn_grid(seq, W * 32, nbh * NPAN), dq = attn_grid(seq, W * 32, nbh);
-        constexpr size_t own_at = attn_lds<HP, NPAN, W, G>(true) > attn_lds<HP, NPAN, W, G>(false) ? attn_lds<HP, NPAN, W, G>(true) : attn_lds<HP, NPAN, W, G>(false);
+        constexpr size_t own_at = attn_lds<HP, NPAN, W, G>(true, true) > attn_lds<HP, NPAN, W, G>(true, false) ? attn_lds<HP, NPAN, W, G>(true, true) : attn_lds<HP, NPAN, W, G>(true, false);
         const size_t lds = own_at + (size_t)HP * ((seq + 63) / 64 * 64) * sizeof(float);
         auto kern = a.drop.thresh ? attn_bwd_kernel<true, HP, NPAN, W, G> : attn_bwd_kernel<false, HP, NPAN, W, G>;
         BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));
