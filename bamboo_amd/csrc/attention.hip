@@ -12,9 +12,10 @@
 // COLUMN per lane: scores are produced transposed (S^T = K Q^T), so the softmax reductions over
 // keys are in-lane plus one cross-half shuffle, and P^T comes out of the accumulators already
 // in the register layout the next MFMA wants as its B operand.  With 32-wide heads (HP = 2) a block
-// owns a PAIR of neighbouring heads, whose columns together are one 64-wide slice: the tiles in LDS,
-// their loads and the fragment layout are those of one 64-wide head, every product takes the k-steps
-// (scores) or the output tile (context, gradients) of its head, the softmax runs once per head.
+// owns a PAIR of neighbouring heads, whose columns together are one 64-wide slice: the tiles in LDS and
+// their loads are those of one 64-wide head, each head has waves of its own, which take the k-steps
+// (scores) and the output tile (context, gradients) of that head.  (Waves that took one head after the
+// other: 8 x 8 pairs, 128 keys, dropout 9.3 us forward, 15.8 backward; so 8.6 and 13.1.)
 // Operands that are contracted
 // over their row index (V in O = PV, Q and dO in dK/dV, K in dQ) are read from LDS with
 // ds_read_b64_tr_b16.  Tiles travel global -> LDS by DMA (global_load_lds_dwordx4),
@@ -176,6 +177,12 @@ __device__ __forceinline__ void drop_acc_rows(const DropKey& k, uint64_t base, i
     }
 }
 
+// the value of lane ^ 32
+__device__ __forceinline__ float other_half(float v) {
+    typedef __attribute__((ext_vector_type(2))) unsigned u2;
+    const u2 w = __builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    return __uint_as_float((threadIdx.x & 32) ? w[0] : w[1]);
+}
 template <int N> __device__ __forceinline__ void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
 }
@@ -210,31 +217,32 @@ static unsigned attn_grid(int seq, int rows, int nbh) { return (unsigned)(8 * ((
 // grid gives every CU more than one block; below that what bounds a launch is a wave's walk over its tiles with nobody beside it on
 // its SIMD, so the walk is shared, and where half the CUs had no block the blocks are halved too (measured: see attn_shape).
 // this wave's column tiles of those the other groups have for the same rows: parts holds [group][wave][tiles][16][64] floats
-template <int W, int G, int T> __device__ __forceinline__ void attn_park(float* parts, int grp, int w, int lane, const f32x16 (&v)[T]) {
+template <int DW, int G, int T> __device__ __forceinline__ void attn_park(float* parts, int grp, int w, int lane, const f32x16 (&v)[T]) {
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) parts[(((grp * W + w) * T + t) * 16 + r) * 64 + lane] = v[t][r];
+        for (int r = 0; r < 16; ++r) parts[(((grp * DW + w) * T + t) * 16 + r) * 64 + lane] = v[t][r];
 }
 
 // =========================================================================================
 // forward: block = 128 queries (4 waves x 32; W, G: see above), loop over 64-key tiles
 // =========================================================================================
-// HP: heads per block (1: one head, 2: a pair of 32-wide heads); NPAN: 64-wide column panels of a head (1; 2 for
+// HP: heads per block (1: one head, 2: a pair of 32-wide heads, W waves each); NPAN: 64-wide column panels of a head (1; 2 for
 // 128-wide heads, HP = 1: a tile in LDS is then two [64][64] panels behind each other, each in the format above);
 // KS k-steps of a head's scores, DT 32-wide output tiles of a head
 template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 1) ? 4 : 2) void attn_fwd_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(W * HP * G * 64, (!DROP && NPAN == 1 && G == 1) ? 4 : 2) void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
-    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];  // G rings of 2 stages x (K, V)
-    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = uw % W, grp = G == 1 ? 0 : uw / W;
+    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];  // G rings of 2 stages of K, then 2 of V
+    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), dw = uw % DW, grp = G == 1 ? 0 : uw / DW;
+    const int wave = dw % W, hh = HP == 1 ? 0 : dw / W;     // rows and head of the pair; of a tile's transfers, the part dw
     unsigned char* smem = smem_all + grp * (4 * TILE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(blockIdx.x, a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
     const int qb = (a.seq + ROWS - 1) / ROWS - 1 - bm.rank;  // long (late) query blocks first
-    const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP;
+    const int b = bm.bh / groups, hg = bm.bh % groups, head = hg * HP + hh;
     const int64_t row_base = (int64_t)b * a.seq;
     const bf16* Q = a.q + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* K = a.k + row_base * a.ld_qkv + hg * (64 * NPAN);
@@ -247,190 +255,174 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
     int kv_end = a.seq;
     if (a.mask == BB_MASK_CAUSAL) kv_end = min(a.seq, qb * ROWS + ROWS);
     else if (a.mask == BB_MASK_KEY_PADDING) kv_end = min(a.seq, a.key_len[b]);
-    const int ntiles = (kv_end + 63) / 64;
+    const int ntiles = (kv_end + 63) / 64, iters = (ntiles + G - 1) / G;
     const int my_limit = kv_limit(a, b, myq);
     const int wave_min_limit = kv_limit(a, b, q0);  // limits grow with the query index
+    // waves whose queries all precede a tile have nothing to add (causal), nor have those past the end
+    const int live_tiles = q0 >= a.seq ? 0 : a.mask == BB_MASK_CAUSAL ? min(ntiles, (q0 + 31) / 64 + 1) : ntiles;
 
-    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
-    auto issue = [&](int t, int slot) {
-        unsigned char* st = smem + slot * (2 * TILE);
-        const int kv0 = t * 64;
+    const LaneOff<DW> lo = lane_off<DW>(a.ld_qkv, dw, lane);
+    auto issue = [&](const bf16* src, int t, unsigned char* to) {
 #pragma unroll
-        for (int p = 0; p < NPAN; ++p) {
-            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
-            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
-        }
+        for (int p = 0; p < NPAN; ++p) dma_tile64<DW>(src + p * 64, a.ld_qkv, t * 64, last, to + p * 8192, dw, lane, lo);
     };
-
-    if (grp < ntiles) issue(grp, 0);
-    bf16x8 qf[4 * NPAN];
+    auto issue_k = [&](int t, int slot) { if (t < ntiles) issue(K, t, smem + slot * TILE); };
+    auto issue_v = [&](int t, int slot) { if (t < ntiles) issue(V, t, smem + (2 + slot) * TILE); };
+    issue_k(grp, 0);
+    issue_v(grp, 0);
+    bf16x8 qf[KS];
     {
-        const bf16* qp = Q + (int64_t)min(myq, last) * a.ld_qkv + (lane >> 5) * 8;
+        const bf16* qp = Q + (int64_t)min(myq, last) * a.ld_qkv + hh * 32 + (lane >> 5) * 8;
 #pragma unroll
-        for (int ks = 0; ks < 4 * NPAN; ++ks) qf[ks] = *(const bf16x8*)(qp + ks * 16);
+        for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const bf16x8*)(qp + ks * 16);
     }
-    f32x16 o[2 * NPAN];
+    f32x16 o[DT];
 #pragma unroll
-    for (int t = 0; t < 2 * NPAN; ++t)
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
-    float m[HP], lsum[HP];
+    float m = -INFINITY, lsum = 0.f;
+
+    auto scores = [&](const unsigned char* kt, f32x16 (&s)[2]) {
 #pragma unroll
-    for (int hh = 0; hh < HP; ++hh) {
-        m[hh] = -INFINITY;
-        lsum[hh] = 0.f;
-    }
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[u][r] = 0.f;
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const int ks = hh * 2 + k;   // k-step ks: panel ks / 4, step ks % 4 inside it
+                s[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_kc(kt + (ks >> 2) * 8192, u * 32, ks & 3, lane), qf[k], s[u], 0, 0, 0);
+            }
+        }
+    };
+    // masking only on tiles that reach past the first key some query of this wave may not see
+    auto mask_tile = [&](int kv0, f32x16 (&s)[2]) {
+        if (kv0 + 64 > wave_min_limit) {
+            asm volatile("" ::: "memory");   // a real branch
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int kv = kv0 + u * 32 + acc_row(r, lane);
+                    s[u][r] = kv < my_limit ? s[u][r] : -INFINITY;
+                }
+        }
+    };
+    auto add_tile = [&](const unsigned char* vt, int kv0, f32x16 (&s)[2]) {
+        // running max on the raw scores (the scale is positive)
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[u][r]);
+        tmax = fmaxf(tmax, other_half(tmax)) * a.scale_log2;
+        const float mnew = fmaxf(m, tmax);
+        const float msafe = mnew == -INFINITY ? 0.f : mnew;
+        const float alpha = __builtin_amdgcn_exp2f(m - msafe);  // m = -inf -> 0
+        float psum = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(s[u][r], a.scale_log2, -msafe));
+                s[u][r] = p;
+                psum += p;
+            }
+        lsum = lsum * alpha + psum;
+        m = mnew;
+        if (DROP && a.drop.thresh) {   // the normaliser takes every probability, the context only the kept ones
+            const uint64_t base = prob_index(a, b, head, min(myq, last)) + kv0;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) drop_acc_rows(a.drop, base + u * 32, lane, s[u]);
+        }
+        if (__any(alpha != 1.0f)) {  // wave-uniform: once the maxima have settled nothing is rescaled
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+        }
+        // O^T += V^T P^T
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const bf16x8 pf = pack_acc(s[kk >> 1], kk & 1);
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const int dt = hh + d;   // output tile dt: panel dt / 2, columns (dt % 2) * 32 inside it
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(vt + (dt >> 1) * 8192, kk * 16, (dt & 1) * 32, lane), pf, o[d], 0, 0, 0);
+            }
+        }
+    };
 
     // The first tile and the queries: waited for in full, or the compiler, which counts its own loads only, puts the waits for the
     // queries into the loop, where they hold for the transfers of the next tile (8 x 16 heads of 64, 1024 causal 37.7 -> 34.6 us).
     asm volatile("" ::: "memory");
     wait_vm<0>();
-    for (int i = 0; i * G < ntiles; ++i) {   // the barriers are the block's: every group goes round as often
+    for (int i = 0; i < iters; ++i) {   // the barriers are the block's: every group goes round as often
         const int t = i * G + grp, slot = i & 1;
         asm volatile("" ::: "memory");
         if (t + G < ntiles) {
-            issue(t + G, slot ^ 1);
-            wait_vm<16 / W * NPAN>();
+            issue_k(t + G, slot ^ 1);
+            issue_v(t + G, slot ^ 1);
+            wait_vm<16 / DW * NPAN>();
         } else {
             wait_vm<0>();
         }
         block_sync();
-        const unsigned char* kt = smem + slot * (2 * TILE);
-        const unsigned char* vt = kt + TILE;
-        const int kv0 = t * 64;
-        // waves whose queries all precede this tile have nothing to add (causal)
-        const bool active = (G == 1 || t < ntiles) && !(a.mask == BB_MASK_CAUSAL && kv0 > q0 + 31);
-        if (active) {
-#pragma unroll
-          for (int hh = 0; hh < HP; ++hh) {
+        if (t < live_tiles) {
             f32x16 s[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[u][r] = 0.f;
-#pragma unroll
-                for (int k = 0; k < KS; ++k) {
-                    const int ks = hh * KS + k;   // k-step ks: panel ks / 4, step ks % 4 inside it
-                    s[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_kc(kt + (ks >> 2) * 8192, u * 32, ks & 3, lane), qf[ks], s[u], 0, 0, 0);
-                }
-            }
-            // running max on the raw scores (the scale is positive), masking only on tiles that
-            // reach past the first key some query of this wave may not see
-            const bool need_mask = kv0 + 64 > wave_min_limit;
-            float tmax = -INFINITY;
-            if (need_mask) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int kv = kv0 + u * 32 + acc_row(r, lane);
-                        s[u][r] = kv < my_limit ? s[u][r] : -INFINITY;
-                    }
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[u][r]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * a.scale_log2;
-            const float mnew = fmaxf(m[hh], tmax);
-            const float msafe = mnew == -INFINITY ? 0.f : mnew;
-            const float alpha = __builtin_amdgcn_exp2f(m[hh] - msafe);  // m = -inf -> 0
-            float psum = 0.f;
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(fmaf(s[u][r], a.scale_log2, -msafe));
-                    s[u][r] = p;
-                    psum += p;
-                }
-            lsum[hh] = lsum[hh] * alpha + psum;
-            m[hh] = mnew;
-            if (DROP && a.drop.thresh) {   // the normaliser takes every probability, the context only the kept ones
-                const uint64_t base = prob_index(a, b, head0 + hh, min(myq, last)) + kv0;
-#pragma unroll
-                for (int u = 0; u < 2; ++u) drop_acc_rows(a.drop, base + u * 32, lane, s[u]);
-            }
-            if (__any(alpha != 1.0f)) {  // wave-uniform: once the maxima have settled nothing is rescaled
-#pragma unroll
-                for (int d = 0; d < DT; ++d)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[hh * DT + d][r] *= alpha;
-            }
-            // O^T += V^T P^T
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                const bf16x8 pf = pack_acc(s[kk >> 1], kk & 1);
-#pragma unroll
-                for (int d = 0; d < DT; ++d) {
-                    const int dt = hh * DT + d;   // output tile dt: panel dt / 2, columns (dt % 2) * 32 inside it
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(vt + (dt >> 1) * 8192, kk * 16, (dt & 1) * 32, lane), pf, o[dt], 0, 0, 0);
-                }
-            }
-          }
+            scores(smem + slot * TILE, s);
+            mask_tile(t * 64, s);
+            add_tile(smem + (2 + slot) * TILE, t * 64, s);
         }
         block_sync();
     }
     if constexpr (G > 1) {
-        // each group's context against the maximum of all of them; the first 2 NPAN groups finish a column tile each
-        float* stats = (float*)smem_all + W * G * (2 * NPAN) * 1024;   // [group][wave][HP][m, sum][64]
-        attn_park<W, G>((float*)smem_all, grp, wave, lane, o);
-#pragma unroll
-        for (int hh = 0; hh < HP; ++hh) {
-            stats[(((grp * W + wave) * HP + hh) * 2) * 64 + lane] = m[hh];
-            stats[(((grp * W + wave) * HP + hh) * 2 + 1) * 64 + lane] = lsum[hh];
-        }
+        // each group's context against the maximum of all of them; the first DT groups finish a column tile each
+        float* stats = (float*)smem_all + DW * G * DT * 1024;   // [group][wave][m, sum][64]
+        attn_park<DW, G>((float*)smem_all, grp, dw, lane, o);
+        stats[((grp * DW + dw) * 2) * 64 + lane] = m;
+        stats[((grp * DW + dw) * 2 + 1) * 64 + lane] = lsum;
         __syncthreads();
-        float scale[G][HP];
+        float scale[G];
+        float all = -INFINITY, sum = 0.f;
 #pragma unroll
-        for (int hh = 0; hh < HP; ++hh) {
-            float all = -INFINITY, sum = 0.f;
+        for (int g = 0; g < G; ++g) all = fmaxf(all, stats[((g * DW + dw) * 2) * 64 + lane]);
+        const float safe = all == -INFINITY ? 0.f : all;
 #pragma unroll
-            for (int g = 0; g < G; ++g) all = fmaxf(all, stats[(((g * W + wave) * HP + hh) * 2) * 64 + lane]);
-            const float safe = all == -INFINITY ? 0.f : all;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                scale[g][hh] = __builtin_amdgcn_exp2f(stats[(((g * W + wave) * HP + hh) * 2) * 64 + lane] - safe);
-                sum += stats[(((g * W + wave) * HP + hh) * 2 + 1) * 64 + lane] * scale[g][hh];
-            }
-            m[hh] = all;
-            lsum[hh] = sum;
+        for (int g = 0; g < G; ++g) {
+            scale[g] = __builtin_amdgcn_exp2f(stats[((g * DW + dw) * 2) * 64 + lane] - safe);
+            sum += stats[((g * DW + dw) * 2 + 1) * 64 + lane] * scale[g];
         }
+        m = all;
+        lsum = sum;
 #pragma unroll
-        for (int dt = 0; dt < 2 * NPAN; ++dt) {
+        for (int dt = 0; dt < DT; ++dt) {
             if (dt % G != grp) continue;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 float v = 0.f;
 #pragma unroll
-                for (int g = 0; g < G; ++g) v += ((float*)smem_all)[(((g * W + wave) * (2 * NPAN) + dt) * 16 + r) * 64 + lane] * scale[g][dt / DT];
+                for (int g = 0; g < G; ++g) v += ((float*)smem_all)[(((g * DW + dw) * DT + dt) * 16 + r) * 64 + lane] * scale[g];
                 o[dt][r] = v;
             }
         }
     }
-    float inv[HP];
-#pragma unroll
-    for (int hh = 0; hh < HP; ++hh) {
-        lsum[hh] += __shfl_xor(lsum[hh], 32, 64);
-        inv[hh] = lsum[hh] > 0.f ? 1.0f / lsum[hh] : 0.f;
-    }
+    lsum += other_half(lsum);
+    const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
     if (myq < a.seq) {
-        bf16* op = a.out + (row_base + myq) * a.ld_o + hg * (64 * NPAN);
+        bf16* op = a.out + (row_base + myq) * a.ld_o + hg * (64 * NPAN) + hh * 32;
 #pragma unroll
-        for (int dt = 0; dt < 2 * NPAN; ++dt) {
+        for (int dt = 0; dt < DT; ++dt) {
             if (dt % G != grp) continue;
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int d = dt * 32 + 8 * g4 + 4 * (lane >> 5);
-                const float iv = inv[dt / DT];
-                u32x2 w = {pack2bf(o[dt][g4 * 4] * iv, o[dt][g4 * 4 + 1] * iv),
-                           pack2bf(o[dt][g4 * 4 + 2] * iv, o[dt][g4 * 4 + 3] * iv)};
+                u32x2 w = {pack2bf(o[dt][g4 * 4] * inv, o[dt][g4 * 4 + 1] * inv),
+                           pack2bf(o[dt][g4 * 4 + 2] * inv, o[dt][g4 * 4 + 3] * inv)};
                 *(u32x2*)(op + d) = w;
             }
         }
-#pragma unroll
-        for (int hh = 0; hh < HP; ++hh)
-            if (lane < 32 && grp == 0) a.lse[((int64_t)b * a.heads + head0 + hh) * a.seq + myq] = m[hh] + log2f(lsum[hh]);
+        if (lane < 32 && grp == 0) a.lse[((int64_t)b * a.heads + head) * a.seq + myq] = m + log2f(lsum);
     }
 }
 
@@ -447,10 +439,9 @@ __global__ __launch_bounds__(W * G * 64, (!DROP && NPAN == 1 && HP == 1 && G == 
 constexpr bool attn_bwd_pipe(int npan) { return npan == 1; }
 // stages of a ring: three where a tile's last products come behind the barrier that hands the next tile out, two where three do not fit
 constexpr int attn_bwd_stages(int npan, int g) { return npan == 1 && g <= 2 ? 3 : 2; }
-template <int HP, int G, int STAGES, int STAGE, bool PIPE, typename Live, typename FetchS, typename FetchG, typename Scores, typename Grads, typename Probs, typename Contract, typename Issue>
+template <int G, int STAGES, int STAGE, bool PIPE, typename Live, typename FetchS, typename FetchG, typename Scores, typename Grads, typename Probs, typename Contract, typename Issue>
 __device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int iters, const Live& live, const FetchS& fetch_scores, const FetchG& fetch_grads, const Scores& scores, const Grads& score_grads,
                                               const Probs& probs, const Contract& contract, const Issue& issue) {
-    constexpr int J = 2 * HP;      // sub-tiles of a tile, heads of a pair one after the other
     using First = std::integral_constant<int, 0>;
     int stage = 0;
     auto begin = [&](const unsigned char* st, auto j_c) {      // a wave's first sub-tile, or the first behind a turn it could not look past
@@ -477,10 +468,10 @@ __device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int it
         };
         auto step = [&](auto j_c) {
             constexpr int j = decltype(j_c)::value;
-            constexpr bool LAST = j == J - 1;
+            constexpr bool LAST = j == 1;
             constexpr bool BEHIND = LAST && STAGES == 2;      // the next tile comes in behind the last products of this one
             using Next = std::integral_constant<int, LAST ? 0 : j + 1>;
-            const bool run = live(t, j / HP), next = LAST ? i + 1 < iters && live(t + G, 0) : live(t, (j + 1) / HP);
+            const bool run = live(t, j), next = LAST ? i + 1 < iters && live(t + G, 0) : live(t, j + 1);
             if constexpr (PIPE && LAST && STAGES == 3) turn();
             const unsigned char* st_next = LAST ? st_after : st;
             if (run) {
@@ -504,10 +495,6 @@ __device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int it
         };
         step(std::integral_constant<int, 0>{});
         step(std::integral_constant<int, 1>{});
-        if constexpr (HP == 2) {
-            step(std::integral_constant<int, 2>{});
-            step(std::integral_constant<int, 3>{});
-        }
         stage = after;
     }
 }
@@ -522,18 +509,19 @@ __device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int it
 template <bool DROP, int HP, int NPAN, int W, int G, bool OWN>
 __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int block, unsigned char* smem_all, const int own_at) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
-    constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192, ROWS = W * 32;
+    constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
     // per group STAGES x (Q tile, dO tile: 8 KiB per panel, lse 256 B per head, delta 256 B per head)
     constexpr bool PIPE = attn_bwd_pipe(NPAN);
     constexpr int STAGE = 2 * TILE + 512 * HP, STAGES = attn_bwd_stages(NPAN, G), BUFS = PIPE ? 2 : 1;
-    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = uw % W, grp = G == 1 ? 0 : uw / W;
+    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), dw = uw % DW, grp = G == 1 ? 0 : uw / DW;
+    const int wave = dw % W, hh = HP == 1 ? 0 : dw / W;
     unsigned char* smem = smem_all + grp * (STAGES * STAGE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(block, a.batch * groups * NPAN);
     if (bm.bh >= a.batch * groups * NPAN) return;
     const int kb = bm.rank;  // early key blocks are seen by the most queries
     const int fh = bm.bh % NPAN, bg = bm.bh / NPAN;
-    const int b = bg / groups, hg = bg % groups, head0 = hg * HP;
+    const int b = bg / groups, hg = bg % groups, head0 = hg * HP, head = head0 + hh;
     const int64_t row_base = (int64_t)b * a.seq;
     const bf16* Q = a.q + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* K = a.k + row_base * a.ld_qkv + hg * (64 * NPAN);
@@ -552,35 +540,35 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
     // a block whose keys are all padding has nothing to accumulate: it only stores its zeros
     const int ntiles = kb * ROWS >= pad_limit ? 0 : (a.seq + 63) / 64;
 
-    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane), lo_o = lane_off<W>(a.ld_o, wave, lane);
+    const LaneOff<DW> lo = lane_off<DW>(a.ld_qkv, dw, lane), lo_o = lane_off<DW>(a.ld_o, dw, lane);
     auto issue = [&](int t, int slot) {
         unsigned char* st = smem + slot * STAGE;
         const int qs = t * 64;
 #pragma unroll
         for (int p = 0; p < NPAN; ++p) {
-            dma_tile64<W>(Q + p * 64, a.ld_qkv, qs, last, st + p * 8192, wave, lane, lo);
-            dma_tile64<W>(DO + p * 64, a.ld_o, qs, last, st + TILE + p * 8192, wave, lane, lo_o);
+            dma_tile64<DW>(Q + p * 64, a.ld_qkv, qs, last, st + p * 8192, dw, lane, lo);
+            dma_tile64<DW>(DO + p * 64, a.ld_o, qs, last, st + TILE + p * 8192, dw, lane, lo_o);
         }
         // extra loads, dealt to the waves: lse of the block's heads, then delta
 #pragma unroll
         for (int j = 0; j < (OWN ? 1 : 2) * HP; ++j)
-            if (j % W == wave) dma_f32x64((j / HP ? DELTA : LSE) + (int64_t)(j % HP) * a.seq, qs, last, st + 2 * TILE + j * 256, lane);
+            if (j % DW == dw) dma_f32x64((j / HP ? DELTA : LSE) + (int64_t)(j % HP) * a.seq, qs, last, st + 2 * TILE + j * 256, lane);
     };
     const int t0 = q_begin + grp, iters = max(0, (ntiles - q_begin + G - 1) / G);
     if (t0 < ntiles) issue(t0, 0);
     if (t0 + G < ntiles) issue(t0 + G, 1);
-    bf16x8 kf[4 * NPAN], vf[4 * NPAN];
+    bf16x8 kf[KS], vf[KS];
     {
-        const int64_t off = (int64_t)min(mykv, last) * a.ld_qkv + (lane >> 5) * 8;
+        const int64_t off = (int64_t)min(mykv, last) * a.ld_qkv + hh * 32 + (lane >> 5) * 8;
 #pragma unroll
-        for (int ks = 0; ks < 4 * NPAN; ++ks) {
+        for (int ks = 0; ks < KS; ++ks) {
             kf[ks] = *(const bf16x8*)(K + off + ks * 16);
             vf[ks] = *(const bf16x8*)(V + off + ks * 16);
         }
     }
-    f32x16 dk[2], dv[2];
+    f32x16 dk[DT], dv[DT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) dk[t][r] = dv[t][r] = 0.f;
 
@@ -590,7 +578,7 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
         // 16-column step of a row
         float* own = (float*)(smem_all + own_at);
         const bf16* O = a.o + row_base * a.ld_o + hg * (64 * NPAN);
-        for (int q = q_begin * 64 + (tid >> 6) * 32 + (lane & 31); q < ntiles * 64; q += W * G * 32) {
+        for (int q = q_begin * 64 + (tid >> 6) * 32 + (lane & 31); q < ntiles * 64; q += DW * G * 32) {
             const int64_t at = (int64_t)min(q, last) * a.ld_o + (lane >> 5) * 8;
             bf16x8 df[4 * NPAN], of[4 * NPAN];
 #pragma unroll
@@ -599,14 +587,14 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
                 of[ks] = *(const bf16x8*)(O + at + ks * 16);
             }
 #pragma unroll
-            for (int hh = 0; hh < HP; ++hh) {
+            for (int hd = 0; hd < HP; ++hd) {
                 float dl = 0.f;
 #pragma unroll
                 for (int k = 0; k < KS; ++k)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) dl = fmaf((float)df[hh * KS + k][e], (float)of[hh * KS + k][e], dl);
-                dl += __shfl_xor(dl, 32, 64);
-                if (lane < 32) own[hh * own_rows + q] = dl;
+                    for (int e = 0; e < 8; ++e) dl = fmaf((float)df[hd * KS + k][e], (float)of[hd * KS + k][e], dl);
+                dl += other_half(dl);
+                if (lane < 32) own[hd * own_rows + q] = dl;
             }
         }
         // (the first tile's wait and barrier make them visible)
@@ -618,33 +606,32 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
     // operands of the scores S and of their gradients dP, from LDS
     bf16x8 fs[KS], fdp[KS];
     auto fetch_scores = [&](const unsigned char* st, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+        constexpr int u = decltype(j_c)::value;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) fs[k] = frag_kc(st + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+        for (int k = 0; k < KS; ++k) fs[k] = frag_kc(st + ((hh * 2 + k) >> 2) * 8192, u * 32, (hh * 2 + k) & 3, lane);
     };
     auto fetch_grads = [&](const unsigned char* st, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+        constexpr int u = decltype(j_c)::value;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) fdp[k] = frag_kc(st + TILE + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+        for (int k = 0; k < KS; ++k) fdp[k] = frag_kc(st + TILE + ((hh * 2 + k) >> 2) * 8192, u * 32, (hh * 2 + k) & 3, lane);
     };
     auto scores = [&](auto j_c) {
-        constexpr int hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        constexpr int n = decltype(j_c)::value % BUFS;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[k], kf[hh * KS + k], s[n], 0, 0, 0);
+        for (int k = 0; k < KS; ++k) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[k], kf[k], s[n], 0, 0, 0);
     };
     auto score_grads = [&](auto j_c) {
-        constexpr int hh = decltype(j_c)::value % HP;
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.f;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fdp[k], vf[hh * KS + k], dp, 0, 0, 0);
+        for (int k = 0; k < KS; ++k) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fdp[k], vf[k], dp, 0, 0, 0);
     };
     // P = exp2(S * c - lse[q]); rows q = acc_row(r), column kv = lane.  Only sub-tiles on the causal diagonal or past the last query
     // mask per element; keys beyond the padding limit are whole lanes and are cleared once, after the loop.
     auto probs = [&](const unsigned char* st, int t, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        constexpr int u = decltype(j_c)::value, n = u % BUFS;
         const float* lse_t = (const float*)(st + 2 * TILE) + 64 * hh;
 #pragma unroll
         for (int g4 = 0; g4 < 4; ++g4) {
@@ -667,9 +654,8 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
     };
     // dS = P * (dP - delta[q]), then dV^T += dO^T P~ ; dK^T += Q^T dS (contraction over the 32 queries of the sub-tile)
     auto contract = [&](const unsigned char* st, int t, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        constexpr int u = decltype(j_c)::value, n = u % BUFS;
         const float* del_t = OWN ? (const float*)(smem_all + own_at) + hh * own_rows + t * 64 : (const float*)(st + 2 * TILE) + 64 * HP + 64 * hh;
-        const int head = head0 + hh;
         // dropout: dP = dP~ o mask / (1 - p) before it meets P; P itself is masked (into what multiplied V in
         // the forward) only after dS has been formed from the unmasked probabilities
         unsigned kept = 0u;   // bit r (sixteen booleans cost the registers that K, V and the sums leave)
@@ -734,9 +720,9 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
             const bf16x8 pf = pack_acc(s[n], kk), dsf = pack_acc(dp, kk);
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
-                const int dt = hh * DT + d;
-                dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + TILE + fh * 8192, u * 32 + kk * 16, dt * 32, lane), pf, dv[dt], 0, 0, 0);
-                dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + fh * 8192, u * 32 + kk * 16, dt * 32, lane), dsf, dk[dt], 0, 0, 0);
+                const int col = (hh + d) * 32;
+                dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + TILE + fh * 8192, u * 32 + kk * 16, col, lane), pf, dv[d], 0, 0, 0);
+                dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + fh * 8192, u * 32 + kk * 16, col, lane), dsf, dk[d], 0, 0, 0);
             }
         }
     };
@@ -744,23 +730,23 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
         asm volatile("" ::: "memory");
         wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
-        attn_bwd_walk<HP, G, STAGES, STAGE, PIPE>(smem, t0, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        attn_bwd_walk<G, STAGES, STAGE, PIPE>(smem, t0, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
         if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
         // the groups' sums, first dV, then dK (one after the other: together they would not find room)
         float* parts = (float*)smem_all;
-        auto join = [&](f32x16 (&v)[2]) {
-            attn_park<W, G>(parts, grp, wave, lane, v);
+        auto join = [&](f32x16 (&v)[DT]) {
+            attn_park<DW, G>(parts, grp, dw, lane, v);
             __syncthreads();
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+            for (int t = 0; t < DT; ++t) {
                 if (t % G != grp) continue;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    float x = parts[((wave * 2 + t) * 16 + r) * 64 + lane];
+                    float x = parts[((dw * DT + t) * 16 + r) * 64 + lane];
 #pragma unroll
-                    for (int g = 1; g < G; ++g) x += parts[(((g * W + wave) * 2 + t) * 16 + r) * 64 + lane];
+                    for (int g = 1; g < G; ++g) x += parts[(((g * DW + dw) * DT + t) * 16 + r) * 64 + lane];
                     v[t][r] = x;
                 }
             }
@@ -771,15 +757,15 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
     }
     if (mykv >= pad_limit) {  // a padded key takes no probability mass: its gradients are zero
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < DT; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) dk[t][r] = dv[t][r] = 0.f;
     }
     if (mykv < a.seq) {
-        bf16* dkp = a.dk + (row_base + mykv) * a.ld_dqkv + hg * (64 * NPAN) + fh * 64;
-        bf16* dvp = a.dv + (row_base + mykv) * a.ld_dqkv + hg * (64 * NPAN) + fh * 64;
+        bf16* dkp = a.dk + (row_base + mykv) * a.ld_dqkv + hg * (64 * NPAN) + fh * 64 + hh * 32;
+        bf16* dvp = a.dv + (row_base + mykv) * a.ld_dqkv + hg * (64 * NPAN) + fh * 64 + hh * 32;
 #pragma unroll
-        for (int dt = 0; dt < 2; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 if (dt % G != grp) continue;
@@ -799,16 +785,17 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
 template <bool DROP, int HP, int NPAN, int W, int G>
 __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int block, unsigned char* smem_all) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
-    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32;
+    constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
     constexpr bool PIPE = attn_bwd_pipe(NPAN);
     constexpr int STAGES = attn_bwd_stages(NPAN, G), BUFS = PIPE ? 2 : 1;
-    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = uw % W, grp = G == 1 ? 0 : uw / W;
+    const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), dw = uw % DW, grp = G == 1 ? 0 : uw / DW;
+    const int wave = dw % W, hh = HP == 1 ? 0 : dw / W;
     unsigned char* smem = smem_all + grp * (STAGES * 2 * TILE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(block, a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
     const int qb = (a.seq + ROWS - 1) / ROWS - 1 - bm.rank;
-    const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP;
+    const int b = bm.bh / groups, hg = bm.bh % groups, head0 = hg * HP, head = head0 + hh;
     const int64_t row_base = (int64_t)b * a.seq;
     const bf16* Q = a.q + row_base * a.ld_qkv + hg * (64 * NPAN);
     const bf16* K = a.k + row_base * a.ld_qkv + hg * (64 * NPAN);
@@ -825,54 +812,47 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
     const int my_limit = kv_limit(a, b, myq);
     const int wave_min_limit = kv_limit(a, b, q0);  // limits grow with the query index
 
-    const LaneOff<W> lo = lane_off<W>(a.ld_qkv, wave, lane);
+    const LaneOff<DW> lo = lane_off<DW>(a.ld_qkv, dw, lane);
     auto issue = [&](int t, int slot) {
         unsigned char* st = smem + slot * (2 * TILE);
         const int kv0 = t * 64;
 #pragma unroll
         for (int p = 0; p < NPAN; ++p) {
-            dma_tile64<W>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, wave, lane, lo);
-            dma_tile64<W>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, wave, lane, lo);
+            dma_tile64<DW>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, dw, lane, lo);
+            dma_tile64<DW>(V + p * 64, a.ld_qkv, kv0, last, st + TILE + p * 8192, dw, lane, lo);
         }
     };
     if (grp < ntiles) issue(grp, 0);
     if (grp + G < ntiles) issue(grp + G, 1);
-    bf16x8 qf[4 * NPAN], dof[4 * NPAN];
+    bf16x8 qf[KS], dof[KS];
     {
         const int64_t r = min(myq, last);
 #pragma unroll
-        for (int ks = 0; ks < 4 * NPAN; ++ks) {
-            qf[ks] = *(const bf16x8*)(Q + r * a.ld_qkv + (lane >> 5) * 8 + ks * 16);
-            dof[ks] = *(const bf16x8*)(DO + r * a.ld_o + (lane >> 5) * 8 + ks * 16);
+        for (int ks = 0; ks < KS; ++ks) {
+            qf[ks] = *(const bf16x8*)(Q + r * a.ld_qkv + hh * 32 + (lane >> 5) * 8 + ks * 16);
+            dof[ks] = *(const bf16x8*)(DO + r * a.ld_o + hh * 32 + (lane >> 5) * 8 + ks * 16);
         }
     }
     // delta[q] = rowsum(dO o O) over the head's columns: the lane and its partner (lane ^ 32) hold the two halves of
     // each 16-column step of the query's dO row; the matching halves of O are fetched once.  Written out for the
     // dK / dV kernel, which runs after this one.
-    float my_lse[HP], my_delta[HP];
+    float my_lse, my_delta = 0.f;
     {
-        const bf16* O = a.o + row_base * a.ld_o + hg * (64 * NPAN);
-        const int64_t r = min(myq, last);
+        const bf16* O = a.o + row_base * a.ld_o + hg * (64 * NPAN) + hh * 32;
+        const int64_t r = min(myq, last), stat = ((int64_t)b * a.heads + head) * a.seq + r;
+        my_lse = a.lse[stat];
 #pragma unroll
-        for (int hh = 0; hh < HP; ++hh) {
-            const int64_t stat = ((int64_t)b * a.heads + head0 + hh) * a.seq + min(myq, last);
-            my_lse[hh] = a.lse[stat];
-            float dl = 0.f;
+        for (int k = 0; k < KS; ++k) {
+            const bf16x8 of = *(const bf16x8*)(O + r * a.ld_o + (lane >> 5) * 8 + k * 16);
 #pragma unroll
-            for (int k = 0; k < KS; ++k) {
-                const int ks = hh * KS + k;
-                const bf16x8 of = *(const bf16x8*)(O + r * a.ld_o + (lane >> 5) * 8 + ks * 16);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) dl = fmaf((float)dof[ks][e], (float)of[e], dl);
-            }
-            dl += __shfl_xor(dl, 32, 64);
-            if (lane < 32 && myq < a.seq && grp == 0) a.delta[stat] = dl;
-            my_delta[hh] = dl;
+            for (int e = 0; e < 8; ++e) my_delta = fmaf((float)dof[k][e], (float)of[e], my_delta);
         }
+        my_delta += other_half(my_delta);
+        if (lane < 32 && myq < a.seq && grp == 0) a.delta[stat] = my_delta;
     }
-    f32x16 dq[2 * NPAN];
+    f32x16 dq[DT];
 #pragma unroll
-    for (int t = 0; t < 2 * NPAN; ++t)
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) dq[t][r] = 0.f;
 
@@ -883,34 +863,33 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
     // operands of the scores S and of their gradients dP, from LDS
     bf16x8 fs[KS], fdp[KS];
     auto fetch_scores = [&](const unsigned char* st, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+        constexpr int u = decltype(j_c)::value;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) fs[k] = frag_kc(st + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+        for (int k = 0; k < KS; ++k) fs[k] = frag_kc(st + ((hh * 2 + k) >> 2) * 8192, u * 32, (hh * 2 + k) & 3, lane);
     };
     auto fetch_grads = [&](const unsigned char* st, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP;
+        constexpr int u = decltype(j_c)::value;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) fdp[k] = frag_kc(st + TILE + ((hh * KS + k) >> 2) * 8192, u * 32, (hh * KS + k) & 3, lane);
+        for (int k = 0; k < KS; ++k) fdp[k] = frag_kc(st + TILE + ((hh * 2 + k) >> 2) * 8192, u * 32, (hh * 2 + k) & 3, lane);
     };
     auto scores = [&](auto j_c) {
-        constexpr int hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        constexpr int n = decltype(j_c)::value % BUFS;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[k], qf[hh * KS + k], s[n], 0, 0, 0);
+        for (int k = 0; k < KS; ++k) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[k], qf[k], s[n], 0, 0, 0);
     };
     auto score_grads = [&](auto j_c) {
-        constexpr int hh = decltype(j_c)::value % HP;
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = 0.f;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fdp[k], dof[hh * KS + k], dp, 0, 0, 0);
+        for (int k = 0; k < KS; ++k) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fdp[k], dof[k], dp, 0, 0, 0);
     };
     auto probs = [&](const unsigned char*, int t, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        constexpr int u = decltype(j_c)::value, n = u % BUFS;
         const int kv = t * 64 + u * 32;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[n][r] = __builtin_amdgcn_exp2f(fmaf(s[n][r], a.scale_log2, -my_lse[hh]));
+        for (int r = 0; r < 16; ++r) s[n][r] = __builtin_amdgcn_exp2f(fmaf(s[n][r], a.scale_log2, -my_lse));
         if (kv + 32 > wave_min_limit) {
             asm volatile("" ::: "memory");  // a real branch: only tiles on the mask boundary pay for it
             const int lim = my_limit - kv - 4 * (lane >> 5);
@@ -919,22 +898,22 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
         }
     };
     auto contract = [&](const unsigned char* st, int t, auto j_c) {
-        constexpr int u = decltype(j_c)::value / HP, hh = decltype(j_c)::value % HP, n = decltype(j_c)::value % BUFS;
+        constexpr int u = decltype(j_c)::value, n = u % BUFS;
         if (DROP && a.drop.thresh) {
             asm volatile("" ::: "memory");
-            const uint64_t base = prob_index(a, b, head0 + hh, min(myq, last)) + t * 64 + u * 32;
+            const uint64_t base = prob_index(a, b, head, min(myq, last)) + t * 64 + u * 32;
             drop_acc_rows(a.drop, base, lane, dp);
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) dp[r] = s[n][r] * (dp[r] - my_delta[hh]);
+        for (int r = 0; r < 16; ++r) dp[r] = s[n][r] * (dp[r] - my_delta);
         // dQ^T += K^T dS^T (contraction over the 32 keys of this sub-tile)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const bf16x8 dsf = pack_acc(dp, kk);
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
-                const int dt = hh * DT + d;
-                dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + (dt >> 1) * 8192, u * 32 + kk * 16, (dt & 1) * 32, lane), dsf, dq[dt], 0, 0, 0);
+                const int dt = hh + d;
+                dq[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + (dt >> 1) * 8192, u * 32 + kk * 16, (dt & 1) * 32, lane), dsf, dq[d], 0, 0, 0);
             }
         }
     };
@@ -943,29 +922,29 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
         asm volatile("" ::: "memory");
         wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
-        attn_bwd_walk<HP, G, STAGES, 2 * TILE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        attn_bwd_walk<G, STAGES, 2 * TILE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
         if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
         float* parts = (float*)smem_all;
-        attn_park<W, G>(parts, grp, wave, lane, dq);
+        attn_park<DW, G>(parts, grp, dw, lane, dq);
         __syncthreads();
 #pragma unroll
-        for (int dt = 0; dt < 2 * NPAN; ++dt) {
+        for (int dt = 0; dt < DT; ++dt) {
             if (dt % G != grp) continue;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                float x = parts[((wave * (2 * NPAN) + dt) * 16 + r) * 64 + lane];
+                float x = parts[((dw * DT + dt) * 16 + r) * 64 + lane];
 #pragma unroll
-                for (int g = 1; g < G; ++g) x += parts[(((g * W + wave) * (2 * NPAN) + dt) * 16 + r) * 64 + lane];
+                for (int g = 1; g < G; ++g) x += parts[(((g * DW + dw) * DT + dt) * 16 + r) * 64 + lane];
                 dq[dt][r] = x;
             }
         }
     }
     if (myq < a.seq) {
-        bf16* dqp = a.dq + (row_base + myq) * a.ld_dqkv + hg * (64 * NPAN);
+        bf16* dqp = a.dq + (row_base + myq) * a.ld_dqkv + hg * (64 * NPAN) + hh * 32;
 #pragma unroll
-        for (int dt = 0; dt < 2 * NPAN; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 if (dt % G != grp) continue;
@@ -978,19 +957,19 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
 }
 
 template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     attn_bwd_dkv_block<DROP, HP, NPAN, W, G, false>(a, blockIdx.x, smem_all, 0);
 }
 template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x, smem_all);
 }
 // Both in one launch, where there is room for all their blocks (attn_bwd_launch): first the dK / dV blocks, whose walks are the
 // longer ones, then the dQ blocks.
 template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * G * 64, 2) void attn_bwd_kernel(const AttnArgs a, const int dkv_blocks, const int own_at) {
+__global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_kernel(const AttnArgs a, const int dkv_blocks, const int own_at) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     if ((int)blockIdx.x < dkv_blocks) attn_bwd_dkv_block<DROP, HP, NPAN, W, G, true>(a, blockIdx.x, smem_all, own_at);
     else attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x - dkv_blocks, smem_all);
@@ -1016,7 +995,7 @@ static int check_attn(const char* name, int dtype, int mask, int batch, int head
 // LDS: the rings, or what the groups leave for each other
 template <int HP, int NPAN, int W, int G> constexpr size_t attn_lds(bool bwd, bool dkv) {
     const size_t ring = G * (size_t)(bwd ? attn_bwd_stages(NPAN, G) : 2) * (2 * NPAN * 8192 + (dkv ? 512 * HP : 0));
-    const size_t parts = G == 1 ? 0 : (size_t)W * G * ((dkv ? 2 : 2 * NPAN) * 4096 + (dkv ? 0 : HP * 512));
+    const size_t parts = G == 1 ? 0 : (size_t)W * HP * G * ((dkv ? 2 : 2 * NPAN) / HP * 4096 + (bwd ? 0 : 512));
     return ring > parts ? ring : parts;
 }
 template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int threads, size_t lds, const AttnArgs& a, hipStream_t st) {
@@ -1029,19 +1008,19 @@ template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int
 struct attn_fwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_fwd_kernel<true, HP, NPAN, W, G> : attn_fwd_kernel<false, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(false, false), a, st);
+        return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(false, false), a, st);
     }
 };
 struct attn_dq_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_bwd_dq_kernel<true, HP, NPAN, W, G> : attn_bwd_dq_kernel<false, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh, W * G * 64, attn_lds<HP, NPAN, W, G>(true, false), a, st);
+        return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, false), a, st);
     }
 };
 struct attn_dkv_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         auto kern = a.drop.thresh ? attn_bwd_dkv_kernel<true, HP, NPAN, W, G> : attn_bwd_dkv_kernel<false, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh * NPAN, W * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);   // 128-wide heads: a block per half
+        return attn_go(kern, seq, W * 32, nbh * NPAN, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);   // 128-wide heads: a block per half
     }
 };
 // Both backward kernels: in one launch where all blocks of the two find room at once (two blocks of four waves a CU, one of eight),
@@ -1055,7 +1034,7 @@ struct attn_dkv_launch {
 static constexpr int kOwnDeltaSeq = 2048;    // longest sequence whose deltas a block keeps in LDS
 struct attn_bwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        const int64_t rows = (seq + W * 32 - 1) / (W * 32), slots = 256 * 8 / (W * G);
+        const int64_t rows = (seq + W * 32 - 1) / (W * 32), slots = 256 * 8 / (W * HP * G);
         if (seq > kOwnDeltaSeq || nbh * rows * (NPAN + 1) > slots) {
             // the dQ kernel first: it also leaves delta = rowsum(dO o O) of its queries for the dK / dV kernel
             const int rc = attn_dq_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
@@ -1066,28 +1045,34 @@ struct attn_bwd_launch {
         const size_t lds = own_at + (size_t)HP * ((seq + 63) / 64 * 64) * sizeof(float);
         auto kern = a.drop.thresh ? attn_bwd_kernel<true, HP, NPAN, W, G> : attn_bwd_kernel<false, HP, NPAN, W, G>;
         BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));
-        bb_launch(kern, dim3(dkv + dq), dim3(W * G * 64), lds, st, a, (int)dkv, (int)own_at);
+        bb_launch(kern, dim3(dkv + dq), dim3(W * HP * G * 64), lds, st, a, (int)dkv, (int)own_at);
         BB_LAUNCH_CHECK();
         return BB_OK;
     }
 };
-// The shape of a block, by the number of blocks of 128 rows and the length of the walk (a pair of heads walks twice).  Four
-// waves / four waves in two groups / two in four (us, forward, backward): 12 heads of 64, 2043 keys (192 blocks) 27 78 / 20 64 /
+// The shape of a block, by the number of blocks of 128 rows and the length of the walk.  Four
+// waves / four waves in two groups / two in four (us, forward, backward; pairs of heads on the same waves, see below): 12 heads of 64, 2043 keys (192 blocks) 27 78 / 20 64 /
 // 24 78; 4 x 16 heads, 512 causal (256) 13.4 31.5 / 10.8 29.7 / 12.1 35.0; 2 x 25 heads, 300 (150) 7.4 20.7 / 7.7 23.3 / 9.6 24.2;
 // 16 heads, 1024 causal (128) 22.1 50.4 / 16.2 42.7 / 11.1 29.8; 2 x 4 heads, 512 causal (32) 12.7 29.4 / 10.3 27.6 / 7.6 20.8; 4
 // heads, 1024 causal with dropout (32) 28.3 80.5 / 24.3 65.6 / 15.2 40.7; 6 x 8 heads, 175 (96) 7.1 17.2 / 7.2 19.9 / 6.2 17.3; 8
 // x 8 pairs of 32, 128, dropout (64) 8.6 23.9 / 8.9 24.7 / 7.4 23.4; 2 x 16 heads, 100 (32) 5.8 14.0 / 5.9 16.4 / 5.6 15.7.  Heads of
-// 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.
+// 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.  Pairs of heads have twice the waves: two
+// a head in two groups (a walk of both heads by two waves in four groups / this: 1 x 4 pairs, 500 causal 9.6 16.4 / 8.3 15.3, 2 x 4,
+// 300, padding, dropout 9.6 20.7 / 7.8 17.0; four waves in two groups / four a head: 4 x 8, 512 causal 10.6 24.8 / 9.2 22.4).
 // Attention without a mask keeps the one walk.  Groups add the same terms in another order: as near the exact sums as before, but
 // not the same last bits, and the stage that ends the reference's script (no mask; a LayerNorm whose rows are summed up, which
 // cancels to 1e-4 of its terms) passes gradients on in which such bits show as 3 to 5 %.
 template <typename L, int HP, int NPAN> static int attn_shape(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-    const int64_t blocks = (int64_t)nbh * ((seq + 127) / 128), walk = (int64_t)seq * HP;
+    const int64_t blocks = (int64_t)nbh * ((seq + 127) / 128);
     if (a.mask != BB_MASK_NONE) {
-        if constexpr (NPAN == 1) {
-            if (blocks <= 128 && walk >= 160) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
+        if constexpr (HP == 2) {
+            if (blocks <= 128 && seq >= 160) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
+        } else {
+            if constexpr (NPAN == 1) {
+                if (blocks <= 128 && seq >= 160) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
+            }
+            if (blocks <= 256 && seq >= 448) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
         }
-        if (blocks <= 256 && walk >= 448) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
     }
     return L::template go<HP, NPAN, 4, 1>(seq, nbh, a, st);
 }
