@@ -37,6 +37,7 @@ struct AttnArgs {
     float* lse;                                    // [batch, heads, seq], log2 domain
     float* delta;                                  // [batch, heads, seq], rowsum(dO * O)
     const int32_t* key_len;
+    uint32_t* keep;                                // dropout: the decisions of the forward (keep_words), or null
     int64_t ld_qkv, ld_o, ld_dqkv;
     int batch, heads, seq, mask;
     float scale_log2;                              // log2(e) / sqrt(d)
@@ -44,8 +45,8 @@ struct AttnArgs {
     DropKey drop;                                  // dropout on the probabilities (thresh 0: none)
 };
 template <> struct BbDropAt<AttnArgs> { static constexpr int32_t value = offsetof(AttnArgs, drop); };
-template <> struct BbPointersAt<AttnArgs> : BbPointerRun<12> {};   // q .. key_len
-static_assert(offsetof(AttnArgs, ld_qkv) == 12 * sizeof(void*), "BbPointersAt<AttnArgs>");
+template <> struct BbPointersAt<AttnArgs> : BbPointerRun<13> {};   // q .. keep
+static_assert(offsetof(AttnArgs, ld_qkv) == 13 * sizeof(void*), "BbPointersAt<AttnArgs>");
 // index of probability (b, head, q, kv) in the [batch, heads, seq, seq] tensor that is never stored
 __device__ __forceinline__ uint64_t prob_index(const AttnArgs& a, int b, int head, int q) {
     return ((uint64_t)(b * a.heads + head) * a.seq + q) * a.seq;
@@ -133,24 +134,53 @@ __device__ __forceinline__ bf16x8 pack_acc(const f32x16& a, int half) {
 }
 // row index (0..31) that register r of a 32x32 accumulator holds in this lane
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+// Kept decisions.  A hash per two decisions, 8 vector instructions each, is what a pass over the probabilities costs beyond an undropped
+// one (19 where a lane's probabilities are not neighbours, as in dK/dV); the forward leaves the decisions as bits instead, for
+// both backward passes: 8 x 16 heads of 64, 1024 keys, dropout: backward 211 -> 172 us, forward 72 -> 80
+// Layout: [batch, heads][queries / 32][keys / 32, tiles of 64 in full][32 words]; a word has the decisions of a query, bit j that of
+// the j-th of 32 keys; the words lie in the order of accumulator rows, those of register r of the lower and the upper half wave next
+// to each other: 64 bits that select lanes as they are.
+__host__ __device__ __forceinline__ int64_t keep_blocks(int seq) { return (int64_t)((seq + 31) / 32) * ((seq + 63) / 64 * 2); }   // per head
+__device__ __forceinline__ uint32_t* keep_at(const AttnArgs& a, int b, int head, int qs, int ks) {
+    return a.keep + (((int64_t)b * a.heads + head) * keep_blocks(a.seq) + (int64_t)qs * ((a.seq + 63) / 64 * 2) + ks) * 32;
+}
+__device__ __forceinline__ int keep_word(int q) { return (q >> 3) * 8 + (q & 3) * 2 + ((q >> 2) & 1); }   // of the q-th of 32 queries
+// bit of register r in a word shifted right by 4 * (lane >> 5): 8 * (r / 4) + r % 4
+__device__ __forceinline__ float keep_bit(uint32_t shifted, int r, float v) {
+    return __uint_as_float(__float_as_uint(v) & (uint32_t)__builtin_amdgcn_sbfe((int)shifted, 8 * (r >> 2) + (r & 3), 1));
+}
+__device__ __forceinline__ float keep_lanes(uint64_t lanes, float v) {
+    float o;
+    asm("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(o) : "v"(v), "s"(lanes));
+    return o;
+}
 // Dropout over the sixteen accumulator registers of a lane whose rows acc_row(r, lane) are consecutive probability
 // indices from `base` on: registers 4g .. 4g + 3 hold four neighbouring indices, i.e. two hash pairs when the first is
 // even (in every lane, where the sequence length is), else parts of three (12 heads x 2043^2 forward: 58 us; 85 where the lanes
-// of odd queries went another way).  Kept values are scaled, dropped ones zeroed.
-__device__ __forceinline__ void drop_acc_rows(const DropKey& k, uint64_t base, int lane, f32x16& v) {
-    if (k.small) {                       // the rule: fewer than 2^32 probabilities
+// of odd queries went another way).  Kept values are scaled, dropped ones zeroed;
+// bit 8 * (r / 4) + r % 4 of what it returns is set where register r was kept.
+template <bool PAIRS = false>
+__device__ __forceinline__ uint32_t drop_acc_rows(const DropKey& k, uint64_t base, int lane, f32x16& v) {
+    uint32_t kept = 0u;
+    auto decide = [&](int r, bool keep) {
+        v[r] = keep ? v[r] * k.scale : 0.f;
+        kept |= keep ? 1u << (8 * (r >> 2) + (r & 3)) : 0u;
+    };
+    if (PAIRS || k.small) {              // the rule: fewer than 2^32 probabilities
         const uint32_t p0 = ((uint32_t)base >> 1) + 2 * (lane >> 5);   // 8 g + 4 (lane >> 5) is even
-        const bool odd = (base & 1) != 0;
-        if (__builtin_amdgcn_ballot_w64(odd) == 0) {
+        const bool odd = !PAIRS && (base & 1) != 0;
+        if (PAIRS || __builtin_amdgcn_ballot_w64(odd) == 0) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const uint32_t x0 = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g), x1 = bb_dropout_pair_bits32(k.k0, k.k1, p0 + 4 * g + 1);
-                v[4 * g] = bb_keep_even(x0, k.thresh) ? v[4 * g] * k.scale : 0.f;
-                v[4 * g + 1] = bb_keep_odd(x0, k.thresh) ? v[4 * g + 1] * k.scale : 0.f;
-                v[4 * g + 2] = bb_keep_even(x1, k.thresh) ? v[4 * g + 2] * k.scale : 0.f;
-                v[4 * g + 3] = bb_keep_odd(x1, k.thresh) ? v[4 * g + 3] * k.scale : 0.f;
+                decide(4 * g, bb_keep_even(x0, k.thresh));
+                decide(4 * g + 1, bb_keep_odd(x0, k.thresh));
+                decide(4 * g + 2, bb_keep_even(x1, k.thresh));
+                decide(4 * g + 3, bb_keep_odd(x1, k.thresh));
+                asm("" : "+v"(kept));      // bits go in as they come: added up at the end they would wait in sixteen registers
+                if (g & 1) __builtin_amdgcn_sched_barrier(0);
             }
-            return;
+            return kept;
         }
         // an odd sequence length: every other query's row starts inside a pair
 #pragma unroll
@@ -163,18 +193,21 @@ __device__ __forceinline__ void drop_acc_rows(const DropKey& k, uint64_t base, i
                 // the 16 bits of element e: half e % 2 of pair e / 2, or of the one further on where the first index is odd
                 const uint32_t even_bits = e & 1 ? x[e >> 1] >> 16 : x[e >> 1] & 0xffffu;
                 const uint32_t odd_bits = e & 1 ? x[(e + 1) >> 1] & 0xffffu : x[e >> 1] >> 16;
-                v[4 * g + e] = (odd ? odd_bits : even_bits) >= k.thresh ? v[4 * g + e] * k.scale : 0.f;
+                decide(4 * g + e, (odd ? odd_bits : even_bits) >= k.thresh);
             }
+            asm("" : "+v"(kept));
+            __builtin_amdgcn_sched_barrier(0);
         }
-        return;
+        return kept;
     }
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const uint64_t i0 = base + 8 * g + 4 * (lane >> 5);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            v[4 * g + e] = bb_dropout_keep(k.k0, k.k1, k.thresh, i0 + e) ? v[4 * g + e] * k.scale : 0.f;
+            decide(4 * g + e, bb_dropout_keep(k.k0, k.k1, k.thresh, i0 + e));
     }
+    return kept;
 }
 
 // the value of lane ^ 32
@@ -224,14 +257,19 @@ template <int DW, int G, int T> __device__ __forceinline__ void attn_park(float*
         for (int r = 0; r < 16; ++r) parts[(((grp * DW + w) * T + t) * 16 + r) * 64 + lane] = v[t][r];
 }
 
+enum { NODROP = 0, MADE = 1, KEPT = 2, PAIRS = 3 };
+
 // =========================================================================================
 // forward: block = 128 queries (4 waves x 32; W, G: see above), loop over 64-key tiles
 // =========================================================================================
 // HP: heads per block (1: one head, 2: a pair of 32-wide heads, W waves each); NPAN: 64-wide column panels of a head (1; 2 for
 // 128-wide heads, HP = 1: a tile in LDS is then two [64][64] panels behind each other, each in the format above);
+// DROP: no dropout; its decisions made from the key, in the forward apart from the case where all of a lane's indices go in whole pairs
+// (even sequences, fewer than 2^32 probabilities; branches between the ways to make them cost moves and a wave in three); read from
+// what the forward kept, in the backward
 // KS k-steps of a head's scores, DT 32-wide output tiles of a head
-template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * HP * G * 64, (!DROP && NPAN == 1 && G == 1) ? 4 : 2) void attn_fwd_kernel(const AttnArgs a) {
+template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+__global__ __launch_bounds__(W * HP * G * 64, NPAN == 1 && G == 1 ? (DROP == NODROP ? 4 : DROP == PAIRS ? 3 : 2) : 2) void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];  // G rings of 2 stages of K, then 2 of V
@@ -330,10 +368,21 @@ __global__ __launch_bounds__(W * HP * G * 64, (!DROP && NPAN == 1 && G == 1) ? 4
             }
         lsum = lsum * alpha + psum;
         m = mnew;
-        if (DROP && a.drop.thresh) {   // the normaliser takes every probability, the context only the kept ones
+        if (DROP != NODROP) asm volatile("" : "+v"(lsum));   // here: left for later, the sum keeps the probabilities beside the dropped-out ones
+        if (DROP != NODROP) {   // the normaliser takes every probability, the context only the kept ones
             const uint64_t base = prob_index(a, b, head, min(myq, last)) + kv0;
+            uint32_t kept[2];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) drop_acc_rows(a.drop, base + u * 32, lane, s[u]);
+            for (int u = 0; u < 2; ++u) kept[u] = drop_acc_rows<DROP == PAIRS>(a.drop, base + u * 32, lane, s[u]);
+            if (a.keep) {
+                // the halves of a wave have each other's nibbles; the lower one stores the words of the first 32 keys
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    kept[u] <<= 4 * (lane >> 5);
+                    kept[u] |= __float_as_uint(other_half(__uint_as_float(kept[u])));
+                }
+                keep_at(a, b, head, q0 / 32, kv0 / 32)[(lane >> 5) * 32 + keep_word(lane & 31)] = lane < 32 ? kept[0] : kept[1];
+            }
         }
         if (__any(alpha != 1.0f)) {  // wave-uniform: once the maxima have settled nothing is rescaled
 #pragma unroll
@@ -506,7 +555,7 @@ __device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int it
 // has two blocks per head and key block); scores and dP take the full 128 columns in both, i.e. are made twice -- a wave
 // that held all four output tiles of dK and of dV next to K, V, S and dP would need more registers than it has.
 // OWN: no dQ kernel has run before this one: the block makes delta of all its queries itself, in LDS from OWN_AT on
-template <bool DROP, int HP, int NPAN, int W, int G, bool OWN>
+template <int DROP, int HP, int NPAN, int W, int G, bool OWN>
 __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int block, unsigned char* smem_all, const int own_at) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
@@ -630,8 +679,15 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
     };
     // P = exp2(S * c - lse[q]); rows q = acc_row(r), column kv = lane.  Only sub-tiles on the causal diagonal or past the last query
     // mask per element; keys beyond the padding limit are whole lanes and are cleared once, after the loop.
+    typedef __attribute__((ext_vector_type(8))) uint64_t u64x8;
+    u64x8 lanes[2];     // kept decisions of the sub-tile: register r's lanes
     auto probs = [&](const unsigned char* st, int t, auto j_c) {
         constexpr int u = decltype(j_c)::value, n = u % BUFS;
+        if (DROP == KEPT) {
+            const auto* w = (const __attribute__((address_space(4))) u64x8*)(uintptr_t)keep_at(a, b, head, t * 2 + u, kv0 / 32);
+            lanes[0] = w[0];
+            lanes[1] = w[1];
+        }
         const float* lse_t = (const float*)(st + 2 * TILE) + 64 * hh;
 #pragma unroll
         for (int g4 = 0; g4 < 4; ++g4) {
@@ -659,7 +715,10 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
         // dropout: dP = dP~ o mask / (1 - p) before it meets P; P itself is masked (into what multiplied V in
         // the forward) only after dS has been formed from the unmasked probabilities
         unsigned kept = 0u;   // bit r (sixteen booleans cost the registers that K, V and the sums leave)
-        if (DROP && a.drop.thresh) {
+        if (DROP == KEPT) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dp[r] = keep_lanes(lanes[r >> 3][r & 7], dp[r] * a.drop.scale);
+        } else if (DROP == MADE) {
             asm volatile("" ::: "memory");
             const int qlane = t * 64 + u * 32 + 4 * (lane >> 5);
             if (a.drop.small) {
@@ -710,7 +769,10 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
 #pragma unroll
             for (int e = 0; e < 4; ++e) dp[g4 * 4 + e] = s[n][g4 * 4 + e] * (dp[g4 * 4 + e] - d4[e]);
         }
-        if (DROP && a.drop.thresh) {
+        if (DROP == KEPT) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[n][r] = keep_lanes(lanes[r >> 3][r & 7], s[n][r] * a.drop.scale);
+        } else if (DROP == MADE) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[n][r] = (kept >> r) & 1u ? s[n][r] * a.drop.scale : 0.f;
         }
@@ -782,7 +844,7 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
 // =========================================================================================
 // backward dQ: block = 128 queries (4 waves x 32), loop over 64-key tiles
 // =========================================================================================
-template <bool DROP, int HP, int NPAN, int W, int G>
+template <int DROP, int HP, int NPAN, int W, int G>
 __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int block, unsigned char* smem_all) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
@@ -790,7 +852,8 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
     constexpr int STAGES = attn_bwd_stages(NPAN, G), BUFS = PIPE ? 2 : 1;
     const int tid = threadIdx.x, lane = tid & 63, uw = __builtin_amdgcn_readfirstlane(tid >> 6), dw = uw % DW, grp = G == 1 ? 0 : uw / DW;
     const int wave = dw % W, hh = HP == 1 ? 0 : dw / W;
-    unsigned char* smem = smem_all + grp * (STAGES * 2 * TILE);
+    constexpr int STAGE = 2 * TILE + (DROP == KEPT ? DW * 256 : 0);      // K tile, V tile, the kept decisions of each wave's queries
+    unsigned char* smem = smem_all + grp * (STAGES * STAGE);
     const int groups = a.heads / HP;
     const BlockMap bm = map_block(block, a.batch * groups);
     if (bm.bh >= a.batch * groups) return;
@@ -814,8 +877,9 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
 
     const LaneOff<DW> lo = lane_off<DW>(a.ld_qkv, dw, lane);
     auto issue = [&](int t, int slot) {
-        unsigned char* st = smem + slot * (2 * TILE);
+        unsigned char* st = smem + slot * STAGE;
         const int kv0 = t * 64;
+        if (DROP == KEPT) dma4(keep_at(a, b, head, min(q0, last) / 32, t * 2) + lane, st + 2 * TILE + dw * 256);
 #pragma unroll
         for (int p = 0; p < NPAN; ++p) {
             dma_tile64<DW>(K + p * 64, a.ld_qkv, kv0, last, st + p * 8192, dw, lane, lo);
@@ -899,10 +963,15 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
     };
     auto contract = [&](const unsigned char* st, int t, auto j_c) {
         constexpr int u = decltype(j_c)::value, n = u % BUFS;
-        if (DROP && a.drop.thresh) {
+        if constexpr (DROP != NODROP) {
             asm volatile("" ::: "memory");
-            const uint64_t base = prob_index(a, b, head, min(myq, last)) + t * 64 + u * 32;
-            drop_acc_rows(a.drop, base, lane, dp);
+            if constexpr (DROP == KEPT) {
+                const uint32_t w = ((const uint32_t*)(st + 2 * TILE))[dw * 64 + u * 32 + keep_word(lane & 31)] >> (4 * (lane >> 5));
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dp[r] = keep_bit(w, r, dp[r] * a.drop.scale);
+            } else {
+                drop_acc_rows(a.drop, prob_index(a, b, head, min(myq, last)) + t * 64 + u * 32, lane, dp);
+            }
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp[r] = s[n][r] * (dp[r] - my_delta);
@@ -922,7 +991,7 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
         asm volatile("" ::: "memory");
         wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
-        attn_bwd_walk<G, STAGES, 2 * TILE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        attn_bwd_walk<G, STAGES, STAGE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
         if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
@@ -956,19 +1025,19 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
     }
 }
 
-template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
 __global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_dkv_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     attn_bwd_dkv_block<DROP, HP, NPAN, W, G, false>(a, blockIdx.x, smem_all, 0);
 }
-template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
 __global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x, smem_all);
 }
 // Both in one launch, where there is room for all their blocks (attn_bwd_launch): first the dK / dV blocks, whose walks are the
 // longer ones, then the dQ blocks.
-template <bool DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
 __global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_kernel(const AttnArgs a, const int dkv_blocks, const int own_at) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     if ((int)blockIdx.x < dkv_blocks) attn_bwd_dkv_block<DROP, HP, NPAN, W, G, true>(a, blockIdx.x, smem_all, own_at);
@@ -994,7 +1063,7 @@ static int check_attn(const char* name, int dtype, int mask, int batch, int head
 
 // LDS: the rings, or what the groups leave for each other
 template <int HP, int NPAN, int W, int G> constexpr size_t attn_lds(bool bwd, bool dkv) {
-    const size_t ring = G * (size_t)(bwd ? attn_bwd_stages(NPAN, G) : 2) * (2 * NPAN * 8192 + (dkv ? 512 * HP : 0));
+    const size_t ring = G * (size_t)(bwd ? attn_bwd_stages(NPAN, G) : 2) * (2 * NPAN * 8192 + (dkv ? 512 * HP : bwd ? W * HP * 256 : 0));
     const size_t parts = G == 1 ? 0 : (size_t)W * HP * G * ((dkv ? 2 : 2 * NPAN) / HP * 4096 + (bwd ? 0 : 512));
     return ring > parts ? ring : parts;
 }
@@ -1007,19 +1076,19 @@ template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int
 // dropout is a kernel of its own: its keep decisions cost registers that decide how many blocks a CU holds
 struct attn_fwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        auto kern = a.drop.thresh ? attn_fwd_kernel<true, HP, NPAN, W, G> : attn_fwd_kernel<false, HP, NPAN, W, G>;
+        auto kern = !a.drop.thresh ? attn_fwd_kernel<NODROP, HP, NPAN, W, G> : a.drop.small && seq % 2 == 0 ? attn_fwd_kernel<PAIRS, HP, NPAN, W, G> : attn_fwd_kernel<MADE, HP, NPAN, W, G>;
         return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(false, false), a, st);
     }
 };
 struct attn_dq_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        auto kern = a.drop.thresh ? attn_bwd_dq_kernel<true, HP, NPAN, W, G> : attn_bwd_dq_kernel<false, HP, NPAN, W, G>;
+        auto kern = a.keep ? attn_bwd_dq_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_dq_kernel<MADE, HP, NPAN, W, G> : attn_bwd_dq_kernel<NODROP, HP, NPAN, W, G>;
         return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, false), a, st);
     }
 };
 struct attn_dkv_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        auto kern = a.drop.thresh ? attn_bwd_dkv_kernel<true, HP, NPAN, W, G> : attn_bwd_dkv_kernel<false, HP, NPAN, W, G>;
+        auto kern = a.keep ? attn_bwd_dkv_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_dkv_kernel<MADE, HP, NPAN, W, G> : attn_bwd_dkv_kernel<NODROP, HP, NPAN, W, G>;
         return attn_go(kern, seq, W * 32, nbh * NPAN, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);   // 128-wide heads: a block per half
     }
 };
@@ -1043,7 +1112,7 @@ struct attn_bwd_launch {
         const unsigned dkv = attn_grid(seq, W * 32, nbh * NPAN), dq = attn_grid(seq, W * 32, nbh);
         constexpr size_t own_at = attn_lds<HP, NPAN, W, G>(true, true) > attn_lds<HP, NPAN, W, G>(true, false) ? attn_lds<HP, NPAN, W, G>(true, true) : attn_lds<HP, NPAN, W, G>(true, false);
         const size_t lds = own_at + (size_t)HP * ((seq + 63) / 64 * 64) * sizeof(float);
-        auto kern = a.drop.thresh ? attn_bwd_kernel<true, HP, NPAN, W, G> : attn_bwd_kernel<false, HP, NPAN, W, G>;
+        auto kern = a.keep ? attn_bwd_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_kernel<MADE, HP, NPAN, W, G> : attn_bwd_kernel<NODROP, HP, NPAN, W, G>;
         BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));
         bb_launch(kern, dim3(dkv + dq), dim3(W * HP * G * 64), lds, st, a, (int)dkv, (int)own_at);
         BB_LAUNCH_CHECK();
@@ -1082,17 +1151,19 @@ template <typename L> static int attn_launch(int head_dim, int seq, int batch, i
     return attn_shape<L, 2, 1>(seq, batch * (heads / 2), a, st);    // pairs of heads
 }
 
-extern "C" int bb_attention_fwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
+static int attention_fwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
                                 const void* k, const void* v, int64_t ld_qkv, void* out, int64_t ld_out, float* lse,
                                 const int32_t* key_len, float dropout_p, uint32_t dropout_k0, uint32_t dropout_k1,
-                                void* stream) {
+                         uint32_t* keep, void* stream) {
     int rc = check_attn("bb_attention_fwd", dtype, mask, batch, heads, seq, head_dim, ld_qkv, ld_out, key_len);
     if (rc) return rc;
     if (batch == 0 || seq == 0) return BB_OK;
     BB_REQUIRE(q && k && v && out && lse, "bb_attention_fwd: null pointer");
     BB_REQUIRE(dropout_p >= 0.f && dropout_p < 1.f, "bb_attention_fwd: dropout_p must be in [0, 1)");
+    BB_REQUIRE((uintptr_t)keep % 128 == 0, "bb_attention_fwd: keep must be aligned to 128 bytes");
     AttnArgs a = {};
     a.drop = bb_drop_key(dropout_p, dropout_k0, dropout_k1, (uint64_t)batch * heads * (uint64_t)seq * (uint64_t)seq);
+    a.keep = a.drop.thresh ? (uint32_t*)keep : nullptr;
     a.q = (const bf16*)q; a.k = (const bf16*)k; a.v = (const bf16*)v;
     a.out = (bf16*)out; a.lse = lse; a.key_len = key_len;
     a.ld_qkv = ld_qkv; a.ld_o = ld_out;
@@ -1102,19 +1173,21 @@ extern "C" int bb_attention_fwd(int dtype, int mask, int batch, int heads, int s
     return attn_launch<attn_fwd_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
 }
 
-extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
+static int attention_bwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q,
                                 const void* k, const void* v, int64_t ld_qkv, const void* out, const void* d_out,
                                 int64_t ld_out, const float* lse, float* delta, void* dq, void* dk, void* dv,
                                 int64_t ld_dqkv, const int32_t* key_len, float dropout_p, uint32_t dropout_k0,
-                                uint32_t dropout_k1, void* stream) {
+                                uint32_t dropout_k1, const uint32_t* keep, void* stream) {
     int rc = check_attn("bb_attention_bwd", dtype, mask, batch, heads, seq, head_dim, ld_qkv, ld_out, key_len);
     if (rc) return rc;
     if (batch == 0 || seq == 0) return BB_OK;
     BB_REQUIRE(q && k && v && out && d_out && lse && delta && dq && dk && dv, "bb_attention_bwd: null pointer");
     BB_REQUIRE(ld_dqkv % 4 == 0 && ld_dqkv >= heads * head_dim, "bb_attention_bwd: bad gradient leading dimension");
     BB_REQUIRE(dropout_p >= 0.f && dropout_p < 1.f, "bb_attention_bwd: dropout_p must be in [0, 1)");
+    BB_REQUIRE((uintptr_t)keep % 128 == 0, "bb_attention_bwd: keep must be aligned to 128 bytes");
     AttnArgs a = {};
     a.drop = bb_drop_key(dropout_p, dropout_k0, dropout_k1, (uint64_t)batch * heads * (uint64_t)seq * (uint64_t)seq);
+    a.keep = a.drop.thresh ? (uint32_t*)keep : nullptr;
     a.q = (const bf16*)q; a.k = (const bf16*)k; a.v = (const bf16*)v;
     a.o = (const bf16*)out; a.d_o = (const bf16*)d_out;
     a.dq = (bf16*)dq; a.dk = (bf16*)dk; a.dv = (bf16*)dv;
@@ -1124,4 +1197,32 @@ extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int s
     a.scale = 1.0f / sqrtf((float)head_dim);
     a.scale_log2 = a.scale * 1.4426950408889634f;
     return attn_launch<attn_bwd_launch>(head_dim, seq, batch, heads, a, (hipStream_t)stream);
+}
+
+extern "C" int64_t bb_attention_keep_words(int batch, int heads, int seq) { return (int64_t)batch * heads * keep_blocks(seq) * 32; }
+extern "C" int bb_attention_fwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k, const void* v,
+                                int64_t ld_qkv, void* out, int64_t ld_out, float* lse, const int32_t* key_len, float dropout_p,
+                                uint32_t dropout_k0, uint32_t dropout_k1, void* stream) {
+    return attention_fwd(dtype, mask, batch, heads, seq, head_dim, q, k, v, ld_qkv, out, ld_out, lse, key_len, dropout_p, dropout_k0,
+                         dropout_k1, nullptr, stream);
+}
+extern "C" int bb_attention_fwd_keep(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k,
+                                     const void* v, int64_t ld_qkv, void* out, int64_t ld_out, float* lse, const int32_t* key_len,
+                                     float dropout_p, uint32_t dropout_k0, uint32_t dropout_k1, uint32_t* keep, void* stream) {
+    return attention_fwd(dtype, mask, batch, heads, seq, head_dim, q, k, v, ld_qkv, out, ld_out, lse, key_len, dropout_p, dropout_k0,
+                         dropout_k1, keep, stream);
+}
+extern "C" int bb_attention_bwd(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k, const void* v,
+                                int64_t ld_qkv, const void* out, const void* d_out, int64_t ld_out, const float* lse, float* delta,
+                                void* dq, void* dk, void* dv, int64_t ld_dqkv, const int32_t* key_len, float dropout_p,
+                                uint32_t dropout_k0, uint32_t dropout_k1, void* stream) {
+    return attention_bwd(dtype, mask, batch, heads, seq, head_dim, q, k, v, ld_qkv, out, d_out, ld_out, lse, delta, dq, dk, dv, ld_dqkv,
+                         key_len, dropout_p, dropout_k0, dropout_k1, nullptr, stream);
+}
+extern "C" int bb_attention_bwd_keep(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k,
+                                     const void* v, int64_t ld_qkv, const void* out, const void* d_out, int64_t ld_out, const float* lse,
+                                     float* delta, void* dq, void* dk, void* dv, int64_t ld_dqkv, const int32_t* key_len, float dropout_p,
+                                     uint32_t dropout_k0, uint32_t dropout_k1, const uint32_t* keep, void* stream) {
+    return attention_bwd(dtype, mask, batch, heads, seq, head_dim, q, k, v, ld_qkv, out, d_out, ld_out, lse, delta, dq, dk, dv, ld_dqkv,
+                         key_len, dropout_p, dropout_k0, dropout_k1, keep, stream);
 }

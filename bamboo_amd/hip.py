@@ -25,7 +25,7 @@ LN_CODES = {"standard": LN_STANDARD, "annotated": LN_ANNOTATED}
 EXPORTS = (
     "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_grouped_sums", "bb_partial_sums_acc", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
     "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_rows", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
-    "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_attention_probs_supported", "bb_attention_probs_fwd", "bb_attention_probs_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
+    "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_attention_keep_words", "bb_attention_fwd_keep", "bb_attention_bwd_keep", "bb_attention_probs_supported", "bb_attention_probs_fwd", "bb_attention_probs_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
     "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_operands", "bb_plan_launches", "bb_plan_launch", "bb_plan_launch_on", "bb_plan_destroy",
     "bb_adam_multi", "bb_adam_multi_scaled", "bb_grad_clip_workspace", "bb_grad_clip_coef", "bb_cast", "bb_fill_f32",
 )
@@ -111,6 +111,10 @@ def lib():
     L.bb_attention_bwd.argtypes = [c_int] * 6 + [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_float, c_uint32,
                                    c_uint32, c_void_p]
+    L.bb_attention_keep_words.argtypes = [c_int] * 3
+    L.bb_attention_keep_words.restype = c_int64
+    for plain, kept in ((L.bb_attention_fwd, L.bb_attention_fwd_keep), (L.bb_attention_bwd, L.bb_attention_bwd_keep)):
+        kept.argtypes = plain.argtypes[:-1] + [c_void_p, c_void_p]
     L.bb_attention_probs_supported.argtypes = [c_int] * 5
     L.bb_attention_probs_fwd.argtypes = [c_int] * 6 + [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
                                          c_void_p, c_float, c_uint32, c_uint32, c_void_p]
@@ -513,32 +517,43 @@ def _check_attention(what, qkv, batch, heads, seq, key_len, lse, out=None, d_out
     _vector(what, batch, torch.int32, key_len=key_len)
 
 
-def attention_fwd(qkv, out, lse, batch, heads, seq, mask, key_len=None, stream=None, dropout=None):
+def attention_keep_words(batch, heads, seq):
+    """int32 words of the kept dropout decisions of :func:`attention_fwd`."""
+    return lib().bb_attention_keep_words(batch, heads, seq)
+
+
+def attention_fwd(qkv, out, lse, batch, heads, seq, mask, key_len=None, stream=None, dropout=None, keep=None):
     """qkv: [batch*seq, 3*heads*d] (Q | K | V thirds), out: [batch*seq, heads*d], lse: fp32 [batch, heads, seq]; head
     dimension d = 64 or 128, or 32 with an even number of heads.
-    ``dropout=(p, (k0, k1))``: dropout on the probabilities with the decisions of that key."""
+    ``dropout=(p, (k0, k1))``: dropout on the probabilities with the decisions of that key; ``keep``: int32
+    [attention_keep_words], takes them for the backward."""
     _check_attention("attention_fwd", qkv, batch, heads, seq, key_len, lse, out=out)
+    if keep is not None:
+        _vector("attention_fwd", attention_keep_words(batch, heads, seq), torch.int32, keep=keep)
     h = qkv.shape[1] // 3
     es = qkv.element_size()
     q = qkv.data_ptr()
-    check(lib().bb_attention_fwd(dtype_code(qkv.dtype), mask, batch, heads, seq, qkv.shape[1] // (3 * heads),
-                                 c_void_p(q), c_void_p(q + h * es), c_void_p(q + 2 * h * es), qkv.stride(0), _ptr(out),
-                                 out.stride(0), _ptr(lse), _ptr(key_len), *_drop_args(dropout), stream_ptr(stream)),
+    check(lib().bb_attention_fwd_keep(dtype_code(qkv.dtype), mask, batch, heads, seq, qkv.shape[1] // (3 * heads),
+                                      c_void_p(q), c_void_p(q + h * es), c_void_p(q + 2 * h * es), qkv.stride(0), _ptr(out),
+                                      out.stride(0), _ptr(lse), _ptr(key_len), *_drop_args(dropout), _ptr(keep), stream_ptr(stream)),
           "bb_attention_fwd")
 
 
-def attention_bwd(qkv, out, d_out, lse, delta, d_qkv, batch, heads, seq, mask, key_len=None, stream=None, dropout=None):
+def attention_bwd(qkv, out, d_out, lse, delta, d_qkv, batch, heads, seq, mask, key_len=None, stream=None, dropout=None, keep=None):
+    """``keep``: the decisions that the forward kept (None: they are made again from the key)."""
     _check_attention("attention_bwd", qkv, batch, heads, seq, key_len, lse, out=out, d_out=d_out, delta=delta, d_qkv=d_qkv)
     if d_out.stride(0) != out.stride(0):
         raise HipKernelError("attention_bwd: out and d_out must share one leading dimension")
+    if keep is not None:
+        _vector("attention_bwd", attention_keep_words(batch, heads, seq), torch.int32, keep=keep)
     h = qkv.shape[1] // 3
     es = qkv.element_size()
     q, dq = qkv.data_ptr(), d_qkv.data_ptr()
-    check(lib().bb_attention_bwd(dtype_code(qkv.dtype), mask, batch, heads, seq, qkv.shape[1] // (3 * heads),
-                                 c_void_p(q), c_void_p(q + h * es), c_void_p(q + 2 * h * es), qkv.stride(0), _ptr(out),
-                                 _ptr(d_out), out.stride(0), _ptr(lse), _ptr(delta), c_void_p(dq),
-                                 c_void_p(dq + h * es), c_void_p(dq + 2 * h * es), d_qkv.stride(0), _ptr(key_len),
-                                 *_drop_args(dropout), stream_ptr(stream)), "bb_attention_bwd")
+    check(lib().bb_attention_bwd_keep(dtype_code(qkv.dtype), mask, batch, heads, seq, qkv.shape[1] // (3 * heads),
+                                      c_void_p(q), c_void_p(q + h * es), c_void_p(q + 2 * h * es), qkv.stride(0), _ptr(out),
+                                      _ptr(d_out), out.stride(0), _ptr(lse), _ptr(delta), c_void_p(dq),
+                                      c_void_p(dq + h * es), c_void_p(dq + 2 * h * es), d_qkv.stride(0), _ptr(key_len),
+                                      *_drop_args(dropout), _ptr(keep), stream_ptr(stream)), "bb_attention_bwd")
 
 
 def attention_probs_supported(dtype, batch, heads, seq, head_dim):

@@ -224,15 +224,21 @@ class TransformerLayer:
         those that lie that close to zero, one in some millions, the gradient of the unit comes or goes."""
         return self.activation != "relu" and hip.attention_probs_supported(ctx.dtype, ctx.batch, self.heads, ctx.seq, self.head_dim)
 
+    def _attention_stash(self, ctx, tag=""):
+        """What the attention keeps for its backward."""
+        if not self.fused_attention(ctx):
+            return [(f"prob{tag}", (ctx.batch, self.heads, ctx.seq, ctx.seq), ctx.dtype)]
+        keep = [(f"keep{tag}", (hip.attention_keep_words(ctx.batch, self.heads, ctx.seq),), torch.int32)] if self.dropout > 0 else []
+        return [(f"lse{tag}", (ctx.batch, self.heads, ctx.seq), torch.float32), *keep]
+
     def stash_specs(self, ctx):
         R, h, f = ctx.rows, self.hidden, self.ffn
         dt, f32 = ctx.dtype, torch.float32
-        attn = ("lse", (ctx.batch, self.heads, ctx.seq), f32) if self.fused_attention(ctx) else \
-            ("prob", (ctx.batch, self.heads, ctx.seq, ctx.seq), dt)
+        attn = self._attention_stash(ctx)
         # ReLU's derivative is read off its kept output (relu'(u) = [relu(u) > 0]); other activations keep act'
         dact = [] if self.activation == "relu" else [("dact", (R, f), dt)]
         return [
-            ("n1", (R, h), dt), ("qkv", (R, 3 * h), dt), attn,
+            ("n1", (R, h), dt), ("qkv", (R, 3 * h), dt), *attn,
             ("ctx", (R, h), dt), ("x1", (R, h), dt), ("n2", (R, h), dt),
             *dact, ("act", (R, f), dt), ("out", (R, h), dt),
             ("mean1", (R,), f32), ("rinv1", (R,), f32), ("mean2", (R,), f32), ("rinv2", (R,), f32),
@@ -291,14 +297,14 @@ class TransformerLayer:
                          ctx.batch, self.heads, alpha=alpha, stream=ctx.stream)
 
     def _attention_fwd(self, st, ctx, site=0, mask=None):
-        """``st``: the entries ``qkv`` ([rows, 3h]: queries, keys, values side by side), ``ctx`` and ``lse`` / ``prob``;
+        """``st``: the entries ``qkv`` ([rows, 3h]: queries, keys, values side by side), ``ctx`` and ``lse``, ``keep`` / ``prob``;
         ``site``: the dropout site of the probabilities; ``mask``: the layer's own unless given."""
         h, d, s = self.hidden, self.head_dim, ctx.seq
         mask = self.mask if mask is None else mask
         drop = self._drop(ctx, site)
         if self.fused_attention(ctx):
             hip.attention_fwd(st["qkv"], st["ctx"], st["lse"], ctx.batch, self.heads, s, hip.MASK_CODES[mask],
-                              ctx.key_len if mask == "key_padding" else None, stream=ctx.stream, dropout=drop)
+                              ctx.key_len if mask == "key_padding" else None, stream=ctx.stream, dropout=drop, keep=st.get("keep"))
             return
         if self.kept_probs_kernels(ctx):
             hip.attention_probs_fwd(st["qkv"], st["ctx"], st["prob"], ctx.batch, self.heads, s, hip.MASK_CODES[mask],
@@ -330,7 +336,7 @@ class TransformerLayer:
             delta = ctx.buf("attn_delta", (ctx.batch, self.heads, s))
             hip.attention_bwd(st["qkv"], st["ctx"], d_ctx, st["lse"], delta, d_qkv, ctx.batch, self.heads, s,
                               hip.MASK_CODES[mask], ctx.key_len if mask == "key_padding" else None, stream=ctx.stream,
-                              dropout=drop)
+                              dropout=drop, keep=st.get("keep"))
             return
         if self.kept_probs_kernels(ctx):
             hip.attention_probs_bwd(st["qkv"], d_ctx, st["prob"], ctx.buf("d_prob", tuple(st["prob"].shape)), d_qkv, ctx.batch,
@@ -518,13 +524,10 @@ class DecoderLayer(TransformerLayer):
     def stash_specs(self, ctx):
         R, h, f = ctx.rows, self.hidden, self.ffn
         dt, f32 = ctx.dtype, torch.float32
-        fused = self.fused_attention(ctx)
-        attn = lambda tag: (f"lse{tag}", (ctx.batch, self.heads, ctx.seq), f32) if fused else \
-            (f"prob{tag}", (ctx.batch, self.heads, ctx.seq, ctx.seq), dt)
         dact = [] if self.activation == "relu" else [("dact", (R, f), dt)]
         return [
-            ("n1", (R, h), dt), ("qkv", (R, 3 * h), dt), attn(""), ("ctx", (R, h), dt), ("x1", (R, h), dt),
-            ("mem", (R, h), dt), ("n_src", (R, h), dt), ("qkv_src", (R, 3 * h), dt), attn("_src"), ("ctx_src", (R, h), dt),
+            ("n1", (R, h), dt), ("qkv", (R, 3 * h), dt), *self._attention_stash(ctx), ("ctx", (R, h), dt), ("x1", (R, h), dt),
+            ("mem", (R, h), dt), ("n_src", (R, h), dt), ("qkv_src", (R, 3 * h), dt), *self._attention_stash(ctx, "_src"), ("ctx_src", (R, h), dt),
             ("x2", (R, h), dt), ("n2", (R, h), dt), *dact, ("act", (R, f), dt), ("out", (R, h), dt),
             ("mean1", (R,), f32), ("rinv1", (R,), f32), ("mean_src", (R,), f32), ("rinv_src", (R,), f32),
             ("mean2", (R,), f32), ("rinv2", (R,), f32),
@@ -542,7 +545,8 @@ class DecoderLayer(TransformerLayer):
         return batch * seq * (16 * h * h + 4 * h * f) + 8 * batch * seq * seq * h
 
     def _src_views(self, st):
-        return {"qkv": st["qkv_src"], "ctx": st["ctx_src"], "lse": st.get("lse_src"), "prob": st.get("prob_src")}
+        return {"qkv": st["qkv_src"], "ctx": st["ctx_src"], "lse": st.get("lse_src"), "prob": st.get("prob_src"),
+                "keep": st.get("keep_src")}
 
     def forward(self, x, st, ctx):
         self.rebuild(x, st, ctx)

@@ -267,6 +267,18 @@ int bb_attention_bwd(int dtype, int mask, int batch, int heads, int seq, int hea
                      int64_t ld_out, const float* lse, float* delta, void* dq, void* dk, void* dv,
                      int64_t ld_dqkv, const int32_t* key_len, float dropout_p, uint32_t dropout_k0, uint32_t dropout_k1, void* stream);
 
+/* Both with the dropout decisions kept as bits: the forward writes them to keep (bb_attention_keep_words(batch, heads, seq) words,
+ * aligned to 128 bytes; those of pairs that no tile of the forward reaches stay as they were), the backward, given the same
+ * shapes and dropout_p > 0, reads them instead of making the decisions again.  Same results.  keep may be null.            */
+int64_t bb_attention_keep_words(int batch, int heads, int seq);
+int bb_attention_fwd_keep(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k, const void* v,
+                          int64_t ld_qkv, void* out, int64_t ld_out, float* lse, const int32_t* key_len, float dropout_p,
+                          uint32_t dropout_k0, uint32_t dropout_k1, uint32_t* keep, void* stream);
+int bb_attention_bwd_keep(int dtype, int mask, int batch, int heads, int seq, int head_dim, const void* q, const void* k, const void* v,
+                          int64_t ld_qkv, const void* out, const void* d_out, int64_t ld_out, const float* lse, float* delta, void* dq,
+                          void* dk, void* dv, int64_t ld_dqkv, const int32_t* key_len, float dropout_p, uint32_t dropout_k0,
+                          uint32_t dropout_k1, const uint32_t* keep, void* stream);
+
 /* The same attention with the probabilities kept (fp32; head_dim 32, 64 or 128, seq a multiple of 4 and at most 1024;
  * bb_attention_probs_supported: and this is the faster way).  prob: [batch, heads, seq, seq], written in full by the forward,
  * in front of dropout; the backward reads it and leaves the gradient of the scaled scores in d_score (same size; key tiles
