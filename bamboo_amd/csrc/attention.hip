@@ -1119,29 +1119,51 @@ struct attn_bwd_launch {
         return BB_OK;
     }
 };
-// The shape of a block, by the number of blocks of 128 rows and the length of the walk.  Four
-// waves / four waves in two groups / two in four (us, forward, backward; pairs of heads on the same waves, see below): 12 heads of 64, 2043 keys (192 blocks) 27 78 / 20 64 /
-// 24 78; 4 x 16 heads, 512 causal (256) 13.4 31.5 / 10.8 29.7 / 12.1 35.0; 2 x 25 heads, 300 (150) 7.4 20.7 / 7.7 23.3 / 9.6 24.2;
-// 16 heads, 1024 causal (128) 22.1 50.4 / 16.2 42.7 / 11.1 29.8; 2 x 4 heads, 512 causal (32) 12.7 29.4 / 10.3 27.6 / 7.6 20.8; 4
-// heads, 1024 causal with dropout (32) 28.3 80.5 / 24.3 65.6 / 15.2 40.7; 6 x 8 heads, 175 (96) 7.1 17.2 / 7.2 19.9 / 6.2 17.3; 8
-// x 8 pairs of 32, 128, dropout (64) 8.6 23.9 / 8.9 24.7 / 7.4 23.4; 2 x 16 heads, 100 (32) 5.8 14.0 / 5.9 16.4 / 5.6 15.7.  Heads of
-// 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.  Pairs of heads have twice the waves: two
-// a head in two groups (a walk of both heads by two waves in four groups / this: 1 x 4 pairs, 500 causal 9.6 16.4 / 8.3 15.3, 2 x 4,
-// 300, padding, dropout 9.6 20.7 / 7.8 17.0; four waves in two groups / four a head: 4 x 8, 512 causal 10.6 24.8 / 9.2 22.4).
+// The shape of a block (waves W of 32 rows x groups G), by the number of blocks of 128 rows and the length of the walk.  Device time in us:
+//                                         forward, W x G                        backward
+//   blocks, heads                  4x1   4x2   2x4   2x2   2x1           4x1   4x2   2x4   2x2   2x1
+//    24  1 x 2,   1500 causal     25.7  22.3  14.9  17.4  25.6          46.9  39.2  30.1  33.0  48.1
+//    32  2 x 4,    512 causal     11.3  10.6   7.7   8.2  10.8          19.5  18.3  14.6  14.7  18.1
+//   128  2 x 8,   1024 causal     18.8  16.9  11.5  12.8  18.7          33.9  29.4  27.8  25.7  34.3
+//   128  4 x 16,   200 causal      7.3   7.2   6.3   6.2   6.6          12.9  13.2  16.8  14.2  12.1
+//   150  2 x 25,   300 padding     8.0   8.2  11.0   7.7   8.0          16.6  22.7  24.0  18.2  15.5
+//   192  1 x 12,  2043 padding    29.2  25.2  31.3  23.3  36.0          67.5  63.2  78.5  87.3   110
+//   240  3 x 10,  1000 causal     19.0  17.0  16.2  13.7  19.2          36.8  40.5  42.2  40.9  38.3
+//   256  4 x 16,   512 causal     11.8  11.1  12.7   9.1  11.4          23.1  28.3  34.1  30.7  23.7
+//   320  2 x 20,  1024 causal     19.7  18.3  22.1  14.9  19.7          49.2  45.3  58.2  55.6  49.2
+//   352  1 x 22,  2000 causal     34.0  29.8  34.8  25.1  34.8          84.5  70.5  85.6  91.9  86.1
+//   384  8 x 12,   512 causal     12.6  13.0  18.8  13.9  12.8          32.7  42.7  51.7  46.8  33.7
+//   384  4 x 12,  1024 padding    22.5  23.4  31.3  26.5  23.2          61.5  76.3  80.0  82.7  60.6
+//   400  1 x 25,  2048 causal     57.4  55.3  65.5  49.5  73.9           118   104   129   148   121      (dropout)
+//   512  8 x 16,   512 causal     13.3  13.6  24.0  15.3  13.6          34.1  47.8  68.6  61.4  37.6
+//    96  6 x 8,    175, no mask    6.6                     6.2          11.0                    10.4
+//   128  2 x 8,   1024, no mask   18.5                    18.6          33.4                    34.2
+// Few blocks want their walks shared by groups, and small blocks, which also even out long and short walks under a causal mask; the
+// backward, whose waves look ahead by themselves, only where the walk is long, and it loses the launch that both passes share.
+// Heads of 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.  Pairs of heads have twice the
+// waves: two a head in two groups (a walk of both heads by two waves in four groups / this: 1 x 4 pairs, 500 causal 9.6 16.4 / 8.3 15.3,
+// 2 x 4, 300, padding, dropout 9.6 20.7 / 7.8 17.0; four waves in two groups / four a head: 4 x 8, 512 causal 10.6 24.8 / 9.2 22.4).
 // Attention without a mask keeps the one walk.  Groups add the same terms in another order: as near the exact sums as before, but
 // not the same last bits, and the stage that ends the reference's script (no mask; a LayerNorm whose rows are summed up, which
 // cancels to 1e-4 of its terms) passes gradients on in which such bits show as 3 to 5 %.
 template <typename L, int HP, int NPAN> static int attn_shape(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
     const int64_t blocks = (int64_t)nbh * ((seq + 127) / 128);
-    if (a.mask != BB_MASK_NONE) {
-        if constexpr (HP == 2) {
-            if (blocks <= 128 && seq >= 160) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
-        } else {
-            if constexpr (NPAN == 1) {
-                if (blocks <= 128 && seq >= 160) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
-            }
-            if (blocks <= 256 && seq >= 448) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
+    const bool masked = a.mask != BB_MASK_NONE;
+    if constexpr (HP == 2) {
+        if (masked && blocks <= 128 && seq >= 160) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
+    } else if constexpr (NPAN == 2) {
+        if (masked && blocks <= 256 && seq >= 448) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
+    } else if constexpr (std::is_same_v<L, attn_fwd_launch>) {
+        if (masked && seq >= 160) {
+            if (blocks <= 128) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
+            if (blocks <= 256 || (blocks <= 400 && seq >= 1024 && a.mask == BB_MASK_CAUSAL)) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
         }
+        if (blocks <= 128 && seq <= 320) return L::template go<HP, NPAN, 2, 1>(seq, nbh, a, st);
+    } else {
+        if (masked && seq >= 1536 && blocks > 128 && blocks <= 400) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
+        if (masked && seq >= 448 && blocks > 64 && blocks <= 128) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
+        if (masked && seq >= 320 && blocks <= 64) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
+        if (blocks <= 128 && seq <= 320) return L::template go<HP, NPAN, 2, 1>(seq, nbh, a, st);
     }
     return L::template go<HP, NPAN, 4, 1>(seq, nbh, a, st);
 }

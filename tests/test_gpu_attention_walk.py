@@ -10,7 +10,7 @@ from tests import test_gpu_kernels as plain
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 2, 31, 64), (2, 1, 32, 64), (1, 3, 33, 64), (1, 2, 63, 32), (2, 2, 65, 32), (1, 2, 96, 128), (1, 1, 97, 64), (3, 2, 129, 64),
-          (1, 4, 191, 32), (2, 6, 385, 32), (2, 260, 161, 64), (1, 600, 129, 64)]   # the last two beyond a round
+          (1, 4, 191, 32), (2, 6, 385, 32), (1, 150, 70, 64), (1, 24, 1025, 64), (2, 260, 161, 64), (1, 600, 129, 64)]   # the last two beyond a round
 
 
 @pytest.mark.parametrize("mask", ["none", "causal", "key_padding"])
