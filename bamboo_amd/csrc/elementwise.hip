@@ -33,6 +33,19 @@ extern "C" int bb_init(void) {
     return ln_bwd_static_setup(dev);   // so that bb_layernorm_bwd_static has nothing left to set up on this device
 }
 
+// 16 raw bytes -> VEC floats
+__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(t[i]);
+}
+__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(t[i] << 16);
+        v[2 * i + 1] = __uint_as_float(t[i] & 0xffff0000u);
+    }
+}
+
 // =========================================================================================
 // LayerNorm
 // =========================================================================================
@@ -41,20 +54,38 @@ template <typename T, int IT>
 __global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, int cols, float eps,
                                                             const T* __restrict__ x, const T* __restrict__ gain,
                                                             const T* __restrict__ shift, T* __restrict__ y,
-                                                            float* __restrict__ mean_out, float* __restrict__ rinv_out) {
+                                                            float* __restrict__ mean_out, float* __restrict__ rinv_out,
+                                                            T* __restrict__ memory) {
     constexpr int VEC = Elem<T>::VEC;
+    constexpr bool EARLY = IT <= 4;
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int nvec = cols / VEC;
     const T* xr = x + (int64_t)row * cols;
     float v[IT][VEC];
+    u32x4 graw[EARLY ? IT : 1], sraw[EARLY ? IT : 1];
     float s = 0.f;
+    if constexpr (EARLY) {
+        // behind the sums each would be another trip to memory
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int c = min(lane + i * 64, nvec - 1);
+            graw[i] = *(const u32x4*)(gain + c * VEC);
+            sraw[i] = *(const u32x4*)(shift + c * VEC);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         const int c = lane + i * 64;
         if (c < nvec) {
             load_vec(xr + c * VEC, v[i]);
+            if (memory) {      // as sqrt1m_fwd_kernel, whose launch and pass over x are saved
+                float mv[VEC];
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) mv[e] = sqrtf(1.0f - v[i][e]);
+                store_vec(memory + (int64_t)row * cols + c * VEC, mv);
+            }
 #pragma unroll
             for (int e = 0; e < VEC; ++e) s += v[i][e];
         } else {
@@ -91,8 +122,13 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, 
         const int c = lane + i * 64;
         if (c < nvec) {
             float gv[VEC], bv[VEC], o[VEC];
-            load_vec(gain + c * VEC, gv);
-            load_vec(shift + c * VEC, bv);
+            if constexpr (EARLY) {
+                unpack16(graw[i], gv);
+                unpack16(sraw[i], bv);
+            } else {
+                load_vec(gain + c * VEC, gv);
+                load_vec(shift + c * VEC, bv);
+            }
 #pragma unroll
             for (int e = 0; e < VEC; ++e) o[e] = gv[e] * ((v[i][e] - mean) * rinv) + bv[e];
             store_vec(yr + c * VEC, o);
@@ -104,19 +140,6 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, 
 template <int N> __device__ __forceinline__ void store_f32s(float* dst, const float* v) {
 #pragma unroll
     for (int e = 0; e < N; e += 4) *(f32x4*)(dst + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
-}
-
-// 16 raw bytes -> VEC floats
-__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(t[i]);
-}
-__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[8]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __uint_as_float(t[i] << 16);
-        v[2 * i + 1] = __uint_as_float(t[i] & 0xffff0000u);
-    }
 }
 
 constexpr int LN_BWD_BLOCKS = 256;
@@ -142,14 +165,15 @@ template <int VEC> __device__ __forceinline__ void drop_vec(const DropKey& key, 
 // dx per row, dgain/dshift partial sums per block (fixed row->block assignment).
 // DROP: dropped = dropout(dx) as well, what dropout_kernel makes of the stored dx: its launch, and its pass over dx, are saved
 // (two launches / one, bf16, us: 8192x1024 21.0 / 16.7, 4096x1600 20.9 / 18.6, 2048x4096 34.3 / 32.4)
-template <typename T, int IT, bool DROP>
+// MEMORY: dx takes what sqrt1m_bwd_kernel would add to it, as stored (m = sqrt(1 - x), dm its gradient)
+template <typename T, int IT, bool DROP, bool MEMORY>
 __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_kernel(int kind, int rows, int cols, float eps,
                                                             const T* __restrict__ x, const T* __restrict__ gain,
                                                             const float* __restrict__ mean_in,
                                                             const float* __restrict__ rinv_in, const T* __restrict__ dy,
                                                             const T* __restrict__ dres, T* __restrict__ dx,
                                                             float* __restrict__ partial, int one_pass, T* __restrict__ dropped,
-                                                            const DropKey key) {
+                                                            const DropKey key, const T* __restrict__ dm, const T* __restrict__ m) {
     constexpr int VEC = Elem<T>::VEC, LN_BWD_WAVES = ln_bwd_waves<T, IT>();
     extern __shared__ float red[];  // [all waves][2][cols] (one pass) or [3 waves][2][cols] for the cross-wave sum
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -167,12 +191,19 @@ __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_ke
         const T* xr = x + (int64_t)row * cols;
         const T* dyr = dy + (int64_t)row * cols;
         float xh[IT][VEC], dyh[IT][VEC];
+        u32x4 rdm[MEMORY ? IT : 1], rm[MEMORY ? IT : 1];
         u32x4 rres[IT];   // the residual gradient, fetched with the row (16 bytes per vector, unpacked at the end)
         float s1 = 0.f, s2 = 0.f;
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
             const int c = lane + i * 64;
             if (dres && c < nvec) rres[i] = *(const u32x4*)(dres + (int64_t)row * cols + c * VEC);
+            if constexpr (MEMORY) {
+                if (c < nvec) {
+                    rdm[i] = *(const u32x4*)(dm + (int64_t)row * cols + c * VEC);
+                    rm[i] = *(const u32x4*)(m + (int64_t)row * cols + c * VEC);
+                }
+            }
         }
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
@@ -218,10 +249,8 @@ __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_ke
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) o[e] += rv[e];
                 }
-                store_vec(dxr + c * VEC, o);
-                if constexpr (DROP) {
-                    const int64_t first = (int64_t)row * cols + c * VEC;
-                    if constexpr (sizeof(T) == 2) {   // as stored
+                auto as_stored = [&]() {
+                    if constexpr (sizeof(T) == 2) {
 #pragma unroll
                         for (int e = 0; e < VEC; e += 2) {
                             const uint32_t pair = pack2bf(o[e], o[e + 1]);
@@ -229,6 +258,19 @@ __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_ke
                             o[e + 1] = __uint_as_float(pair & 0xffff0000u);
                         }
                     }
+                };
+                if constexpr (MEMORY) {
+                    float g[VEC], mv[VEC];
+                    unpack16(rdm[i], g);
+                    unpack16(rm[i], mv);
+                    as_stored();
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) o[e] += g[e] * (-0.5f / mv[e]);
+                }
+                store_vec(dxr + c * VEC, o);
+                if constexpr (DROP) {
+                    const int64_t first = (int64_t)row * cols + c * VEC;
+                    as_stored();
                     drop_vec<VEC>(key, first, o);
                     store_vec(dropped + first, o);
                 }
@@ -369,16 +411,16 @@ extern "C" int bb_partial_sums_acc(const bb_partial_sums* sums, int count, void*
 
 template <typename T, int IT>
 static int ln_fwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift,
-                         void* y, float* mean, float* rinv, hipStream_t st) {
+                         void* y, float* mean, float* rinv, void* memory, hipStream_t st) {
     bb_launch((layernorm_fwd_kernel<T, IT>), dim3((rows + 3) / 4), dim3(256), 0, st, kind, rows, cols, eps,
-                       (const T*)x, (const T*)gain, (const T*)shift, (T*)y, mean, rinv);
+                       (const T*)x, (const T*)gain, (const T*)shift, (T*)y, mean, rinv, (T*)memory);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
 template <typename T, int IT>
 static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const float* mean,
                          const float* rinv, const void* dy, const void* dres, void* dx, float* ws, int& blocks, hipStream_t st,
-                         void* dropped, const DropKey& key) {
+                         void* dropped, const DropKey& key, const void* dm, const void* m) {
     constexpr int LN_BWD_WAVES = ln_bwd_waves<T, IT>();
     // a row per wave: blocks past the last row would only write zeros for the reduction to read (us, backward with its
     // reduction, 256 blocks / as many as have rows: bf16 128 x 128 6.4 / 5.8, 300 x 768 8.5 / 7.5, 1024 x 512 7.2 / 6.7, 333 x 5120
@@ -387,10 +429,10 @@ static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x,
     const size_t all = (size_t)LN_BWD_WAVES * 2 * cols * sizeof(float);
     const int one_pass = all <= 128 * 1024;
     const size_t smem = one_pass ? all : (size_t)3 * 2 * cols * sizeof(float);
-    auto kern = key.thresh ? layernorm_bwd_kernel<T, IT, true> : layernorm_bwd_kernel<T, IT, false>;
+    auto kern = dm ? layernorm_bwd_kernel<T, IT, false, true> : key.thresh ? layernorm_bwd_kernel<T, IT, true, false> : layernorm_bwd_kernel<T, IT, false, false>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));   // raised on the first (never captured) call that needs it
     bb_launch(kern, dim3(blocks), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
-                       (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass, (T*)dropped, key);
+                       (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass, (T*)dropped, key, (const T*)dm, (const T*)m);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -413,8 +455,8 @@ static int check_rowop(const char* name, int dtype, int rows, int cols) {
     return BB_OK;
 }
 
-extern "C" int bb_layernorm_fwd(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
-                                const void* shift, void* y, float* mean, float* rinv, void* stream) {
+static int layernorm_fwd(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift, void* y,
+                         float* mean, float* rinv, void* memory, void* stream) {
     int rc = check_rowop("bb_layernorm_fwd", dtype, rows, cols);
     if (rc) return rc;
     BB_REQUIRE(kind == BB_LN_STANDARD || kind == BB_LN_ANNOTATED, "bb_layernorm_fwd: bad kind %d", kind);
@@ -423,10 +465,18 @@ extern "C" int bb_layernorm_fwd(int dtype, int kind, int rows, int cols, float e
     if (rows == 0) return BB_OK;
     hipStream_t st = (hipStream_t)stream;
     if (dtype == BB_BF16)
-        BB_DISPATCH_IT(bf16, cols / 8, (ln_fwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, shift, y, mean, rinv, st)));
+        BB_DISPATCH_IT(bf16, cols / 8, (ln_fwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, shift, y, mean, rinv, memory, st)));
     else
-        BB_DISPATCH_IT(float, cols / 4, (ln_fwd_launch<float, IT>(kind, rows, cols, eps, x, gain, shift, y, mean, rinv, st)));
+        BB_DISPATCH_IT(float, cols / 4, (ln_fwd_launch<float, IT>(kind, rows, cols, eps, x, gain, shift, y, mean, rinv, memory, st)));
     return BB_EINVAL;
+}
+extern "C" int bb_layernorm_fwd(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
+                                const void* shift, void* y, float* mean, float* rinv, void* stream) {
+    return layernorm_fwd(dtype, kind, rows, cols, eps, x, gain, shift, y, mean, rinv, nullptr, stream);
+}
+extern "C" int bb_layernorm_fwd_memory(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift,
+                                       void* y, float* mean, float* rinv, void* memory, void* stream) {
+    return layernorm_fwd(dtype, kind, rows, cols, eps, x, gain, shift, y, mean, rinv, memory, stream);
 }
 
 extern "C" int64_t bb_layernorm_bwd_workspace(int cols) { return (int64_t)LN_BWD_BLOCKS * 2 * cols; }
@@ -434,7 +484,7 @@ extern "C" int64_t bb_layernorm_bwd_workspace(int cols) { return (int64_t)LN_BWD
 // blocks leaves their number, and the first launch of the two goes out; the second adds up what they left
 static int ln_bwd_rows(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
                        const float* mean, const float* rinv, const void* dy, const void* dres, void* dx, float* workspace, int& blocks,
-                       hipStream_t st, void* dropped = nullptr, const DropKey& key = DropKey{}) {
+                       hipStream_t st, void* dropped = nullptr, const DropKey& key = DropKey{}, const void* dm = nullptr, const void* m = nullptr) {
     blocks = 0;
     int rc = check_rowop(who, dtype, rows, cols);
     if (rc) return rc;
@@ -443,9 +493,9 @@ static int ln_bwd_rows(const char* who, int dtype, int kind, int rows, int cols,
     BB_REQUIRE((size_t)3 * 2 * cols * sizeof(float) <= 160 * 1024, "%s: cols (%d) too large (max 6826)", who, cols);
     if (rows == 0) return BB_OK;
     if (dtype == BB_BF16)
-        BB_DISPATCH_IT(bf16, cols / 8, (ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st, dropped, key)));
+        BB_DISPATCH_IT(bf16, cols / 8, (ln_bwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st, dropped, key, dm, m)));
     else
-        BB_DISPATCH_IT(float, cols / 4, (ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st, dropped, key)));
+        BB_DISPATCH_IT(float, cols / 4, (ln_bwd_launch<float, IT>(kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, workspace, blocks, st, dropped, key, dm, m)));
     return BB_EINVAL;
 }
 static int ln_bwd_run(const char* who, int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
@@ -484,6 +534,15 @@ extern "C" int bb_layernorm_bwd_rows(int dtype, int kind, int rows, int cols, fl
                        (hipStream_t)stream, dropped, key);
 }
 
+extern "C" int bb_layernorm_bwd_rows_memory(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain,
+                                            const float* mean, const float* rinv, const void* dy, const void* dres, void* dx, float* dgain,
+                                            float* dshift, float* partials, bb_partial_sums* sums, const void* dm, const void* m, void* stream) {
+    BB_REQUIRE(dgain && dshift && sums && dm && m, "bb_layernorm_bwd_rows_memory: null pointer");
+    *sums = {partials, dgain, dshift, 0, cols};
+    return ln_bwd_rows("bb_layernorm_bwd_rows_memory", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, partials, sums->parts,
+                       (hipStream_t)stream, nullptr, DropKey{}, dm, m);
+}
+
 // ---- the same for callers that cannot allocate ---------------------------------------------------------------
 // The per-block partial sums of dgain / dshift ([LN_BWD_BLOCKS][2][cols] floats) live in an array that is part of the
 // library's device image instead of a caller's workspace.  Every GPU the library runs on holds its own copy (4 MiB,
@@ -498,7 +557,7 @@ static std::mutex g_ln_static_mu;
 
 template <typename T, int IT> static hipError_t ln_bwd_allow_one_pass() {
     // the largest dynamic LDS request the kernel makes for cols <= BB_LN_BWD_STATIC_MAX_COLS: the one-pass layout
-    return bb_allow_dynamic_lds((const void*)layernorm_bwd_kernel<T, IT, false>, 128 * 1024);
+    return bb_allow_dynamic_lds((const void*)layernorm_bwd_kernel<T, IT, false, false>, 128 * 1024);
 }
 // once per device, with that device current: the address of the device's copy, and every LDS-limit change the
 // entry point could otherwise need on its first call

@@ -25,7 +25,7 @@ LN_CODES = {"standard": LN_STANDARD, "annotated": LN_ANNOTATED}
 EXPORTS = (
     "bb_version", "bb_last_error", "bb_init", "bb_gemm", "bb_gemm_grouped", "bb_gemm_grouped_sums", "bb_partial_sums_acc", "bb_gemm_splitk_workspace", "bb_gemm_grouped_splitk", "bb_gemm_variant", "bb_layernorm_fwd",
     "bb_layernorm_bwd_workspace", "bb_layernorm_bwd", "bb_layernorm_bwd_rows", "bb_layernorm_bwd_static", "bb_colsum_workspace", "bb_colsum_acc", "bb_rowsum_fwd", "bb_rowsum_bwd", "bb_dropout_apply", "bb_dropout_keep_host",
-    "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_attention_keep_words", "bb_attention_fwd_keep", "bb_attention_bwd_keep", "bb_attention_probs_supported", "bb_attention_probs_fwd", "bb_attention_probs_bwd", "bb_residual_add", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
+    "bb_softmax_fwd", "bb_softmax_bwd", "bb_attention_fwd", "bb_attention_bwd", "bb_attention_keep_words", "bb_attention_fwd_keep", "bb_attention_bwd_keep", "bb_attention_probs_supported", "bb_attention_probs_fwd", "bb_attention_probs_bwd", "bb_residual_add", "bb_layernorm_fwd_memory", "bb_layernorm_bwd_rows_memory", "bb_sqrt_one_minus_fwd", "bb_sqrt_one_minus_bwd", "bb_act_fwd", "bb_bn_workspace", "bb_batchnorm_fwd", "bb_batchnorm_bwd", "bb_patch3x3", "bb_patch3x3_strided", "bb_subsample", "bb_conv3x3_supported", "bb_conv3x3", "bb_gemm_strip_stats_supported", "bb_strip_stats_workspace", "bb_batchnorm_fwd_strips", "bb_bn_bwd_strips_workspace", "bb_gemm_bn_bwd_supported", "bb_gemm_bn_bwd", "bb_conv3x3_dgrad_bn", "bb_batchnorm_bwd_strips", "bb_batchnorm_bwd_strip_sums", "bb_mse_workspace", "bb_mse_fwd_bwd", "bb_graph_begin", "bb_graph_end", "bb_graph_launch", "bb_graph_destroy",
     "bb_plan_begin", "bb_plan_end", "bb_plan_abort", "bb_plan_dropout", "bb_plan_operands", "bb_plan_launches", "bb_plan_launch", "bb_plan_launch_on", "bb_plan_destroy",
     "bb_adam_multi", "bb_adam_multi_scaled", "bb_grad_clip_workspace", "bb_grad_clip_coef", "bb_cast", "bb_fill_f32",
 )
@@ -123,6 +123,8 @@ def lib():
     L.bb_dropout_apply.argtypes = [c_int, c_int64, c_void_p, c_void_p, c_float, c_uint32, c_uint32, c_void_p]
     L.bb_dropout_keep_host.argtypes = [c_float, c_uint32, c_uint32, c_uint64]
     L.bb_residual_add.argtypes = [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]
+    L.bb_layernorm_fwd_memory.argtypes = L.bb_layernorm_fwd.argtypes[:-1] + [c_void_p, c_void_p]
+    L.bb_layernorm_bwd_rows_memory.argtypes = L.bb_layernorm_bwd_rows.argtypes[:16] + [c_void_p] * 3
     L.bb_sqrt_one_minus_fwd.argtypes = [c_int, c_int64, c_void_p, c_void_p, c_void_p]
     L.bb_sqrt_one_minus_bwd.argtypes = [c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p]
     L.bb_graph_begin.argtypes = [c_void_p]
@@ -383,13 +385,14 @@ def _vector(what, n, dtype, **tensors):
             raise HipKernelError(f"{what}: {name} must hold {n} contiguous elements of {dtype}, got {tuple(t.shape)} {t.dtype}")
 
 # ------------------------------------------------------------------------- row-wise kernels
-def layernorm_fwd(x, gain, shift, y, mean, rinv, kind, eps, stream=None):
+def layernorm_fwd(x, gain, shift, y, mean, rinv, kind, eps, stream=None, memory=None):
+    """``memory``: sqrt(1 - x) as well, as :func:`sqrt_one_minus_fwd` makes it."""
     rows, cols = x.shape
-    _like("layernorm_fwd", x, y=y)
+    _like("layernorm_fwd", x, y=y, memory=memory)
     _vector("layernorm_fwd", cols, x.dtype, gain=gain, shift=shift)
     _vector("layernorm_fwd", rows, torch.float32, mean=mean, rinv=rinv)
-    check(lib().bb_layernorm_fwd(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(shift),
-                                 _ptr(y), _ptr(mean), _ptr(rinv), stream_ptr(stream)), "bb_layernorm_fwd")
+    check(lib().bb_layernorm_fwd_memory(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(shift),
+                                        _ptr(y), _ptr(mean), _ptr(rinv), _ptr(memory), stream_ptr(stream)), "bb_layernorm_fwd")
 
 
 def layernorm_bwd_workspace(cols):
@@ -414,16 +417,27 @@ def layernorm_bwd(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, workspace, k
                                  _ptr(workspace), stream_ptr(stream)), "bb_layernorm_bwd")
 
 
-def layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partials, kind, eps, stream=None, dropped=None, dropout=None):
+def layernorm_bwd_rows(x, gain, mean, rinv, dy, dres, dx, dgain, dshift, partials, kind, eps, stream=None, dropped=None, dropout=None,
+                       memory=None):
     """:func:`layernorm_bwd` without its second launch: the gain and shift gradients are left as sums per block in ``partials``,
     which stays untouched until ``gemm_grouped(sums=)`` or :func:`partial_sums` has added up what this returns.
-    ``dropped``: what ``dropout_apply(dx, dropped, *dropout)`` would make, in the same launch."""
+    ``dropped``: what ``dropout_apply(dx, dropped, *dropout)`` would make, in the same launch; ``memory = (dm, m)``, not with it:
+    ``sqrt_one_minus_bwd(dm, m, dx)``."""
     rows, cols = x.shape
     p, key = dropout if dropped is not None else (0.0, (0, 0))
     _check_ln_bwd("layernorm_bwd_rows", x, gain, mean, rinv, dy, dres, dx, dgain, dshift, dropped)
     if partials.numel() < layernorm_bwd_workspace(cols) or partials.dtype != torch.float32:
         raise HipKernelError("layernorm_bwd_rows: partials too small")
     sums = PartialSums()
+    if memory is not None:
+        dm, m = memory
+        if dropped is not None:
+            raise HipKernelError("layernorm_bwd_rows: a dropped gradient and a memory do not go together")
+        _like("layernorm_bwd_rows", x, dm=dm, m=m)
+        check(lib().bb_layernorm_bwd_rows_memory(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(mean), _ptr(rinv),
+                                                 _ptr(dy), _ptr(dres), _ptr(dx), _ptr(dgain), _ptr(dshift), _ptr(partials), byref(sums),
+                                                 _ptr(dm), _ptr(m), stream_ptr(stream)), "bb_layernorm_bwd_rows_memory")
+        return sums
     check(lib().bb_layernorm_bwd_rows(dtype_code(x.dtype), kind, rows, cols, eps, _ptr(x), _ptr(gain), _ptr(mean), _ptr(rinv), _ptr(dy),
                                       _ptr(dres), _ptr(dx), _ptr(dgain), _ptr(dshift), _ptr(partials), byref(sums), _ptr(dropped), float(p),
                                       int(key[0]), int(key[1]), stream_ptr(stream)), "bb_layernorm_bwd_rows")

@@ -283,13 +283,13 @@ class TransformerLayer:
         h, f = self.hidden, self.ffn
         return batch * seq * (8 * h * h + 4 * h * f) + 4 * batch * seq * seq * h
 
-    def _layernorm_bwd(self, sums, ctx, x, norm, mean, rinv, dy, dres, dx, dropped=None, site=None):
+    def _layernorm_bwd(self, sums, ctx, x, norm, mean, rinv, dy, dres, dx, dropped=None, site=None, memory=None):
         """LayerNorm backward; its gain's and shift's gradients join ``sums``, at most two until the launch that adds them up.
         ``dropped``: the gradient behind the dropout ``site`` of the sublayer in front as well."""
         partials = ctx.scratch[self.LN_PARTIALS[len(sums)]]
         sums.append(hip.layernorm_bwd_rows(x, self.w[norm + ".a_2"], mean, rinv, dy, dres, dx, self.g[norm + ".a_2"], self.g[norm + ".b_2"],
                                            partials, hip.LN_CODES[self.ln], self.eps, stream=ctx.stream, dropped=dropped,
-                                           dropout=None if dropped is None else self._drop(ctx, site)))
+                                           dropout=None if dropped is None else self._drop(ctx, site), memory=memory))
 
     # ------------------------------------------------------------------ attention core
     def _heads_gemm(self, ctx, layout, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, alpha=1.0):
@@ -559,10 +559,9 @@ class DecoderLayer(TransformerLayer):
         kind, act = hip.LN_CODES[self.ln], hip.ACT_CODES[self.activation]
         h = self.hidden
         st["x0"] = x
-        hip.sqrt_one_minus_fwd(x, st["mem"], stream=sm)                                      # gpt2.py:31
-        # sublayer 0: self-attention
+        # sublayer 0: self-attention; the memory (gpt2.py:31) comes with its LayerNorm
         hip.layernorm_fwd(x, w["sublayer.0.norm.a_2"], w["sublayer.0.norm.b_2"], st["n1"], st["mean1"], st["rinv1"],
-                          kind, self.eps, stream=sm)
+                          kind, self.eps, stream=sm, memory=st["mem"])
         ctx.gemm(hip.NT, st["n1"], w["qkv.weight"], st["qkv"], bias=w["qkv.bias"], stream=sm)
         self._attention_fwd(st, ctx, site=self.SITE_ATTENTION)
         ctx.gemm(hip.NT, st["ctx"], w["self_attn.linears.3.weight"], st["x1"], bias=w["self_attn.linears.3.bias"],
@@ -641,8 +640,7 @@ class DecoderLayer(TransformerLayer):
         wgrad(d_qkv, st["n1"], "qkv.weight")
         ctx.gemm(hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
         # d_x = d_x1 + LN0'(d_n1) + d_mem * dm/dx
-        self._layernorm_bwd(sums, ctx, st["x0"], "sublayer.0.norm", st["mean1"], st["rinv1"], d_h0, d_h1, d_x)
-        hip.sqrt_one_minus_bwd(d_mem, st["mem"], d_x, accumulate=True, stream=sm)
+        self._layernorm_bwd(sums, ctx, st["x0"], "sublayer.0.norm", st["mean1"], st["rinv1"], d_h0, d_h1, d_x, memory=(d_mem, st["mem"]))
         flush()
         return d_x
 

@@ -297,6 +297,13 @@ int bb_attention_probs_bwd(int dtype, int mask, int batch, int heads, int seq, i
 int bb_residual_add(int dtype, int64_t n, const void* a, const void* b, void* out,
                     void* stream);
 
+/* bb_layernorm_fwd that leaves memory = sqrt(1 - x) as well (bb_sqrt_one_minus_fwd; memory may be null), and bb_layernorm_bwd_rows, without
+ * dropout, that adds its backward to the stored dx (bb_sqrt_one_minus_bwd: dm the gradient of m = memory).  Same results as two calls. */
+int bb_layernorm_fwd_memory(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift, void* y,
+                            float* mean, float* rinv, void* memory, void* stream);
+int bb_layernorm_bwd_rows_memory(int dtype, int kind, int rows, int cols, float eps, const void* x, const void* gain, const float* mean,
+                                 const float* rinv, const void* dy, const void* dres, void* dx, float* dgain, float* dshift,
+                                 float* partials, bb_partial_sums* sums, const void* dm, const void* m, void* stream);
 /* m = sqrt(1 - x), elementwise: the stand-in memory of DecoderLayerSimple.forward
  * (DeepSpeedExamples/pipeline_parallelism/gpt2.py:31), and its backward dx (+)= dm * (-1 / (2 m))
  * (accumulate != 0 adds to dx).  n a multiple of 8 (bf16) / 4 (fp32).                       */
