@@ -1329,8 +1329,11 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
                             columns(acc[i][j], std::integral_constant<int, h>{}, v);
                             if (g.bias) unpack_bf16x8(dbias[j][h], b8);
                             const int n = dcol + j * 32 + h * 16, o = j * 32 + h * 16;
+                            // HELD: every lane passes; what it reads on the way (the residual of BB_EPI_MUL_POS) lies inside the matrix
+                            const int mc = HELD ? min(m, g.M - 1) : m, nc = HELD ? min(n, g.N - 8) : n;
+                            const int64_t xr = HELD ? coff + (int64_t)mc * g.ldaux + nc : xi + o;
                             if (HELD || (m < g.M && n < g.N))
-                                epilogue_vec8_at<DROP, true, false, false, kind, HELD>(g, ci + o, xi + o, HELD ? min(m, g.M - 1) : m, HELD ? min(n, g.N - 8) : n, v, b8, dop[t][h],
+                                epilogue_vec8_at<DROP, true, false, false, kind, HELD>(g, ci + o, xr, mc, nc, v, b8, dop[t][h],
                                                                                        u32x4{0u, 0u, 0u, 0u}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, &held[HELD ? j : 0][h]);
                         },
                         std::make_integer_sequence<int, 2 * TN>{});
