@@ -245,6 +245,12 @@ template <bool TA, bool TB, int KW, int BK, int NST> static int launch_bf16_wave
     return BB_OK;
 }
 
+// 64x64 tiles of four waves that are at most half of the CUs' go as two blocks a tile, 32x64 and two waves each (the same bits): a CU has half
+// the LDS reads and transfers to get through in a k-tile.  Whole / halves, device time (us): NN 128x384x128 3.6 / 3.4, 1024x512x512 (128
+// tiles) 4.9 / 4.6, x2048 9.6 / 9.0, 512x768x3072 12.6 / 11.8, 300x1600x1600 8.1 / 7.7; NT 3.7 / 3.6, 4.9 / 4.7, 9.0 / 9.0, 11.9 / 11.6, 7.6 /
+// 7.6; more halves than CUs NN 1050x512x2048 (136 tiles) 9.7 / 11.5, NT 1024x1024x512 (256) 5.1 / 5.9.
+static bool halve_tiles(int M, int N, int64_t batches) { return (int64_t)((M + 31) / 32) * ((N + 63) / 64) * batches <= 256; }
+
 template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     const int layout = TA ? BB_TN : TB ? BB_NN : BB_NT;
     const DmaTile dma = narrow_or_wide(pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.epilogue), layout, g.lda, g.ldb);
@@ -271,7 +277,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D64x128k64s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
         case D64x128s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
         case D64x64k64s4:
-            if constexpr (!TA) return launch_bf16_dma<64, 64, 2, 2, TA, TB, true, 4, 64>(g, batches, st);
+            if constexpr (!TA)
+                return halve_tiles(g.M, g.N, batches) ? launch_bf16_dma<32, 64, 1, 2, TA, TB, true, 4, 64>(g, batches, st)
+                                                      : launch_bf16_dma<64, 64, 2, 2, TA, TB, true, 4, 64>(g, batches, st);
             else break;
         case D256x256p:
             if constexpr (!TA) return launch_bf16_dma_persist<256, 256, 2, 4, TB>(g, st);
@@ -361,7 +369,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
         const DmaTile dt = narrow_or_wide(pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->epilogue), d->layout, d->lda, d->ldb);
         const WaveMode wm = pick_wave(d->M, d->N, d->K, batches, d->layout, dt);
         if (wm != W_NONE) snprintf(out, out_len, "bf16_%s_wave64x64k%d", layouts[d->layout], wm == W_8 ? 8 : 4);
-        else snprintf(out, out_len, "bf16_%s_%s", layouts[d->layout],
+        else snprintf(out, out_len, "bf16_%s_%s%s", layouts[d->layout], dt == D64x64k64s4 && halve_tiles(d->M, d->N, batches) ? "halves_" : "",
                  dt != D_NONE ? kDmaTileNames[dt] : "128x128");
     }
     else if (f32_wide(d->lda, d->ldb)) snprintf(out, out_len, "f32_%s_64x64wide", layouts[d->layout]);
