@@ -50,37 +50,24 @@ __device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[8]) {
 // LayerNorm
 // =========================================================================================
 // Row held in registers: lane owns vectors lane, lane+64, ... (IT of them, VEC elements each).
-template <typename T, int IT>
-__global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, int cols, float eps,
-                                                            const T* __restrict__ x, const T* __restrict__ gain,
-                                                            const T* __restrict__ shift, T* __restrict__ y,
-                                                            float* __restrict__ mean_out, float* __restrict__ rinv_out,
-                                                            T* __restrict__ memory) {
+template <typename T, int IT, bool MEMORY>
+__device__ __forceinline__ void layernorm_fwd_rows(int kind, int rows, int cols, float eps, const T* __restrict__ x, const T* __restrict__ gain,
+                                                   const T* __restrict__ shift, T* __restrict__ y, float* __restrict__ mean_out,
+                                                   float* __restrict__ rinv_out, T* __restrict__ memory) {
     constexpr int VEC = Elem<T>::VEC;
-    constexpr bool EARLY = IT <= 4;
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int nvec = cols / VEC;
     const T* xr = x + (int64_t)row * cols;
     float v[IT][VEC];
-    u32x4 graw[EARLY ? IT : 1], sraw[EARLY ? IT : 1];
     float s = 0.f;
-    if constexpr (EARLY) {
-        // behind the sums each would be another trip to memory
-#pragma unroll
-        for (int i = 0; i < IT; ++i) {
-            const int c = min(lane + i * 64, nvec - 1);
-            graw[i] = *(const u32x4*)(gain + c * VEC);
-            sraw[i] = *(const u32x4*)(shift + c * VEC);
-        }
-    }
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         const int c = lane + i * 64;
         if (c < nvec) {
             load_vec(xr + c * VEC, v[i]);
-            if (memory) {      // as sqrt1m_fwd_kernel, whose launch and pass over x are saved
+            if constexpr (MEMORY) {      // as sqrt1m_fwd_kernel, whose launch and pass over x are saved
                 float mv[VEC];
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) mv[e] = sqrtf(1.0f - v[i][e]);
@@ -122,18 +109,27 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, 
         const int c = lane + i * 64;
         if (c < nvec) {
             float gv[VEC], bv[VEC], o[VEC];
-            if constexpr (EARLY) {
-                unpack16(graw[i], gv);
-                unpack16(sraw[i], bv);
-            } else {
-                load_vec(gain + c * VEC, gv);
-                load_vec(shift + c * VEC, bv);
-            }
+            load_vec(gain + c * VEC, gv);      // (with the row, registers: 4096x1600 6.5 us, 6.9)
+            load_vec(shift + c * VEC, bv);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) o[e] = gv[e] * ((v[i][e] - mean) * rinv) + bv[e];
             store_vec(yr + c * VEC, o);
         }
     }
+}
+// (kernels of their own: with the memory as an argument that may be null 8192x1024 7.1 us, 7.6)
+template <typename T, int IT>
+__global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, int cols, float eps, const T* __restrict__ x,
+                                                            const T* __restrict__ gain, const T* __restrict__ shift, T* __restrict__ y,
+                                                            float* __restrict__ mean_out, float* __restrict__ rinv_out) {
+    layernorm_fwd_rows<T, IT, false>(kind, rows, cols, eps, x, gain, shift, y, mean_out, rinv_out, nullptr);
+}
+template <typename T, int IT>
+__global__ __launch_bounds__(256) void layernorm_fwd_memory_kernel(int kind, int rows, int cols, float eps, const T* __restrict__ x,
+                                                                   const T* __restrict__ gain, const T* __restrict__ shift,
+                                                                   T* __restrict__ y, float* __restrict__ mean_out,
+                                                                   float* __restrict__ rinv_out, T* __restrict__ memory) {
+    layernorm_fwd_rows<T, IT, true>(kind, rows, cols, eps, x, gain, shift, y, mean_out, rinv_out, memory);
 }
 
 // N contiguous floats (N a multiple of 4, 16-byte aligned destination)
@@ -167,13 +163,11 @@ template <int VEC> __device__ __forceinline__ void drop_vec(const DropKey& key, 
 // (two launches / one, bf16, us: 8192x1024 21.0 / 16.7, 4096x1600 20.9 / 18.6, 2048x4096 34.3 / 32.4)
 // MEMORY: dx takes what sqrt1m_bwd_kernel would add to it, as stored (m = sqrt(1 - x), dm its gradient)
 template <typename T, int IT, bool DROP, bool MEMORY>
-__global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_kernel(int kind, int rows, int cols, float eps,
-                                                            const T* __restrict__ x, const T* __restrict__ gain,
-                                                            const float* __restrict__ mean_in,
-                                                            const float* __restrict__ rinv_in, const T* __restrict__ dy,
-                                                            const T* __restrict__ dres, T* __restrict__ dx,
-                                                            float* __restrict__ partial, int one_pass, T* __restrict__ dropped,
-                                                            const DropKey key, const T* __restrict__ dm, const T* __restrict__ m) {
+__device__ __forceinline__ void layernorm_bwd_rows(int kind, int rows, int cols, float eps, const T* __restrict__ x, const T* __restrict__ gain,
+                                                   const float* __restrict__ mean_in, const float* __restrict__ rinv_in,
+                                                   const T* __restrict__ dy, const T* __restrict__ dres, T* __restrict__ dx,
+                                                   float* __restrict__ partial, int one_pass, T* __restrict__ dropped, const DropKey& key,
+                                                   const T* __restrict__ dm, const T* __restrict__ m) {
     constexpr int VEC = Elem<T>::VEC, LN_BWD_WAVES = ln_bwd_waves<T, IT>();
     extern __shared__ float red[];  // [all waves][2][cols] (one pass) or [3 waves][2][cols] for the cross-wave sum
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -344,6 +338,22 @@ __global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_ke
         }
     }
 }
+template <typename T, int IT, bool DROP>
+__global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_kernel(
+    int kind, int rows, int cols, float eps, const T* __restrict__ x, const T* __restrict__ gain, const float* __restrict__ mean_in,
+    const float* __restrict__ rinv_in, const T* __restrict__ dy, const T* __restrict__ dres, T* __restrict__ dx, float* __restrict__ partial,
+    int one_pass, T* __restrict__ dropped, const DropKey key) {
+    layernorm_bwd_rows<T, IT, DROP, false>(kind, rows, cols, eps, x, gain, mean_in, rinv_in, dy, dres, dx, partial, one_pass, dropped, key,
+                                           nullptr, nullptr);
+}
+template <typename T, int IT>
+__global__ __launch_bounds__((ln_bwd_waves<T, IT>() * 64)) void layernorm_bwd_memory_kernel(
+    int kind, int rows, int cols, float eps, const T* __restrict__ x, const T* __restrict__ gain, const float* __restrict__ mean_in,
+    const float* __restrict__ rinv_in, const T* __restrict__ dy, const T* __restrict__ dres, T* __restrict__ dx, float* __restrict__ partial,
+    int one_pass, const T* __restrict__ dm, const T* __restrict__ m) {
+    layernorm_bwd_rows<T, IT, false, true>(kind, rows, cols, eps, x, gain, mean_in, rinv_in, dy, dres, dx, partial, one_pass, nullptr,
+                                           DropKey{}, dm, m);
+}
 
 // out[i] += sum_p partial[p * stride + i].  One block owns 64 columns; its sixteen waves sum
 // interleaved shares of the partial rows (p = w, w+16, ...) and the sixteen results are combined
@@ -412,8 +422,13 @@ extern "C" int bb_partial_sums_acc(const bb_partial_sums* sums, int count, void*
 template <typename T, int IT>
 static int ln_fwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift,
                          void* y, float* mean, float* rinv, void* memory, hipStream_t st) {
-    bb_launch((layernorm_fwd_kernel<T, IT>), dim3((rows + 3) / 4), dim3(256), 0, st, kind, rows, cols, eps,
-                       (const T*)x, (const T*)gain, (const T*)shift, (T*)y, mean, rinv, (T*)memory);
+    const dim3 grid((rows + 3) / 4);
+    if (memory)
+        bb_launch((layernorm_fwd_memory_kernel<T, IT>), grid, dim3(256), 0, st, kind, rows, cols, eps, (const T*)x, (const T*)gain, (const T*)shift,
+                  (T*)y, mean, rinv, (T*)memory);
+    else
+        bb_launch((layernorm_fwd_kernel<T, IT>), grid, dim3(256), 0, st, kind, rows, cols, eps, (const T*)x, (const T*)gain, (const T*)shift,
+                  (T*)y, mean, rinv);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -429,10 +444,18 @@ static int ln_bwd_launch(int kind, int rows, int cols, float eps, const void* x,
     const size_t all = (size_t)LN_BWD_WAVES * 2 * cols * sizeof(float);
     const int one_pass = all <= 128 * 1024;
     const size_t smem = one_pass ? all : (size_t)3 * 2 * cols * sizeof(float);
-    auto kern = dm ? layernorm_bwd_kernel<T, IT, false, true> : key.thresh ? layernorm_bwd_kernel<T, IT, true, false> : layernorm_bwd_kernel<T, IT, false, false>;
+    if (dm) {
+        auto kern = layernorm_bwd_memory_kernel<T, IT>;
+        BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
+        bb_launch(kern, dim3(blocks), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x, (const T*)gain, mean, rinv,
+                  (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass, (const T*)dm, (const T*)m);
+        BB_LAUNCH_CHECK();
+        return BB_OK;
+    }
+    auto kern = key.thresh ? layernorm_bwd_kernel<T, IT, true> : layernorm_bwd_kernel<T, IT, false>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));   // raised on the first (never captured) call that needs it
     bb_launch(kern, dim3(blocks), dim3(LN_BWD_WAVES * 64), smem, st, kind, rows, cols, eps, (const T*)x,
-                       (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass, (T*)dropped, key, (const T*)dm, (const T*)m);
+                       (const T*)gain, mean, rinv, (const T*)dy, (const T*)dres, (T*)dx, ws, one_pass, (T*)dropped, key);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -557,7 +580,7 @@ static std::mutex g_ln_static_mu;
 
 template <typename T, int IT> static hipError_t ln_bwd_allow_one_pass() {
     // the largest dynamic LDS request the kernel makes for cols <= BB_LN_BWD_STATIC_MAX_COLS: the one-pass layout
-    return bb_allow_dynamic_lds((const void*)layernorm_bwd_kernel<T, IT, false, false>, 128 * 1024);
+    return bb_allow_dynamic_lds((const void*)layernorm_bwd_kernel<T, IT, false>, 128 * 1024);
 }
 // once per device, with that device current: the address of the device's copy, and every LDS-limit change the
 // entry point could otherwise need on its first call
