@@ -844,7 +844,8 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
 // =========================================================================================
 // backward dQ: block = 128 queries (4 waves x 32), loop over 64-key tiles
 // =========================================================================================
-template <int DROP, int HP, int NPAN, int W, int G>
+// OWN: the dK / dV blocks of the launch make their deltas themselves, nobody reads this block's
+template <int DROP, int HP, int NPAN, int W, int G, bool OWN>
 __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int block, unsigned char* smem_all) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
@@ -898,8 +899,8 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
         }
     }
     // delta[q] = rowsum(dO o O) over the head's columns: the lane and its partner (lane ^ 32) hold the two halves of
-    // each 16-column step of the query's dO row; the matching halves of O are fetched once.  Written out for the
-    // dK / dV kernel, which runs after this one.
+    // each 16-column step of the query's dO row; the matching halves of O are fetched once.  Written out for a
+    // dK / dV kernel that runs after this one.
     float my_lse, my_delta = 0.f;
     {
         const bf16* O = a.o + row_base * a.ld_o + hg * (64 * NPAN) + hh * 32;
@@ -912,7 +913,7 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
             for (int e = 0; e < 8; ++e) my_delta = fmaf((float)dof[k][e], (float)of[e], my_delta);
         }
         my_delta += other_half(my_delta);
-        if (lane < 32 && myq < a.seq && grp == 0) a.delta[stat] = my_delta;
+        if (!OWN && lane < 32 && myq < a.seq && grp == 0) a.delta[stat] = my_delta;
     }
     f32x16 dq[DT];
 #pragma unroll
@@ -1033,7 +1034,7 @@ __global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_dkv_kernel(const 
 template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
 __global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_dq_kernel(const AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
-    attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x, smem_all);
+    attn_bwd_dq_block<DROP, HP, NPAN, W, G, false>(a, blockIdx.x, smem_all);
 }
 // Both in one launch, where there is room for all their blocks (attn_bwd_launch): first the dK / dV blocks, whose walks are the
 // longer ones, then the dQ blocks.
@@ -1041,7 +1042,7 @@ template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
 __global__ __launch_bounds__(W * HP * G * 64, 2) void attn_bwd_kernel(const AttnArgs a, const int dkv_blocks, const int own_at) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
     if ((int)blockIdx.x < dkv_blocks) attn_bwd_dkv_block<DROP, HP, NPAN, W, G, true>(a, blockIdx.x, smem_all, own_at);
-    else attn_bwd_dq_block<DROP, HP, NPAN, W, G>(a, blockIdx.x - dkv_blocks, smem_all);
+    else attn_bwd_dq_block<DROP, HP, NPAN, W, G, true>(a, blockIdx.x - dkv_blocks, smem_all);
 }
 
 // =========================================================================================

@@ -1,6 +1,7 @@
 """Attention backward in one launch or two: block counts on either side of a round, sequences around the longest whose row sums a
 block keeps, padding that leaves blocks without a key, each head width; against fp64, twice the same bits, without and with dropout."""
 import pytest
+import torch
 
 from tests import test_gpu_dropout as drop
 from tests import test_gpu_kernels as plain
@@ -20,3 +21,20 @@ def test_backward(hiplib, mask, b, a, s, d):
 @pytest.mark.parametrize("mask,b,a,s,d", [t for t in SHAPES if t[3] < 2000])
 def test_backward_with_dropout(hiplib, mask, b, a, s, d):
     drop.test_fused_attention_dropout_fwd_bwd(hiplib, mask, b, a, s, d)
+
+
+@pytest.mark.parametrize("b,a,s,d,together", [(1, 2, 64, 64, True), (2, 4, 130, 32, True), (1, 2, 300, 128, True), (1, 1, 2048, 64, True),
+                                              (1, 2, 2049, 64, False), (2, 256, 65, 64, False)])
+def test_row_sums(hiplib, b, a, s, d, together):
+    """The caller's row sums: left as they were where one launch does both passes, written where the second launch reads them."""
+    g = torch.Generator(device="cuda").manual_seed(s)
+    qkv, d_out = (torch.randn(b * s, w, generator=g, device="cuda").bfloat16() for w in (3 * a * d, a * d))
+    out, lse, delta = torch.empty_like(d_out), torch.empty(b, a, s, device="cuda"), torch.full((b, a, s), -3.0, device="cuda")
+    args = (b, a, s, hiplib.MASK_CODES["causal"])
+    hiplib.attention_fwd(qkv, out, lse, *args)
+    hiplib.attention_bwd(qkv, out, d_out, lse, delta, torch.empty_like(qkv), *args)
+    terms = (out.double() * d_out.double()).view(b, s, a, d).transpose(1, 2)
+    if together:
+        assert (delta == -3.0).all()
+    else:       # d products added in fp32, one rounding each
+        assert ((delta.double() - terms.sum(-1)).abs() <= d * 2.0 ** -24 * terms.abs().sum(-1)).all()
