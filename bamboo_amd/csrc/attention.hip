@@ -1101,17 +1101,29 @@ struct attn_dkv_launch {
 // 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two heads of 128, 512, dropout 69.0 /
 // 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
 // 192) 68 / 73, 4 x 16, 256 causal (256 + 256 of eight) 18.0 / 18.5.  The bits are the same.
+// LDS has room for what the waves allow (of blocks of two waves three instead of four a CU, 768; they are at most 512), but for one shape: blocks of
+// four waves whose two rings fill more than half of it (64-wide heads, two waves in two groups) are one a CU.  A round and
+// a quarter, empty blocks of uneven XCDs among it (they go to no other XCD), is still the faster way with padding: the blocks left over
+// follow those of dQ, whose walks are the shorter ones.  Under a causal mask, which has short blocks to follow the long ones, up to two rounds
+// and a quarter.  One after the other / together: padding, keys in full and at 0.8, 288 blocks (1 x 8, 1100) 31.0 / 26.5 and 29.2 / 25.9, 320
+// (2 x 8, 640) 21.4 / 18.5 and 20.5 / 17.2, 336 (1 x 8, 1344) 35.5 / 43.5 and 33.5 / 29.9, 448 (4 x 7, 448) 19.5 / 21.8 and 18.6 / 20.9, 512 (1 x
+// 8, 2048) 48.2 / 60.9 and 45.1 / 57.6; causal 512 (2 x 8, 1024) 29.3 / 26.4, with dropout 35.5 / 29.3, 528 (3 x 6, 700) 24.5 / 22.8, 608 (1 x 9,
+// 1153) 32.6 / 33.2, 768 (1 x 10, 1500) 39.9 / 47.3.
 static constexpr int kOwnDeltaSeq = 2048;    // longest sequence whose deltas a block keeps in LDS
 struct attn_bwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        const int64_t rows = (seq + W * 32 - 1) / (W * 32), slots = 256 * 8 / (W * HP * G);
-        if (seq > kOwnDeltaSeq || nbh * rows * (NPAN + 1) > slots) {
+        constexpr size_t dq_lds = attn_lds<HP, NPAN, W, G>(true, false), dkv_lds = attn_lds<HP, NPAN, W, G>(true, true);
+        constexpr size_t own_at = dkv_lds > dq_lds ? dkv_lds : dq_lds;
+        constexpr int waves = W * HP * G;
+        constexpr bool one_a_cu = waves == 4 && own_at > 80 * 1024;
+        const unsigned dkv = attn_grid(seq, W * 32, nbh * NPAN), dq = attn_grid(seq, W * 32, nbh);
+        const int64_t rows = (seq + W * 32 - 1) / (W * 32);
+        const bool room = one_a_cu ? dkv + dq <= (a.mask == BB_MASK_CAUSAL ? 576u : 320u) : nbh * rows * (NPAN + 1) <= 256 * 8 / waves;
+        if (seq > kOwnDeltaSeq || !room) {
             // the dQ kernel first: it also leaves delta = rowsum(dO o O) of its queries for the dK / dV kernel
             const int rc = attn_dq_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
             return rc ? rc : attn_dkv_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
         }
-        const unsigned dkv = attn_grid(seq, W * 32, nbh * NPAN), dq = attn_grid(seq, W * 32, nbh);
-        constexpr size_t own_at = attn_lds<HP, NPAN, W, G>(true, true) > attn_lds<HP, NPAN, W, G>(true, false) ? attn_lds<HP, NPAN, W, G>(true, true) : attn_lds<HP, NPAN, W, G>(true, false);
         const size_t lds = own_at + (size_t)HP * ((seq + 63) / 64 * 64) * sizeof(float);
         auto kern = a.keep ? attn_bwd_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_kernel<MADE, HP, NPAN, W, G> : attn_bwd_kernel<NODROP, HP, NPAN, W, G>;
         BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));

@@ -23,14 +23,18 @@ def test_backward_with_dropout(hiplib, mask, b, a, s, d):
     drop.test_fused_attention_dropout_fwd_bwd(hiplib, mask, b, a, s, d)
 
 
-@pytest.mark.parametrize("b,a,s,d,together", [(1, 2, 64, 64, True), (2, 4, 130, 32, True), (1, 2, 300, 128, True), (1, 1, 2048, 64, True),
-                                              (1, 2, 2049, 64, False), (2, 256, 65, 64, False)])
-def test_row_sums(hiplib, b, a, s, d, together):
+@pytest.mark.parametrize("mask,b,a,s,d,together", [
+    ("causal", 1, 2, 64, 64, True), ("causal", 2, 4, 130, 32, True), ("causal", 1, 2, 300, 128, True), ("causal", 1, 1, 2048, 64, True),
+    ("causal", 1, 2, 2049, 64, False), ("causal", 2, 256, 65, 64, False),
+    # blocks that are one a CU: a round and a quarter with padding, two and a quarter under a causal mask
+    ("key_padding", 2, 8, 640, 64, True), ("key_padding", 2, 8, 641, 64, False), ("causal", 2, 8, 1024, 64, True), ("causal", 1, 9, 1153, 64, False)])
+def test_row_sums(hiplib, mask, b, a, s, d, together):
     """The caller's row sums: left as they were where one launch does both passes, written where the second launch reads them."""
     g = torch.Generator(device="cuda").manual_seed(s)
     qkv, d_out = (torch.randn(b * s, w, generator=g, device="cuda").bfloat16() for w in (3 * a * d, a * d))
     out, lse, delta = torch.empty_like(d_out), torch.empty(b, a, s, device="cuda"), torch.full((b, a, s), -3.0, device="cuda")
-    args = (b, a, s, hiplib.MASK_CODES["causal"])
+    lens = torch.full((b,), s, dtype=torch.int32, device="cuda") if mask == "key_padding" else None
+    args = (b, a, s, hiplib.MASK_CODES[mask], lens)
     hiplib.attention_fwd(qkv, out, lse, *args)
     hiplib.attention_bwd(qkv, out, d_out, lse, delta, torch.empty_like(qkv), *args)
     terms = (out.double() * d_out.double()).view(b, s, a, d).transpose(1, 2)
