@@ -1,6 +1,6 @@
 // Fused masked softmax-attention for gfx950, bf16, head dimension 64, 32 or 128: forward and the two
-// backward kernels (dK/dV and dQ).  No [batch, heads, seq, seq] tensor ever reaches HBM; the
-// forward keeps one fp32 log-sum-exp per (batch, head, query) for the backward.
+// backward kernels (dK/dV and dQ).  No scores or probabilities reach HBM; the forward keeps one fp32
+// log-sum-exp per (batch, head, query) for the backward, and, if given room for it, a bit per dropout decision.
 //
 // Stands in for MultiHeadedAttention.attention of the reference
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:117-127: softmax(QK^T/sqrt(d) with

@@ -114,10 +114,15 @@ class TransformerLayer:
     or ``key_padding``.
 
     dropout: probability of the reference's four ``nn.Dropout`` sites (attention probabilities, the two sublayer
-    outputs, the feed-forward's hidden activation; transformer.py:98-103,125-126,154-158).  No mask is stored: each
-    decision is a pure function of (base seed, batch counter, micro-batch, layer, site, element), evaluated inside
+    outputs, the feed-forward's hidden activation; transformer.py:98-103,125-126,154-158).  Each decision is a pure
+    function of (base seed, batch counter, micro-batch, layer, site, element), evaluated inside
     the attention kernels and the GEMM epilogues, so the redundant forward of a layer, its normal forward and its
     backward pass agree bit for bit.
+
+    keep_dropout: the fused attention's forward leaves its decisions to the backward as bits, ``batch * heads * seq^2 / 8`` bytes,
+    where ``seq <= 32 * head_dim``, i.e. where these are at most what two [rows, hidden] tensors of the stash take (which so stays
+    linear in the length).  Beyond, and with ``False``, the backward makes the decisions again: the same bits, and the memory of a
+    layer without dropout.
     """
 
     launches_only = True      # see replay.launches_only
@@ -133,12 +138,12 @@ class TransformerLayer:
         "sublayer.0.norm.a_2", "sublayer.0.norm.b_2", "sublayer.1.norm.a_2", "sublayer.1.norm.b_2")
 
     def __init__(self, hidden, heads, ffn, activation="relu", ln="annotated", mask="none", ln_eps=None,
-                 init_std=0.02, dropout=0.0):
+                 init_std=0.02, dropout=0.0, keep_dropout=True):
         if hidden % heads:
             raise ValueError("hidden must be divisible by heads")
         if not 0.0 <= dropout < 1.0:
             raise ValueError("dropout must be in [0, 1)")
-        self.dropout = float(dropout)
+        self.dropout, self.keep_dropout = float(dropout), keep_dropout
         self.layer_idx = None     # global index, set when the layer is bound to a stage's arenas
         self.hidden, self.heads, self.ffn = hidden, heads, ffn
         self.head_dim = hidden // heads
@@ -228,8 +233,13 @@ class TransformerLayer:
         """What the attention keeps for its backward."""
         if not self.fused_attention(ctx):
             return [(f"prob{tag}", (ctx.batch, self.heads, ctx.seq, ctx.seq), ctx.dtype)]
-        keep = [(f"keep{tag}", (hip.attention_keep_words(ctx.batch, self.heads, ctx.seq),), torch.int32)] if self.dropout > 0 else []
-        return [(f"lse{tag}", (ctx.batch, self.heads, ctx.seq), torch.float32), *keep]
+        specs = [(f"lse{tag}", (ctx.batch, self.heads, ctx.seq), torch.float32)]
+        # The bits buy time by the byte at any length (made again / kept, forward and backward, us: 8 x 16 heads of 64, 1024 keys 88 + 202 /
+        # 80 + 174 for 16 MB; 2 x 16, 2048 causal 56 + 135 / 58 + 119 for 16; 1 x 16, 4096 causal 105 + 252 / 108 + 229 for 32; 2 x 16 of
+        # 32, 2048 causal 77 + 178 / 80 + 133 for 16), but they grow by the square of it and everything else here by the length
+        if self.dropout > 0 and self.keep_dropout and ctx.seq <= 32 * self.head_dim:
+            specs.append((f"keep{tag}", (hip.attention_keep_words(ctx.batch, self.heads, ctx.seq),), torch.int32))
+        return specs
 
     def stash_specs(self, ctx):
         R, h, f = ctx.rows, self.hidden, self.ffn
