@@ -43,6 +43,8 @@ class StageContext:
         # by a backward pass only after a failover); ``deferred`` tells that backward pass to produce it first
         self.defer = False
         self.deferred = False
+        # set while a checkpointed group runs for the first time: its backward pass runs it again and reads what that run leaves
+        self.remade = False
         # optional observer of this lane's GEMM launches (``hip.gemm(..., hook=)``); set through the engine that owns
         # the context, so a probe on one engine sees and changes nothing of another
         self.gemm_hook = None
@@ -314,7 +316,8 @@ class TransformerLayer:
         drop = self._drop(ctx, site)
         if self.fused_attention(ctx):
             hip.attention_fwd(st["qkv"], st["ctx"], st["lse"], ctx.batch, self.heads, s, hip.MASK_CODES[mask],
-                              ctx.key_len if mask == "key_padding" else None, stream=ctx.stream, dropout=drop, keep=st.get("keep"))
+                              ctx.key_len if mask == "key_padding" else None, stream=ctx.stream, dropout=drop,
+                              keep=None if ctx.defer or ctx.remade else st.get("keep"))
             return
         if self.kept_probs_kernels(ctx):
             hip.attention_probs_fwd(st["qkv"], st["ctx"], st["prob"], ctx.batch, self.heads, s, hip.MASK_CODES[mask],
@@ -346,7 +349,7 @@ class TransformerLayer:
             delta = ctx.buf("attn_delta", (ctx.batch, self.heads, s))
             hip.attention_bwd(st["qkv"], st["ctx"], d_ctx, st["lse"], delta, d_qkv, ctx.batch, self.heads, s,
                               hip.MASK_CODES[mask], ctx.key_len if mask == "key_padding" else None, stream=ctx.stream,
-                              dropout=drop, keep=st.get("keep"))
+                              dropout=drop, keep=None if ctx.deferred else st.get("keep"))
             return
         if self.kept_probs_kernels(ctx):
             hip.attention_probs_bwd(st["qkv"], d_ctx, st["prob"], ctx.buf("d_prob", tuple(st["prob"].shape)), d_qkv, ctx.batch,

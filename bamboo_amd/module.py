@@ -547,15 +547,19 @@ class PipelineModule:
             ctx.defer = False
             return x
         kept = self._kept[stage_id][slot]
-        for g, (a, b) in enumerate(self._checkpoint_groups(stage_id)):
-            if x is not kept[g]:
-                hip.cast(x, kept[g], stream=ctx.stream)   # same-type copy: the group's input outlives the work stash
-            x = kept[g]
-            for i in range(a, b - 1):
-                ctx.seq = seqs[i]
-                x = layers[i].forward(x, stash[i], ctx)
-            ctx.seq = seqs[b - 1]
-            x = self._forward_into(kept[g + 1], layers[b - 1], x, stash[b - 1], ctx)
+        ctx.remade = True
+        try:
+            for g, (a, b) in enumerate(self._checkpoint_groups(stage_id)):
+                if x is not kept[g]:
+                    hip.cast(x, kept[g], stream=ctx.stream)   # same-type copy: the group's input outlives the work stash
+                x = kept[g]
+                for i in range(a, b - 1):
+                    ctx.seq = seqs[i]
+                    x = layers[i].forward(x, stash[i], ctx)
+                ctx.seq = seqs[b - 1]
+                x = self._forward_into(kept[g + 1], layers[b - 1], x, stash[b - 1], ctx)
+        finally:
+            ctx.remade = False
         if x is not kept[-1]:
             hip.cast(x, kept[-1], stream=ctx.stream)
         return kept[-1]

@@ -1,5 +1,5 @@
 """A stage whose attention keeps its dropout decisions against one that makes them again: the same bits in every result, on the full and
-on a checkpointed stash, beside redundant forwards."""
+on a checkpointed stash, beside redundant forwards and after a failover onto their stash."""
 import pytest
 import torch
 
@@ -33,3 +33,26 @@ def test_same_results(hiplib, kind, ckpt):
     model, made = batches(kind, False, ckpt)
     assert "keep" not in model._stash[1][0][0]
     assert len(kept) > 1 and all(torch.equal(a, b) for a, b in zip(kept, made)) and all(torch.isfinite(a).all() for a in kept)
+
+
+@pytest.mark.parametrize("kind", [TransformerLayer, DecoderLayer])
+def test_backward_of_a_deferred_forward(hiplib, kind):
+    """The forward of a redundant pass and the backward that follows a failover on its stash, against the normal pair."""
+    model, _ = batches(kind, True, 0)
+    sid, ctx = 1, model.prepare_context([1], 2, 96)
+    g = torch.Generator(device="cuda:0").manual_seed(1)
+    x, d = (torch.randn(192, 128, generator=g, device="cuda:0") * 0.3 - 2.0).bfloat16(), torch.randn(192, 128, generator=g, device="cuda:0").bfloat16()
+    results = []
+    for defer in (False, True):
+        ctx.dropout_base = (99, 7, 1)
+        for st in model._stash[sid][0]:
+            for name in ("keep", "keep_src"):
+                if name in st:
+                    st[name].fill_(0x55555555 if defer else 0)           # neither written nor read
+        model.stage_params[sid].grad.zero_()
+        out = model.forward(x, sid, slot=0, ctx=ctx, defer=defer).clone()
+        if defer:
+            assert all((st[name] == 0x55555555).all() for st in model._stash[sid][0] for name in ("keep", "keep_src") if name in st)
+        dx = model.backward(d, torch.empty_like(x), sid, slot=0, ctx=ctx, deferred=defer)
+        results.append((out, dx, model.stage_params[sid].grad.clone()))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
