@@ -8,8 +8,17 @@ from tests import test_gpu_kernels as plain
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 2, 160, 64), (2, 3, 193, 64), (1, 5, 321, 64), (1, 4, 80, 32), (2, 6, 257, 32),                # two waves in four groups
-          (1, 36, 448, 64), (1, 43, 577, 64), (2, 60, 289, 32), (1, 2, 448, 128), (2, 4, 521, 128)]          # four waves in two
+# waves x groups of a block, forward and backward (4x1: the walk is not shared)
+SHAPES = [(1, 2, 160, 64), (2, 3, 193, 64),                             # 2x4, 2x1
+          (1, 5, 321, 64),                                              # 2x4, 2x4 in one launch
+          (1, 2, 2100, 64),                                             # 2x4, 2x4 in two
+          (2, 8, 520, 64), (1, 22, 450, 64),                            # 2x4, 2x2 in one; with padding the second in two
+          (1, 36, 448, 64), (1, 43, 577, 64),                           # 2x2, 4x1
+          (1, 11, 1537, 64),                                            # 2x2, 4x2
+          (1, 33, 1025, 64),                                            # 2x2 if causal, else 4x1, both backward 4x1
+          (1, 4, 80, 32), (2, 60, 289, 32),                             # pairs of heads: 4x1
+          (2, 6, 257, 32),                                              # 2x2
+          (1, 2, 448, 128), (2, 4, 521, 128)]                           # 4x2
 
 
 @pytest.mark.parametrize("mask", ["causal", "key_padding"])
