@@ -1,5 +1,7 @@
 """Products whose epilogue works on the accumulators in registers, and whose operands are reached by 32-bit offsets from a base
 per tile: rows and columns off the tile, every epilogue kind, results in fp32, leading dimensions on either side of the limit."""
+import itertools
+
 import pytest
 import torch
 
@@ -12,8 +14,8 @@ def rand(*shape, seed, scale=1.0):
     return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
 
 
-def framed(M, N, dtype=torch.bfloat16):
-    wide = torch.full((M + 1, N + 8), 7.0, dtype=dtype, device=DEV)
+def framed(M, N, dtype=torch.bfloat16, guard=True):
+    wide = torch.full((M + guard, N + 8 * guard), 7.0, dtype=dtype, device=DEV)
     return wide, wide[:M, :N]
 
 
@@ -22,11 +24,15 @@ def framed(M, N, dtype=torch.bfloat16):
                                         ("128x128k64s3", 3301, 1032, 512), ("256x128k64s3", 8100, 1000, 512), ("256x128k64s3", 8192, 1024, 512)])
 @pytest.mark.parametrize("layout", ["nt", "nn"])
 def test_register_epilogue(hiplib, layout, tile, M, N, K):
+    for guard in (True, False):     # outputs inside wider buffers, whose rest stays as it is, or contiguous ones
+        every_kind(hiplib, layout, tile, M, N, K, guard)
+
+
+def every_kind(hiplib, layout, tile, M, N, K, guard):
     lay = hiplib.NT if layout == "nt" else hiplib.NN
     A, B = rand(M, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2, scale=0.2)
     bias, X, R = rand(N, seed=3), rand(M, N, seed=4), rand(M, N, seed=5)
-    wide, C = framed(M, N)
-    wide2, D = framed(M, N)
+    (wide, C), (wide2, D) = (framed(M, N, guard=guard) for _ in range(2))
     assert hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C)).endswith(tile)
     a, b = A.double(), (B.double().t() if layout == "nt" else B.double()).contiguous()
     prod, slack = a @ b, K * 2.0 ** -24 * (a.abs() @ b.abs())
@@ -42,44 +48,76 @@ def test_register_epilogue(hiplib, layout, tile, M, N, K):
     near(C, prod)
     hiplib.gemm(lay, A, B, C, bias=bias, alpha=0.5)
     near(C, 0.5 * prod + bias.double())
-    C1, D1 = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
-    hiplib.gemm(lay, A, B, C1, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=R)
-    near(C1, u + r)
-    hiplib.gemm(lay, A, B, C1, epilogue=hiplib.EPI_MUL, aux_in=X)
-    near(C1, prod * x, scale=x.abs())
-    hiplib.gemm(lay, A, B, C1, epilogue=hiplib.EPI_MUL_POS, aux_in=X, resid=R)
-    near(C1, torch.where(x > 0, prod + r, 0.0))
-    hiplib.gemm(lay, A, B, C1, epilogue=hiplib.EPI_DACT, act=hiplib.ACT_RELU, aux_in=X)
-    near(C1, torch.where(x > 0, prod, 0.0))
-    hiplib.gemm(lay, A, B, C1, bias=bias, epilogue=hiplib.EPI_ACT, act=hiplib.ACT_RELU, aux_out=D1)
-    near(D1, u)
-    near(C1, u.clamp_min(0))
-    hiplib.gemm(lay, A, B, C1, bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_GELU_TANH, aux_out=D1)
+    hiplib.gemm(lay, A, B, C, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=R)
+    near(C, u + r)
+    hiplib.gemm(lay, A, B, C, epilogue=hiplib.EPI_MUL, aux_in=X)
+    near(C, prod * x, scale=x.abs())
+    hiplib.gemm(lay, A, B, C, epilogue=hiplib.EPI_MUL_POS, aux_in=X, resid=R)
+    near(C, torch.where(x > 0, prod + r, 0.0))
+    hiplib.gemm(lay, A, B, C, epilogue=hiplib.EPI_DACT, act=hiplib.ACT_RELU, aux_in=X)
+    near(C, torch.where(x > 0, prod, 0.0))
+    hiplib.gemm(lay, A, B, C, bias=bias, epilogue=hiplib.EPI_ACT, act=hiplib.ACT_RELU, aux_out=D)
+    near(D, u)
+    near(C, u.clamp_min(0))
+    hiplib.gemm(lay, A, B, C, bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_GELU_TANH, aux_out=D)
     g = u.clone().requires_grad_()
     y = torch.nn.functional.gelu(g, approximate="tanh")
     dy, = torch.autograd.grad(y.sum(), g)
-    near(C1, y.detach(), scale=2.0)      # |gelu'| and |gelu''| stay below 1.2
-    near(D1, dy.double(), scale=2.0)
+    near(C, y.detach(), scale=2.0)      # |gelu'| and |gelu''| stay below 1.2
+    near(D, dy.double(), scale=2.0)
     F0 = torch.randn(M, N, generator=torch.Generator(device=DEV).manual_seed(6), device=DEV)
-    F = F0.clone()
+    wide3, F = framed(M, N, torch.float32, guard)
+    F.copy_(F0)
     hiplib.gemm(lay, A, B, F, accumulate=True)
     assert ((F.double() - prod - F0.double()).abs() <= slack + 2.0 ** -23 * (prod.abs() + F0.double().abs() + 1.0)).all()
+    assert (wide3[M:] == 7).all() and (wide3[:, N:] == 7).all()
+
+
+def apart(t, step):
+    """The same matrix, its rows ``step`` elements apart."""
+    far = torch.empty(t.shape[0] * step, dtype=t.dtype, device=DEV).view(t.shape[0], step)[:, : t.shape[1]]
+    return far.copy_(t)
 
 
 @pytest.mark.parametrize("layout", ["nt", "nn"])
 def test_rows_far_apart(hiplib, layout):
     M, N, K, ld = 130, 136, 128, 1 << 22
     lay = hiplib.NT if layout == "nt" else hiplib.NN
-    store = torch.empty(M * ld, dtype=torch.bfloat16, device=DEV)
-    for step in (ld, ld - 8):
-        A = store[: M * step].view(M, step)[:, :K]
-        A.copy_(rand(M, K, seed=1))
-        B = rand(*((N, K) if layout == "nt" else (K, N)), seed=2)
+    a, b = rand(M, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2)
+    for far, step in itertools.product("AB", (ld, ld - 8)):
+        A, B = (apart(a, step), b) if far == "A" else (a, apart(b, step))
         C, D = (torch.empty(M, N, dtype=torch.bfloat16, device=DEV) for _ in range(2))
         variant = hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C))
         assert variant.endswith("128x128k64r") == (step == ld)
         hiplib.gemm(lay, A, B, C)
-        hiplib.gemm(lay, A.contiguous(), B, D)
+        hiplib.gemm(lay, a, b, D)
         assert torch.equal(C, D)         # the kernels add up a contraction in one order
         hiplib.gemm_grouped([hiplib.gemm_desc(lay, A, B, C), hiplib.gemm_desc(lay, A, B, D)])
         assert torch.equal(C, D)
+
+
+@pytest.mark.parametrize("far", ["A", "B"])
+@pytest.mark.parametrize("step", [1 << 22, (1 << 22) - 8])
+def test_column_statistics_of_rows_far_apart(hiplib, far, step):
+    """The kernels that leave column sums, forward (of a convolution's output) and backward (of a normalisation's gradient): as from contiguous
+    operands, whose tiles they may not share; a strip's rows are added in one order by all of them."""
+    M, N, K = 170, 136, 128
+    a, b, w = rand(M, K, seed=1) + 1.0, rand(N, K, seed=2), rand(K, N, seed=3)
+    for t in (b, w):
+        A, B = (apart(a, step), t) if far == "A" else (a, apart(t, step))
+        results = []
+        if t is b:
+            for ops in ((a, b), (A, B)):
+                C = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+                strips = torch.full((hiplib.strip_stats_workspace(M, N),), float("nan"), device=DEV)
+                hiplib.gemm(hiplib.NT, *ops, C, strip_stats=strips)
+                results.append((C, strips))
+        else:
+            x, relu_out, skip = rand(M, N, seed=4), rand(M, N, seed=5), rand(M, N, seed=6)
+            mean, rstd = torch.randn(2, N, generator=torch.Generator(device=DEV).manual_seed(7), device=DEV)
+            for ops in ((a, w), (A, B)):
+                C = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+                strips = torch.full((hiplib.bn_bwd_strips_workspace(M, N),), float("nan"), device=DEV)
+                hiplib.gemm_bn_bwd(*ops, C, relu_out, x, mean, rstd, strips, resid=skip)
+                results.append((C, strips))
+        assert all(torch.equal(p, q) for p, q in zip(*results)) and not any(torch.isnan(p).any() for p in results[0])
