@@ -269,7 +269,8 @@ enum { NODROP = 0, MADE = 1, KEPT = 2, PAIRS = 3 };
 // what the forward kept, in the backward
 // KS k-steps of a head's scores, DT 32-wide output tiles of a head
 template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * HP * G * 64, NPAN == 1 && G == 1 ? (DROP == NODROP ? 4 : DROP == PAIRS ? 3 : 2) : 2) void attn_fwd_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(W * HP * G * 64, NPAN == 1 && G == 1 ? (DROP == NODROP ? 4 : DROP == PAIRS ? 3 : 2) : 2)
+void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];  // G rings of 2 stages of K, then 2 of V
@@ -488,8 +489,10 @@ __global__ __launch_bounds__(W * HP * G * 64, NPAN == 1 && G == 1 ? (DROP == NOD
 constexpr bool attn_bwd_pipe(int npan) { return npan == 1; }
 // stages of a ring: three where a tile's last products come behind the barrier that hands the next tile out, two where three do not fit
 constexpr int attn_bwd_stages(int npan, int g) { return npan == 1 && g <= 2 ? 3 : 2; }
-template <int G, int STAGES, int STAGE, bool PIPE, typename Live, typename FetchS, typename FetchG, typename Scores, typename Grads, typename Probs, typename Contract, typename Issue>
-__device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int iters, const Live& live, const FetchS& fetch_scores, const FetchG& fetch_grads, const Scores& scores, const Grads& score_grads,
+template <int G, int STAGES, int STAGE, bool PIPE, typename Live, typename FetchS, typename FetchG, typename Scores, typename Grads,
+          typename Probs, typename Contract, typename Issue>
+__device__ __forceinline__ void attn_bwd_walk(unsigned char* smem, int t, int iters, const Live& live, const FetchS& fetch_scores,
+                                              const FetchG& fetch_grads, const Scores& scores, const Grads& score_grads,
                                               const Probs& probs, const Contract& contract, const Issue& issue) {
     using First = std::integral_constant<int, 0>;
     int stage = 0;
@@ -736,9 +739,11 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
                     uint32_t km = 0u, kt = 0u;   // bit r: this lane's decision of its row, the neighbour's row
 #pragma unroll
                     for (int r = 0; r < 16; r += 2) {
-                        const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, (j0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq) >> 1);
+                        const uint32_t at = j0 + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)a.seq;
+                        const uint32_t x = bb_dropout_pair_bits32(a.drop.k0, a.drop.k1, at >> 1);
                         const bool mine = ((x >> own) & 0xffffu) >= a.drop.thresh;
-                        const uint32_t sent = (uint32_t)__builtin_amdgcn_mov_dpp((int)((x >> other) & 0xffffu), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true);
+                        const uint32_t sent =
+                            (uint32_t)__builtin_amdgcn_mov_dpp((int)((x >> other) & 0xffffu), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true);
                         const bool theirs = sent >= a.drop.thresh;
                         km |= mine ? 1u << r : 0u;
                         kt |= theirs ? 1u << r : 0u;
@@ -792,7 +797,8 @@ __device__ __forceinline__ void attn_bwd_dkv_block(const AttnArgs& a, const int 
         asm volatile("" ::: "memory");
         wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
-        attn_bwd_walk<G, STAGES, STAGE, PIPE>(smem, t0, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        attn_bwd_walk<G, STAGES, STAGE, PIPE>(smem, t0, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract,
+                                              [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
         if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
@@ -983,7 +989,8 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
                 const int dt = hh + d;
-                dq[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(st + (dt >> 1) * 8192, u * 32 + kk * 16, (dt & 1) * 32, lane), dsf, dq[d], 0, 0, 0);
+                const bf16x8 kt = frag_tr(st + (dt >> 1) * 8192, u * 32 + kk * 16, (dt & 1) * 32, lane);
+                dq[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, dsf, dq[d], 0, 0, 0);
             }
         }
     };
@@ -992,7 +999,8 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, const int b
         asm volatile("" ::: "memory");
         wait_vm<0>();      // in full: a wait the compiler left for its own loads would stand in the loop, in front of every transfer
         block_sync();
-        attn_bwd_walk<G, STAGES, STAGE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract, [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
+        attn_bwd_walk<G, STAGES, STAGE, PIPE>(smem, grp, iters, live, fetch_scores, fetch_grads, scores, score_grads, probs, contract,
+                                              [&](int t, int slot) { if (t < ntiles) issue(t, slot); });
         if constexpr (G > 1) block_sync();     // the rings are done with
     }
     if constexpr (G > 1) {
@@ -1077,20 +1085,27 @@ template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int
 // dropout is a kernel of its own: its keep decisions cost registers that decide how many blocks a CU holds
 struct attn_fwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        auto kern = !a.drop.thresh ? attn_fwd_kernel<NODROP, HP, NPAN, W, G> : a.drop.small && seq % 2 == 0 ? attn_fwd_kernel<PAIRS, HP, NPAN, W, G> : attn_fwd_kernel<MADE, HP, NPAN, W, G>;
+        auto kern = !a.drop.thresh ? attn_fwd_kernel<NODROP, HP, NPAN, W, G>
+                    : a.drop.small && seq % 2 == 0 ? attn_fwd_kernel<PAIRS, HP, NPAN, W, G>
+                                                   : attn_fwd_kernel<MADE, HP, NPAN, W, G>;
         return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(false, false), a, st);
     }
 };
 struct attn_dq_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        auto kern = a.keep ? attn_bwd_dq_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_dq_kernel<MADE, HP, NPAN, W, G> : attn_bwd_dq_kernel<NODROP, HP, NPAN, W, G>;
+        auto kern = a.keep ? attn_bwd_dq_kernel<KEPT, HP, NPAN, W, G>
+                    : a.drop.thresh ? attn_bwd_dq_kernel<MADE, HP, NPAN, W, G>
+                                    : attn_bwd_dq_kernel<NODROP, HP, NPAN, W, G>;
         return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, false), a, st);
     }
 };
 struct attn_dkv_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
-        auto kern = a.keep ? attn_bwd_dkv_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_dkv_kernel<MADE, HP, NPAN, W, G> : attn_bwd_dkv_kernel<NODROP, HP, NPAN, W, G>;
-        return attn_go(kern, seq, W * 32, nbh * NPAN, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);   // 128-wide heads: a block per half
+        auto kern = a.keep ? attn_bwd_dkv_kernel<KEPT, HP, NPAN, W, G>
+                    : a.drop.thresh ? attn_bwd_dkv_kernel<MADE, HP, NPAN, W, G>
+                                    : attn_bwd_dkv_kernel<NODROP, HP, NPAN, W, G>;
+        // 128-wide heads: a block per half
+        return attn_go(kern, seq, W * 32, nbh * NPAN, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);
     }
 };
 // Both backward kernels: in one launch where all blocks of the two find room at once (two blocks of four waves a CU, one of eight),
@@ -1125,7 +1140,9 @@ struct attn_bwd_launch {
             return rc ? rc : attn_dkv_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
         }
         const size_t lds = own_at + (size_t)HP * ((seq + 63) / 64 * 64) * sizeof(float);
-        auto kern = a.keep ? attn_bwd_kernel<KEPT, HP, NPAN, W, G> : a.drop.thresh ? attn_bwd_kernel<MADE, HP, NPAN, W, G> : attn_bwd_kernel<NODROP, HP, NPAN, W, G>;
+        auto kern = a.keep ? attn_bwd_kernel<KEPT, HP, NPAN, W, G>
+                    : a.drop.thresh ? attn_bwd_kernel<MADE, HP, NPAN, W, G>
+                                    : attn_bwd_kernel<NODROP, HP, NPAN, W, G>;
         BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, lds));
         bb_launch(kern, dim3(dkv + dq), dim3(W * HP * G * 64), lds, st, a, (int)dkv, (int)own_at);
         BB_LAUNCH_CHECK();

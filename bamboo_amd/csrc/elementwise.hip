@@ -33,19 +33,6 @@ extern "C" int bb_init(void) {
     return ln_bwd_static_setup(dev);   // so that bb_layernorm_bwd_static has nothing left to set up on this device
 }
 
-// 16 raw bytes -> VEC floats
-__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(t[i]);
-}
-__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[8]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __uint_as_float(t[i] << 16);
-        v[2 * i + 1] = __uint_as_float(t[i] & 0xffff0000u);
-    }
-}
-
 // =========================================================================================
 // LayerNorm
 // =========================================================================================
@@ -136,6 +123,19 @@ __global__ __launch_bounds__(256) void layernorm_fwd_memory_kernel(int kind, int
 template <int N> __device__ __forceinline__ void store_f32s(float* dst, const float* v) {
 #pragma unroll
     for (int e = 0; e < N; e += 4) *(f32x4*)(dst + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
+}
+
+// 16 raw bytes -> VEC floats
+__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(t[i]);
+}
+__device__ __forceinline__ void unpack16(const u32x4& t, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(t[i] << 16);
+        v[2 * i + 1] = __uint_as_float(t[i] & 0xffff0000u);
+    }
 }
 
 constexpr int LN_BWD_BLOCKS = 256;

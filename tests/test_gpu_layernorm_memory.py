@@ -1,5 +1,5 @@
 """The decoder layer's memory sqrt(1 - x) beside its LayerNorm: the bits of the separate launches, forward and backward, at row lengths on
-either side of what a wave holds and of what it loads early."""
+either side of what a wave holds."""
 import pytest
 import torch
 
