@@ -136,7 +136,7 @@ __device__ __forceinline__ bf16x8 pack_acc(const f32x16& a, int half) {
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 // Kept decisions.  A hash per two decisions, 8 vector instructions each, is what a pass over the probabilities costs beyond an undropped
 // one (19 where a lane's probabilities are not neighbours, as in dK/dV); the forward leaves the decisions as bits instead, for
-// both backward passes: 8 x 16 heads of 64, 1024 keys, dropout: backward 211 -> 172 us, forward 72 -> 80
+// both backward passes, where its caller has room for them: 8 x 16 heads of 64, 1024 keys, dropout: backward 201 -> 171 us, forward 77 -> 80
 // Layout: [batch, heads][queries / 32][keys / 32, tiles of 64 in full][32 words]; a word has the decisions of a query, bit j that of
 // the j-th of 32 keys; the words lie in the order of accumulator rows, those of register r of the lower and the upper half wave next
 // to each other: 64 bits that select lanes as they are.
@@ -484,7 +484,8 @@ void attn_fwd_kernel(const AttnArgs a) {
 // go beside dS, so that a wave starts a sub-tile on the vector ALU at once, and operands are read from LDS a phase ahead.  What it gives
 // is latency, where a SIMD has one wave: 2 x 8 heads of 64, 1024 keys 38.2 us one after the other, 33.1 this way.  Beyond that the two are
 // equal (8 x 16 heads, 1024: 140 us, 865 TFLOP/s of matrix work; two, three or four waves a SIMD the same within 3 %; without the
-// exponentials 121, without LDS reads 118): what bounds it is power, a clock of 2.1 GHz.  A wave walks only sub-tiles of 32 that
+// exponentials 121, without LDS reads 118): no one of them bounds it, and neither does power alone (causal, of a CU in use: matrix
+// pipe 33 %, vector ALU 35 to 45 %, at 2.2 to 2.3 of 2.4 GHz).  A wave walks only sub-tiles of 32 that
 // hold a pair its mask keeps; with the waits outside of the loop (below) 8 x 16 heads, 1024 causal 100.8 -> 90.9, unmasked 157 -> 139.
 constexpr bool attn_bwd_pipe(int npan) { return npan == 1; }
 // stages of a ring: three where a tile's last products come behind the barrier that hands the next tile out, two where three do not fit

@@ -165,7 +165,7 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     //    accumulator tiles per wave, about 9 % below the 256x256 tile at equal fill) instead of falling back
     //    to 128x128: compared by the share of the occupied tile slots that is real output.  (Alone, the QKV
     //    projection 8192x3072 - 1.5 rounds of 256x256 tiles, exactly two of 256x192 - is 19 % faster on them;
-    //    inside the power-limited stage the whole batch is 1 % slower, so 75 % full rounds stay on 256x256.)
+    //    inside the stage the whole batch is 1 % slower, so 75 % full rounds stay on 256x256.)
     if (nt && k64 && big_ok && t2128 > 256) {
         auto useful = [&](int bn) {   // real output / output slots of whole rounds
             const int64_t t = (int64_t)((M + 255) / 256) * ((N + bn - 1) / bn) * batches;

@@ -236,8 +236,8 @@ class TransformerLayer:
         if not self.fused_attention(ctx):
             return [(f"prob{tag}", (ctx.batch, self.heads, ctx.seq, ctx.seq), ctx.dtype)]
         specs = [(f"lse{tag}", (ctx.batch, self.heads, ctx.seq), torch.float32)]
-        # The bits buy time by the byte at any length (made again / kept, forward and backward, us: 8 x 16 heads of 64, 1024 keys 88 + 202 /
-        # 80 + 174 for 16 MB; 2 x 16, 2048 causal 56 + 135 / 58 + 119 for 16; 1 x 16, 4096 causal 105 + 252 / 108 + 229 for 32; 2 x 16 of
+        # The bits buy time by the byte at any length (made again / kept, forward and backward, us: 8 x 16 heads of 64, 1024 keys 77 + 201 /
+        # 80 + 171 for 16 MB; 2 x 16, 2048 causal 56 + 135 / 58 + 119 for 16; 1 x 16, 4096 causal 105 + 253 / 108 + 229 for 32; 2 x 16 of
         # 32, 2048 causal 77 + 178 / 80 + 133 for 16), but they grow by the square of it and everything else here by the length
         if self.dropout > 0 and self.keep_dropout and ctx.seq <= 32 * self.head_dim:
             specs.append((f"keep{tag}", (hip.attention_keep_words(ctx.batch, self.heads, ctx.seq),), torch.int32))
@@ -406,7 +406,7 @@ class TransformerLayer:
         hip.layernorm_fwd(st["x1"], w["sublayer.1.norm.a_2"], w["sublayer.1.norm.b_2"], st["n2"], st["mean2"],
                           st["rinv2"], kind, self.eps, stream=sm)
         # activation and its derivative (kept for the backward pass, which then multiplies instead of
-        # evaluating act') both leave the GEMM epilogue: on the power-limited stage the saved pass over the
+        # evaluating act') both leave the GEMM epilogue: inside the stage the saved pass over the
         # pre-activation (read 64 MB, write 64 MB at the GPT-2-medium shapes) outweighs the epilogue's
         # transcendental work (measured inside the stage, not on the kernel alone)
         if ctx.defer or self.activation == "relu":
