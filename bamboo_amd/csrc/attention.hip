@@ -15,7 +15,7 @@
 // owns a PAIR of neighbouring heads, whose columns together are one 64-wide slice: the tiles in LDS and
 // their loads are those of one 64-wide head, each head has waves of its own, which take the k-steps
 // (scores) and the output tile (context, gradients) of that head.  (Waves that took one head after the
-// other: 8 x 8 pairs, 128 keys, dropout 9.3 us forward, 15.8 backward; so 8.6 and 13.1.)
+// other: 8 x 8 pairs, 128 keys, dropout 9.1 us forward; so, two waves a head, 6.6.)
 // Operands that are contracted
 // over their row index (V in O = PV, Q and dO in dK/dV, K in dQ) are read from LDS with
 // ds_read_b64_tr_b16.  Tiles travel global -> LDS by DMA (global_load_lds_dwordx4),
@@ -1113,11 +1113,11 @@ struct attn_dkv_launch {
 // else one after the other.  Each alone is bound by its longest walk while at most half of the chip has work; together they take
 // the longer of the two instead of the sum, and a launch less.  What it costs is delta a second time, by every dK / dV block for the
 // queries it will meet, and registers: beyond a round both weigh more than what overlaps.  One after the other / together (us): 2 x 2
-// heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (64 + 64 blocks) 23.8 / 16.1; 6 x 8, 175 (96 + 96) 17.7 / 12.0; 2 x
+// heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (128 + 128 blocks) 12.9 / 8.9, 4 x 8, 512 (256 + 256) 23.4 / 18.8; 6 x 8, 175 (96 + 96) 17.7 / 12.0; 2 x
 // 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two heads of 128, 512, dropout 69.0 /
 // 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
 // 192) 68 / 73, 4 x 16, 256 causal (256 + 256 of eight) 18.0 / 18.5.  The bits are the same.
-// LDS has room for what the waves allow (of blocks of two waves three instead of four a CU, 768; they are at most 512), but for one shape: blocks of
+// LDS has room for what the waves allow (of blocks of two waves three a CU instead of four, 768; they are at most 512), but for one shape: blocks of
 // four waves whose two rings fill more than half of it (64-wide heads, two waves in two groups) are one a CU.  A round and
 // a quarter, empty blocks of uneven XCDs among it (they go to no other XCD), is still the faster way with padding: the blocks left over
 // follow those of dQ, whose walks are the shorter ones.  Under a causal mask, which has short blocks to follow the long ones, up to two rounds
@@ -1173,7 +1173,11 @@ struct attn_bwd_launch {
 // backward, whose waves look ahead by themselves, only where the walk is long, and it loses the launch that both passes share.
 // Heads of 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.  Pairs of heads have twice the
 // waves: two a head in two groups (a walk of both heads by two waves in four groups / this: 1 x 4 pairs, 500 causal 9.6 16.4 / 8.3 15.3,
-// 2 x 4, 300, padding, dropout 9.6 20.7 / 7.8 17.0; four waves in two groups / four a head: 4 x 8, 512 causal 10.6 24.8 / 9.2 22.4).
+// 2 x 4, 300, padding, dropout 9.6 20.7 / 7.8 17.0; four waves in two groups / four a head: 4 x 8, 512 causal 10.6 24.8 / 9.2 22.4); else
+// two a head, blocks as small as those of four waves of one head, for one block of eight waves a CU stands still at every barrier (four
+// a head / two, forward and backward with kept decisions: 8 x 8 pairs, 128, dropout 8.9 11.2 / 6.6 9.6; 4 x 8, 1020, dropout 41.4 73.1 / 40.5 72.0,
+// causal 40.7 73.4 / 29.4 57.1; decisions made again, 7 x 7, 1633 226 559 / 182 455, causal 130 322 / 89 226, padding 163 389 / 127 336, without
+// dropout 81 213 / 74 197).
 // Attention without a mask keeps the one walk.  Groups add the same terms in another order: as near the exact sums as before, but
 // not the same last bits, and the stage that ends the reference's script (no mask; a LayerNorm whose rows are summed up, which
 // cancels to 1e-4 of its terms) passes gradients on in which such bits show as 3 to 5 %.
@@ -1182,6 +1186,7 @@ template <typename L, int HP, int NPAN> static int attn_shape(int seq, int nbh, 
     const bool masked = a.mask != BB_MASK_NONE;
     if constexpr (HP == 2) {
         if (masked && blocks <= 128 && seq >= 160) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
+        return L::template go<HP, NPAN, 2, 1>(seq, nbh, a, st);
     } else if constexpr (NPAN == 2) {
         if (masked && blocks <= 256 && seq >= 448) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
     } else if constexpr (std::is_same_v<L, attn_fwd_launch>) {
@@ -1196,7 +1201,7 @@ template <typename L, int HP, int NPAN> static int attn_shape(int seq, int nbh, 
         if (masked && seq >= 320 && blocks <= 64) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
         if (blocks <= 128 && seq <= 320) return L::template go<HP, NPAN, 2, 1>(seq, nbh, a, st);
     }
-    return L::template go<HP, NPAN, 4, 1>(seq, nbh, a, st);
+    if constexpr (HP == 1) return L::template go<HP, NPAN, 4, 1>(seq, nbh, a, st);
 }
 template <typename L> static int attn_launch(int head_dim, int seq, int batch, int heads, const AttnArgs& a, hipStream_t st) {
     if (head_dim == 128) return attn_shape<L, 1, 2>(seq, batch * heads, a, st);

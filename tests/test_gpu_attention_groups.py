@@ -16,7 +16,7 @@ SHAPES = [(1, 2, 160, 64), (2, 3, 193, 64),                             # 2x4, 2
           (1, 36, 448, 64), (1, 43, 577, 64),                           # 2x2, 4x1
           (1, 11, 1537, 64),                                            # 2x2, 4x2
           (1, 33, 1025, 64),                                            # 2x2 if causal, else 4x1, both backward 4x1
-          (1, 4, 80, 32), (2, 60, 289, 32),                             # pairs of heads: 4x1
+          (1, 4, 80, 32), (2, 60, 289, 32),                             # pairs of heads: 2x1
           (2, 6, 257, 32), (2, 16, 600, 32),                            # 2x2, in one launch and in two
           (1, 2, 448, 128), (2, 4, 521, 128), (1, 30, 500, 128)]        # 4x2, the last in two
 
