@@ -268,8 +268,13 @@ enum { NODROP = 0, MADE = 1, KEPT = 2, PAIRS = 3 };
 // (even sequences, fewer than 2^32 probabilities; branches between the ways to make them cost moves and a wave in three); read from
 // what the forward kept, in the backward
 // KS k-steps of a head's scores, DT 32-wide output tiles of a head
+// waves a SIMD: at least, for the registers; at most, for a kernel whose LDS lets no more in (128-wide heads).  Told of three it could not
+// have anyhow, the compiler read V from LDS in front of each matrix instruction, a wait each, on 160 registers: 1 x 2 heads of 128, 1150 causal
+// 26.4 us in the order of 209 registers, 28.1 in that of 160
+constexpr int attn_fwd_most(int drop, int npan) { return drop == NODROP && npan == 2 ? 2 : 8; }
+constexpr int attn_fwd_waves(int drop, int npan, int g) { return npan == 1 && g == 1 ? (drop == NODROP ? 4 : drop == PAIRS ? 3 : 2) : 2; }
 template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
-__global__ __launch_bounds__(W * HP * G * 64, NPAN == 1 && G == 1 ? (DROP == NODROP ? 4 : DROP == PAIRS ? 3 : 2) : 2)
+__global__ __launch_bounds__(W * HP * G * 64) __attribute__((amdgpu_waves_per_eu(attn_fwd_waves(DROP, NPAN, G), attn_fwd_most(DROP, NPAN))))
 void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
