@@ -136,7 +136,10 @@ __device__ __forceinline__ bf16x8 pack_acc(const f32x16& a, int half) {
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 // Kept decisions.  A hash per two decisions, 8 vector instructions each, is what a pass over the probabilities costs beyond an undropped
 // one (19 where a lane's probabilities are not neighbours, as in dK/dV); the forward leaves the decisions as bits instead, for
-// both backward passes, where its caller has room for them: 8 x 16 heads of 64, 1024 keys, dropout: backward 201 -> 171 us, forward 77 -> 80
+// both backward passes, where its caller has room for them: 8 x 16 heads of 64, 1024 keys, dropout: unmasked backward 201 -> 171 us, forward
+// 80 either way, causal 118 -> 109 and 47 -> 48.  A forward that keeps none is a kernel of its own: putting bits together costs an
+// instruction a decision and 14 to 30 registers (with them all the same, odd sequences: 8 x 16, 1023 padded 84 us, 69 without; 2 x 12, 1021 unmasked
+// 34.5, 32.9; 8 x 8 heads, 175 9.8, 9.6; 4 x 8 of 128, 501 25.4, 24.7).
 // Layout: [batch, heads][queries / 32][keys / 32, tiles of 64 in full][32 words]; a word has the decisions of a query, bit j that of
 // the j-th of 32 keys; the words lie in the order of accumulator rows, those of register r of the lower and the upper half wave next
 // to each other: 64 bits that select lanes as they are.
@@ -273,7 +276,7 @@ enum { NODROP = 0, MADE = 1, KEPT = 2, PAIRS = 3 };
 // 26.4 us in the order of 209 registers, 28.1 in that of 160
 constexpr int attn_fwd_most(int drop, int npan) { return drop == NODROP && npan == 2 ? 2 : 8; }
 constexpr int attn_fwd_waves(int drop, int npan, int g) { return npan == 1 && g == 1 ? (drop == NODROP ? 4 : drop == PAIRS ? 3 : 2) : 2; }
-template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1>
+template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1, bool KEEP = false>
 __global__ __launch_bounds__(W * HP * G * 64) __attribute__((amdgpu_waves_per_eu(attn_fwd_waves(DROP, NPAN, G), attn_fwd_most(DROP, NPAN))))
 void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
@@ -380,7 +383,7 @@ void attn_fwd_kernel(const AttnArgs a) {
             uint32_t kept[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u) kept[u] = drop_acc_rows<DROP == PAIRS>(a.drop, base + u * 32, lane, s[u]);
-            if (a.keep) {
+            if constexpr (KEEP) {
                 // the halves of a wave have each other's nibbles; the lower one stores the words of the first 32 keys
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
@@ -1091,9 +1094,10 @@ template <typename K> static int attn_go(K kern, int seq, int rows, int nbh, int
 // dropout is a kernel of its own: its keep decisions cost registers that decide how many blocks a CU holds
 struct attn_fwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
+        const bool pairs = a.drop.small && seq % 2 == 0;
         auto kern = !a.drop.thresh ? attn_fwd_kernel<NODROP, HP, NPAN, W, G>
-                    : a.drop.small && seq % 2 == 0 ? attn_fwd_kernel<PAIRS, HP, NPAN, W, G>
-                                                   : attn_fwd_kernel<MADE, HP, NPAN, W, G>;
+                    : a.keep       ? (pairs ? attn_fwd_kernel<PAIRS, HP, NPAN, W, G, true> : attn_fwd_kernel<MADE, HP, NPAN, W, G, true>)
+                                   : (pairs ? attn_fwd_kernel<PAIRS, HP, NPAN, W, G> : attn_fwd_kernel<MADE, HP, NPAN, W, G>);
         return attn_go(kern, seq, W * 32, nbh, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(false, false), a, st);
     }
 };
@@ -1118,8 +1122,8 @@ struct attn_dkv_launch {
 // else one after the other.  Each alone is bound by its longest walk while at most half of the chip has work; together they take
 // the longer of the two instead of the sum, and a launch less.  What it costs is delta a second time, by every dK / dV block for the
 // queries it will meet, and registers: beyond a round both weigh more than what overlaps.  One after the other / together (us): 2 x 2
-// heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (128 + 128 blocks) 12.9 / 8.9, 4 x 8, 512 (256 + 256) 23.4 / 18.8; 6 x 8, 175 (96 + 96) 17.7 / 12.0; 2 x
-// 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two heads of 128, 512, dropout 69.0 /
+// heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (128 + 128 blocks) 12.9 / 8.9, 4 x 8, 512 (256 + 256) 23.4 / 18.8; 6 x
+// 8, 175 (96 + 96) 17.7 / 12.0; 2 x 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two heads of 128, 512, dropout 69.0 /
 // 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
 // 192) 68 / 73, 4 x 16, 256 causal (256 + 256 of eight) 18.0 / 18.5.  The bits are the same.
 // LDS has room for what the waves allow (of blocks of two waves three a CU instead of four, 768; they are at most 512), but for one shape: blocks of
