@@ -271,13 +271,14 @@ enum { NODROP = 0, MADE = 1, KEPT = 2, PAIRS = 3 };
 // (even sequences, fewer than 2^32 probabilities; branches between the ways to make them cost moves and a wave in three); read from
 // what the forward kept, in the backward
 // KS k-steps of a head's scores, DT 32-wide output tiles of a head
-// waves a SIMD: at least, for the registers; at most, for a kernel whose LDS lets no more in (128-wide heads).  Told of three it could not
-// have anyhow, the compiler read V from LDS in front of each matrix instruction, a wait each, on 160 registers: 1 x 2 heads of 128, 1150 causal
-// 26.4 us in the order of 209 registers, 28.1 in that of 160
-constexpr int attn_fwd_most(int drop, int npan) { return drop == NODROP && npan == 2 ? 2 : 8; }
+// waves a SIMD: at least, for the registers; at most, for kernels whose LDS lets no more in (128-wide heads, four rings).  Told of three they could
+// not have anyhow, the compiler read V from LDS in front of each matrix instruction, a wait each, on 160 and 115 registers; in the order of 209 and
+// 132 (us): 1 x 2 heads of 128, 1150 causal 28.1 -> 25.5, 2 x 8, 2000 58.5 -> 48.7; two waves in four groups 1 x 2 of 64, 1500 causal 14.9 ->
+// 14.1, 2 x 8, 1024 12.1 -> 11.7.  (Two waves in two groups: 1 x 12, 2043 causal 23.3 -> 21.5, padded 17.0 -> 17.7, 1 x 22, 2000 25.3 -> 26.8: not.)
+constexpr int attn_fwd_most(int drop, int npan, int g) { return drop == NODROP && (npan == 2 || g == 4) ? 2 : 8; }
 constexpr int attn_fwd_waves(int drop, int npan, int g) { return npan == 1 && g == 1 ? (drop == NODROP ? 4 : drop == PAIRS ? 3 : 2) : 2; }
 template <int DROP, int HP, int NPAN = 1, int W = 4, int G = 1, bool KEEP = false>
-__global__ __launch_bounds__(W * HP * G * 64) __attribute__((amdgpu_waves_per_eu(attn_fwd_waves(DROP, NPAN, G), attn_fwd_most(DROP, NPAN))))
+__global__ __launch_bounds__(W * HP * G * 64) __attribute__((amdgpu_waves_per_eu(attn_fwd_waves(DROP, NPAN, G), attn_fwd_most(DROP, NPAN, G))))
 void attn_fwd_kernel(const AttnArgs a) {
     static_assert(HP == 1 || NPAN == 1, "pairs of heads are 32 wide");
     constexpr int KS = 4 * NPAN / HP, DT = 2 * NPAN / HP, TILE = NPAN * 8192, ROWS = W * 32, DW = W * HP;
@@ -1123,8 +1124,8 @@ struct attn_dkv_launch {
 // the longer of the two instead of the sum, and a launch less.  What it costs is delta a second time, by every dK / dV block for the
 // queries it will meet, and registers: beyond a round both weigh more than what overlaps.  One after the other / together (us): 2 x 2
 // heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (128 + 128 blocks) 12.9 / 8.9, 4 x 8, 512 (256 + 256) 23.4 / 18.8; 6 x
-// 8, 175 (96 + 96) 17.7 / 12.0; 2 x 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two heads of 128, 512, dropout 69.0 /
-// 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
+// 8, 175 (96 + 96) 17.7 / 12.0; 2 x 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two
+// heads of 128, 512, dropout 69.0 / 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
 // 192) 68 / 73, 4 x 16, 256 causal (256 + 256 of eight) 18.0 / 18.5.  The bits are the same.
 // LDS has room for what the waves allow (of blocks of two waves three a CU instead of four, 768; they are at most 512), but for one shape: blocks of
 // four waves whose two rings fill more than half of it (64-wide heads, two waves in two groups) are one a CU.  A round and
