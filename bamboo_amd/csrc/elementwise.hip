@@ -162,6 +162,10 @@ template <int VEC> __device__ __forceinline__ void drop_vec(const DropKey& key, 
 // DROP: dropped = dropout(dx) as well, what dropout_kernel makes of the stored dx: its launch, and its pass over dx, are saved
 // (two launches / one, bf16, us: 8192x1024 21.0 / 16.7, 4096x1600 20.9 / 18.6, 2048x4096 34.3 / 32.4)
 // MEMORY: dx takes what sqrt1m_bwd_kernel would add to it, as stored (m = sqrt(1 - x), dm its gradient)
+// EARLY: so many of a lane's vectors of dm and m are fetched with the row, as the registers allow; the others where they are used, so that
+// next to nothing goes to scratch memory.  Two launches / all with the row / this, device time (us): fp32 256x1024 8.2 / 14.5 / 7.8, 8192x1024 44.0 /
+// 58.4 / 36.7, 2048x2048 24.9 / 30.2 / 19.0, 2048x3072 42.8 / 46.4 / 38.0, 8192x2560 148 / 162 / 140; bf16 8192x128 8.1 / 8.9 / 7.5, 2048x768 9.8 /
+// 8.9 / 7.4, 8192x1024 25.7 / 24.8 / 19.4, 256x1600 9.2 / 9.9 / 9.0, 8192x1600 40.7 / 33.7 / 34.2; bf16 beyond 2048 columns, all / none 8192x4096 148 / 179.
 template <typename T, int IT, bool DROP, bool MEMORY>
 __device__ __forceinline__ void layernorm_bwd_rows(int kind, int rows, int cols, float eps, const T* __restrict__ x, const T* __restrict__ gain,
                                                    const float* __restrict__ mean_in, const float* __restrict__ rinv_in,
@@ -172,6 +176,7 @@ __device__ __forceinline__ void layernorm_bwd_rows(int kind, int rows, int cols,
     extern __shared__ float red[];  // [all waves][2][cols] (one pass) or [3 waves][2][cols] for the cross-wave sum
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nvec = cols / VEC;
+    constexpr int EARLY = !MEMORY ? 0 : sizeof(T) == 2 ? (IT >= 8 ? IT : 0) : (IT == 16 ? 8 : 0);
     float gv[IT][VEC], dg[IT][VEC], db[IT][VEC];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
@@ -185,15 +190,15 @@ __device__ __forceinline__ void layernorm_bwd_rows(int kind, int rows, int cols,
         const T* xr = x + (int64_t)row * cols;
         const T* dyr = dy + (int64_t)row * cols;
         float xh[IT][VEC], dyh[IT][VEC];
-        u32x4 rdm[MEMORY ? IT : 1], rm[MEMORY ? IT : 1];
+        u32x4 rdm[EARLY ? EARLY : 1], rm[EARLY ? EARLY : 1];
         u32x4 rres[IT];   // the residual gradient, fetched with the row (16 bytes per vector, unpacked at the end)
         float s1 = 0.f, s2 = 0.f;
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
             const int c = lane + i * 64;
             if (dres && c < nvec) rres[i] = *(const u32x4*)(dres + (int64_t)row * cols + c * VEC);
-            if constexpr (MEMORY) {
-                if (c < nvec) {
+            if constexpr (EARLY) {
+                if (i < EARLY && c < nvec) {
                     rdm[i] = *(const u32x4*)(dm + (int64_t)row * cols + c * VEC);
                     rm[i] = *(const u32x4*)(m + (int64_t)row * cols + c * VEC);
                 }
@@ -255,8 +260,13 @@ __device__ __forceinline__ void layernorm_bwd_rows(int kind, int rows, int cols,
                 };
                 if constexpr (MEMORY) {
                     float g[VEC], mv[VEC];
-                    unpack16(rdm[i], g);
-                    unpack16(rm[i], mv);
+                    if (i < EARLY) {
+                        unpack16(rdm[i], g);
+                        unpack16(rm[i], mv);
+                    } else {
+                        load_vec(dm + (int64_t)row * cols + c * VEC, g);
+                        load_vec(m + (int64_t)row * cols + c * VEC, mv);
+                    }
                     as_stored();
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) o[e] += g[e] * (-0.5f / mv[e]);
@@ -486,6 +496,14 @@ static int layernorm_fwd(int dtype, int kind, int rows, int cols, float eps, con
     BB_REQUIRE(x && gain && shift && y && mean && rinv, "bb_layernorm_fwd: null pointer");
     BB_REQUIRE(kind != BB_LN_ANNOTATED || cols > 1, "bb_layernorm_fwd: annotated LayerNorm needs cols > 1");
     if (rows == 0) return BB_OK;
+    // Few and wide rows leave most CUs without one, and square roots of a row's length to those that have one: two launches / one (us), 256
+    // and 512 rows, bf16 3072 columns 7.3 7.9 / 7.6 8.1, 4096 8.1 9.0 / 9.1 9.7, 2560 6.9 7.4 / 6.7 7.2; fp32 2560 8.1 8.9 / 8.7 9.4, 4096 10.1
+    // 12.5 / 11.9 14.4, 2048 7.2 7.7 / 7.0 7.6; 1024 rows, 4096 bf16 11.1 / 10.7, fp32 18.3 / 17.2.
+    if (memory && rows <= 512 && cols > (dtype == BB_BF16 ? 2560 : 2048)) {
+        rc = bb_sqrt_one_minus_fwd(dtype, (int64_t)rows * cols, x, memory, stream);
+        if (rc) return rc;
+        memory = nullptr;
+    }
     hipStream_t st = (hipStream_t)stream;
     if (dtype == BB_BF16)
         BB_DISPATCH_IT(bf16, cols / 8, (ln_fwd_launch<bf16, IT>(kind, rows, cols, eps, x, gain, shift, y, mean, rinv, memory, st)));
@@ -562,6 +580,12 @@ extern "C" int bb_layernorm_bwd_rows_memory(int dtype, int kind, int rows, int c
                                             float* dshift, float* partials, bb_partial_sums* sums, const void* dm, const void* m, void* stream) {
     BB_REQUIRE(dgain && dshift && sums && dm && m, "bb_layernorm_bwd_rows_memory: null pointer");
     *sums = {partials, dgain, dshift, 0, cols};
+    // (as in the forward: two launches / one, fp32 4096 columns, 256 rows 19.5 / 22.2 us, 512 23.4 / 24.1, 1024 30.2 / 27.7; 3072, 256 14.5 / 13.6)
+    if (dtype == BB_F32 && rows <= 512 && cols > 3072) {
+        const int rc = ln_bwd_rows("bb_layernorm_bwd_rows_memory", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, partials,
+                                   sums->parts, (hipStream_t)stream);
+        return rc ? rc : bb_sqrt_one_minus_bwd(dtype, (int64_t)rows * cols, dm, m, dx, 1, stream);
+    }
     return ln_bwd_rows("bb_layernorm_bwd_rows_memory", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, partials, sums->parts,
                        (hipStream_t)stream, nullptr, DropKey{}, dm, m);
 }

@@ -1,5 +1,5 @@
 """The decoder layer's memory sqrt(1 - x) beside its LayerNorm: the bits of the separate launches, forward and backward, at row lengths on
-either side of what a wave holds."""
+either side of what a wave holds, and of where the launches stay separate."""
 import pytest
 import torch
 
@@ -7,7 +7,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,cols", [(1, 8), (5, 64), (1023, 512), (130, 1032), (33, 2056), (9, 4096)])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (5, 64), (1023, 512), (130, 1032), (33, 2056), (9, 4096),
+                                       (7, 1600), (512, 2560), (512, 2568), (513, 3080), (512, 3072), (513, 4096)])
 def test_memory(hiplib, dtype, rows, cols):
     g = torch.Generator(device="cuda").manual_seed(rows + cols)
     rand = lambda *shape, t=dtype: torch.randn(*shape, generator=g, device="cuda").to(t)
