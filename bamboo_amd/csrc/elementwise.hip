@@ -37,7 +37,12 @@ extern "C" int bb_init(void) {
 // LayerNorm
 // =========================================================================================
 // Row held in registers: lane owns vectors lane, lane+64, ... (IT of them, VEC elements each).
-template <typename T, int IT, bool MEMORY>
+// MEMORY: 1, each of a lane's vectors is followed by its square roots and their store, which spreads the stores of many rows over the
+// kernel; 2, by none of them before the whole row is there: up to 1024 rows (fp32 512) wait for memory and not for its bandwidth,
+// and the stores keep the next vector's load behind the wait for this one (1 / 2, us: 160x1600 bf16 6.4 / 6.1, fp32 6.5 / 5.8; 512x2048 5.8 /
+// 5.6, 7.3 / 7.0; 1024x2560 7.7 / 7.5, 10.3 / 10.4; 1024x3072 8.7 / 8.5, 12.0 / 12.5; 2048x2560 9.3 / 9.7, 13.6 / 14.4; 8192x1024 11.2 / 12.1, 15.7 /
+// 16.2; two vectors a lane, 160x512 bf16 3.0 / 3.1).
+template <typename T, int IT, int MEMORY>
 __device__ __forceinline__ void layernorm_fwd_rows(int kind, int rows, int cols, float eps, const T* __restrict__ x, const T* __restrict__ gain,
                                                    const T* __restrict__ shift, T* __restrict__ y, float* __restrict__ mean_out,
                                                    float* __restrict__ rinv_out, T* __restrict__ memory) {
@@ -47,6 +52,12 @@ __device__ __forceinline__ void layernorm_fwd_rows(int kind, int rows, int cols,
     if (row >= rows) return;
     const int nvec = cols / VEC;
     const T* xr = x + (int64_t)row * cols;
+    auto leave_memory = [&](int c, const float (&xv)[VEC]) {      // as sqrt1m_fwd_kernel, whose launch and pass over x are saved
+        float mv[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) mv[e] = sqrtf(1.0f - xv[e]);
+        store_vec(memory + (int64_t)row * cols + c * VEC, mv);
+    };
     float v[IT][VEC];
     float s = 0.f;
 #pragma unroll
@@ -54,17 +65,19 @@ __device__ __forceinline__ void layernorm_fwd_rows(int kind, int rows, int cols,
         const int c = lane + i * 64;
         if (c < nvec) {
             load_vec(xr + c * VEC, v[i]);
-            if constexpr (MEMORY) {      // as sqrt1m_fwd_kernel, whose launch and pass over x are saved
-                float mv[VEC];
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) mv[e] = sqrtf(1.0f - v[i][e]);
-                store_vec(memory + (int64_t)row * cols + c * VEC, mv);
-            }
+            if constexpr (MEMORY == 1) leave_memory(c, v[i]);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) s += v[i][e];
         } else {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) v[i][e] = 0.f;
+        }
+    }
+    if constexpr (MEMORY == 2) {
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int c = lane + i * 64;
+            if (c < nvec) leave_memory(c, v[i]);
         }
     }
     const float mean = wave_sum(s) / (float)cols;
@@ -109,14 +122,14 @@ template <typename T, int IT>
 __global__ __launch_bounds__(256) void layernorm_fwd_kernel(int kind, int rows, int cols, float eps, const T* __restrict__ x,
                                                             const T* __restrict__ gain, const T* __restrict__ shift, T* __restrict__ y,
                                                             float* __restrict__ mean_out, float* __restrict__ rinv_out) {
-    layernorm_fwd_rows<T, IT, false>(kind, rows, cols, eps, x, gain, shift, y, mean_out, rinv_out, nullptr);
+    layernorm_fwd_rows<T, IT, 0>(kind, rows, cols, eps, x, gain, shift, y, mean_out, rinv_out, nullptr);
 }
-template <typename T, int IT>
+template <typename T, int IT, int MEMORY>
 __global__ __launch_bounds__(256) void layernorm_fwd_memory_kernel(int kind, int rows, int cols, float eps, const T* __restrict__ x,
                                                                    const T* __restrict__ gain, const T* __restrict__ shift,
                                                                    T* __restrict__ y, float* __restrict__ mean_out,
                                                                    float* __restrict__ rinv_out, T* __restrict__ memory) {
-    layernorm_fwd_rows<T, IT, true>(kind, rows, cols, eps, x, gain, shift, y, mean_out, rinv_out, memory);
+    layernorm_fwd_rows<T, IT, MEMORY>(kind, rows, cols, eps, x, gain, shift, y, mean_out, rinv_out, memory);
 }
 
 // N contiguous floats (N a multiple of 4, 16-byte aligned destination)
@@ -433,10 +446,10 @@ template <typename T, int IT>
 static int ln_fwd_launch(int kind, int rows, int cols, float eps, const void* x, const void* gain, const void* shift,
                          void* y, float* mean, float* rinv, void* memory, hipStream_t st) {
     const dim3 grid((rows + 3) / 4);
-    if (memory)
-        bb_launch((layernorm_fwd_memory_kernel<T, IT>), grid, dim3(256), 0, st, kind, rows, cols, eps, (const T*)x, (const T*)gain, (const T*)shift,
-                  (T*)y, mean, rinv, (T*)memory);
-    else
+    if (memory) {
+        auto kern = IT >= 4 && rows * sizeof(T) <= 2048 ? layernorm_fwd_memory_kernel<T, IT, 2> : layernorm_fwd_memory_kernel<T, IT, 1>;
+        bb_launch(kern, grid, dim3(256), 0, st, kind, rows, cols, eps, (const T*)x, (const T*)gain, (const T*)shift, (T*)y, mean, rinv, (T*)memory);
+    } else
         bb_launch((layernorm_fwd_kernel<T, IT>), grid, dim3(256), 0, st, kind, rows, cols, eps, (const T*)x, (const T*)gain, (const T*)shift,
                   (T*)y, mean, rinv);
     BB_LAUNCH_CHECK();
@@ -496,10 +509,10 @@ static int layernorm_fwd(int dtype, int kind, int rows, int cols, float eps, con
     BB_REQUIRE(x && gain && shift && y && mean && rinv, "bb_layernorm_fwd: null pointer");
     BB_REQUIRE(kind != BB_LN_ANNOTATED || cols > 1, "bb_layernorm_fwd: annotated LayerNorm needs cols > 1");
     if (rows == 0) return BB_OK;
-    // Few and wide rows leave most CUs without one, and square roots of a row's length to those that have one: two launches / one (us), 256
-    // and 512 rows, bf16 3072 columns 7.3 7.9 / 7.6 8.1, 4096 8.1 9.0 / 9.1 9.7, 2560 6.9 7.4 / 6.7 7.2; fp32 2560 8.1 8.9 / 8.7 9.4, 4096 10.1
-    // 12.5 / 11.9 14.4, 2048 7.2 7.7 / 7.0 7.6; 1024 rows, 4096 bf16 11.1 / 10.7, fp32 18.3 / 17.2.
-    if (memory && rows <= 512 && cols > (dtype == BB_BF16 ? 2560 : 2048)) {
+    // Few and wide rows leave most CUs without one, and square roots of a row's length to those that have one: two launches / one (us), 32,
+    // 160 and 512 rows, 4096 columns bf16 7.3 7.7 8.7 / 8.1 8.4 9.1, fp32 8.8 9.6 12.3 / 9.8 10.4 12.3; 3072 bf16 6.7 6.8 7.6 / 6.7 7.0 7.5, fp32 7.8
+    // 8.4 9.6 / 8.2 8.6 9.8; 2560 fp32 7.1 7.7 8.7 / 7.3 7.6 8.6; 1024 rows of 4096, bf16 11.1 / 10.7, fp32 18.3 / 17.2.
+    if (memory && rows <= 512 && cols > (dtype == BB_BF16 ? 3072 : 2560)) {
         rc = bb_sqrt_one_minus_fwd(dtype, (int64_t)rows * cols, x, memory, stream);
         if (rc) return rc;
         memory = nullptr;
@@ -580,8 +593,9 @@ extern "C" int bb_layernorm_bwd_rows_memory(int dtype, int kind, int rows, int c
                                             float* dshift, float* partials, bb_partial_sums* sums, const void* dm, const void* m, void* stream) {
     BB_REQUIRE(dgain && dshift && sums && dm && m, "bb_layernorm_bwd_rows_memory: null pointer");
     *sums = {partials, dgain, dshift, 0, cols};
-    // (as in the forward: two launches / one, fp32 4096 columns, 256 rows 19.5 / 22.2 us, 512 23.4 / 24.1, 1024 30.2 / 27.7; 3072, 256 14.5 / 13.6)
-    if (dtype == BB_F32 && rows <= 512 && cols > 3072) {
+    // (as in the forward: two launches / one, fp32 4096 columns, 256 rows 19.5 / 22.2 us, 512 23.4 / 24.1, 1024 30.2 / 27.7; 3072, 256 14.5 / 13.6;
+    // bf16 4096, 25 rows 14.1 / 14.7, 104 14.3 / 14.8, 365 16.0 / 15.4; 3072, 36 11.9 / 11.8)
+    if (rows <= (dtype == BB_F32 ? 512 : 128) && cols > 3072) {
         const int rc = ln_bwd_rows("bb_layernorm_bwd_rows_memory", dtype, kind, rows, cols, eps, x, gain, mean, rinv, dy, dres, dx, partials,
                                    sums->parts, (hipStream_t)stream);
         return rc ? rc : bb_sqrt_one_minus_bwd(dtype, (int64_t)rows * cols, dm, m, dx, 1, stream);
