@@ -1119,32 +1119,31 @@ struct attn_dkv_launch {
         return attn_go(kern, seq, W * 32, nbh * NPAN, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);
     }
 };
-// Both backward kernels: in one launch where all blocks of the two find room at once (two blocks of four waves a CU, one of eight),
-// else one after the other.  Each alone is bound by its longest walk while at most half of the chip has work; together they take
-// the longer of the two instead of the sum, and a launch less.  What it costs is delta a second time, by every dK / dV block for the
-// queries it will meet, and registers: beyond a round both weigh more than what overlaps.  One after the other / together (us): 2 x 2
-// heads of 64, 64 causal 9.5 / 6.0; 8 x 8 pairs of 32, 128, dropout (128 + 128 blocks) 12.9 / 8.9, 4 x 8, 512 (256 + 256) 23.4 / 18.8; 6 x
-// 8, 175 (96 + 96) 17.7 / 12.0; 2 x 8, 1024 (128 + 128) 51.5 / 39.3; 8 x 8, 512 (256 + 256) 34.2 / 29.5; 1 x 2, 1500 69.7 / 52.6; two
-// heads of 128, 512, dropout 69.0 / 52.5; beyond it 4 x 16, 1024, dropout (512 + 512) 130 / 134, 2 x 16, 2000 152 / 170; 12 heads, 2043 in blocks of eight waves (192 +
-// 192) 68 / 73, 4 x 16, 256 causal (256 + 256 of eight) 18.0 / 18.5.  The bits are the same.
-// LDS has room for what the waves allow (of blocks of two waves three a CU instead of four, 768; they are at most 512), but for one shape: blocks of
-// four waves whose two rings fill more than half of it (64-wide heads, two waves in two groups) are one a CU.  A round and
-// a quarter, empty blocks of uneven XCDs among it (they go to no other XCD), is still the faster way with padding: the blocks left over
-// follow those of dQ, whose walks are the shorter ones.  Under a causal mask, which has short blocks to follow the long ones, up to two rounds
-// and a quarter.  One after the other / together: padding, keys in full and at 0.8, 288 blocks (1 x 8, 1100) 31.0 / 26.5 and 29.2 / 25.9, 320
-// (2 x 8, 640) 21.4 / 18.5 and 20.5 / 17.2, 336 (1 x 8, 1344) 35.5 / 43.5 and 33.5 / 29.9, 448 (4 x 7, 448) 19.5 / 21.8 and 18.6 / 20.9, 512 (1 x
-// 8, 2048) 48.2 / 60.9 and 45.1 / 57.6; causal 512 (2 x 8, 1024) 29.3 / 26.4, with dropout 35.5 / 29.3, 528 (3 x 6, 700) 24.5 / 22.8, 608 (1 x 9,
-// 1153) 32.6 / 33.2, 768 (1 x 10, 1500) 39.9 / 47.3.
+// Both backward kernels: in one launch where that ends within a round and a quarter of the blocks that the chip holds, with a causal mask two
+// and a quarter, for its short blocks fill in behind the long ones; else one after the other.  Each alone is bound by its longest walk
+// while at most half of the chip has work; together they take the longer of the two instead of the sum, and a launch less.  What it
+// costs is delta a second time, by every dK / dV block for the queries it will meet, and registers: beyond, both weigh more than
+// what overlaps, and at once where two launches of a whole round each become three rounds.  128-wide heads, which make scores and deltas
+// twice by then, end sooner.  A round is what waves and LDS let in: eight waves a CU, one block of eight or, where two
+// rings fill more than half of LDS (64-wide heads, two waves in two groups), of four.  Heads stay on their XCD, so that uneven ones leave
+// empty blocks in the grid, which go to no other XCD: they count (three heads are on three XCDs, 96 CUs).  One after the
+// other / together (us), by rounds: padding, 64-wide 2x4 7 heads, 1114 keys (1.1) 41.9 / 36.0, 5, 1268 (1.25) 38.2 / 34.3, 1, 1377 (1.4) 34.2 / 42.9,
+// 2, 1997 (2) 44.8 / 57.1; 2x2 16, 640 (1.25) 21.4 / 18.5, 5, 1682 (1.7) 41.3 / 51.3; 4x1 19, 1499 (1.1) 69.0 / 63.4, 46, 1116 (1.7) 53.2 / 50.8; 4x2 12, 1549 (1.6)
+// 56.2 / 63.9; pairs 2x2 2, 1066 (1.1) 31.6 / 26.5, 3, 1323 (1.3) 39.7 / 46.8; no mask, 4x1 25, 1070 (1.1) 65.2 / 56.8, 24, 1934 (1.5) 115.0 / 114.7; pairs 2x1
+// 46, 366 (1.1) 25.3 / 22.1; causal, 2x4 3, 1938 (1.9) 41.4 / 37.3; 2x2 16, 987 (2) 30.8 / 27.0, 9, 1153 (2.4) 32.6 / 33.2, 10, 1500 (3) 39.9 / 47.3; 4x1 28, 1897 (1.9)
+// 88.0 / 77.0; 4x2 16, 1575 (1.6) 54.1 / 42.3; pairs 2x2 12, 1112 (2.25) 35.1 / 33.1, 2x1 17, 1402, dropout (2.1) 90.6 / 78.8, 34, 919 (2.3) 42.5 / 43.8;
+// 128-wide 4x1 no mask 14, 1182 (0.9) 88.0 / 90.0, 20, 1055 (1.1) 88.3 / 106.4, padding 37, 420 (0.9) 43.9 / 37.6, causal 54, 628 (1.6) 58.7 / 58.8, 51, 874 (2.2)
+// 85.6 / 90.0; 4x2 padding 2, 1973, dropout (1) 158 / 122, causal 27, 629 (1.7) 48.1 / 43.4.  The bits are the same.
 static constexpr int kOwnDeltaSeq = 2048;    // longest sequence whose deltas a block keeps in LDS
 struct attn_bwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
         constexpr size_t dq_lds = attn_lds<HP, NPAN, W, G>(true, false), dkv_lds = attn_lds<HP, NPAN, W, G>(true, true);
         constexpr size_t own_at = dkv_lds > dq_lds ? dkv_lds : dq_lds;
         constexpr int waves = W * HP * G;
-        constexpr bool one_a_cu = waves == 4 && own_at > 80 * 1024;
+        constexpr unsigned round = waves == 4 && own_at > 80 * 1024 ? 256 : 256 * 8 / waves;
         const unsigned dkv = attn_grid(seq, W * 32, nbh * NPAN), dq = attn_grid(seq, W * 32, nbh);
-        const int64_t rows = (seq + W * 32 - 1) / (W * 32);
-        const bool room = one_a_cu ? dkv + dq <= (a.mask == BB_MASK_CAUSAL ? 576u : 320u) : nbh * rows * (NPAN + 1) <= 256 * 8 / waves;
+        const unsigned quarters = NPAN == 2 ? (a.mask == BB_MASK_CAUSAL ? 7 : 4) : (a.mask == BB_MASK_CAUSAL ? 9 : 5);
+        const bool room = dkv + dq <= round / 4 * quarters;
         if (seq > kOwnDeltaSeq || !room) {
             // the dQ kernel first: it also leaves delta = rowsum(dO o O) of its queries for the dK / dV kernel
             const int rc = attn_dq_launch::go<HP, NPAN, W, G>(seq, nbh, a, st);
@@ -1180,7 +1179,11 @@ struct attn_bwd_launch {
 //    96  6 x 8,    175, no mask    6.6                     6.2          11.0                    10.4
 //   128  2 x 8,   1024, no mask   18.5                    18.6          33.4                    34.2
 // Few blocks want their walks shared by groups, and small blocks, which also even out long and short walks under a causal mask; the
-// backward, whose waves look ahead by themselves, only where the walk is long, and it loses the launch that both passes share.
+// backward, whose waves look ahead by themselves, only where the walk is long, and it loses the launch that both passes share.  Of
+// 65 to 128 blocks (backward, share of the time of two waves in four groups that do not look ahead, by 4x1, 2x2, 2x4): causal, 224 to 447
+// keys 0.84 0.83 0.93, with dropout kept 0.73 0.63 0.69, 640 to 899 1.03 0.82 0.82 and 0.86 0.63 0.62, 1200 to 1535 1.21 0.94 0.92 and 0.94 0.69
+// 0.62, 1800 to 2048 1.31 0.93 0.84; padding, 224 to 447 0.81 0.82 0.91, 640 to 899 1.00 0.95 0.96 and with dropout 0.79 0.77 0.75, 1200 to 1535 1.07
+// 1.01 0.95, dropout made again 1.10 1.04 0.92, 1800 to 2048 1.38 1.03 0.95.
 // Heads of 128 find room for two groups: 4 heads, 1024 causal with dropout (32) 41.6 118.9 / 33.9 86.4.  Pairs of heads have twice the
 // waves: two a head in two groups (a walk of both heads by two waves in four groups / this: 1 x 4 pairs, 500 causal 9.6 16.4 / 8.3 15.3,
 // 2 x 4, 300, padding, dropout 9.6 20.7 / 7.8 17.0; four waves in two groups / four a head: 4 x 8, 512 causal 10.6 24.8 / 9.2 22.4); else
@@ -1207,7 +1210,10 @@ template <typename L, int HP, int NPAN> static int attn_shape(int seq, int nbh, 
         if (blocks <= 128 && seq <= 320) return L::template go<HP, NPAN, 2, 1>(seq, nbh, a, st);
     } else {
         if (masked && seq >= 1536 && blocks > 128 && blocks <= 400) return L::template go<HP, NPAN, 4, 2>(seq, nbh, a, st);
-        if (masked && seq >= 448 && blocks > 64 && blocks <= 128) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
+        if (masked && blocks > 64 && blocks <= 128) {
+            if (seq >= (a.drop.thresh ? 640 : 1200)) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
+            if (seq >= (a.mask == BB_MASK_CAUSAL ? 224 : 448)) return L::template go<HP, NPAN, 2, 2>(seq, nbh, a, st);
+        }
         if (masked && seq >= 320 && blocks <= 64) return L::template go<HP, NPAN, 2, 4>(seq, nbh, a, st);
         if (blocks <= 128 && seq <= 320) return L::template go<HP, NPAN, 2, 1>(seq, nbh, a, st);
     }

@@ -29,7 +29,7 @@ def test_walk_with_dropout(hiplib, mask, b, a, s, d):
 @pytest.mark.parametrize("b,a,s,d", [(1, 1, 1, 64), (2, 2, 33, 64), (2, 4, 67, 32), (1, 2, 128, 64), (1, 2, 161, 128), (1, 2, 515, 64), (2, 6, 200, 32),
                                      (2, 130, 200, 64), (2, 40, 461, 128), (1, 40, 530, 64),
                                      # walks shared by groups: 2x4 in one launch and in two, 2x2, 4x2; pairs of heads 2x2; 128-wide 4x2
-                                     (1, 2, 600, 64), (1, 2, 2100, 64), (2, 8, 520, 64), (1, 22, 450, 64), (1, 11, 1537, 64),
+                                     (1, 2, 600, 64), (1, 2, 2100, 64), (2, 8, 520, 64), (1, 22, 450, 64), (1, 9, 1210, 64), (1, 11, 1537, 64),
                                      (2, 16, 600, 32), (1, 2, 500, 128), (1, 30, 500, 128)])
 def test_kept_decisions(hiplib, mask, b, a, s, d):
     """The backward that reads the forward's decisions against the one that makes them again: the same bits; the forward does not
