@@ -13,14 +13,15 @@ SHAPES = [(1, 2, 160, 64), (2, 3, 193, 64),                             # 2x4, 2
           (1, 5, 321, 64),                                              # 2x4, 2x4 in one launch
           (1, 2, 2100, 64),                                             # 2x4, 2x4 in two
           (2, 8, 520, 64), (1, 22, 450, 64),                            # 2x4, 2x2 in one; with padding the second in two
-          (2, 17, 225, 64),                                             # 2x2, 2x2 if causal, else 2x1
+          (2, 17, 225, 64),                                             # 2x4, 2x2 if causal, else 2x1
           (1, 11, 641, 64), (1, 9, 1210, 64),                           # 2x4, 2x2 or with dropout 2x4, 2x4
           (1, 36, 448, 64), (1, 43, 577, 64),                           # 2x2, 4x1
           (1, 11, 1537, 64),                                            # 2x2, 4x2
           (1, 33, 1025, 64),                                            # 2x2 if causal, else 4x1, both backward 4x1
           (1, 4, 80, 32), (2, 60, 289, 32),                             # pairs of heads: 2x1
-          (2, 6, 257, 32), (2, 16, 600, 32),                            # 2x2, in one launch and in two
-          (1, 2, 448, 128), (2, 4, 521, 128), (1, 30, 500, 128)]        # 4x2, the last in two
+          (2, 6, 257, 32), (2, 16, 600, 32), (2, 16, 650, 32),          # 2x2, with padding the last in two launches
+          (1, 2, 448, 128), (2, 4, 521, 128), (1, 30, 500, 128),        # 4x2, with padding the last in two
+          (1, 38, 500, 128)]                                            # in two
 
 
 @pytest.mark.parametrize("mask", ["causal", "key_padding"])
