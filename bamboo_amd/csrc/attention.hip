@@ -1119,21 +1119,24 @@ struct attn_dkv_launch {
         return attn_go(kern, seq, W * 32, nbh * NPAN, W * HP * G * 64, attn_lds<HP, NPAN, W, G>(true, true), a, st);
     }
 };
-// Both backward kernels: in one launch where that ends within a round and a quarter of the blocks that the chip holds, with a causal mask two
-// and a quarter, for its short blocks fill in behind the long ones; else one after the other.  Each alone is bound by its longest walk
-// while at most half of the chip has work; together they take the longer of the two instead of the sum, and a launch less.  What it
-// costs is delta a second time, by every dK / dV block for the queries it will meet, and registers: beyond, both weigh more than
-// what overlaps, and at once where two launches of a whole round each become three rounds.  128-wide heads, which make scores and deltas
-// twice by then, end sooner.  A round is what waves and LDS let in: eight waves a CU, one block of eight or, where two
-// rings fill more than half of LDS (64-wide heads, two waves in two groups), of four.  Heads stay on their XCD, so that uneven ones leave
-// empty blocks in the grid, which go to no other XCD: they count (three heads are on three XCDs, 96 CUs).  One after the
-// other / together (us), by rounds: padding, 64-wide 2x4 7 heads, 1114 keys (1.1) 41.9 / 36.0, 5, 1268 (1.25) 38.2 / 34.3, 1, 1377 (1.4) 34.2 / 42.9,
-// 2, 1997 (2) 44.8 / 57.1; 2x2 16, 640 (1.25) 21.4 / 18.5, 5, 1682 (1.7) 41.3 / 51.3; 4x1 19, 1499 (1.1) 69.0 / 63.4, 46, 1116 (1.7) 53.2 / 50.8; 4x2 12, 1549 (1.6)
-// 56.2 / 63.9; pairs 2x2 2, 1066 (1.1) 31.6 / 26.5, 3, 1323 (1.3) 39.7 / 46.8; no mask, 4x1 25, 1070 (1.1) 65.2 / 56.8, 24, 1934 (1.5) 115.0 / 114.7; pairs 2x1
-// 46, 366 (1.1) 25.3 / 22.1; causal, 2x4 3, 1938 (1.9) 41.4 / 37.3; 2x2 16, 987 (2) 30.8 / 27.0, 9, 1153 (2.4) 32.6 / 33.2, 10, 1500 (3) 39.9 / 47.3; 4x1 28, 1897 (1.9)
-// 88.0 / 77.0; 4x2 16, 1575 (1.6) 54.1 / 42.3; pairs 2x2 12, 1112 (2.25) 35.1 / 33.1, 2x1 17, 1402, dropout (2.1) 90.6 / 78.8, 34, 919 (2.3) 42.5 / 43.8;
-// 128-wide 4x1 no mask 14, 1182 (0.9) 88.0 / 90.0, 20, 1055 (1.1) 88.3 / 106.4, padding 37, 420 (0.9) 43.9 / 37.6, causal 54, 628 (1.6) 58.7 / 58.8, 51, 874 (2.2)
-// 85.6 / 90.0; 4x2 padding 2, 1973, dropout (1) 158 / 122, causal 27, 629 (1.7) 48.1 / 43.4.  The bits are the same.
+// Both backward kernels go in one launch where their grids together are at most a round and a quarter of the blocks that the chip holds,
+// under a causal mask two and a quarter, for its short blocks fill in behind the long ones; 128-wide heads, which make scores twice, a
+// round and a round and three quarters.  Else one after the other.  Each alone is bound by its longest walk while at most half of the
+// chip has work; together they take the longer of the two instead of the sum, and a launch less.  What it costs is delta a second time,
+// by every dK / dV block for the queries it will meet, and registers: beyond these lines both weigh more than what overlaps.
+// A round is what waves and LDS let in: eight waves a CU; one block of four where two rings fill more than half of LDS (64-wide heads,
+// two waves in two groups).  Heads stay on their XCD, so uneven ones leave empty blocks in the grid, which go to no other XCD: they count
+// (three heads are on three XCDs, 96 CUs).  Rounds: one after the other / together, us (heads, keys; D: with dropout).  The bits are the same.
+//   padding   64-wide 2x4   1.1: 41.9 / 36.0 (7, 1114 D)   1.25: 38.2 / 34.3 (5, 1268 D)   1.4: 34.2 / 42.9 (1, 1377)   2: 44.8 / 57.1 (2, 1997)
+//             2x2   1.25: 21.4 / 18.5 (16, 640)   1.7: 41.3 / 51.3 (5, 1682)      4x2   1.6: 56.2 / 63.9 (12, 1549)
+//             4x1   1.1: 69.0 / 63.4 (19, 1499)   1.7: 53.2 / 50.8 (46, 1116)     pairs 2x2   1.1: 31.6 / 26.5 (2, 1066)   1.3: 39.7 / 46.8 (3, 1323)
+//   no mask   64-wide 4x1   1.1: 65.2 / 56.8 (25, 1070)   1.5: 115.0 / 114.7 (24, 1934)   pairs 2x1   1.1: 25.3 / 22.1 (46, 366)
+//   causal    64-wide 2x4   1.9: 41.4 / 37.3 (3, 1938)    4x1   1.9: 88.0 / 77.0 (28, 1897)    4x2   1.6: 54.1 / 42.3 (16, 1575)
+//             2x2   2: 30.8 / 27.0 (16, 987)   2.4: 32.6 / 33.2 (9, 1153)   3: 39.9 / 47.3 (10, 1500)
+//             pairs 2x2   2.25: 35.1 / 33.1 (12, 1112)   2x1   2.1: 90.6 / 78.8 (17, 1402 D)   2.3: 42.5 / 43.8 (34, 919)
+//   128-wide  4x1   no mask 0.9: 88.0 / 90.0 (14, 1182)   1.1: 88.3 / 106.4 (20, 1055)   padding 0.9: 43.9 / 37.6 (37, 420 D)
+//             4x1   causal 1.6: 58.7 / 58.8 (54, 628)   2.2: 85.6 / 90.0 (51, 874)
+//             4x2   padding 1: 158 / 122 (2, 1973 D)   causal 1.7: 48.1 / 43.4 (27, 629)
 static constexpr int kOwnDeltaSeq = 2048;    // longest sequence whose deltas a block keeps in LDS
 struct attn_bwd_launch {
     template <int HP, int NPAN, int W, int G> static int go(int seq, int nbh, const AttnArgs& a, hipStream_t st) {
