@@ -1,13 +1,14 @@
-// MFMA GEMM for gfx950: bf16 (v_mfma_f32_32x32x16_bf16) and fp32 (v_mfma_f32_32x32x2_f32),
+// MFMA GEMM for gfx950: bf16 (v_mfma_f32_16x16x32_bf16, v_mfma_f32_32x32x16_bf16) and fp32 (v_mfma_f32_32x32x2_f32),
 // LDS-tiled, double-buffered, batched with two-level strides, fused epilogues.
 //
 // Stands in for F.linear / torch.matmul and their autograd backward in the reference layer
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:121,127,136-146,158).
 //
-// bf16 data paths: tiles by DMA (gemm_bf16_dma_*); 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for weight
+// bf16 data paths: large tiles by DMA on 16x16x32 instructions (gemm_m16.h), others on 32x32x16 (gemm_bf16_dma_*); 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for weight
 // gradients of few tiles and few tiles of an odd contraction length; a register-staged kernel for rows of C that are no
 // whole vectors (N % 8 != 0, NT).  fp32: gemm_f32.h.
 #include "gemm_kernels.h"
+#include "gemm_m16.h"
 #include "gemm_f32.h"
 #include "gemm_wave.h"
 
@@ -43,19 +44,19 @@ static int launch_bf16_dma(GemmArgs& g, int batches, hipStream_t st) {
     return BB_OK;
 }
 
-// persistent kernels: one block per CU walks the tiles
-static constexpr int kPersistBlocks = 256;
-template <int BM, int BN, int WM, int WN, bool TB> static int launch_bf16_dma_persist(GemmArgs& g, hipStream_t st) {
-    constexpr int smem = 3 * (BM + BN) * 32 * 2 + WM * WN * 32 * 64 * 4;
-    auto kern = gemm_bf16_dma_persist_kernel<BM, BN, WM, WN, TB, false>;
-    if constexpr (!TB) {
-        if (g.drop.thresh) kern = gemm_bf16_dma_persist_kernel<BM, BN, WM, WN, TB, true>;
+// One block per CU walks the tiles; a contraction of fewer k-tiles than the ring has stages: a block per tile.
+static constexpr int kCUs = 256;
+template <int TM, int TN, int WM, int WN, int STAGES, bool TB> static int launch_bf16_m16(GemmArgs& g, int batches, hipStream_t st) {
+    constexpr int BM = WM * TM * 16, BN = WN * TN * 16, smem = STAGES * (BM + BN) * 128;
+    auto kern = gemm_bf16_m16_kernel<TM, TN, WM, WN, TB, STAGES, false>;
+    if constexpr (!TB) {       // dropout goes with forward (NT) products only: fill_args refuses the others
+        if (g.drop.thresh) kern = gemm_bf16_m16_kernel<TM, TN, WM, WN, TB, STAGES, true>;
     }
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    const int total = g.tiles_m * g.tiles_n;
-    bb_launch(kern, dim3(total < kPersistBlocks ? (total + 7) / 8 * 8 : kPersistBlocks), dim3(WM * WN * 64), smem, st, g);
+    const int total = g.tiles_m * g.tiles_n, blocks = g.K >= STAGES * 64 && total > kCUs ? kCUs : total;
+    bb_launch(kern, dim3(blocks, 1, batches), dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -115,16 +116,10 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     // Rules read off sweeps of M 2048..16384 x N 768..6400 x K 1024/4096 (NT and NN) on MI355X (256 CUs,
     // one block of the 256-row tiles per CU).
     //  - Operands whose rows are k-contiguous (both of NT, A of NN) load faster as 64-wide k-tiles: one
-    //    DMA instruction then covers 8 whole 128-byte lines instead of 16 half lines.  The smaller the
-    //    tile, the more of its time is loading and the more that buys (128x128: up to +19 %, 256x128:
-    //    +3..8 %, 256x256: +4 % at long K, and +2 % on the whole stage with the K = 1024 FFN product on it).
-    //  - Above one round of 256x256 tiles they win while the last round is well filled; otherwise the
-    //    small tiles, several blocks per CU, smooth the tail.  Where the sweep (outputs that stay in the
-    //    last-level cache) and the stage itself (outputs that go to HBM) disagree, the stage decides: it
-    //    wants the 256x256 tile from a 70 % full last round on for NT, and three stages for every 256x128
-    //    problem.
-    //  - Within one round: 256x256 once 256x128 tiles would need a second round, 256x128 from about half
-    //    a round on, and 128x128 tiles for anything smaller.
+    //    DMA instruction then covers 8 whole 128-byte lines instead of 16 half lines (128x128 tiles: up to +19 %).
+    //  - 32-wide k-tiles (K % 64 != 0): above one round of 256x256 tiles they win while the last round is well filled; otherwise
+    //    the small tiles, several blocks per CU, smooth the tail.  Within one round: 256x256 once 256x128 tiles would need a
+    //    second round, 256x128 from about half a round on, and 128x128 tiles for anything smaller.
     const bool nt = layout == BB_NT, nn = layout == BB_NN;
     const bool k64 = (nt || nn) && K % 64 == 0 && K >= 128;
     const DmaTile small = k64 && (nt || K >= 2048) ? D128x128k64 : D128x128s3;
@@ -161,57 +156,58 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
         if ((K <= 512 || t128 <= 128) && nt) return D128x64s3;
         if (t128 <= 128 && nn) return D64x128s3;
     }
-    //  - NT problems whose 256x256 tiles would fill under 70 % of their rounds may take 256x192 tiles (six
-    //    accumulator tiles per wave, about 9 % below the 256x256 tile at equal fill) instead of falling back
-    //    to 128x128: compared by the share of the occupied tile slots that is real output.  (Alone, the QKV
-    //    projection 8192x3072 - 1.5 rounds of 256x256 tiles, exactly two of 256x192 - is 19 % faster on them;
-    //    inside the stage the whole batch is 1 % slower, so 75 % full rounds stay on 256x256.)
-    if (nt && k64 && big_ok && t2128 > 256) {
-        auto useful = [&](int bn) {   // real output / output slots of whole rounds
-            const int64_t t = (int64_t)((M + 255) / 256) * ((N + bn - 1) / bn) * batches;
-            return (double)M * N * batches / ((double)((t + 255) / 256 * 256) * 256 * bn);
-        };
-        const double s256 = useful(256), s192 = 0.91 * useful(192);
-        if (s256 < 0.70 && s192 > s256 && s192 >= 0.65) return D256x192k64;
+    //  - Larger ones, whole 64-wide k-tiles: the tile of gemm_m16.h whose rounds take least, a round (one tile a CU) of kt k-tiles being
+    //    kt times a step, plus what a tile costs around its loop (prologue, epilogue, the stores of all CUs at once).  Steps and rest as fitted
+    //    to the table; the two of 256x256 are 1500 TFLOP/s, at the card's power.  Before (32x32x16 instructions, several kernels and rules) / 256x256 /
+    //    256x192 / 256x128 (us, plain, the one taken marked):
+    //        NT 8192x3072x1024 66 / 58 / 50* / 48    8192x4096x1024 78 / 63* / 66 / 66    8192x1024x4096 66 / 80 / 69 / 58*
+    //           8192x1024x1024 24 / 29 / 25 / 22*    4096x4800x1600 73 / 73 / 60* / 62    4096x6400x1600, activation 97 / 85* / 101 / 97
+    //           4096x1600x6400 86 / 117 / 97 / 76*
+    //        NN 8192x4096x1024 77 / 62* / 67 / 67    8192x1024x4096 65 / 77 / 69 / 57*    8192x1024x3072 50 / 61 / 54 / 45*
+    //           4096x1600x4800 67 / 87 / 76 / 59*    4096x6400x1600, times a tensor 95 / 81* / 99 / 97
+    if (k64 && big_ok) {
+        static const struct {
+            DmaTile tile;
+            int bn;
+            double step, rest;
+        } tiles[] = {{D256x256k64, 256, 1.36, 8.2}, {D256x192k64, 192, 1.05, 5.9}, {D256x128k64s3, 128, 0.755, 4.2}};
+        DmaTile best = D_NONE;
+        double least = 0.0;
+        for (const auto& t : tiles) {
+            const int64_t n = (int64_t)((M + 255) / 256) * ((N + t.bn - 1) / t.bn) * batches;
+            const double us = (double)((n + 255) / 256) * (K / 64 * t.step + t.rest);
+            if (best == D_NONE || us < least) best = t.tile, least = us;
+        }
+        return best;
     }
     if (t256 > 256) {
         const int64_t slots = (t256 + 255) / 256 * 256;
-        const bool full85 = t256 * 100 >= slots * 85, full70 = t256 * 10 >= slots * 7;
+        const bool full70 = t256 * 10 >= slots * 7;
         if (!big_ok) return small;
-        if (k64 && nt) {
-            // a last round under 85 %: 256x128 tiles if those come out in whole rounds (the QKV projection
-            // 8192x3072: 1.5 rounds of 256x256, exactly three of 256x128; +1 % on the stage)
-            const int64_t slots2 = (t2128 + 255) / 256 * 256;
-            if (full85) return D256x256k64;
-            if (t2128 * 10 >= slots2 * 9) return mid;
-            return full70 ? D256x256k64 : small;
-        }
-        // NN: below 85 % the tiles whose rounds are better filled (256x256 one, 128x128 three a CU; full, they are equal), 128x128 /
-        // 256x256 (us): 4096x6400x1600 (78 % of two rounds, 69 % of three) 103 / 89, 6656x4096x1024 76 / 71, x512 48 / 47,
-        // 6144x4096x1024 (75 %, 100 % of two) 65 / 69
-        if (k64) {
-            const int64_t slots3 = (t128 + 767) / 768 * 768;
-            return full85 || (full70 && (K >= 2048 || t256 * slots3 > t128 * slots)) ? D256x256w8db : small;
-        }
         return full70 || K >= 1536 ? D256x256w8db : small;
     }
-    if (big_ok && t2128 > 256) return k64 && nt ? D256x256k64 : D256x256w8db;
+    if (big_ok && t2128 > 256) return D256x256w8db;
     if (M >= 256 && t2128 > 136) return mid;
     return small;
 }
 
-// The tile of a (shape, layout, epilogue kind): NT / NN problems of more than one round of 256x256 tiles take the
-// persistent kernel (blocks walk their tiles with the DMA ring running through the tile boundaries) unless the epilogue
-// evaluates the activation: that work keeps the vector ALUs busy for about as long as the tile's matrix work does, the
-// boundary is not what such a launch waits for (FFN1 with act + act': 114 us on the plain kernel, 118 persistent;
-// the plain product 95 against 77).  All kernels add up a contraction in the same order: which one runs changes no bit.
-static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, int epilogue) {
+// ... of a problem with an fp32 output: of the tiles of gemm_m16.h, 256x128 has the registers for it.  More than one 256x256 tile a CU goes
+// by a name of its own (the blocks then walk their tiles; so do those of the other two).  All kernels add up a contraction in the same
+// order: which one runs changes no bit.
+static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, bool c_f32) {
     const DmaTile t = pick_dma_tile(M, N, K, batches, layout);
-    const bool light = epilogue != BB_EPI_ACT && epilogue != BB_EPI_ACT_DACT && epilogue != BB_EPI_DACT;
-    const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-    if ((t == D256x256k64 || t == D256x256w8db) && light && batches == 1 && layout != BB_TN && K % 64 == 0 && t256 > kPersistBlocks)
-        return D256x256p;
-    return t;
+    if (c_f32 && (t == D256x256k64 || t == D256x192k64)) return D256x128k64s3;
+    return t == D256x256k64 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches > kCUs ? D256x256p : t;
+}
+
+// The kernels that leave column statistics (128x64, 64x128 or 256x128 tiles) take the largest within a round of them and, forward, where its
+// rounds are filled and those of 256x256 tiles are not.
+static bool stats_256x128(DmaTile t, int M, int N, int layout) {
+    if (t != D256x256k64 && t != D256x192k64 && t != D256x128k64s3) return false;
+    const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256), t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128);
+    if (t2128 <= 256) return t2128 > 136;
+    const int64_t slots = (t256 + 255) / 256 * 256, slots2 = (t2128 + 255) / 256 * 256;
+    return layout == BB_NT && t256 > 256 && t256 * 100 < slots * 85 && t2128 * 10 >= slots2 * 9;
 }
 
 // NT and NN kernels reach a tile's rows by 32-bit offsets (DmaLanes); operands whose rows lie further apart take the kernel with
@@ -253,7 +249,7 @@ static bool halve_tiles(int M, int N, int64_t batches) { return (int64_t)((M + 3
 
 template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     const int layout = TA ? BB_TN : TB ? BB_NN : BB_NT;
-    const DmaTile dma = narrow_or_wide(pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.epilogue), layout, g.lda, g.ldb);
+    const DmaTile dma = narrow_or_wide(pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.c_f32 != 0), layout, g.lda, g.ldb);
     switch (pick_wave(g.M, g.N, g.K, batches, layout, dma)) {
         case W_8: return launch_bf16_wave<TA, TB, 8, 32, 2>(g, batches, st);
         case W_4: return launch_bf16_wave<TA, TB, 4, 64, 1>(g, batches, st);
@@ -263,8 +259,16 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D256x256w8db: return launch_bf16_dma<256, 256, 2, 4, TA, TB, true>(g, batches, st);
         case D256x128w8db: return launch_bf16_dma<256, 128, 4, 2, TA, TB, true>(g, batches, st);
         case D128x128s3: return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
-        case D256x256k64: return launch_bf16_dma<256, 256, 2, 4, TA, TB, true, 2, 64>(g, batches, st);
-        case D256x128k64s3: return launch_bf16_dma<256, 128, 4, 2, TA, TB, true, 3, 64>(g, batches, st);
+        case D256x256k64:
+        case D256x256p:
+            if constexpr (!TA) return launch_bf16_m16<8, 4, 2, 4, 2, TB>(g, batches, st);
+            else break;
+        case D256x192k64:
+            if constexpr (!TA) return launch_bf16_m16<4, 6, 4, 2, 2, TB>(g, batches, st);
+            else break;
+        case D256x128k64s3:
+            if constexpr (!TA) return launch_bf16_m16<4, 4, 4, 2, 3, TB>(g, batches, st);
+            else break;
         case D128x128k64: return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64>(g, batches, st);
         case D128x128k64r:
             if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64, true>(g, batches, st);
@@ -280,13 +284,6 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
             if constexpr (!TA)
                 return halve_tiles(g.M, g.N, batches) ? launch_bf16_dma<32, 64, 1, 2, TA, TB, true, 4, 64>(g, batches, st)
                                                       : launch_bf16_dma<64, 64, 2, 2, TA, TB, true, 4, 64>(g, batches, st);
-            else break;
-        case D256x256p:
-            if constexpr (!TA) return launch_bf16_dma_persist<256, 256, 2, 4, TB>(g, st);
-            else break;
-        case D256x192k64:
-            // k-contiguous operands only (192 rows do not divide into the k-major loader's instructions)
-            if constexpr (!TA && !TB) return launch_bf16_dma<256, 192, 4, 2, TA, TB, true, 2, 64>(g, batches, st);
             else break;
         default: break;
     }
@@ -366,7 +363,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
     BB_REQUIRE(d->layout >= BB_NT && d->layout <= BB_TN, "bb_gemm_variant: bad layout %d", d->layout);
     const int64_t batches = (int64_t)(d->nb1 > 0 ? d->nb1 : 1) * (d->nb2 > 0 ? d->nb2 : 1);
     if (d->dtype == BB_BF16) {
-        const DmaTile dt = narrow_or_wide(pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->epilogue), d->layout, d->lda, d->ldb);
+        const DmaTile dt = narrow_or_wide(pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->c_dtype == BB_F32), d->layout, d->lda, d->ldb);
         const WaveMode wm = pick_wave(d->M, d->N, d->K, batches, d->layout, dt);
         if (wm != W_NONE) snprintf(out, out_len, "bf16_%s_wave64x64k%d", layouts[d->layout], wm == W_8 ? 8 : 4);
         else snprintf(out, out_len, "bf16_%s_%s%s", layouts[d->layout], dt == D64x64k64s4 && halve_tiles(d->M, d->N, batches) ? "halves_" : "",
@@ -491,11 +488,10 @@ extern "C" int bb_gemm_bn_bwd(const bb_gemm_desc* d, const bb_bn_bwd_stats* bn, 
     rc = fill_args(d, g, batches, ta, tb);
     if (rc) return rc;
     const BnBwdArgs b = {bn->x, bn->mean, bn->rstd, bn->strips};
-    // the tile the plain product of this shape would take, where it is one of those built with the sums
     const DmaTile dma = narrow_or_wide(pick_dma_tile(d->M, d->N, d->K, 1, BB_NN), BB_NN, g.lda, g.ldb);
     if (dma == D128x128k64r) return launch_bf16_dma_bnbwd<64, 128, 2, 2, 3, true>(g, b, (hipStream_t)stream);
     if (dma == D64x64k64s4) return launch_bf16_dma_bnbwd<64, 64, 2, 2, 4>(g, b, (hipStream_t)stream);
-    if (dma == D256x128k64s3) return launch_bf16_dma_bnbwd<256, 128, 4, 2>(g, b, (hipStream_t)stream);
+    if (stats_256x128(dma, g.M, g.N, BB_NN)) return launch_bf16_dma_bnbwd<256, 128, 4, 2>(g, b, (hipStream_t)stream);
     return launch_bf16_dma_bnbwd<64, 128, 2, 2>(g, b, (hipStream_t)stream);
 }
 
@@ -511,11 +507,10 @@ extern "C" int bb_gemm(const bb_gemm_desc* d, void* stream) {
         int rc = fill_args(d, g, batches, ta, tb);
         if (rc) return rc;
         g.strip_stats = d->strip_stats;
-        // the tiles that carry the statistics: 64x64 and 256x128 where the ordinary choice would be that tile, else 128x64
         const DmaTile dma = narrow_or_wide(pick_dma_tile(d->M, d->N, d->K, 1, BB_NT), BB_NT, g.lda, g.ldb);
         if (dma == D128x128k64r) return launch_bf16_dma_stats<128, 64, 4, 1, 3, true>(g, (hipStream_t)stream);
         if (dma == D64x64k64s4) return launch_bf16_dma_stats<64, 64, 2, 2, 4>(g, (hipStream_t)stream);
-        if (dma == D256x128k64s3) return launch_bf16_dma_stats<256, 128, 4, 2>(g, (hipStream_t)stream);
+        if (stats_256x128(dma, g.M, g.N, BB_NT)) return launch_bf16_dma_stats<256, 128, 4, 2>(g, (hipStream_t)stream);
         return launch_bf16_dma_stats<128, 64, 4, 1>(g, (hipStream_t)stream);
     }
     GemmArgs g;

@@ -821,7 +821,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // Transposed products (B times A) where the epilogue takes the accumulators as they are: a lane then has a row of C, four
     // neighbouring columns in four registers.  The kernels with column statistics keep a column per lane.
     constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS;
-    constexpr bool DIRECT = STATS == 0 && (AHEAD || (BM == 256 && BN == 128 && PLAIN && BK == 64));
+    constexpr bool DIRECT = STATS == 0 && AHEAD;
     auto mfma = [](const bf16x8& a, const bf16x8& b, const f32x16& c) {
         return DIRECT ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     };
@@ -956,7 +956,6 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // transfers where the registers are there, else at the loop's end, the first tile's operand under the last k-tile.
     constexpr int TILES = TM * TN;
     constexpr bool BEFORE = DIRECT && AHEAD && TILES <= 2;
-    constexpr bool UNDER = DIRECT && BM == 256;
     const int drow = m0 + wm * WTM + (lane & 31), dcol = n0 + wn * WTN + 8 * (lane >> 5);
     u32x4 dop[DIRECT ? TILES : 1][2], dbias[DIRECT ? TN : 1][2];
     auto fetch_bias = [&]() {
@@ -993,7 +992,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // of one; the three operand reads per row of the BatchNorm backward sums are most of their epilogue).
     // EARLY: the kernels whose waves finish one patch each and have the registers fetch it -- and the bias -- before the main loop.
     constexpr bool EARLY = AHEAD && TM * NP == 1 && !DIRECT;
-    constexpr bool PREF = BM * BN >= 256 * 128 && !VIS && CONV == 0 && STATS == 0 && !DIRECT;
+    constexpr bool PREF = BM * BN >= 256 * 128 && !VIS && CONV == 0 && STATS == 0;
     constexpr bool HOIST = STATS == 2;
     const bf16* opnd = PREF || HOIST ? epilogue_operand(g) : nullptr;
     u32x4 opc[PREF || HOIST ? 4 : 1], opn[PREF ? 4 : 1];
@@ -1057,8 +1056,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         // 1024x512x2048 11.7 / 9.5, 512x1024x4096 20.0 / 15.7, 100x1600x6400 29.1 / 21.3, 0.25 -> 0.17 us a k-tile, where LDS moves
         // 32 KB of fragments and 16 KB of transfers; 128x64 and 64x128 gain by the epilogue's early operands: 2043x768x768 with a
         // residual 8.6 / 7.8, x3072 21.2 / 20.2 (NT), 21.0 / 19.4 (NN).  128x128 tiles, one a CU with three stages: the loop below with
-        // two blocks a CU 26.2, this one 21.1 (NT 8192x512x2048).  256x128 tiles are 2 to 6 % faster on it alone and no faster in a
-        // stage, where the matrix cores' clock gives way: they keep the loop below.
+        // two blocks a CU 26.2, this one 21.1 (NT 8192x512x2048).
         struct Tile {
             bf16x8 a[4][TM], b[4][TN];
         } t0, t1;
@@ -1162,12 +1160,6 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
             rs = rs + 1 == STAGES ? 0 : rs + 1;
             const unsigned char* nxt = smem + rs * STAGE_BYTES;
             if constexpr (STAGES >= 3) {
-                if constexpr (PREF) {
-                    if (kt == KT - 1) fetch(std::integral_constant<int, 0>{}, opc);
-                }
-                if constexpr (UNDER) {
-                    if (kt == KT - 1) fetch_operand(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-                }
                 // the DMA instructions of tile kt+STAGES-1 a third each between the MFMAs of the first three quarters
                 // (issued in one burst at the top they queue up in front of the texture path and the waves behind
                 // them: 2-5 % slower), the second half's fragment reads between the first MFMAs
@@ -1287,14 +1279,10 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         // tiles.  (Before, every wave parked pairs of tiles in LDS and read them back by rows of eight lanes, with the branches in every
         // one of four passes: about 2600 cycles for the single 32x32 tile a wave has in the 64x64 kernels, a third of what a
         // product of two k-tiles takes there.)  Back to back with the shorter way to the first transfer, before / now (us): NT
-        // 128x128x128 4.1 / 3.2, 1050x512x512 5.4 / 4.4, 1050x512x2048 9.6 / 8.3; 128x64 tiles 1024x1536x512 7.4 / 6.4; 256x128
-        // tiles 2043x2304x768 15.6 / 13.6, 8192x3072x1024 63.5 / 60.5, NN 8192x1024x1024 23.3 / 21.6; with an operand to multiply by or
-        // two outputs 20.4 / 20.4 and 22.4 / 22.5 (2043x3072x768).  256x256 tiles keep LDS: stores of 32 bytes a row fill a line in
-        // four instructions, and with two outputs and GELU between them 8192x4096x1024 takes 99 us instead of 89 (130 when each
-        // piece is stored as it is made).
+        // 128x128x128 4.1 / 3.2, 1050x512x512 5.4 / 4.4, 1050x512x2048 9.6 / 8.3; 128x64 tiles 1024x1536x512 7.4 / 6.4.
         if constexpr (!BEFORE) {
             fetch_bias();
-            fetch_operand(std::integral_constant<int, UNDER ? 1 : 0>{}, std::integral_constant<int, UNDER ? TILES - 1 : TILES>{});   // (tile 0's is on its way)
+            fetch_operand(std::integral_constant<int, 0>{}, std::integral_constant<int, TILES>{});
         }
         wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before the block's LDS is another's
         // accumulators of columns 16 h .. 16 h + 15 of a tile -> the lane's eight
@@ -1375,7 +1363,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
     // 128-byte row segments (256 bytes for fp32 outputs).
     // An odd tile count per row ends with a single tile: its 32 columns use half of the patch and half of
     // the lanes of the row pass.
-    if constexpr (PREF && !(BK == 64 && STAGES >= 3)) fetch(std::integral_constant<int, 0>{}, opc);
+    if constexpr (PREF) fetch(std::integral_constant<int, 0>{}, opc);
     wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before their stages become the patch
     __syncthreads();
     float* patch = (float*)smem + wave * (32 * PLD);
@@ -1497,225 +1485,6 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_stats_kernel(const 
 template <int BM, int BN, int WM, int WN, int STAGES, bool WIDE>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_bnbwd_kernel(const GemmArgs g, const BnBwdArgs bn) {
     gemm_bf16_dma_body<BM, BN, WM, WN, false, true, true, STAGES, 64, false, 0, 2, false, WIDE>(g, blockIdx.x, 0, false, ConvArgs{}, bn);
-}
-
-// Persistent variant for problems of more than one round of 256x256 tiles (NT and NN, 32-wide k-tiles, three stages,
-// eight waves): a block walks the output tiles b, b + gridDim, ... and treats their k-tiles as ONE stream, so the DMA
-// ring never drains - while the last k-tiles of a tile are multiplied, the first ones of the block's next tile are
-// already landing, and the epilogue's stores go out behind them.  What a tile boundary costs a block of the plain
-// kernel (retiring, the next block's launch, its pipeline prologue) is gone: 95 -> 77 us on the plain product
-// 8192 x 4096 x 1024.  The waits of the first k-tiles after a boundary count the epilogue's stores in (completion is in
-// order): exact counts that spare them changed nothing, the stores are acknowledged quickly.  The epilogue patch
-// cannot share the ring's LDS any more (the ring is live during the epilogue): it has 64 KB of its own behind the
-// three stages, [32][64] floats per wave with the 16-byte chunks of a row swizzled by the row instead of padded.
-// Results are bit-equal to the plain kernels' (same k order, same epilogue function).  Needs K % 64 == 0 (the two
-// fragment sets alternate, a tile takes an even number of k-tiles), unbatched operands, a grid that is a multiple of 8
-// (the tile order's XCD mapping).  Instantiated for 256x256 tiles only: 256x128 tiles on this loop load their 32-wide
-// k-tiles as half lines and lose more than the boundaries give (90 against 71 us on 8192 x 3072 x 1024).
-template <int BM, int BN, int WM, int WN, bool BKM, bool DROP>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_persist_kernel(const GemmArgs g) {
-    constexpr int NW = WM * WN, BK = 32, STAGES = 3;
-    constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
-    static_assert(TN == 2 && TM * TN > 2, "the epilogue patch holds two accumulator tiles side by side");
-    using OpA = DmaOperand<BM, false, NW, BK>;
-    using OpB = DmaOperand<BN, BKM, NW, BK>;
-    constexpr int STAGE_BYTES = OpA::BYTES + OpB::BYTES;
-    constexpr int LOADS = OpA::ROUNDS + OpB::ROUNDS;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WN, wn = wave % WN;
-    const int total = g.tiles_m * g.tiles_n, G = gridDim.x;
-    const bf16* A = (const bf16*)g.A;
-    const bf16* B = (const bf16*)g.B;
-    const int KT = g.K / BK;
-
-    OpA opa;
-    OpB opb;
-    FragReader<BM, TM, false, BK> fa;
-    FragReader<BN, TN, BKM, BK> fb;
-    fa.init(wm * WTM, lane);
-    fb.init(wn * WTN, lane);
-    struct Frags {
-        bf16x8 a[2][TM], b[2][TN];
-    };
-    Frags f0, f1;
-    f32x16 acc[TM][TN];
-
-    // the stream: ki = index of the next k-tile to issue inside output tile issue_tile
-    int issue_stage = 0, read_stage = 0, ki = 0, issue_tile = blockIdx.x;
-    auto point_at = [&](int t) {
-        int tm, tn;
-        tile_coords(t, g.tiles_m, g.tiles_n, tm, tn);
-        opa.init(A, g.lda, tm * BM, g.M, tid);
-        opb.init(B, g.ldb, tn * BN, g.N, tid);
-    };
-    point_at(issue_tile);
-    // before a k-tile is issued: move on to the block's next output tile, or (no tile left) stay on the last k-tile,
-    // which is then fetched again and again into stages nobody reads
-    auto prep_issue = [&]() {
-        if (ki == KT) {
-            if (issue_tile + G < total) {
-                issue_tile += G;
-                ki = 0;
-                point_at(issue_tile);
-            } else {
-                ki = KT - 1;
-            }
-        }
-        if (ki == KT - 1 && issue_tile + G >= total) {
-            opa.stop();
-            opb.stop();
-        }
-    };
-    // MFMA m of step ks, then its share of ND DMA instructions into `dst` and of the fragment reads of `src` into
-    // nf, each group fenced (see gemm_bf16_dma_body)
-    auto placed_step = [&](const Frags& f, auto ks_c, auto nd_c, unsigned char* dst, auto reads_c, Frags& nf,
-                           const unsigned char* src) {
-        constexpr int ks = decltype(ks_c)::value, ND = decltype(nd_c)::value;
-        constexpr bool READS = decltype(reads_c)::value;
-        constexpr int NM = TM * TN, NF = 2 * (TM + TN), FM = NM - 2;
-        static_for(
-            [&](auto idx) {
-                constexpr int m = decltype(idx)::value, i = m / TN, j = m % TN;
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[ks][i], f.b[ks][j], acc[i][j], 0, 0, 0);
-                static_for(
-                    [&](auto d) {
-                        constexpr int k = (ND * m) / NM + decltype(d)::value;
-                        if constexpr (k < OpA::ROUNDS) opa.template issue_one<k>(dst, wave);
-                        else opb.template issue_one<k - OpA::ROUNDS>(dst + OpA::BYTES, wave);
-                    },
-                    std::make_integer_sequence<int, (ND * (m + 1)) / NM - (ND * m) / NM>{});
-                if constexpr (READS && m < FM) {
-                    static_for(
-                        [&](auto r) {
-                            constexpr int q = (NF * m) / FM + decltype(r)::value, fk = q / (TM + TN), t = q % (TM + TN);
-                            if constexpr (t < TM) nf.a[fk][t] = fa.load(src, t, fk);
-                            else nf.b[fk][t - TM] = fb.load(src + OpA::BYTES, t - TM, fk);
-                        },
-                        std::make_integer_sequence<int, (NF * (m + 1)) / FM - (NF * m) / FM>{});
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            },
-            std::make_integer_sequence<int, NM>{});
-    };
-    // one k-tile: first half with the DMA instructions of the stream's k-tile two ahead, the wait for the k-tile
-    // one ahead (in-order completion: whatever the epilogue stored before is acknowledged by then too), second half
-    // with that k-tile's fragment reads
-    auto body = [&](Frags& cur, Frags& nxt, auto reads_c) {
-        prep_issue();
-        unsigned char* dst = smem + issue_stage * STAGE_BYTES;
-        issue_stage = issue_stage + 1 == STAGES ? 0 : issue_stage + 1;
-        placed_step(cur, std::integral_constant<int, 0>{}, std::integral_constant<int, LOADS>{}, dst, std::false_type{}, nxt, smem);
-        ++ki;
-        asm volatile("" ::: "memory");
-        wait_vmcnt_lgkm0<(STAGES - 2) * LOADS>();
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const unsigned char* st = smem + read_stage * STAGE_BYTES;
-        read_stage = read_stage + 1 == STAGES ? 0 : read_stage + 1;
-        placed_step(cur, std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, dst, reads_c, nxt, st);
-    };
-    auto load_frags = [&](Frags& f, const unsigned char* st) {
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) f.a[ks][i] = fa.load(st, i, ks);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) f.b[ks][j] = fb.load(st + OpA::BYTES, j, ks);
-        }
-    };
-
-    // prologue of the stream
-#pragma unroll
-    for (int t = 0; t < STAGES - 1; ++t) {
-        prep_issue();
-        unsigned char* st = smem + issue_stage * STAGE_BYTES;
-        opa.issue(st, wave);
-        opb.issue(st + OpA::BYTES, wave);
-        issue_stage = issue_stage + 1 == STAGES ? 0 : issue_stage + 1;
-        ++ki;
-    }
-    asm volatile("" ::: "memory");
-    wait_vmcnt_lgkm0<(STAGES - 2) * LOADS>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-
-    float* patch = (float*)(smem + STAGES * STAGE_BYTES) + wave * (32 * 64);
-    const int prow = lane >> 3, pchunk = lane & 7;
-    // the two 16-byte chunks of a lane's eight columns, read in an order that keeps the eight lanes of a row on
-    // eight different bank groups: lanes 0..3 of the row take their even chunk first, lanes 4..7 their odd one
-    const int first_chunk = 2 * pchunk + (pchunk >> 2), second_chunk = 2 * pchunk + 1 - (pchunk >> 2);
-    for (int tile = blockIdx.x; tile < total; tile += G) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-        // the tile's first fragments (the k-tile landed and was made visible by the last barrier before this point);
-        // a tile's last k-tile does not fetch the next tile's, so that no fragment registers live through the epilogue
-        load_frags(f0, smem + read_stage * STAGE_BYTES);
-        read_stage = read_stage + 1 == STAGES ? 0 : read_stage + 1;
-        for (int kt = 0; kt + 2 < KT; kt += 2) {
-            body(f0, f1, std::true_type{});
-            body(f1, f0, std::true_type{});
-        }
-        body(f0, f1, std::true_type{});
-        body(f1, f0, std::false_type{});
-        read_stage = read_stage == 0 ? STAGES - 1 : read_stage - 1;   // that k-tile is still to be read
-        int tm, tn;
-        tile_coords(tile, g.tiles_m, g.tiles_n, tm, tn);
-        const int m0 = tm * BM + wm * WTM, n = tn * BN + wn * WTN + pchunk * 8;
-        // the bias of the lane's eight columns once per tile; row offsets by addition (see gemm_bf16_dma_body)
-        float b8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (g.bias && n < g.N) load_vec((const bf16*)g.bias + n, b8);
-        int64_t ci = (int64_t)(m0 + prow) * g.ldc + n, xi = (int64_t)(m0 + prow) * g.ldaux + n;
-        // the operand of the epilogue kinds that read one, fetched a patch ahead of its use (inside the epilogue only:
-        // the main loop has no register to spare for it)
-        const bf16* opnd = epilogue_operand(g);
-        u32x4 opc[4], opn[4];
-        auto fetch = [&](int i, u32x4 (&dst)[4]) {
-#pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int m = m0 + i * 32 + it * 8 + prow;
-                dst[it] = u32x4{0u, 0u, 0u, 0u};
-                if (opnd && m < g.M && n < g.N) dst[it] = *(const u32x4*)(opnd + (int64_t)m * g.ldaux + n);
-            }
-        };
-        fetch(0, opc);
-        // (static_for: a loop the compiler declines to unroll would index the accumulators dynamically, i.e. from scratch)
-        static_for(
-            [&](auto idx) {
-                constexpr int i = decltype(idx)::value;
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), col = h * 32 + (lane & 31);
-                        patch[row * 64 + ((((col >> 2) ^ (row & 15)) << 2) | (col & 3))] = acc[i][h][r] * g.alpha;
-                    }
-                asm volatile("" ::: "memory");
-                if constexpr (i + 1 < TM) fetch(i + 1, opn);
-                static_for(
-                    [&](auto it_c) {
-                    constexpr int it = decltype(it_c)::value;
-                    const int row = it * 8 + prow, m = m0 + i * 32 + row;
-                    const f32x4 c1 = *(const f32x4*)(patch + row * 64 + ((first_chunk ^ (row & 15)) << 2));
-                    const f32x4 c2 = *(const f32x4*)(patch + row * 64 + ((second_chunk ^ (row & 15)) << 2));
-                    const f32x4 lo = pchunk < 4 ? c1 : c2, hi = pchunk < 4 ? c2 : c1;
-                    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    if (m < g.M && n < g.N) epilogue_vec8_at<DROP, true>(g, ci, xi, m, n, v, b8, opc[it]);
-                    ci += 8 * (int64_t)g.ldc;
-                    xi += 8 * (int64_t)g.ldaux;
-                    },
-                    std::make_integer_sequence<int, 4>{});
-                asm volatile("" ::: "memory");
-#pragma unroll
-                for (int it = 0; it < 4; ++it) opc[it] = opn[it];
-            },
-            std::make_integer_sequence<int, TM>{});
-    }
-    wait_vmcnt_lgkm0<0>();   // the k-tiles issued past the end of the stream land before the block leaves
 }
 
 // 3x3 convolution as an implicit GEMM: forward (BKM = false: y = patches(x) W^T) and input gradient

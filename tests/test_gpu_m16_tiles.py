@@ -1,0 +1,64 @@
+"""Products on tiles of 16x16x32 matrix instructions: one and several tiles a block, contractions of fewer, as many and more k-tiles than the
+ring has stages, rows and columns off the tile, batches, fp32 outputs -- against fp64, and bit for bit against the same rows in a product of other tiles."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rand(*shape, seed, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
+
+
+# sums of K products in fp32, in any order: K eps sum |a b|; half an ulp of bf16 (at most 2^-8 of the value) where the result is rounded
+def product(a, b):
+    a, b = a.double(), b.double().contiguous()
+    return a @ b, a.shape[1] * 2.0 ** -24 * (a.abs() @ b.abs())
+
+
+# 256x256: more than one tile a block, 8 rows and 8 columns in the last ones, an odd number of k-tiles; 256x192: 8 columns in the last;
+# 256x128: within a round, and several tiles a block with two k-tiles (fewer than its three stages), three and four
+@pytest.mark.parametrize("tile,M,N,K", [("256x256p", 7176, 4104, 448), ("256x256p", 7176, 4104, 128), ("256x192k64", 8200, 2696, 448),
+                                        ("256x192k64", 8192, 3072, 1024), ("256x128k64s3", 4100, 1032, 704), ("256x128k64s3", 33000, 264, 128),
+                                        ("256x128k64s3", 33000, 264, 192), ("256x128k64s3", 33000, 264, 256)])
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+def test_tiles(hiplib, layout, tile, M, N, K):
+    lay = hiplib.NT if layout == "nt" else hiplib.NN
+    A, B = rand(M, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2, scale=0.2)
+    bias, X = rand(N, seed=3), rand(M, N, seed=4)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    C, D = wide[:M, :N], torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    if layout == "nn" or K >= 256:       # (shorter forward products take 128x64 tiles)
+        assert hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C)).endswith(tile)
+    hiplib.gemm(lay, A, B, C)
+    ref, slack = product(A, B.t() if layout == "nt" else B)
+    assert ((C.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + slack).all()
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
+    kinds = [dict(), dict(bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X), dict(epilogue=hiplib.EPI_MUL, aux_in=X),
+             dict(bias=bias, epilogue=hiplib.EPI_ACT_DACT, act=hiplib.ACT_GELU_TANH, aux_out=D), dict(bias=bias, dropout=(0.1, (7, 9)))]
+    for kw in kinds[: 5 if layout == "nt" else 4]:
+        hiplib.gemm(lay, A, B, C, **kw)
+        for r0 in (0, (M - 100) // 8 * 8):       # 100 rows alone take 64x64 tiles; a dropout decision hangs on the row, so the first ones only
+            if "dropout" in kw and r0:
+                continue
+            r1 = min(M, r0 + 100)
+            c, d = (torch.empty(r1 - r0, N, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+            hiplib.gemm(lay, A[r0:r1], B, c, **{k: d if k == "aux_out" else v[r0:r1] if k in ("resid", "aux_in") else v for k, v in kw.items()})
+            assert torch.equal(c, C[r0:r1]) and ("aux_out" not in kw or torch.equal(d, D[r0:r1])), (kw, r0)
+    F = torch.ones(M, N, device=DEV)
+    hiplib.gemm(lay, A, B, F, accumulate=True, alpha=0.5)
+    assert ((F.double() - 1.0 - 0.5 * ref).abs() <= slack + 2.0 ** -23 * (ref.abs() + 2.0)).all()
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+def test_batches(hiplib, layout):
+    """Batched problems of several tiles a block: operands and outputs of each batch by its strides."""
+    lay, n, M, N, K = getattr(hiplib, layout.upper()), 3, 2056, 2312, 256
+    A, B = rand(n, M, K, seed=1), rand(n, *((N, K) if layout == "nt" else (K, N)), seed=2)
+    C, c = torch.empty(n, M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    hiplib.gemm_batched(lay, hiplib.BF16, M, N, K, A.data_ptr(), K, (M * K, 0), B.data_ptr(), B.shape[2], (N * K, 0), C.data_ptr(), N, (M * N, 0), n, 1)
+    for i in range(n):
+        hiplib.gemm(lay, A[i], B[i], c)
+        assert torch.equal(C[i], c)
