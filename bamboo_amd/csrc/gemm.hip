@@ -655,30 +655,79 @@ extern "C" int bb_conv3x3_dgrad_bn(int dtype, int n, int h, int w, int cin, int 
 template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(GroupedArgs& G, hipStream_t st) {
     constexpr int BM = 128, BN = 128, STAGES = 3;
     constexpr int smem = STAGES * (BM + BN) * 32 * 2;
-    int blocks = 0, kmin = G.p[0].K;
+    int blocks = 0;
     for (int i = 0; i < G.count; ++i) {
         GemmArgs& g = G.p[i];
         g.tiles_m = (g.M + BM - 1) / BM;
         g.tiles_n = (g.N + BN - 1) / BN;
         G.first_block[i] = blocks;
         blocks += g.tiles_m * g.tiles_n;
-        kmin = g.K < kmin ? g.K : kmin;
     }
     G.first_block[G.count] = blocks;
     auto kern = gemm_bf16_dma_grouped_kernel<BM, BN, 2, 2, TA, TB, true, STAGES, CONVB, !TA && !TB>;
-    // Weight gradients over many rows whose blocks, three a CU, fill their rounds: lock step keeps the three, which started
-    // together, on the same operand panels (459 instead of 720 MiB read per launch).  Where blocks of a CU start apart, or the
-    // contraction is too short for them to drift, it only adds waits.  In lock step / free (us), hidden size (x 4 in the feed-forward) and
-    // rows: 1024 8192 222 / 224 (a stage of it gains half a percent), 16384 435 / 449; 4096 119 / 115, 2048 67.2 / 65.8; 768 (56 % of a
-    // round) 2048 48.3 / 45.4, 12000 263 / 209; 960 (94 %) 8192 220 / 216; 1600 (85 % of three rounds) 4096 336 / 305.
-    // ResNet blocks, 6272 pixels: 256 middle channels 41.3 / 37.6, 512 120 / 102.  Forward products 406 / 411 (8192x1024, x 4), input
-    // gradients 384 / 362.
-    if constexpr (TA && !CONVB) {
-        const int slots = (blocks + 767) / 768 * 768;
-        if (kmin >= 8192 && (int64_t)blocks * 100 >= (int64_t)slots * 95) kern = gemm_bf16_dma_grouped_kernel<BM, BN, 2, 2, TA, TB, true, STAGES, false, true>;
-    }
+    // (the waves of a block in lock step, hidden size 1024 (x 4 in the feed-forward) and 8192 rows, in step / free: forward products 406 / 411 us,
+    // input gradients 384 / 362)
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(256), smem, st, G);
+    BB_LAUNCH_CHECK();
+    return BB_OK;
+}
+
+// Weight gradients on the tiles of gemm_m16.h: plain fp32 sums over contractions from kM16WgradRows rows on (below, what such a launch does is
+// read and write C, which three blocks a CU of 128x128 tiles do sooner: hidden size 1024 (x 4 in the feed-forward), 128x128 tiles of
+// gemm_bf16_dma_grouped_kernel / the better of these, us: 128 rows 22.7 / 25.0, 256 26.8 / 27.5, 512 33.5 / 32.5, 1024 43.7 / 42.8).  The tile
+// by its rounds, as in pick_dma_tile: a step of 64 rows, and what a round takes beside.  Before / 256x256 / 192x256 / 128x256 / 128x128 two a CU
+// (the one taken marked), hidden size and rows: 1024 8192 229 / 184* / 280 / 215 / 204, 4096 119 / 101* / 154 / 120 / 110; 1600 4096 282 / 301 /
+// 254* / 295 / 265; 960 8200 219 / 182 / 161* / 215 / 207; 768 16384 285 / 326 / 256 / 223* / 242, 8192 148 / 174 / 135 / 113* / 121, 2043 46 / 59 /
+// 47 / 40* / 40; 640 3000 58 / 78 / 61 / 48* / 51.  Tried: 160-wide tiles (rows of 320 bytes, no whole lines: 1600 284); 32-wide k-tiles in rings
+// of four and five (1024 8192 195, 202 against 187).
+constexpr int kM16WgradRows = 768;
+enum WgradTile { WG_NONE = 0, WG256x256, WG192x256, WG128x256, WG128x128 };
+static WgradTile pick_wgrad_m16(const GroupedArgs& G) {
+    static const struct {
+        WgradTile tile;
+        int bm, bn, slots, sum_columns;
+        double step, rest;
+    } tiles[] = {{WG256x256, 256, 256, kCUs, m16_sum_columns(8, 4), 1.36, 3.0},
+                 {WG192x256, 192, 256, kCUs, m16_sum_columns(6, 4), 1.12, 3.0},
+                 {WG128x256, 128, 256, kCUs, m16_sum_columns(4, 4), 0.80, 3.0},
+                 {WG128x128, 128, 128, 2 * kCUs, m16_sum_columns(4, 2), 0.86, 3.0}};
+    int kmax = 0;
+    for (int i = 0; i < G.count; ++i) {
+        const GemmArgs& g = G.p[i];
+        if (!g.c_f32 || g.bias || g.epilogue != BB_EPI_NONE || g.K < kM16WgradRows || g.lda >= kDmaMaxLd || g.ldb >= kDmaMaxLd || g.conv_c != 0) return WG_NONE;
+        kmax = g.K > kmax ? g.K : kmax;
+    }
+    WgradTile best = WG_NONE;
+    double least = 0.0;
+    for (const auto& t : tiles) {
+        int64_t n = 0;
+        bool fits = true;
+        for (int i = 0; i < G.count; ++i) {
+            const GemmArgs& g = G.p[i];
+            const int columns = (g.N + t.bn - 1) / t.bn;
+            fits = fits && (!g.colsum || columns >= t.sum_columns);
+            n += (int64_t)((g.M + t.bm - 1) / t.bm) * columns;
+        }
+        const double us = (double)((n + t.slots - 1) / t.slots) * ((kmax + 63) / 64 * t.step + t.rest);
+        if (fits && (best == WG_NONE || us < least)) best = t.tile, least = us;
+    }
+    return best;
+}
+template <int TM, int TN, int WM, int WN, int STAGES> static int launch_wgrad_m16(GroupedArgs& G, hipStream_t st) {
+    constexpr int BM = WM * TM * 16, BN = WN * TN * 16, smem = STAGES * (BM + BN) * 128;
+    auto kern = wgrad_m16_grouped_kernel<TM, TN, WM, WN, STAGES>;
+    BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
+    int blocks = 0;
+    for (int i = 0; i < G.count; ++i) {
+        GemmArgs& g = G.p[i];
+        g.tiles_m = (g.M + BM - 1) / BM;
+        g.tiles_n = (g.N + BN - 1) / BN;
+        G.first_block[i] = blocks;
+        blocks += g.tiles_m * g.tiles_n;
+    }
+    G.first_block[G.count] = blocks;
+    bb_launch(kern, dim3(G.ride.blocks + blocks), dim3(WM * WN * 64), smem, st, G);
     BB_LAUNCH_CHECK();
     return BB_OK;
 }
@@ -837,7 +886,13 @@ extern "C" int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const 
     if (layout == BB_NT) return launch_grouped<false, false>(G, st);
     if (layout == BB_NN) return launch_grouped<false, true>(G, st);
     if (has_conv) return launch_grouped<true, true, true>(G, st);
-    return launch_grouped<true, true>(G, st);
+    switch (pick_wgrad_m16(G)) {
+        case WG256x256: return launch_wgrad_m16<8, 4, 2, 4, 2>(G, st);
+        case WG192x256: return launch_wgrad_m16<6, 4, 2, 4, 2>(G, st);
+        case WG128x256: return launch_wgrad_m16<4, 4, 2, 4, 3>(G, st);
+        case WG128x128: return launch_wgrad_m16<4, 4, 2, 2, 2>(G, st);
+        default: return launch_grouped<true, true>(G, st);
+    }
 }
 extern "C" int bb_gemm_grouped(const bb_gemm_desc* descs, int count, void* stream) {
     return bb_gemm_grouped_sums(descs, count, nullptr, 0, stream);

@@ -132,26 +132,24 @@ template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int S
     static constexpr bool ROWS = TM >= 8;
     static constexpr int WAIT = 2 * TN;
     static constexpr int READS = NM / 2, BARRIER = ROWS ? NM + WAIT : NM * 5 / 8, FEEDS = ROWS ? NM - WAIT : NM;
-    // SUMS: a wave adds up the k of its first SUM_FRAGS fragments of A, which are others than those of the other waves of its rows
-    static constexpr int SUM_FRAGS = (TM + WN - 1) / WN;
-
     OpA opa;
     OpB opb;
     FragA fa;
     M16Frags<BN, TN, BKM, PAIRED> fb;
     f32x4 acc[TM][TN];
     bf16x8 a[ROWS ? 1 : 2][TM], b[2][TN];
-    float sum[SUM_FRAGS];
+    float sum, part;
     int wave, stage, first;
     unsigned lds0;
     unsigned char* smem;
 
-    __device__ __forceinline__ void init(unsigned char* lds, int tid) {
+    // (first_fragment: KM, of the wave's fragments of A the one it starts with)
+    __device__ __forceinline__ void init(unsigned char* lds, int tid, int first_fragment = 0) {
         smem = lds;
         lds0 = (unsigned)(uintptr_t)(lds_ptr_t*)lds;
         wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         stage = 0;
-        first = AKM ? wave % WN * SUM_FRAGS % TM : 0;
+        first = first_fragment;
         fa.init(wave / WN * (TM * 16), tid & 63, first);
         fb.init(wave % WN * (TN * 16), tid & 63);
     }
@@ -182,9 +180,9 @@ template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int S
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < SUM_FRAGS; ++q) sum[q] = 0.f;
+        sum = 0.f;
     }
+    // SUMS: the wave adds up the k of its first fragment of A, a few beside each product of the row (at once they would hold up the next one).
     // One k-tile: multiplied, its second step's and the next k-tile's first fragments read, the k-tile STAGES on sent for (live -1).
     template <bool SUMS = false> __device__ __forceinline__ void step(int live) {
         fa.here();
@@ -199,14 +197,16 @@ template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int S
                 if constexpr (m == BARRIER) landed<STAGES - 2>();
                 const bf16x8& row = a[ROWS ? 0 : s][i];
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j], row, acc[i][j], 0, 0, 0);
-                if constexpr (SUMS && j == 0 && i < SUM_FRAGS) {
-                    float t = 0.f;
+                if constexpr (SUMS && i == 0) {
+                    if constexpr (j == 0) part = 0.f;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) t += (float)row[e];
-                    typedef __attribute__((ext_vector_type(2))) unsigned u2;
-                    const u2 both = __builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(__float_as_uint(t), __float_as_uint(t), false, false));
-                    sum[i] += __uint_as_float(both[0]);
-                    sum[i] += __uint_as_float(both[1]);
+                    for (int e = 8 * j / TN; e < 8 * (j + 1) / TN; ++e) part += (float)row[e];
+                    if constexpr (j == TN - 1) {
+                        typedef __attribute__((ext_vector_type(2))) unsigned u2;
+                        const u2 both = __builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(__float_as_uint(part), __float_as_uint(part), false, false));
+                        sum += __uint_as_float(both[0]);
+                        sum += __uint_as_float(both[1]);
+                    }
                 }
                 if constexpr (m >= BARRIER && m < BARRIER + FEEDS)
                     static_for([&](auto d) { feed<LOADS * (m - BARRIER) / FEEDS + decltype(d)::value>(into, live); },
@@ -362,4 +362,112 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_m16_kernel(const GemmAr
         tm = next_m;
         tn = next_n;
     }
+}
+
+// Weight gradients: C[m][n] (fp32) = or += alpha * sum over k of A[k][m] B[k][n], both operands k-major, any K > 0.
+//
+// A last k-tile that is not whole: its transfers read the last row again (nothing lies behind it), and once they have landed the rows
+// past the end are cleared in LDS, in both operands, before they are read.
+//
+// Column sums of A (a bias gradient): the waves of a row of waves, in the blocks of the first tile columns, hold the same fragments of A; each
+// starts with another and adds that one up beside its products.  (By its number in the code: nothing is chosen inside the loop.  One fragment a
+// wave: with two, in the first column alone, the blocks of that column took a tenth longer, and a launch of one round with them.)  Per 32 k a lane
+// adds its eight, then (the lower half of the wave) what the lane 32 further on has; the two chains of a row are put together at the end.
+// That is the order of gemm_bf16_dma_body, whose lanes add eight of sixteen k a step.
+constexpr int m16_sum_columns(int TM, int WN) { return (TM + WN - 1) / WN; }   // tile columns that takes: a problem with sums has as many
+template <int TM, int TN, int WM, int WN, int STAGES>
+__device__ __forceinline__ void wgrad_m16_body(const GemmArgs& g, const int id) {
+    using Loop = M16Loop<TM, TN, WM, WN, true, true, false, STAGES>;
+    constexpr int BM = Loop::BM, BN = Loop::BN, NT = Loop::NW * 64;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x;
+    const int KT = (g.K + 63) / 64, tail = g.K & 63;
+    int tm, tn;
+    panel_coords<8>(id, g.tiles_m, g.tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    Loop p;
+    p.opa.init((const bf16*)g.A, g.lda, m0, g.M, tid, KT == 1 && tail ? tail : 64);
+    p.opb.init((const bf16*)g.B, g.ldb, n0, g.N, tid, KT == 1 && tail ? tail : 64);
+    constexpr int SC = m16_sum_columns(TM, WN);
+    const int first = __builtin_amdgcn_readfirstlane((tid >> 6) % WN * SC + tn);
+    const bool do_sums = g.colsum != nullptr && tn < SC && first < TM;
+    p.init(smem, tid, do_sums ? first : 0);
+    auto last_tile = [&]() {     // the transfers that go out next are those of the last k-tile
+        if (!tail) return;
+        const int t = m16_here(tid);
+        p.opa.reach((int)g.lda * 2, g.M - 8 - m0, t, tail);
+        p.opb.reach((int)g.ldb * 2, g.N - 8 - n0, t, tail);
+    };
+    p.clear();
+#pragma unroll
+    for (int t = 0; t < STAGES; ++t) {
+        if (t > 0 && t == KT - 1) last_tile();
+        p.feed_all(t, __builtin_amdgcn_readfirstlane((t - KT) >> 31));
+    }
+    p.template landed<STAGES - 1>();
+
+    const int wm = p.wave / WN, wn = p.wave % WN;
+    auto walk = [&](auto sums_c) {
+        constexpr bool SUMS = decltype(sums_c)::value;
+        p.read_first();
+        int kt = 0;
+        for (const int whole = KT - (tail ? 1 : 0); kt + STAGES < whole; ++kt) p.template step<SUMS>(-1);
+        for (; kt < KT; ++kt) {
+            if (tail && kt + STAGES == KT - 1) last_tile();
+            if (tail && kt == KT - 1) {
+                // everything has landed (the ring holds nothing behind it), no wave reads on before the rows are cleared
+                p.template landed<0>();
+                const int t = m16_here(tid);
+                unsigned char* st = smem + p.stage * Loop::STAGE_BYTES;
+                for (int b = tail * BM * 2 + t * 16; b < Loop::OpA::BYTES; b += NT * 16) *(u32x4*)(st + b) = u32x4{0u, 0u, 0u, 0u};
+                for (int b = tail * BN * 2 + t * 16; b < Loop::OpB::BYTES; b += NT * 16) *(u32x4*)(st + Loop::OpA::BYTES + b) = u32x4{0u, 0u, 0u, 0u};
+                p.template landed<0>();
+                p.read_first();
+            }
+            p.template step<SUMS>(__builtin_amdgcn_readfirstlane((kt + STAGES - KT) >> 31));
+        }
+    };
+    if (do_sums) walk(std::true_type{});
+    else walk(std::false_type{});
+    const int lane = m16_here(tid) & 63;
+    if (do_sums) {
+        const float t = p.sum + __shfl_xor(p.sum, 16, 64);
+        const int m = m0 + (wm * TM + first) * 16 + (lane & 15);
+        if (lane < 16 && m < g.M) g.colsum[m] += t;
+    }
+
+    const int row0 = m0 + wm * (TM * 16) + (lane & 15), col = n0 + wn * (TN * 16) + 4 * (lane >> 4);
+    auto row = [&](int i) { return row0 + Loop::FragA::place(i, p.first) * 16; };
+    constexpr int AHEAD = TM > 4 ? 2 : TM;
+    f32x4 old[AHEAD][TN];
+    auto fetch = [&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        if (!g.accumulate) return;
+        const float* c = (const float*)g.C + (int64_t)min(row(i), g.M - 1) * g.ldc;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) old[i % AHEAD][j] = *(const f32x4*)(c + min(col + j * 16, g.N - 4));
+    };
+    static_for([&](auto i_c) { fetch(i_c); }, std::make_integer_sequence<int, AHEAD>{});
+    static_for(
+        [&](auto i_c) {
+            constexpr int i = decltype(i_c)::value;
+            const int m = row(i);
+            float* c = (float*)g.C + (int64_t)m * g.ldc + col;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                f32x4 v = p.acc[i][j] * g.alpha;
+                if (g.accumulate) v = old[i % AHEAD][j] + v;
+                if (m < g.M && col + j * 16 < g.N) *(f32x4*)(c + j * 16) = v;
+            }
+            if constexpr (i + AHEAD < TM) fetch(std::integral_constant<int, i + AHEAD>{});
+        },
+        std::make_integer_sequence<int, TM>{});
+}
+// a layer's in one launch (the tiles of all problems one list, see gemm_bf16_dma_grouped_kernel); two waves a SIMD
+template <int TM, int TN, int WM, int WN, int STAGES> __global__ __launch_bounds__(WM* WN * 64, 2) void wgrad_m16_grouped_kernel(const GroupedArgs G) {
+    const int id = grouped_place<WM * WN>(G);
+    if (id < 0) return;
+    int pi = 0;
+    while (pi + 1 < G.count && id >= G.first_block[pi + 1]) ++pi;
+    wgrad_m16_body<TM, TN, WM, WN, STAGES>(G.p[pi], id - G.first_block[pi]);
 }

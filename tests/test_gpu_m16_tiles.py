@@ -62,3 +62,26 @@ def test_batches(hiplib, layout):
     for i in range(n):
         hiplib.gemm(lay, A[i], B[i], c)
         assert torch.equal(C[i], c)
+
+
+# weight gradients by the tile that two of them in one launch take: 256x256, 192x256, 128x256, 128x128, 8 rows and columns in the last ones
+@pytest.mark.parametrize("shapes", [[(4104, 1544), (1544, 4104)], [(4104, 1032), (1032, 4104)], [(1032, 2056), (2056, 1032)], [(2056, 2056), (2056, 1544)]])
+@pytest.mark.parametrize("K", [768, 769, 831, 1000])      # whole k-tiles, one row in the last, all but one, 40
+def test_weight_gradients(hiplib, shapes, K):
+    """A layer's weight gradients in one launch, with the bias gradients: as one by one, bit for bit (which other tiles run), and against fp64."""
+    ops = [(rand(K, M, seed=1 + i), rand(K, N, seed=5 + i)) for i, (M, N) in enumerate(shapes)]
+    for accumulate in (False, True):
+        def outputs():
+            return [(torch.full((a.shape[1] + 1, b.shape[1]), 3.0, device=DEV), torch.full((a.shape[1],), 3.0, device=DEV)) for a, b in ops]
+        both, single = outputs(), outputs()
+        descs = [[hiplib.gemm_desc(hiplib.TN, a, b, c[:-1], accumulate=accumulate, colsum_out=s, alpha=0.5) for (a, b), (c, s) in zip(ops, o)] for o in (both, single)]
+        hiplib.gemm_grouped(descs[0])
+        for d in descs[1]:
+            hiplib.gemm_grouped([d])
+        for (c, s), (c1, s1), (a, b) in zip(both, single, ops):
+            assert torch.equal(c, c1) and torch.equal(s, s1) and (c[-1] == 3).all()
+            ref, slack = product(a.t().contiguous(), b)
+            start = 3.0 if accumulate else 0.0
+            assert ((c[:-1].double() - start - 0.5 * ref).abs() <= slack + 2.0 ** -23 * (ref.abs() + start)).all()
+            sums = a.double().sum(0)
+            assert ((s.double() - 3.0 - sums).abs() <= K * 2.0 ** -24 * (a.double().abs().sum(0) + 3.0)).all()
