@@ -10,6 +10,7 @@
 #include "gemm_kernels.h"
 #include "gemm_m16.h"
 #include "gemm_f32.h"
+#include "gemm_f32_pieces.h"
 #include "gemm_wave.h"
 
 // =========================================================================================
@@ -369,6 +370,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
         else snprintf(out, out_len, "bf16_%s_%s%s", layouts[d->layout], dt == D64x64k64s4 && halve_tiles(d->M, d->N, batches) ? "halves_" : "",
                  dt != D_NONE ? kDmaTileNames[dt] : "128x128");
     }
+    else if (const PiecesTile tile = pick_pieces(d, 1)) snprintf(out, out_len, "f32_%s_pieces128x%d", layouts[d->layout], tile == P128x128 ? 128 : 64);
     else if (f32_wide(d->lda, d->ldb)) snprintf(out, out_len, "f32_%s_64x64wide", layouts[d->layout]);
     else if (pick_f32_wave(d->M, d->N, d->K, batches, d->layout)) snprintf(out, out_len, "f32_%s_wave32x32k%d", layouts[d->layout], kF32Waves);
     else {
@@ -529,6 +531,7 @@ extern "C" int bb_gemm(const bb_gemm_desc* d, void* stream) {
         if (!ta && tb) return dispatch_bf16<false, true>(g, (int)batches, st);
         return dispatch_bf16<true, true>(g, (int)batches, st);
     }
+    if (const PiecesTile tile = pick_pieces(d, 1)) return launch_pieces(g, d->layout, tile, st);
     if (!ta && !tb) return dispatch_f32<false, false>(g, (int)batches, st);
     if (!ta && tb) return dispatch_f32<false, true>(g, (int)batches, st);
     return dispatch_f32<true, true>(g, (int)batches, st);
@@ -813,6 +816,19 @@ extern "C" int bb_gemm_grouped_sums(const bb_gemm_desc* descs, int count, const 
     }
     // weight gradients of few tiles: 64x64 tiles, the contraction dealt to the waves (see kGroupedWaveTiles)
     wave = wave && (!dma || tiles <= (count > 1 ? kGroupedWaveTiles : 256));   // alone: as bb_gemm takes it
+    if (!fuse && count >= 2 && pick_pieces(descs, count)) {
+        GroupedArgs G;
+        G.count = count;
+        G.ride = ride;
+        for (int i = 0; i < count; ++i) {
+            int64_t batches;
+            bool ta, tb;
+            int rc = fill_args(&descs[i], G.p[i], batches, ta, tb);
+            if (rc) return rc;
+        }
+        const int rc = colsum_f32(descs, count, stream);
+        return rc ? rc : launch_pieces_grouped(G, st);
+    }
     // fp32: unbatched problems of one layout share a launch where one kernel takes them all (weight gradients of both kinds:
     // the 64x64 tiles)
     bool fuse32 = !fuse && !has_conv && count >= 2 && count <= GROUP_MAX;

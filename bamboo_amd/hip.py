@@ -50,7 +50,7 @@ class GemmDesc(Structure):
         ("ldaux", c_int64), ("colsum_out", c_void_p), ("colsum_ws", c_void_p),
         ("conv_h", c_int32), ("conv_w", c_int32), ("conv_c", c_int32), ("conv_row0", c_int32),
         ("strip_stats", c_void_p),
-        ("dropout_p", c_float), ("dropout_k0", c_uint32), ("dropout_k1", c_uint32),
+        ("dropout_p", c_float), ("dropout_k0", c_uint32), ("dropout_k1", c_uint32), ("pieces", c_int32),
     ]
 
 
@@ -220,10 +220,11 @@ def _row_major(t, name):
 # ------------------------------------------------------------------------------------- GEMM
 def gemm_desc(layout, A, B, C, *, alpha=1.0, bias=None, epilogue=EPI_NONE, act=ACT_RELU, accumulate=False,
               aux_in=None, aux_out=None, resid=None, colsum_out=None, colsum_ws=None, conv=None, strip_stats=None,
-              dropout=None):
+              dropout=None, pieces=False):
     """Descriptor of C = epilogue(alpha * op(A) op(B) [+ bias]) on 2-D row-major views.
     ``conv=(h, w)`` (TN only): B is the NHWC tensor ``[pixels, c]`` whose 3x3 patch matrix ``[pixels, 9c]`` is
-    the operand, gathered inside the kernel (weight gradient of a 3x3 convolution)."""
+    the operand, gathered inside the kernel (weight gradient of a 3x3 convolution).
+    ``pieces``: an fp32 product may run on bf16 matrix instructions (see ``bb_gemm_desc``)."""
     lda, ldb, ldc = _row_major(A, "A"), _row_major(B, "B"), _row_major(C, "C")
     if conv is not None:
         if layout != TN or not B.is_contiguous():
@@ -248,7 +249,7 @@ def gemm_desc(layout, A, B, C, *, alpha=1.0, bias=None, epilogue=EPI_NONE, act=A
     d.nb1 = d.nb2 = 1
     if conv is not None:
         d.conv_h, d.conv_w, d.conv_c, d.conv_row0 = conv[0], conv[1], B.shape[1], 0
-    d.alpha, d.epilogue, d.act, d.accumulate = alpha, epilogue, act, int(accumulate)
+    d.alpha, d.epilogue, d.act, d.accumulate, d.pieces = alpha, epilogue, act, int(accumulate), int(pieces)
     ldaux = 0
     for t in (aux_in, aux_out, resid):
         if t is not None:

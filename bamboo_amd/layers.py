@@ -231,6 +231,15 @@ class TransformerLayer:
         those that lie that close to zero, one in some millions, the gradient of the unit comes or goes."""
         return self.activation != "relu" and hip.attention_probs_supported(ctx.dtype, ctx.batch, self.heads, ctx.seq, self.head_dim)
 
+    @property
+    def pieces(self):
+        """Whether fp32 products may run on bf16 matrix instructions, their operands as sums of bf16 pieces: nearer to the exact results
+        (``gemm_f32_pieces.hip``), but other last bits, which a ReLU does not take (see above)."""
+        return self.activation != "relu"
+
+    def _gemm(self, ctx, *a, **kw):
+        return ctx.gemm(*a, pieces=self.pieces, **kw)
+
     def _attention_stash(self, ctx, tag=""):
         """What the attention keeps for its backward."""
         if not self.fused_attention(ctx):
@@ -388,7 +397,7 @@ class TransformerLayer:
     def forward(self, x, st, ctx):
         """x: [rows, hidden] (kept by reference in the stash); returns st['out']."""
         self.rebuild(x, st, ctx)
-        ctx.gemm(hip.NT, st["act"], self.w["feed_forward.w_2.weight"], st["out"], bias=self.w["feed_forward.w_2.bias"],
+        self._gemm(ctx, hip.NT, st["act"], self.w["feed_forward.w_2.weight"], st["out"], bias=self.w["feed_forward.w_2.bias"],
                  epilogue=hip.EPI_RESIDUAL, resid=st["x1"], dropout=self._drop(ctx, self.SITE_SUBLAYER1), stream=ctx.stream)
         return st["out"]
 
@@ -399,9 +408,9 @@ class TransformerLayer:
         st["x0"] = x
         hip.layernorm_fwd(x, w["sublayer.0.norm.a_2"], w["sublayer.0.norm.b_2"], st["n1"], st["mean1"],
                           st["rinv1"], kind, self.eps, stream=sm)
-        ctx.gemm(hip.NT, st["n1"], w["qkv.weight"], st["qkv"], bias=w["qkv.bias"], stream=sm)
+        self._gemm(ctx, hip.NT, st["n1"], w["qkv.weight"], st["qkv"], bias=w["qkv.bias"], stream=sm)
         self._attention_fwd(st, ctx)
-        ctx.gemm(hip.NT, st["ctx"], w["self_attn.linears.3.weight"], st["x1"], bias=w["self_attn.linears.3.bias"],
+        self._gemm(ctx, hip.NT, st["ctx"], w["self_attn.linears.3.weight"], st["x1"], bias=w["self_attn.linears.3.bias"],
                  epilogue=hip.EPI_RESIDUAL, resid=x, dropout=self._drop(ctx, self.SITE_SUBLAYER0), stream=sm)
         hip.layernorm_fwd(st["x1"], w["sublayer.1.norm.a_2"], w["sublayer.1.norm.b_2"], st["n2"], st["mean2"],
                           st["rinv2"], kind, self.eps, stream=sm)
@@ -412,7 +421,7 @@ class TransformerLayer:
         if ctx.defer or self.activation == "relu":
             # act' is read by the backward pass only: a forward that most likely has none writes act alone (and a
             # ReLU layer never writes it: its backward pass reads the derivative off act)
-            ctx.gemm(hip.NT, st["n2"], w["feed_forward.w_1.weight"], st["act"], bias=w["feed_forward.w_1.bias"],
+            self._gemm(ctx, hip.NT, st["n2"], w["feed_forward.w_1.weight"], st["act"], bias=w["feed_forward.w_1.bias"],
                      epilogue=hip.EPI_ACT, act=act, dropout=self._drop(ctx, self.SITE_FFN), stream=sm)
         else:
             self._ffn1(st, ctx)
@@ -421,7 +430,7 @@ class TransformerLayer:
         """act and act' of the feed-forward's hidden layer; under dropout both carry the keep factor, so the backward
         pass multiplies by the stored derivative as before."""
         w = self.w
-        ctx.gemm(hip.NT, st["n2"], w["feed_forward.w_1.weight"], st["act"], bias=w["feed_forward.w_1.bias"],
+        self._gemm(ctx, hip.NT, st["n2"], w["feed_forward.w_1.weight"], st["act"], bias=w["feed_forward.w_1.bias"],
                  epilogue=hip.EPI_ACT_DACT, act=hip.ACT_CODES[self.activation], aux_out=st["dact"],
                  dropout=self._drop(ctx, self.SITE_FFN), stream=ctx.stream)
 
@@ -437,7 +446,8 @@ class TransformerLayer:
         wgrads, sums = [], []
         # ... and each carries its bias gradient (column sums of dy) in the same kernel
         wgrad = lambda dy, x, name: wgrads.append(hip.gemm_desc(
-            hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[name[:-len("weight")] + "bias"], colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
+            hip.TN, dy, x, g[name], accumulate=True, pieces=self.pieces, colsum_out=g[name[:-len("weight")] + "bias"],
+            colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
         if ctx.deferred and self.activation != "relu":
             self._ffn1(st, ctx)   # the forward of this stash left act' out: same kernel, same bits as a normal forward
         # the gradient behind a sublayer's dropout feeds the sublayer; the residual branch takes the one in front of it
@@ -449,23 +459,23 @@ class TransformerLayer:
         wgrad(d_ff2, st["act"], "feed_forward.w_2.weight")
         if self.activation == "relu":
             # act = relu(u) * keep / (1 - p): positive exactly where the gradient passes, and then with factor 1 / (1 - p)
-            ctx.gemm(hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL_POS, aux_in=st["act"],
+            self._gemm(ctx, hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL_POS, aux_in=st["act"],
                      alpha=1.0 / (1.0 - self.dropout) if self.dropout > 0 else 1.0, stream=sm)
         else:
-            ctx.gemm(hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL, aux_in=st["dact"], stream=sm)
+            self._gemm(ctx, hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL, aux_in=st["dact"], stream=sm)
         wgrad(d_ffn, st["n2"], "feed_forward.w_1.weight")
-        ctx.gemm(hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
         # d_x1 = d_out + LN2'(d_n2)
         d_drop = ctx.buf("d_drop0", (R, h)) if self.dropout > 0 else None
         self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h1, d_drop, self.SITE_SUBLAYER0)
         # attention output projection
         d_proj = d_h1 if d_drop is None else d_drop
         wgrad(d_proj, st["ctx"], "self_attn.linears.3.weight")
-        ctx.gemm(hip.NN, d_proj, w["self_attn.linears.3.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_proj, w["self_attn.linears.3.weight"], d_h0, stream=sm)
         self._attention_bwd(d_h0, d_qkv, st, ctx)
         # QKV projection
         wgrad(d_qkv, st["n1"], "qkv.weight")
-        ctx.gemm(hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
         # d_x0 = d_x1 + LN1'(d_n1)
         self._layernorm_bwd(sums, ctx, st["x0"], "sublayer.0.norm", st["mean1"], st["rinv1"], d_h0, d_h1, d_x)
         # d_out (d_drop1), d_ffn, d_h1 (d_drop0) and d_qkv still hold the four output gradients here
@@ -563,7 +573,7 @@ class DecoderLayer(TransformerLayer):
 
     def forward(self, x, st, ctx):
         self.rebuild(x, st, ctx)
-        ctx.gemm(hip.NT, st["act"], self.w["feed_forward.w_2.weight"], st["out"], bias=self.w["feed_forward.w_2.bias"],
+        self._gemm(ctx, hip.NT, st["act"], self.w["feed_forward.w_2.weight"], st["out"], bias=self.w["feed_forward.w_2.bias"],
                  epilogue=hip.EPI_RESIDUAL, resid=st["x2"], dropout=self._drop(ctx, self.SITE_SUBLAYER1), stream=ctx.stream)
         return st["out"]
 
@@ -575,24 +585,24 @@ class DecoderLayer(TransformerLayer):
         # sublayer 0: self-attention; the memory (gpt2.py:31) comes with its LayerNorm
         hip.layernorm_fwd(x, w["sublayer.0.norm.a_2"], w["sublayer.0.norm.b_2"], st["n1"], st["mean1"], st["rinv1"],
                           kind, self.eps, stream=sm, memory=st["mem"])
-        ctx.gemm(hip.NT, st["n1"], w["qkv.weight"], st["qkv"], bias=w["qkv.bias"], stream=sm)
+        self._gemm(ctx, hip.NT, st["n1"], w["qkv.weight"], st["qkv"], bias=w["qkv.bias"], stream=sm)
         self._attention_fwd(st, ctx, site=self.SITE_ATTENTION)
-        ctx.gemm(hip.NT, st["ctx"], w["self_attn.linears.3.weight"], st["x1"], bias=w["self_attn.linears.3.bias"],
+        self._gemm(ctx, hip.NT, st["ctx"], w["self_attn.linears.3.weight"], st["x1"], bias=w["self_attn.linears.3.bias"],
                  epilogue=hip.EPI_RESIDUAL, resid=x, dropout=self._drop(ctx, self.SITE_SUBLAYER0), stream=sm)
         # sublayer 1: queries from the stream, keys and values from the memory
         hip.layernorm_fwd(st["x1"], w["sublayer.1.norm.a_2"], w["sublayer.1.norm.b_2"], st["n_src"], st["mean_src"],
                           st["rinv_src"], kind, self.eps, stream=sm)
         qs = st["qkv_src"]
-        ctx.gemm(hip.NT, st["n_src"], w["src_attn.linears.0.weight"], qs[:, :h], bias=w["src_attn.linears.0.bias"], stream=sm)
-        ctx.gemm(hip.NT, st["mem"], w["kv.weight"], qs[:, h:], bias=w["kv.bias"], stream=sm)
+        self._gemm(ctx, hip.NT, st["n_src"], w["src_attn.linears.0.weight"], qs[:, :h], bias=w["src_attn.linears.0.bias"], stream=sm)
+        self._gemm(ctx, hip.NT, st["mem"], w["kv.weight"], qs[:, h:], bias=w["kv.bias"], stream=sm)
         self._attention_fwd(self._src_views(st), ctx, site=self.SITE_SRC_ATTENTION, mask="none")
-        ctx.gemm(hip.NT, st["ctx_src"], w["src_attn.linears.3.weight"], st["x2"], bias=w["src_attn.linears.3.bias"],
+        self._gemm(ctx, hip.NT, st["ctx_src"], w["src_attn.linears.3.weight"], st["x2"], bias=w["src_attn.linears.3.bias"],
                  epilogue=hip.EPI_RESIDUAL, resid=st["x1"], dropout=self._drop(ctx, self.SITE_SUBLAYER_SRC), stream=sm)
         # sublayer 2: feed-forward
         hip.layernorm_fwd(st["x2"], w["sublayer.2.norm.a_2"], w["sublayer.2.norm.b_2"], st["n2"], st["mean2"],
                           st["rinv2"], kind, self.eps, stream=sm)
         if ctx.defer or self.activation == "relu":
-            ctx.gemm(hip.NT, st["n2"], w["feed_forward.w_1.weight"], st["act"], bias=w["feed_forward.w_1.bias"],
+            self._gemm(ctx, hip.NT, st["n2"], w["feed_forward.w_1.weight"], st["act"], bias=w["feed_forward.w_1.bias"],
                      epilogue=hip.EPI_ACT, act=act, dropout=self._drop(ctx, self.SITE_FFN), stream=sm)
         else:
             self._ffn1(st, ctx)
@@ -605,7 +615,8 @@ class DecoderLayer(TransformerLayer):
         d_qkv, d_mem = ctx.buf("d_qkv", (R, 3 * h)), ctx.buf("d_mem", (R, h))
         wgrads, sums = [], []
         wgrad = lambda dy, x, name, bias=None: wgrads.append(hip.gemm_desc(
-            hip.TN, dy, x, g[name], accumulate=True, colsum_out=g[bias or (name[:-len("weight")] + "bias")], colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
+            hip.TN, dy, x, g[name], accumulate=True, pieces=self.pieces, colsum_out=g[bias or (name[:-len("weight")] + "bias")],
+            colsum_ws=ctx.colsum_ws(wgrads, dy.shape[1])))
 
         def flush():
             # the weight gradients collected so far, before a scratch buffer they read is written again
@@ -622,25 +633,25 @@ class DecoderLayer(TransformerLayer):
             hip.dropout_apply(d_out, d_ff2, *self._drop(ctx, self.SITE_SUBLAYER1), stream=sm)
         wgrad(d_ff2, st["act"], "feed_forward.w_2.weight")
         if self.activation == "relu":
-            ctx.gemm(hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL_POS, aux_in=st["act"],
+            self._gemm(ctx, hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL_POS, aux_in=st["act"],
                      alpha=1.0 / (1.0 - self.dropout) if self.dropout > 0 else 1.0, stream=sm)
         else:
-            ctx.gemm(hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL, aux_in=st["dact"], stream=sm)
+            self._gemm(ctx, hip.NN, d_ff2, w["feed_forward.w_2.weight"], d_ffn, epilogue=hip.EPI_MUL, aux_in=st["dact"], stream=sm)
         wgrad(d_ffn, st["n2"], "feed_forward.w_1.weight")
-        ctx.gemm(hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_ffn, w["feed_forward.w_1.weight"], d_h0, stream=sm)
         # d_x2 = d_out + LN2'(d_n2)  -> d_h2
         d_drop = ctx.buf("d_drop_src", (R, h)) if self.dropout > 0 else None
         self._layernorm_bwd(sums, ctx, st["x2"], "sublayer.2.norm", st["mean2"], st["rinv2"], d_h0, d_out, d_h2, d_drop, self.SITE_SUBLAYER_SRC)
         # ---- sublayer 1: attention over the memory
         d_proj = d_h2 if d_drop is None else d_drop
         wgrad(d_proj, st["ctx_src"], "src_attn.linears.3.weight")
-        ctx.gemm(hip.NN, d_proj, w["src_attn.linears.3.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_proj, w["src_attn.linears.3.weight"], d_h0, stream=sm)
         self._attention_bwd(d_h0, d_qkv, self._src_views(st), ctx, site=self.SITE_SRC_ATTENTION, mask="none")
         wgrad(d_qkv[:, :h], st["n_src"], "src_attn.linears.0.weight")
-        wgrads.append(hip.gemm_desc(hip.TN, d_qkv[:, h:], st["mem"], g["kv.weight"], accumulate=True,
+        wgrads.append(hip.gemm_desc(hip.TN, d_qkv[:, h:], st["mem"], g["kv.weight"], accumulate=True, pieces=self.pieces,
                                     colsum_out=g["kv.bias"], colsum_ws=ctx.colsum_ws(wgrads, 2 * h)))
-        ctx.gemm(hip.NN, d_qkv[:, :h], w["src_attn.linears.0.weight"], d_h0, stream=sm)        # d_n_src
-        ctx.gemm(hip.NN, d_qkv[:, h:], w["kv.weight"], d_mem, stream=sm)                       # gradient of the memory
+        self._gemm(ctx, hip.NN, d_qkv[:, :h], w["src_attn.linears.0.weight"], d_h0, stream=sm)        # d_n_src
+        self._gemm(ctx, hip.NN, d_qkv[:, h:], w["kv.weight"], d_mem, stream=sm)                       # gradient of the memory
         # d_x1 = d_x2 + LN_src'(d_n_src)  -> d_h1
         d_drop = ctx.buf("d_drop0", (R, h)) if self.dropout > 0 else None
         self._layernorm_bwd(sums, ctx, st["x1"], "sublayer.1.norm", st["mean_src"], st["rinv_src"], d_h0, d_h2, d_h1, d_drop, self.SITE_SUBLAYER0)
@@ -648,10 +659,10 @@ class DecoderLayer(TransformerLayer):
         # ---- sublayer 0: self-attention
         d_proj0 = d_h1 if d_drop is None else d_drop
         wgrad(d_proj0, st["ctx"], "self_attn.linears.3.weight")
-        ctx.gemm(hip.NN, d_proj0, w["self_attn.linears.3.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_proj0, w["self_attn.linears.3.weight"], d_h0, stream=sm)
         self._attention_bwd(d_h0, d_qkv, st, ctx, site=self.SITE_ATTENTION)
         wgrad(d_qkv, st["n1"], "qkv.weight")
-        ctx.gemm(hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
+        self._gemm(ctx, hip.NN, d_qkv, w["qkv.weight"], d_h0, stream=sm)
         # d_x = d_x1 + LN0'(d_n1) + d_mem * dm/dx
         self._layernorm_bwd(sums, ctx, st["x0"], "sublayer.0.norm", st["mean1"], st["rinv1"], d_h0, d_h1, d_x, memory=(d_mem, st["mem"]))
         flush()

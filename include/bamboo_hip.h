@@ -128,6 +128,10 @@ typedef struct bb_gemm_desc {
      * the same factor.  dropout_p = 0: none.  Not with BB_EPI_DACT / BB_EPI_MUL / BB_EPI_MUL_POS, not batched.            */
     float dropout_p;
     uint32_t dropout_k0, dropout_k1;
+    /* 1: an unbatched fp32 problem may run on bf16 matrix instructions, every operand value as the exact sum of three
+     * bf16 pieces, where that is faster: nearer to the exact result than the fp32 instructions, other last bits, which
+     * may differ between a problem alone and in a group.  0: the fp32 instructions.                              */
+    int32_t pieces;
 } bb_gemm_desc;
 
 /* library ------------------------------------------------------------------------------ */
