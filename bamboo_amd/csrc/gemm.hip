@@ -4,7 +4,7 @@
 // Stands in for F.linear / torch.matmul and their autograd backward in the reference layer
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:121,127,136-146,158).
 //
-// bf16 data paths: large tiles by DMA on 16x16x32 instructions (gemm_m16.h), others on 32x32x16 (gemm_bf16_dma_*); 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for weight
+// bf16 data paths: NT and NN tiles by DMA on 16x16x32 instructions (gemm_m16.h), others on 32x32x16 (gemm_bf16_dma_*); 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for weight
 // gradients of few tiles and few tiles of an odd contraction length; a register-staged kernel for rows of C that are no
 // whole vectors (N % 8 != 0, NT).  fp32: gemm_f32.h.
 #include "gemm_kernels.h"
@@ -45,18 +45,18 @@ static int launch_bf16_dma(GemmArgs& g, int batches, hipStream_t st) {
     return BB_OK;
 }
 
-// One block per CU walks the tiles; a contraction of fewer k-tiles than the ring has stages: a block per tile.
+// 256-row tiles: one block per CU walks the tiles; smaller ones, and a contraction of fewer k-tiles than the ring has stages: a block per tile.
 static constexpr int kCUs = 256;
-template <int TM, int TN, int WM, int WN, int STAGES, bool TB> static int launch_bf16_m16(GemmArgs& g, int batches, hipStream_t st) {
+template <int TM, int TN, int WM, int WN, int STAGES, bool TB, bool WHOLE = false> static int launch_bf16_m16(GemmArgs& g, int batches, hipStream_t st) {
     constexpr int BM = WM * TM * 16, BN = WN * TN * 16, smem = STAGES * (BM + BN) * 128;
-    auto kern = gemm_bf16_m16_kernel<TM, TN, WM, WN, TB, STAGES, false>;
+    auto kern = gemm_bf16_m16_kernel<TM, TN, WM, WN, TB, STAGES, WHOLE, false>;
     if constexpr (!TB) {       // dropout goes with forward (NT) products only: fill_args refuses the others
-        if (g.drop.thresh) kern = gemm_bf16_m16_kernel<TM, TN, WM, WN, TB, STAGES, true>;
+        if (g.drop.thresh) kern = gemm_bf16_m16_kernel<TM, TN, WM, WN, TB, STAGES, WHOLE, true>;
     }
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    const int total = g.tiles_m * g.tiles_n, blocks = g.K >= STAGES * 64 && total > kCUs ? kCUs : total;
+    const int total = g.tiles_m * g.tiles_n, blocks = BM == 256 && g.K >= STAGES * 64 && total > kCUs ? kCUs : total;
     bb_launch(kern, dim3(blocks, 1, batches), dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -129,30 +129,23 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches;
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
-    //  - Problems of at most one tile of 128x64 per CU (NT; 64x128 NN: a k-major operand needs 128 rows for its swizzle)
-    //    take those, short contractions also up to 400, very short ones up to 512, whose chains run under each other; then
-    //    128x128 tiles of three stages, one per CU, up to a round of them.  128x64 / 128x128 (64x128 / 128x128), plain and
-    //    with a residual (us): NT 1200x1600x1600 (250 tiles of 128x64) 12.3 12.9 / 15.1 16.8, 2300x1024x1024 (288) 12.2 12.8
-    //    / 11.7 12.9, 4096x768x768 (384) 10.8 11.3 / 10.4 11.4, x3072 30.2 30.8 / 25.1 26.5, 3136x1024x256 (400) 7.4 8.1 /
-    //    7.8 8.7, 6272x512x128 (392) 6.7 7.4 / 7.1 8.0, 8112x512x128 (512) 6.8 / 7.8; NN 12.1 12.7 / 15.1 16.5, 12.2 12.9 /
-    //    11.8 13.1, 10.9 11.5 / 10.7 11.5, 30.4 30.6 / 25.3 26.7, 7.4 8.2 / 7.9 8.8.  A round of 128x128 with two stages or
-    //    32-wide k-tiles (two and three blocks per CU) / this: NT 8192x512x512 10.7 11.9 / 9.6 10.5, x2048 26.2 28.9 / 21.1
-    //    22.4, NN 10.2 11.5 / 9.8 10.6, 26.2 28.9 / 21.4 22.4; 256x128 / this where a few rows stand against many columns:
-    //    640x6400x1600 24.1 25.6 / 17.3 19.0.  More of them: 256x128 tiles, also for short contractions (NT 6272x1024x256
-    //    12.8 14.0 on 128x64, 10.3 11.4 on 256x128).
-    //    (Their loop reads a k-tile ahead, which alone is not the faster way for all of them: with no operand for the epilogue
-    //    to fetch and blocks that share a CU, or few k-tiles, the loop of the larger tiles / this is (us) NT 12168x512x128 9.7 /
-    //    10.3, 25088x512x128 17.2 / 18.5, 3136x1024x256 7.4 / 7.9, 12168x256x512 9.3 / 9.6, but 12168x128x512 6.8 / 6.7, and with a
-    //    residual from memory 12168x512x128 16.5 / 13.1.  Split by such a rule no stage gained: 18 images of 26x26, 128 channels
-    //    (us, this / split) 2841 / 2846, 32 of 28x28, 64 channels 3213 / 3220, 384-wide encoders over 3066 rows 3060 / 3081,
-    //    512-wide over 2048 2818 / 2795.  In the third the products that stayed on this loop went from 9.9 to 10.7 us, with the
-    //    same code, as if it had to be fetched again where two kernels alternate.)
+    //  - Problems of at most one tile of 128x64 per CU take those or, NN and long contractions, 64x128 (gemm_m16.h; NT 128x64 / 64x128: 1050x1536x512
+    //    6.6 / 6.6, 12168x128x512 5.3 / 5.3, 2043x768x768 6.5 / 6.2, 2043x768x3072 17.9 / 16.7, 6272x256x1024 8.4 / 7.1); then 128x128 tiles of three
+    //    stages, one per CU, up to a round of them.  64x128 or 128x64, the better / 128x128 (us, more than one of the first per CU): NT with activation
+    //    1200x2048x512 (304) 9.6 / 9.1, 1600x2048x640 (400) 11.5 / 10.6, 3136x1024x256 (392) 8.5 / 8.0, 8112x512x128 (508) 8.2 / 7.9, 4096x1024x192
+    //    (512) 8.6 / 8.2; NN times a tensor 8.1 / 7.7, 9.9 / 8.9, 6.6 / 6.5, 6.0 / 6.0, 6.5 / 6.3; 4096x768x3072 (384) 28.2 / 22.9; within a round
+    //    2043x768x768 (192) 6.2 / 8.2, 2048x1024x1024 (256) 7.3 / 9.6.  A round of 128x128 against 256x128 where a few rows stand against many
+    //    columns: 640x6400x1600 17.3 / 24.1.  More of them: 256x128 tiles, also for short contractions (NT 6272x1024x256
+    //    with activation 12.7, on 128x128 13.5), and 128x64 for what has one to three k-tiles forward, where the launch is its epilogue (NT with activation,
+    //    128x64 / 128x128: 25088x512x128 19.5 / 22.2, 6272x1024x128 11.9 / 12.3), or few columns.
     //    32-wide k-tiles (K % 64 != 0) as before: 128x64 tiles up to 128 tiles of 128x128 and for short forward contractions.
     if (k64) {
-        const int64_t halves = nt ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
-        // (one or two k-tiles forward: whatever their size -- the launch is its epilogue, which many small tiles share out)
-        if ((nt && K < 256) || halves <= (K >= 768 ? 256 : K >= 512 ? 400 : 512)) return nt ? D128x64k64s3 : D64x128k64s3;
-        if (t128 <= 256) return D128x128k64s3;
+        const bool tall = nt && K < 768;
+        const int64_t halves = tall ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
+        const DmaTile half = tall ? D128x64k64s3 : D64x128k64s3;
+        if (halves <= kCUs) return half;
+        if (t128 <= kCUs) return D128x128k64s3;
+        if ((nt && K < 256) || halves <= (K >= 768 ? 256 : K >= 512 ? 400 : 512)) return half;
     } else {
         if ((K <= 512 || t128 <= 128) && nt) return D128x64s3;
         if (t128 <= 128 && nn) return D64x128s3;
@@ -242,10 +235,12 @@ template <bool TA, bool TB, int KW, int BK, int NST> static int launch_bf16_wave
     return BB_OK;
 }
 
-// 64x64 tiles of four waves that are at most half of the CUs' go as two blocks a tile, 32x64 and two waves each (the same bits): a CU has half
-// the LDS reads and transfers to get through in a k-tile.  Whole / halves, device time (us): NN 128x384x128 3.6 / 3.4, 1024x512x512 (128
-// tiles) 4.9 / 4.6, x2048 9.6 / 9.0, 512x768x3072 12.6 / 11.8, 300x1600x1600 8.1 / 7.7; NT 3.7 / 3.6, 4.9 / 4.7, 9.0 / 9.0, 11.9 / 11.6, 7.6 /
-// 7.6; more halves than CUs NN 1050x512x2048 (136 tiles) 9.7 / 11.5, NT 1024x1024x512 (256) 5.1 / 5.9.
+// 64x64 tiles that are at most half of the CUs' go as two blocks a tile, 32x64 and four waves each, of 16x32 (gemm_m16.h; the same bits): a CU has half
+// the LDS reads and transfers to get through in a k-tile.  Before (two waves, 32x32x16 instructions) / now, us: NN 128x256x128 3.3 / 3.0, 1024x512x512 (128
+// tiles) 4.4 / 3.8, x2048 8.8 / 6.9, 512x768x3072 11.6 / 9.0, 300x1600x1600 7.4 / 6.0; NT 3.7 / 3.3, 4.3 / 3.8, 8.6 / 6.8, 11.3 / 8.6, 7.3 / 5.9.  More
+// halves than CUs, 64x64 / halves: NN 1050x512x2048 (136 tiles) 9.1 / 9.3, NT 8.3 / 9.0, 2048x512x512 (256) 4.5 / 4.8.  NT 64x64 tiles have eight
+// waves of 16x32 (four on 32x32x16 / this: 1050x512x512 4.5 / 4.3, x2048 8.5 / 8.3, 1024x1024x512 with activation 5.7 / 5.2, 640x1024x4096
+// 14.8 / 14.8), NN ones four of 32x32 (9.1 / 9.9, 15.9 / 17.0: the four waves of a column each read its k-major fragments, two reads apiece).
 static bool halve_tiles(int M, int N, int64_t batches) { return (int64_t)((M + 31) / 32) * ((N + 63) / 64) * batches <= 256; }
 
 template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, hipStream_t st) {
@@ -275,16 +270,20 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
             if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64, true>(g, batches, st);
             else break;
         case D128x128k64s3:
-            if constexpr (!TA) return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
+            if constexpr (!TA) return launch_bf16_m16<4, 2, 2, 4, 3, TB, true>(g, batches, st);
             else break;
-        case D128x64k64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3, 64>(g, batches, st);
+        case D128x64k64s3:
+            if constexpr (!TA && !TB) return launch_bf16_m16<2, 2, 4, 2, 3, TB, true>(g, batches, st);
+            else break;
         case D128x64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3>(g, batches, st);
-        case D64x128k64s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3, 64>(g, batches, st);
+        case D64x128k64s3:
+            if constexpr (!TA) return launch_bf16_m16<2, 2, 2, 4, 3, TB>(g, batches, st);
+            else break;
         case D64x128s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
         case D64x64k64s4:
             if constexpr (!TA)
-                return halve_tiles(g.M, g.N, batches) ? launch_bf16_dma<32, 64, 1, 2, TA, TB, true, 4, 64>(g, batches, st)
-                                                      : launch_bf16_dma<64, 64, 2, 2, TA, TB, true, 4, 64>(g, batches, st);
+                return halve_tiles(g.M, g.N, batches) ? launch_bf16_m16<1, 2, 2, 2, 4, TB, true>(g, batches, st)
+                       : TB ? launch_bf16_dma<64, 64, 2, 2, TA, true, true, 4, 64>(g, batches, st) : launch_bf16_m16<1, 2, 4, 2, 4, false, true>(g, batches, st);
             else break;
         default: break;
     }

@@ -1,4 +1,4 @@
-// bf16 products on v_mfma_f32_16x16x32_bf16: large tiles of NT and NN products, and of a layer's weight gradients (TN).
+// bf16 products on v_mfma_f32_16x16x32_bf16: NT and NN products on tiles of 256x256 down to 32x64, and large weight gradients (TN).
 //
 // Why this instruction: what bounds a large product is the card's power.  From registers, on normal data, 32x32x16 sustains 1777
 // TFLOP/s and 16x16x32 2030 (on zeros both 2470): per multiplication it moves half the accumulators.  The sums are the same: one
@@ -8,6 +8,16 @@
 // step's fragments the other step's are read into a second register set.  One barrier a k-tile: behind it the k-tile's own stage is
 // read and the next k-tile has landed, so the transfers of the k-tile STAGES further on go into that stage, spread over the matrix
 // instructions that follow.  No branch inside: what changes towards the end of a contraction is done by the loops around the step.
+//
+// Small tiles (at most about a round of them): such a launch waits for its chain of k-tiles, each a few hundred nanoseconds of LDS latency, barrier
+// and transfers with the matrix pipe idle most of the time.  Two things shorten it.  Twice the waves of half the size (16 to 64 rows, 32 columns):
+// a SIMD has another wave to go on with.  And WHOLE: fragments are read a whole k-tile ahead, into a second set of registers for both steps; the
+// barrier at the head of a k-tile then says that everybody holds it (its stage is free) and that the next one has landed.  Device time, us, kernel
+// before (32x32x16, half the waves, a k-tile ahead) / half a k-tile ahead / a whole one: 32x64 tiles NT 1024x512x2048 8.4 / 7.6 / 6.8, x512
+// 4.2 / 4.3 / 3.8, NN 8.8 / 8.5 / 6.9; 64x128 NN 2043x768x3072 17.9 / 16.4 / 17.0, 2048x1024x4096 23.9 / 22.0 / 22.9, NT 25.0 / 21.9 / 23.4; 128x64 NT
+// 1024x2048x512 with activation 8.2 / 7.1 / 6.8; 128x128 with a residual NT 4096x768x3072 25.1 / 24.5 / 24.0, NN 8192x512x2048 21.8 / - / 20.5.
+// Twice the waves on 32x32x16 take half of that (64x128 NN 2043x768x3072 17.4, 2048x1024x4096 23.7); one wave a SIMD half a k-tile ahead is
+// twice as slow (64x128 2043x768x3072 32.3).
 //
 // LDS: rows of a k-contiguous operand are 128 bytes, of a k-major one a k each; 16-byte chunks are swizzled so that the sixteen or
 // thirty-two lanes LDS serves at a time fall on different banks (counted: none conflicts).  The product is made transposed (B times A):
@@ -118,7 +128,7 @@ template <int BR, int T, bool KM, bool PAIRED> struct M16Frags {
 };
 
 // The tile's accumulators, its place in the ring, and the step over one k-tile.
-template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int STAGES> struct M16Loop {
+template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int STAGES, bool WHOLE = false> struct M16Loop {
     static constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16;
     using OpA = M16Lanes<BM, NW, AKM, false>;
     using OpB = M16Lanes<BN, NW, BKM, PAIRED>;
@@ -137,7 +147,9 @@ template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int S
     FragA fa;
     M16Frags<BN, TN, BKM, PAIRED> fb;
     f32x4 acc[TM][TN];
-    bf16x8 a[ROWS ? 1 : 2][TM], b[2][TN];
+    static constexpr int SETS = WHOLE ? 4 : 2;     // one a step of the k-tiles whose fragments are held
+    static_assert(!ROWS || !WHOLE, "one set of rows, half a k-tile ahead");
+    bf16x8 a[ROWS ? 1 : SETS][TM], b[SETS][TN];
     float sum, part;
     int wave, stage, first;
     unsigned lds0;
@@ -160,14 +172,16 @@ template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int S
     __device__ __forceinline__ void feed_all(int t, int live) {
         static_for([&](auto i) { feed<decltype(i)::value>(lds0 + t * STAGE_BYTES, live); }, std::make_integer_sequence<int, LOADS>{});
     }
-    // step ks's fragments in the order of their use
-    template <int Q> __device__ __forceinline__ void read(const unsigned char* st, int ks) {
-        if constexpr (Q == 0) a[ROWS ? 0 : ks][0] = fa.load(st, 0, ks);
-        else if constexpr (Q <= TN) b[ks][Q - 1] = fb.load(st + OpA::BYTES, Q - 1, ks);
-        else a[ROWS ? 0 : ks][Q - TN] = fa.load(st, Q - TN, ks);
+    // step ks's fragments in the order of their use (SET: WHOLE, which k-tile's registers)
+    template <int Q, int SET = 0> __device__ __forceinline__ void read(const unsigned char* st, int ks) {
+        const int s = ROWS ? 0 : 2 * SET + ks;
+        if constexpr (Q == 0) a[s][0] = fa.load(st, 0, ks);
+        else if constexpr (Q <= TN) b[2 * SET + ks][Q - 1] = fb.load(st + OpA::BYTES, Q - 1, ks);
+        else a[s][Q - TN] = fa.load(st, Q - TN, ks);
     }
     __device__ __forceinline__ void read_first() {
-        static_for([&](auto q) { read<decltype(q)::value>(smem + stage * STAGE_BYTES, 0); }, std::make_integer_sequence<int, NF>{});
+        static_for([&](auto q) { read<decltype(q)::value % NF>(smem + stage * STAGE_BYTES, decltype(q)::value / NF); },
+                   std::make_integer_sequence<int, WHOLE ? 2 * NF : NF>{});
     }
     template <int NEWER> __device__ __forceinline__ void landed() {   // all but the NEWER latest k-tiles of this wave; then everybody's
         asm volatile("" ::: "memory");
@@ -226,6 +240,32 @@ template <int TM, int TN, int WM, int WN, bool AKM, bool BKM, bool PAIRED, int S
             },
             std::make_integer_sequence<int, 2 * NM>{});
     }
+    // WHOLE: one k-tile out of the registers SET, the next one's fragments into the others beside three quarters of its products (what is left
+    // covers the last reads), the transfers of the k-tile STAGES on, into this one's stage, beside all of them.  Behind the last k-tile the
+    // reads bring what nothing uses.
+    template <int SET> __device__ __forceinline__ void step_whole(int live) {
+        constexpr int CARRY = 2 * NM - (NM + 1) / 2;
+        const unsigned into = lds0 + stage * STAGE_BYTES;
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+        const unsigned char* nxt = smem + stage * STAGE_BYTES;
+        landed<STAGES - 2>();
+        static_for(
+            [&](auto idx) {
+                constexpr int m = decltype(idx)::value, s = 2 * SET + m / NM, i = m % NM / TN, j = m % TN;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j], a[s][i], acc[i][j], 0, 0, 0);
+                if constexpr (m < CARRY)
+                    static_for(
+                        [&](auto d) {
+                            constexpr int q = 2 * NF * m / CARRY + decltype(d)::value;
+                            read<q % NF, 1 - SET>(nxt, q / NF);
+                        },
+                        std::make_integer_sequence<int, 2 * NF * (m + 1) / CARRY - 2 * NF * m / CARRY>{});
+                static_for([&](auto d) { feed<LOADS * m / (2 * NM) + decltype(d)::value>(into, live); },
+                           std::make_integer_sequence<int, LOADS * (m + 1) / (2 * NM) - LOADS * m / (2 * NM)>{});
+                __builtin_amdgcn_sched_barrier(0);
+            },
+            std::make_integer_sequence<int, 2 * NM>{});
+    }
 };
 
 // the tiles that store fp32, too (larger ones have no registers left for it)
@@ -233,10 +273,10 @@ template <int TM, int TN> constexpr bool kM16F32Out = TM * TN <= 16;
 
 // NT and NN products over whole k-tiles.  A block walks the tiles b, b + gridDim.x, ... (a multiple of 8 apart, so that they stay on its XCD, or
 // one tile a block): the next tile's first k-tiles go out under the last of this one and land under its epilogue.  More than one tile
-// a block needs K >= STAGES * 64: the waits count on a tile's transfers filling the ring.
-template <int TM, int TN, int WM, int WN, bool BKM, int STAGES, bool DROP>
+// a block needs K >= STAGES * 64: the waits count on a tile's transfers filling the ring.  WHOLE: one tile a block.
+template <int TM, int TN, int WM, int WN, bool BKM, int STAGES, bool WHOLE, bool DROP>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_m16_kernel(const GemmArgs g) {
-    using Loop = M16Loop<TM, TN, WM, WN, false, BKM, true, STAGES>;
+    using Loop = M16Loop<TM, TN, WM, WN, false, BKM, true, STAGES, WHOLE>;
     constexpr int BM = Loop::BM, BN = Loop::BN, NP = TN / 2;
     static_assert(TN % 2 == 0, "fragments in pairs");
     constexpr int GROUP_M = BM == 256 && BN < 256 ? 4 : 8;   // (32 tiles of an XCD: 4 x 8 of 256 x 128 read fewer rows than 8 x 4)
@@ -269,14 +309,25 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_m16_kernel(const GemmAr
     for (;;) {
         p.clear();
         p.read_first();
-        for (int kt = STAGES; kt < KT; ++kt) p.step(-1);
-        const int next = tile + G, live = __builtin_amdgcn_readfirstlane((next - total) >> 31);
+        if constexpr (WHOLE) {
+            auto live_at = [&](int kt) { return __builtin_amdgcn_readfirstlane((kt + STAGES - KT) >> 31); };
+            int kt = 0;
+            for (; kt + 1 < KT; kt += 2) {
+                p.template step_whole<0>(live_at(kt));
+                p.template step_whole<1>(live_at(kt + 1));
+            }
+            if (kt < KT) p.template step_whole<0>(0);
+        } else {
+            for (int kt = STAGES; kt < KT; ++kt) p.step(-1);
+        }
+        const int next = tile + G, live = WHOLE ? 0 : __builtin_amdgcn_readfirstlane((next - total) >> 31);
         int next_m = 0, next_n = 0;
         if (live) {
             tile_coords<GROUP_M>(next, g.tiles_m, g.tiles_n, next_m, next_n);
             point_at(next_m, next_n);
         }
-        for (int t = min(KT, STAGES); t > 0; --t) p.step(live);
+        if constexpr (!WHOLE)
+            for (int t = min(KT, STAGES); t > 0; --t) p.step(live);
 
         // Epilogue from the registers: the lane's row of 16 row groups, eight columns of each pair of fragments.  The operand of the kinds
         // that read one is fetched AHEAD row groups before its use, the pieces of a row are made first and stored one behind the

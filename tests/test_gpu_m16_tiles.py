@@ -1,4 +1,4 @@
-"""Products on tiles of 16x16x32 matrix instructions: one and several tiles a block, contractions of fewer, as many and more k-tiles than the
+"""Products on tiles of 16x16x32 matrix instructions, 256x256 down to 32x64: one and several tiles a block, contractions of fewer, as many and more k-tiles than the
 ring has stages, rows and columns off the tile, batches, fp32 outputs -- against fp64, and bit for bit against the same rows in a product of other tiles."""
 import pytest
 import torch
@@ -85,3 +85,34 @@ def test_weight_gradients(hiplib, shapes, K):
             assert ((c[:-1].double() - start - 0.5 * ref).abs() <= slack + 2.0 ** -23 * (ref.abs() + start)).all()
             sums = a.double().sum(0)
             assert ((s.double() - 3.0 - sums).abs() <= K * 2.0 ** -24 * (a.double().abs().sum(0) + 3.0)).all()
+
+
+# small tiles: 32x64 and 64x64, 128x64 (NT below 768) or 64x128, 128x128, with a row, a row group and 8 columns in the last ones; fewer, as many and
+# more k-tiles than the ring has stages, odd and even numbers of them (the registers of a k-tile read ahead change places)
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 832])
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("M,N,tile", [(1, 8, "halves_dma64x64k64s4"), (65, 72, "halves_dma64x64k64s4"), (1033, 520, "dma64x64k64s4"), (2041, 776, None), (4089, 776, "dma128x128k64s3")])
+def test_small_tiles(hiplib, layout, M, N, K, tile):
+    lay = hiplib.NT if layout == "nt" else hiplib.NN
+    A, B = rand(M, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2, scale=0.2)
+    bias, X = rand(N, seed=3), rand(M, N, seed=4)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    C = wide[:M, :N]
+    name = hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C))
+    if K >= 128 or M < 2000:       # (larger problems of a single k-tile take 32-wide ones)
+        assert name == f"bf16_{layout}_{tile or ('dma128x64k64s3' if layout == 'nt' and K < 768 else 'dma64x128k64s3')}"
+    ref, slack = product(A, B.t() if layout == "nt" else B)
+    near = lambda got, want: bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack + 2.0 ** -22 * (ref.abs() + 8.0)).all())
+    hiplib.gemm(lay, A, B, C)
+    assert near(C, ref)
+    hiplib.gemm(lay, A, B, C, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X)
+    assert near(C, ref + bias.double() + X.double())
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
+    F = torch.ones(M, N, device=DEV)
+    hiplib.gemm(lay, A, B, F, accumulate=True, alpha=0.5)
+    assert ((F.double() - 1.0 - 0.5 * ref).abs() <= slack + 2.0 ** -23 * (ref.abs() + 2.0)).all()
+    # two of them in one launch, by strides
+    Cs = torch.zeros(2, M, N, dtype=torch.bfloat16, device=DEV)
+    As, Bs = torch.stack([A, A.flip(0)]), torch.stack([B, B])
+    hiplib.gemm_batched(lay, hiplib.BF16, M, N, K, As.data_ptr(), K, (M * K, 0), Bs.data_ptr(), B.shape[1], (N * K, 0), Cs.data_ptr(), N, (M * N, 0), 2, 1)
+    assert near(Cs[0], ref) and torch.equal(Cs[0], Cs[1].flip(0))
