@@ -88,10 +88,10 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
 
 // DMA kernels need at least one full vector of rows, and but for weight gradients and D128x128k64r K % 32 == 0; tile by problem size
 enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, D256x128k64s3, D128x128k64, D128x64k64s3, D128x64s3,
-               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3 };
+               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3, D64x128k64s5 };
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
-                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3"};
+                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3", "dma64x128k64s5"};
 // The kernel of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
 // what ran before): a redundant forward and a normal forward of the same layer give the same bits.  All tiles below add up
 // a contraction in the same order; the wave-sliced kernels (pick_wave) in another.
@@ -130,7 +130,8 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
     //  - Problems of at most one tile of 128x64 per CU take those or, NN and long contractions, 64x128 (gemm_m16.h; NT 128x64 / 64x128: 1050x1536x512
-    //    6.6 / 6.6, 12168x128x512 5.3 / 5.3, 2043x768x768 6.5 / 6.2, 2043x768x3072 17.9 / 16.7, 6272x256x1024 8.4 / 7.1); then 128x128 tiles of three
+    //    6.6 / 6.6, 12168x128x512 5.3 / 5.3, 2043x768x768 6.5 / 6.2, 2043x768x3072 17.9 / 16.7, 6272x256x1024 8.4 / 7.1; there five stages and fragments a whole k-tile ahead, forward, K 1024 7.1 / 7.3, with a
+    //    residual 1200x1600x1600 11.4 / 11.1, 3000x448x1792 11.8 / 11.0, 2043x768x3072 17.6 / 16.6, 2048x1024x4096 22.7 / 22.1, NN 22.8 / 23.2); then 128x128 tiles of three
     //    stages, one per CU, up to a round of them.  64x128 or 128x64, the better / 128x128 (us, more than one of the first per CU): NT with activation
     //    1200x2048x512 (304) 9.6 / 9.1, 1600x2048x640 (400) 11.5 / 10.6, 3136x1024x256 (392) 8.5 / 8.0, 8112x512x128 (508) 8.2 / 7.9, 4096x1024x192
     //    (512) 8.6 / 8.2; NN times a tensor 8.1 / 7.7, 9.9 / 8.9, 6.6 / 6.5, 6.0 / 6.0, 6.5 / 6.3; 4096x768x3072 (384) 28.2 / 22.9; within a round
@@ -142,7 +143,7 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     if (k64) {
         const bool tall = nt && K < 768;
         const int64_t halves = tall ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
-        const DmaTile half = tall ? D128x64k64s3 : D64x128k64s3;
+        const DmaTile half = tall ? D128x64k64s3 : nt && K >= 1536 ? D64x128k64s5 : D64x128k64s3;
         if (halves <= kCUs) return half;
         if (t128 <= kCUs) return D128x128k64s3;
         if ((nt && K < 256) || halves <= (K >= 768 ? 256 : K >= 512 ? 400 : 512)) return half;
@@ -278,6 +279,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
         case D128x64s3: return launch_bf16_dma<128, 64, 4, 1, TA, TB, true, 3>(g, batches, st);
         case D64x128k64s3:
             if constexpr (!TA) return launch_bf16_m16<2, 2, 2, 4, 3, TB>(g, batches, st);
+            else break;
+        case D64x128k64s5:
+            if constexpr (!TA && !TB) return launch_bf16_m16<2, 2, 2, 4, 5, TB, true>(g, batches, st);
             else break;
         case D64x128s3: return launch_bf16_dma<64, 128, 2, 2, TA, TB, true, 3>(g, batches, st);
         case D64x64k64s4:

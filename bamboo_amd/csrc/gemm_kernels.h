@@ -820,7 +820,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
 
     // Transposed products (B times A) where the epilogue takes the accumulators as they are: a lane then has a row of C, four
     // neighbouring columns in four registers.  The kernels with column statistics keep a column per lane.
-    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && (TM * TN <= 2 || (BM * BN <= 128 * 128 && STATS == 0 && CONV == 0)) && !AKM && !RAGK && !VIS;
+    constexpr bool AHEAD = BK == 64 && STAGES >= 3 && TM * TN <= 2 && !AKM && !RAGK && !VIS;
     constexpr bool DIRECT = STATS == 0 && AHEAD;
     auto mfma = [](const bf16x8& a, const bf16x8& b, const f32x16& c) {
         return DIRECT ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -952,10 +952,9 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
 
     // DIRECT: the lane's row and first column of the wave's tiles; of a 32x32 tile it finishes columns 16 h .. 16 h + 7 (h = 0, 1; the
     // lane 32 further on the eight behind them).  What the epilogue reads beside the product -- the bias, the operand of the
-    // kinds that have one -- is fetched in one go, clamped to the matrix (what lies outside is not stored): behind the first
-    // transfers where the registers are there, else at the loop's end, the first tile's operand under the last k-tile.
+    // kinds that have one -- is fetched in one go, clamped to the matrix (what lies outside is not stored), behind the first
+    // transfers.
     constexpr int TILES = TM * TN;
-    constexpr bool BEFORE = DIRECT && AHEAD && TILES <= 2;
     const int drow = m0 + wm * WTM + (lane & 31), dcol = n0 + wn * WTN + 8 * (lane >> 5);
     u32x4 dop[DIRECT ? TILES : 1][2], dbias[DIRECT ? TN : 1][2];
     auto fetch_bias = [&]() {
@@ -1054,9 +1053,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         // are masked off (as branches around them the same loop was slower than the one below, 100x1600x6400 42 us: accumulators moved
         // between register sets at every merge).  Before (halves of a k-tile read half a k-tile ahead) and now, us: 64x64 tiles, NT
         // 1024x512x2048 11.7 / 9.5, 512x1024x4096 20.0 / 15.7, 100x1600x6400 29.1 / 21.3, 0.25 -> 0.17 us a k-tile, where LDS moves
-        // 32 KB of fragments and 16 KB of transfers; 128x64 and 64x128 gain by the epilogue's early operands: 2043x768x768 with a
-        // residual 8.6 / 7.8, x3072 21.2 / 20.2 (NT), 21.0 / 19.4 (NN).  128x128 tiles, one a CU with three stages: the loop below with
-        // two blocks a CU 26.2, this one 21.1 (NT 8192x512x2048).
+        // 32 KB of fragments and 16 KB of transfers.  (Plain products that run here: NN on 64x64 tiles; the others are in gemm_m16.h.)
         struct Tile {
             bf16x8 a[4][TM], b[4][TN];
         } t0, t1;
@@ -1105,7 +1102,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         // (behind the transfers: the waits below count those that are newer than the one waited for, more of them do no harm)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (BEFORE) {
+        if constexpr (DIRECT) {
             fetch_bias();
             fetch_operand(std::integral_constant<int, 0>{}, std::integral_constant<int, TILES>{});
         }
@@ -1279,11 +1276,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmArgs& g, const int 
         // tiles.  (Before, every wave parked pairs of tiles in LDS and read them back by rows of eight lanes, with the branches in every
         // one of four passes: about 2600 cycles for the single 32x32 tile a wave has in the 64x64 kernels, a third of what a
         // product of two k-tiles takes there.)  Back to back with the shorter way to the first transfer, before / now (us): NT
-        // 128x128x128 4.1 / 3.2, 1050x512x512 5.4 / 4.4, 1050x512x2048 9.6 / 8.3; 128x64 tiles 1024x1536x512 7.4 / 6.4.
-        if constexpr (!BEFORE) {
-            fetch_bias();
-            fetch_operand(std::integral_constant<int, 0>{}, std::integral_constant<int, TILES>{});
-        }
+        // 128x128x128 4.1 / 3.2, 1050x512x512 5.4 / 4.4, 1050x512x2048 9.6 / 8.3.
         wait_vmcnt_lgkm0<0>();  // the tiles issued past the end of K have to land before the block's LDS is another's
         // accumulators of columns 16 h .. 16 h + 15 of a tile -> the lane's eight
         auto columns = [&](const f32x16& c, auto h_c, float (&v)[8]) {

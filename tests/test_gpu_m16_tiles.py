@@ -87,9 +87,9 @@ def test_weight_gradients(hiplib, shapes, K):
             assert ((s.double() - 3.0 - sums).abs() <= K * 2.0 ** -24 * (a.double().abs().sum(0) + 3.0)).all()
 
 
-# small tiles: 32x64 and 64x64, 128x64 (NT below 768) or 64x128, 128x128, with a row, a row group and 8 columns in the last ones; fewer, as many and
+# small tiles: 32x64 and 64x64, 128x64 (NT below 768) or 64x128 (NT from 1536 on another kernel), 128x128, with a row, a row group and 8 columns in the last ones; fewer, as many and
 # more k-tiles than the ring has stages, odd and even numbers of them (the registers of a k-tile read ahead change places)
-@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 832])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 832, 1600, 1664])
 @pytest.mark.parametrize("layout", ["nt", "nn"])
 @pytest.mark.parametrize("M,N,tile", [(1, 8, "halves_dma64x64k64s4"), (65, 72, "halves_dma64x64k64s4"), (1033, 520, "dma64x64k64s4"), (2041, 776, None), (4089, 776, "dma128x128k64s3")])
 def test_small_tiles(hiplib, layout, M, N, K, tile):
@@ -100,7 +100,7 @@ def test_small_tiles(hiplib, layout, M, N, K, tile):
     C = wide[:M, :N]
     name = hiplib.gemm_variant(hiplib.gemm_desc(lay, A, B, C))
     if K >= 128 or M < 2000:       # (larger problems of a single k-tile take 32-wide ones)
-        assert name == f"bf16_{layout}_{tile or ('dma128x64k64s3' if layout == 'nt' and K < 768 else 'dma64x128k64s3')}"
+        assert name == f"bf16_{layout}_{tile or ('dma64x128k64s3' if layout == 'nn' or 768 <= K < 1536 else 'dma128x64k64s3' if K < 768 else 'dma64x128k64s5')}"
     ref, slack = product(A, B.t() if layout == "nt" else B)
     near = lambda got, want: bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack + 2.0 ** -22 * (ref.abs() + 8.0)).all())
     hiplib.gemm(lay, A, B, C)
