@@ -7,7 +7,7 @@
 // instructions (2-norm against 64 bits, K 64 / 768 / 3072 / 8192: 4.9e-8, 1.6e-7, 3.4e-7, 5.7e-7 against 1.5e-7, 3.5e-7, 7.0e-7, 1.15e-6).
 //
 // What that cannot do is found in the result: a value that is not finite, or larger than the largest bf16, makes its row or column of the tile
-// not finite.  A wave that finds one such sum makes its part of the tile again, in plain fp32 multiply-adds.
+// not finite.  A wave that finds one such sum makes its part of the tile again, on fp32 instructions (pieces_again).
 //
 // What bounds it: of large problems the card's power; of smaller ones what the waves issue: beside every matrix instruction about two for the
 // splitting (an instruction is free beside the first 16 cycles' two), LDS' write path (64 bytes a cycle) and the waits at the barrier.
@@ -72,6 +72,63 @@ template <int BR, int T, bool KM> struct PiecesFrags {
         else return *(const bf16x8*)(plane + off + t * 1024);
     }
 };
+
+// A wave's part of a tile on fp32 instructions, from memory.  A lane holds four k of a row of A, and of a row (BKM: column) of B: 16 k
+// are four instructions.  What bounds it is the latency of its loads, 16 k ahead of their use; nothing is staged: sixteen lanes read 16 lines
+// (k-major: one), and the waves of a row or column of waves the same ones.  The whole product, us, all values finite / one NaN in A / all NaN (one
+// element's multiply-adds a lane before): NT 2048x3072x768 66 / 108 (887) / 215 (3391), NN 2048x768x3072 78 / 183 (1985) / 251 (3594), a weight
+// gradient 3072x768x2048 79 / 223 (3070) / 308 (4369); the fp32 kernels 85, 85 and 102 on any values.
+template <bool KM> __device__ __forceinline__ f32x4 pieces_four(const float* p, int64_t ld, int k, int K) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!KM) {
+        if (k < K) v = *(const f32x4*)(p + k);       // (whole fours: a k-contiguous operand has K % 4 == 0)
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (k + e < K) v[e] = p[(int64_t)(k + e) * ld];
+    }
+    return v;
+}
+template <int TM, int TN, bool AKM, bool BKM> __device__ __forceinline__ void pieces_again(const GemmArgs& g, int row0, int col0, int lane, f32x4 (&acc)[TM][TN]) {
+    const float *A[TM], *B[TN];
+    f32x4 a[2][TM], b[2][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = min(row0 + i * 16 + (lane & 15), g.M - 1);
+        A[i] = (const float*)g.A + (AKM ? m : (int64_t)m * g.lda);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int n = min(col0 + j * 16 + (lane & 15), g.N - 1);
+        B[j] = (const float*)g.B + (BKM ? n : (int64_t)n * g.ldb);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](int s, int k) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[s][i] = pieces_four<AKM>(A[i], g.lda, k, g.K);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[s][j] = pieces_four<BKM>(B[j], g.ldb, k, g.K);
+    };
+    auto add = [&](int s) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[s][j][e], a[s][i][e], acc[i][j], 0, 0, 0);
+    };
+    int k = 4 * (lane >> 4);
+    fetch(0, k);
+    for (int left = g.K; left > 0; left -= 32, k += 32) {
+        fetch(1, k + 16);
+        add(0);
+        fetch(0, k + 32);
+        add(1);
+    }
+}
 
 // four neighbouring elements of a row of C; the epilogue of epilogue_f32
 __device__ __forceinline__ void pieces_epilogue(const GemmArgs& g, int m, int n, f32x4 v) {
@@ -266,7 +323,7 @@ __device__ __forceinline__ void gemm_f32_pieces_body(const GemmArgs& g, const in
 #pragma unroll
             for (int e = 0; e < 4; ++e) finite = finite && fabsf(large[i][j][e]) < __builtin_inff();
         }
-    const bool again = __any(!finite);
+    if (__any(!finite)) pieces_again<TM, TN, AKM, BKM>(g, m0 + wave / WN * (TM * 16), n0 + wave % WN * (TN * 16), lane, large);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         const int m = row + i * 16;
@@ -274,20 +331,7 @@ __device__ __forceinline__ void gemm_f32_pieces_body(const GemmArgs& g, const in
         for (int j = 0; j < TN; ++j) {
             const int n = col + j * 16;
             if (m >= g.M || n >= g.N) continue;
-            f32x4 v = large[i][j];
-            if (again) {
-                const float* A = (const float*)g.A + (AKM ? m : (int64_t)m * g.lda);
-                const float* B = (const float*)g.B + (BKM ? n : (int64_t)n * g.ldb);
-                v = f32x4{0.f, 0.f, 0.f, 0.f};
-                for (int k = 0; k < g.K; ++k) {
-                    const float x = *A;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = fmaf(x, B[BKM ? e : e * g.ldb], v[e]);
-                    A += AKM ? g.lda : 1;
-                    B += BKM ? g.ldb : 1;
-                }
-            }
-            pieces_epilogue(g, m, n, v);
+            pieces_epilogue(g, m, n, large[i][j]);
         }
     }
 }

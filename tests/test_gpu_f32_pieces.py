@@ -107,3 +107,29 @@ def test_grouped_weight_gradients(hiplib):
         assert ((outs[0][0][i].double() - ref).abs() <= (R + 3) * 2.0 ** -24 * size).all()
         assert off(outs[0][0][i], ref) < off(outs[1][0][i], ref)       # (the pieces were taken)
         assert torch.equal(outs[0][1][i], outs[1][1][i])
+
+
+@pytest.mark.parametrize("layout,M,N,K", [("nt", 2048, 3072, 768), ("nn", 2048, 768, 3072), ("tn", 3072, 768, 2048)])
+def test_time_of_values_that_bf16_does_not_hold(hiplib, layout, M, N, K):
+    """A product that is made again costs the fp32 instructions' time beside its own, not a multiple: all of it (a diverged step), or what one row
+    spoils.  (Measured: at most 3 times; 6 leaves room for a slow clock.)"""
+    lay = getattr(hiplib, layout.upper())
+    a, b, _, _ = operands(layout, M, N, K)
+    C = torch.empty(M, N, device=DEV)
+    one, every = a.clone(), torch.full_like(a, float("nan"))
+    one[3, 5] = float("nan")
+
+    def least(x):
+        times = []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                hiplib.gemm(lay, x, b, C, pieces=True)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    finite = least(a)
+    assert least(one) <= 6 * finite and least(every) <= 6 * finite
