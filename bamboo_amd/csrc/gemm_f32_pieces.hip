@@ -2,12 +2,20 @@
 //
 // Why: fp32 matrix instructions do 157 TFLOP/s, bf16 ones 2500, and six of these make one fp32 product: x = x0 + x1 + x2 exactly
 // (three times eight bits, each piece the nearest bf16 of what the ones before leave), and of the nine products of two such sums the three of
-// x1 y2, x2 y1 and x2 y2 are below 2^-24 of x y and left out.  x0 y0 has an accumulator of its own, the five small ones share another:
-// the large sum is rounded once per instruction instead of once per k, so that the result is nearer to the exact one than that of the fp32
-// instructions (2-norm against 64 bits, K 64 / 768 / 3072 / 8192: 4.9e-8, 1.6e-7, 3.4e-7, 5.7e-7 against 1.5e-7, 3.5e-7, 7.0e-7, 1.15e-6).
+// x1 y2, x2 y1 and x2 y2 are below 2^-24 of x y and left out.  (G. Henry, P. Tang, A. Heinecke: Leveraging the bfloat16 Artificial Intelligence
+// Datatype For Higher-Precision Computations, ARITH 2019.)  x0 y0 has an accumulator of its own, the five small ones share another: the large sum is
+// rounded once per instruction instead of once per k, so that the result is nearer to the exact one than that of the fp32 instructions (2-norm
+// against 64 bits, K 64 / 768 / 3072 / 8192: 4.9e-8, 1.6e-7, 3.4e-7, 5.7e-7 against 1.5e-7, 3.5e-7, 7.0e-7, 1.15e-6; values of one, 20 and 40
+// octaves in either operand, K 772: 1.6e-7, 1.9e-7, 1.6e-7 against 3.5e-7, 2.9e-7, 1.6e-7).  Beyond that the instruction's way of adding shows: it drops, towards
+// minus infinity, what lies below the last bit of its largest addend (80 octaves: 1.3e-7 against 1.2e-7).
 //
-// What that cannot do is found in the result: a value that is not finite, or larger than the largest bf16, makes its row or column of the tile
-// not finite.  A wave that finds one such sum makes its part of the tile again, on fp32 instructions (pieces_again).
+// Range: a last piece lies up to 23 bits below its value, and bf16 has nothing below 2^-133.  So values are taken times 2^16: the last bit of the
+// smallest, 2^-149, is then a bf16, and every fp32 value the sum of its pieces (the instruction keeps subnormals); the sums carry 2^32, taken out of
+// the result.  Without that, normal values of 2^-120 lose eleven bits (2-norm 3.5e-5).  It costs two of thirteen instructions of a pair's splitting,
+// 2.5 % of a product.
+//
+// What leaves the range at its upper end -- values from 2^112, sums from 2^96 on, infinities, NaN -- is found in the result: it makes its row or column
+// of the tile, or the one sum, not finite.  A wave that finds such a sum makes its part of the tile again, on fp32 instructions (pieces_again).
 //
 // What bounds it: of large problems the card's power; of smaller ones what the waves issue: beside every matrix instruction about two for the
 // splitting (an instruction is free beside the first 16 cycles' two), LDS' write path (64 bytes a cycle) and the waits at the barrier.
@@ -19,6 +27,7 @@
 #include "gemm_f32_pieces.h"
 #include "gemm_m16.h"
 
+constexpr float kPiecesScale = 65536.f;     // of either operand, see above
 // chunk swizzle of 64-byte rows by the row: 0, 2, 3, 1 by its block of four
 __device__ __forceinline__ int pieces_row_swizzle(int r) { return ((r >> 1) & 2) ^ ((r >> 3) & 1) * 3; }
 // A thread's share of one operand tile, BR rows (columns of a k-major operand) x 32 k: fours of neighbouring values, neighbouring lanes next to
@@ -73,11 +82,12 @@ template <int BR, int T, bool KM> struct PiecesFrags {
     }
 };
 
-// A wave's part of a tile on fp32 instructions, from memory.  A lane holds four k of a row of A, and of a row (BKM: column) of B: 16 k
-// are four instructions.  What bounds it is the latency of its loads, 16 k ahead of their use; nothing is staged: sixteen lanes read 16 lines
-// (k-major: one), and the waves of a row or column of waves the same ones.  The whole product, us, all values finite / one NaN in A / all NaN (one
-// element's multiply-adds a lane before): NT 2048x3072x768 66 / 108 (887) / 215 (3391), NN 2048x768x3072 78 / 183 (1985) / 251 (3594), a weight
-// gradient 3072x768x2048 79 / 223 (3070) / 308 (4369); the fp32 kernels 85, 85 and 102 on any values.
+// A wave's part of a tile on fp32 instructions, from memory.  A lane holds four k of a row of A, and of a row (BKM: column) of B: 16 k are four
+// instructions; the even and the odd sixteens have a sum each, as where two groups share a contraction (gemm_f32.h).  What bounds it is the latency
+// of its loads, 16 k ahead of their use; nothing is staged: sixteen lanes read 16 lines (k-major: one), and the waves of a row or column of waves
+// the same ones.  The whole product, us, all values finite / one NaN in A / all NaN (before, one element's multiply-adds a lane): NT 2048x3072x768
+// 66 / 108 (887) / 215 (3391), NN 2048x768x3072 78 / 183 (1985) / 251 (3594), a weight gradient 3072x768x2048 79 / 223 (3070) / 308 (4369); the
+// fp32 kernels 85, 85 and 102 on any values.
 template <bool KM> __device__ __forceinline__ f32x4 pieces_four(const float* p, int64_t ld, int k, int K) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if constexpr (!KM) {
@@ -89,7 +99,7 @@ template <bool KM> __device__ __forceinline__ f32x4 pieces_four(const float* p, 
     }
     return v;
 }
-template <int TM, int TN, bool AKM, bool BKM> __device__ __forceinline__ void pieces_again(const GemmArgs& g, int row0, int col0, int lane, f32x4 (&acc)[TM][TN]) {
+template <int TM, int TN, bool AKM, bool BKM> __device__ __forceinline__ void pieces_again(const GemmArgs& g, int row0, int col0, int lane, f32x4 (&acc)[TM][TN], f32x4 (&odd)[TM][TN]) {
     const float *A[TM], *B[TN];
     f32x4 a[2][TM], b[2][TN];
 #pragma unroll
@@ -105,29 +115,33 @@ template <int TM, int TN, bool AKM, bool BKM> __device__ __forceinline__ void pi
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TN; ++j) acc[i][j] = odd[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto fetch = [&](int s, int k) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) a[s][i] = pieces_four<AKM>(A[i], g.lda, k, g.K);
 #pragma unroll
         for (int j = 0; j < TN; ++j) b[s][j] = pieces_four<BKM>(B[j], g.ldb, k, g.K);
     };
-    auto add = [&](int s) {
+    auto add = [&](int s, f32x4 (&to)[TM][TN]) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[s][j][e], a[s][i][e], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TN; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[s][j][e], a[s][i][e], to[i][j], 0, 0, 0);
     };
     int k = 4 * (lane >> 4);
     fetch(0, k);
     for (int left = g.K; left > 0; left -= 32, k += 32) {
         fetch(1, k + 16);
-        add(0);
+        add(0, acc);
         fetch(0, k + 32);
-        add(1);
+        add(1, odd);
     }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += odd[i][j];
 }
 
 // four neighbouring elements of a row of C; the epilogue of epilogue_f32
@@ -182,7 +196,7 @@ __device__ __forceinline__ void gemm_f32_pieces_body(const GemmArgs& g, const in
     constexpr int NT = WM * WN * 64, BM = WM * TM * 16, BN = WN * TN * 16;
     using OpA = PiecesOperand<BM, NT, AKM>;
     using OpB = PiecesOperand<BN, NT, BKM>;
-    constexpr int STAGE = OpA::BYTES + OpB::BYTES, PARTS = (OpA::FOURS + OpB::FOURS) * 14, NM = TM * TN * 6, AHEAD = 4;
+    constexpr int STAGE = OpA::BYTES + OpB::BYTES, PARTS = (OpA::FOURS + OpB::FOURS) * 16, NM = TM * TN * 6, AHEAD = 4;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tm, tn;
@@ -216,21 +230,24 @@ __device__ __forceinline__ void gemm_f32_pieces_body(const GemmArgs& g, const in
         if constexpr (I == LOADS - 1) left -= 32;
     };
     auto load_all = [&](Held& h) { static_for([&](auto i) { load(i, h); }, std::make_integer_sequence<int, LOADS>{}); };
-    // The pieces of a pair of values are made in seven parts of one or two instructions (nearest bf16; the same as fp32; what they leave; again; the
-    // upper halves of what those leave), two pairs in turn; a plane's pieces of a four go into the stage when it is whole.  A k-tile's parts are
+    // The pieces of a pair of values are made in eight parts of one or two instructions (times kPiecesScale; nearest bf16; the same as fp32; what they
+    // leave; again; the upper halves of what those leave), two pairs in turn; a plane's pieces of a four go into the stage when it is whole.  A k-tile's parts are
     // spread evenly over NM slots, a matrix instruction each: two vector instructions beside one cost it nothing, more four cycles each.
     // (v_dot2_f32_bf16 would make two parts one, but waits for the matrix pipe: 17 cycles.)
     typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
     u32x2 made[3];
     float near[2][2];
     auto part = [&](auto n_c, Held& h, unsigned char* st) {
-        constexpr int N = decltype(n_c)::value, Q = N / 14 * 2 + N % 2, at = N % 14 / 2, p = at / 3, c = Q / 2, q = Q % 2, e = q * 2;
+        constexpr int N = decltype(n_c)::value, Q = N / 16 * 2 + N % 2, at = N % 16 / 2 - 1, p = at / 3, c = Q / 2, q = Q % 2, e = q * 2;
         constexpr bool OF_A = c < OpA::FOURS;
         auto& v = [&]() -> auto& {
             if constexpr (OF_A) return h.a[c];
             else return h.b[c - OpA::FOURS];
         }();
-        if constexpr (at % 3 == 1) {
+        if constexpr (at < 0) {
+            v[e] *= kPiecesScale;
+            v[e + 1] *= kPiecesScale;
+        } else if constexpr (at % 3 == 1) {
             near[Q % 2][0] = __uint_as_float(made[p][q] << 16);
             near[Q % 2][1] = __uint_as_float(made[p][q] & 0xffff0000u);
         } else if constexpr (at % 3 == 2) {
@@ -323,7 +340,9 @@ __device__ __forceinline__ void gemm_f32_pieces_body(const GemmArgs& g, const in
 #pragma unroll
             for (int e = 0; e < 4; ++e) finite = finite && fabsf(large[i][j][e]) < __builtin_inff();
         }
-    if (__any(!finite)) pieces_again<TM, TN, AKM, BKM>(g, m0 + wave / WN * (TM * 16), n0 + wave % WN * (TN * 16), lane, large);
+    const bool again = __any(!finite);
+    const float unscale = again ? 1.f : 1.f / (kPiecesScale * kPiecesScale);
+    if (again) pieces_again<TM, TN, AKM, BKM>(g, m0 + wave / WN * (TM * 16), n0 + wave % WN * (TN * 16), lane, large, small);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         const int m = row + i * 16;
@@ -331,7 +350,7 @@ __device__ __forceinline__ void gemm_f32_pieces_body(const GemmArgs& g, const in
         for (int j = 0; j < TN; ++j) {
             const int n = col + j * 16;
             if (m >= g.M || n >= g.N) continue;
-            pieces_epilogue(g, m, n, large[i][j]);
+            pieces_epilogue(g, m, n, large[i][j] * unscale);
         }
     }
 }

@@ -49,6 +49,31 @@ def test_products(hiplib, layout, M, N, K, tile):
     assert ((F.double() - 1.0 - 0.5 * ref).abs() <= K * 2.0 ** -24 * size + 2.0 ** -23 * (ref.abs() + 2.0)).all()
 
 
+@pytest.mark.parametrize("layout,M,N,K,tile", CASES[:5])
+@pytest.mark.parametrize("of_a,of_b", [((-126, -112), (40, 60)), ((50, 60), (-126, -120)), ((-149, -126), (60, 80)), ((-70, -55), (-70, -60)), ((-126, 60), (-20, 20)),
+                                       ((44, 49), (44, 49)), ((100, 115), (-30, 0))])
+def test_powers_of_two(hiplib, layout, M, N, K, tile, of_a, of_b):
+    """Values of every size fp32 has, the smallest ones and subnormals (against large ones) among them: within the bound of test_products, no further from fp64
+    than the fp32 instructions, also where the scaled sums leave fp32's range and are made again."""
+    lay = getattr(hiplib, layout.upper())
+    a, b, _, _ = operands(layout, M, N, K)
+    for x, (lo, hi), seed in ((a, of_a, 11), (b, of_b, 12)):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        x.copy_(x.double() * 2.0 ** torch.randint(lo, hi + 1, x.shape, generator=g, device=DEV).double())
+    a64, b64 = (a.double().t() if layout == "tn" else a.double()).contiguous(), (b.double().t() if layout == "nt" else b.double()).contiguous()
+    C, F = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    hiplib.gemm(lay, a, b, C, pieces=True)
+    hiplib.gemm(lay, a, b, F)
+    ref, size = a64 @ b64, a64.abs() @ b64.abs()
+    # (a product or sum below 2^-126 is rounded to a multiple of 2^-149 by either)
+    assert ((C.double() - ref).abs() <= (K + 3) * (2.0 ** -24 * size + 2.0 ** -150)).all()
+    # Values of up to 20 octaves in either operand: no further from fp64 than the fp32 instructions.  1 %: where all is made again it is the same arithmetic in
+    # another order.  (Of many more, one product is most of a sum, which fp32 then rounds once, and the bf16 instruction drops what lies below the
+    # last bit of the largest of its addends: up to a quarter further off than fp32, within the bound above.)
+    if max(of_a[1] - of_a[0], of_b[1] - of_b[0]) <= 23:
+        assert off(C, ref) <= 1.01 * off(F, ref)
+
+
 @pytest.mark.parametrize("layout,M,N,K,tile", CASES[:4])
 def test_epilogues(hiplib, layout, M, N, K, tile):
     """Against the same epilogue on the fp32 instructions: both products lie within the bound of test_products of the exact one, and what is
