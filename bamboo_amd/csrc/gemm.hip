@@ -308,13 +308,8 @@ static bool pick_f32_wave(int M, int N, int K, int64_t batches, int layout) {
     if (layout == BB_NT && batches == 1) return false;
     return K <= kF32WaveK && tiles <= (layout == BB_TN && batches == 1 ? 256 : 1024);
 }
-// Longer fp32 contractions: problems with fewer than two 64x64 tiles per CU and at least 16 k-tiles take 64x32 tiles whose contraction two groups of
-// two waves share: twice the tiles to deal to the CUs, each wave's chain of matrix instructions as long as before.  NT and NN
-// only: the weight gradients (TN) of a layer share a grouped launch.
+// problems of longer contractions on shared ones, see pick_f32_split
 static constexpr int kF32SplitGroups = 2, kF32SplitBN = 32;
-static bool pick_f32_split(int M, int N, int K, int64_t batches, int layout) {
-    return layout != BB_TN && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batches < 2 * 256 && K >= 512;
-}
 // Of what is left for the tiles of 64x64 and 64x32, problems of at most 128 64x64 tiles take four blocks a tile instead, with the
 // same bits (gemm_f32_quarter_kernel): until then every CU has at most two of them.  Larger tiles / this (us, back to back): NT
 // 128x128x128 7.0 / 5.2, 512x512x256 (64 tiles) 10.7 / 5.8, 1000x448x448 (112) 16.3 / 10.2, 1024x512x512 (128) 11.2 / 11.4,

@@ -368,19 +368,38 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f32_pieces_grouped_kernel(co
     gemm_f32_pieces_body<TM, TN, WM, WN, true, true>(G.p[pi], id - G.first_block[pi], true);
 }
 
-// All of a launch's problems, or one of any layout.  By an estimate of both ways: a tile's rounds (one a CU) of K / 32 steps, against the fp32
-// instructions at their rate, or the chain of one tile's.  fp32 / 128x128 / 128x64 (us, back to back; the one taken marked):
-//     NT 2048x3072x768 88 / 63* / 65   2048x768x768 25* / 30 / 21*   2048x768x3072 84 / 99 / 70*   2048x1024x256 14.1 / 14.5 / 11.0*
-//        2048x256x1024 16* / 36 / 26   512x512x512 8* / 21 / 15      4096x4096x4096 990 / 630* / 800
-//     NN 2048x3072x768 78 / 63* / 66   2048x768x3072 82 / 101 / 73*  2048x768x2304 62 / 77 / 56*
+// All of a launch's problems, or one of any layout.  By an estimate of both ways, operands and outputs not in the caches.  Pieces: rounds (one tile a
+// CU) of K steps, and K steps by the share of the CUs that have a tile.  fp32 instructions: K steps of the fullest CU by how many 64x64 (64x32,
+// pick_f32_split) tiles it has, four of which run at a time, one alone at two thirds of their rate.  Fitted to 2900 products (100..8000 rows, 64..6400
+// columns, K 32..4096) and the weight gradients of 3500 layers and 900 single ones; the estimates are off by 10, 5 and 4 % (2-norm), which is what the
+// lines (a launch of few k-tiles is its epilogue: 5 %) allow for.  Where both tiles come out alike it is 128x128: 128x64 split A's values twice as often, which
+// other work on the CUs feels (a stage of 2048x2304x768 and 2048x3072x768 products, two streams: 15.5 and 16.9 ms).  Of the products two in
+// a thousand are more than 3 % slower on pieces than on fp32 instructions, at most 12 %, of the weight gradients none more than 5 %; the line before, by
+// flops, had 45 and 75 in a thousand, up to 27 and 30 %.
+// us, fp32 / 128x128 / 128x64 (the one taken marked; - what the line before took and this does not):
+//     NT 2048x3072x768 88 / 63* / 65   2048x768x768 25 / 30 / 21*   2048x768x3072 84 / 99 / 70*   2048x1024x256 14.1 / 14.5 / 11.0*
+//        2048x256x1024 16* / 36 / 26   512x512x512 8* / 21 / 15      4096x4096x4096 990 / 630* / 800   2048x2304x768 75.3 / 69.0* / 67.8
+//     NN 2048x3072x768 78 / 63* / 66   2048x768x3072 82 / 101 / 73*  2048x768x2304 62 / 77 / 56*   1305x1536x384 20.0* / 23.4- / 21.0
 //     a layer's weight gradients, hidden size (x 4) and rows: 768 2048 232 / 166* / 215, 512 68 / 56* / 70; 1024 2048 390 / 268* / 339; 1600 2048
-//        955 / 700* / 867; 512 513 37 / 31* / 38; 256 2048 47* / 77 / 55
+//        955 / 700* / 867; 576 1077 88* / 109-, 2697 192* / 229-; 832 256 57* / 70-; 256 2048 47* / 77 / 55
 // Large ones are 1300 TFLOP/s of bf16 on ordinary data, two thirds of what the instruction sustains from registers.  Tried: 64x64 accumulators a wave
 // (768x3072 135, 4096 720), 64x64 tiles (76; 840), two blocks a CU of 128x64 (128 registers: 74), all values of a k-tile split at once (4096 690).
 PiecesTile pick_pieces(const bb_gemm_desc* descs, int count) {
-    double flops = 0.0;
-    int64_t tiles[2] = {0, 0};
+    struct Estimate {
+        double base, outputs, full, first[5], after[5], split[5];     // fp32: us, us per 10^6 outputs; us a k of four tiles, of up to four, of as many behind fours
+        struct {
+            double base, outputs, round, step, more, share;           // (more: a k of several rounds)
+        } tile[2];                                                    // 128x128, 128x64
+    };
+    static const Estimate products = {4.0, 1.15, 0.0563, {0, 0.0215, 0.0343, 0.0491, 0.0643}, {0, 0.0272, 0.0384, 0.0535, 0.0685}, {0, 0.0122, 0.0195, 0.0263, 0.0335},
+                                      {{3.9, 0.76, 3.3, 0.0317, 0.0036, 0.0062}, {2.4, 0.70, 2.9, 0.0216, 0.0020, 0.0026}}};
+    static const Estimate wgrad = {3.5, 0.97, 0.0583, {0, 0.0209, 0.0340, 0.0487, 0.0633}, {0, 0.0209, 0.0340, 0.0487, 0.0633}, {}, {{2.7, 0.50, 3.4, 0.0338, 0.0, 0.0051}, {}}};
+    // (their column sums' launches in both)
+    static const Estimate wgrads = {9.6, 2.21, 0.0595, {0, 0.0225, 0.0374, 0.0515, 0.0653}, {0, 0.0225, 0.0374, 0.0515, 0.0653}, {}, {{7.2, 1.14, 7.6, 0.0360, 0.0, 0.0061}, {}}};
+    int64_t tiles[2] = {0, 0}, t64 = 0, t32 = 0;
+    double outputs = 0.0;
     int k = 0;
+    if (count < 1 || count > GROUP_MAX) return P_NONE;
     for (int i = 0; i < count; ++i) {
         const bb_gemm_desc& d = descs[i];
         if (!d.pieces || d.dtype != BB_F32 || d.nb1 > 1 || d.nb2 > 1 || d.conv_c != 0 || (count > 1 && d.layout != BB_TN)) return P_NONE;
@@ -388,16 +407,28 @@ PiecesTile pick_pieces(const bb_gemm_desc* descs, int count) {
         if (d.M <= 0 || d.N <= 0 || d.K <= 0 || d.N % 4 || d.ldc % 4 || d.ldaux % 4 || d.lda >= (1 << 21) || d.ldb >= (1 << 21)) return P_NONE;
         for (const void* p : {(const void*)d.C, d.bias, d.aux_in, (const void*)d.aux_out, d.resid})
             if ((uintptr_t)p % 16) return P_NONE;
-        flops += 2.0 * d.M * d.N * d.K;
-        tiles[0] += (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128);
-        tiles[1] += (int64_t)((d.M + 127) / 128) * ((d.N + 63) / 64);
+        auto count_tiles = [&](int m, int n) { return (int64_t)((d.M + m - 1) / m) * ((d.N + n - 1) / n); };
+        tiles[0] += count_tiles(128, 128);
+        tiles[1] += count_tiles(128, 64);
+        t64 += count_tiles(64, 64);
+        t32 += count_tiles(64, 32);
+        outputs += 1e-6 * d.M * d.N;
         k = d.K > k ? d.K : k;
     }
-    if (count < 1 || count > GROUP_MAX) return P_NONE;
-    const double fp32 = 4.0 + (flops > 0.82e6 * k ? flops / 105e6 : 0.0078 * k);
-    const double large = (double)((tiles[0] + 255) / 256) * (4.5 + 0.0322 * k), small = (double)((tiles[1] + 255) / 256) * (4.0 + 0.0206 * k);
-    if (descs[0].layout != BB_TN && small < large) return small < 0.95 * fp32 ? P128x64 : P_NONE;
-    return large < 0.95 * fp32 ? P128x128 : P_NONE;
+    if (t64 < 128) return P_NONE;       // (half of the CUs: the fp32 kernels share such a contraction out)
+    auto rounds = [](int64_t n) { return (double)((n + 255) / 256); };
+    const bool product = descs[0].layout != BB_TN;
+    const Estimate& e = product ? products : count == 1 ? wgrad : wgrads;
+    const bool split = count == 1 && pick_f32_split(descs[0].M, descs[0].N, descs[0].K, 1, descs[0].layout);
+    const int64_t fours = split ? 0 : t64 / 1024, most = ((split ? t32 : t64) - 1024 * fours + 255) / 256;
+    const double fp32 = e.base + e.outputs * outputs + (split ? e.split[most] : fours ? fours * e.full + e.after[most] : e.first[most]) * k;
+    auto pieces = [&](int t) {
+        const double r = rounds(tiles[t]);
+        return e.tile[t].base + e.tile[t].outputs * outputs + r * e.tile[t].round + (r * e.tile[t].step + (r > 1 ? e.tile[t].more : 0.0) + e.tile[t].share / 256 * tiles[t]) * k;
+    };
+    const double large = pieces(0), small = product ? pieces(1) : large, line = (!product ? 0.97 : k < 256 ? 0.95 : 1.0) * fp32;
+    if (large < line && large < 1.05 * small) return P128x128;
+    return small < line ? P128x64 : P_NONE;
 }
 
 template <int TM, int TN, int WM, int WN, bool TA, bool TB> static int launch(GemmArgs& g, hipStream_t st) {

@@ -158,3 +158,21 @@ def test_time_of_values_that_bf16_does_not_hold(hiplib, layout, M, N, K):
 
     finite = least(a)
     assert least(one) <= 6 * finite and least(every) <= 6 * finite
+
+
+def test_problems_that_fp32_instructions_do_sooner(hiplib):
+    """What the rounds of the tiles leave to the fp32 kernels, bit for bit: a product of one half-filled round, the weight gradients of a layer 576 wide over
+    1077 rows (275 tiles on 256 CUs: 109 us on pieces, 88) and of one 832 wide over 256 (70, 57)."""
+    a, b, _, _ = operands("nn", 1305, 1536, 384)
+    C, F = torch.empty(1305, 1536, device=DEV), torch.empty(1305, 1536, device=DEV)
+    hiplib.gemm(hiplib.NN, a, b, C, pieces=True)
+    hiplib.gemm(hiplib.NN, a, b, F)
+    assert torch.equal(C, F)
+    for h, R in ((576, 1077), (832, 256)):
+        ops = [(rand(R, m, seed=m), rand(R, n, seed=n + 1)) for m, n in ((3 * h, h), (h, h), (4 * h, h), (h, 4 * h))]
+        outs = []
+        for pieces in (True, False):
+            g = [torch.zeros(d.shape[1], v.shape[1], device=DEV) for d, v in ops]
+            hiplib.gemm_grouped([hiplib.gemm_desc(hiplib.TN, d, v, G, accumulate=True, pieces=pieces) for (d, v), G in zip(ops, g)])
+            outs.append(g)
+        assert all(torch.equal(p, q) for p, q in zip(*outs))
