@@ -129,24 +129,28 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     const int64_t t2128 = (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches;
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
     const bool big_ok = M >= 256 && N >= 256;
-    //  - Problems of at most one tile of 128x64 per CU take those or, NN and long contractions, 64x128 (gemm_m16.h; NT 128x64 / 64x128: 1050x1536x512
-    //    6.6 / 6.6, 12168x128x512 5.3 / 5.3, 2043x768x768 6.5 / 6.2, 2043x768x3072 17.9 / 16.7, 6272x256x1024 8.4 / 7.1; there five stages and fragments a whole k-tile ahead, forward, K 1024 7.1 / 7.3, with a
-    //    residual 1200x1600x1600 11.4 / 11.1, 3000x448x1792 11.8 / 11.0, 2043x768x3072 17.6 / 16.6, 2048x1024x4096 22.7 / 22.1, NN 22.8 / 23.2); then 128x128 tiles of three
-    //    stages, one per CU, up to a round of them.  64x128 or 128x64, the better / 128x128 (us, more than one of the first per CU): NT with activation
-    //    1200x2048x512 (304) 9.6 / 9.1, 1600x2048x640 (400) 11.5 / 10.6, 3136x1024x256 (392) 8.5 / 8.0, 8112x512x128 (508) 8.2 / 7.9, 4096x1024x192
-    //    (512) 8.6 / 8.2; NN times a tensor 8.1 / 7.7, 9.9 / 8.9, 6.6 / 6.5, 6.0 / 6.0, 6.5 / 6.3; 4096x768x3072 (384) 28.2 / 22.9; within a round
-    //    2043x768x768 (192) 6.2 / 8.2, 2048x1024x1024 (256) 7.3 / 9.6.  A round of 128x128 against 256x128 where a few rows stand against many
-    //    columns: 640x6400x1600 17.3 / 24.1.  More of them: 256x128 tiles, also for short contractions (NT 6272x1024x256
-    //    with activation 12.7, on 128x128 13.5), and 128x64 for what has one to three k-tiles forward, where the launch is its epilogue (NT with activation,
-    //    128x64 / 128x128: 25088x512x128 19.5 / 22.2, 6272x1024x128 11.9 / 12.3), or few columns.
+    //  - Problems of at most one half tile per CU take those: forward 128x64, from K 768 on 64x128, from 1536 on those of five stages, or 128x64
+    //    where only these fit into a round; NN 64x128.  us, plain or with a residual (+):
+    //        NT, both fit, 128x64 / 64x128           1050x1536x512 6.6* / 6.6    12168x128x512 5.3* / 5.3    6272x256x1024 8.4 / 7.1*    2043x768x768 6.5 / 6.2*
+    //        NT, one fits, 128x64 / 128x128          627x3264x960+ 9.3* / 10.8   4427x448x1088+ 12.4* / 14.0   8680x192x7040+ 55.7* / 61.9
+    //        NT, 64x128 of three stages / of five    2048x768x1024 7.1* / 7.3    1200x1600x1600+ 11.4 / 11.1*   2043x768x3072+ 17.6 / 16.6*   2048x1024x4096 22.7 / 22.1*
+    //    Then 128x128 tiles of three stages, one per CU, up to a round of them.  The better half / 128x128:
+    //        more than one half per CU, activation   1200x2048x512 9.6 / 9.1*    1600x2048x640 11.5 / 10.6*    3136x1024x256 8.5 / 8.0*    8112x512x128 8.2 / 7.9*
+    //        NN, times a tensor                      1200x2048x512 8.1 / 7.7*    1600x2048x640 9.9 / 8.9*      3136x1024x256 6.6 / 6.5*    4096x768x3072 28.2 / 22.9*
+    //        within a round of halves                2043x768x768 6.2* / 8.2     2048x1024x1024 7.3* / 9.6
+    //        (a few rows, many columns, 256x128 / 128x128   640x6400x1600 24.1 / 17.3*)
+    //    Larger ones: 256x128 and larger tiles, also for short contractions (NT 6272x1024x256 with activation 12.7, on 128x128 13.5), but halves for
+    //    what has one to three k-tiles forward, where the launch is its epilogue (with activation, 128x64 / 128x128: 25088x512x128 19.5 / 22.2,
+    //    6272x1024x128 11.9 / 12.3), or few columns.
     //    32-wide k-tiles (K % 64 != 0) as before: 128x64 tiles up to 128 tiles of 128x128 and for short forward contractions.
     if (k64) {
-        const bool tall = nt && K < 768;
-        const int64_t halves = tall ? (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches : (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
+        const int64_t talls = (int64_t)((M + 127) / 128) * ((N + 63) / 64) * batches, flats = (int64_t)((M + 63) / 64) * ((N + 127) / 128) * batches;
+        const bool tall = nt && (K < 768 || (flats > kCUs && talls <= kCUs));
+        const int64_t halves = tall ? talls : flats;
         const DmaTile half = tall ? D128x64k64s3 : nt && K >= 1536 ? D64x128k64s5 : D64x128k64s3;
         if (halves <= kCUs) return half;
         if (t128 <= kCUs) return D128x128k64s3;
-        if ((nt && K < 256) || halves <= (K >= 768 ? 256 : K >= 512 ? 400 : 512)) return half;
+        if ((nt && K < 256) || (K < 768 && halves <= (K >= 512 ? 400 : 512))) return half;
     } else {
         if ((K <= 512 || t128 <= 128) && nt) return D128x64s3;
         if (t128 <= 128 && nn) return D64x128s3;

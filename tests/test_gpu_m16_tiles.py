@@ -116,3 +116,23 @@ def test_small_tiles(hiplib, layout, M, N, K, tile):
     As, Bs = torch.stack([A, A.flip(0)]), torch.stack([B, B])
     hiplib.gemm_batched(lay, hiplib.BF16, M, N, K, As.data_ptr(), K, (M * K, 0), Bs.data_ptr(), B.shape[1], (N * K, 0), Cs.data_ptr(), N, (M * N, 0), 2, 1)
     assert near(Cs[0], ref) and torch.equal(Cs[0], Cs[1].flip(0))
+
+
+@pytest.mark.parametrize("M,N,tile", [(1275, 1600, "dma128x64k64s3"), (10335, 192, "dma128x64k64s3"), (627, 3264, "dma128x64k64s3"), (2041, 776, None), (1217, 1672, "dma128x128k64s3")])
+@pytest.mark.parametrize("K", [768, 1536, 1600])
+def test_half_tiles_that_fit_into_a_round(hiplib, M, N, K, tile):
+    """Forward contractions from 768 on: 64x128 tiles, 128x64 ones where these alone are at most one a CU (250, 243, 255 of 128x64, 260, 324, 260 of 64x128);
+    neither fits 1217x1672.  Bit for bit what the rows give among ten times as many, on larger tiles."""
+    A, B, bias, X = rand(M, K, seed=1), rand(N, K, seed=2, scale=0.2), rand(N, seed=3), rand(M, N, seed=4)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    C = wide[:M, :N]
+    assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NT, A, B, C)) == "bf16_nt_" + (tile or ("dma64x128k64s3" if K < 1536 else "dma64x128k64s5"))
+    hiplib.gemm(hiplib.NT, A, B, C, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X)
+    ref, slack = product(A, B.t())
+    want = ref + bias.double() + X.double()
+    assert ((C.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack + 2.0 ** -22 * (ref.abs() + 8.0)).all()
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
+    many = torch.empty(10 * M, N, dtype=torch.bfloat16, device=DEV)
+    assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NT, A.repeat(10, 1), B, many)).endswith(("dma256x192k64", "dma128x128k64"))
+    hiplib.gemm(hiplib.NT, A.repeat(10, 1), B, many, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X.repeat(10, 1))
+    assert torch.equal(many[:M], C) and torch.equal(many[9 * M:], C)
