@@ -92,9 +92,10 @@ enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, 
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
                                             "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3", "dma64x128k64s5"};
-// The kernel of a problem depends on its shape, layout and epilogue kind only (never on the stream, the environment or
-// what ran before): a redundant forward and a normal forward of the same layer give the same bits.  All tiles below add up
-// a contraction in the same order; the wave-sliced kernels (pick_wave) in another.
+// The kernel of a bf16 problem depends on its shape, layout, output type and epilogue only (never on the stream, the environment or what
+// ran before).  All tiles below add up a contraction in the same order, whichever runs changes no bit; the wave-sliced kernels (pick_wave)
+// in another, and which of the two orders a problem has is its shape and layout alone: a redundant forward and a normal forward of the
+// same layer give the same bits.  (fp32: shape and layout, the caller's word that pieces may be used, and their alignment, see pick_pieces.)
 static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     //  - Problems of at most one 64x64 tile per CU take those, four stages deep: what such a launch waits for is the chain of
     //    its k-tiles and its epilogue, and the more CUs share the loads the shorter both are.  128x64 / 64x64 tiles (us, back
@@ -190,12 +191,15 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     return small;
 }
 
-// ... of a problem with an fp32 output: of the tiles of gemm_m16.h, 256x128 has the registers for it.  More than one 256x256 tile a CU goes
-// by a name of its own (the blocks then walk their tiles; so do those of the other two).  All kernels add up a contraction in the same
-// order: which one runs changes no bit.
-static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, bool c_f32) {
+// ... of a problem with an fp32 output: of the tiles of gemm_m16.h, 256x128 has the registers for it.  ... and by what the epilogue reads (input
+// gradients; us, before this rule / with it):
+//  - Two operands, a few k-tiles, on 256x192 tiles: these wait for the second operand row by row; 128x128 tiles have other blocks to go on with.
+//    15600x1088x192 43.2 / 35.6, 3999x4288x256 44.5 / 36.7, 4796x4608x384 51.8 / 49.3; from K 512 on no gain (0.97, 1.00 at K 320..448, 512..704).
+static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, bool c_f32, int epilogue, bool resid) {
     const DmaTile t = pick_dma_tile(M, N, K, batches, layout);
     if (c_f32 && (t == D256x256k64 || t == D256x192k64)) return D256x128k64s3;
+    if (t == D256x192k64 && layout == BB_NN && K < 512 && epilogue == BB_EPI_MUL_POS && resid) return D128x128s3;
+    // (more than one 256x256 tile a CU goes by a name of its own: the blocks then walk their tiles; so do those of the other two)
     return t == D256x256k64 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches > kCUs ? D256x256p : t;
 }
 
@@ -250,7 +254,7 @@ static bool halve_tiles(int M, int N, int64_t batches) { return (int64_t)((M + 3
 
 template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, hipStream_t st) {
     const int layout = TA ? BB_TN : TB ? BB_NN : BB_NT;
-    const DmaTile dma = narrow_or_wide(pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.c_f32 != 0), layout, g.lda, g.ldb);
+    const DmaTile dma = narrow_or_wide(pick_dma_tile_for(g.M, g.N, g.K, batches, layout, g.c_f32 != 0, g.epilogue, g.resid != nullptr), layout, g.lda, g.ldb);
     switch (pick_wave(g.M, g.N, g.K, batches, layout, dma)) {
         case W_8: return launch_bf16_wave<TA, TB, 8, 32, 2>(g, batches, st);
         case W_4: return launch_bf16_wave<TA, TB, 4, 64, 1>(g, batches, st);
@@ -366,7 +370,7 @@ extern "C" int bb_gemm_variant(const bb_gemm_desc* d, char* out, int out_len) {
     BB_REQUIRE(d->layout >= BB_NT && d->layout <= BB_TN, "bb_gemm_variant: bad layout %d", d->layout);
     const int64_t batches = (int64_t)(d->nb1 > 0 ? d->nb1 : 1) * (d->nb2 > 0 ? d->nb2 : 1);
     if (d->dtype == BB_BF16) {
-        const DmaTile dt = narrow_or_wide(pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->c_dtype == BB_F32), d->layout, d->lda, d->ldb);
+        const DmaTile dt = narrow_or_wide(pick_dma_tile_for(d->M, d->N, d->K, batches, d->layout, d->c_dtype == BB_F32, d->epilogue, d->resid != nullptr), d->layout, d->lda, d->ldb);
         const WaveMode wm = pick_wave(d->M, d->N, d->K, batches, d->layout, dt);
         if (wm != W_NONE) snprintf(out, out_len, "bf16_%s_wave64x64k%d", layouts[d->layout], wm == W_8 ? 8 : 4);
         else snprintf(out, out_len, "bf16_%s_%s%s", layouts[d->layout], dt == D64x64k64s4 && halve_tiles(d->M, d->N, batches) ? "halves_" : "",

@@ -136,3 +136,24 @@ def test_half_tiles_that_fit_into_a_round(hiplib, M, N, K, tile):
     assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NT, A.repeat(10, 1), B, many)).endswith(("dma256x192k64", "dma128x128k64"))
     hiplib.gemm(hiplib.NT, A.repeat(10, 1), B, many, bias=bias, epilogue=hiplib.EPI_RESIDUAL, resid=X.repeat(10, 1))
     assert torch.equal(many[:M], C) and torch.equal(many[9 * M:], C)
+
+
+@pytest.mark.parametrize("M,N,K,resid,tile", [(4000, 4296, 256, True, "128x128s3"), (15600, 1088, 192, True, "128x128s3"), (4000, 4296, 448, True, "128x128s3"),
+                                              (4000, 4296, 512, True, "256x192k64"), (4000, 4296, 256, False, "256x192k64")])
+def test_tiles_by_what_the_epilogue_reads(hiplib, M, N, K, resid, tile):
+    """Input gradients masked by sign, with and without a residual: the tiles that this leads to, and the results bit for bit as a tenth of the rows
+    (another tile) gives them."""
+    A, B, X, R = rand(M, K, seed=1), rand(K, N, seed=2, scale=0.2), rand(M, N, seed=4), rand(M, N, seed=5)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    C, rows = wide[:M, :N], M // 10
+    kw = lambda a, b: dict(epilogue=hiplib.EPI_MUL_POS, aux_in=X[a:b], **(dict(resid=R[a:b]) if resid else {}))
+    assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NN, A, B, C, **kw(0, M))) == "bf16_nn_dma" + tile
+    hiplib.gemm(hiplib.NN, A, B, C, **kw(0, M))
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
+    ref, slack = product(A, B)
+    want = torch.where(X.double() > 0, ref + R.double() if resid else ref, 0.0)
+    assert ((C.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack + 2.0 ** -22 * (ref.abs() + 8.0)).all()
+    for a in (0, M - rows):
+        c = torch.empty(rows, N, dtype=torch.bfloat16, device=DEV)
+        hiplib.gemm(hiplib.NN, A[a:a + rows], B, c, **kw(a, a + rows))
+        assert torch.equal(c, C[a:a + rows])
