@@ -157,3 +157,23 @@ def test_tiles_by_what_the_epilogue_reads(hiplib, M, N, K, resid, tile):
         c = torch.empty(rows, N, dtype=torch.bfloat16, device=DEV)
         hiplib.gemm(hiplib.NN, A[a:a + rows], B, c, **kw(a, a + rows))
         assert torch.equal(c, C[a:a + rows])
+
+
+@pytest.mark.parametrize("M,N,K,epilogue,tile", [(6724, 2120, 128, "MUL", "256x256w8db"), (2323, 5440, 256, "MUL", "256x256w8db"), (4192, 3072, 768, "MUL", "256x256w8db"),
+                                                 (4192, 3072, 832, "MUL", "256x256k64"), (4192, 3072, 768, "MUL_POS", "256x256k64"), (7176, 4104, 128, "MUL", "256x256p")])
+def test_tiles_of_products_times_a_tensor(hiplib, M, N, K, epilogue, tile):
+    """As above, for one operand: up to twelve k-tiles and a round of 256x256 tiles on 32x32x16 instructions."""
+    A, B, X = rand(M, K, seed=1), rand(K, N, seed=2, scale=0.2), rand(M, N, seed=4)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    C, rows = wide[:M, :N], M // 10
+    kw = lambda a, b: dict(epilogue=getattr(hiplib, "EPI_" + epilogue), aux_in=X[a:b])
+    assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NN, A, B, C, **kw(0, M))) == "bf16_nn_dma" + tile
+    hiplib.gemm(hiplib.NN, A, B, C, **kw(0, M))
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
+    ref, slack = product(A, B)
+    x = X.double() if epilogue == "MUL" else (X > 0).double()
+    assert ((C.double() - ref * x).abs() <= 2.0 ** -8 * (ref * x).abs() + 1.01 * x.abs() * (slack + 2.0 ** -22 * (ref.abs() + 8.0))).all()
+    for a in (0, M - rows):
+        c = torch.empty(rows, N, dtype=torch.bfloat16, device=DEV)
+        hiplib.gemm(hiplib.NN, A[a:a + rows], B, c, **kw(a, a + rows))
+        assert torch.equal(c, C[a:a + rows])
