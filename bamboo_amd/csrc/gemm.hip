@@ -88,10 +88,10 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
 
 // DMA kernels need at least one full vector of rows, and but for weight gradients and D128x128k64r K % 32 == 0; tile by problem size
 enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, D256x128k64s3, D128x128k64, D128x64k64s3, D128x64s3,
-               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3, D64x128k64s5 };
+               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3, D64x128k64s5, D256x128k64s2 };
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
-                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3", "dma64x128k64s5"};
+                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3", "dma64x128k64s5", "short_dma256x128k64s3"};
 // The kernel of a bf16 problem depends on its shape, layout, output type and epilogue only (never on the stream, the environment or what
 // ran before).  All tiles below add up a contraction in the same order, whichever runs changes no bit; the wave-sliced kernels (pick_wave)
 // in another, and which of the two orders a problem has is its shape and layout alone: a redundant forward and a normal forward of the
@@ -198,11 +198,16 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
 //  - One operand to multiply by, up to twelve k-tiles, at most a round of 256x256 tiles: on the 32x32x16 loop, whose epilogue goes through LDS.  Multiplied
 //    by a tensor, mean of 440 products, 16x16x32 / 32x32x16: K 128 1.037 / 1.012, 320..384 1.027 / 1.003, 576..768 1.019 / 1.009, 800..1100 1.011 / 1.009
 //    (of the time before 16x16x32); masked by sign 0.99 / 1.01, plain 0.91 / 1.02, more than a round 0.96 / 0.95.
+//  - Two to four k-tiles in a round of 256x128 tiles: two stages instead of three ("short_"), as the
+//    third's transfers would only be in the way of the first's.  Three / two, of the time
+//    on the 32x32x16 loop before, K 128, 192, 256: plain 1.015 / 0.983, 1.024 / 0.987, 1.019 / 1.005 (5376x1024x256 9.54 / 9.35 us), times a tensor 0.97 / 0.95, 0.99 /
+//    0.97, 0.99 / 0.99; K 320..448 1.01 / 1.03.
 static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, bool c_f32, int epilogue, bool resid) {
     const DmaTile t = pick_dma_tile(M, N, K, batches, layout);
     if (c_f32 && (t == D256x256k64 || t == D256x192k64)) return D256x128k64s3;
     if (t == D256x192k64 && layout == BB_NN && K < 512 && epilogue == BB_EPI_MUL_POS && resid) return D128x128s3;
     if (t == D256x256k64 && layout == BB_NN && K <= 768 && epilogue == BB_EPI_MUL && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches <= kCUs) return D256x256w8db;
+    if (t == D256x128k64s3 && layout == BB_NN && K <= 256 && (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches <= kCUs) return D256x128k64s2;
     // (more than one 256x256 tile a CU goes by a name of its own: the blocks then walk their tiles; so do those of the other two)
     return t == D256x256k64 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches > kCUs ? D256x256p : t;
 }
@@ -277,6 +282,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
             else break;
         case D256x128k64s3:
             if constexpr (!TA) return launch_bf16_m16<4, 4, 4, 2, 3, TB>(g, batches, st);
+            else break;
+        case D256x128k64s2:
+            if constexpr (TB && !TA) return launch_bf16_m16<4, 4, 4, 2, 2, TB>(g, batches, st);
             else break;
         case D128x128k64: return launch_bf16_dma<128, 128, 2, 2, TA, TB, true, 2, 64>(g, batches, st);
         case D128x128k64r:
