@@ -696,29 +696,35 @@ template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(Groupe
 
 // Weight gradients on the tiles of gemm_m16.h: plain fp32 sums over contractions from kM16WgradRows rows on (below, what such a launch does is
 // read and write C, which three blocks a CU of 128x128 tiles do sooner: hidden size 1024 (x 4 in the feed-forward), 128x128 tiles of
-// gemm_bf16_dma_grouped_kernel / the better of these, us: 128 rows 22.7 / 25.0, 256 26.8 / 27.5, 512 33.5 / 32.5, 1024 43.7 / 42.8).  The tile
-// by its rounds, as in pick_dma_tile: a step of 64 rows, and what a round takes beside.  Before / 256x256 / 192x256 / 128x256 / 128x128 two a CU
-// (the one taken marked), hidden size and rows: 1024 8192 229 / 184* / 280 / 215 / 204, 4096 119 / 101* / 154 / 120 / 110; 1600 4096 282 / 301 /
-// 254* / 295 / 265; 960 8200 219 / 182 / 161* / 215 / 207; 768 16384 285 / 326 / 256 / 223* / 242, 8192 148 / 174 / 135 / 113* / 121, 2043 46 / 59 /
-// 47 / 40* / 40; 640 3000 58 / 78 / 61 / 48* / 51.  Tried: 160-wide tiles (rows of 320 bytes, no whole lines: 1600 284); 32-wide k-tiles in rings
-// of four and five (1024 8192 195, 202 against 187).
+// gemm_bf16_dma_grouped_kernel / the better of these, us: 128 rows 22.7 / 25.0, 256 26.8 / 27.5, 512 33.5 / 32.5, 1024 43.7 / 42.8).  The tile -- or that
+// kernel -- by an estimate: outputs, rounds, K steps of the fullest CU and of the share of the CUs that have a tile.  Fitted to 660 layers of 600 to
+// 16000 rows, 384 to 2048 wide (off by 4 to 6 %, 2-norm); of 595 from 768 rows on it leaves two more than 3 % slower than that kernel (3.2), where rounds alone,
+// without it among the choices, left 37, up to 14 %.  Before these tiles / 256x256 / 192x256 / 128x256 / 128x128 two a CU (the one taken marked; - what
+// rounds alone took), hidden size and rows: 1024 8192 229 / 184* / 280 / 215 / 204, 4096 119 / 101* / 154 / 120 / 110; 1600 4096 282 / 301 / 254* / 295 / 265; 960
+// 8200 219 / 182 / 161* / 215 / 207; 768 16384 285 / 326 / 256 / 223* / 242, 8192 148 / 174 / 135 / 113* / 121, 2043 46 / 59 / 47 / 40* / 40; 640 3000 58 / 78 / 61 / 48* /
+// 51; 1408 917 88* / 99- / 107 / 96 / 86 (in the cache 70* / 85 / 94 / 93 / 79); 1472 (x 2) 1031 76* / 96 / 85- / 83 / 77; 1184 1285 86* / 104 / 93- / 91 / 88; 1792 976 141 / 151- / 153 / 139* / 141.
+// Tried: 160-wide tiles (rows of 320 bytes, no whole lines: 1600 284); 32-wide k-tiles in rings of four and five (1024 8192 195, 202 against 187).
 constexpr int kM16WgradRows = 768;
 enum WgradTile { WG_NONE = 0, WG256x256, WG192x256, WG128x256, WG128x128 };
 static WgradTile pick_wgrad_m16(const GroupedArgs& G) {
     static const struct {
         WgradTile tile;
-        int bm, bn, slots, sum_columns;
-        double step, rest;
-    } tiles[] = {{WG256x256, 256, 256, kCUs, m16_sum_columns(8, 4), 1.36, 3.0},
-                 {WG192x256, 192, 256, kCUs, m16_sum_columns(6, 4), 1.12, 3.0},
-                 {WG128x256, 128, 256, kCUs, m16_sum_columns(4, 4), 0.80, 3.0},
-                 {WG128x128, 128, 128, 2 * kCUs, m16_sum_columns(4, 2), 0.86, 3.0}};
+        int bm, bn, blocks, sum_columns;                    // blocks a CU
+        double base, outputs, round, share, full, step[4];  // us; us per 10^6 outputs, per round; per k: times the share, of a full CU, of one with so many blocks
+    } tiles[] = {{WG_NONE, 128, 128, 3, 0, 7.2, 1.45, 2.0, 0.0087, 0.0126, {0, 0.0112, 0.0116, 0.0160}},
+                 {WG256x256, 256, 256, 1, m16_sum_columns(8, 4), 9.2, 1.32, 8.3, -0.0005, 0.0215, {0, 0.0215}},
+                 {WG192x256, 192, 256, 1, m16_sum_columns(6, 4), 8.0, 1.26, 6.1, 0.0002, 0.0181, {0, 0.0181}},
+                 {WG128x256, 128, 256, 1, m16_sum_columns(4, 4), 7.2, 0.96, 6.0, 0.0031, 0.0098, {0, 0.0098}},
+                 {WG128x128, 128, 128, 2, m16_sum_columns(4, 2), 5.6, 1.14, 3.6, 0.0054, 0.0090, {0, 0.0107, 0.0112}}};
     int kmax = 0;
+    double outputs = 0.0;
     for (int i = 0; i < G.count; ++i) {
         const GemmArgs& g = G.p[i];
         if (!g.c_f32 || g.bias || g.epilogue != BB_EPI_NONE || g.K < kM16WgradRows || g.lda >= kDmaMaxLd || g.ldb >= kDmaMaxLd || g.conv_c != 0) return WG_NONE;
         kmax = g.K > kmax ? g.K : kmax;
+        outputs += 1e-6 * g.M * g.N;
     }
+    const int k = (kmax + 63) / 64 * 64;
     WgradTile best = WG_NONE;
     double least = 0.0;
     for (const auto& t : tiles) {
@@ -730,8 +736,11 @@ static WgradTile pick_wgrad_m16(const GroupedArgs& G) {
             fits = fits && (!g.colsum || columns >= t.sum_columns);
             n += (int64_t)((g.M + t.bm - 1) / t.bm) * columns;
         }
-        const double us = (double)((n + t.slots - 1) / t.slots) * ((kmax + 63) / 64 * t.step + t.rest);
-        if (fits && (best == WG_NONE || us < least)) best = t.tile, least = us;
+        const int64_t slots = (int64_t)t.blocks * kCUs, full = (n - 1) / slots, most = (n - slots * full + kCUs - 1) / kCUs;
+        const double us = t.base + t.outputs * outputs + t.round * (full + 1) + (full * t.full + t.step[most] + t.share * n / slots) * k;
+        // (few k-tiles and all of it in the last-level cache: that kernel is another tenth faster)
+        if (t.tile == WG_NONE) least = (k < 2048 ? 0.95 : 1.0) * us;
+        else if (fits && us < least) best = t.tile, least = us;
     }
     return best;
 }
