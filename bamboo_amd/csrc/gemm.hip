@@ -746,6 +746,7 @@ static WgradTile pick_wgrad_m16(const GroupedArgs& G) {
 }
 template <int TM, int TN, int WM, int WN, int STAGES> static int launch_wgrad_m16(GroupedArgs& G, hipStream_t st) {
     constexpr int BM = WM * TM * 16, BN = WN * TN * 16, smem = STAGES * (BM + BN) * 128;
+    static_assert(kM16WgradRows > STAGES * 64, "the ring is filled before the last k-tile");
     auto kern = wgrad_m16_grouped_kernel<TM, TN, WM, WN, STAGES>;
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     int blocks = 0;

@@ -31,7 +31,8 @@ __device__ __forceinline__ const char* m16_uniform(const char* p) {
     return (const char*)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b));
 }
 // the same value, made anew where this stands: the compiler computes what depends on it only there, not in front of the loops, where it
-// would lie in registers that the fragments need (256x256 tiles: nothing but a spilt register away from a wait for every transfer)
+// would lie in registers that the fragments need: 256x256 tiles have none left, and a spilt one inside the loop is a wait for every transfer (the
+// weight gradients' spill eight, around their loops)
 __device__ __forceinline__ int m16_here(int v) {
     asm volatile("" : "+v"(v));
     return v;
@@ -54,8 +55,7 @@ template <int BR, int NW, bool KM, bool PAIRED> struct M16Lanes {
     int64_t step;      // bytes per k-tile
     unsigned off[ROUNDS];
 
-    // (left: KM only, k rows the tile has; a lane past them reads the last one again)
-    __device__ __forceinline__ void init(const bf16* at, int64_t ld, int row0, int rows, int tid, int left = 64) {
+    __device__ __forceinline__ void init(const bf16* at, int64_t ld, int row0, int rows, int tid) {
         const int ld2 = (int)ld * 2;
         if constexpr (!KM) {
             const int r0 = tid >> 3, last = rows - 1 - row0;
@@ -66,11 +66,12 @@ template <int BR, int NW, bool KM, bool PAIRED> struct M16Lanes {
             base = (const char*)(at + (int64_t)row0 * ld);
             step = 128;
         } else {
-            reach(ld2, rows - 8 - row0, tid, left);
+            reach(ld2, rows - 8 - row0, tid, 64);
             base = (const char*)(at + row0);
             step = 128 * ld;
         }
     }
+    // (left: KM only, k rows the tile has; a lane past them reads the last one again)
     __device__ __forceinline__ void reach(int ld2, int last, int tid, int left) {
 #pragma unroll
         for (int i = 0; i < ROUNDS; ++i) {
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_m16_kernel(const GemmAr
     }
 }
 
-// Weight gradients: C[m][n] (fp32) = or += alpha * sum over k of A[k][m] B[k][n], both operands k-major, any K > 0.
+// Weight gradients: C[m][n] (fp32) = or += alpha * sum over k of A[k][m] B[k][n], both operands k-major, K > STAGES * 64.
 //
 // A last k-tile that is not whole: its transfers read the last row again (nothing lies behind it), and once they have landed the rows
 // past the end are cleared in LDS, in both operands, before they are read.
@@ -437,8 +438,8 @@ __device__ __forceinline__ void wgrad_m16_body(const GemmArgs& g, const int id) 
     panel_coords<8>(id, g.tiles_m, g.tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     Loop p;
-    p.opa.init((const bf16*)g.A, g.lda, m0, g.M, tid, KT == 1 && tail ? tail : 64);
-    p.opb.init((const bf16*)g.B, g.ldb, n0, g.N, tid, KT == 1 && tail ? tail : 64);
+    p.opa.init((const bf16*)g.A, g.lda, m0, g.M, tid);
+    p.opb.init((const bf16*)g.B, g.ldb, n0, g.N, tid);
     constexpr int SC = m16_sum_columns(TM, WN);
     const int first = __builtin_amdgcn_readfirstlane((tid >> 6) % WN * SC + tn);
     const bool do_sums = g.colsum != nullptr && tn < SC && first < TM;
@@ -451,10 +452,7 @@ __device__ __forceinline__ void wgrad_m16_body(const GemmArgs& g, const int id) 
     };
     p.clear();
 #pragma unroll
-    for (int t = 0; t < STAGES; ++t) {
-        if (t > 0 && t == KT - 1) last_tile();
-        p.feed_all(t, __builtin_amdgcn_readfirstlane((t - KT) >> 31));
-    }
+    for (int t = 0; t < STAGES; ++t) p.feed_all(t, -1);
     p.template landed<STAGES - 1>();
 
     const int wm = p.wave / WN, wn = p.wave % WN;
