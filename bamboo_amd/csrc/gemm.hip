@@ -208,8 +208,8 @@ static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layou
     if (t == D256x192k64 && layout == BB_NN && K < 512 && epilogue == BB_EPI_MUL_POS && resid) return D128x128s3;
     if (t == D256x256k64 && layout == BB_NN && K <= 768 && epilogue == BB_EPI_MUL && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches <= kCUs) return D256x256w8db;
     if (t == D256x128k64s3 && layout == BB_NN && K <= 256 && (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches <= kCUs) return D256x128k64s2;
-    // (more than one 256x256 tile a CU goes by a name of its own: the blocks then walk their tiles; so do those of the other two)
-    return t == D256x256k64 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches > kCUs ? D256x256p : t;
+    // (more than one 256x256 tile of a batch a CU goes by a name of its own: the blocks then walk their batch's tiles; so do those of the other two)
+    return t == D256x256k64 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) > kCUs ? D256x256p : t;
 }
 
 // The kernels that leave column statistics (128x64, 64x128 or 256x128 tiles) take the largest within a round of them and, forward, where its

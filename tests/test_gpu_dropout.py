@@ -81,6 +81,17 @@ def test_gemm_epilogue_dropout(hiplib, dtype, M, N, K, epi):
     assert torch.equal(C, C2)
 
 
+@pytest.mark.parametrize("epi", ["none", "act_dact", "residual"])
+@pytest.mark.parametrize("variant,M,N,K", [("halves_dma64x64k64s4", 300, 392, 192), ("dma64x64k64s4", 1033, 520, 192), ("dma128x64k64s3", 2041, 776, 192), ("dma64x128k64s3", 2041, 776, 832),
+                                           ("dma64x128k64s5", 2041, 776, 1600), ("dma128x128k64s3", 4089, 776, 192), ("dma256x128k64s3", 8100, 1000, 320), ("dma256x192k64", 8200, 2696, 320)])
+def test_gemm_epilogue_dropout_of_every_tile(hiplib, variant, M, N, K, epi):
+    """The kernels of test_gemm_epilogue_dropout's bf16 cases are three of those with dropout in them: here the others, by name."""
+    name = hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NT, torch.empty(M, K, dtype=torch.bfloat16, device=DEV), torch.empty(N, K, dtype=torch.bfloat16, device=DEV),
+                                                torch.empty(M, N, dtype=torch.bfloat16, device=DEV), dropout=(0.25, KEY)))
+    assert name == "bf16_nt_" + variant
+    test_gemm_epilogue_dropout(hiplib, torch.bfloat16, M, N, K, epi)
+
+
 @pytest.mark.parametrize("mask", ["none", "causal", "key_padding"])
 @pytest.mark.parametrize("batch,heads,seq,d", [(2, 2, 128, 64), (1, 3, 200, 64), (2, 4, 128, 32), (1, 2, 200, 32), (2, 2, 128, 128),
                                                (1, 1, 200, 128)])

@@ -54,7 +54,7 @@ def test_tiles(hiplib, layout, tile, M, N, K):
 
 @pytest.mark.parametrize("layout", ["nt", "nn"])
 def test_batches(hiplib, layout):
-    """Batched problems of several tiles a block: operands and outputs of each batch by its strides."""
+    """Batched problems, a tile a block: operands and outputs of each batch by its strides."""
     lay, n, M, N, K = getattr(hiplib, layout.upper()), 3, 2056, 2312, 256
     A, B = rand(n, M, K, seed=1), rand(n, *((N, K) if layout == "nt" else (K, N)), seed=2)
     C, c = torch.empty(n, M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
@@ -62,6 +62,37 @@ def test_batches(hiplib, layout):
     for i in range(n):
         hiplib.gemm(lay, A[i], B[i], c)
         assert torch.equal(C[i], c)
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("tile,M,N,K", [("256x256p", 7688, 3848, 320), ("256x128k64s3", 33000, 264, 256), ("256x192k64", 10520, 1672, 320)])
+def test_batches_whose_blocks_walk(hiplib, layout, tile, M, N, K):
+    """Batches of more tiles than CUs each (496, 387, 378): a block goes on to the next tile of its own batch.  As one by one, bit for bit; what lies behind a
+    batch's output stays as it is."""
+    lay, n = getattr(hiplib, layout.upper()), 2
+    A, B = rand(n, M, K, seed=1), rand(n, *((N, K) if layout == "nt" else (K, N)), seed=2)
+    C, c = torch.full((n, M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    desc = hiplib.gemm_desc(lay, A[0], B[0], c)
+    desc.nb1 = n
+    assert hiplib.gemm_variant(desc).endswith(tile)
+    hiplib.gemm_batched(lay, hiplib.BF16, M, N, K, A.data_ptr(), K, (M * K, 0), B.data_ptr(), B.shape[2], (N * K, 0), C.data_ptr(), N, ((M + 1) * N, 0), n, 1)
+    for i in range(n):
+        hiplib.gemm(lay, A[i], B[i], c)
+        assert torch.equal(C[i, :M], c) and (C[i, M] == 7).all()
+
+
+# 256x256 (one and several tiles a block), 256x192, 256x128 (three stages, two NN), 128x128, 128x64 and 64x128 (three and five stages), 64x64, 32x64
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("M,N", [(7176, 4104), (8200, 2696), (4192, 3072), (4100, 1032), (2300, 1040), (2041, 776), (1033, 520), (136, 392)])
+@pytest.mark.parametrize("K", [128, 192, 832, 1600])
+def test_bits_of_both_instructions(hiplib, layout, M, N, K):
+    """Two problems that share a launch run on 32x32x16 instructions (gemm_bf16_dma_grouped_kernel), forward and backward: the bits of 16x16x32."""
+    lay = getattr(hiplib, layout.upper())
+    A, B = rand(M, K, seed=1), rand(*((N, K) if layout == "nt" else (K, N)), seed=2)
+    C, G, H = (torch.empty(M, N, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    hiplib.gemm(lay, A, B, C)
+    hiplib.gemm_grouped([hiplib.gemm_desc(lay, A, B, G), hiplib.gemm_desc(lay, A, B, H)])
+    assert torch.equal(C, G) and torch.equal(C, H)
 
 
 # weight gradients by the tile that two of them in one launch take: 128x128 or 256x256, 128x128 of the 32x32x16 loop, 128x128 twice; 256x256, 192x256, 128x256, 128x128,
