@@ -194,7 +194,7 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
 // ... of a problem with an fp32 output: of the tiles of gemm_m16.h, 256x128 has the registers for it.  ... and by what the epilogue reads (input
 // gradients; us, before this rule / with it):
 //  - Two operands, a few k-tiles, on 256x192 tiles: these wait for the second operand row by row; 128x128 tiles have other blocks to go on with.
-//    15600x1088x192 43.2 / 35.6, 3999x4288x256 44.5 / 36.7, 4796x4608x384 51.8 / 49.3; from K 512 on no gain (0.97, 1.00 at K 320..448, 512..704).
+//    15600x1088x192 43.2 / 35.6, 3999x4288x256 44.5 / 36.7, 4796x4608x384 51.8 / 49.3; K 448 0.96, 512 0.95 (9196x2048x512 54.6 / 49.8), 576 1.02.
 //  - One operand to multiply by, up to twelve k-tiles, at most a round of 256x256 tiles: on the 32x32x16 loop, whose epilogue goes through LDS.  Multiplied
 //    by a tensor, mean of 440 products, 16x16x32 / 32x32x16: K 128 1.037 / 1.012, 320..384 1.027 / 1.003, 576..768 1.019 / 1.009, 800..1100 1.011 / 1.009
 //    (of the time before 16x16x32); masked by sign 0.99 / 1.01, plain 0.91 / 1.02, more than a round 0.96 / 0.95.
@@ -205,7 +205,7 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
 static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, bool c_f32, int epilogue, bool resid) {
     const DmaTile t = pick_dma_tile(M, N, K, batches, layout);
     if (c_f32 && (t == D256x256k64 || t == D256x192k64)) return D256x128k64s3;
-    if (t == D256x192k64 && layout == BB_NN && K < 512 && epilogue == BB_EPI_MUL_POS && resid) return D128x128s3;
+    if (t == D256x192k64 && layout == BB_NN && K <= 512 && epilogue == BB_EPI_MUL_POS && resid) return D128x128s3;
     if (t == D256x256k64 && layout == BB_NN && K <= 768 && epilogue == BB_EPI_MUL && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches <= kCUs) return D256x256w8db;
     if (t == D256x128k64s3 && layout == BB_NN && K <= 256 && (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches <= kCUs) return D256x128k64s2;
     // (more than one 256x256 tile of a batch a CU goes by a name of its own: the blocks then walk their batch's tiles; so do those of the other two)

@@ -172,7 +172,7 @@ def test_half_tiles_that_fit_into_a_round(hiplib, M, N, K, tile):
 
 
 @pytest.mark.parametrize("M,N,K,resid,tile", [(4000, 4296, 256, True, "128x128s3"), (15600, 1088, 192, True, "128x128s3"), (4000, 4296, 448, True, "128x128s3"),
-                                              (4000, 4296, 512, True, "256x192k64"), (4000, 4296, 256, False, "256x192k64")])
+                                              (4000, 4296, 512, True, "128x128s3"), (4000, 4296, 576, True, "256x192k64"), (4000, 4296, 256, False, "256x192k64")])
 def test_tiles_by_what_the_epilogue_reads(hiplib, M, N, K, resid, tile):
     """Input gradients masked by sign, with and without a residual: the tiles that this leads to, and the results bit for bit as a tenth of the rows
     (another tile) gives them."""
