@@ -31,8 +31,7 @@ __device__ __forceinline__ const char* m16_uniform(const char* p) {
     return (const char*)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b));
 }
 // the same value, made anew where this stands: the compiler computes what depends on it only there, not in front of the loops, where it
-// would lie in registers that the fragments need: 256x256 tiles have none left, and a spilt one inside the loop is a wait for every transfer (the
-// weight gradients' spill eight, around their loops)
+// would lie in registers that the fragments need (256x256 tiles: none spills, and one that did inside the loop would be a wait for every transfer)
 __device__ __forceinline__ int m16_here(int v) {
     asm volatile("" : "+v"(v));
     return v;
