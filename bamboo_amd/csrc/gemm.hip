@@ -56,7 +56,7 @@ template <int TM, int TN, int WM, int WN, int STAGES, bool TB, bool WHOLE = fals
     BB_HIP_CHECK(bb_allow_dynamic_lds((const void*)kern, smem));
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    const int total = g.tiles_m * g.tiles_n, blocks = BM == 256 && g.K >= STAGES * 64 && total > kCUs ? kCUs : total;
+    const int total = g.tiles_m * g.tiles_n, blocks = !WHOLE && BM == 256 && g.K >= STAGES * 64 && total > kCUs ? kCUs : total;
     bb_launch(kern, dim3(blocks, 1, batches), dim3(WM * WN * 64), smem, st, g);
     BB_LAUNCH_CHECK();
     return BB_OK;
@@ -88,10 +88,11 @@ static int launch_bf16_dma_bnbwd(GemmArgs& g, const BnBwdArgs& bn, hipStream_t s
 
 // DMA kernels need at least one full vector of rows, and but for weight gradients and D128x128k64r K % 32 == 0; tile by problem size
 enum DmaTile { D_NONE = 0, D256x256w8db, D256x128w8db, D128x128s3, D256x256k64, D256x128k64s3, D128x128k64, D128x64k64s3, D128x64s3,
-               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3, D64x128k64s5, D256x128k64s2 };
+               D64x128k64s3, D64x128s3, D256x192k64, D256x256p, D64x64k64s4, D128x128k64r, D128x128k64s3, D64x128k64s5, D256x128k64s2, D256x128k64w };
 static const char* const kDmaTileNames[] = {"", "dma256x256w8db", "dma256x128w8db", "dma128x128s3", "dma256x256k64", "dma256x128k64s3",
                                             "dma128x128k64", "dma128x64k64s3", "dma128x64s3", "dma64x128k64s3", "dma64x128s3",
-                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3", "dma64x128k64s5", "short_dma256x128k64s3"};
+                                            "dma256x192k64", "dma256x256p", "dma64x64k64s4", "dma128x128k64r", "dma128x128k64s3", "dma64x128k64s5", "short_dma256x128k64s3",
+                                            "whole_dma256x128k64s3"};
 // The kernel of a bf16 problem depends on its shape, layout, output type and epilogue only (never on the stream, the environment or what
 // ran before).  All tiles below add up a contraction in the same order, whichever runs changes no bit; the wave-sliced kernels (pick_wave)
 // in another, and which of the two orders a problem has is its shape and layout alone: a redundant forward and a normal forward of the
@@ -198,16 +199,23 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
 //  - One operand to multiply by, up to twelve k-tiles, at most a round of 256x256 tiles: on the 32x32x16 loop, whose epilogue goes through LDS.  Multiplied
 //    by a tensor, mean of 440 products, 16x16x32 / 32x32x16: K 128 1.037 / 1.012, 320..384 1.027 / 1.003, 576..768 1.019 / 1.009, 800..1100 1.011 / 1.009
 //    (of the time before 16x16x32); masked by sign 0.99 / 1.01, plain 0.91 / 1.02, more than a round 0.96 / 0.95.
-//  - Two to four k-tiles in a round of 256x128 tiles: two stages instead of three ("short_"), as the
-//    third's transfers would only be in the way of the first's.  Three / two, of the time
-//    on the 32x32x16 loop before, K 128, 192, 256: plain 1.015 / 0.983, 1.024 / 0.987, 1.019 / 1.005 (5376x1024x256 9.54 / 9.35 us), times a tensor 0.97 / 0.95, 0.99 /
-//    0.97, 0.99 / 0.99; K 320..448 1.01 / 1.03.
+//  - Few k-tiles in a round of 256x128 tiles.  NN, two or three: two stages instead of three ("short_"), as the third's transfers would only be in the way of the
+//    first's.  Up to eleven: fragments a whole k-tile ahead ("whole_"), but where GELU and its derivative want the registers.  Of the time on the 32x32x16 loop
+//    before, half a k-tile ahead / two stages / whole (mean of 3000 products):
+//        NN plain, K 128 1.015 / 0.983* / 1.024     192 1.024 / 0.987* / 1.022     256 1.019 / 1.005 / 1.010*      320..448 1.009 / 1.025 / 0.998*     512..704 0.995 / 1.065 / 0.981*
+//        times a tensor  0.971 / 0.947* / 0.953     0.989 / 0.967* / 0.952         0.991 / 0.989 / 0.957*          0.981 / 1.018 / 0.945*              0.984 / 1.080 / 0.953*
+//        NT residual                                                               0.979 / 0.984 / 0.949*          0.993 / 1.039 / 0.958*              0.974 / 1.074 / 0.949*
+//        NT GELU and derivative                                                    0.922* / 0.922 / 0.984          0.934* / 0.971 / 0.983              0.941* / 1.028 / 0.988
+//    (operands and outputs not in the last-level cache: 5054x1024x256 10.15 / 10.07 / 10.06 us, before 9.65; 13362x320x320 11.85 / 12.33 / 11.49, 11.25)
 static DmaTile pick_dma_tile_for(int M, int N, int K, int64_t batches, int layout, bool c_f32, int epilogue, bool resid) {
     const DmaTile t = pick_dma_tile(M, N, K, batches, layout);
     if (c_f32 && (t == D256x256k64 || t == D256x192k64)) return D256x128k64s3;
     if (t == D256x192k64 && layout == BB_NN && K <= 512 && epilogue == BB_EPI_MUL_POS && resid) return D128x128s3;
     if (t == D256x256k64 && layout == BB_NN && K <= 768 && epilogue == BB_EPI_MUL && (int64_t)((M + 255) / 256) * ((N + 255) / 256) * batches <= kCUs) return D256x256w8db;
-    if (t == D256x128k64s3 && layout == BB_NN && K <= 256 && (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches <= kCUs) return D256x128k64s2;
+    if (t == D256x128k64s3 && K < 768 && (int64_t)((M + 255) / 256) * ((N + 127) / 128) * batches <= kCUs) {
+        if (layout == BB_NN && K <= 192) return D256x128k64s2;
+        if (epilogue != BB_EPI_ACT_DACT) return D256x128k64w;
+    }
     // (more than one 256x256 tile of a batch a CU goes by a name of its own: the blocks then walk their batch's tiles; so do those of the other two)
     return t == D256x256k64 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) > kCUs ? D256x256p : t;
 }
@@ -282,6 +290,9 @@ template <bool TA, bool TB> static int dispatch_bf16(GemmArgs& g, int batches, h
             else break;
         case D256x128k64s3:
             if constexpr (!TA) return launch_bf16_m16<4, 4, 4, 2, 3, TB>(g, batches, st);
+            else break;
+        case D256x128k64w:
+            if constexpr (!TA) return launch_bf16_m16<4, 4, 4, 2, 3, TB, true>(g, batches, st);
             else break;
         case D256x128k64s2:
             if constexpr (TB && !TA) return launch_bf16_m16<4, 4, 4, 2, 2, TB>(g, batches, st);

@@ -32,7 +32,8 @@ def test_register_epilogue(hiplib, layout, tile, M, N, K):
 @pytest.mark.parametrize("variant,M,N,K", [("bf16_nt_dma128x64k64s3", 2041, 776, 448), ("bf16_nt_dma128x64k64s3", 627, 3264, 832), ("bf16_nn_dma64x128k64s3", 2041, 776, 448),
                                            ("bf16_nn_dma64x128k64s3", 2041, 776, 1600), ("bf16_nt_dma64x128k64s3", 2041, 776, 832), ("bf16_nt_dma64x128k64s5", 2041, 776, 1600),
                                            ("bf16_nt_dma128x128k64s3", 2300, 1040, 448), ("bf16_nn_dma128x128k64s3", 2300, 1040, 448),
-                                           ("bf16_nn_short_dma256x128k64s3", 8100, 1000, 192)])
+                                           ("bf16_nn_short_dma256x128k64s3", 8100, 1000, 192),
+                                           ("bf16_nn_whole_dma256x128k64s3", 8100, 1000, 320), ("bf16_nt_whole_dma256x128k64s3", 8100, 1000, 320), ("bf16_nt_dma256x128k64s3", 8100, 1000, 768)])
 def test_register_epilogue_of_half_tiles(hiplib, variant, M, N, K):
     for guard in (True, False):
         every_kind(hiplib, variant[5:7], variant, M, N, K, guard)

@@ -212,10 +212,10 @@ def test_tiles_of_products_times_a_tensor(hiplib, M, N, K, epilogue, tile):
         assert torch.equal(c, C[a:a + rows])
 
 
-@pytest.mark.parametrize("K,tile", [(128, "short_dma256x128k64s3"), (192, "short_dma256x128k64s3"), (256, "short_dma256x128k64s3"), (320, "dma256x128k64s3")])
+@pytest.mark.parametrize("K,tile", [(128, "short_"), (192, "short_"), (256, "whole_"), (320, "whole_"), (704, "whole_"), (768, "")])
 @pytest.mark.parametrize("M,N", [(6272, 1024), (17993, 200), (4361, 1352)])
-def test_short_products_on_two_stages(hiplib, M, N, K, tile):
-    """Input gradients of two to four k-tiles within a round of 256x128 tiles, nothing, a row and 8 columns in the last ones: fewer, as many and more k-tiles
+def test_short_products_within_a_round(hiplib, M, N, K, tile):
+    """Input gradients of few k-tiles within a round of 256x128 tiles, nothing, a row and 8 columns in the last ones: fewer, as many and more k-tiles
     than the ring has stages; every operand of the epilogue, a result in fp32, and bit for bit as a tenth of the rows gives them."""
     A, B, X, R, bias = rand(M, K, seed=1), rand(K, N, seed=2, scale=0.2), rand(M, N, seed=4), rand(M, N, seed=5), rand(N, seed=3)
     wide = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
@@ -226,7 +226,7 @@ def test_short_products_on_two_stages(hiplib, M, N, K, tile):
                                  (dict(epilogue=hiplib.EPI_MUL_POS), dict(aux_in=X, resid=R), torch.where(x > 0, ref + r, 0.0)),
                                  (dict(bias=bias, epilogue=hiplib.EPI_RESIDUAL), dict(resid=R), ref + bias.double() + r)):
         kw = lambda a, b: dict(kind, **{k: v[a:b] for k, v in operands.items()})
-        assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NN, A, B, C, **kw(0, M))) == "bf16_nn_" + tile
+        assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NN, A, B, C, **kw(0, M))) == f"bf16_nn_{tile}dma256x128k64s3"
         hiplib.gemm(hiplib.NN, A, B, C, **kw(0, M))
         scale = x.abs().clamp_min(1.0)
         assert ((C.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1.01 * scale * (slack + 2.0 ** -22 * (ref.abs() + 8.0))).all()
@@ -236,7 +236,7 @@ def test_short_products_on_two_stages(hiplib, M, N, K, tile):
             hiplib.gemm(hiplib.NN, A[a:a + rows], B, c, **kw(a, a + rows))
             assert torch.equal(c, C[a:a + rows])
     F = torch.ones(M, N, device=DEV)
-    assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NN, A, B, F)) == "bf16_nn_" + tile
+    assert hiplib.gemm_variant(hiplib.gemm_desc(hiplib.NN, A, B, F)) == f"bf16_nn_{tile}dma256x128k64s3"
     hiplib.gemm(hiplib.NN, A, B, F, accumulate=True, alpha=0.5)
     assert ((F.double() - 1.0 - 0.5 * ref).abs() <= slack + 2.0 ** -23 * (ref.abs() + 2.0)).all()
 
