@@ -1,12 +1,12 @@
-// MFMA GEMM for gfx950: bf16 (v_mfma_f32_16x16x32_bf16, v_mfma_f32_32x32x16_bf16) and fp32 (v_mfma_f32_32x32x2_f32),
-// LDS-tiled, double-buffered, batched with two-level strides, fused epilogues.
+// MFMA GEMM for gfx950: bf16 (v_mfma_f32_16x16x32_bf16, v_mfma_f32_32x32x16_bf16) and fp32 (v_mfma_f32_16x16x4_f32, v_mfma_f32_32x32x2_f32, or six
+// bf16 products of pieces), LDS-tiled, double-buffered, batched with two-level strides, fused epilogues.
 //
 // Stands in for F.linear / torch.matmul and their autograd backward in the reference layer
 // (DeepSpeedExamples/pipeline_parallelism/transformer.py:121,127,136-146,158).
 //
-// bf16 data paths: NT and NN tiles by DMA on 16x16x32 instructions (gemm_m16.h), others on 32x32x16 (gemm_bf16_dma_*); 64x64 tiles with the contraction dealt to the waves (gemm_wave.h) for weight
-// gradients of few tiles and few tiles of an odd contraction length; a register-staged kernel for rows of C that are no
-// whole vectors (N % 8 != 0, NT).  fp32: gemm_f32.h.
+// bf16 data paths: NT and NN tiles by DMA on 16x16x32 instructions (gemm_m16.h), others on 32x32x16 (gemm_bf16_dma_*); 64x64 tiles with the
+// contraction dealt to the waves (gemm_wave.h) for weight gradients of few tiles and few tiles of an odd contraction length; a register-staged
+// kernel for rows of C that are no whole vectors (N % 8 != 0, NT).  fp32: gemm_f32.h, gemm_f32_pieces.hip.
 #include "gemm_kernels.h"
 #include "gemm_m16.h"
 #include "gemm_f32.h"
@@ -159,7 +159,7 @@ static DmaTile pick_dma_tile(int M, int N, int K, int64_t batches, int layout) {
     }
     //  - Larger ones, whole 64-wide k-tiles: the tile of gemm_m16.h whose rounds take least, a round (one tile a CU) of kt k-tiles being
     //    kt times a step, plus what a tile costs around its loop (prologue, epilogue, the stores of all CUs at once).  Steps and rest as fitted
-    //    to the table; the two of 256x256 are 1500 TFLOP/s, at the card's power.  Before (32x32x16 instructions, several kernels and rules) / 256x256 /
+    //    to the table (a step of 256x256 is 1500 TFLOP/s).  Before (32x32x16 instructions, several kernels and rules) / 256x256 /
     //    256x192 / 256x128 (us, plain, the one taken marked):
     //        NT 8192x3072x1024 66 / 58 / 50* / 48    8192x4096x1024 78 / 63* / 66 / 66    8192x1024x4096 66 / 80 / 69 / 58*
     //           8192x1024x1024 24 / 29 / 25 / 22*    4096x4800x1600 73 / 73 / 60* / 62    4096x6400x1600, activation 97 / 85* / 101 / 97
@@ -710,10 +710,20 @@ template <bool TA, bool TB, bool CONVB = false> static int launch_grouped(Groupe
 // gemm_bf16_dma_grouped_kernel / the better of these, us: 128 rows 22.7 / 25.0, 256 26.8 / 27.5, 512 33.5 / 32.5, 1024 43.7 / 42.8).  The tile -- or that
 // kernel -- by an estimate: outputs, rounds, K steps of the fullest CU and of the share of the CUs that have a tile.  Fitted to 660 layers of 600 to
 // 16000 rows, 384 to 2048 wide (off by 4 to 6 %, 2-norm); of 595 from 768 rows on it leaves two more than 3 % slower than that kernel (3.2), where rounds alone,
-// without it among the choices, left 37, up to 14 %.  Before these tiles / 256x256 / 192x256 / 128x256 / 128x128 two a CU (the one taken marked; - what
-// rounds alone took), hidden size and rows: 1024 8192 229 / 184* / 280 / 215 / 204, 4096 119 / 101* / 154 / 120 / 110; 1600 4096 282 / 301 / 254* / 295 / 265; 960
-// 8200 219 / 182 / 161* / 215 / 207; 768 16384 285 / 326 / 256 / 223* / 242, 8192 148 / 174 / 135 / 113* / 121, 2043 46 / 59 / 47 / 40* / 40; 640 3000 58 / 78 / 61 / 48* /
-// 51; 1408 917 88* / 99- / 107 / 96 / 86 (in the cache 70* / 85 / 94 / 93 / 79); 1472 (x 2) 1031 76* / 96 / 85- / 83 / 77; 1184 1285 86* / 104 / 93- / 91 / 88; 1792 976 141 / 151- / 153 / 139* / 141.
+// without it among the choices, left 37, up to 14 %.  us (the one taken marked; - what rounds alone took):
+//     hidden size, rows    before, three a CU    256x256    192x256    128x256    128x128, two a CU
+//     1024      8192             229               184*       280        215         204
+//     1024      4096             119               101*       154        120         110
+//     1600      4096             282               301        254*       295         265
+//      960      8200             219               182        161*       215         207
+//      768     16384             285               326        256        223*        242
+//      768      8192             148               174        135        113*        121
+//      768      2043              46                59         47         40*         40
+//      640      3000              58                78         61         48*         51
+//     1408       917              88*               99-       107         96          86     (in the cache 70 / 85 / 94 / 93 / 79)
+//     1472 (x2) 1031              76*               96         85-        83          77
+//     1184      1285              86*              104         93-        91          88
+//     1792       976             141               151-       153        139*        141
 // Tried: 160-wide tiles (rows of 320 bytes, no whole lines: 1600 284); 32-wide k-tiles in rings of four and five (1024 8192 195, 202 against 187).
 constexpr int kM16WgradRows = 768;
 enum WgradTile { WG_NONE = 0, WG256x256, WG192x256, WG128x256, WG128x128 };

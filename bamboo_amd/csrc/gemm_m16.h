@@ -1,8 +1,12 @@
 // bf16 products on v_mfma_f32_16x16x32_bf16: NT and NN products on tiles of 256x256 down to 32x64, and large weight gradients (TN).
 //
-// Why this instruction: what bounds a large product is the card's power.  From registers, on normal data, 32x32x16 sustains 1777
-// TFLOP/s and 16x16x32 2030 (on zeros both 2470): per multiplication it moves half the accumulators.  The sums are the same: one
-// 16x16x32 adds its contraction in the order in which two 32x32x16 do, so these kernels and those of gemm_kernels.h give equal bits.
+// Why this instruction: the card's power.  From registers, on normal data, 32x32x16 sustains 1777 TFLOP/s and 16x16x32 2030 (on zeros both
+// 2470): per multiplication it moves half the accumulators.  The sums are the same: one 16x16x32 adds its contraction in the order in which
+// two 32x32x16 do, so these kernels and those of gemm_kernels.h give equal bits.
+//
+// What bounds a large product, counted in stages of 1024 and 1600 columns: power a tenth (2.05 to 2.25 of 2.4 GHz); the matrix pipe is 34 to 50 %
+// busy, 36 to 62 % of a CU in use.  The rest is CUs without a tile (the last round, 192 tiles of weight gradients), what a tile costs around its
+// loop -- 256x256 tiles with two outputs or times a tensor 34 and 37 % --, and waits for LDS and transfers.
 //
 // Loop: 64-wide k-tiles, global -> LDS by DMA, a ring of STAGES of them, two steps of 32 a k-tile.  While the matrix cores work on one
 // step's fragments the other step's are read into a second register set.  One barrier a k-tile: behind it the k-tile's own stage is
@@ -20,8 +24,9 @@
 // twice as slow (64x128 2043x768x3072 32.3).
 //
 // LDS: rows of a k-contiguous operand are 128 bytes, of a k-major one a k each; 16-byte chunks are swizzled so that the sixteen or
-// thirty-two lanes LDS serves at a time fall on different banks (counted: none conflicts).  The product is made transposed (B times A):
-// a lane holds one row of C.  NT and NN read the columns of two neighbouring fragments interleaved, so that its two accumulators are
+// thirty-two lanes LDS serves at a time fall on different banks (counted: none conflicts, but of NN's B, whose two groups of sixteen lanes, eight k
+// apart, meet on the same half of their chunks: conflicts are a quarter, of 256x128 tiles a third of LDS' cycles, LDS 19 and 38 % busy).  The product is made
+// transposed (B times A): a lane holds one row of C.  NT and NN read the columns of two neighbouring fragments interleaved, so that its two accumulators are
 // eight neighbouring columns and a store is 16 bytes; weight gradients store fp32, where four columns are.
 #pragma once
 #include "gemm_kernels.h"
